@@ -135,6 +135,22 @@ std::pair<int64_t, uint32_t> read_back(CallState& st, void* stream)
 
 int dtype_of(const torch::Tensor& t) { return t.scalar_type() == torch::kFloat32 ? FGL_F32 : FGL_BF16; }
 
+// a^T b, a layer's weight gradient: through fgl_weight_grad (which splits the long dimension) where the product has few output
+// tiles or a long k, through the library GEMM otherwise (fastgl/ops.py weight_grad: the same rule and its measurements)
+torch::Tensor weight_grad(const torch::Tensor& a, const torch::Tensor& b)
+{
+    const int64_t k = a.size(0), m = a.size(1), n = b.size(1);
+    const bool splits_k = m * n <= 65536 || k * k >= 256 * m * n;
+    if (!splits_k || k == 0 || m == 0 || n == 0 || b.size(0) != k || a.scalar_type() != b.scalar_type() || a.device() != b.device() ||
+        m >= (1 << 16) || n >= (1 << 16))
+        return torch::mm(a.transpose(0, 1), b);
+    auto out = torch::empty({m, n}, a.options());
+    auto ws = scratch(fgl_weight_grad_workspace_bytes(k, (int)m, (int)n), a);
+    ok(fgl_weight_grad(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), k, (int)m, (int)n, dtype_of(a), out.data_ptr(), n, nullptr,
+                       ws.data_ptr(), (size_t)ws.numel(), stream_of(a)));
+    return out;
+}
+
 // out[r] = sum_e w * feat[indices[e]] through fgl_aggregate; longest_row < 0: nothing known about the rows
 torch::Tensor aggregate(const torch::Tensor& indptr, const torch::Tensor& indices, const torch::Tensor& feat, int64_t n_rows,
                         int mode, int zero_policy, const torch::Tensor* row_norm, const torch::Tensor* col_norm,
@@ -321,7 +337,7 @@ std::vector<torch::Tensor> backward_gcn(torch::Tensor edge_ptr, torch::Tensor sr
     const int64_t n_src = input_feat.size(0), n_dst = d_input.size(0);
     auto t = transpose(edge_ptr, src_edges, n_dst, n_src, false);
     auto g = aggregate(t.ptr, t.idx, d_input, n_src, FGL_AGG_GCN, FGL_ZERO_ZEROS, &by_src, &by_dst, nullptr, 1, nullptr, -1, &t.longest);
-    return {torch::mm(g, weight.transpose(0, 1)), torch::mm(input_feat.transpose(0, 1), g)};
+    return {torch::mm(g, weight.transpose(0, 1)), weight_grad(input_feat, g)};
 }
 
 // aggregate_acc.cpp:173-199, exported under this spelling at :613 (kernel :375-427): [tmp W, tmp]
@@ -349,7 +365,7 @@ std::vector<torch::Tensor> backward_gin(torch::Tensor edge_ptr, torch::Tensor sr
     CHECK_FEAT(input_feat);
     c10::hip::HIPGuard guard(d_input.get_device());
     auto d_tmp = torch::mm(d_input, weight.transpose(0, 1));
-    auto d_w = torch::mm(input_feat.transpose(0, 1), d_input);
+    auto d_w = weight_grad(input_feat, d_input);
     auto t = transpose(edge_ptr, src_edges, d_input.size(0), src_nodes, false);
     auto d_x = aggregate(t.ptr, t.idx, d_tmp, src_nodes, FGL_AGG_SUM, FGL_ZERO_ZEROS, nullptr, nullptr, nullptr, 1, nullptr, -1, &t.longest);
     return {d_x, d_w};

@@ -84,7 +84,7 @@ class MA_Function(torch.autograd.Function):
             # rows without edges took no part in the sum: no gradient through them (as in the reference)
             has_edges = (edge_ptr[1:] != edge_ptr[:-1]).to(d_input.dtype)[:, None]
             d_out = d_input * has_edges
-            d_w = torch.mm(ax.transpose(0, 1), d_out)
+            d_w = ops.weight_grad(ax, d_out)
             d_x = None
             if ctx.needs_input_grad[5]:
                 d_ax = torch.mm(d_out, weight.transpose(0, 1))
@@ -104,13 +104,13 @@ class MA_Function(torch.autograd.Function):
             # reference's backward kernel, aggregate_acc_kernel.cu:498-500)
             ax = ops.aggregate(edge_ptr, src_edges, input_feat, mode="gcn", zero_policy="zeros", row_norm=dst_norm_degs,
                                col_norm=src_norm_degs, n_rows=int(d_input.size(0)))
-            d_x, d_w = None, torch.mm(ax.transpose(0, 1), d_input)
+            d_x, d_w = None, ops.weight_grad(ax, d_input)
         else:  # same arithmetic as backward_gcn, with the block's cached transpose
             t_ptr, t_idx = _transposed(ctx.transposed)
             g = ops.aggregate(t_ptr, t_idx, d_input, mode="gcn", zero_policy="zeros", row_norm=src_norm_degs,
                               col_norm=dst_norm_degs, n_rows=int(input_feat.size(0)))
             d_x = torch.mm(g, weight.transpose(0, 1))
-            d_w = torch.mm(input_feat.transpose(0, 1), g)
+            d_w = ops.weight_grad(input_feat, g)
         return None, None, None, None, None, d_x, d_w, None, None, None
 
 
@@ -194,7 +194,7 @@ class MA_Function_GIN(torch.autograd.Function):
         if ctx.transposed is None:
             d_x, d_w = ops.backward_gin(edge_ptr, src_edges, d_input, weight, tmp, ctx.src_nodes)
         else:
-            d_w = torch.mm(tmp.transpose(0, 1), d_input)
+            d_w = ops.weight_grad(tmp, d_input)
             d_x = None
             if ctx.needs_input_grad[3]:  # not for the first layer: its transposed block is never built
                 t_ptr, t_idx = _transposed(ctx.transposed)
@@ -225,6 +225,48 @@ class GIN(nn.Module):
             transposed = graph if isinstance(graph, Block) and torch.is_grad_enabled() else None
             h = layer(edge_ptr, src_edges, dst_nodes, h, neighbor_list[i], transposed)
         return h
+
+
+# ---------------------------------------------------------------------------------------
+# dense layers
+# ---------------------------------------------------------------------------------------
+class _LinearFunction(torch.autograd.Function):
+    """``x W^T + b`` whose weight and bias gradients come from one pass over the output's gradient (ops.weight_grad)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        ctx.with_bias = bias is not None
+        return nn.functional.linear(x, weight, bias)
+
+    @staticmethod
+    def backward(ctx, d_out):
+        x, weight = ctx.saved_tensors
+        d_x = d_w = d_b = None
+        if ctx.needs_input_grad[0]:
+            d_x = torch.mm(d_out, weight)
+        want_bias = ctx.with_bias and ctx.needs_input_grad[2]
+        if torch.is_grad_enabled():  # (a graph of the gradients is being built: operators that have gradients themselves)
+            d_w = torch.mm(d_out.transpose(0, 1), x)
+            d_b = d_out.sum(0) if want_bias else None
+        elif ctx.needs_input_grad[1] and want_bias:
+            d_w, d_b = ops.weight_grad(d_out, x, column_sums=True)
+        elif ctx.needs_input_grad[1]:
+            d_w = ops.weight_grad(d_out, x)
+        elif want_bias:
+            d_b = d_out.sum(0)
+        return d_x, d_w, d_b
+
+
+class _Linear(nn.Linear):
+    """``nn.Linear`` with ``_LinearFunction``'s backward pass for the inputs it is made for: matrices on the GPU in the
+    weight's own type (fp32 or bf16), outside autocast."""
+
+    def forward(self, x):
+        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and torch.is_grad_enabled()
+                and not torch.is_autocast_enabled()):
+            return super().forward(x)
+        return _LinearFunction.apply(x, self.weight, self.bias)
 
 
 # ---------------------------------------------------------------------------------------
@@ -275,7 +317,7 @@ class GATConv(nn.Module):
         super().__init__()
         self.out_feats = output_dim
         self.num_heads = num_heads
-        self.fc = nn.Linear(input_dim, output_dim * num_heads, bias=False)
+        self.fc = _Linear(input_dim, output_dim * num_heads, bias=False)
         self.attn_l = nn.Parameter(torch.empty(1, num_heads, output_dim))
         self.attn_r = nn.Parameter(torch.empty(1, num_heads, output_dim))
         self.feat_drop = nn.Dropout(feat_drop)
@@ -360,8 +402,8 @@ class SAGEConv(nn.Module):
 
     def __init__(self, input_dim, output_dim, bias=True):
         super().__init__()
-        self.fc_self = nn.Linear(input_dim, output_dim, bias=False)
-        self.fc_neigh = nn.Linear(input_dim, output_dim, bias=bias)
+        self.fc_self = _Linear(input_dim, output_dim, bias=False)
+        self.fc_neigh = _Linear(input_dim, output_dim, bias=bias)
 
     def forward(self, block, feat_src, feat_dst=None, use_global=False):
         h_neigh = MA_Function_Mean.apply(block, feat_src, use_global)

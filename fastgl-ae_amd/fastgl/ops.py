@@ -269,7 +269,7 @@ def backward_gcn(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, d_input, wei
     t_ptr, t_idx = block_transpose(edge_ptr, src_edges, n_dst, n_src)
     g = aggregate(t_ptr, t_idx, d_input, mode="gcn", zero_policy="zeros", row_norm=by_src, col_norm=by_dst, n_rows=n_src)
     d_x = torch.mm(g, weight.transpose(0, 1))
-    d_w = torch.mm(input_feat.transpose(0, 1), g)
+    d_w = weight_grad(input_feat, g)
     return [d_x, d_w]
 
 
@@ -294,7 +294,7 @@ def backward_gin(edge_ptr, src_edges, d_input, weight, input_feat, src_nodes):
     _check_input(weight, "weight", _FEAT)
     _check_input(input_feat, "input_feat", _FEAT)
     d_tmp = torch.mm(d_input, weight.transpose(0, 1))
-    d_w = torch.mm(input_feat.transpose(0, 1), d_input)
+    d_w = weight_grad(input_feat, d_input)
     n_dst = int(d_input.size(0))
     t_ptr, t_idx = block_transpose(edge_ptr, src_edges, n_dst, int(src_nodes))
     d_x = aggregate(t_ptr, t_idx, d_tmp, mode="sum", zero_policy="zeros", n_rows=int(src_nodes))
@@ -330,6 +330,37 @@ def backward_gat(edge_ptr, edge_data, src_edges, d_input, src_nodes, num_heads):
 # ---------------------------------------------------------------------------------------
 # extensions
 # ---------------------------------------------------------------------------------------
+def _splits_k(k, m, n):
+    """Whether ``weight_grad`` forms its product with the library's k-splitting kernel.  A weight gradient has a few output
+    tiles and a long k, where a GEMM that parallelises over tiles leaves the chip idle (100 x 256 outputs, k = 105 K: fp32
+    190 -> 72 us, bf16 245 -> 25 us; 256 x 256, k = 500: 119 -> 27 us).  Many tiles and a short k are the library GEMM's
+    (1024 x 1024, k = 8192: 145 us against 268 in fp32, 57 against 63 in bf16; 256 x 1024, k = 2000: 20 against 31)."""
+    return m * n <= 65536 or k * k >= 256 * m * n
+
+
+def weight_grad(a, b, column_sums=False):
+    """``a^T b`` for ``a`` [k, m] and ``b`` [k, n]: a dense layer's weight gradient from its input rows and the gradient of
+    its output (fp32 sums, result in the operands' dtype).  ``column_sums=True``: ``(a^T b, a.sum(0))``, with ``a`` the
+    gradient of the output the transposed weight gradient and the bias gradient of the layer."""
+    k, m, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
+    if not (a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
+            a.stride(1) == 1 and b.stride(1) == 1 and m <= a.stride(0) < 1 << 24 and n <= b.stride(0) < 1 << 24 and
+            m < 1 << 16 and n < 1 << 16 and b.size(0) == k and
+            _splits_k(k, m, n)):
+        d_w = torch.mm(a.transpose(0, 1), b)
+        return (d_w, a.sum(0)) if column_sums else d_w
+    lib = L.lib()
+    dev = a.device
+    with _on_device(dev):
+        d_w = torch.empty((m, n), dtype=a.dtype, device=dev)
+        sums = torch.empty(m, dtype=a.dtype, device=dev) if column_sums else None
+        ws = L.workspace(lib.fgl_weight_grad_workspace_bytes(k, m, n), dev)
+        L.check(lib.fgl_weight_grad(L.ptr(a), int(a.stride(0)), L.ptr(b), int(b.stride(0)), k, m, n,
+                                    L.F32 if a.dtype == torch.float32 else L.BF16, L.ptr(d_w), n, L.ptr(sums), L.ptr(ws), ws.numel(),
+                                    L.stream_handle()))
+    return (d_w, sums) if column_sums else d_w
+
+
 _MODES = {"sum": L.AGG_SUM, "mean": L.AGG_MEAN, "gcn": L.AGG_GCN, "colmean": L.AGG_COLMEAN, "edge": L.AGG_EDGE,
           "colmean_ptr": L.AGG_COLMEAN_PTR}
 _ZERO = {"self": L.ZERO_COPY_SELF, "zeros": L.ZERO_ZEROS}

@@ -378,6 +378,18 @@ int fgl_edge_softmax(const int32_t* d_indptr, const int32_t* d_indices, int64_t 
                      float negative_slope, float* d_alpha, void* stream);
 
 /* ---------------------------------------------------------------------------------
+ * Weight gradient of a dense layer: C[i, j] = sum over r < k of A[r, i] * B[r, j] -- the d_w = X^T G of backward_gcn /
+ * backward_gin (aggregate_acc.cpp:371-374,402-405, torch::mm on a transposed view there).  A: [k, m] with row stride
+ * lda, B: [k, n] with row stride ldb, C: [m, n] with row stride ldc, all of `dtype` (fp32, or bf16 with fp32 sums).
+ * d_sum_a (may be NULL): m elements of `dtype`, the column sums of A (with A = the gradient of the layer's output: its
+ * bias gradient), from the same pass.
+ * Meant for k far above m and n; the k splits are added in a fixed order (the same bits on every run).
+ * ------------------------------------------------------------------------------- */
+size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n);
+int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int64_t k, int m, int n, int dtype,
+                    void* d_c, int64_t ldc, void* d_sum_a, void* d_ws, size_t ws_bytes, void* stream);
+
+/* ---------------------------------------------------------------------------------
  * Seeded R-MAT key generator for the synthetic graphs (a=.57 b=.19 c=.19 d=.05).
  * For draw e in [first_edge, first_edge+n_edges): writes the two symmetrised keys
  * (row<<32 | col) of the in-neighbour CSR, or INT64_MAX twice for a self loop / an
