@@ -285,7 +285,10 @@ torch::Tensor cal_deg(torch::Tensor edges, int nodes_num)
     TORCH_CHECK(nodes_num >= 0, "negative node count");
     c10::hip::HIPGuard guard(edges.get_device());
     auto deg = torch::empty({std::max(nodes_num, 1)}, edges.options()).slice(0, 0, nodes_num);
-    ok(fgl_cal_deg(edges.data_ptr<int32_t>(), edges.numel(), nullptr, deg.data_ptr<int32_t>(), nodes_num, stream_of(edges)));
+    const size_t need = fgl_cal_deg_workspace_bytes(edges.numel(), nodes_num);
+    auto ws = need > 0 ? scratch(need, edges) : torch::Tensor();
+    ok(fgl_cal_deg_ws(edges.data_ptr<int32_t>(), edges.numel(), nullptr, deg.data_ptr<int32_t>(), nodes_num, need > 0 ? ws.data_ptr() : nullptr,
+                      need, stream_of(edges)));
     return deg;
 }
 

@@ -18,6 +18,7 @@
 // caller's knowledge of the longest row decides whether that launch is enqueued at all.
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
+#include "fgl_tile_rows.hpp"
 
 namespace fgl {
 
@@ -1107,58 +1108,89 @@ __global__ __launch_bounds__(kBlock) void transpose_count_kernel(const int32_t* 
 }
 
 // split counters, after their scan: the column offsets are every split-th prefix
-__global__ __launch_bounds__(kBlock) void transpose_offsets_kernel(const int32_t* __restrict__ scanned, int split,
-                                                                   int64_t n_cols_max, int32_t* __restrict__ t_indptr,
+// (split == 1: `scanned` is t_indptr itself, only the longest row is looked for)
+__global__ __launch_bounds__(kBlock) void transpose_offsets_kernel(const int32_t* scanned, int split,
+                                                                   int64_t n_cols_max, int32_t* t_indptr,
                                                                    int32_t* __restrict__ longest)
 {
     const int64_t stride = (int64_t)gridDim.x * kBlock;
+    int32_t most = 0;
     for (int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x; c <= n_cols_max; c += stride) {
         const int32_t begin = scanned[c * split];
-        t_indptr[c] = begin;
+        if (t_indptr != scanned) t_indptr[c] = begin;
         if (longest != nullptr && c < n_cols_max) {
             const int32_t len = scanned[(c + 1) * split] - begin;
-            if (len > FGL_SHORT_ROW_ENTRIES) atomicMax(longest, len);
+            most = len > most ? len : most;
         }
     }
+    // (one atomic per wave: thousands of long rows that report one by one queue up on the one address, 220 us on a whole graph)
+#pragma unroll
+    for (int d = kWave / 2; d >= 1; d >>= 1) {
+        const int32_t o = __shfl_xor(most, d, kWave);
+        most = o > most ? o : most;
+    }
+    if (longest != nullptr && lane_id() == 0 && most > FGL_SHORT_ROW_ENTRIES) atomicMax(longest, most);
 }
 
-__global__ __launch_bounds__(kBlock) void transpose_init_kernel(int32_t* __restrict__ counts, int64_t n, int32_t* __restrict__ longest)
+constexpr int kFillItems = 4;
+constexpr int kFillTile = kBlock * kFillItems;
+
+// counters to zero, and the row of every fill tile's first entry
+__global__ __launch_bounds__(kBlock) void transpose_init_kernel(int32_t* __restrict__ counts, int64_t n, int32_t* __restrict__ longest,
+                                                                const int32_t* __restrict__ indptr, int64_t n_rows_max,
+                                                                const int32_t* __restrict__ d_n_rows, int64_t tiles,
+                                                                int32_t* __restrict__ tile_row)
 {
     const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) counts[i] = 0;
-    if (longest != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *longest = 0;
+    const int64_t first = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    for (int64_t i = first; i < n; i += stride) counts[i] = 0;
+    if (longest != nullptr && first == 0) *longest = 0;
+    if (tile_row == nullptr) return;
+    const int64_t n_rows = actual_count(n_rows_max, d_n_rows);
+    for (int64_t r = first; r < n_rows; r += stride) mark_tile_rows<kFillTile>(indptr, r, tiles, tile_row);
 }
 
-// sixteen lanes per row: the row's entries are read coalesced and scattered in parallel
+// A lane per entry, a tile of 1024 entries per workgroup: the rows' lengths do not matter.  (Sixteen lanes per row before: 5.9
+// against 7.3 us on 8192 rows of 25 entries, but a hub's row of 85 K entries took 21 ms and one of 3 K half a millisecond.)
 __global__ __launch_bounds__(kBlock) void transpose_fill_kernel(const int32_t* __restrict__ indptr,
                                                                 const int32_t* __restrict__ indices, int64_t n_rows_max,
                                                                 const int32_t* __restrict__ d_n_rows, int64_t n_edges_max,
                                                                 const int32_t* __restrict__ t_indptr, int split,
-                                                                const int32_t* __restrict__ rank,
+                                                                const int32_t* __restrict__ rank, const int32_t* __restrict__ tile_row,
                                                                 int32_t* __restrict__ t_indices,
                                                                 int32_t* __restrict__ t_edge)
 {
-    constexpr int kLanes = 16;
+    __shared__ __align__(16) int s_row[kFillTile];
+    __shared__ int s_wave[kBlock / kWave];
     const int64_t n_rows = actual_count(n_rows_max, d_n_rows);
-    const int lane = (int)threadIdx.x % kLanes;
-    const int64_t stride = (int64_t)gridDim.x * (kBlock / kLanes);
-    for (int64_t r = (int64_t)blockIdx.x * (kBlock / kLanes) + (int)threadIdx.x / kLanes; r < n_rows; r += stride) {
-        const int64_t a = indptr[r];
-        int64_t b = indptr[r + 1];
-        if (b > n_edges_max) b = n_edges_max;
-        for (int64_t e = a + lane; e < b; e += kLanes) {
-            const int32_t k = rank[e];
-            if (k >= 0) {
-                // t_indptr: the column offsets, or (split > 1) the scanned split counters
-                const int64_t pos = (int64_t)t_indptr[(int64_t)indices[e] * split + (int)(e & (split - 1))] + k;
-                t_indices[pos] = (int32_t)r;
-                if (t_edge) t_edge[pos] = (int32_t)e;
-            }
-        }
+    int64_t n = n_rows > 0 ? (int64_t)indptr[n_rows] : 0;
+    if (n > n_edges_max) n = n_edges_max;
+    const int64_t tile = blockIdx.x, e0 = tile * kFillTile;
+    if (e0 >= n) return;  // (uniform over the workgroup)
+    int32_t k[kFillItems], base[kFillItems];
+#pragma unroll
+    for (int j = 0; j < kFillItems; ++j) {
+        const int64_t e = e0 + j * kBlock + threadIdx.x;
+        k[j] = e < n ? rank[e] : -1;
+        base[j] = k[j] >= 0 ? indices[e] : 0;
+    }
+    // t_indptr: the column offsets, or (split > 1) the scanned split counters
+#pragma unroll
+    for (int j = 0; j < kFillItems; ++j)
+        if (k[j] >= 0) base[j] = t_indptr[(int64_t)base[j] * split + (int)((e0 + j * kBlock + threadIdx.x) & (split - 1))];
+    tile_rows<kBlock, kFillItems>(indptr, n_rows, tile_row, tile, n, s_row, s_wave);
+#pragma unroll
+    for (int j = 0; j < kFillItems; ++j) {
+        if (k[j] < 0) continue;
+        const int64_t pos = (int64_t)base[j] + k[j];
+        const int at = j * kBlock + (int)threadIdx.x;
+        t_indices[pos] = s_row[at];
+        if (t_edge) t_edge[pos] = (int32_t)(e0 + at);
     }
 }
 
-// Blocks of at least this many entries count with kCountSplit counters per column (the extra scan and the
+// Blocks whose sizes are on the device only, and blocks too wide for buckets (fgl_bucket.hip takes the other large ones):
+// with at least this many entries they count with kCountSplit counters per column (the extra scan and the
 // offsets pass cost a few microseconds; below, the contention they remove costs less than that).
 constexpr int64_t kCountSplitMinEdges = (int64_t)1 << 20;
 constexpr int kCountSplit = 8;
@@ -1169,10 +1201,16 @@ size_t transpose_workspace_bytes(int64_t n_cols_max, int64_t n_edges_max, int so
     const int split = count_split(n_edges_max, sorted);
     Carver c(nullptr);
     c.take<int32_t>((size_t)n_edges_max);
+    c.take<int32_t>((size_t)ceil_div(n_edges_max, kFillTile));
     c.take<char>(scan_workspace_bytes(n_cols_max * split));
     if (split > 1) c.take<int32_t>((size_t)(n_cols_max * split + 1));
     if (sorted) c.take<char>(sorted_transpose_workspace_bytes(n_cols_max, n_edges_max));
-    return c.used();
+    size_t bytes = c.used();
+    if (!sorted && bucket_transpose_form(n_edges_max, n_cols_max)) {
+        const size_t b = bucket_workspace_bytes(n_edges_max, n_cols_max, true, true);
+        if (b > bytes) bytes = b;
+    }
+    return bytes;
 }
 
 // ---- dispatch ----------------------------------------------------------------------
@@ -1471,18 +1509,32 @@ FGL_EXPORT int fgl_block_transpose(const int32_t* d_indptr, const int32_t* d_ind
         return FGL_ERR_WORKSPACE;
     }
     hipStream_t s = as_stream(stream);
+    if (!sorted && d_n_rows == nullptr && d_n_cols == nullptr && n_rows_max > 0 && bucket_transpose_form(n_edges_max, n_cols_max)) {
+        int rc = launch_bucket_transpose(d_indptr, d_indices, n_rows_max, n_cols_max, n_edges_max, d_t_indptr, d_t_indices, d_t_edge,
+                                         d_t_longest_row, d_ws, s);
+        if (rc != FGL_OK || d_t_longest_row == nullptr) return rc;
+        int64_t blocks = ceil_div(n_cols_max + 1, kBlock);
+        if (blocks > 1024) blocks = 1024;
+        hipLaunchKernelGGL(transpose_offsets_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, d_t_indptr, 1, n_cols_max, d_t_indptr,
+                           d_t_longest_row);
+        FGL_CHECK_LAUNCH("transpose_offsets_kernel");
+        return FGL_OK;
+    }
     const int split = count_split(n_edges_max, sorted);
     Carver c(d_ws);
     int32_t* rank = c.take<int32_t>((size_t)n_edges_max);
+    const int64_t fill_tiles = ceil_div(n_edges_max, kFillTile);
+    int32_t* tile_row = c.take<int32_t>((size_t)fill_tiles);
+    const bool fills = !sorted && n_edges_max > 0 && n_rows_max > 0;
     char* scan_ws = c.take<char>(scan_workspace_bytes(n_cols_max * split));
     // the counts live in t_indptr and are scanned in place; with split counters they live in the workspace
     int32_t* counts = split > 1 ? c.take<int32_t>((size_t)(n_cols_max * split + 1)) : d_t_indptr;
     const int64_t n_counts = n_cols_max * split;
     {
-        int64_t blocks = ceil_div(n_counts + 1, kBlock);
+        int64_t blocks = ceil_div(n_counts + 1 > n_rows_max ? n_counts + 1 : n_rows_max, kBlock);
         if (blocks > 4096) blocks = 4096;
         hipLaunchKernelGGL(transpose_init_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, counts, n_counts + 1,
-                           d_t_longest_row);
+                           d_t_longest_row, d_indptr, n_rows_max, d_n_rows, fill_tiles, fills ? tile_row : nullptr);
         FGL_CHECK_LAUNCH("transpose_init_kernel");
     }
     if (n_edges_max > 0 && n_rows_max > 0) {
@@ -1508,11 +1560,9 @@ FGL_EXPORT int fgl_block_transpose(const int32_t* d_indptr, const int32_t* d_ind
         return launch_sorted_transpose_fill(d_indptr, d_indices, n_rows_max, n_cols_max, n_rows_max > 0 ? n_edges_max : 0,
                                             d_t_indices, d_t_edge, sort_ws, sort_bytes, s);
     }
-    if (n_edges_max > 0 && n_rows_max > 0) {
-        int64_t fill_blocks = ceil_div(n_rows_max, kBlock / 16);
-        if (fill_blocks > 16384) fill_blocks = 16384;
-        hipLaunchKernelGGL(transpose_fill_kernel, dim3((unsigned)fill_blocks), dim3(kBlock), 0, s, d_indptr,
-                           d_indices, n_rows_max, d_n_rows, n_edges_max, counts, split, rank, d_t_indices, d_t_edge);
+    if (fills) {
+        hipLaunchKernelGGL(transpose_fill_kernel, dim3((unsigned)fill_tiles), dim3(kBlock), 0, s, d_indptr, d_indices, n_rows_max, d_n_rows,
+                           n_edges_max, counts, split, rank, tile_row, d_t_indices, d_t_edge);
         FGL_CHECK_LAUNCH("transpose_fill_kernel");
     }
     return FGL_OK;

@@ -1,0 +1,418 @@
+// Counting and block transpose for large inputs, without an atomic per entry in device memory (stands in for the reference's
+// cal_deg, cuda_operators/utilis.cu:43-79, and -- as the transposed block that its backward kernels are gathers over -- for
+// its atomic scatter, aggregate_acc_kernel.cu:467-517,554-596).
+//
+// What bounds the plain form: every entry is one atomic on its id's counter.  The chip retires about 24 G of them a second
+// on random addresses, but updates of one address complete one after the other, some 90 ns each with a returned value, and
+// graphs have hubs: one id mentioned 85 K times holds a count of 54 M ids for 8.5 ms whatever the rest does.
+//
+// Two forms, by size:
+//
+// (1) ids against ranges (count_ranges_kernel, up to a few million ids over half a million counters): a workgroup owns a range
+//     of 16384 counters in LDS and reads a slice of the ids, counting those in its range; the slices' counts are stored and
+//     added by a second launch.  Every id is read once per range -- from cache -- and no counter is shared between workgroups.
+//     (1.2 M ids of a sampled block over 310 K counters: 66 -> 23 us.)
+//
+// (2) partition, then count (bucket_*): the entries are dealt into buckets of neighbouring columns (2^11 .. 2^13 wide) with one
+//     stable pass -- per tile of entries a histogram over the buckets in LDS, one scan over (bucket, tile), and a pass
+//     that stores every entry at its bucket's place -- and then counted bucket by bucket in LDS, a workgroup per
+//     segment of a bucket.  The transpose goes on from there: a segment learns its place in each of its columns from the
+//     add that delivers its counts (one atomic per segment and column), the counts are scanned into offsets, and every
+//     entry takes its position from its column's counter in LDS and is stored within its bucket's part of the output,
+//     which L2 holds.  Traffic: 4 reads and 2 writes of the entries in all.
+//     (54 M entries of a 2.4 M-node graph, hubs of 85 K: counts 5.9 / 13.2 ms -- unordered / sorted ids -- -> 0.50 / 0.67 ms;
+//     transpose 24.7 -> 1.55 ms, of which the scatter takes 0.48, the fill 0.74, each histogram 0.15.)
+#include "fgl_common.hpp"
+#include "fgl_kernels.hpp"
+#include "fgl_tile_rows.hpp"
+
+namespace fgl {
+
+// ---- (1) ids against ranges -------------------------------------------------------------------------------------
+constexpr int kRangeCounters = 16384;  // 64 KiB of LDS: two workgroups per CU
+constexpr int kRangeBlock = 1024;
+
+__global__ __launch_bounds__(kRangeBlock) void count_ranges_kernel(const int32_t* __restrict__ ids, int64_t n_max,
+                                                                   const int32_t* __restrict__ d_n, int64_t per_slice,
+                                                                   int64_t n_counters, int32_t* __restrict__ partial)
+{
+    __shared__ int s_cnt[kRangeCounters];
+    for (int i = (int)threadIdx.x; i < kRangeCounters; i += kRangeBlock) s_cnt[i] = 0;
+    __syncthreads();
+    const int64_t n = actual_count(n_max, d_n);
+    const int64_t first = (int64_t)blockIdx.y * per_slice;
+    const int64_t last = first + per_slice < n ? first + per_slice : n;
+    const int64_t base = (int64_t)blockIdx.x * kRangeCounters;
+    const int width = n_counters - base < kRangeCounters ? (int)(n_counters - base) : kRangeCounters;
+    constexpr int kInFlight = 8;
+    int64_t i = first + threadIdx.x;
+    for (; i + (kInFlight - 1) * kRangeBlock < last; i += kInFlight * kRangeBlock) {
+        int32_t id[kInFlight];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) id[j] = ids[i + (int64_t)j * kRangeBlock];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+            const int64_t at = (int64_t)id[j] - base;
+            if (at >= 0 && at < width) atomicAdd(&s_cnt[at], 1);
+        }
+    }
+    for (; i < last; i += kRangeBlock) {
+        const int64_t at = (int64_t)ids[i] - base;
+        if (at >= 0 && at < width) atomicAdd(&s_cnt[at], 1);
+    }
+    __syncthreads();
+    for (int c = (int)threadIdx.x; c < width; c += kRangeBlock) partial[(int64_t)blockIdx.y * n_counters + base + c] = s_cnt[c];
+}
+
+__global__ __launch_bounds__(kBlock) void count_ranges_sum_kernel(const int32_t* __restrict__ partial, int slices, int64_t n_counters,
+                                                                  int32_t* __restrict__ out)
+{
+    const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (c >= n_counters) return;
+    int s = 0;
+    int q = 0;
+    for (; q + 4 <= slices; q += 4) {
+        const int v0 = partial[q * n_counters + c], v1 = partial[(q + 1) * n_counters + c];
+        const int v2 = partial[(q + 2) * n_counters + c], v3 = partial[(q + 3) * n_counters + c];
+        s += (v0 + v1) + (v2 + v3);
+    }
+    for (; q < slices; ++q) s += partial[q * n_counters + c];
+    out[c] = s;
+}
+
+// ---- (2) buckets ------------------------------------------------------------------------------------------------
+constexpr int kBucketBlock = 512;
+constexpr int kBucketItems = 16;
+constexpr int kBucketTile = kBucketBlock * kBucketItems;  // entries per tile of the partition
+constexpr int kMaxBuckets = 2048;
+constexpr int kMaxWidthLog = 13;
+constexpr int kSegment = 32768;  // entries per workgroup of the passes over buckets
+
+struct BucketArgs {
+    const int32_t* ids;          // column of every entry
+    int64_t n_max;               // entries: at most this many, *d_n or indptr[n_rows] of them
+    const int32_t* d_n;
+    const int32_t* indptr;       // transpose only: rows of the entries
+    int64_t n_rows;
+    int64_t n_cols;
+    int width_log, buckets;
+    int64_t tiles;
+    int32_t* hist;               // [bucket][tile] counts, then their prefix sums (+ 1 entry: the total)
+    int32_t* tile_row;           // [tile] the row that holds the tile's first entry
+    int32_t* b_col;              // entries by bucket: column, row, position in ids
+    int32_t* b_row;
+    int32_t* b_edge;
+    int32_t* segments;           // [0] = how many, then per segment {bucket, first entry, entries}
+    int32_t* seg_base;           // [segment][2^width_log] a segment's first place in each of its columns
+    int32_t* counts;             // n_cols
+    int32_t* longest;            // (may be null) zeroed by the first launch
+    int32_t* t_indices;
+    int32_t* t_edge;
+};
+
+__device__ __forceinline__ int64_t bucket_entries(const BucketArgs& g)
+{
+    if (g.indptr == nullptr) return actual_count(g.n_max, g.d_n);
+    const int64_t n = g.n_rows > 0 ? (int64_t)g.indptr[g.n_rows] : 0;
+    return n < g.n_max ? n : g.n_max;
+}
+
+// counters to zero; the row of every tile's first entry (each row names the tiles that begin inside it)
+__global__ __launch_bounds__(kBlock) void bucket_init_kernel(const BucketArgs g)
+{
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    const int64_t first = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (g.longest != nullptr && first == 0) *g.longest = 0;
+    for (int64_t i = first; i < g.n_cols; i += stride) g.counts[i] = 0;
+    if (g.indptr == nullptr) return;
+    for (int64_t r = first; r < g.n_rows; r += stride) mark_tile_rows<kBucketTile>(g.indptr, r, g.tiles, g.tile_row);
+}
+
+__global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
+{
+    __shared__ int s_cnt[kMaxBuckets];
+    const int64_t n = bucket_entries(g);
+    const int64_t tile = blockIdx.x, e0 = tile * kBucketTile;
+    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) s_cnt[b] = 0;
+    __syncthreads();
+    int32_t c[kBucketItems];
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j) {
+        const int64_t e = e0 + j * kBucketBlock + threadIdx.x;
+        c[j] = e < n ? g.ids[e] : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j)
+        if (c[j] >= 0 && c[j] < g.n_cols) atomicAdd(&s_cnt[c[j] >> g.width_log], 1);
+    __syncthreads();
+    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) g.hist[(int64_t)b * g.tiles + tile] = s_cnt[b];
+}
+
+// every entry to its bucket's place
+template <bool ROWS, bool EDGES>
+__global__ __launch_bounds__(kBucketBlock) void bucket_scatter_kernel(const BucketArgs g)
+{
+    __shared__ int s_next[kMaxBuckets];
+    __shared__ __align__(16) int s_row[ROWS ? kBucketTile : 4];
+    __shared__ int s_wave[kBucketBlock / kWave];
+    const int64_t n = bucket_entries(g);
+    const int64_t tile = blockIdx.x, e0 = tile * kBucketTile;
+    if (e0 >= n) return;  // (uniform over the workgroup)
+    int32_t c[kBucketItems];
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j) {
+        const int64_t e = e0 + j * kBucketBlock + threadIdx.x;
+        c[j] = e < n ? g.ids[e] : -1;
+    }
+    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) s_next[b] = g.hist[(int64_t)b * g.tiles + tile];
+    if constexpr (ROWS) tile_rows<kBucketBlock, kBucketItems>(g.indptr, g.n_rows, g.tile_row, tile, n, s_row, s_wave);
+    else __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j) {
+        if (c[j] < 0 || c[j] >= g.n_cols) continue;
+        const int at = j * kBucketBlock + (int)threadIdx.x;
+        const int pos = atomicAdd(&s_next[c[j] >> g.width_log], 1);
+        g.b_col[pos] = c[j];
+        if constexpr (ROWS) g.b_row[pos] = s_row[at];
+        if constexpr (EDGES) g.b_edge[pos] = (int32_t)(e0 + at);
+    }
+}
+
+// One workgroup: the buckets cut into segments of at most kSegment entries.
+__global__ __launch_bounds__(1024) void bucket_segments_kernel(const BucketArgs g)
+{
+    __shared__ int smem[1024 / kWave + 1];
+    int carry = 0;
+    for (int start = 0; start < g.buckets; start += 1024) {
+        const int b = start + (int)threadIdx.x;
+        int first = 0, size = 0;
+        if (b < g.buckets) {
+            first = g.hist[(int64_t)b * g.tiles];
+            size = g.hist[(int64_t)(b + 1) * g.tiles] - first;
+        }
+        const int segs = (size + kSegment - 1) / kSegment;
+        int total;
+        const int at = carry + block_exclusive_scan<1024>(segs, smem, &total);
+        for (int q = 0; q < segs; ++q) {
+            int32_t* s = g.segments + 1 + 3 * (at + q);
+            s[0] = b;
+            s[1] = first + q * kSegment;
+            s[2] = size - q * kSegment < kSegment ? size - q * kSegment : kSegment;
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) g.segments[0] = carry;
+}
+
+// a segment's columns counted in LDS and added to the counters; PLACES: the sums before it are its places in the columns
+template <bool PLACES>
+__global__ __launch_bounds__(kBucketBlock) void bucket_count_kernel(const BucketArgs g)
+{
+    __shared__ int s_cnt[1 << kMaxWidthLog];
+    const int seg = (int)blockIdx.x;
+    if (seg >= g.segments[0]) return;
+    const int width = 1 << g.width_log;
+    const int bucket = g.segments[1 + 3 * seg], first = g.segments[2 + 3 * seg], size = g.segments[3 + 3 * seg];
+    const int col0 = bucket << g.width_log;
+    for (int c = (int)threadIdx.x; c < width; c += kBucketBlock) s_cnt[c] = 0;
+    __syncthreads();
+    constexpr int kInFlight = 8;
+    int i = (int)threadIdx.x;
+    for (; i + (kInFlight - 1) * kBucketBlock < size; i += kInFlight * kBucketBlock) {
+        int32_t c[kInFlight];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) c[j] = g.b_col[(int64_t)first + i + j * kBucketBlock];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) atomicAdd(&s_cnt[c[j] - col0], 1);
+    }
+    for (; i < size; i += kBucketBlock) atomicAdd(&s_cnt[g.b_col[(int64_t)first + i] - col0], 1);
+    __syncthreads();
+    for (int c = (int)threadIdx.x; c < width; c += kBucketBlock) {
+        const int v = s_cnt[c];
+        if (v == 0) continue;
+        if constexpr (PLACES) g.seg_base[((int64_t)seg << g.width_log) + c] = atomicAdd(&g.counts[(int64_t)col0 + c], v);
+        else atomicAdd(&g.counts[(int64_t)col0 + c], v);
+    }
+}
+
+// ... and, once the counts have become offsets, every entry into its column's row of the transposed block
+template <bool EDGES>
+__global__ __launch_bounds__(kBucketBlock) void bucket_fill_kernel(const BucketArgs g)
+{
+    __shared__ int s_next[1 << kMaxWidthLog];
+    const int seg = (int)blockIdx.x;
+    if (seg >= g.segments[0]) return;
+    const int width = 1 << g.width_log;
+    const int bucket = g.segments[1 + 3 * seg], first = g.segments[2 + 3 * seg], size = g.segments[3 + 3 * seg];
+    const int col0 = bucket << g.width_log;
+    for (int c = (int)threadIdx.x; c < width; c += kBucketBlock)  // (columns that the segment does not mention: never used)
+        if (col0 + c < g.n_cols) s_next[c] = g.counts[(int64_t)col0 + c] + g.seg_base[((int64_t)seg << g.width_log) + c];
+    __syncthreads();
+    constexpr int kInFlight = 4;
+    for (int i0 = (int)threadIdx.x; i0 < size; i0 += kInFlight * kBucketBlock) {
+        int32_t c[kInFlight], r[kInFlight], e[kInFlight];
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+            const int i = i0 + j * kBucketBlock;
+            if (i < size) {
+                c[j] = g.b_col[(int64_t)first + i];
+                r[j] = g.b_row[(int64_t)first + i];
+                if constexpr (EDGES) e[j] = g.b_edge[(int64_t)first + i];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kInFlight; ++j) {
+            if (i0 + j * kBucketBlock < size) {
+                const int pos = atomicAdd(&s_next[c[j] - col0], 1);
+                g.t_indices[pos] = r[j];
+                if constexpr (EDGES) g.t_edge[pos] = e[j];
+            }
+        }
+    }
+}
+
+// ---- sizes and launches -----------------------------------------------------------------------------------------
+static int range_slices(int64_t n_ids, int64_t n_counters)
+{
+    const int64_t ranges = ceil_div(n_counters, kRangeCounters);
+    int64_t s = 512 / ranges;  // two workgroups per CU
+    const int64_t most = ceil_div(n_ids, 16384);
+    if (s > most) s = most;
+    return (int)(s > 0 ? s : 1);
+}
+
+// What the forms measured (us, MI355X, replayed from a graph; atomics / ranges / buckets), counting:
+//   75 K ids, 27 K counters, R-MAT          24 /   7 /  -           205 K, 200 K, uniform    11.5 / 14 / 23
+//   144 K, 400 K, uniform                    9 /  15 /  -           251 K, 27 K, R-MAT         60 /  9 / 29
+//   2.5 M, 100 K, R-MAT                    314 /  24 / 45           3.1 M, 2.4 M, R-MAT       433 /  - / 60
+//   54 M, 2.4 M, R-MAT                    5900 /   - / 499          54 M, 2.4 M, sorted     13200 /  - / 674
+// Ranges read every id once per range and store every counter once per slice: they are kept to half a million counters (32
+// ranges) and four million ids, and small inputs take them where a counter is mentioned twice on average.
+static bool count_by_ranges(int64_t n_ids, int64_t n_counters)
+{
+    return n_ids >= ((int64_t)1 << 16) && n_ids < ((int64_t)1 << 22) && n_counters <= ((int64_t)1 << 19) &&
+           (n_ids >= ((int64_t)1 << 18) || 2 * n_counters <= n_ids);
+}
+static bool fits_buckets(int64_t n_entries, int64_t n_cols) { return n_entries <= 0x7FFFFFFF && n_cols > 0 && n_cols <= ((int64_t)kMaxBuckets << kMaxWidthLog); }
+static bool count_by_buckets(int64_t n_ids, int64_t n_counters)
+{
+    return n_ids >= ((int64_t)1 << 20) && !count_by_ranges(n_ids, n_counters) && fits_buckets(n_ids, n_counters);
+}
+// Transposing (atomics with the fill by entries / buckets): 205 K entries, 200 K columns, uniform 26 / 43; 251 K, 27 K, R-MAT 88 / 72;
+// 434 K, a sampled block 93 / 75; 600 K, 200 K, uniform 47 / 50; 1.15 M, a sampled block 113 / 91; 2.5 M, 100 K, R-MAT 335 / 108;
+// 54 M, 2.4 M, R-MAT 24700 (sixteen lanes per row) / 1550.  Columns of graphs are skewed: the line is where those gain.
+bool bucket_transpose_form(int64_t n_entries, int64_t n_cols) { return n_entries >= ((int64_t)1 << 18) && fits_buckets(n_entries, n_cols); }
+
+static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edges, void* ws, BucketArgs* g, size_t* bytes)
+{
+    int w = 11;
+    while ((n_cols + ((int64_t)1 << w) - 1) >> w > kMaxBuckets) ++w;
+    g->width_log = w;
+    g->buckets = (int)((n_cols + ((int64_t)1 << w) - 1) >> w);
+    g->tiles = ceil_div(n_entries, kBucketTile);
+    const int64_t max_segments = g->buckets + n_entries / kSegment + 1;
+    Carver c(ws);
+    g->hist = c.take<int32_t>((size_t)(g->buckets * g->tiles + 1));
+    g->segments = c.take<int32_t>((size_t)(1 + 3 * max_segments));
+    g->b_col = c.take<int32_t>((size_t)n_entries);
+    if (rows) {
+        g->tile_row = c.take<int32_t>((size_t)g->tiles);
+        g->b_row = c.take<int32_t>((size_t)n_entries);
+        g->seg_base = c.take<int32_t>((size_t)(max_segments << w));
+    }
+    if (edges) g->b_edge = c.take<int32_t>((size_t)n_entries);
+    *bytes = c.used();
+}
+
+size_t bucket_workspace_bytes(int64_t n_entries, int64_t n_cols, bool rows, bool edges)
+{
+    BucketArgs g;
+    size_t bytes;
+    bucket_layout(n_entries, n_cols, rows, edges, nullptr, &g, &bytes);
+    return bytes;
+}
+
+static int launch_partition(const BucketArgs& g, bool rows, bool edges, hipStream_t stream)
+{
+    int64_t init_items = g.n_cols;
+    if (rows && g.n_rows > init_items) init_items = g.n_rows;
+    int64_t blocks = ceil_div(init_items, kBlock);
+    if (blocks > 8192) blocks = 8192;
+    hipLaunchKernelGGL(bucket_init_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
+    hipLaunchKernelGGL(bucket_hist_kernel, dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    FGL_CHECK_LAUNCH("bucket_hist_kernel");
+    const int64_t n_hist = g.buckets * g.tiles;
+    char* scan_ws = reinterpret_cast<char*>(g.b_edge ? g.b_edge : g.b_col);  // (not written yet: the scan's scratch fits into any of the entry arrays)
+    int rc = launch_exclusive_sum(g.hist, n_hist, nullptr, g.hist, nullptr, scan_ws, scan_workspace_bytes(n_hist), stream);
+    if (rc != FGL_OK) return rc;
+    if (rows && edges) hipLaunchKernelGGL((bucket_scatter_kernel<true, true>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    else if (rows) hipLaunchKernelGGL((bucket_scatter_kernel<true, false>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    else hipLaunchKernelGGL((bucket_scatter_kernel<false, false>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    hipLaunchKernelGGL(bucket_segments_kernel, dim3(1), dim3(1024), 0, stream, g);
+    const unsigned segs = (unsigned)(g.buckets + g.n_max / kSegment + 1);
+    if (rows) hipLaunchKernelGGL(bucket_count_kernel<true>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    else hipLaunchKernelGGL(bucket_count_kernel<false>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    FGL_CHECK_LAUNCH("bucket_count_kernel");
+    return FGL_OK;
+}
+
+size_t count_workspace_bytes(int64_t n_ids, int64_t n_counters)
+{
+    if (count_by_buckets(n_ids, n_counters)) return bucket_workspace_bytes(n_ids, n_counters, false, false);
+    if (count_by_ranges(n_ids, n_counters)) return align_up((size_t)range_slices(n_ids, n_counters) * n_counters * sizeof(int32_t), 256);
+    return 0;
+}
+
+// counts[0 .. n_counters) of the ids; false if this size has no form here (the caller counts with atomics)
+bool launch_count(const int32_t* d_ids, int64_t n_ids, const int32_t* d_n, int64_t n_counters, int32_t* d_counts, void* d_ws,
+                  hipStream_t stream, int* rc)
+{
+    *rc = FGL_OK;
+    if (count_by_buckets(n_ids, n_counters)) {
+        BucketArgs g;
+        memset(&g, 0, sizeof(g));
+        size_t bytes;
+        bucket_layout(n_ids, n_counters, false, false, d_ws, &g, &bytes);
+        g.ids = d_ids; g.n_max = n_ids; g.d_n = d_n; g.n_cols = n_counters; g.counts = d_counts;
+        *rc = launch_partition(g, false, false, stream);
+        return true;
+    }
+    if (!count_by_ranges(n_ids, n_counters)) return false;
+    const int slices = range_slices(n_ids, n_counters);
+    int32_t* partial = static_cast<int32_t*>(d_ws);
+    hipLaunchKernelGGL(count_ranges_kernel, dim3((unsigned)ceil_div(n_counters, kRangeCounters), (unsigned)slices), dim3(kRangeBlock), 0, stream,
+                       d_ids, n_ids, d_n, ceil_div(n_ids, slices), n_counters, partial);
+    hipLaunchKernelGGL(count_ranges_sum_kernel, dim3((unsigned)ceil_div(n_counters, kBlock)), dim3(kBlock), 0, stream, partial, slices,
+                       n_counters, d_counts);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error("count_ranges_kernel: launch failed: %s", hipGetErrorString(e));
+        *rc = FGL_ERR_HIP;
+    }
+    return true;
+}
+
+// d_t_indptr, d_t_indices and d_t_edge (may be null) of the transposed block; *d_longest (may be null) becomes zero.
+int launch_bucket_transpose(const int32_t* d_indptr, const int32_t* d_indices, int64_t n_rows, int64_t n_cols, int64_t n_edges,
+                            int32_t* d_t_indptr, int32_t* d_t_indices, int32_t* d_t_edge, int32_t* d_longest, void* d_ws, hipStream_t stream)
+{
+    BucketArgs g;
+    memset(&g, 0, sizeof(g));
+    size_t bytes;
+    const bool edges = d_t_edge != nullptr;
+    bucket_layout(n_edges, n_cols, true, edges, d_ws, &g, &bytes);
+    g.ids = d_indices; g.n_max = n_edges; g.indptr = d_indptr; g.n_rows = n_rows; g.n_cols = n_cols;
+    g.counts = d_t_indptr; g.longest = d_longest; g.t_indices = d_t_indices; g.t_edge = d_t_edge;
+    int rc = launch_partition(g, true, edges, stream);
+    if (rc != FGL_OK) return rc;
+    // (the histogram is no longer needed: scratch of this scan)
+    rc = launch_exclusive_sum(d_t_indptr, n_cols, nullptr, d_t_indptr, nullptr, g.hist, scan_workspace_bytes(n_cols), stream);
+    if (rc != FGL_OK) return rc;
+    const unsigned segs = (unsigned)(g.buckets + n_edges / kSegment + 1);
+    if (edges) hipLaunchKernelGGL(bucket_fill_kernel<true>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    else hipLaunchKernelGGL(bucket_fill_kernel<false>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    FGL_CHECK_LAUNCH("bucket_fill_kernel");
+    return FGL_OK;
+}
+
+}  // namespace fgl

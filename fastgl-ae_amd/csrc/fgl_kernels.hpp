@@ -121,6 +121,15 @@ int launch_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, 
                          const int32_t* d_readback_counts = nullptr, // (may be null) instead of those two words: a copy of this array, which holds
                          int n_readback_counts = 0);                 //   *d_n_total_out and the status word, taken when the node total is final
 
+// counting and transpose of large inputs (fgl_bucket.hip)
+size_t count_workspace_bytes(int64_t n_ids, int64_t n_counters);  // 0: counted with atomics, no workspace
+bool launch_count(const int32_t* d_ids, int64_t n_ids, const int32_t* d_n, int64_t n_counters, int32_t* d_counts, void* d_ws,
+                  hipStream_t stream, int* rc);
+bool bucket_transpose_form(int64_t n_entries, int64_t n_cols);
+size_t bucket_workspace_bytes(int64_t n_entries, int64_t n_cols, bool rows, bool edges);
+int launch_bucket_transpose(const int32_t* d_indptr, const int32_t* d_indices, int64_t n_rows, int64_t n_cols, int64_t n_edges,
+                            int32_t* d_t_indptr, int32_t* d_t_indices, int32_t* d_t_edge, int32_t* d_longest, void* d_ws, hipStream_t stream);
+
 // deterministic block transpose (fgl_transpose_sort.hip): fills t_indices / t_edge given the offsets
 size_t sorted_transpose_workspace_bytes(int64_t n_cols, int64_t n_edges);
 int launch_sorted_transpose_fill(const int32_t* d_indptr, const int32_t* d_indices, int64_t n_rows, int64_t n_cols,

@@ -240,19 +240,45 @@ FGL_EXPORT int fgl_exclusive_sum_i32(const int32_t* d_in, int64_t n_max, const i
     return launch_exclusive_sum(d_in, n_max, d_n, d_out, nullptr, d_ws, ws_bytes, as_stream(stream));
 }
 
+static int cal_deg_atomic(const int32_t* d_ids, int64_t n_ids_max, const int32_t* d_n_ids, int32_t* d_deg, int64_t n_nodes, hipStream_t stream)
+{
+    int rc = launch_fill_u32(reinterpret_cast<uint32_t*>(d_deg), n_nodes, 0u, stream);
+    if (rc != FGL_OK) return rc;
+    if (n_ids_max == 0) return FGL_OK;
+    const int64_t blocks = ceil_div(n_ids_max, kBlock);
+    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "cal_deg: too many ids");
+    hipLaunchKernelGGL(cal_deg_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, d_ids, n_ids_max, d_n_ids, d_deg, n_nodes);
+    FGL_CHECK_LAUNCH("cal_deg_kernel");
+    return FGL_OK;
+}
+
 FGL_EXPORT int fgl_cal_deg(const int32_t* d_ids, int64_t n_ids_max, const int32_t* d_n_ids, int32_t* d_deg,
                            int64_t n_nodes, void* stream)
 {
     FGL_REQUIRE(n_ids_max >= 0 && n_nodes >= 0, "cal_deg: negative size");
     FGL_REQUIRE(d_deg != nullptr || n_nodes == 0, "cal_deg: null output");
     FGL_REQUIRE(d_ids != nullptr || n_ids_max == 0, "cal_deg: null input");
-    int rc = launch_fill_u32(reinterpret_cast<uint32_t*>(d_deg), n_nodes, 0u, as_stream(stream));
-    if (rc != FGL_OK) return rc;
-    if (n_ids_max == 0) return FGL_OK;
-    const int64_t blocks = ceil_div(n_ids_max, kBlock);
-    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "cal_deg: too many ids");
-    hipLaunchKernelGGL(cal_deg_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, as_stream(stream), d_ids, n_ids_max,
-                       d_n_ids, d_deg, n_nodes);
-    FGL_CHECK_LAUNCH("cal_deg_kernel");
-    return FGL_OK;
+    return cal_deg_atomic(d_ids, n_ids_max, d_n_ids, d_deg, n_nodes, as_stream(stream));
+}
+
+FGL_EXPORT size_t fgl_cal_deg_workspace_bytes(int64_t n_ids_max, int64_t n_nodes)
+{
+    if (n_ids_max < 0 || n_nodes < 0) return 0;
+    return count_workspace_bytes(n_ids_max, n_nodes);
+}
+
+FGL_EXPORT int fgl_cal_deg_ws(const int32_t* d_ids, int64_t n_ids_max, const int32_t* d_n_ids, int32_t* d_deg, int64_t n_nodes,
+                              void* d_ws, size_t ws_bytes, void* stream)
+{
+    FGL_REQUIRE(n_ids_max >= 0 && n_nodes >= 0, "cal_deg: negative size");
+    FGL_REQUIRE(d_deg != nullptr || n_nodes == 0, "cal_deg: null output");
+    FGL_REQUIRE(d_ids != nullptr || n_ids_max == 0, "cal_deg: null input");
+    const size_t need = count_workspace_bytes(n_ids_max, n_nodes);
+    if (need > 0 && (d_ws == nullptr || ws_bytes < need)) {
+        set_error("cal_deg: workspace too small (%zu < %zu)", ws_bytes, need);
+        return FGL_ERR_WORKSPACE;
+    }
+    int rc;
+    if (need > 0 && launch_count(d_ids, n_ids_max, d_n_ids, n_nodes, d_deg, d_ws, as_stream(stream), &rc)) return rc;
+    return cal_deg_atomic(d_ids, n_ids_max, d_n_ids, d_deg, n_nodes, as_stream(stream));
 }

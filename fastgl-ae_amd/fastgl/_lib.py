@@ -36,6 +36,8 @@ SIGNATURES = {
     "fgl_exclusive_sum_workspace_bytes": (_sz, [_i64]),
     "fgl_exclusive_sum_i32": (_i32, [_vp, _i64, _vp, _vp, _vp, _sz, _vp]),
     "fgl_cal_deg": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp]),
+    "fgl_cal_deg_workspace_bytes": (_sz, [_i64, _i64]),
+    "fgl_cal_deg_ws": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp, _sz, _vp]),
     "fgl_sample_workspace_bytes": (_sz, [_i64, _i32]),
     "fgl_sample_node": (_i32, [_vp, _i32, _vp, _i64, _vp, _i64, _vp, _i32, _u64, _u32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fgl_sample_node_static": (_i32, [_vp, _i32, _vp, _i64, _vp, _i64, _vp, _i32, _u64, _u32, _vp, _vp, _vp, _vp, _vp, _vp]),

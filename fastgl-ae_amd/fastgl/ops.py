@@ -211,7 +211,10 @@ def cal_deg(edges, nodes_num):
     dev = edges.device
     with _on_device(dev):
         deg = torch.empty(max(n, 1), dtype=torch.int32, device=dev)[:n]
-        L.check(L.lib().fgl_cal_deg(L.ptr(edges), int(edges.numel()), None, L.ptr(deg), n, L.stream_handle()))
+        lib = L.lib()
+        ws_bytes = lib.fgl_cal_deg_workspace_bytes(int(edges.numel()), n)
+        ws = L.workspace(ws_bytes, dev) if ws_bytes else None
+        L.check(lib.fgl_cal_deg_ws(L.ptr(edges), int(edges.numel()), None, L.ptr(deg), n, L.ptr(ws), ws_bytes, L.stream_handle()))
     return deg
 
 

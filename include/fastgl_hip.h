@@ -116,6 +116,12 @@ int fgl_exclusive_sum_i32(const int32_t* d_in, int64_t n_max, const int32_t* d_n
  * d_deg[0..n_nodes) = histogram of d_ids[0..n_ids).  d_deg is cleared by the call. */
 int fgl_cal_deg(const int32_t* d_ids, int64_t n_ids_max, const int32_t* d_n_ids, int32_t* d_deg,
                 int64_t n_nodes, void* stream);
+/* The same with a workspace, for inputs where one atomic per id is the slow way (from 65 536 ids on; updates of a
+ * hub id's counter run one after the other): the counts are formed in LDS.  fgl_cal_deg_workspace_bytes may
+ * be 0 (small inputs), d_ws may be NULL then. */
+size_t fgl_cal_deg_workspace_bytes(int64_t n_ids_max, int64_t n_nodes);
+int fgl_cal_deg_ws(const int32_t* d_ids, int64_t n_ids_max, const int32_t* d_n_ids, int32_t* d_deg, int64_t n_nodes,
+                   void* d_ws, size_t ws_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------
  * sample_node -- replaces fastgl.sample_node (aggregate_acc.cpp:491-512, sample.cu:102-203).

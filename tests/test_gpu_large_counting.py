@@ -1,0 +1,87 @@
+"""cal_deg and block_transpose where they change form (counted with atomics, in LDS ranges, or partitioned into buckets first), hub ids, ids outside the range, rows of every length and gaps of empty rows.  Whole
+numbers throughout: equal to torch.bincount, and to the stable sort by column where order is promised or sorted away."""
+import pytest
+import torch
+
+import fastgl
+
+pytestmark = pytest.mark.gpu
+
+M = 1 << 20
+
+
+def _ids(n, bins, gen, device, hub):
+    ids = torch.randint(0, bins, (n,), generator=gen, device=device, dtype=torch.int32)
+    if hub:  # a third of the mentions to one id, and a few that are no ids at all
+        ids[torch.rand(n, generator=gen, device=device) < 0.33] = bins // 2
+        ids[::1001] = -1
+        ids[5::1003] = bins + 7
+    return ids
+
+
+@pytest.mark.parametrize("hub", [False, True])
+@pytest.mark.parametrize("n,bins", [((1 << 16) - 1, 1000), (1 << 16, 1 << 15), (1 << 16, (1 << 15) + 1), ((1 << 18) - 1, 1000), (1 << 18, 16384), ((1 << 18) + 3, 16385), (M + 5, 1 << 19), (M, (1 << 19) + 1),
+                                    (300_001, 1), (4 * M - 1, 300_000), (4 * M, 1), (4 * M, 2048), (4 * M + 8191, 2049),
+                                    (5 * M + 77, 3_000_001), (4 * M, 5 * M)])
+def test_cal_deg(cuda, n, bins, hub):
+    gen = torch.Generator(device=cuda).manual_seed(n + bins)
+    ids = _ids(n, bins, gen, cuda, hub)
+    got = fastgl.cal_deg(ids, bins)
+    valid = ids[(ids >= 0) & (ids < bins)].long()
+    assert torch.equal(got.long(), torch.bincount(valid, minlength=bins))
+
+
+def _csr(lengths, device):
+    ptr = torch.zeros(len(lengths) + 1, dtype=torch.int64)
+    ptr[1:] = torch.cumsum(lengths, 0)
+    return ptr.int().to(device)
+
+
+def _lengths(kind, gen):
+    if kind == "fanout":      # rows of a sampled block
+        return torch.randint(0, 26, (20_000,), generator=gen)
+    if kind == "hub":         # one row of 100 K entries among short and empty ones
+        x = torch.randint(0, 4, (30_000,), generator=gen)
+        x[17] = 100_000
+        return x
+    if kind == "gaps":        # long gaps of empty rows, also in front and at the end
+        x = torch.zeros(200_000, dtype=torch.int64)
+        x[100_000:100_040] = 701
+        x[199_000] = 3
+        return x
+    if kind == "large":       # past the partition's threshold, hub rows and a gap
+        x = torch.randint(0, 15, (600_000,), generator=gen)
+        x[5] = 300_000
+        x[400_000:520_000] = 0
+        x[599_000] = 50_001
+        return x
+    return torch.tensor([1])  # "one"
+
+
+@pytest.mark.parametrize("edge_ids", [False, True])
+@pytest.mark.parametrize("kind,n_cols", [("one", 1), ("fanout", 3000), ("hub", 70_000), ("gaps", 500), ("large", 1), ("large", 2_500_000),
+                                         ("large", 4096)])
+def test_block_transpose(cuda, kind, n_cols, edge_ids):
+    gen = torch.Generator().manual_seed(n_cols)
+    lengths = _lengths(kind, gen)
+    ptr = _csr(lengths, cuda)
+    nnz = int(lengths.sum())
+    cols = torch.randint(0, n_cols, (nnz,), generator=gen, dtype=torch.int32)
+    cols[torch.rand(nnz, generator=gen) < 0.1] = n_cols // 3  # a hub column
+    cols = cols.to(cuda)
+    n_rows = len(lengths)
+    got = fastgl.block_transpose(ptr, cols, n_rows, n_cols, edge_ids=edge_ids)
+    rows = torch.repeat_interleave(torch.arange(n_rows, device=cuda), lengths.to(cuda))
+    counts = torch.bincount(cols.long(), minlength=n_cols)
+    want_ptr = torch.zeros(n_cols + 1, dtype=torch.int64, device=cuda)
+    want_ptr[1:] = torch.cumsum(counts, 0)
+    assert torch.equal(got[0].long(), want_ptr)
+    longest = int(counts.max())
+    assert int(got[0].fgl_longest_row) == longest if longest > 32 else int(got[0].fgl_longest_row) <= 32
+    # the order inside a column is not promised: compare (column, row[, entry]) after sorting
+    col_of = torch.repeat_interleave(torch.arange(n_cols, device=cuda), counts)
+    assert torch.equal(torch.sort(col_of * n_rows + got[1].long()).values, torch.sort(cols.long() * n_rows + rows).values)
+    if edge_ids:
+        e = got[2].long()
+        assert torch.equal(torch.sort(e).values, torch.arange(nnz, device=cuda))
+        assert torch.equal(cols.long()[e], col_of) and torch.equal(rows[e], got[1].long())
