@@ -144,20 +144,29 @@ struct AggArgs {
     int skip_rows_longer_than;  // aggregate_kernel leaves rows with more entries to aggregate_long_rows_kernel
     int n_heads;
     int unit_dim;               // D / n_heads
-    int col_norm_is_ptr;        // FGL_AGG_COLMEAN: col_norm is an offsets array, the counts are its differences
+    int col_norm_is_ptr;        // col_norm is an offsets array, the counts are its differences
 };
 
 // per-edge weight, evaluated by the lane that loaded the neighbour id
 template <int MODE>
 __device__ __forceinline__ float edge_weight(int col, float row_factor, const int32_t* __restrict__ col_norm, int col_norm_is_ptr)
 {
-    if (MODE == FGL_AGG_GCN) return row_factor * (1.0f / sqrtf((float)col_norm[col]));
-    if (MODE == FGL_AGG_COLMEAN) {
+    if (MODE == FGL_AGG_GCN || MODE == FGL_AGG_COLMEAN) {
         // (the columns' entry counts, or the offsets array they are the differences of)
         const int c = col_norm_is_ptr ? col_norm[col + 1] - col_norm[col] : col_norm[col];
+        if (MODE == FGL_AGG_GCN) return row_factor * (1.0f / sqrtf((float)c));
         return 1.0f / (float)(c > 1 ? c : 1);
     }
     return row_factor;  // SUM: 1, MEAN: 1/deg(row)
+}
+
+// the row's share of its entries' weights; `entries`: how many the row has (which is its GCN degree where none is given)
+template <int MODE>
+__device__ __forceinline__ float row_weight(const int32_t* __restrict__ row_norm, int64_t row, int entries)
+{
+    if (MODE == FGL_AGG_MEAN) return 1.0f / (float)entries;
+    if (MODE == FGL_AGG_GCN) return 1.0f / sqrtf((float)(row_norm != nullptr ? row_norm[row] : entries));
+    return 1.0f;
 }
 
 // The last lane of a row whose length is not a multiple of VEC can move the row's last VEC columns
@@ -272,9 +281,7 @@ __device__ __forceinline__ void gather_row(const AggArgs& g, const LaneSlice<T, 
 {
     const int32_t* __restrict__ indices = g.indices;
     const T* __restrict__ X = static_cast<const T*>(g.x);
-    float row_factor = 1.0f;
-    if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(b - a);
-    if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[row]);
+    const float row_factor = row_weight<MODE>(g.row_norm, row, b - a);
 
     for (int base = a; base < b; base += LPR) {
         const int cnt = (b - base) < LPR ? (b - base) : LPR;
@@ -534,9 +541,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_split_kernel(const AggArgs g
     if (a == b) {
         if (part == 0 && live && g.zero_policy == FGL_ZERO_COPY_SELF) IO::fma(acc, 1.0f, ls.load(X + row * ldx + col0));
     } else {
-        float row_factor = 1.0f;
-        if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(b - a);
-        if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[row]);
+        const float row_factor = row_weight<MODE>(g.row_norm, row, b - a);
         for (int base = a; base < b; base += W) {
             const int cnt = (b - base) < W ? (b - base) : W;
             int my_col = 0;
@@ -654,9 +659,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_bundle_kernel(const AggArgs 
                         end_j = off[k + 1];
                     }
                 }
-                float row_factor = 1.0f;
-                if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(end_j - begin_j);
-                if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[r0 + j]);
+                const float row_factor = row_weight<MODE>(g.row_norm, r0 + j, end_j - begin_j);
                 if (MODE != FGL_AGG_EDGE) my_w = edge_weight<MODE>(my_col, row_factor, g.col_norm, g.col_norm_is_ptr);
                 my_tag = j | (e + 1 == end_j ? 256 : 0);
             }
@@ -771,9 +774,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_flat_kernel(const AggArgs g,
     if (a == b) {
         if (g.zero_policy == FGL_ZERO_COPY_SELF) IO::fma(acc, 1.0f, load(X + row * ldx + col0));
     } else {
-        float row_factor = 1.0f;
-        if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(b - a);
-        if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[row]);
+        const float row_factor = row_weight<MODE>(g.row_norm, row, b - a);
         for (int base = a; base < b; base += kFlatChunk) {
             const int end = b - base < kFlatChunk ? b : base + kFlatChunk;
             float part[VEC];
@@ -880,9 +881,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_flat_bundle_kernel(const Agg
                         end_j = off[k + 1];
                     }
                 }
-                float row_factor = 1.0f;
-                if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(end_j - begin_j);
-                if (MODE == FGL_AGG_GCN && cb + j < total) row_factor = 1.0f / sqrtf((float)g.row_norm[r0 + row_j]);
+                const float row_factor = cb + j < total ? row_weight<MODE>(g.row_norm, r0 + row_j, end_j - begin_j) : 0.0f;
                 w[j] = cb + j < total ? edge_weight<MODE>(c[j], row_factor, g.col_norm, g.col_norm_is_ptr) : 0.0f;
                 tag[j] = row_j | (e + 1 == end_j ? 256 : 0);
             }
@@ -921,9 +920,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_flat_bundle_kernel(const Agg
         if (a == b) {
             if (g.zero_policy == FGL_ZERO_COPY_SELF) IO::fma(acc, 1.0f, load(X + row * ldx + col0));
         } else {
-            float row_factor = 1.0f;
-            if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(b - a);
-            if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[row]);
+            const float row_factor = row_weight<MODE>(g.row_norm, row, b - a);
             for (int base = a; base < b; base += kFlatChunk) {
                 const int end = b - base < kFlatChunk ? b : base + kFlatChunk;
                 float part[VEC];
@@ -990,9 +987,7 @@ __global__ __launch_bounds__(kLongBlock) void aggregate_long_rows_kernel(const A
             // the order in which the long rows of a pass are taken does not matter: each is summed on its own
             const int64_t row = (pass * kLongBlock + found[i]) * gridDim.x + blockIdx.x;
             const int a = indptr[row], b = indptr[row + 1];
-            float row_factor = 1.0f;
-            if (MODE == FGL_AGG_MEAN) row_factor = 1.0f / (float)(b - a);
-            if (MODE == FGL_AGG_GCN) row_factor = 1.0f / sqrtf((float)g.row_norm[row]);
+            const float row_factor = row_weight<MODE>(g.row_norm, row, b - a);
             float acc[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
@@ -1441,6 +1436,23 @@ static int launch_agg_vec(int mode, int64_t longest_row_max, int64_t n_entries_m
     }
 }
 
+// Rows of x without entries in the CSR become zeros.  A lane looks at a row; the few rows found are cleared by the whole wave.
+__global__ __launch_bounds__(kBlock) void zero_empty_rows_kernel(const int32_t* __restrict__ indptr, int64_t n_rows_max,
+                                                                 const int32_t* __restrict__ d_n_rows, char* __restrict__ x,
+                                                                 int64_t row_stride, int row_bytes)
+{
+    const int64_t n_rows = actual_count(n_rows_max, d_n_rows);
+    const int64_t row = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    unsigned long long todo = __ballot(row < n_rows && indptr[row] == indptr[row + 1]);
+    const int64_t first = row - lane_id();
+    while (todo != 0) {
+        const int64_t r = first + __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        uint16_t* p = reinterpret_cast<uint16_t*>(x + r * row_stride);
+        for (int i = lane_id(); i < row_bytes / 2; i += kWave) p[i] = 0;
+    }
+}
+
 // bf16 rows can be moved eight elements at a time when every row starts on a 4-byte boundary
 static bool bf16_rows_dword_aligned(int64_t ldx, int64_t ldo, const void* x, const void* out)
 {
@@ -1462,11 +1474,16 @@ FGL_EXPORT int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices, 
     FGL_REQUIRE(D >= 1, "aggregate: feature length %d < 1", D);
     FGL_REQUIRE(ldx >= D && ldo >= D, "aggregate: row stride smaller than the row length");
     FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "aggregate: unknown dtype %d", dtype);
-    FGL_REQUIRE(mode >= FGL_AGG_SUM && mode <= FGL_AGG_COLMEAN_PTR, "aggregate: unknown mode %d", mode);
-    const int col_norm_is_ptr = mode == FGL_AGG_COLMEAN_PTR;
-    if (col_norm_is_ptr) mode = FGL_AGG_COLMEAN;
+    FGL_REQUIRE(mode >= FGL_AGG_SUM && mode <= FGL_AGG_GCN_OWN_PTR, "aggregate: unknown mode %d", mode);
+    const int col_norm_is_ptr = mode == FGL_AGG_COLMEAN_PTR || mode == FGL_AGG_GCN_OWN_PTR;
+    if (mode == FGL_AGG_COLMEAN_PTR) mode = FGL_AGG_COLMEAN;
+    const bool own_degree = mode == FGL_AGG_GCN_OWN || mode == FGL_AGG_GCN_OWN_PTR;
+    if (own_degree) {
+        mode = FGL_AGG_GCN;
+        d_row_norm = nullptr;
+    }
     FGL_REQUIRE(zero_policy == FGL_ZERO_COPY_SELF || zero_policy == FGL_ZERO_ZEROS, "aggregate: unknown zero policy %d", zero_policy);
-    FGL_REQUIRE(mode != FGL_AGG_GCN || (d_row_norm && d_col_norm), "aggregate: gcn mode needs row_norm and col_norm");
+    FGL_REQUIRE(mode != FGL_AGG_GCN || ((d_row_norm || own_degree) && d_col_norm), "aggregate: gcn mode needs row_norm and col_norm");
     FGL_REQUIRE(mode != FGL_AGG_COLMEAN || d_col_norm, "aggregate: colmean mode needs col_norm");
     FGL_REQUIRE(mode != FGL_AGG_EDGE || (d_edge_w && n_heads >= 1 && D % n_heads == 0),
                 "aggregate: edge mode needs edge weights and a head count that divides the row length");
@@ -1482,6 +1499,22 @@ FGL_EXPORT int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices, 
     if (dtype == FGL_F32) return launch_agg_vec<float, 4>(mode, longest_row_max, n_entries_max, s, g);
     if (bf16_rows_dword_aligned(ldx, ldo, d_x, d_out)) return launch_agg_vec<uint16_t, 8>(mode, longest_row_max, n_entries_max, s, g);
     return launch_agg_vec<uint16_t, 1>(mode, longest_row_max, n_entries_max, s, g);
+}
+
+FGL_EXPORT int fgl_zero_empty_rows(const int32_t* d_indptr, int64_t n_rows_max, const int32_t* d_n_rows, void* d_x, int64_t ldx, int D,
+                                   int dtype, void* stream)
+{
+    FGL_REQUIRE(n_rows_max >= 0 && D >= 1 && ldx >= D, "zero_empty_rows: bad sizes");
+    FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "zero_empty_rows: unknown dtype %d", dtype);
+    if (n_rows_max == 0) return FGL_OK;
+    FGL_REQUIRE(d_indptr && d_x, "zero_empty_rows: null pointer");
+    const int64_t blocks = ceil_div(n_rows_max, kBlock);
+    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "zero_empty_rows: too many rows");
+    const int size = dtype == FGL_F32 ? 4 : 2;
+    hipLaunchKernelGGL(zero_empty_rows_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, as_stream(stream), d_indptr, n_rows_max, d_n_rows,
+                       static_cast<char*>(d_x), ldx * size, D * size);
+    FGL_CHECK_LAUNCH("zero_empty_rows_kernel");
+    return FGL_OK;
 }
 
 FGL_EXPORT const char* fgl_aggregate_last_mapping(void) { return g_mapping; }

@@ -17,7 +17,7 @@ CSRC_DIR = os.path.normpath(os.path.join(_PKG_DIR, "..", "csrc"))
 
 # enum values of include/fastgl_hip.h
 F32, BF16 = 0, 1
-AGG_SUM, AGG_MEAN, AGG_GCN, AGG_COLMEAN, AGG_EDGE, AGG_COLMEAN_PTR = 0, 1, 2, 3, 4, 5
+AGG_SUM, AGG_MEAN, AGG_GCN, AGG_COLMEAN, AGG_EDGE, AGG_COLMEAN_PTR, AGG_GCN_OWN, AGG_GCN_OWN_PTR = 0, 1, 2, 3, 4, 5, 6, 7
 ZERO_COPY_SELF, ZERO_ZEROS = 0, 1
 ABI_VERSION = 11  # FGL_ABI_VERSION of include/fastgl_hip.h that the signatures below follow
 STATUS_TABLE_FULL, STATUS_UNIQ_OVERFLOW, STATUS_MISSING_KEY, STATUS_BAD_SEED, STATUS_BAD_ID = 1, 2, 4, 8, 16
@@ -60,6 +60,7 @@ SIGNATURES = {
     "fgl_block_transpose_batch": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fgl_aggregate": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _i64,
                              _vp, _i64, _vp]),
+    "fgl_zero_empty_rows": (_i32, [_vp, _i64, _vp, _vp, _i64, _i32, _i32, _vp]),
     "fgl_aggregate_last_mapping": (C.c_char_p, []),
     "fgl_edge_softmax": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i32, C.c_float, _vp, _vp]),
     "fgl_weight_grad_workspace_bytes": (_sz, [_i64, _i32, _i32]),

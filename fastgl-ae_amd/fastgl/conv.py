@@ -56,7 +56,26 @@ class MA_Function(torch.autograd.Function):
     for most layers it is cheaper to gather rows of ``X`` and multiply the (fewer) gathered rows --
     ``order="auto"`` (default) prices both and picks; ``"product_first"`` is the reference's order.  Either
     way a destination row without edges passes ``(X W)[d]`` through and sends no gradient back
-    (aggregate_acc_kernel.cu:307-309,498-500)."""
+    (aggregate_acc_kernel.cu:307-309,498-500).
+    ``src_norm_degs`` and ``dst_norm_degs`` may be ``None`` when ``transposed`` is the ``Block`` itself: its degrees are
+    then read from its row pointers, with no arrays made of them (what ``GCN`` does: six launches per layer less)."""
+
+    @staticmethod
+    def _gather(edge_ptr, src_edges, feat, src_norm_degs, dst_norm_degs, n_dst, block, zero_policy, longest_row):
+        if src_norm_degs is not None:
+            mode, row_norm, col_norm = "gcn", dst_norm_degs, src_norm_degs
+        elif block._transposed is not None:
+            mode, row_norm, col_norm = "gcn_own_ptr", None, block._transposed[0]
+        else:
+            mode, row_norm, col_norm = "gcn_own", None, block.out_degrees()
+        return ops.aggregate(edge_ptr, src_edges, feat, mode=mode, zero_policy=zero_policy, row_norm=row_norm, col_norm=col_norm,
+                             n_rows=n_dst, longest_row=longest_row)
+
+    @staticmethod
+    def _gather_back(t_ptr, t_idx, d_out, src_norm_degs, dst_norm_degs, n_src, edge_ptr):
+        if src_norm_degs is not None:
+            return ops.aggregate(t_ptr, t_idx, d_out, mode="gcn", zero_policy="zeros", row_norm=src_norm_degs, col_norm=dst_norm_degs, n_rows=n_src)
+        return ops.aggregate(t_ptr, t_idx, d_out, mode="gcn_own_ptr", zero_policy="zeros", col_norm=edge_ptr, n_rows=n_src)
 
     @staticmethod
     def forward(ctx, edge_ptr, src_edges, src_norm_degs, dst_norm_degs, dst_nodes, input_feat, weight, neighbor_num,
@@ -66,34 +85,34 @@ class MA_Function(torch.autograd.Function):
         gather_first = order == "gather_first" or (order == "auto" and _aggregate_first_is_cheaper(
             input_feat.size(0), n_dst, src_edges.numel(), weight.size(0), weight.size(1)))
         ctx.gather_first = gather_first
+        longest = ops._fanout_bound(edge_ptr, neighbor_num)
         if not gather_first:
             ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, input_feat)
-            return ops.forward_gcn(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, input_feat, weight, neighbor_num,
-                                   dst_nodes)[0]
-        ax = ops.aggregate(edge_ptr, src_edges, input_feat, mode="gcn", zero_policy="self", row_norm=dst_norm_degs,
-                           col_norm=src_norm_degs, n_rows=n_dst, longest_row=ops._fanout_bound(edge_ptr, neighbor_num))
+            return MA_Function._gather(edge_ptr, src_edges, torch.mm(input_feat, weight), src_norm_degs, dst_norm_degs, n_dst, transposed,
+                                       "self", longest)
+        ax = MA_Function._gather(edge_ptr, src_edges, input_feat, src_norm_degs, dst_norm_degs, n_dst, transposed, "self", longest)
         ctx.n_src = int(input_feat.size(0))
-        ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax)
-        return torch.mm(ax, weight)
+        out = torch.mm(ax, weight)
+        if any(ctx.needs_input_grad):
+            # what the weight gradient wants of the gathered rows: rows without edges send no gradient back
+            ops.zero_empty_rows_(edge_ptr, ax, n_dst)
+            ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax)
+        return out
 
     @staticmethod
     def backward(ctx, d_input):
         d_input = d_input.contiguous()
         if ctx.gather_first:
             edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax = ctx.saved_tensors
-            # rows without edges took no part in the sum: no gradient through them (as in the reference)
-            has_edges = (edge_ptr[1:] != edge_ptr[:-1]).to(d_input.dtype)[:, None]
-            d_out = d_input * has_edges
-            d_w = ops.weight_grad(ax, d_out)
+            d_w = ops.weight_grad(ax, d_input)
             d_x = None
             if ctx.needs_input_grad[5]:
-                d_ax = torch.mm(d_out, weight.transpose(0, 1))
+                d_ax = torch.mm(d_input, weight.transpose(0, 1))  # (rows without edges are in no source's list)
                 if ctx.transposed is None:
                     t_ptr, t_idx = ops.block_transpose(edge_ptr, src_edges, int(d_input.size(0)), ctx.n_src)
                 else:
                     t_ptr, t_idx = _transposed(ctx.transposed)
-                d_x = ops.aggregate(t_ptr, t_idx, d_ax, mode="gcn", zero_policy="zeros", row_norm=src_norm_degs,
-                                    col_norm=dst_norm_degs, n_rows=ctx.n_src)
+                d_x = MA_Function._gather_back(t_ptr, t_idx, d_ax, src_norm_degs, dst_norm_degs, ctx.n_src, edge_ptr)
             return None, None, None, None, None, d_x, d_w, None, None, None
         edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, input_feat = ctx.saved_tensors
         if ctx.transposed is None:
@@ -102,13 +121,12 @@ class MA_Function(torch.autograd.Function):
             # the first layer: nobody wants d_x, and d_w = X^T (A^T d_out) = (A X)^T d_out needs no transposed
             # block -- one more forward-direction gather (rows without edges contribute nothing, as in the
             # reference's backward kernel, aggregate_acc_kernel.cu:498-500)
-            ax = ops.aggregate(edge_ptr, src_edges, input_feat, mode="gcn", zero_policy="zeros", row_norm=dst_norm_degs,
-                               col_norm=src_norm_degs, n_rows=int(d_input.size(0)))
+            ax = MA_Function._gather(edge_ptr, src_edges, input_feat, src_norm_degs, dst_norm_degs, int(d_input.size(0)), ctx.transposed,
+                                     "zeros", None)
             d_x, d_w = None, ops.weight_grad(ax, d_input)
         else:  # same arithmetic as backward_gcn, with the block's cached transpose
             t_ptr, t_idx = _transposed(ctx.transposed)
-            g = ops.aggregate(t_ptr, t_idx, d_input, mode="gcn", zero_policy="zeros", row_norm=src_norm_degs,
-                              col_norm=dst_norm_degs, n_rows=int(input_feat.size(0)))
+            g = MA_Function._gather_back(t_ptr, t_idx, d_input, src_norm_degs, dst_norm_degs, int(input_feat.size(0)), edge_ptr)
             d_x = torch.mm(g, weight.transpose(0, 1))
             d_w = ops.weight_grad(input_feat, g)
         return None, None, None, None, None, d_x, d_w, None, None, None
@@ -165,14 +183,14 @@ class GCN(nn.Module):
                 h = self.dropout(h)
             graph = blocks[i]
             dst_nodes = graph.num_dst_nodes()
-            edge_ptr, src_edges, raw_dst_norm_degs = _block_csr(graph)
             if isinstance(graph, Block):
-                src_norm_degs = graph.out_degrees().clamp(min=1)
-                transposed = graph if torch.is_grad_enabled() else None  # transposed on demand, in backward
+                edge_ptr, src_edges, transposed = graph.edge_ptr, graph.src_local, graph  # (degrees from its row pointers)
+                src_norm_degs = dst_norm_degs = None
             else:
+                edge_ptr, src_edges, raw_dst_norm_degs = _block_csr(graph)
                 src_norm_degs = ops.cal_deg(src_edges, graph.num_src_nodes()).clamp(min=1)
+                dst_norm_degs = raw_dst_norm_degs.clamp(min=1)
                 transposed = None
-            dst_norm_degs = raw_dst_norm_degs.clamp(min=1)
             h = layer(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, dst_nodes, h, neighbor_list[i], transposed)
         return h
 
@@ -221,7 +239,7 @@ class GIN(nn.Module):
                 h = self.dropout(h)
             graph = blocks[i]
             dst_nodes = graph.num_dst_nodes()
-            edge_ptr, src_edges, _ = _block_csr(graph)
+            edge_ptr, src_edges = (graph.edge_ptr, graph.src_local) if isinstance(graph, Block) else _block_csr(graph)[:2]
             transposed = graph if isinstance(graph, Block) and torch.is_grad_enabled() else None
             h = layer(edge_ptr, src_edges, dst_nodes, h, neighbor_list[i], transposed)
         return h
@@ -337,7 +355,7 @@ class GATConv(nn.Module):
         feat_dst = feat_src[:dst_nodes]
         el = (feat_src * self.attn_l).sum(dim=-1)  # [n_src, H]
         er = (feat_dst * self.attn_r).sum(dim=-1)  # [n_dst, H]
-        edge_ptr, src_edges, _ = _block_csr(graph)
+        edge_ptr, src_edges = (graph.edge_ptr, graph.src_local) if isinstance(graph, Block) else _block_csr(graph)[:2]
         # u_add_v + leaky_relu + edge_softmax (DGL calls in the reference, GraphConv.py:265-272) in one launch.
         # No gradient reaches the coefficients (the aggregation's backward returns none for them, as in the
         # reference, GraphConv.py:227), so they are computed outside the autograd graph.

@@ -347,6 +347,7 @@ def weight_grad(a, b, column_sums=False):
     gradient of the output the transposed weight gradient and the bias gradient of the layer."""
     k, m, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
     if not (a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
+            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and  # (a graph is being built: torch's product has a gradient)
             a.stride(1) == 1 and b.stride(1) == 1 and m <= a.stride(0) < 1 << 24 and n <= b.stride(0) < 1 << 24 and
             m < 1 << 16 and n < 1 << 16 and b.size(0) == k and
             _splits_k(k, m, n)):
@@ -365,7 +366,7 @@ def weight_grad(a, b, column_sums=False):
 
 
 _MODES = {"sum": L.AGG_SUM, "mean": L.AGG_MEAN, "gcn": L.AGG_GCN, "colmean": L.AGG_COLMEAN, "edge": L.AGG_EDGE,
-          "colmean_ptr": L.AGG_COLMEAN_PTR}
+          "colmean_ptr": L.AGG_COLMEAN_PTR, "gcn_own": L.AGG_GCN_OWN, "gcn_own_ptr": L.AGG_GCN_OWN_PTR}
 _ZERO = {"self": L.ZERO_COPY_SELF, "zeros": L.ZERO_ZEROS}
 
 
@@ -373,7 +374,8 @@ def aggregate(indptr, indices, feat, mode="sum", zero_policy="self", row_norm=No
               out=None, edge_weight=None, n_heads=1, edge_index=None, longest_row=None, n_rows_dev=None, mapping="auto"):
     """``out[r] = sum_e w(r, indices[e]) * feat[indices[e]]`` over the CSR rows (fp32
     accumulation; fp32 or bf16 storage).  ``mode``: sum | mean | gcn | colmean | edge | colmean_ptr (colmean with
-    ``col_norm`` holding the offsets array whose differences are the counts: a block's ``edge_ptr``);
+    ``col_norm`` holding the offsets array whose differences are the counts: a block's ``edge_ptr``) | gcn_own,
+    gcn_own_ptr (gcn with the rows' own entry counts as ``row_norm``, and ``col_norm`` as counts or as offsets);
     ``zero_policy``: what a row without entries gets -- ``self`` (``feat[r]``) or ``zeros``.
     ``longest_row``: what is known about the longest row's entry count -- an ``int`` bound (the fanout of a
     sampled block) or a one-element int32 device tensor (as ``block_transpose`` makes).  Speed only: hub rows
@@ -448,6 +450,14 @@ def aggregate(indptr, indices, feat, mode="sum", zero_policy="self", row_norm=No
                                           int(indices.numel()) if mapping == "auto" else -1, L.ptr(out),
                                           int(out.stride(0)), L.stream_handle()))
     return out
+
+
+def zero_empty_rows_(indptr, x, n_rows):
+    """Rows of ``x`` [n_rows, D] that have no entries in the CSR become zeros, in place."""
+    with _on_device(x.device):
+        L.check(L.lib().fgl_zero_empty_rows(L.ptr(indptr), int(n_rows), None, L.ptr(x), int(x.stride(0)), int(x.size(1)),
+                                            L.F32 if x.dtype == torch.float32 else L.BF16, L.stream_handle()))
+    return x
 
 
 def edge_softmax(indptr, indices, el, er, negative_slope=0.2, n_rows=None):

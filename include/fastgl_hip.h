@@ -51,9 +51,12 @@ enum fgl_agg_mode {
     FGL_AGG_GCN = 2,     /* w = (1/sqrt(row_norm[row])) * (1/sqrt(col_norm[col]))    */
     FGL_AGG_COLMEAN = 3, /* w = 1 / max(col_norm[col], 1)   (backward of MEAN)        */
     FGL_AGG_EDGE = 4,    /* w = edge_w[entry_id * n_heads + column / (D / n_heads)]  (GAT) */
-    FGL_AGG_COLMEAN_PTR = 5 /* FGL_AGG_COLMEAN with the columns' entry counts given as an offsets array:
+    FGL_AGG_COLMEAN_PTR = 5, /* FGL_AGG_COLMEAN with the columns' entry counts given as an offsets array:
                                col_norm[col+1] - col_norm[col] -- the row pointer of the block whose transpose is
                                being gathered, so the backward of MEAN needs no degree array */
+    FGL_AGG_GCN_OWN = 6,     /* FGL_AGG_GCN with the row's own entry count as its degree (row_norm unused) ... */
+    FGL_AGG_GCN_OWN_PTR = 7  /* ... and the columns' degrees given as an offsets array, as in FGL_AGG_COLMEAN_PTR: a block and
+                                its transpose carry every degree that a GCN layer needs in their row pointers */
 };
 
 /* what an output row with no entries gets */
@@ -364,6 +367,12 @@ int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices,
                   const float* d_edge_w, int n_heads, const int32_t* d_edge_index,
                   int64_t longest_row_max, const int32_t* d_longest_row, int64_t n_entries_max,
                   void* d_out, int64_t ldo, void* stream);
+/* Rows of x (n_rows rows of D elements of `dtype`, row stride ldx) that have no entries become zeros: what the weight
+ * gradient of a layer that passes such rows through in its forward pass wants of the gathered rows it has kept (rows
+ * without edges send no gradient back, aggregate_acc_kernel.cu:498-500). */
+int fgl_zero_empty_rows(const int32_t* d_indptr, int64_t n_rows_max, const int32_t* d_n_rows, void* d_x, int64_t ldx, int D,
+                        int dtype, void* stream);
+
 /* Which kernel and lane mapping the calling thread's last fgl_aggregate call launched, as text ("aggregate_kernel
  * lanes/row=32", "aggregate_bundle_kernel lanes/row=64 (rows bundled by 4) + long_rows", ...): for benchmark
  * records and bug reports.  No counterpart in the reference, whose kernels have one fixed mapping
