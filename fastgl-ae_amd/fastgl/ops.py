@@ -460,6 +460,27 @@ def zero_empty_rows_(indptr, x, n_rows):
     return x
 
 
+def head_scores(feat, attn_l, attn_r, n_dst):
+    """``(el, er)`` of a GAT layer: ``el[i, h] = sum_f feat[i, h * F + f] * attn_l[h, f]`` for all rows and ``er`` with
+    ``attn_r`` for the first ``n_dst`` rows, in one pass over ``feat`` (float32 [n, H * F]; attn_*: float32 [.., H, F]).
+    No gradients."""
+    _check_input(feat, "feat", (torch.float32,))
+    _check_input(attn_l, "attn_l", (torch.float32,))
+    _check_input(attn_r, "attn_r", (torch.float32,))
+    H, F = int(attn_l.size(-2)), int(attn_l.size(-1))
+    n, n_dst = int(feat.size(0)), int(n_dst)
+    if feat.dim() != 2 or feat.size(1) != H * F or attn_l.numel() != H * F or attn_r.numel() != H * F or not 0 <= n_dst <= n:
+        raise RuntimeError("feat %s does not match the attention vectors %s, %s and %d rows" % (
+            tuple(feat.shape), tuple(attn_l.shape), tuple(attn_r.shape), n_dst))
+    dev = _same_device(feat, attn_l, attn_r)
+    with _on_device(dev):
+        scores = torch.empty((n + n_dst, H), dtype=torch.float32, device=dev)
+        el, er = scores[:n], scores[n:]
+        if n > 0 and H * F > 0:
+            L.check(L.lib().fgl_head_scores(L.ptr(feat), H * F, n, n_dst, H, F, L.ptr(attn_l), L.ptr(attn_r), L.ptr(el), L.ptr(er), L.stream_handle()))
+    return el, er
+
+
 def edge_softmax(indptr, indices, el, er, negative_slope=0.2, n_rows=None):
     """Attention coefficients of a GAT layer over a block CSR, ``float32 [n_entries, n_heads]``:
     ``softmax`` over the entries of each row of ``leaky_relu(el[indices[e]] + er[row])`` -- the reference's

@@ -392,6 +392,12 @@ int fgl_edge_softmax(const int32_t* d_indptr, const int32_t* d_indices, int64_t 
                      const int32_t* d_n_rows, const float* d_el, const float* d_er, int n_heads,
                      float negative_slope, float* d_alpha, void* stream);
 
+/* The two halves of those scores: d_el[i, h] = sum_f x[i, h, f] * attn_l[h, f] for n_rows rows of x (float, n_heads * width
+ * columns, row stride ldx) and d_er[i, h] with attn_r for the first n_er of them (the feat * attn sums of the reference's
+ * GATConv.forward, GraphConv.py:259-264). */
+int fgl_head_scores(const float* d_x, int64_t ldx, int64_t n_rows, int64_t n_er, int n_heads, int width, const float* d_attn_l,
+                    const float* d_attn_r, float* d_el, float* d_er, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * Weight gradient of a dense layer: C[i, j] = sum over r < k of A[r, i] * B[r, j] -- the d_w = X^T G of backward_gcn /
  * backward_gin (aggregate_acc.cpp:371-374,402-405, torch::mm on a transposed view there).  A: [k, m] with row stride
