@@ -164,12 +164,15 @@ torch::Tensor aggregate(const torch::Tensor& indptr, const torch::Tensor& indice
     auto out = torch::empty({n_rows, D}, feat.options());
     if (n_rows == 0) return out;
     const void* idx = indices.numel() ? indices.data_ptr() : indptr.data_ptr();  // a block without entries: never read
-    ok(fgl_aggregate(indptr.data_ptr<int32_t>(), static_cast<const int32_t*>(idx), n_rows, nullptr, feat.data_ptr(), feat.stride(0),
-                     (int)D, dtype_of(feat), mode, zero_policy, row_norm ? row_norm->data_ptr<int32_t>() : nullptr,
-                     col_norm ? col_norm->data_ptr<int32_t>() : nullptr, edge_w ? edge_w->data_ptr<float>() : nullptr, n_heads,
-                     edge_index ? edge_index->data_ptr<int32_t>() : nullptr, longest_row,
-                     longest_dev ? longest_dev->data_ptr<int32_t>() : nullptr, indices.numel(), out.data_ptr(), out.stride(0),
-                     stream_of(feat)));
+    const size_t ws_bytes = fgl_aggregate_workspace_bytes(indices.numel(), (int)D, mode, longest_row);
+    torch::Tensor ws;
+    if (ws_bytes > 0) ws = torch::empty({(int64_t)ws_bytes}, feat.options().dtype(torch::kUInt8));
+    ok(fgl_aggregate_ws(indptr.data_ptr<int32_t>(), static_cast<const int32_t*>(idx), n_rows, nullptr, feat.data_ptr(), feat.stride(0),
+                        (int)D, dtype_of(feat), mode, zero_policy, row_norm ? row_norm->data_ptr<int32_t>() : nullptr,
+                        col_norm ? col_norm->data_ptr<int32_t>() : nullptr, edge_w ? edge_w->data_ptr<float>() : nullptr, n_heads,
+                        edge_index ? edge_index->data_ptr<int32_t>() : nullptr, longest_row,
+                        longest_dev ? longest_dev->data_ptr<int32_t>() : nullptr, indices.numel(), out.data_ptr(), out.stride(0),
+                        ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(feat)));
     return out;
 }
 

@@ -145,6 +145,8 @@ struct AggArgs {
     int n_heads;
     int unit_dim;               // D / n_heads
     int col_norm_is_ptr;        // col_norm is an offsets array, the counts are its differences
+    void* ws;                   // scratch of aggregate_workspace_bytes(n_entries_max, D) bytes: long rows go in segments (NULL: row by row)
+    int64_t n_entries_max;      // (with ws) no fewer entries than the rows hold
 };
 
 // per-edge weight, evaluated by the lane that loaded the neighbour id
@@ -1078,6 +1080,232 @@ __global__ __launch_bounds__(kLongBlock) void aggregate_long_rows_kernel(const A
     }
 }
 
+// ---- long rows of large inputs, in segments -------------------------------------------
+// aggregate_long_rows_kernel gives a row to one workgroup: over a whole graph the workgroups' shares differ (2.4 M nodes, 54 M
+// entries, three quarters of them in rows longer than kLongRowEntries: 110 K entries in the fullest share, 40 K on average), and a
+// row of 129 entries keeps 9 of its 32 lane groups busy.  Here a row is cut into segments of at most kSegEntries entries, a wave
+// takes one -- few enough entries that the hardware's own scheduling of workgroups evens out what the rows' lengths do
+// not -- and the sums of a row of several segments are added in the segments' order by a second launch.
+// Measured (that graph, 64 fp32 columns, gcn weights, MI355X): 54 M entries 3403 -> 3137 us
+// in all (4.4 TB/s of gathered rows, the memory's bound; 100 columns 5154 -> 4307); 100 K nodes, 2.5 M entries: 274 -> 117 us.
+constexpr int kSegEntries = 512;
+struct SegLists {
+    int32_t* counts;    // [0] segments of rows of several, [1] rows of one segment, [2] rows of several segments
+    int32_t* seg_row;   // segments of rows of several: the row ...
+    int32_t* seg_first; // ... and the first entry; the segment's number is its partial sum's place
+    int32_t* one_row;   // rows of one segment
+    int32_t* many_row;  // rows of several segments: the row ...
+    int32_t* many_seg;  // ... and its first segment's number (a row's segments are neighbours)
+    float* partial;     // [seg][ldp]
+    int ldp;
+    int32_t cap_seg, cap_one, cap_many;
+};
+
+// A row of n > kSegEntries entries has at most 2 n / kSegEntries segments.
+static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, size_t* bytes)
+{
+    SegLists l;
+    l.cap_seg = (int32_t)(2 * n_entries_max / kSegEntries + 1);
+    l.cap_one = (int32_t)(n_entries_max / kLongRowEntries + 1);
+    l.cap_many = (int32_t)(n_entries_max / kSegEntries + 1);
+    l.ldp = (D + 7) / 8 * 8;
+    Carver c(ws);
+    l.counts = c.take<int32_t>(3);
+    l.seg_row = c.take<int32_t>((size_t)l.cap_seg);
+    l.seg_first = c.take<int32_t>((size_t)l.cap_seg);
+    l.one_row = c.take<int32_t>((size_t)l.cap_one);
+    l.many_row = c.take<int32_t>((size_t)l.cap_many);
+    l.many_seg = c.take<int32_t>((size_t)l.cap_many);
+    l.partial = c.take<float>((size_t)l.cap_seg * (size_t)l.ldp);
+    if (bytes) *bytes = c.used();
+    return l;
+}
+
+__global__ void seg_init_kernel(int32_t* __restrict__ counts)
+{
+    if (threadIdx.x < 3) counts[threadIdx.x] = 0;
+}
+
+// The lists.  Their order is up to scheduling, the sums are not: a row's segments are cut and added the same way on every run.
+// A workgroup looks through kSegRows rows per lane and takes its places in the lists with three atomics (one address each:
+// their updates run one after the other, so there are few of them).
+constexpr int kSegBlock = 1024, kSegRows = 8;
+__global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, const SegLists l)
+{
+    __shared__ int s_scan[kSegBlock / kWave + 1];
+    __shared__ int s_base[3];
+    const int threshold = g.skip_rows_longer_than;
+    if (g.longest_row != nullptr && *g.longest_row <= threshold) return;
+    const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
+    const int64_t row0 = (int64_t)blockIdx.x * kSegBlock * kSegRows + threadIdx.x;
+    int first[kSegRows], entries[kSegRows];
+    int segs = 0, ones = 0, many = 0;
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i) {
+        const int64_t row = row0 + (int64_t)i * kSegBlock;
+        first[i] = row < n_rows ? g.indptr[row] : 0;
+        entries[i] = row < n_rows ? g.indptr[row + 1] - first[i] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i) {
+        if (entries[i] <= threshold) continue;
+        if (entries[i] <= kSegEntries) {
+            ++ones;
+        } else {
+            ++many;
+            segs += (entries[i] + kSegEntries - 1) / kSegEntries;
+        }
+    }
+    int total_segs, total_ones, total_many;
+    int at_seg = block_exclusive_scan<kSegBlock>(segs, s_scan, &total_segs);
+    int at_one = block_exclusive_scan<kSegBlock>(ones, s_scan, &total_ones);
+    int at_many = block_exclusive_scan<kSegBlock>(many, s_scan, &total_many);
+    if (threadIdx.x < 3) {
+        const int total = threadIdx.x == 0 ? total_segs : threadIdx.x == 1 ? total_ones : total_many;
+        s_base[threadIdx.x] = total > 0 ? atomicAdd(&l.counts[threadIdx.x], total) : 0;
+    }
+    __syncthreads();
+    at_seg += s_base[0];
+    at_one += s_base[1];
+    at_many += s_base[2];
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i) {
+        if (entries[i] <= threshold) continue;
+        const int row = (int)(row0 + (int64_t)i * kSegBlock);
+        if (entries[i] <= kSegEntries) {
+            if (at_one < l.cap_one) l.one_row[at_one] = row;
+            ++at_one;
+            continue;
+        }
+        if (at_many < l.cap_many) {
+            l.many_row[at_many] = row;
+            l.many_seg[at_many] = at_seg;
+        }
+        ++at_many;
+        for (int e = 0; e < entries[i]; e += kSegEntries, ++at_seg) {
+            if (at_seg >= l.cap_seg) continue;
+            l.seg_row[at_seg] = row;
+            l.seg_first[at_seg] = first[i] + e;
+        }
+    }
+}
+
+// One wave, one segment: its lane groups take every fourth (LPR = 16) chunk of LPR entries, the next chunk's ids under way while the
+// current one's rows are gathered; the groups' sums are added by a __shfl_xor tree.
+template <typename T, int VEC, int LPR, int MODE>
+__global__ __launch_bounds__(kBlock) void aggregate_segments_kernel(const AggArgs g, const SegLists l)
+{
+    using IO = RowIO<T, VEC>;
+    typedef float Vec __attribute__((ext_vector_type(VEC), aligned(4)));
+    constexpr int kInFlight = LPR < 16 ? LPR : 16;
+    const int n_seg = l.counts[0] < l.cap_seg ? l.counts[0] : l.cap_seg;
+    const int n_one = l.counts[1] < l.cap_one ? l.counts[1] : l.cap_one;
+    const int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    if (unit >= (int64_t)n_seg + n_one) return;
+    const bool part_of_row = unit < n_seg;
+    const int row = part_of_row ? l.seg_row[unit] : l.one_row[unit - n_seg];
+    const int row_a = g.indptr[row], row_b = g.indptr[row + 1];
+    const int a = part_of_row ? l.seg_first[unit] : row_a;
+    const int b = row_b - a > kSegEntries ? a + kSegEntries : row_b;
+    const float row_factor = row_weight<MODE>(g.row_norm, row, row_b - row_a);
+
+    const int32_t* __restrict__ indices = g.indices;
+    const T* __restrict__ X = static_cast<const T*>(g.x);
+    const int64_t ldx = g.ldx;
+    const int lane = lane_id();
+    const int gl = lane % LPR, grp = lane / LPR;
+    const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, gl, g.D);
+    const int col0 = ls.col0;
+    const bool all_full = all_lanes_full<T, VEC>(g.D);
+    float acc[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
+    int next_col = a + lane < b ? indices[a + lane] : 0;  // (the wave's groups take neighbouring chunks: lane i, entry i)
+    for (int wave_base = a; wave_base < b; wave_base += kWave) {
+        const int base = wave_base + grp * LPR;
+        const int cnt = b - base < LPR ? b - base : LPR;  // (may be <= 0: this group has no chunk in the last pass)
+        const int my_col = next_col;
+        const float my_w = gl < cnt ? edge_weight<MODE>(my_col, row_factor, g.col_norm, g.col_norm_is_ptr) : 0.0f;
+        const int ahead = wave_base + kWave + lane;
+        next_col = ahead < b ? indices[ahead] : 0;
+        float part[VEC];  // two-level summation, as in gather_row
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) part[k] = 0.0f;
+        for (int t = 0; t < cnt; t += kInFlight) {
+            int c[kInFlight];
+            float w[kInFlight];
+            typename IO::Raw x[kInFlight];
+#pragma unroll
+            for (int j = 0; j < kInFlight; ++j) {
+                const int src = t + j < cnt ? t + j : t;  // lanes past the end repeat entry t and are not added
+                c[j] = __shfl(my_col, src, LPR);
+                w[j] = __shfl(my_w, src, LPR);
+            }
+            if (ls.live) {
+                if (all_full) {
+#pragma unroll
+                    for (int j = 0; j < kInFlight; ++j) x[j] = IO::load(X + (int64_t)c[j] * ldx + col0);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < kInFlight; ++j) x[j] = ls.load(X + (int64_t)c[j] * ldx + col0);
+                }
+#pragma unroll
+                for (int j = 0; j < kInFlight; ++j)
+                    if (t + j < cnt) IO::fma(part, w[j], x[j]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[k] += part[k];
+    }
+#pragma unroll
+    for (int d = LPR; d < kWave; d <<= 1)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[k] += __shfl_xor(acc[k], d, kWave);
+    if (grp != 0 || !ls.live) return;
+    if (!part_of_row) {
+        ls.store(static_cast<T*>(g.out) + (int64_t)row * g.ldo + col0, acc);
+        return;
+    }
+    Vec v;  // (whole vectors also where the row ends inside one: ldp is padded)
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) v[k] = acc[k];
+    *reinterpret_cast<Vec*>(l.partial + unit * l.ldp + col0) = v;
+}
+
+// The rows of several segments: a lane group adds a row's partial sums in order.
+template <typename T, int VEC, int LPR>
+__global__ __launch_bounds__(kBlock) void seg_reduce_kernel(const AggArgs g, const SegLists l)
+{
+    typedef float Vec __attribute__((ext_vector_type(VEC), aligned(4)));
+    const int n_many = l.counts[2] < l.cap_many ? l.counts[2] : l.cap_many;
+    const int64_t i = (int64_t)blockIdx.x * (kBlock / LPR) + threadIdx.x / LPR;
+    if (i >= n_many) return;
+    const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, (int)threadIdx.x % LPR, g.D);
+    if (!ls.live) return;
+    const int64_t row = l.many_row[i];
+    const int n = (g.indptr[row + 1] - g.indptr[row] + kSegEntries - 1) / kSegEntries;
+    int64_t seg = l.many_seg[i];
+    const int64_t end = seg + n < l.cap_seg ? seg + n : l.cap_seg;
+    float acc[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
+    auto add = [&](const Vec& v) {
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[k] += v[k];
+    };
+    const float* p = l.partial + ls.col0;
+    for (; seg + 8 <= end; seg += 8) {
+        Vec v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const Vec*>(p + (seg + j) * l.ldp);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) add(v[j]);
+    }
+    for (; seg < end; ++seg) add(*reinterpret_cast<const Vec*>(p + seg * l.ldp));
+    ls.store(static_cast<T*>(g.out) + row * g.ldo + ls.col0, acc);
+}
+
+
 // ---- block transpose ---------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void transpose_count_kernel(const int32_t* __restrict__ indptr,
                                                                  const int32_t* __restrict__ indices, int64_t n_rows_max,
@@ -1221,6 +1449,29 @@ static void note_mapping(const char* kernel, int lpr, int extra, bool second_pas
 constexpr int kLongRowBlocks = 1021;  // a prime: rows are dealt round robin, and ids that agree in their low bits are
                                        // alike in synthetic (R-MAT) graphs -- a power of two would hand all hubs to a few workgroups
 
+// The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
+// for large inputs), else a workgroup per row.
+template <typename T, int VEC, int LPR, int MODE>
+static void launch_long_rows(unsigned gy, hipStream_t stream, const AggArgs& g)
+{
+    if constexpr (MODE != FGL_AGG_EDGE) {
+        if (g.ws != nullptr) {
+            const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
+            hipLaunchKernelGGL(seg_init_kernel, dim3(1), dim3(kWave), 0, stream, l.counts);
+            hipLaunchKernelGGL(seg_lists_kernel, dim3((unsigned)ceil_div(g.n_rows_max, kSegBlock * kSegRows)), dim3(kSegBlock), 0, stream, g, l);
+            // (a unit has more than kLongRowEntries entries, or is one of at most two per kSegEntries > 2 * kLongRowEntries of them)
+            static_assert(kSegEntries > 2 * kLongRowEntries, "the bound on the number of units");
+            hipLaunchKernelGGL((aggregate_segments_kernel<T, VEC, LPR, MODE>), dim3((unsigned)ceil_div(l.cap_one, kBlock / kWave), gy),
+                               dim3(kBlock), 0, stream, g, l);
+            hipLaunchKernelGGL((seg_reduce_kernel<T, VEC, LPR>), dim3((unsigned)ceil_div(l.cap_many, kBlock / LPR), gy), dim3(kBlock), 0, stream, g, l);
+            return;
+        }
+    }
+    int64_t blocks = ceil_div(g.n_rows_max, kLongBlock);
+    if (blocks > kLongRowBlocks) blocks = kLongRowBlocks;
+    hipLaunchKernelGGL((aggregate_long_rows_kernel<T, VEC, LPR, MODE>), dim3((unsigned)blocks, gy), dim3(kLongBlock), 0, stream, g);
+}
+
 template <typename T, int VEC, int LPR>
 static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStream_t stream, AggArgs g)
 {
@@ -1246,12 +1497,7 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
 #define FGL_LAUNCH_MODE(M)                                                                                         \
     do {                                                                                                           \
         hipLaunchKernelGGL((aggregate_kernel<T, VEC, LPR, M>), grid, dim3(kBlock), 0, stream, g);                  \
-        if (second_pass) {                                                                                         \
-            int64_t blocks = ceil_div(g.n_rows_max, kLongBlock);                                                   \
-            if (blocks > kLongRowBlocks) blocks = kLongRowBlocks;                                                  \
-            hipLaunchKernelGGL((aggregate_long_rows_kernel<T, VEC, LPR, M>), dim3((unsigned)blocks, grid.y),       \
-                               dim3(kLongBlock), 0, stream, g);                                                    \
-        }                                                                                                          \
+        if (second_pass) launch_long_rows<T, VEC, LPR, M>(grid.y, stream, g);                                      \
     } while (0)
     switch (mode) {
         case FGL_AGG_SUM: FGL_LAUNCH_MODE(FGL_AGG_SUM); break;
@@ -1284,12 +1530,7 @@ static int launch_agg_flat(int mode, bool long_rows_possible, int lanes, bool bu
         else                                                                                                        \
             hipLaunchKernelGGL((aggregate_flat_kernel<T, VEC, M>), dim3((unsigned)blocks), dim3(kBlock), 0, stream,  \
                                g, lanes);                                                                           \
-        if (long_rows_possible) {                                                                                   \
-            int64_t lb = ceil_div(g.n_rows_max, kLongBlock);                                                        \
-            if (lb > kLongRowBlocks) lb = kLongRowBlocks;                                                           \
-            hipLaunchKernelGGL((aggregate_long_rows_kernel<T, VEC, 64, M>),                                          \
-                               dim3((unsigned)lb, (unsigned)ceil_div(lanes, 64)), dim3(kLongBlock), 0, stream, g);   \
-        }                                                                                                           \
+        if (long_rows_possible) launch_long_rows<T, VEC, 64, M>((unsigned)ceil_div(lanes, 64), stream, g);           \
     } while (0)
     switch (mode) {
         case FGL_AGG_SUM: FGL_LAUNCH_FLAT(FGL_AGG_SUM); break;
@@ -1342,12 +1583,7 @@ static int launch_agg_bundle(int mode, bool long_rows_possible, unsigned gy, hip
 #define FGL_LAUNCH_BUNDLE(M)                                                                                          \
     do {                                                                                                              \
         hipLaunchKernelGGL((aggregate_bundle_kernel<T, VEC, LPR, M>), dim3((unsigned)gx, gy), dim3(kBlock), 0, stream, g); \
-        if (long_rows_possible) {                                                                                     \
-            int64_t lb = ceil_div(g.n_rows_max, kLongBlock);                                                          \
-            if (lb > kLongRowBlocks) lb = kLongRowBlocks;                                                             \
-            hipLaunchKernelGGL((aggregate_long_rows_kernel<T, VEC, LPR, M>), dim3((unsigned)lb, gy), dim3(kLongBlock), \
-                               0, stream, g);                                                                         \
-        }                                                                                                             \
+        if (long_rows_possible) launch_long_rows<T, VEC, LPR, M>(gy, stream, g);                                      \
     } while (0)
     FGL_FOR_ANY_MODE(mode, FGL_LAUNCH_BUNDLE)
 #undef FGL_LAUNCH_BUNDLE
@@ -1470,6 +1706,32 @@ FGL_EXPORT int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices, 
                              int64_t longest_row_max, const int32_t* d_longest_row, int64_t n_entries_max,
                              void* d_out, int64_t ldo, void* stream)
 {
+    return fgl_aggregate_ws(d_indptr, d_indices, n_rows_max, d_n_rows, d_x, ldx, D, dtype, mode, zero_policy, d_row_norm, d_col_norm, d_edge_w,
+                            n_heads, d_edge_index, longest_row_max, d_longest_row, n_entries_max, d_out, ldo, nullptr, 0, stream);
+}
+
+// From this many entries on, long rows are summed in segments.  Graphs with hubs gain at every size measured (64 fp32 columns: 416 K
+// entries 233 -> 50 us, 994 K 177 -> 73, 10 M 773 -> 423); a block without long rows pays three more launches that end at once
+// (about 8 us, where the caller has no bound on the host that rules long rows out), so blocks of a few hundred
+// thousand entries -- a transposed block of a mini-batch, 50 us and more -- keep the one launch.
+constexpr int64_t kSegMinEntries = (int64_t)1 << 19;
+
+FGL_EXPORT size_t fgl_aggregate_workspace_bytes(int64_t n_entries_max, int D, int mode, int64_t longest_row_max)
+{
+    if (n_entries_max < kSegMinEntries || n_entries_max > 0x7FFFFFFF || D < 1 || mode == FGL_AGG_EDGE) return 0;
+    if (longest_row_max >= 0 && longest_row_max <= kLongRowEntries) return 0;
+    size_t bytes = 0;
+    (void)seg_lists(nullptr, n_entries_max, D, &bytes);
+    return bytes;
+}
+
+FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indices, int64_t n_rows_max,
+                                const int32_t* d_n_rows, const void* d_x, int64_t ldx, int D, int dtype, int mode,
+                                int zero_policy, const int32_t* d_row_norm, const int32_t* d_col_norm,
+                                const float* d_edge_w, int n_heads, const int32_t* d_edge_index,
+                                int64_t longest_row_max, const int32_t* d_longest_row, int64_t n_entries_max,
+                                void* d_out, int64_t ldo, void* d_ws, size_t ws_bytes, void* stream)
+{
     FGL_REQUIRE(n_rows_max >= 0, "aggregate: negative row count");
     FGL_REQUIRE(D >= 1, "aggregate: feature length %d < 1", D);
     FGL_REQUIRE(ldx >= D && ldo >= D, "aggregate: row stride smaller than the row length");
@@ -1495,6 +1757,9 @@ FGL_EXPORT int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices, 
     g.x = d_x; g.ldx = ldx; g.D = D; g.zero_policy = zero_policy; g.row_norm = d_row_norm; g.col_norm = d_col_norm;
     g.out = d_out; g.ldo = ldo; g.edge_w = d_edge_w; g.edge_index = d_edge_index; g.longest_row = d_longest_row;
     g.n_heads = n_heads > 0 ? n_heads : 1; g.unit_dim = D / g.n_heads; g.col_norm_is_ptr = col_norm_is_ptr;
+    const size_t ws_needed = n_rows_max <= 0x7FFFFFFF ? fgl_aggregate_workspace_bytes(n_entries_max, D, mode, longest_row_max) : 0;
+    g.ws = ws_needed > 0 && d_ws != nullptr && ws_bytes >= ws_needed ? d_ws : nullptr;
+    g.n_entries_max = n_entries_max;
     hipStream_t s = as_stream(stream);
     if (dtype == FGL_F32) return launch_agg_vec<float, 4>(mode, longest_row_max, n_entries_max, s, g);
     if (bf16_rows_dword_aligned(ldx, ldo, d_x, d_out)) return launch_agg_vec<uint16_t, 8>(mode, longest_row_max, n_entries_max, s, g);

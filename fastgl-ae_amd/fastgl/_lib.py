@@ -25,6 +25,7 @@ IDMAP_ORDERED, IDMAP_ARRIVAL, IDMAP_FINAL, IDMAP_LEAVE_TABLE_EMPTY = 0, 1, 2, 8
 BLOCKS_TABLE_EMPTY, BLOCKS_LEAVE_TABLE_EMPTY, BLOCKS_SORT_TRANSPOSED = 4, 8, 16
 MAX_FANOUT = 192
 SHORT_ROW_ENTRIES = 32
+AGG_SEG_MIN_ENTRIES = 1 << 19  # fgl_aggregate_workspace_bytes asks for nothing below
 TRANSPOSE_BATCH_MAX, TRANSPOSE_BATCH_MAX_EDGES, TRANSPOSE_BATCH_MAX_COLS = 8, 1 << 20, 1 << 23
 
 _i64, _i32, _u64, _u32, _vp, _sz = C.c_int64, C.c_int, C.c_uint64, C.c_uint32, C.c_void_p, C.c_size_t
@@ -60,6 +61,9 @@ SIGNATURES = {
     "fgl_block_transpose_batch": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fgl_aggregate": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _i64,
                              _vp, _i64, _vp]),
+    "fgl_aggregate_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64]),
+    "fgl_aggregate_ws": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _i64,
+                                _vp, _i64, _vp, _sz, _vp]),
     "fgl_zero_empty_rows": (_i32, [_vp, _i64, _vp, _vp, _i64, _i32, _i32, _vp]),
     "fgl_aggregate_last_mapping": (C.c_char_p, []),
     "fgl_edge_softmax": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i32, C.c_float, _vp, _vp]),

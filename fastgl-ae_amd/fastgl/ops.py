@@ -443,12 +443,18 @@ def aggregate(indptr, indices, feat, mode="sum", zero_policy="self", row_norm=No
         if n > 0:
             # a block without entries has no index array to point at; the kernel then reads none
             idx_ptr = L.ptr(indices) if indices.numel() else L.ptr(indptr)
-            L.check(L.lib().fgl_aggregate(L.ptr(indptr), idx_ptr, n, L.ptr(n_rows_dev), L.ptr(feat), int(feat.stride(0)), D,
-                                          L.F32 if feat.dtype == torch.float32 else L.BF16, m, z, L.ptr(row_norm),
-                                          L.ptr(col_norm), L.ptr(edge_weight), int(n_heads), L.ptr(edge_index),
-                                          longest_host if mapping == "auto" else -1, L.ptr(longest_dev),
-                                          int(indices.numel()) if mapping == "auto" else -1, L.ptr(out),
-                                          int(out.stride(0)), L.stream_handle()))
+            n_entries = int(indices.numel()) if mapping == "auto" else -1
+            longest_known = longest_host if mapping == "auto" else -1
+            ws, ws_bytes = None, 0
+            if n_entries >= L.AGG_SEG_MIN_ENTRIES:
+                ws_bytes = L.lib().fgl_aggregate_workspace_bytes(n_entries, D, m, longest_known)
+                # (the allocator's own, not the stream's shared scratch: a captured call must not see that one grow)
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+            L.check(L.lib().fgl_aggregate_ws(L.ptr(indptr), idx_ptr, n, L.ptr(n_rows_dev), L.ptr(feat), int(feat.stride(0)), D,
+                                             L.F32 if feat.dtype == torch.float32 else L.BF16, m, z, L.ptr(row_norm),
+                                             L.ptr(col_norm), L.ptr(edge_weight), int(n_heads), L.ptr(edge_index),
+                                             longest_known, L.ptr(longest_dev), n_entries, L.ptr(out),
+                                             int(out.stride(0)), L.ptr(ws), ws_bytes, L.stream_handle()))
     return out
 
 

@@ -367,6 +367,17 @@ int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices,
                   const float* d_edge_w, int n_heads, const int32_t* d_edge_index,
                   int64_t longest_row_max, const int32_t* d_longest_row, int64_t n_entries_max,
                   void* d_out, int64_t ldo, void* stream);
+/* fgl_aggregate with scratch for the hub rows of large inputs: given fgl_aggregate_workspace_bytes bytes (0: none is used, and
+ * less than that is not used either), rows of hundreds of entries are summed in segments that are spread over the
+ * chip.  n_entries_max must then be no smaller than the number of entries the rows hold. */
+size_t fgl_aggregate_workspace_bytes(int64_t n_entries_max, int D, int mode, int64_t longest_row_max);
+int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indices,
+                     int64_t n_rows_max, const int32_t* d_n_rows,
+                     const void* d_x, int64_t ldx, int D, int dtype, int mode, int zero_policy,
+                     const int32_t* d_row_norm, const int32_t* d_col_norm,
+                     const float* d_edge_w, int n_heads, const int32_t* d_edge_index,
+                     int64_t longest_row_max, const int32_t* d_longest_row, int64_t n_entries_max,
+                     void* d_out, int64_t ldo, void* d_ws, size_t ws_bytes, void* stream);
 /* Rows of x (n_rows rows of D elements of `dtype`, row stride ldx) that have no entries become zeros: what the weight
  * gradient of a layer that passes such rows through in its forward pass wants of the gathered rows it has kept (rows
  * without edges send no gradient back, aggregate_acc_kernel.cu:498-500). */
