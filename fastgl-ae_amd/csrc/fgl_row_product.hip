@@ -1,0 +1,330 @@
+// A dense layer's product over the rows of a block: C[m, n] = sum over k of A[m, k] * B[k, n] (+ bias[n]), with m the node count of
+// a block -- 10^2 .. 10^6, another one with every mini-batch -- and k, n layer widths.  B is the layer's weight, either [k, n] or,
+// transposed, [n, k] (the reference forms these products with torch::mm, cuda_operators/aggregate_acc.cpp:144,188,371,402).
+//
+// Why not the library: it looks for a kernel by the exact sizes on every call, and a new m each time means 60-80 us of host time
+// per product (74 against 13 through here), which is what a training step over mini-batches waited for: GCN step 994 -> 843 us, GraphSAGE
+// in bf16 1482 -> 1094, GAT 1224 -> 941.  Where such products gain is ops._forms_row_product's rule.
+//
+// What bounds it: in fp32 the matrix cores, in bf16 the one pass over A and C.
+//
+// Tile: a wave holds (32 VA) x (32 VB) outputs in its accumulators.  Nothing goes through LDS: the order of the k within a step
+// is free, so lane i of a half-wave reads its own row of A with one 16-byte load along k (half 0 the step's first values, half 1 the rest) and
+// has the operands of four matrix instructions (fp32; in bf16 of one, v_mfma_f32_32x32x16_bf16 wants eight consecutive k per lane).
+// B comes the same way where it is transposed, and with one VB-wide load per k where it is not.  A lane's VB columns are
+// neighbours, so C is stored in whole vectors, 32 lanes side by side.  B is read by every wave; it is a few hundred
+// kilobytes that stay in the L2s, and the waves of a workgroup read it at the same time through one L1.
+// Workgroups that share rows of A (different columns of C) are neighbours on one XCD.
+// The next step's operands are requested before the current ones are multiplied.
+//
+// Measured (MI355X, us, the library's kernel / this one, the same sizes again and again): fp32 1000 x 100 x 64 21 / 13, 107 K x 100 x 256 84 / 80,
+// 107 K x 256 x 256 140 / 149 (94 TFLOP/s), 300 K x 128 x 128 134 / 113; bf16 107 K x 100 x 256 30 / 24, 107 K x 256 x 256 30 / 39; a transposed B, whose
+// loads touch a line per lane, costs up to a quarter more in fp32 and a third in bf16.
+//
+// Rows past the end repeat the last one and are not stored; a lane whose columns would leave the row takes the row's last VB columns
+// (bit-equal copies of its neighbour's); k past the end is zero in both operands.  No access leaves the operands.
+#include "fgl_common.hpp"
+#include "fgl_kernels.hpp"
+
+namespace fgl {
+
+typedef float RpF32x16 __attribute__((ext_vector_type(16)));
+typedef float RpF4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t RpU4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 RpBf16x8 __attribute__((ext_vector_type(8)));
+
+// One lane's values of a step: kLane values along k of one row (A, or a column of a transposed B).
+template <typename T>
+struct RpRow;
+template <>
+struct RpRow<float> {
+    static constexpr int kLane = 4;  // per half-wave: a step is 8 k
+    RpF4 v;
+    __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const RpF4*>(p); }
+    __device__ __forceinline__ void load_tail(const float* p, int n)
+    {
+#pragma unroll
+        for (int j = 0; j < kLane; ++j) {
+            v[j] = 0.0f;
+            if (j < n) v[j] = p[j];
+        }
+    }
+};
+template <>
+struct RpRow<uint16_t> {
+    static constexpr int kLane = 8;  // per half-wave: a step is 16 k
+    RpU4 v;
+    __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const RpU4*>(p); }
+    __device__ __forceinline__ void load_tail(const uint16_t* p, int n)
+    {
+#pragma unroll
+        for (int j = 0; j < kLane / 2; ++j) {
+            uint32_t lo = 0, hi = 0;
+            if (2 * j < n) lo = p[2 * j];
+            if (2 * j + 1 < n) hi = p[2 * j + 1];
+            v[j] = lo | hi << 16;
+        }
+    }
+    __device__ __forceinline__ RpBf16x8 operand() const { return __builtin_bit_cast(RpBf16x8, v); }
+};
+
+// One lane's values of a step of an untransposed B: kLane rows (k) of VB neighbouring columns.
+template <typename T, int VB>
+struct RpCols;
+template <int VB>
+struct RpCols<float, VB> {
+    typedef float Vec __attribute__((ext_vector_type(VB), aligned(4)));
+    Vec r[4];
+    __device__ __forceinline__ void load_one(const float* p, int j) { r[j] = *reinterpret_cast<const Vec*>(p); }
+    __device__ __forceinline__ void zero(int j) { r[j] = Vec{}; }
+};
+template <int VB>
+struct RpCols<uint16_t, VB> {
+    static constexpr int kWords = VB == 4 ? 2 : 1;
+    typedef uint32_t Vec2 __attribute__((ext_vector_type(2), aligned(4)));
+    uint32_t r[8][kWords];
+    __device__ __forceinline__ void load_one(const uint16_t* p, int j)
+    {
+        if constexpr (VB == 1) {
+            r[j][0] = *p;
+        } else if constexpr (VB == 2) {
+            r[j][0] = *reinterpret_cast<const uint32_t*>(p);
+        } else {
+            const Vec2 v = *reinterpret_cast<const Vec2*>(p);
+            r[j][0] = v[0];
+            r[j][1] = v[1];
+        }
+    }
+    __device__ __forceinline__ void zero(int j)
+    {
+#pragma unroll
+        for (int w = 0; w < kWords; ++w) r[j][w] = 0u;
+    }
+    // column c of the lane's eight rows, as the instruction's operand
+    __device__ __forceinline__ RpBf16x8 operand(int c) const
+    {
+        RpU4 o;
+        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;  // the high or the low halves of two words
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(r[2 * j + 1][c >> 1], r[2 * j][c >> 1], sel);
+        return __builtin_bit_cast(RpBf16x8, o);
+    }
+};
+
+struct RowProductArgs {
+    const void* a;
+    const void* b;
+    const void* bias;
+    void* c;
+    int64_t lda, ldb, ldc, m;
+    int n, k;
+    int tiles_n;          // tiles of C along n
+    int64_t row_blocks;   // workgroups along m
+};
+
+template <typename T, int VA, int VB, bool BT>
+struct RpStep {
+    static constexpr int kLane = RpRow<T>::kLane;
+    RpRow<T> a[VA];
+    RpRow<T> bt[BT ? VB : 1];
+    RpCols<T, VB> bn;  // (unused where B is transposed, and then no registers)
+
+    // k0: the half-wave's first k of the step; a whole step
+    __device__ __forceinline__ void load(const T* const (&pa)[VA], const T* pb, int64_t ldb, int k0)
+    {
+#pragma unroll
+        for (int i = 0; i < VA; ++i) a[i].load(pa[i] + k0);
+        if constexpr (BT) {
+#pragma unroll
+            for (int t = 0; t < VB; ++t) bt[t].load(pb + t * ldb + k0);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kLane; ++j) bn.load_one(pb + (int64_t)(k0 + j) * ldb, j);
+        }
+    }
+    // only the first n of the half-wave's values exist (n may be <= 0)
+    __device__ __forceinline__ void load_tail(const T* const (&pa)[VA], const T* pb, int64_t ldb, int k0, int n)
+    {
+#pragma unroll
+        for (int i = 0; i < VA; ++i) a[i].load_tail(pa[i] + k0, n);
+        if constexpr (BT) {
+#pragma unroll
+            for (int t = 0; t < VB; ++t) bt[t].load_tail(pb + t * ldb + k0, n);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kLane; ++j) {
+                bn.zero(j);
+                if (j < n) bn.load_one(pb + (int64_t)(k0 + j) * ldb, j);
+            }
+        }
+    }
+    __device__ __forceinline__ void multiply(RpF32x16 (&acc)[VA * VB]) const
+    {
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int j = 0; j < kLane; ++j)
+#pragma unroll
+                for (int i = 0; i < VA; ++i)
+#pragma unroll
+                    for (int t = 0; t < VB; ++t) {
+                        float b;
+                        if constexpr (BT) b = bt[t].v[j];
+                        else b = bn.r[j][t];
+                        acc[i * VB + t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i].v[j], b, acc[i * VB + t], 0, 0, 0);
+                    }
+        } else {
+#pragma unroll
+            for (int t = 0; t < VB; ++t) {
+                RpBf16x8 b;
+                if constexpr (BT) b = bt[t].operand();
+                else b = bn.operand(t);
+#pragma unroll
+                for (int i = 0; i < VA; ++i) acc[i * VB + t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i].operand(), b, acc[i * VB + t], 0, 0, 0);
+            }
+        }
+    }
+};
+
+template <typename T, int VB>
+__device__ __forceinline__ void rp_store(T* p, const float (&v)[VB])
+{
+    if constexpr (sizeof(T) == 4) {
+        typedef float Vec __attribute__((ext_vector_type(VB), aligned(4)));
+        Vec o;
+#pragma unroll
+        for (int t = 0; t < VB; ++t) o[t] = v[t];
+        *reinterpret_cast<Vec*>(p) = o;
+    } else if constexpr (VB == 1) {
+        *reinterpret_cast<__bf16*>(p) = (__bf16)v[0];
+    } else {
+        typedef __bf16 Vec __attribute__((ext_vector_type(VB), aligned(4)));
+        Vec o;
+#pragma unroll
+        for (int t = 0; t < VB; ++t) o[t] = (__bf16)v[t];
+        *reinterpret_cast<Vec*>(p) = o;
+    }
+}
+
+template <typename T, int VA, int VB, bool BT>
+__global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kernel(const RowProductArgs g)
+{
+    constexpr int kLane = RpRow<T>::kLane, kStep = 2 * kLane;
+    const int lane = lane_id();
+    const int half = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    // workgroup -> (rows, columns): eight neighbouring row groups (one per XCD) take turns, so the tiles of a row group share an XCD
+    const unsigned per_group = 8u * (unsigned)g.tiles_n;
+    const int64_t rb = (int64_t)(blockIdx.x / per_group) * 8 + blockIdx.x % per_group % 8;
+    const int tn = (int)(blockIdx.x % per_group / 8);
+    const int64_t row0 = (rb * (kBlock / kWave) + wave) * (32 * VA);
+    if (rb >= g.row_blocks || row0 >= g.m) return;  // (uniform over the wave)
+
+    const T* pa[VA];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) {
+        const int64_t row = row0 + 32 * i + lane % 32;
+        pa[i] = static_cast<const T*>(g.a) + (row < g.m ? row : g.m - 1) * g.lda;
+    }
+    int col = (tn * 32 + lane % 32) * VB;
+    if (col + VB > g.n) col = g.n - VB;
+    const T* pb = static_cast<const T*>(g.b) + (BT ? (int64_t)col * g.ldb : (int64_t)col);
+    RpF32x16 acc[VA * VB];
+#pragma unroll
+    for (int t = 0; t < VA * VB; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+    float add[VB];
+#pragma unroll
+    for (int t = 0; t < VB; ++t) {
+        add[t] = 0.0f;
+        if (g.bias != nullptr) {
+            if constexpr (sizeof(T) == 4) add[t] = static_cast<const float*>(g.bias)[col + t];
+            else add[t] = __uint_as_float((uint32_t)static_cast<const uint16_t*>(g.bias)[col + t] << 16);
+        }
+    }
+
+    // Steps before the last one are whole.  As in wgrad_kernel nothing branches between the last products and the first reads of
+    // the accumulators, and every branch around a product is one of the whole wave.
+    const int whole = (g.k - 1) / kStep;
+    RpStep<T, VA, VB, BT> cur, next;
+    int k0 = half * kLane;
+    if (whole > 0) cur.load(pa, pb, g.ldb, k0);
+    else cur.load_tail(pa, pb, g.ldb, k0, 0);  // (zeros)
+    for (int s = 1; s < whole; ++s) {
+        k0 += kStep;
+        next.load(pa, pb, g.ldb, k0);
+        __builtin_amdgcn_sched_barrier(0);  // (left alone, the compiler moves the loads behind the products to save registers)
+        cur.multiply(acc);
+        cur = next;
+    }
+    k0 = whole * kStep + half * kLane;
+    if (g.k % kStep == 0) next.load(pa, pb, g.ldb, k0);
+    else next.load_tail(pa, pb, g.ldb, k0, g.k - k0);
+    cur.multiply(acc);
+    next.multiply(acc);
+
+    // accumulator register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32x32 tile
+#pragma unroll
+    for (int i = 0; i < VA; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int64_t row = row0 + 32 * i + 8 * (r / 4) + 4 * half + r % 4;
+            float v[VB];
+#pragma unroll
+            for (int t = 0; t < VB; ++t) v[t] = acc[i * VB + t][r] + add[t];
+            if (row < g.m) rp_store<T, VB>(static_cast<T*>(g.c) + row * g.ldc + col, v);
+        }
+}
+
+template <typename T, int VA, int VB, bool BT>
+static int launch_row_product(RowProductArgs g, hipStream_t stream)
+{
+    g.tiles_n = (int)ceil_div(g.n, 32 * VB);
+    g.row_blocks = ceil_div(g.m, (int64_t)(kBlock / kWave) * 32 * VA);
+    const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
+    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");
+    hipLaunchKernelGGL((row_product_kernel<T, VA, VB, BT>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
+    FGL_CHECK_LAUNCH("row_product_kernel");
+    return FGL_OK;
+}
+
+// Tile: what pads n least, wide tiles where they still make a thousand waves (four per CU).
+template <typename T, bool BT>
+static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStream_t stream)
+{
+    const int64_t pad1 = ceil_div(g.n, 32) * 32;
+    int vb = 1;
+    for (int v = 2; v <= 4 && vectors; v *= 2) {
+        const int64_t p = ceil_div(g.n, 32 * v) * 32 * v;
+        const int64_t waves = ceil_div(g.m, 32) * (p / (32 * v));
+        if (g.n >= v && p * 10 <= pad1 * 12 && waves >= 1024) vb = v;
+    }
+    const bool tall = vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048;
+    if (vb == 4) return tall ? launch_row_product<T, 2, 4, BT>(g, stream) : launch_row_product<T, 1, 4, BT>(g, stream);
+    if (vb == 2) return tall ? launch_row_product<T, 2, 2, BT>(g, stream) : launch_row_product<T, 1, 2, BT>(g, stream);
+    return launch_row_product<T, 1, 1, BT>(g, stream);
+}
+
+}  // namespace fgl
+
+using namespace fgl;
+
+FGL_EXPORT int fgl_row_product(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
+                               const void* d_bias, void* d_c, int64_t ldc, void* stream)
+{
+    FGL_REQUIRE(m >= 0 && k >= 1 && n >= 1 && k <= 65536 && n <= 65536, "row_product: sizes %lld x %d x %d", (long long)m, k, n);
+    FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "row_product: unknown dtype %d", dtype);
+    FGL_REQUIRE(lda >= k && ldb >= (b_transposed ? k : n) && ldc >= n, "row_product: row stride smaller than the row length");
+    if (m == 0) return FGL_OK;
+    FGL_REQUIRE(d_a && d_b && d_c, "row_product: null pointer");
+    RowProductArgs g;
+    g.a = d_a; g.b = d_b; g.bias = d_bias; g.c = d_c; g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.m = m; g.n = n; g.k = k;
+    g.tiles_n = 0; g.row_blocks = 0;
+    hipStream_t s = as_stream(stream);
+    if (dtype == FGL_F32) return b_transposed ? launch_row_product_any<float, true>(g, true, s) : launch_row_product_any<float, false>(g, true, s);
+    // bf16 moves in words: every row that is read along k starts on one, and so does every vector of C (and of an untransposed B)
+    FGL_REQUIRE(lda % 2 == 0 && (uintptr_t)d_a % 4 == 0 && (!b_transposed || (ldb % 2 == 0 && (uintptr_t)d_b % 4 == 0)),
+                "row_product: bf16 rows must start on 4-byte boundaries");
+    const bool vectors = n % 2 == 0 && ldc % 2 == 0 && (uintptr_t)d_c % 4 == 0 && (b_transposed || (ldb % 2 == 0 && (uintptr_t)d_b % 4 == 0));
+    return b_transposed ? launch_row_product_any<uint16_t, true>(g, vectors, s) : launch_row_product_any<uint16_t, false>(g, vectors, s);
+}

@@ -88,11 +88,11 @@ class MA_Function(torch.autograd.Function):
         longest = ops._fanout_bound(edge_ptr, neighbor_num)
         if not gather_first:
             ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, input_feat)
-            return MA_Function._gather(edge_ptr, src_edges, torch.mm(input_feat, weight), src_norm_degs, dst_norm_degs, n_dst, transposed,
+            return MA_Function._gather(edge_ptr, src_edges, ops.row_product(input_feat, weight), src_norm_degs, dst_norm_degs, n_dst, transposed,
                                        "self", longest)
         ax = MA_Function._gather(edge_ptr, src_edges, input_feat, src_norm_degs, dst_norm_degs, n_dst, transposed, "self", longest)
         ctx.n_src = int(input_feat.size(0))
-        out = torch.mm(ax, weight)
+        out = ops.row_product(ax, weight)
         if any(ctx.needs_input_grad):
             # what the weight gradient wants of the gathered rows: rows without edges send no gradient back
             ops.zero_empty_rows_(edge_ptr, ax, n_dst)
@@ -107,7 +107,7 @@ class MA_Function(torch.autograd.Function):
             d_w = ops.weight_grad(ax, d_input)
             d_x = None
             if ctx.needs_input_grad[5]:
-                d_ax = torch.mm(d_input, weight.transpose(0, 1))  # (rows without edges are in no source's list)
+                d_ax = ops.row_product(d_input, weight, transposed=True)  # (rows without edges are in no source's list)
                 if ctx.transposed is None:
                     t_ptr, t_idx = ops.block_transpose(edge_ptr, src_edges, int(d_input.size(0)), ctx.n_src)
                 else:
@@ -127,7 +127,7 @@ class MA_Function(torch.autograd.Function):
         else:  # same arithmetic as backward_gcn, with the block's cached transpose
             t_ptr, t_idx = _transposed(ctx.transposed)
             g = MA_Function._gather_back(t_ptr, t_idx, d_input, src_norm_degs, dst_norm_degs, int(input_feat.size(0)), edge_ptr)
-            d_x = torch.mm(g, weight.transpose(0, 1))
+            d_x = ops.row_product(g, weight, transposed=True)
             d_w = ops.weight_grad(input_feat, g)
         return None, None, None, None, None, d_x, d_w, None, None, None
 
@@ -216,7 +216,7 @@ class MA_Function_GIN(torch.autograd.Function):
             d_x = None
             if ctx.needs_input_grad[3]:  # not for the first layer: its transposed block is never built
                 t_ptr, t_idx = _transposed(ctx.transposed)
-                d_tmp = torch.mm(d_input, weight.transpose(0, 1))
+                d_tmp = ops.row_product(d_input, weight, transposed=True)
                 d_x = ops.aggregate(t_ptr, t_idx, d_tmp, mode="sum", zero_policy="zeros", n_rows=int(ctx.src_nodes))
         return None, None, None, d_x, d_w, None, None
 
@@ -255,14 +255,14 @@ class _LinearFunction(torch.autograd.Function):
     def forward(ctx, x, weight, bias):
         ctx.save_for_backward(x, weight)
         ctx.with_bias = bias is not None
-        return nn.functional.linear(x, weight, bias)
+        return ops.row_product(x, weight, transposed=True, bias=bias)
 
     @staticmethod
     def backward(ctx, d_out):
         x, weight = ctx.saved_tensors
         d_x = d_w = d_b = None
         if ctx.needs_input_grad[0]:
-            d_x = torch.mm(d_out, weight)
+            d_x = ops.row_product(d_out, weight)
         want_bias = ctx.with_bias and ctx.needs_input_grad[2]
         if torch.is_grad_enabled():  # (a graph of the gradients is being built: operators that have gradients themselves)
             d_w = torch.mm(d_out.transpose(0, 1), x)
@@ -281,9 +281,14 @@ class _Linear(nn.Linear):
     weight's own type (fp32 or bf16), outside autocast."""
 
     def forward(self, x):
-        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and torch.is_grad_enabled()
-                and not torch.is_autocast_enabled()):
+        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()):
             return super().forward(x)
+        if not torch.is_grad_enabled():
+            # (tensors that something watches the operators on keep the operator)
+            if type(x) is not torch.Tensor or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch.jit.is_tracing() or \
+                    torch.autograd.forward_ad._current_level >= 0:
+                return super().forward(x)
+            return ops.row_product(x, self.weight, transposed=True, bias=self.bias)
         return _LinearFunction.apply(x, self.weight, self.bias)
 
 

@@ -249,7 +249,7 @@ def forward_gcn(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, input_feat, w
         _check_input(t, n, _I32)
     _check_input(input_feat, "input_feat", _FEAT)
     _check_input(weight, "weight", _FEAT)
-    tmp = torch.mm(input_feat, weight)
+    tmp = row_product(input_feat, weight)
     out = aggregate(edge_ptr, src_edges, tmp, mode="gcn", zero_policy="self", row_norm=dst_norm_degs,
                     col_norm=src_norm_degs, n_rows=int(dst_nodes), longest_row=_fanout_bound(edge_ptr, neighbor_num))
     return [out]
@@ -271,7 +271,7 @@ def backward_gcn(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, d_input, wei
     n_dst = int(d_input.size(0))
     t_ptr, t_idx = block_transpose(edge_ptr, src_edges, n_dst, n_src)
     g = aggregate(t_ptr, t_idx, d_input, mode="gcn", zero_policy="zeros", row_norm=by_src, col_norm=by_dst, n_rows=n_src)
-    d_x = torch.mm(g, weight.transpose(0, 1))
+    d_x = row_product(g, weight, transposed=True)
     d_w = weight_grad(input_feat, g)
     return [d_x, d_w]
 
@@ -285,7 +285,7 @@ def forwaed_gin(edge_ptr, src_edges, input_feat, weight, neighbor_num, dst_nodes
     _check_input(weight, "weight", _FEAT)
     tmp = aggregate(edge_ptr, src_edges, input_feat, mode="sum", zero_policy="self", n_rows=int(dst_nodes),
                     longest_row=_fanout_bound(edge_ptr, neighbor_num))
-    return [torch.mm(tmp, weight), tmp]
+    return [row_product(tmp, weight), tmp]
 
 
 def backward_gin(edge_ptr, src_edges, d_input, weight, input_feat, src_nodes):
@@ -296,7 +296,7 @@ def backward_gin(edge_ptr, src_edges, d_input, weight, input_feat, src_nodes):
     _check_input(d_input, "d_input", _FEAT)
     _check_input(weight, "weight", _FEAT)
     _check_input(input_feat, "input_feat", _FEAT)
-    d_tmp = torch.mm(d_input, weight.transpose(0, 1))
+    d_tmp = row_product(d_input, weight, transposed=True)
     d_w = weight_grad(input_feat, d_input)
     n_dst = int(d_input.size(0))
     t_ptr, t_idx = block_transpose(edge_ptr, src_edges, n_dst, int(src_nodes))
@@ -339,6 +339,40 @@ def _splits_k(k, m, n):
     190 -> 72 us, bf16 245 -> 25 us; 256 x 256, k = 500: 119 -> 27 us).  Many tiles and a short k are the library GEMM's
     (1024 x 1024, k = 8192: 145 us against 268 in fp32, 57 against 63 in bf16; 256 x 1024, k = 2000: 20 against 31)."""
     return m * n <= 65536 or k * k >= 256 * m * n
+
+
+def _forms_row_product(a, b, transposed, m, k, n):
+    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call, no
+    autocast to change the types, and a size where it gains.  The library looks for a kernel on every call with sizes it has not just
+    seen -- 74 us of the host's time against 13 -- which is what a product of a mini-batch takes; on the GPU the two are
+    alike (us, library / here: fp32 1000 x 100 x 64 21 / 13, 8192 x 602 x 256 29 / 29, 107 K x 256 x 256 140 / 149, bf16 107 K x 100 x 256
+    30 / 24, 107 K x 256 x 256 30 / 39 and, with a transposed weight, 27 / 53).  Larger ones keep the GPU busy for longer than
+    the host takes, and there the library's tiles through LDS are ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; 20 K x 512 x 512
+    89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all)."""
+    return (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
+            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and not torch.is_autocast_enabled() and
+            a.stride(1) == 1 and a.stride(0) >= k and b.stride(1) == 1 and b.stride(0) >= b.size(1) and
+            (a.dtype == torch.float32 or (a.stride(0) % 2 == 0 and a.data_ptr() % 4 == 0 and
+                                          (not transposed or (b.stride(0) % 2 == 0 and b.data_ptr() % 4 == 0)))))
+
+
+def row_product(a, b, transposed=False, bias=None):
+    """``a b`` (``transposed``: ``a b^T``) ``+ bias`` for the rows ``a`` [m, k] of a block and a layer's weight ``b`` [k, n]
+    (transposed: [n, k]); fp32 sums, result in the operands' dtype."""
+    if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(1 if transposed else 0):
+        raise RuntimeError("row_product: shapes %s and %s do not match" % (tuple(a.shape), tuple(b.shape)))
+    m, k, n = int(a.size(0)), int(a.size(1)), int(b.size(0 if transposed else 1))
+    if not (_forms_row_product(a, b, transposed, m, k, n) and
+            (bias is None or (bias.device == a.device and bias.dtype == a.dtype and bias.is_contiguous() and bias.numel() == n and
+                              not (torch.is_grad_enabled() and bias.requires_grad)))):
+        w = b.transpose(0, 1) if transposed else b
+        return torch.mm(a, w) if bias is None else torch.addmm(bias, a, w)
+    dev = a.device
+    with _on_device(dev):
+        out = torch.empty((m, n), dtype=a.dtype, device=dev)
+        L.check(L.lib().fgl_row_product(L.ptr(a), a.stride(0), L.ptr(b), b.stride(0), int(transposed), m, k, n,
+                                        L.F32 if a.dtype == torch.float32 else L.BF16, L.ptr(bias), L.ptr(out), n, L.stream_handle()))
+    return out
 
 
 def weight_grad(a, b, column_sums=False):

@@ -409,6 +409,13 @@ int fgl_edge_softmax(const int32_t* d_indptr, const int32_t* d_indices, int64_t 
 int fgl_head_scores(const float* d_x, int64_t ldx, int64_t n_rows, int64_t n_er, int n_heads, int width, const float* d_attn_l,
                     const float* d_attn_r, float* d_el, float* d_er, void* stream);
 
+/* A dense layer's product over the rows of a block: C[m, n] = A[m, k] B (+ bias[n]; d_bias may be NULL), with B [k, n] or, where
+ * b_transposed is not zero, [n, k] (replaces torch::mm in aggregate_acc.cpp:144,188,371,402).  Operands and result of
+ * `dtype`, sums in fp32, row strides in elements.  bf16: lda even and d_a on a 4-byte boundary, and where b_transposed ldb and d_b
+ * likewise (else an error). */
+int fgl_row_product(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
+                    const void* d_bias, void* d_c, int64_t ldc, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * Weight gradient of a dense layer: C[i, j] = sum over r < k of A[r, i] * B[r, j] -- the d_w = X^T G of backward_gcn /
  * backward_gin (aggregate_acc.cpp:371-374,402-405, torch::mm on a transposed view there).  A: [k, m] with row stride
