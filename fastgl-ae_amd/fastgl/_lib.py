@@ -124,7 +124,10 @@ _workspaces = {}
 
 def workspace(nbytes: int, device) -> torch.Tensor:
     """A scratch buffer of at least nbytes for (device, current stream).  Kernels are
-    stream-ordered, so consecutive calls on one stream may share it."""
+    stream-ordered, so consecutive calls on one stream may share it.  A call that is being captured gets a buffer of its own
+    from the graph's memory: the shared one is replaced when a later call needs more, and replays would go on writing to it."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
     key = (torch.device(device).index, stream_handle())
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
