@@ -276,18 +276,22 @@ class _LinearFunction(torch.autograd.Function):
         return d_x, d_w, d_b
 
 
+def _watched(t):
+    """Whether something follows the operators that ``t`` goes through: a tensor subclass, a transform of ``torch.func``."""
+    return type(t) not in (torch.Tensor, nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+
+
 class _Linear(nn.Linear):
-    """``nn.Linear`` with ``_LinearFunction``'s backward pass for the inputs it is made for: matrices on the GPU in the
-    weight's own type (fp32 or bf16), outside autocast."""
+    """``nn.Linear`` with ``_LinearFunction``'s backward pass for the inputs it is made for: plain matrices on the GPU in the
+    weight's own type (fp32 or bf16), outside autocast, tracing, compilation and forward-mode differentiation (``_LinearFunction`` has
+    no rule for those; the operator has)."""
 
     def forward(self, x):
-        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()):
+        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()) or \
+                _watched(x) or _watched(self.weight) or (self.bias is not None and _watched(self.bias)) or torch.jit.is_tracing() or torch.compiler.is_compiling() or \
+                torch.autograd.forward_ad._current_level >= 0:
             return super().forward(x)
         if not torch.is_grad_enabled():
-            # (tensors that something watches the operators on keep the operator)
-            if type(x) is not torch.Tensor or torch._C._functorch.is_functorch_wrapped_tensor(x) or torch.jit.is_tracing() or \
-                    torch.autograd.forward_ad._current_level >= 0:
-                return super().forward(x)
             return ops.row_product(x, self.weight, transposed=True, bias=self.bias)
         return _LinearFunction.apply(x, self.weight, self.bias)
 

@@ -62,3 +62,19 @@ def test_linear_without_gradients():
         with torch.autograd.forward_ad.dual_level():
             out = lin(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
             assert torch.autograd.forward_ad.unpack_dual(out).tangent is not None
+
+
+def test_linear_with_gradients_under_transforms():
+    """What torch's operator can do with a gradient being recorded, the layer still can: vmap, torch.func, forward mode, tracing."""
+    lin = fastgl.conv._Linear(20, 7).to(DEV)
+    x = torch.randn(33, 20, device=DEV)
+    with torch.enable_grad():
+        want = torch.nn.functional.linear(x, lin.weight, lin.bias)
+        assert torch.func.vmap(lin)(x[None]).shape == (1, 33, 7)
+        g = torch.func.grad(lambda p: torch.func.functional_call(lin, p, (x,)).sum())(dict(lin.named_parameters()))
+        assert torch.allclose(g["weight"], x.sum(0).expand(7, 20), rtol=1e-4, atol=1e-4)
+        with torch.autograd.forward_ad.dual_level():
+            out = lin(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+            assert torch.autograd.forward_ad.unpack_dual(out).tangent is not None
+        traced = torch.jit.trace(lin, (x,))
+        assert torch.allclose(traced(x[:5]), want[:5], rtol=1e-4, atol=1e-4)
