@@ -382,6 +382,7 @@ def weight_grad(a, b, column_sums=False):
     k, m, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
     if not (a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
             not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and  # (a graph is being built: torch's product has a gradient)
+            not torch.is_autocast_enabled() and
             a.stride(1) == 1 and b.stride(1) == 1 and m <= a.stride(0) < 1 << 24 and n <= b.stride(0) < 1 << 24 and
             m < 1 << 16 and n < 1 << 16 and b.size(0) == k and
             _splits_k(k, m, n)):

@@ -141,3 +141,18 @@ def test_compiled_module_errors_are_runtime_errors(cuda, ext):
     with pytest.raises(RuntimeError, match="negative id"):
         ext.transfer_edge_id(torch.tensor([1, -1], dtype=torch.int32, device=cuda), torch.tensor([0, 0], dtype=torch.int32, device=cuda),
                              torch.tensor([0], dtype=torch.int32, device=cuda), 1, 3, 2, 2)
+
+
+def test_weight_gradients_follow_grad_mode_and_autocast(ext, cuda):
+    """The dense products of backward_gin are torch's where a graph is being recorded or autocast picks the types."""
+    import fastgl
+    ptr = torch.arange(0, 41, 4, dtype=torch.int32, device=cuda)
+    src = torch.arange(40, dtype=torch.int32, device=cuda) % 20
+    d, w, x = (torch.randn(s, device=cuda) for s in ((10, 8), (6, 8), (10, 6)))
+    want = x.t() @ d
+    _, d_w = ext.backward_gin(ptr, src, d, w, x, 20)
+    assert rel_err(d_w, want.cpu().numpy()) < 1e-5 and not d_w.requires_grad
+    _, d_w = ext.backward_gin(ptr, src, d, w, x.clone().requires_grad_(True), 20)
+    assert d_w.requires_grad and rel_err(d_w.detach(), want.cpu().numpy()) < 1e-5
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert fastgl.ops.weight_grad(x, d).dtype == torch.bfloat16
