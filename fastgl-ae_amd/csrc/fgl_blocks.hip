@@ -238,11 +238,11 @@ __global__ __launch_bounds__(kBlock) void transpose_sort_rows_kernel(const SortJ
 }
 
 // ... and the rows of more than 64 entries that it listed, a workgroup per row
-__global__ __launch_bounds__(kBlock) void transpose_sort_long_rows_kernel(const SortJobs jobs)
+__global__ __launch_bounds__(kSortBlock) void transpose_sort_long_rows_kernel(const SortJobs jobs)
 {
     __shared__ int s_key[kSortLds];
     __shared__ int s_val[kSortLds];
-    tjob_sort_long_rows<kBlock>(jobs, s_key, s_val);
+    tjob_sort_long_rows<kSortBlock>(jobs, s_key, s_val);
 }
 
 // ---- R-MAT -------------------------------------------------------------------------
@@ -469,7 +469,7 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
                 const int64_t gx = ceil_div(most_cols, kBlock) < 4096 ? ceil_div(most_cols, kBlock) : 4096;
                 hipLaunchKernelGGL(transpose_sort_rows_kernel, dim3((unsigned)gx, (unsigned)n_jobs), dim3(kBlock), 0, s, jobs);
                 const int64_t gl = p.sort_long_max < 2048 ? p.sort_long_max : 2048;
-                hipLaunchKernelGGL(transpose_sort_long_rows_kernel, dim3((unsigned)(gl > 0 ? gl : 1)), dim3(kBlock), 0, s, jobs);
+                hipLaunchKernelGGL(transpose_sort_long_rows_kernel, dim3((unsigned)(gl > 0 ? gl : 1)), dim3(kSortBlock), 0, s, jobs);
                 FGL_CHECK_LAUNCH("transpose_sort_rows_kernel");
                 n_jobs = 0;
                 most_cols = 1;

@@ -183,6 +183,7 @@ __device__ __forceinline__ void tjob_fill(const TransposeJob& j)
 //                       hub of a whole graph taken as one block).
 // Keys are distinct (positions), or -- without t_edge -- destination rows, whose ties are interchangeable.
 constexpr int kSortLds = 4096;
+constexpr int kSortBlock = 512;  // threads of a workgroup of the second launch
 constexpr int kSortMax = 0x7FFFFFFF;
 
 struct SortJobs {
@@ -203,8 +204,25 @@ __device__ __forceinline__ void sort_exchange(int& ka, int& va, int& kb, int& vb
     }
 }
 
-// bitonic sort of n (a power of two, <= kSortLds) pairs in LDS by the whole workgroup; `merge_only`: the two
-// halves are sorted already (ascending), only the last merge is needed
+// the comparisons of a bitonic merge at distances below a wave, jj = first, first / 2, .. 1: one pair per lane, by shuffles
+__device__ __forceinline__ void sort_lanes(int& k, int& v, int first, bool up)
+{
+    const int lane = lane_id();
+    for (int jj = first; jj > 0; jj >>= 1) {
+        const int ok = __shfl_xor(k, jj, kWave), ov = __shfl_xor(v, jj, kWave);
+        const bool want_min = ((lane & jj) == 0) == up;
+        if (want_min ? ok < k : k < ok) {  // (equal keys: both lanes keep theirs)
+            k = ok;
+            v = ov;
+        }
+    }
+}
+
+// bitonic sort of n (a power of two, 128 <= n <= kSortLds) pairs in LDS by the whole workgroup; `merge_only`: the two
+// halves are sorted already (ascending), only the last merge is needed.  What bounds it is the chain of steps (78 for 4096
+// pairs), each a pass over LDS and a barrier: the 57 at distances below a wave are done in registers, a wave per 64 neighbours,
+// which leaves 21 barriers of that kind and 7 around the register passes.  The long rows of a five-hop mini-batch (1000 seeds,
+// 2.4 M nodes), with 512 threads a row instead of 256: 98 -> 67 us (1024 threads: 65, and half as many rows at a time).
 template <int NT>
 __device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n, bool merge_only)
 {
@@ -218,9 +236,17 @@ __device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n, bool mer
             s_val[b] = v;
         }
         __syncthreads();
+    } else {
+        for (int i = threadIdx.x; i < n; i += NT) {  // (n and NT are multiples of a wave)
+            int k = s_key[i], v = s_val[i];
+            for (int run = 2; run <= kWave; run <<= 1) sort_lanes(k, v, run >> 1, (i & run) == 0);
+            s_key[i] = k;
+            s_val[i] = v;
+        }
+        __syncthreads();
     }
-    for (int k = merge_only ? n : 2; k <= n; k <<= 1) {
-        for (int jj = k >> 1; jj > 0; jj >>= 1) {
+    for (int k = merge_only ? n : 2 * kWave; k <= n; k <<= 1) {
+        for (int jj = k >> 1; jj >= kWave; jj >>= 1) {
             for (int t = threadIdx.x; t < n / 2; t += NT) {
                 const int i = 2 * t - (t & (jj - 1));  // the lower index of the t-th pair at distance jj
                 const int o = i + jj;
@@ -235,6 +261,13 @@ __device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n, bool mer
             }
             __syncthreads();
         }
+        for (int i = threadIdx.x; i < n; i += NT) {
+            int key = s_key[i], val = s_val[i];
+            sort_lanes(key, val, kWave / 2, (i & k) == 0 || k == n);
+            s_key[i] = key;
+            s_val[i] = val;
+        }
+        __syncthreads();
     }
 }
 
