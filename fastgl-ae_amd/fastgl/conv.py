@@ -92,18 +92,17 @@ class MA_Function(torch.autograd.Function):
                                        "self", longest)
         ax = MA_Function._gather(edge_ptr, src_edges, input_feat, src_norm_degs, dst_norm_degs, n_dst, transposed, "self", longest)
         ctx.n_src = int(input_feat.size(0))
-        out = ops.row_product(ax, weight)
-        if any(ctx.needs_input_grad):
-            # what the weight gradient wants of the gathered rows: rows without edges send no gradient back
-            ops.zero_empty_rows_(edge_ptr, ax, n_dst)
-            ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax)
-        return out
+        ctx.save_for_backward(edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax)
+        return ops.row_product(ax, weight)
 
     @staticmethod
     def backward(ctx, d_input):
         d_input = d_input.contiguous()
         if ctx.gather_first:
             edge_ptr, src_edges, src_norm_degs, dst_norm_degs, weight, ax = ctx.saved_tensors
+            # what the weight gradient wants of the gathered rows (nobody else has them): rows without edges send no gradient
+            # back.  Here and not in forward, where a pass that records nothing would pay for it (two launches of infer's twenty).
+            ops.zero_empty_rows_(edge_ptr, ax, int(d_input.size(0)))
             d_w = ops.weight_grad(ax, d_input)
             d_x = None
             if ctx.needs_input_grad[5]:
