@@ -290,7 +290,7 @@ static int range_slices(int64_t n_ids, int64_t n_counters)
 // ranges) and four million ids, and small inputs take them where a counter is mentioned twice on average.
 static bool count_by_ranges(int64_t n_ids, int64_t n_counters)
 {
-    return n_ids >= ((int64_t)1 << 16) && n_ids < ((int64_t)1 << 22) && n_counters <= ((int64_t)1 << 19) &&
+    return n_ids >= ((int64_t)1 << 16) && n_ids < ((int64_t)1 << 22) && n_counters > 0 && n_counters <= ((int64_t)1 << 19) &&
            (n_ids >= ((int64_t)1 << 18) || 2 * n_counters <= n_ids);
 }
 static bool fits_buckets(int64_t n_entries, int64_t n_cols) { return n_entries <= 0x7FFFFFFF && n_cols > 0 && n_cols <= ((int64_t)kMaxBuckets << kMaxWidthLog); }

@@ -42,6 +42,13 @@ def test_pure_host_entry_points():
     assert lib.fgl_wait_words(words, 0, -1, None, 1000) != 0 and lib.fgl_wait_words(None, 3, -1, None, 1000) != 0
 
 
+def test_counting_into_no_counters_asks_for_no_scratch():
+    # (the ranges of counters are divided among workgroups: there must be some)
+    for n_ids in (0, 1, (1 << 16) - 1, 1 << 16, 1 << 18, 1 << 20, (1 << 22) - 1, 1 << 22, 1 << 31):
+        assert fastgl.lib().fgl_cal_deg_workspace_bytes(n_ids, 0) == 0
+    assert fastgl.lib().fgl_cal_deg_workspace_bytes(1 << 16, 1) > 0
+
+
 def test_static_scratch_holds_the_workspace_of_its_largest_call():
     # fgl_sample_node_static's 16 MiB array against what the workspace formula asks for at the stated seed limit
     lib = fastgl.lib()

@@ -31,6 +31,11 @@ def test_cal_deg(cuda, n, bins, hub):
     assert torch.equal(got.long(), torch.bincount(valid, minlength=bins))
 
 
+@pytest.mark.parametrize("n", [(1 << 16) - 1, 1 << 16, 1 << 18, 4 * M])
+def test_cal_deg_into_no_bins(cuda, n):
+    assert fastgl.cal_deg(torch.zeros(n, dtype=torch.int32, device=cuda), 0).shape == (0,)
+
+
 def _csr(lengths, device):
     ptr = torch.zeros(len(lengths) + 1, dtype=torch.int64)
     ptr[1:] = torch.cumsum(lengths, 0)
