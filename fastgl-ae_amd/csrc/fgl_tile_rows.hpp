@@ -9,11 +9,14 @@ namespace fgl {
 
 #if defined(__HIPCC__)
 
-// row r names the tiles that begin inside it
+// row r names the tiles that begin inside it.  Row 0 also names those in front of its first entry (offsets that do not start at
+// zero, as a slice of a larger CSR has them): tile_rows reads the entry of every tile below the last offset and goes by it.
 template <int TILE>
 __device__ __forceinline__ void mark_tile_rows(const int32_t* __restrict__ indptr, int64_t r, int64_t tiles, int32_t* __restrict__ tile_row)
 {
-    const int64_t a = indptr[r], b = indptr[r + 1];
+    int64_t a = indptr[r];
+    const int64_t b = indptr[r + 1];
+    if (r == 0 || a < 0) a = 0;
     for (int64_t t = (a + TILE - 1) / TILE; t * TILE < b && t < tiles; ++t) tile_row[t] = (int32_t)r;
 }
 

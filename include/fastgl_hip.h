@@ -308,6 +308,7 @@ int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const int32_t* d_in
  * by ascending row (deterministic output, needs exact sizes: d_n_rows = d_n_cols = NULL, and
  * n_edges_max = the number of entries); sorted = 0 is faster and leaves the order within a
  * column to scheduling.
+ * d_indptr[0] must be 0; entries in front of another first offset are listed as row 0's.
  * d_t_longest_row (may be NULL) receives one int32 for fgl_aggregate's d_longest_row: the
  * entry count of the transposed block's longest row if that exceeds FGL_SHORT_ROW_ENTRIES,
  * else some value not above it.

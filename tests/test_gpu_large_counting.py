@@ -90,3 +90,24 @@ def test_block_transpose(cuda, kind, n_cols, edge_ids):
         e = got[2].long()
         assert torch.equal(torch.sort(e).values, torch.arange(nnz, device=cuda))
         assert torch.equal(cols.long()[e], col_of) and torch.equal(rows[e], got[1].long())
+
+
+@pytest.mark.parametrize("sorted_rows", [False, True])
+@pytest.mark.parametrize("first,lengths,n_cols", [
+    (1, [3, 0, 2], 4), (1023, [1], 5), (5000, [3, 0, 4000, 3000], 900),  # tiles of 1024 entries, one by one
+    (9000, [40_000, 0, 230_000], 3000), (300_000, [1] * 9, 70_000)])     # tiles of 8192, through the buckets
+def test_block_transpose_of_a_slice(cuda, first, lengths, n_cols, sorted_rows):
+    """Offsets that do not start at zero: the entries in front count as row 0's, whatever the form."""
+    print("slice from", first, lengths, n_cols, sorted_rows, flush=True)
+    lens = torch.tensor(lengths)
+    ptr = _csr(lens, cuda) + first
+    nnz = first + int(lens.sum())
+    cols = torch.randint(0, n_cols, (nnz,), generator=torch.Generator().manual_seed(first), dtype=torch.int32).to(cuda)
+    t_ptr, t_idx, t_edge = fastgl.block_transpose(ptr, cols, len(lengths), n_cols, edge_ids=True, sorted_rows=sorted_rows)
+    lens[0] += first
+    rows = torch.repeat_interleave(torch.arange(len(lengths)), lens).to(cuda)
+    counts = torch.bincount(cols.long(), minlength=n_cols)
+    assert torch.equal(t_ptr[1:].long(), torch.cumsum(counts, 0)) and int(t_ptr[0]) == 0
+    e = t_edge.long()
+    assert torch.equal(torch.sort(e).values, torch.arange(nnz, device=cuda))
+    assert torch.equal(cols.long()[e], torch.repeat_interleave(torch.arange(n_cols, device=cuda), counts)) and torch.equal(rows[e], t_idx.long())
