@@ -119,21 +119,11 @@ def stream_handle() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-_workspaces = {}
-
-
 def workspace(nbytes: int, device) -> torch.Tensor:
-    """A scratch buffer of at least nbytes for (device, current stream).  Kernels are
-    stream-ordered, so consecutive calls on one stream may share it.  A call that is being captured gets a buffer of its own
-    from the graph's memory: the shared one is replaced when a later call needs more, and replays would go on writing to it."""
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-    key = (torch.device(device).index, stream_handle())
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(int(nbytes), 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    """Scratch of at least nbytes for one call on the current stream: the call's own, from torch's allocator (in stream order, also
+    under capture).  Not kept between calls: a call makes several launches, and threads that share a stream (autograd runs
+    backward passes on its own) get theirs in between; and a large graph's would never be given back."""
+    return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
 def status_message(bits: int) -> str:

@@ -483,8 +483,7 @@ def aggregate(indptr, indices, feat, mode="sum", zero_policy="self", row_norm=No
             ws, ws_bytes = None, 0
             if n_entries >= L.AGG_SEG_MIN_ENTRIES:
                 ws_bytes = L.lib().fgl_aggregate_workspace_bytes(n_entries, D, m, longest_known)
-                # (the allocator's own, not the stream's shared scratch: a captured call must not see that one grow)
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+                ws = L.workspace(ws_bytes, dev) if ws_bytes else None
             L.check(L.lib().fgl_aggregate_ws(L.ptr(indptr), idx_ptr, n, L.ptr(n_rows_dev), L.ptr(feat), int(feat.stride(0)), D,
                                              L.F32 if feat.dtype == torch.float32 else L.BF16, m, z, L.ptr(row_norm),
                                              L.ptr(col_norm), L.ptr(edge_weight), int(n_heads), L.ptr(edge_index),

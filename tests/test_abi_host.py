@@ -49,6 +49,11 @@ def test_counting_into_no_counters_asks_for_no_scratch():
     assert fastgl.lib().fgl_cal_deg_workspace_bytes(1 << 16, 1) > 0
 
 
+def test_scratch_is_the_calls_own():
+    a, b = L.workspace(1000, "cpu"), L.workspace(1000, "cpu")
+    assert a.data_ptr() != b.data_ptr() and a.numel() >= 1000 and L.workspace(0, "cpu").numel() > 0
+
+
 def test_static_scratch_holds_the_workspace_of_its_largest_call():
     # fgl_sample_node_static's 16 MiB array against what the workspace formula asks for at the stated seed limit
     lib = fastgl.lib()
