@@ -282,13 +282,13 @@ def _watched(t):
 
 class _Linear(nn.Linear):
     """``nn.Linear`` with ``_LinearFunction``'s backward pass for the inputs it is made for: plain matrices on the GPU in the
-    weight's own type (fp32 or bf16), outside autocast, tracing, compilation and forward-mode differentiation (``_LinearFunction`` has
-    no rule for those; the operator has)."""
+    weight's own type (fp32 or bf16), outside autocast, tracing, compilation, modes that follow the operators and forward-mode
+    differentiation (``_LinearFunction`` has no rule for those; the operator has)."""
 
     def forward(self, x):
         if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()) or \
                 _watched(x) or _watched(self.weight) or (self.bias is not None and _watched(self.bias)) or torch.jit.is_tracing() or torch.compiler.is_compiling() or \
-                torch.autograd.forward_ad._current_level >= 0:
+                torch.autograd.forward_ad._current_level >= 0 or ops._followed():
             return super().forward(x)
         if not torch.is_grad_enabled():
             return ops.row_product(x, self.weight, transposed=True, bias=self.bias)
@@ -362,7 +362,7 @@ class GATConv(nn.Module):
         products and sums that it replaces (105 K rows of 4 x 64 columns: 200 us)."""
         if (feat_src.is_cuda and feat_src.dtype == torch.float32 and self.attn_l.dtype == torch.float32 and self.attn_r.dtype == torch.float32
                 and feat_src.is_contiguous() and self.attn_l.is_contiguous() and self.attn_r.is_contiguous() and self.attn_l.size(0) == 1
-                and self.attn_r.size(0) == 1):
+                and self.attn_r.size(0) == 1 and not ops._followed()):
             return ops.head_scores(feat_src, self.attn_l, self.attn_r, dst_nodes)
         feat_src = feat_src.view(-1, self.num_heads, self.out_feats)
         return (feat_src * self.attn_l).sum(dim=-1).contiguous(), (feat_src[:dst_nodes] * self.attn_r).sum(dim=-1).contiguous()

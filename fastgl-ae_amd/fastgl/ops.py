@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes as C
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib as L
 
@@ -333,6 +334,14 @@ def backward_gat(edge_ptr, edge_data, src_edges, d_input, src_nodes, num_heads):
 # ---------------------------------------------------------------------------------------
 # extensions
 # ---------------------------------------------------------------------------------------
+def _followed():
+    """Whether something follows torch's operators as they are called (a tracer, a FLOP counter or another dispatch or function mode)
+    and would miss a product that does not go through one.  A default device is a function mode too, and follows nothing."""
+    if torch._C._len_torch_dispatch_stack() > 0:
+        return True
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 def _splits_k(k, m, n):
     """Whether ``weight_grad`` forms its product with the library's k-splitting kernel.  A weight gradient has a few output
     tiles and a long k, where a GEMM that parallelises over tiles leaves the chip idle (100 x 256 outputs, k = 105 K: fp32
@@ -342,7 +351,7 @@ def _splits_k(k, m, n):
 
 
 def _forms_row_product(a, b, transposed, m, k, n):
-    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call, no
+    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it, no
     autocast to change the types, and a size where it gains.  The library looks for a kernel on every call with sizes it has not just
     seen -- 74 us of the host's time against 13 -- which is what a product of a mini-batch takes; on the GPU the two are
     alike (us, library / here: fp32 1000 x 100 x 64 21 / 13, 8192 x 602 x 256 29 / 29, 107 K x 256 x 256 140 / 149, bf16 107 K x 100 x 256
@@ -350,7 +359,7 @@ def _forms_row_product(a, b, transposed, m, k, n):
     the host takes, and there the library's tiles through LDS are ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; 20 K x 512 x 512
     89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all)."""
     return (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
-            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and not torch.is_autocast_enabled() and
+            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and not torch.is_autocast_enabled() and not _followed() and
             a.stride(1) == 1 and a.stride(0) >= k and b.stride(1) == 1 and b.stride(0) >= b.size(1) and
             (a.dtype == torch.float32 or (a.stride(0) % 2 == 0 and a.data_ptr() % 4 == 0 and
                                           (not transposed or (b.stride(0) % 2 == 0 and b.data_ptr() % 4 == 0)))))
@@ -382,7 +391,7 @@ def weight_grad(a, b, column_sums=False):
     k, m, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
     if not (a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
             not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and  # (a graph is being built: torch's product has a gradient)
-            not torch.is_autocast_enabled() and
+            not torch.is_autocast_enabled() and not _followed() and
             a.stride(1) == 1 and b.stride(1) == 1 and m <= a.stride(0) < 1 << 24 and n <= b.stride(0) < 1 << 24 and
             m < 1 << 16 and n < 1 << 16 and b.size(0) == k and
             _splits_k(k, m, n)):

@@ -1,0 +1,54 @@
+"""Products of the layers while something follows torch's operators: those stay torch's own then."""
+import pytest
+import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils.flop_counter import FlopCounterMode
+
+import fastgl
+from fastgl import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def layer(cuda):
+    torch.manual_seed(0)
+    return fastgl.conv._Linear(20, 7).to(cuda)
+
+
+def test_dispatch_modes_see_the_products(cuda, layer):
+    x = torch.randn(33, 20, device=cuda)
+    with torch.no_grad():
+        graph = make_fx(lambda t: layer(t))(x)  # (real tensors under a dispatch mode)
+        other = torch.randn(33, 20, device=cuda)
+        assert torch.allclose(graph(other), torch.nn.functional.linear(other, layer.weight, layer.bias), rtol=1e-5, atol=1e-5)
+    w = torch.randn(20, 7, device=cuda)
+    with FlopCounterMode(display=False) as count:
+        ops.row_product(x, w)
+        ops.weight_grad(x, x[:, :5])
+    assert count.get_total_flops() == 2 * 33 * 20 * 7 + 2 * 33 * 20 * 5
+    x.requires_grad_()
+    with FlopCounterMode(display=False) as count:
+        layer(x).square().sum().backward()
+    assert count.get_total_flops() == 3 * 2 * 33 * 20 * 7
+
+
+def test_function_modes_see_the_layer(cuda, layer):
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        layer(torch.randn(33, 20, device=cuda))
+    assert torch.nn.functional.linear in seen
+
+
+def test_a_default_device_follows_nothing(cuda):
+    assert not ops._followed()
+    with torch.device("cpu"):
+        assert not ops._followed()
+    with FlopCounterMode(display=False):
+        assert ops._followed()
