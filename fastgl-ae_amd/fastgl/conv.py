@@ -286,8 +286,10 @@ class _Linear(nn.Linear):
     differentiation (``_LinearFunction`` has no rule for those; the operator has)."""
 
     def forward(self, x):
-        if not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()) or \
-                _watched(x) or _watched(self.weight) or (self.bias is not None and _watched(self.bias)) or torch.jit.is_tracing() or torch.compiler.is_compiling() or \
+        # (compilation and tracing first: the compiler cannot look into the other questions)
+        if torch.compiler.is_compiling() or torch.jit.is_tracing() or \
+                not (x.is_cuda and x.dim() == 2 and x.dtype == self.weight.dtype and x.dtype in ops._FEAT and not torch.is_autocast_enabled()) or \
+                _watched(x) or _watched(self.weight) or (self.bias is not None and _watched(self.bias)) or \
                 torch.autograd.forward_ad._current_level >= 0 or ops._followed():
             return super().forward(x)
         if not torch.is_grad_enabled():

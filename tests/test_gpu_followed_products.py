@@ -52,3 +52,11 @@ def test_a_default_device_follows_nothing(cuda):
         assert not ops._followed()
     with FlopCounterMode(display=False):
         assert ops._followed()
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_compiled(cuda, layer, grad):
+    x = torch.randn(33, 20, device=cuda)
+    with torch.set_grad_enabled(grad):
+        got = torch.compile(layer, fullgraph=True, backend="eager")(x)
+        assert torch.allclose(got, torch.nn.functional.linear(x, layer.weight, layer.bias), rtol=1e-5, atol=1e-5)
