@@ -276,8 +276,8 @@ class _LinearFunction(torch.autograd.Function):
 
 
 def _watched(t):
-    """Whether something follows the operators that ``t`` goes through: a tensor subclass, a transform of ``torch.func``."""
-    return type(t) not in (torch.Tensor, nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+    """Whether the operators that ``t`` goes through are its class's business (for what else may follow them see ``ops._followed``)."""
+    return type(t) not in (torch.Tensor, nn.Parameter)
 
 
 class _Linear(nn.Linear):

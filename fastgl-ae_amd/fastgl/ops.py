@@ -334,12 +334,27 @@ def backward_gat(edge_ptr, edge_data, src_edges, d_input, src_nodes, num_heads):
 # ---------------------------------------------------------------------------------------
 # extensions
 # ---------------------------------------------------------------------------------------
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms = torch._C._functorch.peek_interpreter_stack
+
+
 def _followed():
-    """Whether something follows torch's operators as they are called (a tracer, a FLOP counter or another dispatch or function mode)
-    and would miss a product that does not go through one.  A default device is a function mode too, and follows nothing."""
-    if torch._C._len_torch_dispatch_stack() > 0:
+    """Whether something follows torch's operators as they are called and would miss a product that does not go through one: a
+    transform of ``torch.func``, a tracer, a FLOP counter or another dispatch or function mode.  (A default device is a function mode
+    too, and follows nothing.)"""
+    if _dispatch_modes() > 0 or _transforms() is not None:
         return True
-    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+    n = _function_modes()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
+
+
+def _addresses(a, b):
+    """Where the two tensors lie, or None if one has no memory of its own: the gradients that ``torch.autograd.grad`` hands to
+    backward passes with ``is_grads_batched`` (and ``jacobian`` with ``vectorize``) look like matrices, but only torch's operators take them."""
+    try:
+        return a.data_ptr(), b.data_ptr()
+    except RuntimeError:
+        return None
 
 
 def _splits_k(k, m, n):
@@ -357,12 +372,17 @@ def _forms_row_product(a, b, transposed, m, k, n):
     alike (us, library / here: fp32 1000 x 100 x 64 21 / 13, 8192 x 602 x 256 29 / 29, 107 K x 256 x 256 140 / 149, bf16 107 K x 100 x 256
     30 / 24, 107 K x 256 x 256 30 / 39 and, with a transposed weight, 27 / 53).  Larger ones keep the GPU busy for longer than
     the host takes, and there the library's tiles through LDS are ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; 20 K x 512 x 512
-    89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all)."""
-    return (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
-            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and not torch.is_autocast_enabled() and not _followed() and
-            a.stride(1) == 1 and a.stride(0) >= k and b.stride(1) == 1 and b.stride(0) >= b.size(1) and
-            (a.dtype == torch.float32 or (a.stride(0) % 2 == 0 and a.data_ptr() % 4 == 0 and
-                                          (not transposed or (b.stride(0) % 2 == 0 and b.data_ptr() % 4 == 0)))))
+    89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all).
+    Returns the operands' addresses and row strides if so, else None."""
+    if not (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
+            0 < n <= 65536 and a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
+            not torch.is_autocast_enabled() and not _followed()):
+        return None
+    (lda, unit_a), (ldb, unit_b), at = a.stride(), b.stride(), _addresses(a, b)
+    if (at is not None and unit_a == 1 and lda >= k and unit_b == 1 and ldb >= b.size(1) and
+            (a.dtype == torch.float32 or (lda % 2 == 0 and at[0] % 4 == 0 and (not transposed or (ldb % 2 == 0 and at[1] % 4 == 0))))):
+        return at[0], lda, at[1], ldb
+    return None
 
 
 def row_product(a, b, transposed=False, bias=None):
@@ -371,16 +391,16 @@ def row_product(a, b, transposed=False, bias=None):
     if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(1 if transposed else 0):
         raise RuntimeError("row_product: shapes %s and %s do not match" % (tuple(a.shape), tuple(b.shape)))
     m, k, n = int(a.size(0)), int(a.size(1)), int(b.size(0 if transposed else 1))
-    if not (_forms_row_product(a, b, transposed, m, k, n) and
-            (bias is None or (bias.device == a.device and bias.dtype == a.dtype and bias.is_contiguous() and bias.numel() == n and
-                              not (torch.is_grad_enabled() and bias.requires_grad)))):
+    at = _forms_row_product(a, b, transposed, m, k, n)
+    if at is None or not (bias is None or (bias.device == a.device and bias.dtype == a.dtype and bias.is_contiguous() and bias.numel() == n and
+                                           not (torch.is_grad_enabled() and bias.requires_grad))):
         w = b.transpose(0, 1) if transposed else b
         return torch.mm(a, w) if bias is None else torch.addmm(bias, a, w)
     dev = a.device
     with _on_device(dev):
         out = torch.empty((m, n), dtype=a.dtype, device=dev)
-        L.check(L.lib().fgl_row_product(L.ptr(a), a.stride(0), L.ptr(b), b.stride(0), int(transposed), m, k, n,
-                                        L.F32 if a.dtype == torch.float32 else L.BF16, L.ptr(bias), L.ptr(out), n, L.stream_handle()))
+        L.check(L.lib().fgl_row_product(*at, int(transposed), m, k, n, L.F32 if a.dtype == torch.float32 else L.BF16, L.ptr(bias), out.data_ptr(), n,
+                                        L.stream_handle()))
     return out
 
 
@@ -388,11 +408,12 @@ def weight_grad(a, b, column_sums=False):
     """``a^T b`` for ``a`` [k, m] and ``b`` [k, n]: a dense layer's weight gradient from its input rows and the gradient of
     its output (fp32 sums, result in the operands' dtype).  ``column_sums=True``: ``(a^T b, a.sum(0))``, with ``a`` the
     gradient of the output the transposed weight gradient and the bias gradient of the layer."""
-    k, m, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
-    if not (a.is_cuda and a.device == b.device and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
+    (k, m), n = a.shape, int(b.size(1))
+    (lda, unit_a), (ldb, unit_b), at = a.stride(), b.stride(), _addresses(a, b)
+    if not (a.is_cuda and a.get_device() == b.get_device() and a.dtype == b.dtype and a.dtype in _FEAT and k > 0 and m > 0 and n > 0 and
             not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and  # (a graph is being built: torch's product has a gradient)
-            not torch.is_autocast_enabled() and not _followed() and
-            a.stride(1) == 1 and b.stride(1) == 1 and m <= a.stride(0) < 1 << 24 and n <= b.stride(0) < 1 << 24 and
+            not torch.is_autocast_enabled() and not _followed() and at is not None and
+            unit_a == 1 and unit_b == 1 and m <= lda < 1 << 24 and n <= ldb < 1 << 24 and
             m < 1 << 16 and n < 1 << 16 and b.size(0) == k and
             _splits_k(k, m, n)):
         d_w = torch.mm(a.transpose(0, 1), b)
@@ -403,9 +424,8 @@ def weight_grad(a, b, column_sums=False):
         d_w = torch.empty((m, n), dtype=a.dtype, device=dev)
         sums = torch.empty(m, dtype=a.dtype, device=dev) if column_sums else None
         ws = L.workspace(lib.fgl_weight_grad_workspace_bytes(k, m, n), dev)
-        L.check(lib.fgl_weight_grad(L.ptr(a), int(a.stride(0)), L.ptr(b), int(b.stride(0)), k, m, n,
-                                    L.F32 if a.dtype == torch.float32 else L.BF16, L.ptr(d_w), n, L.ptr(sums), L.ptr(ws), ws.numel(),
-                                    L.stream_handle()))
+        L.check(lib.fgl_weight_grad(at[0], lda, at[1], ldb, k, m, n, L.F32 if a.dtype == torch.float32 else L.BF16, d_w.data_ptr(), n, L.ptr(sums),
+                                    ws.data_ptr(), ws.numel(), L.stream_handle()))
     return (d_w, sums) if column_sums else d_w
 
 

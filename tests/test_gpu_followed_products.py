@@ -60,3 +60,33 @@ def test_compiled(cuda, layer, grad):
     with torch.set_grad_enabled(grad):
         got = torch.compile(layer, fullgraph=True, backend="eager")(x)
         assert torch.allclose(got, torch.nn.functional.linear(x, layer.weight, layer.bias), rtol=1e-5, atol=1e-5)
+
+
+def test_batched_gradients_of_the_layer(cuda, layer):
+    x = torch.randn(6, 20, device=cuda, requires_grad=True)
+    y = layer(x)
+    v = torch.eye(42, device=cuda).view(42, 6, 7)
+    got = torch.autograd.grad(y, (x, layer.weight, layer.bias), v, is_grads_batched=True)
+    want = torch.autograd.grad(torch.nn.functional.linear(x, layer.weight, layer.bias), (x, layer.weight, layer.bias), v, is_grads_batched=True)
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["gcn", "gin"])
+def test_batched_gradients_of_a_first_layer(cuda, kind):
+    edge_ptr, edge_src = fastgl.graph.rmat_csr(2000, 20000, seed=3, device=cuda)
+    sampler = fastgl.FusedMapSampler([3], rng_seed=1).set_graph(edge_ptr, edge_src)
+    _, _, (block,) = sampler.sample_blocks(None, torch.arange(5, dtype=torch.int32, device=cuda) * 31)
+    x = torch.randn(block.num_src_nodes(), 8, device=cuda)
+    if kind == "gcn":
+        layer = fastgl.GCNConv(8, 3, weight=True).to(cuda)
+        layer.order = "gather_first"
+        y = layer(block.edge_ptr, block.src_local, None, None, block.num_dst_nodes(), x, 3, block)
+    else:
+        layer = fastgl.GINConv(8, 3, weight=True).to(cuda)
+        y = layer(block.edge_ptr, block.src_local, block.num_dst_nodes(), x, 3, block)
+    v = torch.eye(y.numel(), device=cuda).view(-1, *y.shape)
+    (got,) = torch.autograd.grad(y, (layer.weights,), v, is_grads_batched=True, retain_graph=True)
+    for i in (0, y.numel() - 1):
+        (want,) = torch.autograd.grad(y, (layer.weights,), v[i], retain_graph=True)
+        assert torch.allclose(got[i], want, rtol=1e-5, atol=1e-5)
