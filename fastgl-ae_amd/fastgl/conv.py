@@ -371,7 +371,7 @@ class GATConv(nn.Module):
 
     def forward(self, graph, input_feat, neighbor_num):
         dst_nodes = graph.num_dst_nodes()
-        feat_src = self.fc(input_feat)
+        feat_src = self.fc(input_feat).reshape(-1, self.out_feats * self.num_heads)  # (any leading shape of the input)
         edge_ptr, src_edges = (graph.edge_ptr, graph.src_local) if isinstance(graph, Block) else _block_csr(graph)[:2]
         # u_add_v + leaky_relu + edge_softmax (DGL calls in the reference, GraphConv.py:265-272) in one launch.
         # No gradient reaches the coefficients (the aggregation's backward returns none for them, as in the
@@ -380,7 +380,6 @@ class GATConv(nn.Module):
             el, er = self._scores(feat_src.detach(), dst_nodes)
             alpha = ops.edge_softmax(edge_ptr, src_edges, el, er, self.leaky_relu.negative_slope, n_rows=dst_nodes)
             edge_data = self.attn_drop(alpha).contiguous()
-        feat_src = feat_src.view(-1, self.out_feats * self.num_heads)
         transposed = graph if isinstance(graph, Block) and torch.is_grad_enabled() else None
         return MA_Function_GAT.apply(edge_ptr, edge_data, src_edges, None, dst_nodes, feat_src, self.num_heads,
                                      neighbor_num, transposed)

@@ -3,6 +3,7 @@ vectors, rows that do not fill a group of four, no destination rows and all of t
 import pytest
 import torch
 
+import fastgl
 from fastgl import ops
 
 pytestmark = pytest.mark.gpu
@@ -32,3 +33,24 @@ def test_refuses_shapes_that_do_not_match(cuda):
         ops.head_scores(x[:, :8].contiguous(), a, a, 5)
     with pytest.raises(RuntimeError):
         ops.head_scores(x.cpu(), a, a, 5)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_layer_takes_any_leading_shape(cuda, grad):
+    edge_ptr, edge_src = fastgl.graph.rmat_csr(2000, 20000, seed=3, device=cuda)
+    sampler = fastgl.FusedMapSampler([5], rng_seed=1).set_graph(edge_ptr, edge_src)
+    _, _, (block,) = sampler.sample_blocks(None, torch.arange(40, dtype=torch.int32, device=cuda) * 31)
+    n = block.num_src_nodes()
+    layer = fastgl.GATConv(12, 8, num_heads=2).to(cuda)
+    x = torch.randn(n, 12, device=cuda)
+    with torch.set_grad_enabled(grad):
+        want = layer(block, x, 5)
+        for shape in ((n, 1, 12), (1, n, 12)):
+            assert torch.allclose(layer(block, x.view(shape), 5), want, rtol=1e-5, atol=1e-5)
+
+
+def test_layer_takes_a_single_row_as_a_vector(cuda):
+    block = fastgl.Block(torch.tensor([0, 1], dtype=torch.int32, device=cuda), torch.zeros(1, dtype=torch.int32, device=cuda), 1, 1)
+    layer = fastgl.GATConv(12, 8, num_heads=2).to(cuda)
+    x = torch.randn(12, device=cuda)
+    assert torch.allclose(layer(block, x, 1), layer(block, x[None], 1), rtol=1e-5, atol=1e-5)
