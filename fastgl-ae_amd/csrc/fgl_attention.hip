@@ -127,7 +127,7 @@ FGL_EXPORT int fgl_head_scores(const float* d_x, int64_t ldx, int64_t n_rows, in
                                const float* d_attn_r, float* d_el, float* d_er, void* stream)
 {
     FGL_REQUIRE(n_rows >= 0 && n_er >= 0 && n_er <= n_rows, "head_scores: row counts %lld, %lld", (long long)n_rows, (long long)n_er);
-    FGL_REQUIRE(n_heads >= 1 && n_heads <= 1024 && width >= 1, "head_scores: %d heads of %d columns", n_heads, width);
+    FGL_REQUIRE(n_heads >= 1 && width >= 1, "head_scores: %d heads of %d columns", n_heads, width);
     FGL_REQUIRE(ldx >= (int64_t)n_heads * width, "head_scores: row stride smaller than the row length");
     if (n_rows == 0) return FGL_OK;
     FGL_REQUIRE(d_x && d_attn_l && d_attn_r && d_el && (d_er || n_er == 0), "head_scores: null pointer");

@@ -9,7 +9,7 @@ from fastgl import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("heads,width", [(1, 1), (1, 16), (4, 64), (4, 37), (3, 66), (8, 5), (2, 300), (1, 172)])
+@pytest.mark.parametrize("heads,width", [(1, 1), (1, 16), (4, 64), (4, 37), (3, 66), (8, 5), (2, 300), (1, 172), (1500, 2)])
 @pytest.mark.parametrize("n,n_dst", [(1, 0), (1, 1), (3, 2), (4, 4), (1001, 250), (4099, 4097)])
 def test_matches_float64(cuda, heads, width, n, n_dst):
     gen = torch.Generator(device=cuda).manual_seed(heads * 1000 + width + n)
