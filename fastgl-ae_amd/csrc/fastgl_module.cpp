@@ -145,7 +145,8 @@ torch::Tensor weight_grad(const torch::Tensor& a, const torch::Tensor& b)
     // (a graph is being built, or autocast picks the types: torch's product knows about both)
     const bool followed = (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) || at::autocast::is_autocast_enabled(at::kCUDA);
     if (!splits_k || followed || k == 0 || m == 0 || n == 0 || b.size(0) != k || a.scalar_type() != b.scalar_type() || a.device() != b.device() ||
-        m >= (1 << 16) || n >= (1 << 16))
+        m >= (1 << 16) || n >= (1 << 16) || a.stride(0) < m || b.stride(0) < n ||  // (a single row is contiguous whatever its row stride says)
+        a.stride(0) >= (1 << 24) || b.stride(0) >= (1 << 24))
         return torch::mm(a.transpose(0, 1), b);
     auto out = torch::empty({m, n}, a.options());
     auto ws = scratch(fgl_weight_grad_workspace_bytes(k, (int)m, (int)n), a);

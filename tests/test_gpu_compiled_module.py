@@ -156,3 +156,16 @@ def test_weight_gradients_follow_grad_mode_and_autocast(ext, cuda):
     assert d_w.requires_grad and rel_err(d_w.detach(), want.cpu().numpy()) < 1e-5
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert fastgl.ops.weight_grad(x, d).dtype == torch.bfloat16
+
+
+@pytest.mark.parametrize("stride", [1, 1 << 24])
+def test_weight_gradient_of_a_single_row(ext, cuda, stride):
+    """A single row is contiguous whatever its row stride says."""
+    ptr = torch.tensor([0, 1], dtype=torch.int32, device=cuda)
+    idx = torch.zeros(1, dtype=torch.int32, device=cuda)
+    x, g, w = (torch.randn(s, device=cuda) for s in (20, 7, (20, 7)))
+    x, g = x.as_strided((1, 20), (stride, 1)), g.as_strided((1, 7), (stride, 1))
+    assert x.is_contiguous() and g.is_contiguous()
+    one = torch.ones(1, dtype=torch.int32, device=cuda)
+    for d_x, d_w in (ext.backward_gin(ptr, idx, g, w, x, 1), ext.backward_gcn(ptr, idx, one, one, torch.cat([g[0]]).view(1, 7), w, x)):
+        assert torch.allclose(d_w, x.t() @ g, rtol=1e-5, atol=1e-5) and torch.allclose(d_x, g @ w.t(), rtol=1e-5, atol=1e-5)
