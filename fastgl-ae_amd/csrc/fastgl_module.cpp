@@ -10,6 +10,7 @@
 // sizes (the reference reads its sizes back at the same points: sample.cu:202, id_map.cu:454,491).
 #include <torch/extension.h>
 #include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
 
@@ -142,8 +143,9 @@ torch::Tensor weight_grad(const torch::Tensor& a, const torch::Tensor& b)
 {
     const int64_t k = a.size(0), m = a.size(1), n = b.size(1);
     const bool splits_k = m * n <= 65536 || k * k >= 256 * m * n;
-    // (a graph is being built, or autocast picks the types: torch's product knows about both)
-    const bool followed = (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) || at::autocast::is_autocast_enabled(at::kCUDA);
+    // (a graph is being built, autocast picks the types, or a tracer or counter looks on: torch's product knows about them)
+    const bool followed = (at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad())) || at::autocast::is_autocast_enabled(at::kCUDA) ||
+                          c10::impl::dispatch_mode_enabled();
     if (!splits_k || followed || k == 0 || m == 0 || n == 0 || b.size(0) != k || a.scalar_type() != b.scalar_type() || a.device() != b.device() ||
         m >= (1 << 16) || n >= (1 << 16) || a.stride(0) < m || b.stride(0) < n ||  // (a single row is contiguous whatever its row stride says)
         a.stride(0) >= (1 << 24) || b.stride(0) >= (1 << 24))

@@ -169,3 +169,13 @@ def test_weight_gradient_of_a_single_row(ext, cuda, stride):
     one = torch.ones(1, dtype=torch.int32, device=cuda)
     for d_x, d_w in (ext.backward_gin(ptr, idx, g, w, x, 1), ext.backward_gcn(ptr, idx, one, one, torch.cat([g[0]]).view(1, 7), w, x)):
         assert torch.allclose(d_w, x.t() @ g, rtol=1e-5, atol=1e-5) and torch.allclose(d_x, g @ w.t(), rtol=1e-5, atol=1e-5)
+
+
+def test_dispatch_modes_see_the_weight_gradient(ext, cuda):
+    from torch.utils.flop_counter import FlopCounterMode
+    ptr = torch.arange(6, dtype=torch.int32, device=cuda)
+    idx = torch.arange(5, dtype=torch.int32, device=cuda)
+    x, g, w = (torch.randn(s, device=cuda) for s in ((5, 20), (5, 7), (20, 7)))
+    with FlopCounterMode(display=False) as count:
+        ext.backward_gin(ptr, idx, g, w, x, 5)
+    assert count.get_total_flops() == 2 * 2 * 5 * 20 * 7  # the input's gradient and the weight's
