@@ -263,6 +263,19 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
     cur.multiply(acc);
     next.multiply(acc);
 
+    // Every sum leaves the accumulators here, before the branches around the stores: the empty statement keeps the compiler from moving
+    // the additions behind them, which it did.  (fp32 107 K x 256 x 256: 149 us with them behind, 144 here; other sizes alike.)
+#pragma unroll
+    for (int i = 0; i < VA; ++i)
+#pragma unroll
+        for (int t = 0; t < VB; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float s = acc[i * VB + t][r] + add[t];
+                asm volatile("" : "+v"(s));
+                acc[i * VB + t][r] = s;
+            }
+
     // accumulator register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of its 32x32 tile
 #pragma unroll
     for (int i = 0; i < VA; ++i)
@@ -271,7 +284,7 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
             const int64_t row = row0 + 32 * i + 8 * (r / 4) + 4 * half + r % 4;
             float v[VB];
 #pragma unroll
-            for (int t = 0; t < VB; ++t) v[t] = acc[i * VB + t][r] + add[t];
+            for (int t = 0; t < VB; ++t) v[t] = acc[i * VB + t][r];
             if (row < g.m) rp_store<T, VB>(static_cast<T*>(g.c) + row * g.ldc + col, v);
         }
 }
