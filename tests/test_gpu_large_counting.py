@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import fastgl
+from fastgl import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -22,13 +23,25 @@ def _ids(n, bins, gen, device, hub):
 @pytest.mark.parametrize("hub", [False, True])
 @pytest.mark.parametrize("n,bins", [((1 << 16) - 1, 1000), (1 << 16, 1 << 15), (1 << 16, (1 << 15) + 1), ((1 << 18) - 1, 1000), (1 << 18, 16384), ((1 << 18) + 3, 16385), (M + 5, 1 << 19), (M, (1 << 19) + 1),
                                     (300_001, 1), (4 * M - 1, 300_000), (4 * M, 1), (4 * M, 2048), (4 * M + 8191, 2049),
-                                    (5 * M + 77, 3_000_001), (4 * M, 5 * M)])
+                                    (5 * M + 77, 3_000_001), (4 * M, 5 * M), (M, 8 * M + 9)])
 def test_cal_deg(cuda, n, bins, hub):
     gen = torch.Generator(device=cuda).manual_seed(n + bins)
     ids = _ids(n, bins, gen, cuda, hub)
     got = fastgl.cal_deg(ids, bins)
     valid = ids[(ids >= 0) & (ids < bins)].long()
     assert torch.equal(got.long(), torch.bincount(valid, minlength=bins))
+
+
+@pytest.mark.parametrize("n_max,n,bins", [(1 << 16, 60_000, 1 << 15), (1 << 18, 5, 16385), (1 << 18, 0, 1000), (4 * M, M + 1, 300_000), (4 * M, 0, 2048)])
+def test_cal_deg_of_a_count_on_the_device(cuda, n_max, n, bins):
+    gen = torch.Generator(device=cuda).manual_seed(n_max + n)
+    ids = _ids(n_max, bins, gen, cuda, False)
+    lib = fastgl.lib()
+    d_n = torch.tensor([n], dtype=torch.int32, device=cuda)
+    got = torch.full((bins,), -7, dtype=torch.int32, device=cuda)
+    ws = L.workspace(lib.fgl_cal_deg_workspace_bytes(n_max, bins), cuda)
+    L.check(lib.fgl_cal_deg_ws(L.ptr(ids), n_max, L.ptr(d_n), L.ptr(got), bins, L.ptr(ws), ws.numel(), L.stream_handle()))
+    assert torch.equal(got.long(), torch.bincount(ids[:n].long(), minlength=bins))
 
 
 @pytest.mark.parametrize("n", [(1 << 16) - 1, 1 << 16, 1 << 18, 4 * M])
@@ -65,7 +78,8 @@ def _lengths(kind, gen):
 
 @pytest.mark.parametrize("edge_ids", [False, True])
 @pytest.mark.parametrize("kind,n_cols", [("one", 1), ("fanout", 3000), ("hub", 70_000), ("gaps", 500), ("large", 1), ("large", 2_500_000),
-                                         ("large", 4096)])
+                                         ("large", 4096), ("large", 8 * M + 9),  # (buckets of 2^13 columns)
+                                         ("large", 16 * M + 5)])                 # (too wide for buckets: eight counters a column)
 def test_block_transpose(cuda, kind, n_cols, edge_ids):
     gen = torch.Generator().manual_seed(n_cols)
     lengths = _lengths(kind, gen)
@@ -111,3 +125,40 @@ def test_block_transpose_of_a_slice(cuda, first, lengths, n_cols, sorted_rows):
     e = t_edge.long()
     assert torch.equal(torch.sort(e).values, torch.arange(nnz, device=cuda))
     assert torch.equal(cols.long()[e], torch.repeat_interleave(torch.arange(n_cols, device=cuda), counts)) and torch.equal(rows[e], t_idx.long())
+
+
+@pytest.mark.parametrize("rows,cols,nnz_max", [(5000, 3000, M), (4999, 1, M + 7), (0, 3000, M), (5000, 3000, M - 1)])
+def test_block_transpose_of_sizes_on_the_device(cuda, rows, cols, nnz_max):
+    """A block whose sizes the host knows bounds of only: from 2^20 entries on with eight counters a column, below with one."""
+    print("device sizes", rows, cols, nnz_max, flush=True)
+    gen = torch.Generator().manual_seed(rows + nnz_max)
+    rows_max, cols_max = 6000, 4000
+    lens = torch.randint(0, 300, (rows,), generator=gen)
+    if rows:
+        lens[rows // 2] = 50_000  # a hub
+    ptr = torch.full((rows_max + 1,), -1, dtype=torch.int32, device=cuda)  # (past the actual rows: never read)
+    ptr[:rows + 1] = _csr(lens, cuda)
+    nnz = int(lens.sum())
+    assert nnz <= nnz_max
+    idx = torch.full((nnz_max,), -1, dtype=torch.int32)
+    idx[:nnz] = torch.randint(0, cols, (nnz,), generator=gen, dtype=torch.int32)
+    idx[:nnz][torch.rand(nnz, generator=gen) < 0.1] = cols // 3
+    idx = idx.to(cuda)
+    d_rows, d_cols = (torch.tensor([v], dtype=torch.int32, device=cuda) for v in (rows, cols))
+    t_ptr = torch.full((cols_max + 1,), -7, dtype=torch.int32, device=cuda)
+    t_idx, t_edge = (torch.full((nnz_max,), -7, dtype=torch.int32, device=cuda) for _ in range(2))
+    longest = torch.full((1,), -7, dtype=torch.int32, device=cuda)
+    lib = fastgl.lib()
+    ws = L.workspace(lib.fgl_block_transpose_workspace_bytes(cols_max, nnz_max, 0), cuda)
+    L.check(lib.fgl_block_transpose(L.ptr(ptr), L.ptr(idx), rows_max, L.ptr(d_rows), cols_max, L.ptr(d_cols), nnz_max, L.ptr(t_ptr), L.ptr(t_idx),
+                                    L.ptr(t_edge), L.ptr(longest), 0, L.ptr(ws), ws.numel(), L.stream_handle()))
+    of_row = torch.repeat_interleave(torch.arange(rows), lens).to(cuda)
+    counts = torch.bincount(idx[:nnz].long(), minlength=cols)
+    assert int(t_ptr[0]) == 0 and torch.equal(t_ptr[1:cols + 1].long(), torch.cumsum(counts, 0))
+    top = int(counts.max())
+    assert int(longest) == top if top > 32 else int(longest) <= 32
+    e = t_edge[:nnz].long()
+    assert torch.equal(torch.sort(e).values, torch.arange(nnz, device=cuda))
+    assert torch.equal(idx[:nnz].long()[e], torch.repeat_interleave(torch.arange(cols, device=cuda), counts))
+    assert torch.equal(of_row[e], t_idx[:nnz].long())
+    assert bool((t_idx[nnz:] == -7).all()) and bool((t_edge[nnz:] == -7).all())
