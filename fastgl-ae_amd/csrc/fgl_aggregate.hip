@@ -1439,10 +1439,11 @@ size_t transpose_workspace_bytes(int64_t n_cols_max, int64_t n_edges_max, int so
 // ---- dispatch ----------------------------------------------------------------------
 // Which lane mapping the calling thread's last fgl_aggregate call chose (for benchmarks and bug reports).
 static thread_local char g_mapping[96] = "";
-static void note_mapping(const char* kernel, int lpr, int extra, bool second_pass)
+static void note_mapping(const char* kernel, int lpr, int extra, bool second_pass, bool segments = false)
 {
     snprintf(g_mapping, sizeof(g_mapping), "%s lanes/row=%d%s%s", kernel, lpr,
-             extra > 1 ? (extra >= 100 ? " (rows bundled by 4)" : " (groups/row>1)") : "", second_pass ? " + long_rows" : "");
+             extra > 1 ? (extra >= 100 ? " (rows bundled by 4)" : " (groups/row>1)") : "",
+             !second_pass ? "" : segments ? " + segments" : " + long_rows");
 }
 
 // Workgroups of the long-row pass: each looks through an equal share of the row offsets.
@@ -1493,7 +1494,7 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
         return FGL_OK;
       }
     }
-    note_mapping("aggregate_kernel", LPR, 1, second_pass);
+    note_mapping("aggregate_kernel", LPR, 1, second_pass, g.ws != nullptr);
 #define FGL_LAUNCH_MODE(M)                                                                                         \
     do {                                                                                                           \
         hipLaunchKernelGGL((aggregate_kernel<T, VEC, LPR, M>), grid, dim3(kBlock), 0, stream, g);                  \
@@ -1516,7 +1517,7 @@ template <typename T, int VEC>
 static int launch_agg_flat(int mode, bool long_rows_possible, int lanes, bool bundle, hipStream_t stream, AggArgs g)
 {
     g.skip_rows_longer_than = long_rows_possible ? kLongRowEntries : 0x7FFFFFFF;
-    note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible);
+    note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible, g.ws != nullptr);
     const int64_t blocks = ceil_div((bundle ? ceil_div(g.n_rows_max, kBundleRows) : g.n_rows_max) * lanes, kBlock);
     if (blocks > 0x7FFFFFFF) {
         set_error("aggregate: grid too large (%lld workgroups)", (long long)blocks);
@@ -1578,7 +1579,7 @@ template <typename T, int VEC, int LPR>
 static int launch_agg_bundle(int mode, bool long_rows_possible, unsigned gy, hipStream_t stream, AggArgs g)
 {
     g.skip_rows_longer_than = long_rows_possible ? kLongRowEntries : 0x7FFFFFFF;
-    note_mapping("aggregate_bundle_kernel", LPR, 100, long_rows_possible);
+    note_mapping("aggregate_bundle_kernel", LPR, 100, long_rows_possible, g.ws != nullptr);
     const int64_t gx = ceil_div(ceil_div(g.n_rows_max, kBundleRows), kBlock / LPR);
 #define FGL_LAUNCH_BUNDLE(M)                                                                                          \
     do {                                                                                                              \

@@ -54,3 +54,12 @@ def test_the_least_entry_count_is_the_librarys():
     assert L.lib().fgl_aggregate_workspace_bytes(L.AGG_SEG_MIN_ENTRIES - 1, 64, L.AGG_SUM, -1) == 0
     assert L.lib().fgl_aggregate_workspace_bytes(L.AGG_SEG_MIN_ENTRIES, 64, L.AGG_EDGE, -1) == 0
     assert L.lib().fgl_aggregate_workspace_bytes(L.AGG_SEG_MIN_ENTRIES, 64, L.AGG_SUM, 128) == 0
+
+
+@pytest.mark.parametrize("dim", [64, 300])
+def test_the_mapping_names_the_second_pass(dim):
+    ptr, idx, lens = _block(500)
+    x = torch.zeros((500, dim), device=DEV)
+    for kw, want in ((dict(mode="sum"), "segments"), (dict(mode="edge", edge_weight=torch.zeros((idx.numel(), 1), device=DEV)), "long_rows")):
+        ops.aggregate(ptr, idx, x, zero_policy="zeros", **kw)
+        assert L.lib().fgl_aggregate_last_mapping().decode().endswith(" + " + want)
