@@ -207,6 +207,16 @@ def test_traffic_record_is_only_used_while_it_matches(tmp_path, monkeypatch, cap
     assert bench.traffic_from_profile("c3", 800e6) is None
 
 
+def test_tracked_traffic_record_is_of_the_kernel_as_it_is():
+    """The counter summary in profiles/ was taken with the aggregation source that is built now; otherwise bench.py has no traffic to
+    report (after a change to that file: the two counter runs that the summary names)."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("bench_mod", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    assert bench.traffic_from_profile("c3", 829742452.0) is not None
+
+
 def test_size_limits_are_stated_before_anything_is_launched():
     """Sizes that would overflow the library's 32-bit offsets come back as errors with the limit in the message."""
     lib = fastgl.lib()
