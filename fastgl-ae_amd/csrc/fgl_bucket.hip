@@ -300,7 +300,9 @@ static bool count_by_buckets(int64_t n_ids, int64_t n_counters)
 }
 // Transposing (atomics with the fill by entries / buckets): 205 K entries, 200 K columns, uniform 26 / 43; 251 K, 27 K, R-MAT 88 / 72;
 // 434 K, a sampled block 93 / 75; 600 K, 200 K, uniform 47 / 50; 1.15 M, a sampled block 113 / 91; 2.5 M, 100 K, R-MAT 335 / 108;
-// 54 M, 2.4 M, R-MAT 24700 (sixteen lanes per row) / 1550.  Columns of graphs are skewed: the line is where those gain.
+// 54 M, 2.4 M, R-MAT 24700 (sixteen lanes per row) / 1550.  Columns of graphs are skewed: the line is where those gain, and uniform
+// ones pay up to twice the time there (300 K entries, 30 K columns 31 / 57, columns drawn as u^4 319 / 67; 600 K, 30 K 47 / 70, 591 / 71;
+// 300 K, 300 K 32 / 47, 207 / 70); from 1.2 M on neither does.
 bool bucket_transpose_form(int64_t n_entries, int64_t n_cols) { return n_entries >= ((int64_t)1 << 18) && fits_buckets(n_entries, n_cols); }
 
 static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edges, void* ws, BucketArgs* g, size_t* bytes)

@@ -60,6 +60,19 @@ inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 // ---- device side -----------------------------------------------------------------
 #if defined(__HIPCC__)
 
+// Column c of eight rows of bf16 (r[i]: row i's words, two columns each) as an operand of v_mfma_f32_32x32x16_bf16.
+typedef __bf16 Bf16x8 __attribute__((ext_vector_type(8)));
+template <int WORDS>
+__device__ __forceinline__ Bf16x8 bf16_column(const uint32_t (&r)[8][WORDS], int c)
+{
+    typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+    U4 o;
+    const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;  // the high or the low halves of two words
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(r[2 * j + 1][c >> 1], r[2 * j][c >> 1], sel);
+    return __builtin_bit_cast(Bf16x8, o);
+}
+
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
 
 // actual element count of a (max, device count) pair

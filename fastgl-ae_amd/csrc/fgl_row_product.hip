@@ -31,7 +31,6 @@ namespace fgl {
 typedef float RpF32x16 __attribute__((ext_vector_type(16)));
 typedef float RpF4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t RpU4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef __bf16 RpBf16x8 __attribute__((ext_vector_type(8)));
 
 // One lane's values of a step: kLane values along k of one row (A, or a column of a transposed B).
 template <typename T>
@@ -65,7 +64,7 @@ struct RpRow<uint16_t> {
             v[j] = lo | hi << 16;
         }
     }
-    __device__ __forceinline__ RpBf16x8 operand() const { return __builtin_bit_cast(RpBf16x8, v); }
+    __device__ __forceinline__ Bf16x8 operand() const { return __builtin_bit_cast(Bf16x8, v); }
 };
 
 // One lane's values of a step of an untransposed B: kLane rows (k) of VB neighbouring columns.
@@ -101,14 +100,7 @@ struct RpCols<uint16_t, VB> {
         for (int w = 0; w < kWords; ++w) r[j][w] = 0u;
     }
     // column c of the lane's eight rows, as the instruction's operand
-    __device__ __forceinline__ RpBf16x8 operand(int c) const
-    {
-        RpU4 o;
-        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;  // the high or the low halves of two words
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(r[2 * j + 1][c >> 1], r[2 * j][c >> 1], sel);
-        return __builtin_bit_cast(RpBf16x8, o);
-    }
+    __device__ __forceinline__ Bf16x8 operand(int c) const { return bf16_column(r, c); }
 };
 
 struct RowProductArgs {
@@ -175,7 +167,7 @@ struct RpStep {
         } else {
 #pragma unroll
             for (int t = 0; t < VB; ++t) {
-                RpBf16x8 b;
+                Bf16x8 b;
                 if constexpr (BT) b = bt[t].operand();
                 else b = bn.operand(t);
 #pragma unroll

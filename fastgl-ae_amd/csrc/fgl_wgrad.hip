@@ -33,7 +33,6 @@
 namespace fgl {
 
 typedef float F32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 Bf16x8 __attribute__((ext_vector_type(8)));
 
 // The rows that one step of a wave multiplies, as loaded (GROUPS row groups of the matrix instruction's depth).
 template <typename T, int V>
@@ -104,15 +103,7 @@ struct WgradRows<uint16_t, V> {
         }
     }
     // column c of the lane's eight rows, as the instruction's operand
-    __device__ __forceinline__ Bf16x8 column(int c) const
-    {
-        typedef uint32_t U4 __attribute__((ext_vector_type(4)));
-        U4 o;
-        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;  // the high or the low halves of two words
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_perm(r[2 * j + 1][c >> 1], r[2 * j][c >> 1], sel);
-        return __builtin_bit_cast(Bf16x8, o);
-    }
+    __device__ __forceinline__ Bf16x8 column(int c) const { return bf16_column(r, c); }
     __device__ __forceinline__ void add_columns(float (&sum)[V]) const
     {
 #pragma unroll
