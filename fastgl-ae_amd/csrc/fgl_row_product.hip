@@ -3,8 +3,9 @@
 // transposed, [n, k] (the reference forms these products with torch::mm, cuda_operators/aggregate_acc.cpp:144,188,371,402).
 //
 // Why not the library: it looks for a kernel by the exact sizes on every call, and a new m each time means 60-80 us of host time
-// per product (74 against 13 through here), which is what a training step over mini-batches waited for: GCN step 994 -> 843 us, GraphSAGE
-// in bf16 1482 -> 1094, GAT 1224 -> 941.  Where such products gain is ops._forms_row_product's rule.
+// per product (74 against 12 through here), which is what a training step over mini-batches waited for: GCN step 1000 -> 840 us, GAT 1270 ->
+// 890..940, GraphSAGE in bf16 1430..1630 -> 1110..1140 (three runs; the autograd thread makes two of them uneven).  Where such products
+// gain is ops._forms_row_product's rule.
 //
 // What bounds it: in fp32 the matrix cores, in bf16 the one pass over A and C.
 //
@@ -17,9 +18,9 @@
 // Workgroups that share rows of A (different columns of C) are neighbours on one XCD.
 // The next step's operands are requested before the current ones are multiplied.
 //
-// Measured (MI355X, us, the library's kernel / this one, the same sizes again and again): fp32 1000 x 100 x 64 21 / 13, 107 K x 100 x 256 84 / 80,
-// 107 K x 256 x 256 140 / 149 (94 TFLOP/s), 300 K x 128 x 128 134 / 113; bf16 107 K x 100 x 256 30 / 24, 107 K x 256 x 256 30 / 39; a transposed B, whose
-// loads touch a line per lane, costs up to a quarter more in fp32 and a third in bf16.
+// Measured (MI355X, us, the library's kernel / this one, the same sizes again and again): fp32 107 K x 100 x 256 81 / 78, 107 K x 256 x 256
+// 138 / 144 (97 TFLOP/s), 200 K x 128 x 128 81 / 85; bf16 107 K x 100 x 256 29 / 24, 107 K x 256 x 256 29 / 39; a transposed B, whose loads touch a
+// line per lane, costs up to an eighth more in fp32 and, from k = 128 on, a third in bf16 (107 K x 256 x 256: 27 / 52).
 //
 // Rows past the end repeat the last one and are not stored; a lane whose columns would leave the row takes the row's last VB columns
 // (bit-equal copies of its neighbour's); k past the end is zero in both operands.  No access leaves the operands.
