@@ -366,19 +366,17 @@ def _splits_k(k, m, n):
 
 
 def _forms_row_product(a, b, transposed, m, k, n):
-    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it,
-    no autocast to change the types, and a size where it gains.  The library looks for a kernel on every call with sizes it has not just
-    seen -- 74 us of the host's time against 13 -- which is what a product of a mini-batch takes.  On the GPU, sizes repeated (us, library /
-    here): up to k = 128 the two are alike or this one is ahead (fp32 107 K x 100 x 256 81 / 79, 200 K x 128 x 128 81 / 85, 107 K x 64 x 64 29 / 21; bf16
-    29 / 24, 30 / 29, 22 / 8), with a transposed weight too (84 / 85, 81 / 91, 29 / 20; bf16 30 / 30, 28 / 33, 20 / 10).  A longer k costs it more
-    than the library, whose tiles go through LDS (256 x 256, fp32: 8192 rows 13 / 14, 20 K 26 / 43, 107 K 138 / 149, transposed 141 / 162; bf16: 7 / 7, 10 / 15,
-    29 / 40, transposed 27 / 52): there it is taken up to 2e9 products, 30 K such rows, where a step over fresh blocks still waits for the host
-    more than it loses here.  Larger ones keep the GPU busy for longer than the host takes (fp32 2.4 M x 64 x 100, transposed: 534 / 640; a GIN layer of
-    602 x 256 over 8192 rows, forward and backward, 394 / 418 in all; 256 x 384 and 300 x 300 are like 256 x 256).
+    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it, no
+    autocast to change the types, and a size where it gains.  The library looks for a kernel on every call with sizes it has not just
+    seen -- 74 us of the host's time against 13 -- which is what a product of a mini-batch takes; on the GPU the two are
+    alike (us, library / here: fp32 1000 x 100 x 64 21 / 13, 8192 x 602 x 256 29 / 29, 107 K x 256 x 256 140 / 149, bf16 107 K x 100 x 256
+    30 / 24, 107 K x 256 x 256 30 / 39 and, with a transposed weight, 27 / 53).  Larger ones keep the GPU busy for longer than
+    the host takes, and there the library's tiles through LDS are ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; 20 K x 512 x 512
+    89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all).
     Returns the operands' addresses and row strides if so, else None."""
-    if not (m * k * n <= (8 * 10 ** 9 if k <= 128 else 2 * 10 ** 9) and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and
-            m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and a.get_device() == b.get_device() and
-            not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and not torch.is_autocast_enabled() and not _followed()):
+    if not (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
+            0 < n <= 65536 and a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
+            not torch.is_autocast_enabled() and not _followed()):
         return None
     (lda, unit_a), (ldb, unit_b), at = a.stride(), b.stride(), _addresses(a, b)
     if (at is not None and unit_a == 1 and lda >= k and unit_b == 1 and ldb >= b.size(1) and

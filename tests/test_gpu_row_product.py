@@ -52,17 +52,6 @@ def test_row_product_forms_left_to_torch():
         assert ops.row_product(x, p.detach()).dtype == torch.bfloat16
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_sizes_that_the_library_is_faster_at_are_its_own(dtype):
-    w = torch.empty(256, 256, device=DEV, dtype=dtype)
-    rows = torch.empty(107_000, 256, device=DEV, dtype=dtype)
-    for transposed in (False, True):
-        assert ops._forms_row_product(rows[:17_000], w, transposed, 17_000, 256, 256)
-        assert not ops._forms_row_product(rows, w, transposed, 107_000, 256, 256)
-        thin = w[:, :100].contiguous() if transposed else w[:100]
-        assert ops._forms_row_product(rows[:, :100].contiguous(), thin, transposed, 107_000, 100, 256)
-
-
 def test_linear_without_gradients():
     lin = fastgl.conv._Linear(100, 47).to(DEV)
     x = torch.randn(333, 100, device=DEV)
