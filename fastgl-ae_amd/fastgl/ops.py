@@ -366,13 +366,17 @@ def _splits_k(k, m, n):
 
 
 def _forms_row_product(a, b, transposed, m, k, n):
-    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it, no
-    autocast to change the types, and a size where it gains.  The library looks for a kernel on every call with sizes it has not just
-    seen -- 74 us of the host's time against 13 -- which is what a product of a mini-batch takes; on the GPU the two are
-    alike (us, library / here: fp32 1000 x 100 x 64 21 / 13, 8192 x 602 x 256 29 / 29, 107 K x 256 x 256 140 / 149, bf16 107 K x 100 x 256
-    30 / 24, 107 K x 256 x 256 30 / 39 and, with a transposed weight, 27 / 53).  Larger ones keep the GPU busy for longer than
-    the host takes, and there the library's tiles through LDS are ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; 20 K x 512 x 512
-    89 / 122, bf16 21 / 37; a GIN layer of 602 x 256 over 8192 rows, forward and backward, 394 / 418 in all).
+    """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it,
+    no autocast to change the types, and a size where steps over fresh blocks gain.  The library looks for a kernel on every call with sizes
+    it has not just seen -- 74 us of the host's time against 12 -- which is what a product of a mini-batch takes.  On the GPU, sizes repeated (us,
+    library / here): up to k = 128 the two are alike or this one is ahead (fp32 107 K x 100 x 256 81 / 78, 200 K x 128 x 128 81 / 85, 107 K x 64 x 64 29 / 21;
+    bf16 29 / 24, 30 / 29, 22 / 8; with a transposed weight 84 / 84, 81 / 91, 29 / 20; bf16 30 / 30, 28 / 33, 20 / 10).  A longer k costs it more than the
+    library, whose tiles go through LDS (256 x 256, fp32: 8192 rows 13 / 13, 20 K 26 / 43, 107 K 138 / 144, transposed 141 / 161; bf16: 7 / 7, 10 / 15, 28 / 39,
+    transposed 27 / 52; 256 x 384 and 300 x 300 are no worse): a caller of ever the same sizes whom the GPU keeps waiting loses that much.  Steps
+    over fresh blocks gain all the same: drawing the line for k > 128 at 2e9 instead made GCN inference of 256 x 256 (60 K rows) 330 -> 349 us, GraphSAGE in
+    bf16, 87 K rows of 256 x 256, 996 -> 1294 us a training step and 360 -> 423 in inference, and 3 % better at most (in fp32, 1663 -> 1625).  Products beyond the
+    line keep the GPU busy for longer than the host takes, and there the library is ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; a GIN layer of
+    602 x 256 over 8192 rows, forward and backward, 394 / 418 in all).
     Returns the operands' addresses and row strides if so, else None."""
     if not (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
             0 < n <= 65536 and a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
