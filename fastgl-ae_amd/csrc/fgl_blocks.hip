@@ -10,6 +10,7 @@
 #include "fgl_kernels.hpp"
 #include "fgl_table.hpp"
 #include "fgl_transpose_job.hpp"
+#include "fgl_idmap_device.hpp"
 
 namespace fgl {
 
@@ -28,9 +29,12 @@ __global__ __launch_bounds__(TS) void blocks_prepare_kernel(TableRef t, const vo
                                                             int64_t* __restrict__ row_start, int32_t* __restrict__ deg_out,
                                                             int32_t* __restrict__ tile_sums, int32_t* __restrict__ later_sums,
                                                             int64_t n_later_sums, int32_t* __restrict__ counts, int n_counts,
-                                                            int32_t* __restrict__ sort_n_long)
+                                                            int32_t* __restrict__ sort_n_long, const TransposeJob zero,
+                                                            const ZeroJob zero_marks)
 {
     __shared__ int smem[TS / kWave + 1];
+    tjob_zero<TS>(zero);  // (the first hop's counters and marks)
+    zero_job<TS>(zero_marks);
     const int64_t first = (int64_t)blockIdx.x * TS + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * TS;
     for (int64_t i = first; i < n_counts; i += stride) counts[i] = (i == 0) ? (int32_t)n_seeds : 0;
@@ -86,7 +90,7 @@ struct BlocksPlan {
     int64_t n_positions;       // row start / degree entries: one per node that is a seed of some hop
     int64_t tile_first[33];    // per-tile edge counts of hop h start at entry tile_first[h]; [n_hops] = their total
     int64_t max_tiles;
-    int64_t max_edges;
+    int n_hops;
     size_t idmap_bytes;
     // transposed blocks built inside the call (bit h of transpose_hops: hop h's)
     uint32_t transpose_hops;
@@ -100,8 +104,8 @@ struct BlocksScratch {
     int32_t* deg;
     int32_t* tile_sums;
     int32_t* tile_prefix;
-    uint8_t* lowered;  // one byte per edge of a hop: cleared by the hop's sampling kernel, used by its id-map passes
     char* idmap_ws;
+    uint32_t* marks[32];  // per hop: which of its edges are first mentions (cleared by the launch before the hop's first)
     // per hop whose transposed block is wanted (null otherwise)
     int32_t* t_rank[32];
     int32_t* t_tile_sums[32];
@@ -117,7 +121,6 @@ static size_t carve_scratch(const BlocksPlan& p, void* ws, BlocksScratch* out)
     int32_t* deg = c.take<int32_t>((size_t)p.n_positions);
     int32_t* tile_sums = c.take<int32_t>((size_t)p.tile_first[32]);
     int32_t* tile_prefix = c.take<int32_t>((size_t)p.max_tiles);
-    uint8_t* lowered = c.take<uint8_t>((size_t)p.max_edges);
     char* idmap_ws = c.take<char>(p.idmap_bytes);
     int32_t* sort_long_rows = c.take<int32_t>((size_t)(2 * p.sort_long_max));
     int32_t* sort_n_long = c.take<int32_t>(4);
@@ -129,8 +132,11 @@ static size_t carve_scratch(const BlocksPlan& p, void* ws, BlocksScratch* out)
         out->deg = deg;
         out->tile_sums = tile_sums;
         out->tile_prefix = tile_prefix;
-        out->lowered = lowered;
         out->idmap_ws = idmap_ws;
+    }
+    for (int h = 0; h < p.n_hops; ++h) {
+        uint32_t* marks = c.take<uint32_t>(mark_words(p.cap_edges[h]));
+        if (out) out->marks[h] = marks;
     }
     for (int h = 0; h < 32; ++h) {
         if (!((p.transpose_hops >> h) & 1u)) continue;
@@ -164,7 +170,7 @@ static int make_plan(int64_t n_nodes, int64_t n_seeds, const int32_t* fanouts, i
     FGL_REQUIRE(n_nodes >= 0 && n_seeds >= 0 && fanouts != nullptr, "sample_blocks: bad sizes");
     int64_t cur = n_seeds;
     size_t idmap_ws = 0;
-    int64_t tiles_total = 0, max_tiles = 1, max_edges = 1;
+    int64_t tiles_total = 0, max_tiles = 1;
     for (int h = 0; h < n_hops; ++h) {
         FGL_REQUIRE(fanouts[h] >= 1 && fanouts[h] <= FGL_MAX_FANOUT, "sample_blocks: fanout %d outside [1, %d]", fanouts[h], FGL_MAX_FANOUT);
         if (node_capacity) {
@@ -176,10 +182,9 @@ static int make_plan(int64_t n_nodes, int64_t n_seeds, const int32_t* fanouts, i
         p->cap_dst[h] = cur;
         p->cap_edges[h] = cur * fanouts[h];
         FGL_REQUIRE(p->cap_edges[h] <= 0x7FFFFFFF, "sample_blocks: hop %d may produce %lld edges, beyond int32 offsets", h, (long long)p->cap_edges[h]);
-        if (p->cap_edges[h] > max_edges) max_edges = p->cap_edges[h];
-        const size_t w = idmap_map_src_workspace_bytes(p->cap_edges[h]);
+        const size_t w = idmap_map_src_workspace_bytes(p->cap_edges[h], false);
         if (w > idmap_ws) idmap_ws = w;
-        const int64_t tiles = sample_tile_count(p->cap_dst[h], fanouts[h]);
+        const int64_t tiles = ceil_div(p->cap_dst[h] > 0 ? p->cap_dst[h] : 1, sample_hop_tile_seeds(fanouts[h], p->cap_dst[h]));
         p->tile_first[h] = tiles_total;
         tiles_total += tiles;
         if (tiles > max_tiles) max_tiles = tiles;
@@ -209,25 +214,36 @@ static int make_plan(int64_t n_nodes, int64_t n_seeds, const int32_t* fanouts, i
     FGL_REQUIRE(p->table_slots <= ((int64_t)1 << 31), "sample_blocks: table too large");
     p->n_positions = p->cap_dst[n_hops - 1] > 0 ? p->cap_dst[n_hops - 1] : 1;
     p->max_tiles = max_tiles;
-    p->max_edges = max_edges;
+    p->n_hops = n_hops;
     p->idmap_bytes = idmap_ws;
     p->ws_bytes = carve_scratch(*p, nullptr, nullptr);
     return FGL_OK;
 }
 
-// The three closing steps of a transposed block as launches of their own: for the last hop of a call, which has no
+// The last two closing steps of a transposed block as launches of their own: for the last hop of a call, which has no
 // later hop whose launches could carry them.
-// The last of them also hands the call's counts to the host, if asked: everything in them is final by then.
+// The first of them also hands the call's counts to the host, if asked: everything in them is final by then.
 template <int STEP>
 __global__ __launch_bounds__(kBlock) void transpose_step_kernel(const TransposeJob j, int32_t* __restrict__ readback,
                                                                 const int32_t* __restrict__ counts, int n_counts)
 {
-    if (STEP == 0) tjob_tile_sums<kBlock>(j);
+    if (readback != nullptr && blockIdx.x == 0 && (int)threadIdx.x < n_counts) readback[threadIdx.x] = counts[threadIdx.x];
     if (STEP == 1) tjob_scan<kBlock>(j);
-    if (STEP == 2) {
-        if (readback != nullptr && blockIdx.x == 0 && (int)threadIdx.x < n_counts) readback[threadIdx.x] = counts[threadIdx.x];
-        tjob_fill<kBlock>(j);
-    }
+    if (STEP == 2) tjob_fill<kBlock>(j);
+}
+
+// The launch behind the last hop's passes: the entries of the hop before's transposed block into their rows, the tile sums of the
+// last hop's counters, and every slot of the table empty for the next mini-batch (its passes no longer read the table).
+__global__ __launch_bounds__(kBlock) void blocks_close_kernel(const TransposeJob sums, const TransposeJob fill, uint32_t* __restrict__ clear_words,
+                                                              int64_t n_clear_words, int n_side)
+{
+    tjob_tile_sums<kBlock>(sums);
+    tjob_fill<kBlock>(fill);
+    const int64_t own_blocks = (int64_t)gridDim.x - n_side;
+    if ((int64_t)blockIdx.x >= own_blocks) return;
+    uint4* v = reinterpret_cast<uint4*>(clear_words);  // (a table is 8-byte slots, a power of two of them, 16-byte aligned)
+    const uint4 empty = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n_clear_words / 4; i += own_blocks * kBlock) v[i] = empty;
 }
 
 // Every row of the call's transposed blocks into ascending order of its entries' positions in the block (one launch
@@ -350,12 +366,10 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
         rc = launch_fill_u32(t.words, table_slots * 2, kEmpty, s);
         if (rc != FGL_OK) return rc;
     }
-    TransposeJob job_before;
-    memset(&job_before, 0, sizeof(job_before));
     auto make_job = [&](int h) {
         TransposeJob j;
         memset(&j, 0, sizeof(j));
-        if (!((transpose_hops >> h) & 1u)) return j;
+        if (h < 0 || h >= n_hops || !((transpose_hops >> h) & 1u)) return j;
         j.split = p.split[h];
         j.cnt = j.split > 1 ? ws.t_split_cnt[h] : t_ptr[h];
         j.tile_sums = ws.t_tile_sums[h];
@@ -374,26 +388,53 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
         j.edges_max = p.cap_edges[h];
         return j;
     };
+    const bool arrival = order != 0;
+    auto marks_of = [&](int h) { return marks_at(ws.marks[h]); };
+    auto zero_marks_of = [&](int h) {
+        ZeroJob z{};
+        if (h < n_hops && !arrival) {
+            z.p = reinterpret_cast<uint4*>(ws.marks[h]);
+            z.n16 = (int64_t)mark_words(p.cap_edges[h]) / 4;
+        }
+        return z;
+    };
     // launch 2: counts, the later hops' tile sums, the seeds into the table, the first hop's rows and tile sums
     {
-        const int ts0 = sample_tile_seeds(fanouts[0], n_seeds);
-        const int64_t tiles0 = sample_tile_count(n_seeds, fanouts[0]);
+        const int ts0 = sample_hop_tile_seeds(fanouts[0], p.cap_dst[0]);
+        const int64_t tiles0 = ceil_div(n_seeds > 0 ? n_seeds : 1, ts0);
         const int64_t n_later = p.tile_first[n_hops] - p.tile_first[1];
         int64_t blocks = tiles0;
         if (blocks < ceil_div(n_later, ts0)) blocks = ceil_div(n_later, ts0);
         if (blocks > 8192) blocks = 8192;
         if (blocks < 1) blocks = 1;
+        TransposeJob zero = make_job(0);
+        ZeroJob zero_marks = zero_marks_of(0);
+        if (zero.cnt != nullptr) {
+            zero.side_first = 0;
+            zero.side_blocks = side_blocks_for(zero.cols_max * zero.split + 1, (int64_t)ts0 * 16);
+            blocks += zero.side_blocks;
+        }
+        if (zero_marks.n16 > 0) {
+            zero_marks.side_first = zero.side_blocks;
+            zero_marks.side_blocks = side_blocks_for(zero_marks.n16, (int64_t)ts0 * 4);
+            blocks += zero_marks.side_blocks;
+        }
         if (ts0 == 256)
             hipLaunchKernelGGL(blocks_prepare_kernel<256>, dim3((unsigned)blocks), dim3(256), 0, s, t, d_indptr, indptr_is64, n_nodes,
                                d_seeds, n_seeds, fanouts[0], d_uniq, ws.row_start, ws.deg, ws.tile_sums,
-                               ws.tile_sums + p.tile_first[1], n_later, d_counts, n_counts, ws.sort_n_long);
+                               ws.tile_sums + p.tile_first[1], n_later, d_counts, n_counts, ws.sort_n_long, zero, zero_marks);
         else
             hipLaunchKernelGGL(blocks_prepare_kernel<64>, dim3((unsigned)blocks), dim3(64), 0, s, t, d_indptr, indptr_is64, n_nodes,
                                d_seeds, n_seeds, fanouts[0], d_uniq, ws.row_start, ws.deg, ws.tile_sums,
-                               ws.tile_sums + p.tile_first[1], n_later, d_counts, n_counts, ws.sort_n_long);
+                               ws.tile_sums + p.tile_first[1], n_later, d_counts, n_counts, ws.sort_n_long, zero, zero_marks);
         FGL_CHECK_LAUNCH("blocks_prepare_kernel");
     }
 
+    // the host's copy of the counts is written as soon as the last of them is final: with the last hop's node total (the longest
+    // rows of the earlier hops' transposed blocks are known by then), or, its own transposed block being wanted, by the launch
+    // behind the one that finds its longest row
+    const TransposeJob job_last = make_job(n_hops - 1), job_before_last = make_job(n_hops - 2);
+    const bool counts_final_with_total = job_last.cnt == nullptr;
     for (int h = 0; h < n_hops; ++h) {
         const bool last = h == n_hops - 1;
         const int32_t* hop_seeds = (h == 0) ? d_seeds : d_uniq;
@@ -412,42 +453,67 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
             next.deg = ws.deg;
             next.tile_sums = ws.tile_sums + p.tile_first[h + 1];
             next.fanout = fanouts[h + 1];
-            next.tile_seeds = sample_tile_seeds(fanouts[h + 1], p.cap_dst[h + 1]);
+            next.tile_seeds = sample_hop_tile_seeds(fanouts[h + 1], p.cap_dst[h + 1]);
         }
-        // transposed blocks: this hop's (if wanted) has its counters cleared by the sampling launch and its ranks
-        // taken by the id-map passes; the one of the hop before is closed by this hop's first three launches
+        // transposed blocks: this hop's has its ranks taken by the hop's launches; those of the two hops before are closed by them
+        const TransposeJob job = make_job(h), job_before = make_job(h - 1), job_next = make_job(h + 1);
         TransposeSteps steps;
-        steps.before = job_before;
-        steps.zero = make_job(h);
+        steps.sums = job_before;
+        steps.fill = make_job(h - 2);
+        const bool insert = !arrival && sample_can_insert(fanouts[h], p.cap_dst[h]);
+        const InsertWork work = idmap_insert_work(d_table, table_slots, ws.idmap_ws, p.cap_edges[h], src_local[h], marks_of(h), &job);
         rc = launch_sample_edges(d_indices, hop_seeds, p.cap_dst[h], d_n_dst, fanouts[h], ws.row_start, ws.deg,
                                  ws.tile_sums + p.tile_first[h], ws.tile_prefix, rng_seed, stream_base + (uint32_t)h, sampled,
                                  nullptr, block_ptr[h], d_n_edges, d_status, s, d_stream_offset, last ? nullptr : &next,
-                                 ws.lowered, &steps);
+                                 &steps, nullptr, insert ? &work : nullptr, sample_hop_tile_seeds(fanouts[h], p.cap_dst[h]));
         if (rc != FGL_OK) return rc;
         // the node count this hop may grow to: what the next hop's buffers (or the unique list) hold;
         // growing past it is reported as FGL_STATUS_UNIQ_OVERFLOW and the count is clamped
         const int64_t grow_to = (!last && p.cap_dst[h + 1] < p.cap_uniq) ? p.cap_dst[h + 1] : p.cap_uniq;
-        // the host's copy of the counts: written by whichever launch makes the last of them final -- the last hop's
-        // node total, or (if the last hop's transposed block is wanted) its longest row, below
-        const bool counts_final_here = last && steps.zero.cnt == nullptr;
+        MapSrcExtras x;
+        memset(&x, 0, sizeof(x));
+        x.marks = marks_of(h);
+        x.inserted = insert;
+        x.next_hop = last ? nullptr : &next;
+        x.rank_job = &job;
+        x.scan_job = &job_before;
+        x.zero_job = &job_next;
+        x.zero_marks = zero_marks_of(h + 1);
+        x.d_readback = last && counts_final_with_total ? d_readback : nullptr;
+        x.d_readback_counts = d_counts;
+        x.n_readback_counts = n_counts;
         rc = launch_idmap_map_src(d_table, table_slots, sampled, src_local[h], p.cap_edges[h], d_n_edges, 0, d_n_dst,
                                   d_counts + h + 1, d_uniq, grow_to, order | (last ? FGL_IDMAP_FINAL : 0), d_status,
-                                  ws.idmap_ws, p.idmap_bytes, s, /*counter_is_zeroed=*/true, last ? nullptr : &next,
-                                  /*leave_table_empty=*/last && leave_empty, ws.lowered, &steps.zero, &job_before, nullptr,
-                                  counts_final_here ? d_readback : nullptr, d_counts, n_counts);
+                                  ws.idmap_ws, p.idmap_bytes, s, /*counter_is_zeroed=*/true, /*leave_table_empty=*/false, &x);
         if (rc != FGL_OK) return rc;
-        job_before = steps.zero;
     }
-    if (job_before.cnt != nullptr) {  // the last hop's transposed block: no later launch to carry its closing steps
-        job_before.side_first = 0;
-        job_before.side_blocks = side_blocks_for(job_before.cols_max * job_before.split + 1, kTjobTile, 8192);
-        hipLaunchKernelGGL(transpose_step_kernel<0>, dim3((unsigned)job_before.side_blocks), dim3(kBlock), 0, s, job_before,
-                           nullptr, nullptr, 0);
-        hipLaunchKernelGGL(transpose_step_kernel<1>, dim3((unsigned)job_before.side_blocks), dim3(kBlock), 0, s, job_before,
-                           nullptr, nullptr, 0);
-        job_before.side_blocks = side_blocks_for(job_before.rows_max, kBlock / 16, 16384);
-        hipLaunchKernelGGL(transpose_step_kernel<2>, dim3((unsigned)job_before.side_blocks), dim3(kBlock), 0, s, job_before,
-                           d_readback, d_counts, n_counts);
+    if (leave_empty || job_last.cnt != nullptr || job_before_last.cnt != nullptr) {
+        TransposeJob sums = job_last, fill = job_before_last;
+        unsigned side = 0;
+        if (sums.cnt != nullptr) {
+            sums.side_first = 0;
+            sums.side_blocks = side_blocks_for(sums.cols_max * sums.split + 1, kTjobTile, 8192);
+            side += (unsigned)sums.side_blocks;
+        }
+        if (fill.cnt != nullptr) {
+            fill.side_first = (int)side;
+            fill.side_blocks = side_blocks_for(fill.rows_max, kBlock / 16, 16384);
+            side += (unsigned)fill.side_blocks;
+        }
+        const int64_t n_clear_words = leave_empty ? table_slots * 2 : 0;
+        const int64_t clear_blocks = ceil_div(n_clear_words, kBlock * 16);
+        const unsigned own = (unsigned)(clear_blocks < 1 ? 1 : clear_blocks < 4096 ? clear_blocks : 4096);
+        hipLaunchKernelGGL(blocks_close_kernel, dim3(own + side), dim3(kBlock), 0, s, sums, fill, leave_empty ? t.words : nullptr,
+                           n_clear_words, (int)side);
+        FGL_CHECK_LAUNCH("blocks_close_kernel");
+    }
+    if (job_last.cnt != nullptr) {  // the last hop's transposed block: the rest of its closing steps
+        TransposeJob j = job_last;
+        j.side_first = 0;
+        j.side_blocks = side_blocks_for(j.cols_max * j.split + 1, kTjobTile, 8192);
+        hipLaunchKernelGGL(transpose_step_kernel<1>, dim3((unsigned)j.side_blocks), dim3(kBlock), 0, s, j, d_readback, d_counts, n_counts);
+        j.side_blocks = side_blocks_for(j.rows_max, kBlock / 16, 16384);
+        hipLaunchKernelGGL(transpose_step_kernel<2>, dim3((unsigned)j.side_blocks), dim3(kBlock), 0, s, j, nullptr, nullptr, 0);
         FGL_CHECK_LAUNCH("transpose_step_kernel");
     }
     if (sort_rows && transpose_hops != 0) {

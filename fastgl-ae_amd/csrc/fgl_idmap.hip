@@ -9,24 +9,25 @@
 // new ids are numbered in first-occurrence order -- deterministic, and the order DGL's
 // to_block gives -- instead of the reference's race on one global counter (id_map.cu:317-320).
 //
-// map_src = four launches (three for small inputs):
+// map_src = two launches (three beyond 1 M edges, four beyond 8 M):
 //   1. insert     per edge: probe (one 8-byte load per slot), install {key, pending first-edge index}
 //                 with one 64-bit CAS if new, else atomicMin the first-edge index; remember the slot.
 //                 An id that was numbered before this call is relabelled on the spot from the val
 //                 the probe has loaded anyway, and the edge takes no further part.
-//   2. mark       per edge: "am I the first edge of a new id?" -> one flag bit per edge
-//                 (8 edges per lane, one byte), the count of flags before each byte within its tile
-//                 of 2048 edges, and per-tile counts
-//   3. prefix     single workgroup over the tile counts; publishes the new node total
-//                 (the edge-parallel launches are grid-stride loops over the actual count,
-//                 so a bound much larger than the batch costs nothing).  Skipped while the bound
-//                 is at most 2048 tiles (4 M edges): the number pass then scans the tile counts
-//                 itself in every workgroup, and its first workgroup publishes the total
-//   4. number     per edge, coalesced: the local id follows from the first-edge index that the mark
-//                 pass left for the edge and the three counts (cache-resident arrays): no table read.
-//                 The first edge of a new id appends the id to the unique list and stores the local id
-//                 in the id's slot for later calls -- skipped with FGL_IDMAP_FINAL, when the caller
-//                 will not consult the table again (the last hop of a mini-batch: most of its edges).
+//                 The edges that are first mentions of new ids are kept track of as they change, a bit
+//                 per edge (MentionMarks, mark_first).  In a mini-batch's small hops the sampling kernel
+//                 does this itself with the edges it has just drawn.
+//   2. number     per edge: an edge whose bit is set is its id's first mention, and its local id is the
+//                 number of bits before it: a prefix per 512 edges (64 bytes of bits, which every
+//                 workgroup counts and scans into LDS for itself) plus the bits of its own line.  It appends
+//                 the id to the unique list and stores the local id in the id's slot for later calls --
+//                 skipped with FGL_IDMAP_FINAL, when the caller will not consult the table again (the last
+//                 hop of a mini-batch: most of its edges).  Any other edge reads its slot: the local id, if
+//                 the first mention's lane has been there already, else the index of that first mention,
+//                 and counts the bits before that.
+//   (count)       larger inputs: the bits counted once, per line and per 4096 edges; the number pass then scans
+//                 the latter only
+//   (prefix)      ... and where even those are too many for every workgroup, a single workgroup scans them
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_table.hpp"
@@ -34,9 +35,6 @@
 #include "fgl_idmap_device.hpp"
 
 namespace fgl {
-
-constexpr int kItems = 8;
-constexpr int kTile = kBlock * kItems;
 
 __global__ __launch_bounds__(kBlock) void idmap_insert_dst_kernel(TableRef t, const int32_t* __restrict__ ids,
                                                                   int64_t n_max, const int32_t* __restrict__ d_n,
@@ -59,199 +57,51 @@ __global__ __launch_bounds__(kBlock) void idmap_insert_dst_kernel(TableRef t, co
     if (p == kEmpty && d_status) atomicOr(d_status, FGL_STATUS_TABLE_FULL);
 }
 
-// Edges per lane of the insert pass: the lane's first slot loads go out together, then the compare-and-swaps of
-// the edges that found their slot empty, then each sequence is finished (most are, by then).  Measured on the
-// 1.5 M-edge outer hop of a 111 M-node graph: 1 edge per lane 56 us, 2 -> 62 us, 4 -> 70 us -- the pass is bound
-// by the rate at which the chip retires atomics, and fewer, longer-lived waves only take parallelism away.
-#ifndef FGL_INSERT_ITEMS
-#define FGL_INSERT_ITEMS 1
-#endif
-
+// One edge per lane: the pass is bound by the rate at which the chip retires atomics, and several edges in flight per lane only
+// take parallelism away (a hop of 1.5 M edges on a 111 M-node graph: 1 edge 56 us, 2 -> 62 us, 4 -> 70 us).
 // `src` and `out` may be the same array (relabelling in place): neither is __restrict__.
-// lowered (may be null; one byte per edge, zero on entry): lowered[e] is set when a later-running insert takes the
-// place of edge e as its id's first known mention.  Together with the holder bit in slot_of[] it tells the mark pass
-// which edges are first mentions without a look at the table.
-template <int ITEMS>
-__global__ __launch_bounds__(kBlock) void idmap_insert_src_kernel(TableRef t, const int32_t* src,
-                                                                  int64_t e_max, const int32_t* __restrict__ d_e,
-                                                                  uint32_t* __restrict__ slot_of, int32_t* out,
-                                                                  uint8_t* __restrict__ lowered,
-                                                                  uint32_t* __restrict__ d_status, const TransposeRank tr,
-                                                                  const TransposeJob before, int32_t* dst_inout)
+__global__ __launch_bounds__(kBlock) void idmap_insert_src_kernel(const int32_t* src, int64_t e_max, const int32_t* __restrict__ d_e,
+                                                                  const InsertWork w, uint32_t* __restrict__ d_status, int32_t* dst_inout)
 {
-    tjob_scan<kBlock>(before);  // (the hop before, if its transposed block is being built: counters -> offsets)
-    unsigned long long* slots = reinterpret_cast<unsigned long long*>(t.words);
+    unsigned long long* slots = reinterpret_cast<unsigned long long*>(w.t.words);
     const int64_t n_e = actual_count(e_max, d_e);
-    constexpr int kEdges = kBlock * ITEMS;
-    const int64_t n_tiles = (n_e + kEdges - 1) / kEdges;
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t first = tile * kEdges + threadIdx.x;
-        int32_t id[ITEMS];
-        uint32_t p[ITEMS];
-        unsigned long long s[ITEMS];
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            const int64_t e = first + (int64_t)j * kBlock;
-            id[j] = e < n_e ? src[e] : -1;
-        }
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            p[j] = ((uint32_t)id[j] * kHashMul) >> t.shift;
-            s[j] = id[j] >= 0 ? slots[p[j]] : 0ull;
-        }
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t base = (int64_t)blockIdx.x * kBlock; base < n_e; base += stride) {
+        const int64_t e = base + threadIdx.x;
+        const int32_t id = e < n_e ? src[e] : -1;
+        const uint32_t p = ((uint32_t)id * kHashMul) >> w.t.shift;
+        const unsigned long long s = id >= 0 ? slots[p] : 0ull;
         // The destination half of transfer_edge_id (id_map.cu:377-381) rides on this pass when the caller asks: the
         // edge's destination id -- numbered by an earlier launch -- is looked up and relabelled in place, its first
         // probe travelling together with the source id's.
-        if (dst_inout != nullptr) {
-#pragma unroll
-            for (int j = 0; j < ITEMS; ++j) {
-                const int64_t e = first + (int64_t)j * kBlock;
-                if (e >= n_e) continue;
-                const uint32_t d = (uint32_t)dst_inout[e];
-                int32_t local = -1;
-                if ((int32_t)d >= 0) {
-                    uint32_t q = (d * kHashMul) >> t.shift;
-                    const uint32_t limit = t.mask < kMaxProbes ? t.mask + 1 : kMaxProbes;
-                    for (uint32_t n = 0; n < limit; ++n) {
-                        const unsigned long long v = slots[q];
-                        if ((uint32_t)v == d) {
-                            // (a destination id holds its number; one that only an edge of this call has mentioned
-                            // so far -- pending -- is not a destination: missing)
-                            if (!((uint32_t)(v >> 32) & kPending)) local = (int32_t)(v >> 32);
-                            break;
-                        }
-                        if ((uint32_t)v == kEmpty) break;
-                        q = (q + 1) & t.mask;
+        if (dst_inout != nullptr && e < n_e) {
+            const uint32_t d = (uint32_t)dst_inout[e];
+            int32_t local = -1;
+            if ((int32_t)d >= 0) {
+                uint32_t q = (d * kHashMul) >> w.t.shift;
+                const uint32_t limit = w.t.mask < kMaxProbes ? w.t.mask + 1 : kMaxProbes;
+                for (uint32_t n = 0; n < limit; ++n) {
+                    const unsigned long long v = slots[q];
+                    if ((uint32_t)v == d) {
+                        // (a destination id holds its number; one that only an edge of this call has mentioned
+                        // so far -- pending -- is not a destination: missing)
+                        if (!((uint32_t)(v >> 32) & kPending)) local = (int32_t)(v >> 32);
+                        break;
                     }
+                    if ((uint32_t)v == kEmpty) break;
+                    q = (q + 1) & w.t.mask;
                 }
-                if (local < 0 && d_status) atomicOr(d_status, FGL_STATUS_MISSING_KEY);
-                dst_inout[e] = local;
             }
+            if (local < 0 && d_status) atomicOr(d_status, FGL_STATUS_MISSING_KEY);
+            dst_inout[e] = local;
         }
-        // (the compare-and-swaps of the edges whose first slot is empty -- most edges of an outer hop -- are issued
-        // before any of their results is looked at)
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            const int64_t e = first + (int64_t)j * kBlock;
-            if (id[j] >= 0 && (uint32_t)s[j] == kEmpty) {
-                const unsigned long long fresh = (unsigned long long)(uint32_t)id[j] | ((unsigned long long)(kPending | (uint32_t)e) << 32);
-                const unsigned long long seen = atomicCAS(&slots[p[j]], ~0ull, fresh);
-                // what the slot held: still empty = this edge's key went in; (an installed slot is never empty again,
-                // so "our own key with our own pending index" tells the continuation below that the install is done)
-                s[j] = seen == ~0ull ? fresh : seen;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < ITEMS; ++j) {
-            const int64_t e = first + (int64_t)j * kBlock;
-            if (e >= n_e) continue;
-            // ids numbered earlier hold a local id (no pending bit) and stay as they are; a new id keeps
-            // the smallest pending edge index among the edges that mention it
-            const uint32_t mine = kPending | (uint32_t)e;
+        bool holder = false;
+        if (e < n_e) {
             uint32_t seen = 0, displaced = kEmpty, q = kEmpty;
-            bool holder = false;
-            if (id[j] >= 0) {
-                if (s[j] == ((unsigned long long)(uint32_t)id[j] | ((unsigned long long)mine << 32))) {
-                    // installed by the compare-and-swap above (no other edge carries this pending index)
-                    q = p[j];
-                    seen = mine;
-                    holder = true;
-                } else {
-                    q = insert_mention_from(t, (uint32_t)id[j], mine, p[j], s[j], &seen, &holder, &displaced);
-                }
-            }
-            if (q == kEmpty) {
-                // table full, or not a node id: reported; the edge's local id becomes -1 (written by the number pass)
-                if (d_status) atomicOr(d_status, id[j] >= 0 ? FGL_STATUS_TABLE_FULL : FGL_STATUS_BAD_ID);
-            } else if (!(seen & kPending)) {
-                // numbered in an earlier hop (or a destination node): the edge is relabelled right here and
-                // takes no further part (`out` may be `src`: this lane is the only one that touches entry e)
-                out[e] = (int32_t)seen;
-                take_rank(tr, e, (int32_t)seen);
-                q = kDone;
-            } else if (lowered != nullptr) {
-                if (holder) q |= kHolderBit;
-                // (a pending value left over from an earlier call's overflow may name an edge beyond this call's)
-                if ((displaced & kPending) && displaced != kEmpty && (int64_t)(displaced & ~kPending) < n_e) lowered[displaced & ~kPending] = 1;
-            }
-            slot_of[e] = q;
+            if (id >= 0) q = insert_mention_from(w.t, (uint32_t)id, kPending | (uint32_t)e, p, s, &seen, &holder, &displaced);
+            finish_insert(w, e, n_e, id, q, seen, displaced, d_status);
         }
-    }
-}
-
-__device__ __forceinline__ int64_t tiles_of(int64_t n) { return (n + kTile - 1) / kTile; }
-
-// flags8[tile*256 + lane] bit j  <=>  edge (tile*2048 + lane*8 + j) is the first edge of a new id;
-// before8[tile*256 + lane] = number of flagged edges of the tile before edge tile*2048 + lane*8;
-// first_of[e] = pending | index of the first edge that mentions e's id (edges that take part only)
-__global__ __launch_bounds__(kBlock) void idmap_mark_kernel(TableRef t, int64_t e_max, const int32_t* __restrict__ d_e,
-                                                            const uint32_t* __restrict__ slot_of,
-                                                            const uint8_t* __restrict__ lowered,
-                                                            uint32_t* __restrict__ first_of,
-                                                            uint8_t* __restrict__ flags8, uint16_t* __restrict__ before8,
-                                                            int32_t* __restrict__ tile_sums, const TransposeJob before)
-{
-    __shared__ int smem[kBlock / kWave + 1];
-    tjob_fill<kBlock>(before);  // (the hop before, if its transposed block is being built: entries into their rows)
-    const int64_t n_e = actual_count(e_max, d_e);
-    const int64_t n_tiles = tiles_of(n_e);
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t first = tile * kTile + (int64_t)threadIdx.x * kItems;
-        const bool whole = first + kItems <= n_e;  // the lane's eight edges all exist: 32-byte vector accesses
-        uint32_t p[kItems];
-        if (whole) {
-            const uint4 lo = *reinterpret_cast<const uint4*>(slot_of + first);
-            const uint4 hi = *reinterpret_cast<const uint4*>(slot_of + first + 4);
-            p[0] = lo.x; p[1] = lo.y; p[2] = lo.z; p[3] = lo.w;
-            p[4] = hi.x; p[5] = hi.y; p[6] = hi.z; p[7] = hi.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < kItems; ++j) p[j] = (first + j < n_e) ? slot_of[first + j] : kEmpty;
-        }
-        // An edge that became its id's first known mention when it was inserted and was not displaced afterwards
-        // is the first mention: nothing to read.  The others (an eighth of the edges of a large hop, where the
-        // inserts run nearly in edge order) read what the slot holds now.
-        uint32_t low[kItems];
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) low[j] = 1u;  // without the bookkeeping: every edge reads its slot
-        if (lowered != nullptr) {
-            if (whole) {
-                const uint2 b = *reinterpret_cast<const uint2*>(lowered + first);
-#pragma unroll
-                for (int j = 0; j < kItems; ++j) low[j] = ((j < 4 ? b.x : b.y) >> (8 * (j & 3))) & 0xFFu;
-            } else {
-#pragma unroll
-                for (int j = 0; j < kItems; ++j) low[j] = (first + j < n_e) ? lowered[first + j] : 1u;
-            }
-        }
-        uint32_t v[kItems];
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            v[j] = 0u;
-            if (p[j] < kDone) {
-                if ((p[j] & kHolderBit) && low[j] == 0u) v[j] = kPending | (uint32_t)(first + j);
-                else v[j] = t.words[2 * (size_t)(p[j] & ~kHolderBit) + 1];
-            }
-        }
-        uint32_t bits = 0;
-#pragma unroll
-        for (int j = 0; j < kItems; ++j)
-            if (p[j] < kDone && v[j] == (kPending | (uint32_t)(first + j))) bits |= 1u << j;
-        // what the slot holds now -- pending | index of the id's first edge -- is all the number pass
-        // needs to know about the edge: it never goes back to the table for it
-        if (whole) {
-            *reinterpret_cast<uint4*>(first_of + first) = make_uint4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<uint4*>(first_of + first + 4) = make_uint4(v[4], v[5], v[6], v[7]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < kItems; ++j)
-                if (first + j < n_e) first_of[first + j] = v[j];
-        }
-        flags8[tile * kBlock + threadIdx.x] = (uint8_t)bits;
-        int total;
-        const int before = block_exclusive_scan<kBlock>(__popc(bits), smem, &total);
-        before8[tile * kBlock + threadIdx.x] = (uint16_t)before;
-        if (threadIdx.x == 0) tile_sums[tile] = total;
+        mark_first(w.marks, base + threadIdx.x / kWave * kWave, holder);
     }
 }
 
@@ -300,7 +150,7 @@ __global__ __launch_bounds__(1024) void idmap_prefix_publish_kernel(const int32_
                                                                     const int32_t* __restrict__ rb_counts, int rb_n)
 {
     __shared__ int smem[1024 / kWave + 1];
-    const int n_tiles = (int)tiles_of(actual_count(e_max, d_e));
+    const int n_tiles = (int)mark_tiles(actual_count(e_max, d_e));
     int carry = 0;
     for (int start = 0; start < n_tiles; start += 1024) {
         const int i = start + (int)threadIdx.x;
@@ -314,14 +164,31 @@ __global__ __launch_bounds__(1024) void idmap_prefix_publish_kernel(const int32_
         publish_node_total(d_n_base ? (int64_t)(*d_n_base) : n_base_h, carry, capacity, d_n_total_out, d_status, readback, rb_counts, rb_n);
 }
 
-// Up to this many tiles the number pass scans the tile counts itself (every workgroup, into LDS) and
-// its first workgroup publishes the node total: one launch less per call where launches, not
-// edges, set the time.  Above it the single-workgroup prefix launch prepares the array once.
-constexpr int kSelfTilesPerLane = 8;
-#ifndef FGL_NUMBER_SELF_MAX_BLOCKS
-#define FGL_NUMBER_SELF_MAX_BLOCKS 1024
-#endif
-constexpr int kIdmapSelfPrefixTiles = kBlock * kSelfTilesPerLane;
+// How a number pass comes by the marks before a line of edges (kMode):
+//   kFromBits     every workgroup counts all lines' bits itself and scans the counts in LDS: up to kLinesInLds lines, i.e. one
+//                 launch fewer where launches, not edges, set the time (128 KB of bits a workgroup at most);
+//   kFromTiles    a count launch has counted lines and tiles of eight lines; every workgroup scans the tiles' counts in LDS;
+//   kFromPrefix   as kFromTiles, with a prefix launch behind the count launch that has scanned them.
+// In the first two the first workgroup publishes the node total.
+constexpr int kFromBits = 0, kFromTiles = 1, kFromPrefix = 2;
+constexpr int kEntriesPerLane = 8;
+constexpr int kLinesInLds = kBlock * kEntriesPerLane;
+constexpr int kNumberMaxBlocks = 1024;
+
+// eight lanes per tile of 4096 edges, a line each
+__global__ __launch_bounds__(kBlock) void idmap_count_kernel(const MentionMarks marks, int64_t e_max, const int32_t* __restrict__ d_e,
+                                                             int32_t* __restrict__ line_counts, int32_t* __restrict__ tile_sums)
+{
+    const int64_t n_lines = mark_tiles(actual_count(e_max, d_e)) * (kMarkTile / kMarkLine);
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t line = (int64_t)blockIdx.x * kBlock + threadIdx.x; line < n_lines; line += stride) {  // (eight lanes at a time)
+        int c = line_count(marks, line);
+        line_counts[line] = c;
+#pragma unroll
+        for (int d = 1; d < kMarkTile / kMarkLine; d <<= 1) c += __shfl_xor(c, d, kWave);
+        if (line % (kMarkTile / kMarkLine) == 0) tile_sums[line / (kMarkTile / kMarkLine)] = c;
+    }
+}
 
 // The new nodes that the lanes of a wave number in one step have consecutive positions (a position is a count of
 // earlier new nodes, and the lanes hold consecutive edges), so their tiles of the next hop are at most two:
@@ -351,72 +218,71 @@ __device__ __forceinline__ void add_next_tile_sums(const NextHop& next, int k, i
 }
 
 // Lane per edge, coalesced.  `src` and `out` may be the same array: an entry is read and written by one lane only.
-// (Edges whose id was numbered before this call were relabelled by the insert pass.)  The local id of an
-// edge's node follows from the index of the node's first edge (first_of, from the mark pass) and the three
-// counts -- small arrays that stay in cache -- so no lane reads the table; the first edge of a new id also
-// appends the id to the unique list and, unless the caller has said that the table will not be consulted
-// again (WRITE_BACK = false), stores the local id in the id's slot.
-// SELF: no prefix launch ran; tile_prefix is unused, the tile counts are scanned here.
-template <bool SELF, bool WRITE_BACK>
+// (Edges whose id was numbered before this call were relabelled by the insert pass.)  A first mention's local id is the number
+// of marks before its edge; it appends the id to the unique list and, unless the caller has said that the table will not be
+// consulted again (WRITE_BACK = false), stores the local id in the id's slot.  The other edges of new ids -- a fifth to two
+// fifths of a hop's -- read the slot: it holds the local id already, or still the index of the first mention.
+// (A pass between insert and number used to read every edge's slot, flag the first mentions and count them: 5.3-6.6 us of a small
+// hop's three launches, 10.4 us for 1.5 M edges; this pass took 17.7 us for those, now 19.2 + 4.7 for the count.)
+// The launch also carries (in workgroups behind its own) what the hops around it need: `scan` turns the counters of the hop
+// before's transposed block into offsets, `zero` and zero_marks clear the counters and marks of the next hop.
+template <int kMode, bool WRITE_BACK>
 __global__ __launch_bounds__(kBlock) void idmap_number_kernel(TableRef t, const int32_t* src, int64_t e_max,
                                                               const int32_t* __restrict__ d_e, int64_t n_base_h,
                                                               const int32_t* __restrict__ d_n_base,
-                                                              const uint32_t* __restrict__ slot_of,
-                                                              const uint32_t* __restrict__ first_of,
-                                                              const uint8_t* __restrict__ flags8,
-                                                              const uint16_t* __restrict__ before8,
-                                                              const int32_t* __restrict__ tile_sums,
-                                                              const int32_t* __restrict__ tile_prefix,
+                                                              const uint32_t* __restrict__ slot_of, const MentionMarks marks,
+                                                              const int32_t* __restrict__ line_counts,
+                                                              const int32_t* __restrict__ tile_counts,  // kFromPrefix: their prefixes
                                                               int32_t* __restrict__ uniq, int64_t capacity, int32_t* out,
                                                               int32_t* __restrict__ d_n_total_out,
                                                               uint32_t* __restrict__ d_status, const NextHop next,
-                                                              uint32_t* __restrict__ clear_words, int64_t n_clear_words,
-                                                              const TransposeRank tr, int32_t* __restrict__ readback,
+                                                              const TransposeRank tr, const TransposeJob scan, const TransposeJob zero,
+                                                              const ZeroJob zero_marks, int n_side, int32_t* __restrict__ readback,
                                                               const int32_t* __restrict__ rb_counts, int rb_n)
 {
-    __shared__ int s_prefix[SELF ? kIdmapSelfPrefixTiles : 1];
+    __shared__ int s_prefix[kMode != kFromPrefix ? kLinesInLds : 1];
     __shared__ int smem[kBlock / kWave + 1];
+    tjob_scan<kBlock>(scan);
+    tjob_zero<kBlock>(zero);
+    zero_job<kBlock>(zero_marks);
+    const int64_t own_blocks = (int64_t)gridDim.x - n_side;
+    if ((int64_t)blockIdx.x >= own_blocks) return;
     const int64_t n_e = actual_count(e_max, d_e);
     const int64_t n_base = d_n_base ? (int64_t)(*d_n_base) : n_base_h;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    const int64_t stride = own_blocks * kBlock;
+    if ((int64_t)blockIdx.x * kBlock >= n_e && blockIdx.x != 0) return;  // (workgroup 0 publishes the total in any case)
     // What the first trip of the loop below reads about its edge is fetched now, so that it travels together with
-    // the tile counts that the scan waits for (a small hop is one trip per workgroup: a chain of memory latencies).
-    uint32_t p_ahead = kDone, first_ahead = 0;
+    // the counts that the scan waits for (a small hop is one trip per workgroup: a chain of memory latencies).
+    uint32_t p_ahead = kDone;
+    unsigned long long bits_ahead = 0;
     int32_t id_ahead = 0;
     {
         const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
         if (e < n_e) {
             p_ahead = slot_of[e];
-            first_ahead = first_of[e];
+            bits_ahead = marks.bits[e >> 6];
             id_ahead = src[e];
         }
     }
-    if constexpr (SELF) {
-        const int n_tiles = (int)tiles_of(n_e);  // <= kIdmapSelfPrefixTiles: the launcher checks the bound
-        int v[kSelfTilesPerLane];
+    if constexpr (kMode != kFromPrefix) {
+        // (<= kLinesInLds entries: the launcher checks the bound)
+        const int n_entries = (int)(kMode == kFromBits ? (n_e + kMarkLine - 1) / kMarkLine : mark_tiles(n_e));
+        const int n_used = (n_entries + kBlock - 1) / kBlock * kBlock;
+        for (int i = threadIdx.x; i < n_used; i += kBlock)
+            s_prefix[i] = i < n_entries ? (kMode == kFromBits ? line_count(marks, i) : tile_counts[i]) : 0;
+        __syncthreads();
+        const int per_lane = n_used / kBlock;  // <= kEntriesPerLane
         int s = 0;
-#pragma unroll
-        for (int j = 0; j < kSelfTilesPerLane; ++j) {
-            const int i = (int)threadIdx.x * kSelfTilesPerLane + j;
-            v[j] = i < n_tiles ? tile_sums[i] : 0;
-            s += v[j];
-        }
+        for (int j = 0; j < per_lane; ++j) s += s_prefix[(int)threadIdx.x * per_lane + j];
         int total;
         int run = block_exclusive_scan<kBlock>(s, smem, &total);
-#pragma unroll
-        for (int j = 0; j < kSelfTilesPerLane; ++j) {
-            s_prefix[(int)threadIdx.x * kSelfTilesPerLane + j] = run;
-            run += v[j];
+        for (int j = 0; j < per_lane; ++j) {
+            const int c = s_prefix[(int)threadIdx.x * per_lane + j];
+            s_prefix[(int)threadIdx.x * per_lane + j] = run;
+            run += c;
         }
         __syncthreads();
         if (blockIdx.x == 0 && threadIdx.x == 0) publish_node_total(n_base, total, capacity, d_n_total_out, d_status, readback, rb_counts, rb_n);
-    }
-    // the last pass of a mini-batch, which no longer reads the table, can leave it empty for the next one
-    // (first, so that the stores drain while the edges are being numbered)
-    if (!WRITE_BACK && clear_words != nullptr) {
-        uint4* v = reinterpret_cast<uint4*>(clear_words);  // (a table is 8-byte slots, a power of two of them, 16-byte aligned)
-        const uint4 empty = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
-        for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n_clear_words / 4; i += stride) v[i] = empty;
     }
     // (the trip count is the same for all lanes of a wave: they add up their next-hop tile sums together)
     for (int64_t base = (int64_t)blockIdx.x * kBlock; base < n_e; base += stride) {
@@ -424,26 +290,46 @@ __global__ __launch_bounds__(kBlock) void idmap_number_kernel(TableRef t, const 
         int next_k = 0, next_tile = 0;
         const bool first_trip = base == (int64_t)blockIdx.x * kBlock;
         const uint32_t p = first_trip ? p_ahead : (e < n_e ? slot_of[e] : kDone);
-        int32_t id = first_trip ? id_ahead : 0;
+        const unsigned long long bits = first_trip ? bits_ahead : (e < n_e ? marks.bits[e >> 6] : 0ull);
+        const bool is_first = p < kDone && ((bits >> (e & 63)) & 1ull);
+        int32_t id = 0;
+        if (is_first) id = first_trip ? id_ahead : src[e];
         int64_t row_a = kRowBadId, row_deg = 0;
-        if (next.row_start != nullptr && p < kDone) {  // most such edges are first mentions: fetch their node's row now
-            if (!first_trip) id = src[e];
-            load_row_of(next, id, &row_a, &row_deg);
-        }
+        if (next.row_start != nullptr && is_first) load_row_of(next, id, &row_a, &row_deg);
         if (p != kDone) {
             int64_t local = -1;
-            if (p != kEmpty) {
-                const int64_t ef = (int64_t)((first_trip ? first_ahead : first_of[e]) & ~kPending);  // first edge of this edge's id (ef <= e)
-                if (ef < n_e) {
-                    const int64_t tile = ef / kTile;
-                    const int before_tile = SELF ? s_prefix[tile] : tile_prefix[tile];
-                    local = n_base + before_tile + before8[ef >> 3] + __popc((uint32_t)flags8[ef >> 3] & ((1u << (ef & 7)) - 1u));
+            if (p < kDone) {
+                int64_t ef = e;
+                if (!is_first) {
+                    const uint32_t v = t.words[2 * (size_t)p + 1];
+                    if (v & kPending) ef = (int64_t)(v & ~kPending);  // first edge of this edge's id (< e)
+                    else {
+                        local = v;
+                        ef = n_e;
+                    }
                 }
-                if (local >= capacity) local = -1;  // the unique list is full (reported with the node total)
-                if (ef == e && local >= 0) {
-                    if (next.row_start == nullptr && !first_trip) id = src[e];
+                if (ef < n_e) {
+                    local = n_base + marks_before_in_line(marks, ef);
+                    if (kMode == kFromBits) {
+                        local += s_prefix[ef / kMarkLine];
+                    } else {
+                        const int64_t tile = ef / kMarkTile;
+                        local += kMode == kFromTiles ? s_prefix[tile] : tile_counts[tile];
+                        const int4* c = reinterpret_cast<const int4*>(line_counts + tile * (kMarkTile / kMarkLine));
+                        const int4 a = c[0], b = c[1];
+                        const int before[7] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z};
+#pragma unroll
+                        for (int j = 0; j < 7; ++j) local += j < (int)(ef / kMarkLine % (kMarkTile / kMarkLine)) ? before[j] : 0;
+                    }
+                }
+                if (local < 0 || local >= capacity) local = -1;  // the unique list is full (reported with the node total)
+                if (is_first && local < 0) {
+                    // (left unnumbered, and without an edge's index: a later hop that meets the id must not take this hop's
+                    // edge for one of its own)
+                    if (WRITE_BACK) t.words[2 * (size_t)p + 1] = kEmpty;
+                } else if (is_first) {
                     uniq[local] = id;
-                    if (WRITE_BACK) t.words[2 * (size_t)(p & ~kHolderBit) + 1] = (uint32_t)local;
+                    if (WRITE_BACK) t.words[2 * (size_t)p + 1] = (uint32_t)local;
                     if (next.row_start != nullptr) {
                         next_k = store_next_hop(next, local, row_a, row_deg);
                         next_tile = (int)(local / next.tile_seeds);
@@ -489,11 +375,10 @@ __global__ __launch_bounds__(kBlock) void idmap_insert_arrival_kernel(TableRef t
                                                                       uint32_t* __restrict__ slot_of, int32_t* __restrict__ counter,
                                                                       int32_t* __restrict__ uniq, int64_t capacity, int32_t* out,
                                                                       uint32_t* __restrict__ d_status, const NextHop next,
-                                                                      const TransposeRank tr, const TransposeJob before)
+                                                                      const TransposeRank tr)
 {
     __shared__ int smem[kBlock / kWave + 1];
     __shared__ int s_base;
-    tjob_scan<kBlock>(before);  // (the hop before, if its transposed block is being built: counters -> offsets)
     constexpr int kNextTiles = kBlock * ITEMS / kWave + 2;  // next-hop tiles (64 seeds or more each) that a tile's new nodes can touch
     __shared__ int s_next[kNextTiles];
     unsigned long long* slots = reinterpret_cast<unsigned long long*>(t.words);
@@ -608,10 +493,12 @@ __global__ __launch_bounds__(kBlock) void idmap_relabel_publish_kernel(TableRef 
                                                                        int64_t n_base_h, const int32_t* __restrict__ d_n_base,
                                                                        int64_t capacity, int32_t* __restrict__ d_n_total_out,
                                                                        uint32_t* __restrict__ d_status, const TransposeRank tr,
-                                                                       const TransposeJob before, int32_t* __restrict__ readback,
+                                                                       const TransposeJob scan, const TransposeJob zero,
+                                                                       int32_t* __restrict__ readback,
                                                                        const int32_t* __restrict__ rb_counts, int rb_n)
 {
-    tjob_fill<kBlock>(before);  // (the hop before, if its transposed block is being built: entries into their rows)
+    tjob_scan<kBlock>(scan);  // (carried along for the hops around this one, as in idmap_number_kernel)
+    tjob_zero<kBlock>(zero);
     const int64_t n_e = actual_count(e_max, d_e);
     const int64_t stride = (int64_t)gridDim.x * kBlock;
     for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < n_e; e += stride) {
@@ -667,28 +554,51 @@ int launch_idmap_insert_dst(void* d_table, int64_t slots, const int32_t* d_dst_i
     return FGL_OK;
 }
 
-size_t idmap_map_src_workspace_bytes(int64_t n_edges_max)
+// the workspace of map_src: one slot index per edge, the counts of inputs too large to do without, the marks
+struct IdmapScratch {
+    uint32_t* slot_of;
+    int32_t* line_counts;
+    int32_t* tile_sums;
+    int32_t* tile_prefix;
+    MentionMarks marks;
+    size_t used;
+};
+static IdmapScratch carve_idmap(void* ws, int64_t n_edges_max, bool with_marks)
 {
-    const int64_t tiles = ceil_div(n_edges_max > 0 ? n_edges_max : 1, kTile);
-    Carver c(nullptr);
-    c.take<uint32_t>((size_t)n_edges_max);      // slot_of
-    c.take<uint32_t>((size_t)n_edges_max);      // first_of
-    c.take<uint8_t>((size_t)tiles * kBlock);    // flags8
-    c.take<uint16_t>((size_t)tiles * kBlock);   // before8
-    c.take<int32_t>((size_t)tiles);             // tile sums
-    c.take<int32_t>((size_t)tiles);             // tile prefix
-    c.take<uint32_t>((size_t)(n_edges_max + 3) / 4);  // one byte per edge ("displaced as first mention"), used by fgl_idmap_transfer
-    return c.used();
+    Carver c(ws);
+    IdmapScratch o{};
+    o.slot_of = c.take<uint32_t>((size_t)n_edges_max);
+    o.line_counts = c.take<int32_t>((size_t)mark_tiles(n_edges_max) * (kMarkTile / kMarkLine));
+    o.tile_sums = c.take<int32_t>((size_t)mark_tiles(n_edges_max));
+    o.tile_prefix = c.take<int32_t>((size_t)mark_tiles(n_edges_max));
+    if (with_marks) o.marks = marks_at(c.take<uint32_t>(mark_words(n_edges_max)));
+    o.used = c.used();
+    return o;
+}
+
+size_t idmap_map_src_workspace_bytes(int64_t n_edges_max, bool with_marks) { return carve_idmap(nullptr, n_edges_max, with_marks).used; }
+
+InsertWork idmap_insert_work(void* d_table, int64_t slots, void* d_ws, int64_t n_edges_max, int32_t* d_src_out, const MentionMarks& marks,
+                             const TransposeJob* rank_job)
+{
+    InsertWork w;
+    w.t = make_ref(d_table, slots);
+    w.slot_of = carve_idmap(d_ws, n_edges_max, false).slot_of;
+    w.out = d_src_out;
+    w.marks = marks;
+    w.rank = rank_of(rank_job);
+    return w;
 }
 
 int launch_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, int32_t* d_src_out, int64_t n_edges_max,
                          const int32_t* d_n_edges, int64_t n_base, const int32_t* d_n_base, int32_t* d_n_total_out,
                          int32_t* d_uniq, int64_t uniq_capacity, int flags, uint32_t* d_status, void* d_ws,
-                         size_t ws_bytes, hipStream_t stream, bool counter_is_zeroed, const NextHop* next_hop,
-                         bool leave_table_empty, uint8_t* d_lowered, const TransposeJob* rank_job,
-                         const TransposeJob* before_job, int32_t* d_dst_inout, int32_t* d_readback,
-                         const int32_t* d_readback_counts, int n_readback_counts)
+                         size_t ws_bytes, hipStream_t stream, bool counter_is_zeroed, bool leave_table_empty,
+                         const MapSrcExtras* extras)
 {
+    MapSrcExtras x;
+    memset(&x, 0, sizeof(x));
+    if (extras != nullptr) x = *extras;
     FGL_REQUIRE(d_table != nullptr && valid_slots(slots), "idmap: slot count %lld is not a power of two in [64, 2^31]", (long long)slots);
     FGL_REQUIRE((flags & ~(FGL_IDMAP_ARRIVAL | FGL_IDMAP_FINAL)) == 0, "idmap_map_src: unknown flags %d", flags);
     const bool final_call = (flags & FGL_IDMAP_FINAL) != 0;
@@ -696,114 +606,120 @@ int launch_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, 
     FGL_REQUIRE(n_base + n_edges_max <= 0x7FFFFFFDll, "idmap_map_src: n_base + n_edges exceeds 31 bits");
     FGL_REQUIRE(n_edges_max == 0 || (d_src_in && d_src_out && d_uniq), "idmap_map_src: null pointer");
     FGL_REQUIRE(d_n_total_out == nullptr || d_n_total_out != d_n_base, "idmap_map_src: n_total_out must not alias n_base");
-    if (d_ws == nullptr || ws_bytes < idmap_map_src_workspace_bytes(n_edges_max)) {
-        set_error("idmap_map_src: workspace too small (%zu < %zu)", ws_bytes, idmap_map_src_workspace_bytes(n_edges_max));
+    const bool own_marks = x.marks.bits == nullptr;
+    if (d_ws == nullptr || ws_bytes < idmap_map_src_workspace_bytes(n_edges_max, own_marks)) {
+        set_error("idmap_map_src: workspace too small (%zu < %zu)", ws_bytes, idmap_map_src_workspace_bytes(n_edges_max, own_marks));
         return FGL_ERR_WORKSPACE;
     }
     FGL_REQUIRE(((uintptr_t)d_ws & 15) == 0, "idmap_map_src: the workspace must be 16-byte aligned");
-    const int64_t tiles = ceil_div(n_edges_max > 0 ? n_edges_max : 1, kTile);
-    Carver c(d_ws);
-    uint32_t* slot_of = c.take<uint32_t>((size_t)n_edges_max);
-    uint32_t* first_of = c.take<uint32_t>((size_t)n_edges_max);
-    uint8_t* flags8 = c.take<uint8_t>((size_t)tiles * kBlock);
-    uint16_t* before8 = c.take<uint16_t>((size_t)tiles * kBlock);
-    int32_t* sums = c.take<int32_t>((size_t)tiles);
-    int32_t* prefix = c.take<int32_t>((size_t)tiles);
+    const int64_t tiles = mark_tiles(n_edges_max);
+    const IdmapScratch ws = carve_idmap(d_ws, n_edges_max, own_marks);
+    uint32_t* slot_of = ws.slot_of;
     const TableRef t = make_ref(d_table, slots);
     unsigned edge_blocks = stride_grid(n_edges_max, kBlock);
-    const unsigned tile_blocks = stride_grid(n_edges_max, kTile);
     NextHop next{};  // all null: nothing to prepare
-    if (next_hop != nullptr) next = *next_hop;
-    const TransposeRank tr = rank_of(rank_job);
-    TransposeJob before;
-    memset(&before, 0, sizeof(before));
-    if (before_job != nullptr) before = *before_job;
-    // the two passes that carry the hop before's scan and fill steps get workgroups of their own for those,
+    if (x.next_hop != nullptr) next = *x.next_hop;
+    const TransposeRank tr = rank_of(x.rank_job);
+    // the last pass carries steps for the transposed blocks of the hops around this one, in workgroups of their own
     // behind the pass's own
-    TransposeJob scan_job = before, fill_job = before;
-    unsigned scan_blocks = 0, fill_blocks_t = 0;
-    if (before.cnt != nullptr) {
-        scan_job.side_first = fill_job.side_first = 0;
-        scan_blocks = scan_job.side_blocks = side_blocks_for(before.cols_max * before.split + 1, kTjobTile);
-        fill_blocks_t = fill_job.side_blocks = side_blocks_for(before.rows_max, kBlock / 16, 16384);
+    TransposeJob scan, zero;
+    memset(&scan, 0, sizeof(scan));
+    memset(&zero, 0, sizeof(zero));
+    ZeroJob zero_marks{};
+    unsigned side_blocks = 0;
+    if (x.scan_job != nullptr && x.scan_job->cnt != nullptr) {
+        scan = *x.scan_job;
+        scan.side_first = (int)side_blocks;
+        scan.side_blocks = side_blocks_for(scan.cols_max * scan.split + 1, kTjobTile);
+        side_blocks += (unsigned)scan.side_blocks;
+    }
+    if (x.zero_job != nullptr && x.zero_job->cnt != nullptr) {
+        zero = *x.zero_job;
+        zero.side_first = (int)side_blocks;
+        zero.side_blocks = side_blocks_for(zero.cols_max * zero.split + 1, kBlock * 16);
+        side_blocks += (unsigned)zero.side_blocks;
+    }
+    if (x.zero_marks.n16 > 0 && !(flags & FGL_IDMAP_ARRIVAL)) {
+        zero_marks = x.zero_marks;
+        zero_marks.side_first = (int)side_blocks;
+        zero_marks.side_blocks = side_blocks_for(zero_marks.n16, kBlock * 4);
+        side_blocks += (unsigned)zero_marks.side_blocks;
     }
     FGL_REQUIRE(!leave_table_empty || final_call, "idmap_map_src: only a final call can leave the table empty");
 
     if (flags & FGL_IDMAP_ARRIVAL) {
-        if (d_dst_inout != nullptr && n_edges_max > 0) {  // (this numbering's passes do not carry the destination half: a launch of its own)
-            hipLaunchKernelGGL(idmap_lookup_kernel, dim3(edge_blocks), dim3(kBlock), 0, stream, t, d_dst_inout, n_edges_max, d_n_edges, d_status);
+        if (x.d_dst_inout != nullptr && n_edges_max > 0) {  // (this numbering's passes do not carry the destination half: a launch of its own)
+            hipLaunchKernelGGL(idmap_lookup_kernel, dim3(edge_blocks), dim3(kBlock), 0, stream, t, x.d_dst_inout, n_edges_max, d_n_edges, d_status);
             FGL_CHECK_LAUNCH("idmap_lookup_kernel");
         }
         // the counter of new ids: *d_n_total_out itself when the caller vouches that it holds zero (the all-hops
         // entry point zeroes its counts when it resets the table), else one int of the (otherwise unused)
-        // tile-sum array, zeroed by a launch of its own
-        int32_t* counter = (counter_is_zeroed && d_n_total_out) ? d_n_total_out : sums;
-        if (counter == sums) {
+        // prefix array, zeroed by a launch of its own
+        int32_t* counter = (counter_is_zeroed && d_n_total_out) ? d_n_total_out : ws.tile_prefix;
+        if (counter == ws.tile_prefix) {
             int rc0 = launch_fill_u32(reinterpret_cast<uint32_t*>(counter), 1, 0u, stream);
             if (rc0 != FGL_OK) return rc0;
         }
         if (n_edges_max > kArrivalSmallEdges)
-            hipLaunchKernelGGL(idmap_insert_arrival_kernel<kArrivalItems>,
-                               dim3(stride_grid(n_edges_max, kBlock * kArrivalItems) + scan_blocks),
+            hipLaunchKernelGGL(idmap_insert_arrival_kernel<kArrivalItems>, dim3(stride_grid(n_edges_max, kBlock * kArrivalItems)),
                                dim3(kBlock), 0, stream, t, d_src_in,
                                n_edges_max, d_n_edges, n_base, d_n_base, slot_of, counter, d_uniq, uniq_capacity, d_src_out,
-                               d_status, next, tr, scan_job);
+                               d_status, next, tr);
         else
-            hipLaunchKernelGGL(idmap_insert_arrival_kernel<1>, dim3(edge_blocks + scan_blocks), dim3(kBlock), 0, stream, t, d_src_in,
+            hipLaunchKernelGGL(idmap_insert_arrival_kernel<1>, dim3(edge_blocks), dim3(kBlock), 0, stream, t, d_src_in,
                                n_edges_max, d_n_edges, n_base, d_n_base, slot_of, counter, d_uniq, uniq_capacity, d_src_out,
-                               d_status, next, tr, scan_job);
+                               d_status, next, tr);
         FGL_CHECK_LAUNCH("idmap_insert_arrival_kernel");
-        hipLaunchKernelGGL(idmap_relabel_publish_kernel, dim3(edge_blocks + fill_blocks_t), dim3(kBlock), 0, stream, t, n_edges_max, d_n_edges,
-                           slot_of, d_src_out, counter, n_base, d_n_base, uniq_capacity, d_n_total_out, d_status, tr, fill_job, d_readback,
-                           d_readback_counts, n_readback_counts);
+        hipLaunchKernelGGL(idmap_relabel_publish_kernel, dim3(edge_blocks + side_blocks), dim3(kBlock), 0, stream, t, n_edges_max, d_n_edges,
+                           slot_of, d_src_out, counter, n_base, d_n_base, uniq_capacity, d_n_total_out, d_status, tr, scan, zero, x.d_readback,
+                           x.d_readback_counts, x.n_readback_counts);
         FGL_CHECK_LAUNCH("idmap_relabel_publish_kernel");
-        // (the second pass reads the table, so emptying it takes a launch of its own here)
-        if (leave_table_empty) return launch_fill_u32(t.words, slots * 2, kEmpty, stream);
-        return FGL_OK;
-    }
-
-    // (the holder bit shares a word with the slot index: tables of 2^31 slots go without the bookkeeping)
-    uint8_t* lowered = slots <= ((int64_t)1 << 30) ? d_lowered : nullptr;
-    // (small inputs need the workgroups more than the edges in flight per lane)
-    if (n_edges_max > kArrivalSmallEdges)
-        hipLaunchKernelGGL(idmap_insert_src_kernel<FGL_INSERT_ITEMS>, dim3(stride_grid(n_edges_max, kBlock * FGL_INSERT_ITEMS) + scan_blocks),
-                           dim3(kBlock), 0, stream, t, d_src_in, n_edges_max, d_n_edges, slot_of, d_src_out, lowered, d_status, tr, scan_job,
-                           d_dst_inout);
-    else
-        hipLaunchKernelGGL(idmap_insert_src_kernel<1>, dim3(edge_blocks + scan_blocks), dim3(kBlock), 0, stream, t, d_src_in,
-                           n_edges_max, d_n_edges, slot_of, d_src_out, lowered, d_status, tr, scan_job, d_dst_inout);
-    FGL_CHECK_LAUNCH("idmap_insert_src_kernel");
-    hipLaunchKernelGGL(idmap_mark_kernel, dim3(tile_blocks + fill_blocks_t), dim3(kBlock), 0, stream, t, n_edges_max, d_n_edges,
-                       slot_of, lowered, first_of, flags8, before8, sums, fill_job);
-    FGL_CHECK_LAUNCH("idmap_mark_kernel");
-#define FGL_LAUNCH_NUMBER(SELF, WB, PREFIX, TOTAL, STATUS, READBACK)                                                              \
-    hipLaunchKernelGGL((idmap_number_kernel<SELF, WB>), dim3(edge_blocks), dim3(kBlock), 0, stream, t, d_src_in,        \
-                       n_edges_max, d_n_edges, n_base, d_n_base, slot_of, first_of, flags8, before8, sums, PREFIX, d_uniq, \
-                       uniq_capacity, d_src_out, TOTAL, STATUS, next, clear_words, n_clear_words, tr, READBACK, d_readback_counts,   \
-                       n_readback_counts)
-    // emptying the table rides on the last pass: enough workgroups for a fill of that size
-    uint32_t* clear_words = leave_table_empty ? t.words : nullptr;
-    const int64_t n_clear_words = leave_table_empty ? slots * 2 : 0;
-    if (leave_table_empty) {
-        const unsigned fill_blocks = stride_grid(n_clear_words, kBlock * 8);
-        if (fill_blocks > edge_blocks) edge_blocks = fill_blocks;
-    }
-    // every workgroup of a pass that scans the tile counts itself pays for that scan once: a few workgroups per
-    // compute unit, each looping over several tiles of edges, instead of one per 256 edges
-    if (tiles <= kIdmapSelfPrefixTiles && edge_blocks > FGL_NUMBER_SELF_MAX_BLOCKS) edge_blocks = FGL_NUMBER_SELF_MAX_BLOCKS;
-    if (tiles <= kIdmapSelfPrefixTiles) {
-        if (final_call) FGL_LAUNCH_NUMBER(true, false, nullptr, d_n_total_out, d_status, d_readback);
-        else FGL_LAUNCH_NUMBER(true, true, nullptr, d_n_total_out, d_status, d_readback);
     } else {
-        hipLaunchKernelGGL(idmap_prefix_publish_kernel, dim3(1), dim3(1024), 0, stream, sums, prefix, n_edges_max,
-                           d_n_edges, n_base, d_n_base, uniq_capacity, d_n_total_out, d_status, d_readback, d_readback_counts,
-                           n_readback_counts);
-        FGL_CHECK_LAUNCH("idmap_prefix_publish_kernel");
-        if (final_call) FGL_LAUNCH_NUMBER(false, false, prefix, nullptr, nullptr, nullptr);
-        else FGL_LAUNCH_NUMBER(false, true, prefix, nullptr, nullptr, nullptr);
-    }
+        MentionMarks marks = x.marks;
+        if (own_marks) {  // (nobody has cleared them)
+            marks = ws.marks;
+            int rc0 = launch_fill_u32(reinterpret_cast<uint32_t*>(marks.bits), (int64_t)mark_words(n_edges_max), 0u, stream);
+            if (rc0 != FGL_OK) return rc0;
+        }
+        if (!x.inserted) {
+            const InsertWork w = idmap_insert_work(d_table, slots, d_ws, n_edges_max, d_src_out, marks, x.rank_job);
+            hipLaunchKernelGGL(idmap_insert_src_kernel, dim3(edge_blocks), dim3(kBlock), 0, stream, d_src_in, n_edges_max, d_n_edges, w,
+                               d_status, x.d_dst_inout);
+            FGL_CHECK_LAUNCH("idmap_insert_src_kernel");
+        }
+#define FGL_LAUNCH_NUMBER(MODE, WB, TILES, TOTAL, STATUS, READBACK)                                                              \
+    hipLaunchKernelGGL((idmap_number_kernel<MODE, WB>), dim3(edge_blocks + side_blocks), dim3(kBlock), 0, stream, t, d_src_in,    \
+                       n_edges_max, d_n_edges, n_base, d_n_base, slot_of, marks, ws.line_counts, TILES, d_uniq, uniq_capacity,      \
+                       d_src_out, TOTAL, STATUS, next, tr, scan, zero, zero_marks, (int)side_blocks, READBACK, x.d_readback_counts, \
+                       x.n_readback_counts)
+        const bool from_bits = n_edges_max <= (int64_t)kLinesInLds * kMarkLine;
+        if (!from_bits) {
+            const int64_t count_blocks = ceil_div(tiles * (kMarkTile / kMarkLine), kBlock);
+            hipLaunchKernelGGL(idmap_count_kernel, dim3((unsigned)(count_blocks < 2048 ? count_blocks : 2048)), dim3(kBlock), 0, stream, marks,
+                               n_edges_max, d_n_edges, ws.line_counts, ws.tile_sums);
+            FGL_CHECK_LAUNCH("idmap_count_kernel");
+        }
+        // every workgroup of a pass that scans the counts itself pays for that scan once: a few workgroups per
+        // compute unit, each looping over several tiles of edges, instead of one per 256 edges
+        if (tiles <= kLinesInLds) {
+            if (edge_blocks > kNumberMaxBlocks) edge_blocks = kNumberMaxBlocks;
+            if (from_bits && final_call) FGL_LAUNCH_NUMBER(kFromBits, false, nullptr, d_n_total_out, d_status, x.d_readback);
+            else if (from_bits) FGL_LAUNCH_NUMBER(kFromBits, true, nullptr, d_n_total_out, d_status, x.d_readback);
+            else if (final_call) FGL_LAUNCH_NUMBER(kFromTiles, false, ws.tile_sums, d_n_total_out, d_status, x.d_readback);
+            else FGL_LAUNCH_NUMBER(kFromTiles, true, ws.tile_sums, d_n_total_out, d_status, x.d_readback);
+        } else {
+            hipLaunchKernelGGL(idmap_prefix_publish_kernel, dim3(1), dim3(1024), 0, stream, ws.tile_sums, ws.tile_prefix, n_edges_max,
+                               d_n_edges, n_base, d_n_base, uniq_capacity, d_n_total_out, d_status, x.d_readback, x.d_readback_counts,
+                               x.n_readback_counts);
+            FGL_CHECK_LAUNCH("idmap_prefix_publish_kernel");
+            if (final_call) FGL_LAUNCH_NUMBER(kFromPrefix, false, ws.tile_prefix, nullptr, nullptr, nullptr);
+            else FGL_LAUNCH_NUMBER(kFromPrefix, true, ws.tile_prefix, nullptr, nullptr, nullptr);
+        }
 #undef FGL_LAUNCH_NUMBER
-    FGL_CHECK_LAUNCH("idmap_number_kernel");
+        FGL_CHECK_LAUNCH("idmap_number_kernel");
+    }
+    // (the last pass reads the table: emptying it takes a launch of its own)
+    if (leave_table_empty) return launch_idmap_reset(d_table, slots, stream);
     return FGL_OK;
 }
 
@@ -841,7 +757,7 @@ FGL_EXPORT int fgl_idmap_insert_dst(void* d_table, int64_t slots, const int32_t*
     return launch_idmap_insert_dst(d_table, slots, d_dst_ids, n_max, d_n, d_uniq, d_status, as_stream(stream), nullptr, 0);
 }
 
-FGL_EXPORT size_t fgl_idmap_map_src_workspace_bytes(int64_t n_edges_max) { return idmap_map_src_workspace_bytes(n_edges_max < 0 ? 0 : n_edges_max); }
+FGL_EXPORT size_t fgl_idmap_map_src_workspace_bytes(int64_t n_edges_max) { return idmap_map_src_workspace_bytes(n_edges_max < 0 ? 0 : n_edges_max, true); }
 
 FGL_EXPORT int fgl_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, int32_t* d_src_out,
                                  int64_t n_edges_max, const int32_t* d_n_edges, int64_t n_base, const int32_t* d_n_base,
@@ -852,7 +768,7 @@ FGL_EXPORT int fgl_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_
     FGL_REQUIRE(!leave_empty || (flags & FGL_IDMAP_FINAL), "idmap_map_src: FGL_IDMAP_LEAVE_TABLE_EMPTY needs FGL_IDMAP_FINAL");
     return launch_idmap_map_src(d_table, slots, d_src_in, d_src_out, n_edges_max, d_n_edges, n_base, d_n_base,
                                 d_n_total_out, d_uniq, uniq_capacity, flags & ~FGL_IDMAP_LEAVE_TABLE_EMPTY, d_status, d_ws, ws_bytes,
-                                as_stream(stream), false, nullptr, leave_empty, nullptr, nullptr, nullptr, nullptr);
+                                as_stream(stream), false, leave_empty, nullptr);
 }
 
 FGL_EXPORT int fgl_idmap_transfer(void* d_table, int64_t slots, const int32_t* d_dst_unique, int64_t n_dst,
@@ -866,27 +782,23 @@ FGL_EXPORT int fgl_idmap_transfer(void* d_table, int64_t slots, const int32_t* d
     FGL_REQUIRE(d_uniq != nullptr && uniq_capacity >= n_dst, "idmap_transfer: the unique list cannot hold the destination ids");
     const bool leave_empty = (flags & FGL_IDMAP_LEAVE_TABLE_EMPTY) != 0;
     FGL_REQUIRE(!leave_empty || (flags & FGL_IDMAP_FINAL), "idmap_transfer: FGL_IDMAP_LEAVE_TABLE_EMPTY needs FGL_IDMAP_FINAL");
-    if (d_ws == nullptr || ws_bytes < idmap_map_src_workspace_bytes(n_edges)) {
-        set_error("idmap_transfer: workspace too small (%zu < %zu)", ws_bytes, idmap_map_src_workspace_bytes(n_edges));
+    if (d_ws == nullptr || ws_bytes < idmap_map_src_workspace_bytes(n_edges, true)) {
+        set_error("idmap_transfer: workspace too small (%zu < %zu)", ws_bytes, idmap_map_src_workspace_bytes(n_edges, true));
         return FGL_ERR_WORKSPACE;
     }
-    // the last piece of the workspace: one byte per edge that lets the mark pass skip most of its table reads;
-    // cleared by the launch that inserts the destination ids
-    const int64_t tiles = ceil_div(n_edges > 0 ? n_edges : 1, kTile);
-    Carver c(d_ws);
-    c.take<uint32_t>((size_t)n_edges);
-    c.take<uint32_t>((size_t)n_edges);
-    c.take<uint8_t>((size_t)tiles * kBlock);
-    c.take<uint16_t>((size_t)tiles * kBlock);
-    c.take<int32_t>((size_t)tiles);
-    c.take<int32_t>((size_t)tiles);
-    uint32_t* lowered_words = c.take<uint32_t>((size_t)(n_edges + 3) / 4);
-    int rc = launch_idmap_insert_dst(d_table, slots, d_dst_unique, n_dst, nullptr, d_uniq, d_status, as_stream(stream), lowered_words,
-                                     (n_edges + 3) / 4);
+    FGL_REQUIRE(((uintptr_t)d_ws & 15) == 0, "idmap_transfer: the workspace must be 16-byte aligned");
+    // the marks of the source ids' first mentions are cleared by the launch that inserts the destination ids
+    MapSrcExtras x;
+    memset(&x, 0, sizeof(x));
+    x.marks = carve_idmap(d_ws, n_edges, true).marks;
+    x.d_dst_inout = d_dst_edges;
+    x.d_readback = d_readback;
+    int rc = launch_idmap_insert_dst(d_table, slots, d_dst_unique, n_dst, nullptr, d_uniq, d_status, as_stream(stream),
+                                     reinterpret_cast<uint32_t*>(x.marks.bits), (int64_t)mark_words(n_edges));
     if (rc != FGL_OK) return rc;
     return launch_idmap_map_src(d_table, slots, d_src_edges, d_src_edges, n_edges, nullptr, n_dst, nullptr, d_n_total_out, d_uniq,
                                 uniq_capacity, flags & ~FGL_IDMAP_LEAVE_TABLE_EMPTY, d_status, d_ws, ws_bytes, as_stream(stream), false,
-                                nullptr, leave_empty, reinterpret_cast<uint8_t*>(lowered_words), nullptr, nullptr, d_dst_edges, d_readback);
+                                leave_empty, &x);
 }
 
 FGL_EXPORT int fgl_idmap_lookup(const void* d_table, int64_t slots, int32_t* d_ids, int64_t n_max, const int32_t* d_n,

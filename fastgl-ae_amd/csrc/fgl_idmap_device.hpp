@@ -4,15 +4,23 @@
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_table.hpp"
+#include "fgl_transpose_job.hpp"
 
 namespace fgl {
 
+// what a launch needs to insert the ids of a hop's edges (idmap_insert_src_kernel, the sampling kernels)
+struct InsertWork {
+    TableRef t;
+    uint32_t* slot_of;  // per edge: the id's slot; kDone: relabelled already; kEmpty: no slot
+    int32_t* out;       // the edges' local ids
+    MentionMarks marks;
+    TransposeRank rank;
+};
+
 #if defined(__HIPCC__)
 
-constexpr uint32_t kHolderBit = 0x80000000u;  // slot_of[]: the edge was the first known mention of its id when its insert ran
-
-// find_or_insert for an edge's source id, which also says what the mark pass would otherwise have to read back
-// from the table: *holder = this edge became the first known mention of the id (it installed the key, or lowered
+// find_or_insert for an edge's source id, which also says what becomes of the marks:
+// *holder = this edge became the first known mention of the id (it installed the key, or lowered
 // the key's first-edge index to its own); *displaced = the pending value it took that place from (kEmpty: none).
 // An edge that became holder and is never displaced is the id's first mention.
 // The probe sequence is entered at slot p with that slot's value already in hand (`s`: loaded, or returned by a
@@ -53,6 +61,58 @@ __device__ __forceinline__ uint32_t insert_mention_from(const TableRef t, uint32
         s = slots[p];
     }
     return kEmpty;
+}
+
+// What is left of edge e's insert once its slot is known (q; kEmpty: none found): the slot is noted for the number pass, or the
+// edge relabelled here and now; the edge whose place it took loses its mark.  n_e bounds the indices that marks exist for.
+__device__ __forceinline__ void finish_insert(const InsertWork& w, int64_t e, int64_t n_e, int32_t id, uint32_t q, uint32_t seen,
+                                              uint32_t displaced, uint32_t* __restrict__ d_status)
+{
+    if (q == kEmpty) {
+        // table full, or not a node id: reported; the edge's local id becomes -1 (written by the number pass)
+        if (d_status) atomicOr(d_status, id >= 0 ? FGL_STATUS_TABLE_FULL : FGL_STATUS_BAD_ID);
+    } else if (!(seen & kPending)) {
+        // numbered in an earlier hop (or a destination node): the edge is relabelled right here and
+        // takes no further part (`out` may be the array the id came from: this lane is the only one that touches entry e)
+        w.out[e] = (int32_t)seen;
+        take_rank(w.rank, e, (int32_t)seen);
+        q = kDone;
+    } else if (displaced != kEmpty) {
+        // (an edge of this hop: ids of earlier hops hold their local id, or all ones if the unique list had no room for them.
+        // The bound only matters to a caller that goes on with a table which a final call has left unnumbered.)
+        const int64_t d = (int64_t)(displaced & ~kPending);
+        if (d < n_e) atomicXor(&w.marks.bits[d >> 6], 1ull << (d & 63));
+    }
+    w.slot_of[e] = q;
+}
+
+// The marks of the wave's edges that became holders: lane l's edge is first + l.  Every lane of the wave calls it.
+__device__ __forceinline__ void mark_first(const MentionMarks& m, int64_t first, bool holder)
+{
+    const unsigned long long won = __ballot(holder);
+    const int lane = lane_id(), off = (int)(first & 63);
+    if (lane == 0 && (won << off) != 0) atomicXor(&m.bits[first >> 6], won << off);
+    if (lane == 1 && off != 0 && (won >> (64 - off)) != 0) atomicXor(&m.bits[(first >> 6) + 1], won >> (64 - off));
+}
+
+// marks of a line of edges, and of its edges before edge ef (final once every insert of the hop is done)
+__device__ __forceinline__ int line_count(const MentionMarks& m, int64_t line)
+{
+    const ulonglong2* w = reinterpret_cast<const ulonglong2*>(m.bits + line * (kMarkLine / 64));
+    const ulonglong2 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+    return __popcll(w0.x) + __popcll(w0.y) + __popcll(w1.x) + __popcll(w1.y) + __popcll(w2.x) + __popcll(w2.y) + __popcll(w3.x) + __popcll(w3.y);
+}
+__device__ __forceinline__ int marks_before_in_line(const MentionMarks& m, int64_t ef)
+{
+    const ulonglong2* w = reinterpret_cast<const ulonglong2*>(m.bits + ef / kMarkLine * (kMarkLine / 64));
+    const ulonglong2 w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+    const int word = (int)(ef >> 6) & 7;
+    const unsigned long long bits[8] = {w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
+    const unsigned long long below = (1ull << (ef & 63)) - 1ull;
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) n += __popcll(j < word ? bits[j] : j == word ? bits[j] & below : 0ull);
+    return n;
 }
 
 // A node that has just been given a position in the unique list is a seed of the next hop: its row start and

@@ -74,26 +74,49 @@ __host__ __device__ inline TransposeRank rank_of(const TransposeJob* j)
 {
     return j && j->cnt ? TransposeRank{j->cnt, j->rank, j->cols_max, j->split} : TransposeRank{nullptr, nullptr, 0, 1};
 }
-// what one launch carries along for the transposed blocks: steps of the hop before (tile sums / scan / fill, by the
-// launch's place in the hop) and the zeroing of this hop's counters (sampling launch only)
+// what a hop's sampling launch carries along for the transposed blocks of the hops before it: the tile sums of the last hop's
+// counters, the filling of the rows of the hop before that
 struct TransposeSteps {
-    TransposeJob before;
-    TransposeJob zero;
+    TransposeJob sums;
+    TransposeJob fill;
+};
+// memory to clear in side workgroups of a launch
+struct ZeroJob {
+    uint4* p;
+    int64_t n16;  // 16-byte pieces; 0: no such work
+    int side_blocks, side_first;
 };
 
+// Which edges of a hop are the first mentions of new ids, kept exact while the ids are being inserted: a bit per edge, changed
+// with commutative integer atomics only (fgl_idmap_device.hpp), so that an edge can be marked by its own wave and unmarked by
+// whoever finds an earlier mention, in either order; when the last insert is done they are the final state.  All zero before the
+// first insert of a hop.
+constexpr int kMarkLine = 512;   // edges whose bits are one 64-byte line
+constexpr int kMarkTile = 4096;  // edges per entry of the scanned counts of large hops: eight lines
+struct MentionMarks {
+    unsigned long long* bits;
+};
+__host__ __device__ inline int64_t mark_tiles(int64_t n_edges) { return n_edges > 0 ? (n_edges + kMarkTile - 1) / kMarkTile : 1; }
+inline size_t mark_words(int64_t n_edges) { return (size_t)mark_tiles(n_edges) * (kMarkTile / 32); }  // 32-bit words, a multiple of 4
+inline MentionMarks marks_at(uint32_t* words) { return MentionMarks{reinterpret_cast<unsigned long long*>(words)}; }
+
 // neighbour sampling (fgl_sample.hip)
-int sample_tile_seeds(int fanout, int64_t n_seeds_max);
+int sample_tile_seeds(int fanout, int64_t n_seeds_max);      // seeds per tile of the per-hop operator ...
+int sample_hop_tile_seeds(int fanout, int64_t n_seeds_max);  // ... and of a mini-batch's hops
 int64_t sample_tile_count(int64_t n_seeds_max, int fanout);
 size_t sample_workspace_bytes(int64_t n_seeds_max, int fanout);
 // the second half of launch_sample, for callers that hold row starts, degrees and tile sums already
+struct InsertWork;
+bool sample_can_insert(int fanout, int64_t n_seeds_max);  // the launch can put the ids it samples into the id-map's table itself
 int launch_sample_edges(const int32_t* d_indices, const int32_t* d_seeds, int64_t n_seeds_max, const int32_t* d_n_seeds,
                         int fanout, const int64_t* row_start, const int32_t* deg, const int32_t* tile_sums,
                         int32_t* tile_prefix, uint64_t rng_seed, uint32_t stream_id, int32_t* d_src_out,
                         int32_t* d_dst_out, int32_t* d_block_ptr, int32_t* d_n_edges_out, uint32_t* d_status,
                         hipStream_t stream, const uint32_t* d_stream_add, const NextHop* next,
-                        uint8_t* d_zero_per_edge = nullptr,   // (optional) one byte per output edge, cleared along with the writes
-                        const TransposeSteps* steps = nullptr,   // (optional) zero this hop's counters, tile sums of the hop before
-                        int32_t* d_readback = nullptr);          // (optional) {edge count, status word} once both are final; may be host memory
+                        const TransposeSteps* steps,             // (optional) steps for the transposed blocks of earlier hops
+                        int32_t* d_readback,                     // (optional) {edge count, status word} once both are final; may be host memory
+                        const InsertWork* insert,                // (optional, where sample_can_insert) insert the sampled ids
+                        int tile_seeds);                         // seeds per entry of tile_sums: sample_hop_tile_seeds / sample_tile_seeds
 int launch_sample(const void* d_indptr, int indptr_is64, const int32_t* d_indices, int64_t n_nodes,
                   const int32_t* d_seeds, int64_t n_seeds_max, const int32_t* d_n_seeds, int fanout,
                   uint64_t rng_seed, uint32_t stream_id, int32_t* d_src_out, int32_t* d_dst_out,
@@ -101,25 +124,34 @@ int launch_sample(const void* d_indptr, int indptr_is64, const int32_t* d_indice
                   hipStream_t stream, const uint32_t* d_stream_add = nullptr, int32_t* d_readback = nullptr);
 
 // id-map (fgl_idmap.hip)
-size_t idmap_map_src_workspace_bytes(int64_t n_edges_max);
+size_t idmap_map_src_workspace_bytes(int64_t n_edges_max, bool with_marks);  // with_marks: the marks live there too
 int launch_idmap_reset(void* d_table, int64_t slots, hipStream_t stream);
 int launch_idmap_insert_dst(void* d_table, int64_t slots, const int32_t* d_dst_ids, int64_t n_max,
                             const int32_t* d_n, int32_t* d_uniq, uint32_t* d_status, hipStream_t stream,
                             uint32_t* d_zero_words, int64_t n_zero_words);  // (optional) scratch words to clear on the way
+// what the callers inside the library add to map_src (all optional)
+struct MapSrcExtras {
+    MentionMarks marks;          // cleared already; bits == null: the call clears and uses marks of its own, in its workspace
+    bool inserted;               // the sampling launch has inserted the edges' ids (idmap_insert_work): only the number pass is left
+    const NextHop* next_hop;     // the new nodes are seeds of a next hop: prepare its sampling
+    const TransposeJob* rank_job;  // the edges take their ranks in this block's transposed rows
+    const TransposeJob* scan_job;  // scan step of the hop before, carried by the last pass
+    const TransposeJob* zero_job;  // the next hop's counters, cleared by the last pass
+    ZeroJob zero_marks;            // the next hop's marks, cleared by the last pass (first-occurrence order only)
+    int32_t* d_dst_inout;          // n_edges_max ids that are in the table already: relabelled in place by the first pass
+    int32_t* d_readback;           // {node total, status word} once both are final; may be host memory
+    const int32_t* d_readback_counts;  // instead of those two words: a copy of this array, which holds *d_n_total_out and
+    int n_readback_counts;             //   the status word, taken when the node total is final
+};
 int launch_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, int32_t* d_src_out,
                          int64_t n_edges_max, const int32_t* d_n_edges, int64_t n_base, const int32_t* d_n_base,
                          int32_t* d_n_total_out, int32_t* d_uniq, int64_t uniq_capacity, int flags,
                          uint32_t* d_status, void* d_ws, size_t ws_bytes, hipStream_t stream,
                          bool counter_is_zeroed,          // arrival order: *d_n_total_out holds zero and may count the new ids
-                         const NextHop* next_hop,         // (may be null) the new nodes are seeds of a next hop: prepare its sampling
                          bool leave_table_empty,          // final calls only: every slot of the table is empty when the call's work is done
-                         uint8_t* d_lowered,              // (may be null) n_edges_max bytes, zero on entry: lets the mark pass skip most table reads
-                         const TransposeJob* rank_job = nullptr,     // (may be null) the edges take their ranks in this block's transposed rows
-                         const TransposeJob* before_job = nullptr,   // (may be null) scan and fill steps of the hop before, carried by the first two passes
-                         int32_t* d_dst_inout = nullptr,             // (may be null) n_edges_max ids that are in the table already: relabelled in place by the first pass
-                         int32_t* d_readback = nullptr,              // (may be null) {node total, status word} once both are final; may be host memory
-                         const int32_t* d_readback_counts = nullptr, // (may be null) instead of those two words: a copy of this array, which holds
-                         int n_readback_counts = 0);                 //   *d_n_total_out and the status word, taken when the node total is final
+                         const MapSrcExtras* extras);
+InsertWork idmap_insert_work(void* d_table, int64_t slots, void* d_ws, int64_t n_edges_max, int32_t* d_src_out, const MentionMarks& marks,
+                             const TransposeJob* rank_job);
 
 // counting and transpose of large inputs (fgl_bucket.hip)
 size_t count_workspace_bytes(int64_t n_ids, int64_t n_counters);  // 0: counted with atomics, no workspace

@@ -5,7 +5,8 @@
 //   1. sample_degree_kernel   one lane per seed: two offsets of the row, k = min(fanout, deg),
 //                             staged row start / degree, per-tile sum of k
 //   2. tile prefix            single workgroup; also writes block_ptr[n] and the edge count
-//   3. sample_edges_reg_kernel (fanout <= 32) / sample_edges_kernel (larger fanouts)
+//   3. sample_edges_reg_kernel (fanout <= 32) / sample_edges_kernel (larger fanouts), or, in the small hops of
+//                             a mini-batch, sample_insert_kernel
 //                             per tile of TS seeds: wave64 scan of k -> output offsets,
 //                             Floyd subset selection for rows longer than the fanout (one lane
 //                             per seed, Philox stream keyed by the node id, picks kept in LDS in a
@@ -20,6 +21,7 @@
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_transpose_job.hpp"
+#include "fgl_idmap_device.hpp"
 
 // Scratch of fgl_sample_node_static: device memory that belongs to the library, one copy per GPU, held
 // until the process ends.  In host code this name is only a handle for hipGetSymbolAddress -- it is
@@ -29,6 +31,9 @@ constexpr size_t kStaticScratchBytes = (size_t)16 << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 namespace fgl {
+
+constexpr int kInsertTile = 64;   // seeds per entry of the tile sums that sample_insert_kernel works with ...
+constexpr int kInsertSeeds = 16;  // ... and per workgroup
 
 constexpr int64_t kStaticMaxSeeds = FGL_STATIC_MAX_SEEDS;  // 12.2 bytes of scratch per seed at most: fits 16 MiB
 constexpr int kStaticMaxDevices = 64;
@@ -178,7 +183,7 @@ __global__ __launch_bounds__(TS) void sample_edges_kernel(const int32_t* __restr
                                                           int32_t* __restrict__ src_out, int32_t* __restrict__ dst_out,
                                                           int32_t* __restrict__ block_ptr, int32_t* __restrict__ n_edges_out,
                                                           uint32_t* __restrict__ d_status, int next_fanout, int next_tile_seeds,
-                                                          int32_t* __restrict__ next_tile_sums, uint8_t* __restrict__ zero_per_edge,
+                                                          int32_t* __restrict__ next_tile_sums,
                                                           const TransposeSteps steps, int32_t* __restrict__ readback)
 {
     extern __shared__ uint32_t s_sel[];  // [fanout][TS] picked positions
@@ -191,8 +196,8 @@ __global__ __launch_bounds__(TS) void sample_edges_kernel(const int32_t* __restr
     const int tid = (int)threadIdx.x;
     if (d_stream_add) stream_id += *d_stream_add;  // lets a captured launch sequence advance its random stream
     // work for the transposed blocks that this launch carries along (nothing in the per-hop operator)
-    tjob_zero<TS>(steps.zero);
-    tjob_tile_sums<TS>(steps.before);
+    tjob_tile_sums<TS>(steps.sums);
+    tjob_fill<TS>(steps.fill);
     const int64_t n = actual_count(n_max, d_n);
     const int64_t n_tiles = (n + TS - 1) / TS;
     publish_empty(tile_prefix, n_tiles, block_ptr, n_edges_out, readback, d_status);
@@ -262,7 +267,6 @@ __global__ __launch_bounds__(TS) void sample_edges_kernel(const int32_t* __restr
                 if (x < total) {
                     src_out[(int64_t)base + x] = got[u];
                     if (dst_out) dst_out[(int64_t)base + x] = seed_of[u];
-                    if (zero_per_edge) zero_per_edge[(int64_t)base + x] = 0;
                 }
             }
         }
@@ -287,7 +291,7 @@ __global__ __launch_bounds__(TS) void sample_edges_reg_kernel(const int32_t* __r
                                                               int32_t* __restrict__ src_out, int32_t* __restrict__ dst_out,
                                                               int32_t* __restrict__ block_ptr, int32_t* __restrict__ n_edges_out,
                                                               uint32_t* __restrict__ d_status, int next_fanout, int next_tile_seeds,
-                                                              int32_t* __restrict__ next_tile_sums, uint8_t* __restrict__ zero_per_edge,
+                                                              int32_t* __restrict__ next_tile_sums,
                                                               const TransposeSteps steps, int32_t* __restrict__ readback)
 {
     extern __shared__ int32_t s_stage[];  // [TS*fanout] sampled ids (+ [TS*fanout] seed ids when dst_out is wanted)
@@ -298,8 +302,8 @@ __global__ __launch_bounds__(TS) void sample_edges_reg_kernel(const int32_t* __r
     const int tid = (int)threadIdx.x;
     if (d_stream_add) stream_id += *d_stream_add;  // lets a captured launch sequence advance its random stream
     // work for the transposed blocks that this launch carries along (nothing in the per-hop operator)
-    tjob_zero<TS>(steps.zero);
-    tjob_tile_sums<TS>(steps.before);
+    tjob_tile_sums<TS>(steps.sums);
+    tjob_fill<TS>(steps.fill);
     const int64_t n = actual_count(n_max, d_n);
     const int64_t n_tiles = (n + TS - 1) / TS;
     publish_empty(tile_prefix, n_tiles, block_ptr, n_edges_out, readback, d_status);
@@ -354,27 +358,173 @@ __global__ __launch_bounds__(TS) void sample_edges_reg_kernel(const int32_t* __r
         for (int x = tid; x < total; x += TS) {
             src_out[(int64_t)base + x] = s_val[x];
             if (dst_out) dst_out[(int64_t)base + x] = s_dst[x];
-            if (zero_per_edge) zero_per_edge[(int64_t)base + x] = 0;
         }
         __syncthreads();  // the staging area is reused by the next tile
     }
 }
 
+// The sampling of a mini-batch's hop together with the insert pass of its id-map (idmap_insert_src_kernel): the ids are in LDS
+// already, and a launch and the trip of the ids through memory go away.  Small hops are chains of latencies with most of the chip
+// idle, so the chain is kept short and the work spread out: a workgroup of four waves takes a quarter of a tile, 16 seeds, with
+// sixteen lanes a seed -- a lane per pick (two for fanouts beyond 16), drawn in parallel and told apart from the picks
+// before it through LDS -- and then a lane per edge for the insert: one round for fanouts up to 16.  (64 seeds a workgroup, four
+// lanes a seed: 17.4 and 19.4 us for hops of 6 K and 22 K seeds, against 11.2 and 14.6; a lane per seed and the edges of its
+// wave inserted eight at a time: 35 and 44.)
+template <int F>
+__global__ __launch_bounds__(kBlock) void sample_insert_kernel(const int32_t* __restrict__ indices,
+                                                               const int32_t* __restrict__ seeds, int64_t n_max,
+                                                               const int32_t* __restrict__ d_n, int fanout,
+                                                               const int64_t* __restrict__ row_start,
+                                                               const int32_t* __restrict__ deg_arr,
+                                                               const int32_t* __restrict__ tile_sums,
+                                                               const int32_t* __restrict__ tile_prefix, uint32_t seed_lo,
+                                                               uint32_t seed_hi, uint32_t stream_id,
+                                                               const uint32_t* __restrict__ d_stream_add, int32_t* src_out,
+                                                               int32_t* __restrict__ block_ptr, int32_t* __restrict__ n_edges_out,
+                                                               uint32_t* __restrict__ d_status, int next_fanout, int next_tile_seeds,
+                                                               int32_t* __restrict__ next_tile_sums, const TransposeSteps steps,
+                                                               const InsertWork ins)
+{
+    constexpr int TS = kInsertTile, SUB = kInsertSeeds, kParts = TS / SUB;
+    constexpr int kLanes = kBlock / SUB;                      // lanes per seed
+    constexpr int kShare = F > kLanes ? F / kLanes : 1;       // picks per lane
+    static_assert(TS == kWave, "every wave holds a tile's seeds, one per lane");
+    __shared__ uint32_t s_draw[F * SUB];
+    __shared__ int32_t s_val[F * SUB];
+    __shared__ int s_scan[kBlock / kWave + 1];
+    const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    const int ls = tid % SUB, group = tid / SUB;
+    if (d_stream_add) stream_id += *d_stream_add;  // lets a captured launch sequence advance its random stream
+    tjob_tile_sums<kBlock>(steps.sums);
+    tjob_fill<kBlock>(steps.fill);
+    unsigned long long* slots = reinterpret_cast<unsigned long long*>(ins.t.words);
+    const int64_t e_max = n_max * fanout;
+    const int64_t n = actual_count(n_max, d_n);
+    const int64_t n_tiles = (n + TS - 1) / TS;
+    publish_empty(tile_prefix, n_tiles, block_ptr, n_edges_out, nullptr, d_status);
+    for (int64_t sub = blockIdx.x; sub < n_tiles * kParts; sub += gridDim.x) {
+        const int64_t tile = sub / kParts;
+        const int part = (int)(sub % kParts);
+        const int64_t i = tile * TS + lane;
+        int deg = 0, seed = 0;
+        int64_t row = 0;
+        if (i < n) {
+            deg = deg_arr[i];
+            row = row_start[i];
+            seed = seeds[i];
+        }
+        // (the earlier tiles' sums are fetched while the seed's own three loads are still under way)
+        const int sum_before = tile_prefix ? 0 : lane_sum_before<kBlock>(tile_sums, tile);
+        if (wave == 0 && part == 0) {
+            seed_checks_and_next_hop<TS>(i < n, tile, row, deg, d_status, next_fanout, next_tile_seeds, next_tile_sums);
+        } else if (row < 0) {
+            row = 0;
+            deg = 0;
+        }
+        const int incl = wave_inclusive_scan(deg < fanout ? deg : fanout);
+        const int excl = incl - (deg < fanout ? deg : fanout), total = __shfl(incl, kWave - 1, kWave);
+        const int ex_tile = excl;
+        // this lane's seed of the part
+        const int from = part * SUB + ls;
+        const int first = __shfl(excl, part * SUB, kWave);
+        const int count = __shfl(incl, part * SUB + SUB - 1, kWave) - first;
+        const int ex = __shfl(excl, from, kWave) - first;
+        deg = __shfl(deg, from, kWave);
+        seed = __shfl(seed, from, kWave);
+        row = __shfl(row, from, kWave);
+        const int k = deg < fanout ? deg : fanout;
+        if (deg > fanout) {
+#pragma unroll
+            for (int c = 0; c < kShare; ++c) {
+                const int m = group * kShare + c;
+                if (m < fanout) {
+                    uint32_t o[4];
+                    philox4x32_10((uint32_t)seed, 0u, stream_id, (uint32_t)(m >> 1), seed_lo, seed_hi, o);
+                    const uint64_t r = (m & 1) ? ((uint64_t)o[2] | ((uint64_t)o[3] << 32)) : ((uint64_t)o[0] | ((uint64_t)o[1] << 32));
+                    const uint32_t j = (uint32_t)(deg - fanout + m);
+                    s_draw[m * SUB + ls] = (uint32_t)__umul64hi(r, (uint64_t)j + 1u);
+                }
+            }
+        }
+        // (barriers: the draws are in place behind them)
+        const int base = tile_base<kBlock>(sum_before, tile_prefix, tile, n_tiles, n, total, s_scan, block_ptr, n_edges_out, nullptr, d_status);
+        if (tile_prefix) __syncthreads();
+        if (wave == 1 && part == 0 && i < n) block_ptr[i] = base + ex_tile;
+        // Floyd: for j = deg-k .. deg-1 draw t in [0, j]; take t unless already taken, else j.  (deg <= fanout: the whole row, in
+        // CSR order)
+        int64_t pos[kShare];
+#pragma unroll
+        for (int c = 0; c < kShare; ++c) pos[c] = group * kShare + c;
+        if (deg > fanout) {
+            uint32_t sel[F];
+#pragma unroll
+            for (int m = 0; m < F; ++m) {
+                if (m < fanout && m < group * kShare + kShare) {
+                    const uint32_t t = s_draw[m * SUB + ls];
+                    bool dup = false;
+#pragma unroll
+                    for (int q = 0; q < m; ++q) dup |= (sel[q] == t);
+                    sel[m] = dup ? (uint32_t)(deg - fanout + m) : t;
+                    if (m / kShare == group) pos[m % kShare] = (int64_t)sel[m];
+                } else {
+                    sel[m] = kEmpty;
+                }
+            }
+        }
+        int32_t v[kShare];
+#pragma unroll
+        for (int c = 0; c < kShare; ++c) v[c] = group * kShare + c < k ? indices[row + pos[c]] : 0;
+#pragma unroll
+        for (int c = 0; c < kShare; ++c)
+            if (group * kShare + c < k) s_val[ex + group * kShare + c] = v[c];
+        __syncthreads();
+        const int64_t lo = (int64_t)base + first;
+        for (int c = 0; c < count; c += kBlock) {
+            const int64_t e = lo + c + tid;
+            bool holder = false;
+            if (c + tid < count) {
+                const int32_t id = s_val[c + tid];
+                const uint32_t p = ((uint32_t)id * kHashMul) >> ins.t.shift;
+                const unsigned long long slot = id >= 0 ? slots[p] : 0ull;
+                src_out[e] = id;
+                uint32_t seen = 0, displaced = kEmpty, q = kEmpty;
+                if (id >= 0) q = insert_mention_from(ins.t, (uint32_t)id, kPending | (uint32_t)e, p, slot, &seen, &holder, &displaced);
+                finish_insert(ins, e, e_max, id, q, seen, displaced, d_status);
+            }
+            mark_first(ins.marks, lo + c + wave * kWave, holder);
+        }
+        __syncthreads();  // the part's LDS is reused by the next iteration
+    }
+}
+
 // Seeds per workgroup of the sampling kernels.  Small hops take one wave per tile: a hop of a few ten thousand
 // seeds is a chain of latencies, and 64-seed tiles spread it over four times the compute units.
-#ifndef FGL_SMALL_HOP_SEEDS
-#define FGL_SMALL_HOP_SEEDS 65536
-#endif
-int sample_tile_seeds(int fanout, int64_t n_seeds_max) { return (fanout <= 48 && n_seeds_max > FGL_SMALL_HOP_SEEDS) ? 256 : 64; }
+constexpr int64_t kSmallHopSeeds = 65536;
+int sample_tile_seeds(int fanout, int64_t n_seeds_max) { return (fanout <= 48 && n_seeds_max > kSmallHopSeeds) ? 256 : kInsertTile; }
+
+// Up to this many tiles of seeds the edges kernel derives its tile offsets itself (at most 16 KiB of
+// tile sums per workgroup, read from L2); above it a scan launch prepares them.
+constexpr int64_t kSampleSelfPrefixTiles = 4096;
+
+// Hops whose ids the sampling launch inserts.  Sampling + insert as two launches against one, us (2.4 M nodes unless said): 6 K seeds of
+// a graph of 100 K nodes 15.0 -> 11.2, 22 K of it 17.6 -> 14.6, 27 K seeds of 111 M nodes 22.7 -> 16.5, 130 K of them 91 -> 89 (both
+// bound by random accesses), 145 K seeds 78 -> 69; a million seeds of which nine tenths of the edges lead to known nodes
+// 90 -> 108, and the tile sums need their scan launch (7 us) again.  So the line lies where every workgroup still sums them itself.
+bool sample_can_insert(int fanout, int64_t n_seeds_max)
+{
+    return fanout <= 32 && n_seeds_max <= kSampleSelfPrefixTiles * kInsertTile;
+}
+
+// seeds per tile of a mini-batch's hop
+int sample_hop_tile_seeds(int fanout, int64_t n_seeds_max)
+{
+    return sample_can_insert(fanout, n_seeds_max) ? kInsertTile : sample_tile_seeds(fanout, n_seeds_max);
+}
 
 int64_t sample_tile_count(int64_t n_seeds_max, int fanout)
 {
     return ceil_div(n_seeds_max > 0 ? n_seeds_max : 1, sample_tile_seeds(fanout, n_seeds_max));
 }
-
-// Up to this many tiles of seeds the edges kernel derives its tile offsets itself (at most 16 KiB of
-// tile sums per workgroup, read from L2); above it a scan launch prepares them.
-constexpr int64_t kSampleSelfPrefixTiles = 4096;
 
 size_t sample_workspace_bytes(int64_t n_seeds_max, int fanout)
 {
@@ -392,26 +542,26 @@ static int launch_edges_ts(const int32_t* d_indices, const int32_t* d_seeds, int
                            int fanout, const int64_t* row_start, const int32_t* deg, const int32_t* sums, int32_t* prefix,
                            uint64_t rng_seed, uint32_t stream_id, int32_t* d_src_out, int32_t* d_dst_out,
                            int32_t* d_block_ptr, int32_t* d_n_edges_out, uint32_t* d_status, hipStream_t stream,
-                           const uint32_t* d_stream_add, const NextHop* next, uint8_t* d_zero_per_edge,
-                           const TransposeSteps* steps_in, int32_t* d_readback)
+                           const uint32_t* d_stream_add, const NextHop* next,
+                           const TransposeSteps* steps_in, int32_t* d_readback, const InsertWork* insert)
 {
     const int64_t tiles = ceil_div(n_seeds_max > 0 ? n_seeds_max : 1, TS);
-    unsigned grid = (unsigned)(tiles < 8192 ? tiles : 8192);
+    const int64_t parts = insert != nullptr ? tiles * (kInsertTile / kInsertSeeds) : tiles;
+    unsigned grid = (unsigned)(parts < 8192 ? parts : 8192);
     TransposeSteps steps;
     memset(&steps, 0, sizeof(steps));
     if (steps_in) {
+        // the carried steps get workgroups of their own behind the sampling ones
         steps = *steps_in;
-        // the carried steps get workgroups of their own behind the sampling ones: clearing this hop's counters
-        // (16 per lane), then the tile sums of the hop before
-        if (steps.zero.cnt != nullptr) {
-            steps.zero.side_first = 0;
-            steps.zero.side_blocks = side_blocks_for(steps.zero.cols_max * steps.zero.split + 1, (int64_t)TS * 16);
-            grid += (unsigned)steps.zero.side_blocks;
+        if (steps.sums.cnt != nullptr) {
+            steps.sums.side_first = 0;
+            steps.sums.side_blocks = side_blocks_for(steps.sums.cols_max * steps.sums.split + 1, kTjobTile);
+            grid += (unsigned)steps.sums.side_blocks;
         }
-        if (steps.before.cnt != nullptr) {
-            steps.before.side_first = steps.zero.cnt != nullptr ? steps.zero.side_blocks : 0;
-            steps.before.side_blocks = side_blocks_for(steps.before.cols_max * steps.before.split + 1, kTjobTile);
-            grid += (unsigned)steps.before.side_blocks;
+        if (steps.fill.cnt != nullptr) {
+            steps.fill.side_first = steps.sums.cnt != nullptr ? steps.sums.side_blocks : 0;
+            steps.fill.side_blocks = side_blocks_for(steps.fill.rows_max, (insert ? kBlock : TS) / 16, 16384);
+            grid += (unsigned)steps.fill.side_blocks;
         }
     }
     // few tiles: each workgroup of the edges kernel sums the earlier tile sums itself (the last one
@@ -426,6 +576,20 @@ static int launch_edges_ts(const int32_t* d_indices, const int32_t* d_seeds, int
     const int next_fanout = next ? next->fanout : 0;
     const int next_ts = next ? next->tile_seeds : TS;
     int32_t* next_sums = next ? next->tile_sums : nullptr;
+    if (insert != nullptr) {
+        FGL_REQUIRE(TS == kInsertTile && d_dst_out == nullptr && d_readback == nullptr && fanout <= 32, "sample_edges: this form does not insert");
+#define FGL_LAUNCH_INSERT(F)                                                                                                  \
+    hipLaunchKernelGGL((sample_insert_kernel<F>), dim3(grid), dim3(kBlock), 0, stream, d_indices, d_seeds,                \
+                       n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, prefix, (uint32_t)rng_seed,                   \
+                       (uint32_t)(rng_seed >> 32), stream_id, d_stream_add, d_src_out, d_block_ptr, d_n_edges_out, d_status,  \
+                       next_fanout, next_ts, next_sums, steps, *insert)
+        if (fanout <= 8) FGL_LAUNCH_INSERT(8);
+        else if (fanout <= 16) FGL_LAUNCH_INSERT(16);
+        else FGL_LAUNCH_INSERT(32);
+#undef FGL_LAUNCH_INSERT
+        FGL_CHECK_LAUNCH("sample_insert_kernel");
+        return FGL_OK;
+    }
     // the register variant stages the tile's output (and, if wanted, the seed ids) in LDS: it is used
     // while that fits comfortably in the 64 KiB a workgroup may take
     const size_t lds_reg = (size_t)fanout * TS * sizeof(int32_t) * (d_dst_out ? 2 : 1);
@@ -434,7 +598,7 @@ static int launch_edges_ts(const int32_t* d_indices, const int32_t* d_seeds, int
     hipLaunchKernelGGL((sample_edges_reg_kernel<TS, F>), dim3(grid), dim3(TS), lds_reg, stream, d_indices, d_seeds,   \
                        n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, prefix, (uint32_t)rng_seed,                   \
                        (uint32_t)(rng_seed >> 32), stream_id, d_stream_add, d_src_out, d_dst_out, d_block_ptr, d_n_edges_out, \
-                       d_status, next_fanout, next_ts, next_sums, d_zero_per_edge, steps, d_readback)
+                       d_status, next_fanout, next_ts, next_sums, steps, d_readback)
         if (fanout <= 8) FGL_LAUNCH_REG(8);
         else if (fanout <= 16) FGL_LAUNCH_REG(16);
         else FGL_LAUNCH_REG(32);
@@ -446,7 +610,7 @@ static int launch_edges_ts(const int32_t* d_indices, const int32_t* d_seeds, int
     hipLaunchKernelGGL((sample_edges_kernel<TS, 16>), dim3(grid), dim3(TS), lds, stream, d_indices, d_seeds,
                        n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, prefix, (uint32_t)rng_seed,
                        (uint32_t)(rng_seed >> 32), stream_id, d_stream_add, d_src_out, d_dst_out, d_block_ptr, d_n_edges_out,
-                       d_status, next_fanout, next_ts, next_sums, d_zero_per_edge, steps, d_readback);
+                       d_status, next_fanout, next_ts, next_sums, steps, d_readback);
     FGL_CHECK_LAUNCH("sample_edges_kernel");
     return FGL_OK;
 }
@@ -455,16 +619,16 @@ int launch_sample_edges(const int32_t* d_indices, const int32_t* d_seeds, int64_
                         int fanout, const int64_t* row_start, const int32_t* deg, const int32_t* tile_sums,
                         int32_t* tile_prefix, uint64_t rng_seed, uint32_t stream_id, int32_t* d_src_out,
                         int32_t* d_dst_out, int32_t* d_block_ptr, int32_t* d_n_edges_out, uint32_t* d_status,
-                        hipStream_t stream, const uint32_t* d_stream_add, const NextHop* next, uint8_t* d_zero_per_edge,
-                        const TransposeSteps* steps, int32_t* d_readback)
+                        hipStream_t stream, const uint32_t* d_stream_add, const NextHop* next,
+                        const TransposeSteps* steps, int32_t* d_readback, const InsertWork* insert, int tile_seeds)
 {
-    if (sample_tile_seeds(fanout, n_seeds_max) == 256)
+    if (tile_seeds == 256)
         return launch_edges_ts<256>(d_indices, d_seeds, n_seeds_max, d_n_seeds, fanout, row_start, deg, tile_sums, tile_prefix,
                                     rng_seed, stream_id, d_src_out, d_dst_out, d_block_ptr, d_n_edges_out, d_status, stream,
-                                    d_stream_add, next, d_zero_per_edge, steps, d_readback);
+                                    d_stream_add, next, steps, d_readback, insert);
     return launch_edges_ts<64>(d_indices, d_seeds, n_seeds_max, d_n_seeds, fanout, row_start, deg, tile_sums, tile_prefix,
                                rng_seed, stream_id, d_src_out, d_dst_out, d_block_ptr, d_n_edges_out, d_status, stream,
-                               d_stream_add, next, d_zero_per_edge, steps, d_readback);
+                               d_stream_add, next, steps, d_readback, insert);
 }
 
 int launch_sample(const void* d_indptr, int indptr_is64, const int32_t* d_indices, int64_t n_nodes,
@@ -500,7 +664,7 @@ int launch_sample(const void* d_indptr, int indptr_is64, const int32_t* d_indice
     FGL_CHECK_LAUNCH("sample_degree_kernel");
     return launch_sample_edges(d_indices, d_seeds, n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, prefix, rng_seed,
                                stream_id, d_src_out, d_dst_out, d_block_ptr, d_n_edges_out, d_status, stream, d_stream_add,
-                               nullptr, nullptr, nullptr, d_readback);
+                               nullptr, nullptr, d_readback, nullptr, ts);
 }
 
 }  // namespace fgl

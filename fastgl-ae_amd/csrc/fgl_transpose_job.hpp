@@ -5,14 +5,14 @@
 //
 // A counting sort by source node in five steps, each a grid-stride device function that any kernel of the
 // right stream position can call on entry, before its own work:
-//   zero        the per-column counters                                  (hop h's sampling kernel)
+//   zero        the per-column counters                    (the last launch of hop h-1; the call's first launch for h = 0)
 //   rank        k = counter[col]++ for every edge, as its local source id becomes known
-//                                                                         (hop h's id-map passes: take_rank)
-//   tile sums   per 2048 counters                                        (hop h+1's sampling kernel)
-//   scan        counters -> offsets in place, the transposed row pointer, the longest row
-//                                                                         (hop h+1's first id-map pass)
-//   fill        t_dst[offset[col] + k] = row, t_edge[...] = edge         (hop h+1's second id-map pass)
-// The last hop of a call has no hop after it: its three closing steps are launches of their own.
+//                                                           (hop h's sampling and id-map launches: take_rank)
+//   tile sums   per 2048 counters; the longest row         (hop h+1's sampling launch)
+//   scan        counters -> offsets in place, the transposed row pointer
+//                                                           (hop h+1's last id-map launch)
+//   fill        t_dst[offset[col] + k] = row, t_edge[...] = edge     (hop h+2's sampling launch, or the call's closing launch)
+// The last hop of a call has no hop after it: its closing steps are launches of their own.
 // A carried step runs in workgroups of its own, appended to the carrying launch's grid (side_blocks of them,
 // the last of the grid, see side_block): in front of the launch's own work it would lengthen the chain of
 // memory latencies that a small hop's launch is (measured: 20 us per mini-batch, what the separate launches cost).
@@ -64,6 +64,17 @@ __device__ __forceinline__ void tjob_zero(const TransposeJob& j)
 }
 
 template <int NT>
+__device__ __forceinline__ void zero_job(const ZeroJob& j)
+{
+    if (j.n16 == 0) return;
+    const int64_t sb = (int64_t)gridDim.x - 1 - (int64_t)blockIdx.x - j.side_first;
+    if (sb < 0 || sb >= j.side_blocks) return;
+    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
+    for (int64_t i = sb * NT + threadIdx.x; i < j.n16; i += (int64_t)j.side_blocks * NT) j.p[i] = z;
+}
+
+// ... and the longest row (if it holds more than FGL_SHORT_ROW_ENTRIES entries) into *longest, which starts at zero
+template <int NT>
 __device__ __forceinline__ void tjob_tile_sums(const TransposeJob& j)
 {
     if (j.cnt == nullptr) return;
@@ -79,17 +90,21 @@ __device__ __forceinline__ void tjob_tile_sums(const TransposeJob& j)
             const int64_t i = tile * kTjobTile + (int64_t)q * NT + threadIdx.x;
             v[q] = (i < n - 1) ? j.cnt[i] : 0;  // (the last entry is the slot of the total: not a counter)
         }
-        int s = 0;
+        int s = 0, longest = 0;
 #pragma unroll
-        for (int q = 0; q < kTjobTile / NT; ++q) s += v[q];
+        for (int q = 0; q < kTjobTile / NT; ++q) {
+            s += v[q];
+            int len = v[q];  // (a column's counters sit in neighbouring lanes)
+            for (int d = 1; d < j.split; d <<= 1) len += __shfl_xor(len, d, kWave);
+            longest = len > longest ? len : longest;
+        }
+        if (j.longest != nullptr && longest > FGL_SHORT_ROW_ENTRIES) atomicMax(j.longest, longest);
         const int total = block_sum_of_lanes<NT>(s, smem);
         if (threadIdx.x == 0) j.tile_sums[tile] = total;
     }
 }
 
-// counters -> exclusive prefix sums in place; t_ptr[c] = the prefix of column c's first counter; the longest
-// row (if it holds more than FGL_SHORT_ROW_ENTRIES entries) into *longest, which starts at zero.
-// A lane scans kItems consecutive counters: with split counters those are exactly one column's.
+// counters -> exclusive prefix sums in place; t_ptr[c] = the prefix of column c's first counter
 template <int NT>
 __device__ __forceinline__ void tjob_scan(const TransposeJob& j)
 {
@@ -114,28 +129,16 @@ __device__ __forceinline__ void tjob_scan(const TransposeJob& j)
         const int before = block_sum_before<NT>(j.tile_sums, tile, smem);
         int total;
         int run = block_exclusive_scan<NT>(s, smem, &total) + before;
-        int longest = 0, len = 0;
 #pragma unroll
         for (int q = 0; q < kItems; ++q) {
             const int64_t i = base + q;
             if (i < n) {
                 if (split > 1 || j.cnt != j.t_ptr) j.cnt[i] = run;
-                if (split == 1) {
-                    j.t_ptr[i] = run;
-                    longest = v[q] > longest ? v[q] : longest;
-                } else {
-                    // (split is a power of two that divides kItems: a column's counters never straddle lanes)
-                    if ((i & (split - 1)) == 0) {
-                        j.t_ptr[i / split] = run;
-                        len = 0;
-                    }
-                    len += v[q];
-                    longest = len > longest ? len : longest;
-                }
+                if (split == 1) j.t_ptr[i] = run;
+                else if ((i & (split - 1)) == 0) j.t_ptr[i / split] = run;
             }
             run += v[q];
         }
-        if (j.longest != nullptr && longest > FGL_SHORT_ROW_ENTRIES) atomicMax(j.longest, longest);
     }
 }
 

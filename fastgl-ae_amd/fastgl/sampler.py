@@ -224,7 +224,7 @@ class FusedMapSampler:
         self.deterministic = bool(deterministic)
         if self.deterministic and id_order != "first":
             raise ValueError("deterministic=True needs id_order='first'")
-        # graph_slots = R > 0: the fused path's launch sequence (26 kernels for three hops) is captured once in a
+        # graph_slots = R > 0: the fused path's launch sequence (8 kernels for three hops) is captured once in a
         # HIP graph per output slot and replayed, which takes the host's launch cost out of the small hops.  It
         # pays off where the GPU would otherwise wait for the host -- one mini-batch at a time from an idle GPU:
         # -11 % at batch 8192, -26 % at batch 1024 -- and not in a loop that keeps the GPU busy, where the launches

@@ -74,19 +74,18 @@ enum fgl_zero_policy {
 
 #define FGL_IDMAP_ORDERED 0 /* new ids numbered by first occurrence (deterministic) */
 #define FGL_IDMAP_ARRIVAL 1 /* new ids numbered as their inserts land (the reference's rule,
-                               id_map.cu:314-321): two passes instead of three or four and about a
-                               tenth faster; the order of the new ids depends on scheduling */
+                               id_map.cu:314-321): the order of the new ids depends on scheduling */
 #define FGL_IDMAP_FINAL 2   /* (or'ed in) the table is not consulted after this call: the local ids of the
                                new ids go to the edges and the unique list, not back into the table */
-#define FGL_IDMAP_LEAVE_TABLE_EMPTY 8 /* (or'ed in, with FGL_IDMAP_FINAL only) the call's last pass, which no longer reads
-                               the table, stores the empty marker over all `slots` of it: the next call on the same slots
+#define FGL_IDMAP_LEAVE_TABLE_EMPTY 8 /* (or'ed in, with FGL_IDMAP_FINAL only) the call's last launch
+                               stores the empty marker over all `slots` of the table: the next call on the same slots
                                needs no fgl_idmap_reset (same value and meaning as FGL_BLOCKS_LEAVE_TABLE_EMPTY) */
 /* fgl_sample_blocks only, or'ed into idmap_flags: */
 #define FGL_BLOCKS_TABLE_EMPTY 4       /* the caller vouches that every slot of the table is empty (as fgl_idmap_reset
                                           leaves it, or an earlier fgl_sample_blocks call with FGL_BLOCKS_LEAVE_TABLE_EMPTY
                                           on the same slots): the call's fill launch is skipped */
-#define FGL_BLOCKS_LEAVE_TABLE_EMPTY 8 /* the last pass of the call also empties the table again (it no longer reads
-                                          it), so that the next call may say FGL_BLOCKS_TABLE_EMPTY */
+#define FGL_BLOCKS_LEAVE_TABLE_EMPTY 8 /* the call's closing launch empties the table again, so that the next
+                                          call may say FGL_BLOCKS_TABLE_EMPTY */
 #define FGL_BLOCKS_SORT_TRANSPOSED 16  /* the rows of the transposed blocks that the call builds come out sorted by the
                                           position of their entries in the block (= by destination row), instead of in the
                                           order in which the entries' atomics landed: the same arrays from run to run, and
@@ -206,8 +205,8 @@ int fgl_idmap_map_src(void* d_table, int64_t slots, const int32_t* d_src_in, int
  * d_uniq[0..n_dst); d_src_edges and d_dst_edges (n_edges global ids each, distinct arrays) are relabelled in place;
  * new source ids are numbered from n_dst on and appended to d_uniq; *d_n_total_out = n_dst + their number.
  * A destination id of an edge that is not in d_dst_unique becomes -1 and sets FGL_STATUS_MISSING_KEY.
- * Four launches with first-occurrence numbering (the destination half rides on the first pass over the
- * edges), against the reference's table allocation, fill and four kernels per call.  flags and workspace
+ * Three launches with first-occurrence numbering (destination ids, insert, number; the destination half of the edges
+ * rides on the insert), a fourth beyond a million edges and a fifth beyond eight million, against the reference's table allocation, fill and four kernels per call.  flags and workspace
  * (fgl_idmap_map_src_workspace_bytes(n_edges)) as for fgl_idmap_map_src; a caller that keeps the table between
  * calls passes FGL_IDMAP_FINAL | FGL_IDMAP_LEAVE_TABLE_EMPTY and never fills it again.
  * d_readback (optional): {node total, status word}, written once both are final; may be device-writable pinned host
@@ -231,9 +230,11 @@ int fgl_idmap_lookup(const void* d_table, int64_t slots, int32_t* d_ids, int64_t
  * idmap_flags is FGL_IDMAP_ORDERED or FGL_IDMAP_ARRIVAL (the last hop adds FGL_IDMAP_FINAL by itself), optionally
  * or'ed with FGL_BLOCKS_TABLE_EMPTY, FGL_BLOCKS_LEAVE_TABLE_EMPTY and / or FGL_BLOCKS_SORT_TRANSPOSED.
  * Launches for H hops, first-occurrence numbering: one that starts the batch (counts, seeds into the table, the
- * first hop's row offsets) and four per hop (sample, insert, mark, number) = 4H + 1, plus a table fill unless the
- * caller vouches for an empty table, plus one scan per hop beyond a million seeds or four million edges, plus three
- * if the last hop's transposed block is wanted, plus two with FGL_BLOCKS_SORT_TRANSPOSED.  Each
+ * first hop's row offsets), two per hop of up to 262144 seeds and fanout 32 (sample and insert, number) or three per larger
+ * one (sample, insert, number), and one that closes the batch (the table empty again, the last inner transposed block's rows),
+ * plus a table fill unless the caller vouches for an empty table, plus one per hop beyond a million seeds, a million
+ * edges and eight million edges each, plus two if the last hop's transposed block is wanted, plus two with
+ * FGL_BLOCKS_SORT_TRANSPOSED.  (All limits in the plan's bounds.)  Each
  * hop's passes also prepare the next hop's sampling (row starts, degrees and per-tile edge counts of the nodes
  * they touch), so no hop after the first reads the graph's offsets in a pass of its own.
  * (The reference lists fanouts the other way round and iterates reversed(); the caller
@@ -279,8 +280,8 @@ int fgl_idmap_lookup(const void* d_table, int64_t slots, int32_t* d_ids, int64_t
  * given), t_edge[h] (optional) = the
  * position in src_local[h] of every transposed entry.  Sizes are the call's own device-side counts, so nothing
  * waits for the host.  The work rides on launches the call makes anyway -- a hop's edges take their place in their
- * transposed rows as the id-map numbers them, and the next hop's launches turn the counts into offsets and
- * fill the rows -- except for the last hop, whose transposed block costs three short launches of its own.
+ * transposed rows as the id-map numbers them, and the next two hops' launches (or the closing one) turn the counts into offsets
+ * and fill the rows -- except for the last hop, whose transposed block costs two short launches of its own.
  * fgl_sample_blocks_plan takes the same choice as a bit mask (bit h: hop h), since the workspace depends on it.
  * The table is scratch: after the call it holds the local ids of the nodes of every hop but the
  * last (whose new nodes keep a transient value there) -- or nothing, with FGL_BLOCKS_LEAVE_TABLE_EMPTY;
