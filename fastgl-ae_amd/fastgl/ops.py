@@ -678,10 +678,15 @@ class BlocksPlan:
         self.cap_edges = list(cap_edges)
         self.cap_uniq, self.slots, self.ws_bytes = cap_uniq.value, slots.value, ws_bytes.value
         self.cap_src = self.cap_dst[1:] + [self.cap_uniq]  # source nodes (columns) of each hop's block
+        self.host = L.host().Plan(self.hop_fanouts, None if node_capacity is None else [int(c) for c in node_capacity], self.cap_dst,
+                                  self.cap_edges, self.cap_src, self.cap_uniq, self.transpose_mask)
         self.table = torch.empty(self.slots, dtype=torch.int64, device=self.device)
         self.ws = torch.empty(max(self.ws_bytes, 256), dtype=torch.uint8, device=self.device)
         # the slot count that the last call on this plan's table left empty (None: unknown contents)
         self.empty_slots = None
+
+
+_ID_ORDER = {"first": L.IDMAP_ORDERED, "arrival": L.IDMAP_ARRIVAL}
 
 
 def sample_blocks_fused(plan: BlocksPlan, edge_ptr, indices, seeds, rng_seed: int, stream_base: int,
@@ -723,40 +728,24 @@ def sample_blocks_fused(plan: BlocksPlan, edge_ptr, indices, seeds, rng_seed: in
     if readback is not None and not (readback.dtype == torch.int32 and readback.is_pinned() and readback.is_contiguous()
                                      and readback.numel() >= 3 * H + 2):
         raise RuntimeError("readback must be a contiguous pinned int32 host tensor of at least %d elements" % (3 * H + 2))
-    keep = {(h + H) % H for h in keep_global}
+    keep_mask = 0
+    for h in keep_global:
+        keep_mask |= 1 << ((h + H) % H)
     slots = plan.slots if table_slots is None else min(int(table_slots), plan.slots)
-    lib = L.lib()
+    # every call leaves the table empty for the next one, so only a
+    # plan's first call -- or the first after a failed one, or with another slot count -- pays for a fill
+    flags = _ID_ORDER[id_order] | L.BLOCKS_LEAVE_TABLE_EMPTY
+    if plan.empty_slots == slots:
+        flags |= L.BLOCKS_TABLE_EMPTY
+    if sort_transposed:
+        flags |= L.BLOCKS_SORT_TRANSPOSED
+    plan.empty_slots = None
     with _on_device(dev):
-        uniq = torch.empty(max(plan.cap_uniq, 1), dtype=torch.int32, device=dev)
-        block_ptr = [torch.empty(plan.cap_dst[h] + 1, dtype=torch.int32, device=dev) for h in range(H)]
-        src_local = [torch.empty(max(plan.cap_edges[h], 1), dtype=torch.int32, device=dev) for h in range(H)]
-        src_global = [torch.empty(max(plan.cap_edges[h], 1), dtype=torch.int32, device=dev) if h in keep else None
-                      for h in range(H)]
-        counts = torch.empty(3 * H + 2, dtype=torch.int32, device=dev)
-        arr = lambda ts: (C.c_void_p * H)(*[L.ptr(t) for t in ts])
-        transposed = [None] * H
-        for h in plan.transpose_hops:
-            transposed[h] = (torch.empty(plan.cap_src[h] + 1, dtype=torch.int32, device=dev),
-                             torch.empty(max(plan.cap_edges[h], 1), dtype=torch.int32, device=dev),
-                             torch.empty(max(plan.cap_edges[h], 1), dtype=torch.int32, device=dev))
-        t_arr = lambda k: arr([None if t is None else t[k] for t in transposed]) if plan.transpose_hops else None
-        # every call leaves the table empty for the next one (its last pass no longer reads it), so only a
-        # plan's first call -- or the first after a failed one, or with another slot count -- pays for a fill
-        flags = {"first": L.IDMAP_ORDERED, "arrival": L.IDMAP_ARRIVAL}[id_order] | L.BLOCKS_LEAVE_TABLE_EMPTY
-        if plan.empty_slots == slots:
-            flags |= L.BLOCKS_TABLE_EMPTY
-        if sort_transposed:
-            flags |= L.BLOCKS_SORT_TRANSPOSED
-        plan.empty_slots = None
-        L.check(lib.fgl_sample_blocks(L.ptr(edge_ptr), int(edge_ptr.dtype == torch.int64), L.ptr(indices),
-                                      int(edge_ptr.numel()) - 1, L.ptr(seeds), plan.n_seeds, plan._fan, H, plan._node_cap,
-                                      int(rng_seed) & 0xFFFFFFFFFFFFFFFF, int(stream_base) & 0xFFFFFFFF, L.ptr(stream_offset),
-                                      flags, L.ptr(plan.table), slots, L.ptr(uniq), plan.cap_uniq, arr(block_ptr),
-                                      arr(src_local), arr(src_global), t_arr(0), t_arr(1), t_arr(2), L.ptr(counts),
-                                      None if readback is None else readback.data_ptr(), L.ptr(plan.ws),
-                                      plan.ws.numel(), L.stream_handle() if launch_stream is None else launch_stream.cuda_stream))
-        plan.empty_slots = slots
-    return uniq, block_ptr, src_local, src_global, counts, transposed
+        out = L.host().sample_blocks(plan.host, edge_ptr, indices, seeds, int(rng_seed) & 0xFFFFFFFFFFFFFFFF, int(stream_base) & 0xFFFFFFFF,
+                                     stream_offset, keep_mask, flags, plan.table, slots, plan.ws, readback,
+                                     None if launch_stream is None else launch_stream.cuda_stream)
+    plan.empty_slots = slots
+    return out
 
 
 def rmat_keys(first_edge: int, n_edges: int, scale: int, n_nodes: int, seed: int, device) -> torch.Tensor:

@@ -127,6 +127,7 @@ class _ShapeState:
     def __init__(self):
         self.plans = {}         # node-capacity tuple (None = worst case) -> BlocksPlan
         self.nodes_seen = None  # per hop: the node counts that the buffer sizes are derived from
+        self.sizes = None       # what _sizes worked out, with the node counts it worked from
         self.graphs = None      # (plan, table slots) -> captured launch sequences, see FusedMapSampler._replay
         self.graph_turn = 0     # which of them is next
 
@@ -144,7 +145,7 @@ class _HostCounts:
         self.stream = None
 
     def expect(self, stream):
-        """Before the call is enqueued on ``stream``: every word pending."""
+        """Before the call is enqueued on ``stream`` (its handle): every word pending."""
         self.words.fill_(self.PENDING)
         self.stream = stream
         return self.words
@@ -154,7 +155,7 @@ class _HostCounts:
         when it starts, so this returns while that launch is still running, without the wake-up of a stream wait
         (bounded: after a few milliseconds the stream is waited for instead) -- and returns them as a list."""
         ops.L.check(ops.L.lib().fgl_wait_words(self.words.data_ptr(), int(self.words.numel()), self.PENDING,
-                                               self.stream.cuda_stream, 5000))
+                                               self.stream, 5000))
         values = self.words.tolist()
         self.busy = False
         return values
@@ -253,6 +254,7 @@ class FusedMapSampler:
         self._states = {}       # shape of a mini-batch -> _ShapeState
         self._lanes = []         # streams of iter_batches, one per mini-batch in flight
         self._lane_events = []   # per lane: recorded behind the lane's latest mini-batch
+        self._lane_ready = []    # per lane: recorded on the caller's stream before the lane's latest mini-batch
         self._host_counts = {}   # word count -> pinned words for the per-batch size read-back, handed out in turn (_HostCounts)
         self._host_turn = 0
 
@@ -289,6 +291,17 @@ class FusedMapSampler:
             return None
         return tuple(max(n_seeds, -(-int(1.5 * n) // 4096) * 4096) for n in state.nodes_seen)
 
+    def _sizes(self, state, n_seeds):
+        """(node capacities, table slots) derived from the largest batch seen, or (None, None) before the first one; worked out
+        again only when those sizes change."""
+        seen = state.nodes_seen
+        if seen is None:
+            return None, None
+        if state.sizes is None or state.sizes[0] != seen:
+            slots = ops.L.lib().fgl_idmap_slots
+            state.sizes = (list(seen), self._caps(state, n_seeds), max(slots(2 * seen[-1]), slots(n_seeds)))
+        return state.sizes[1:]
+
     def _state_for(self, seeds, lane=0):
         # Plans, learned buffer sizes and captured graphs are kept per shape: the short last batch of an epoch gets
         # an entry of its own and does not throw away what the full-size batches have learned.  Mini-batches that are
@@ -308,12 +321,11 @@ class FusedMapSampler:
     def _launch_fused(self, seeds, stream_base, worst_case=False, state=None, lane=0, stream=None):
         """stream: enqueue on this stream instead of the current one (eager path only); the outputs are allocated on
         the current stream all the same."""
-        hop_fanouts = list(reversed(self.fanouts))
-        lib = ops.L.lib()
+        hop_fanouts = self.fanouts[::-1]
         n_seeds = int(seeds.numel())
         if state is None:
             state = self._state_for(seeds, lane)
-        caps = None if worst_case else self._caps(state, n_seeds)
+        caps, slots_wanted = (None, None) if worst_case else self._sizes(state, n_seeds)
         plan = state.plans.get(caps)
         if plan is None:
             n_hops = len(hop_fanouts)
@@ -324,14 +336,12 @@ class FusedMapSampler:
                 plan = ops.BlocksPlan(self.nodes_num, n_seeds, hop_fanouts, seeds.device, node_capacity=caps, transpose_hops=hops)
             state.plans = {k: v for k, v in state.plans.items() if k is None}  # keep the worst-case plan only
             state.plans[caps] = plan
-        slots = plan.slots
-        if caps is not None:
-            slots = min(slots, max(lib.fgl_idmap_slots(2 * state.nodes_seen[-1]), lib.fgl_idmap_slots(n_seeds)))
+        slots = plan.slots if slots_wanted is None else min(plan.slots, slots_wanted)
         if self.graph_slots and caps is not None:  # steady state only: the worst-case plan (first batch, redo) runs eagerly
             out, host = self._replay(state, plan, slots, seeds, stream_base)
         else:
             host = self._take_host_counts(3 * len(hop_fanouts) + 2)
-            run_on = stream if stream is not None else torch.cuda.current_stream(seeds.device)
+            run_on = stream.cuda_stream if stream is not None else ops.L.stream_handle_of(seeds.device)
             out = ops.sample_blocks_fused(plan, self.edge_ptr, self.edge_src, seeds, self.rng_seed, stream_base,
                                           keep_global=(len(hop_fanouts) - 1,), table_slots=slots, id_order=self.id_order,
                                           readback=host.expect(run_on), launch_stream=stream, sort_transposed=self.deterministic)
@@ -375,7 +385,7 @@ class FusedMapSampler:
         if plan.empty_slots != slots:
             ops.L.check(ops.L.lib().fgl_idmap_reset(ops.L.ptr(plan.table), slots, ops.L.stream_handle()))
         plan.empty_slots = None
-        slot["host"].expect(torch.cuda.current_stream(seeds.device))
+        slot["host"].expect(ops.L.stream_handle_of(seeds.device))
         slot["graph"].replay()
         plan.empty_slots = slots
         return slot["out"], slot["host"]
@@ -426,21 +436,19 @@ class FusedMapSampler:
         elif any(a > 1.25 * b for a, b in zip(seen, state.nodes_seen)):
             state.nodes_seen = [max(a, b) for a, b in zip(seen, state.nodes_seen)]
         uniq, bptr, src_l, src_g, _, transposed = pending["out"]
+        uniq, hops = ops.L.host().trim(uniq, bptr, src_l, src_g, transposed, c)
         blocks = []
-        for h in range(H):
-            n_dst, n_src, n_e = c[h], c[h + 1], c[H + 1 + h]
-            block_ptr = bptr[h][:n_dst + 1]
-            block_ptr.fgl_longest_row = int(self.fanouts[H - 1 - h])  # no row exceeds the fanout (read by ops.aggregate)
-            block = Block(block_ptr, src_l[h][:n_e], n_src, n_dst, None if src_g[h] is None else src_g[h][:n_e],
-                          sorted_transpose=self.deterministic)
-            if transposed[h] is not None:
+        for i, (block_ptr, src_local, src_global, trans) in enumerate(hops):  # (outermost hop first)
+            h = H - 1 - i
+            block_ptr.fgl_longest_row = int(self.fanouts[i])  # no row exceeds the fanout (read by ops.aggregate)
+            block = Block(block_ptr, src_local, c[h + 1], c[h], src_global, sorted_transpose=self.deterministic)
+            if trans is not None:
                 # built by the same call; its longest row came back with the sizes, so the backward gather knows
                 # on the host whether any row needs the hub-row launch
-                t_ptr = transposed[h][0][:n_src + 1]
-                t_ptr.fgl_longest_row = max(int(c[2 * H + 2 + h]), ops.L.SHORT_ROW_ENTRIES)
-                block._transposed = (t_ptr, transposed[h][1][:n_e], transposed[h][2][:n_e])
-            blocks.insert(0, block)
-        return uniq[:c[H]], pending["seeds"], blocks
+                trans[0].fgl_longest_row = max(c[2 * H + 2 + h], ops.L.SHORT_ROW_ENTRIES)
+                block._transposed = trans
+            blocks.append(block)
+        return uniq, pending["seeds"], blocks
 
     def begin_sample(self, seed_nodes):
         """First half of ``sample_blocks`` (fused path): enqueue every hop and return at once, without the host
@@ -492,7 +500,9 @@ class FusedMapSampler:
             stream_base = (self.batches * 64) & 0xFFFFFFFF
             self.batches += 1
             side = self._lane_stream(dev, lane)
-            side.wait_stream(main)  # the seeds (and anything else the caller produced) are ready
+            ready = self._lane_ready[lane]  # the seeds (and anything else the caller produced) are ready
+            ready.record(main)
+            side.wait_event(ready)
             if self.graph_slots:  # (a graph replays on the current stream)
                 with torch.cuda.stream(side):
                     pending = self._launch_fused(seeds, stream_base, lane=lane)
@@ -524,6 +534,7 @@ class FusedMapSampler:
 
         while len(self._lane_events) < prefetch:
             self._lane_events.append(torch.cuda.Event())
+            self._lane_ready.append(torch.cuda.Event())
         it = iter(seed_batches)
         in_flight = collections.deque()
         n_launched = 0
