@@ -14,14 +14,15 @@
 //     (1.2 M ids of a sampled block over 310 K counters: 66 -> 23 us.)
 //
 // (2) partition, then count (bucket_*): the entries are dealt into buckets of neighbouring columns (2^11 .. 2^13 wide) with one
-//     stable pass -- per tile of entries a histogram over the buckets in LDS, one scan over (bucket, tile), and a pass
-//     that stores every entry at its bucket's place -- and then counted bucket by bucket in LDS, a workgroup per
-//     segment of a bucket.  The transpose goes on from there: a segment learns its place in each of its columns from the
-//     add that delivers its counts (one atomic per segment and column), the counts are scanned into offsets, and every
-//     entry takes its position from its column's counter in LDS and is stored within its bucket's part of the output,
-//     which L2 holds.  Traffic: 4 reads and 2 writes of the entries in all.
-//     (54 M entries of a 2.4 M-node graph, hubs of 85 K: counts 5.9 / 13.2 ms -- unordered / sorted ids -- -> 0.50 / 0.67 ms;
-//     transpose 24.7 -> 1.55 ms, of which the scatter takes 0.48, the fill 0.74, each histogram 0.15.)
+//     pass -- per tile of entries a histogram over the buckets in LDS, one scan over (bucket, tile), and a pass
+//     that puts the tile in order in LDS and stores every bucket's entries at its place -- and then counted bucket by bucket in
+//     LDS, a workgroup per segment of a bucket.  The transpose goes on from there: a segment learns its place in each of its
+//     columns from the add that delivers its counts (one atomic per segment and column), the counts are scanned into offsets,
+//     and the segment's entries are put in order by column in LDS and stored as runs.
+//     Within a bucket a column is 16 bits.  Traffic: 2 reads of the ids, 2 writes and reads of the rows, 1 write and 2 reads of
+//     half the columns.
+//     (54 M entries of a 2.4 M-node graph, hubs of 85 K, us: counts, with an atomic per entry 5900 / 13200 -- unordered / sorted
+//     ids --, with 4-byte stores all over the buckets 499 / 674, now 310 / 270; transpose 24700, 1550, now 700.)
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_tile_rows.hpp"
@@ -82,10 +83,10 @@ __global__ __launch_bounds__(kBlock) void count_ranges_sum_kernel(const int32_t*
 
 // ---- (2) buckets ------------------------------------------------------------------------------------------------
 constexpr int kBucketBlock = 512;
-constexpr int kBucketItems = 16;
-constexpr int kBucketTile = kBucketBlock * kBucketItems;  // entries per tile of the partition
+constexpr int kBucketItems = 16;  // entries per lane
+constexpr int kBucketTile = kBucketBlock * kBucketItems;  // entries that are put in order in LDS together
 constexpr int kMaxBuckets = 2048;
-constexpr int kMaxWidthLog = 13;
+constexpr int kMinWidthLog = 11, kMaxWidthLog = 13;
 constexpr int kSegment = 32768;  // entries per workgroup of the passes over buckets
 
 struct BucketArgs {
@@ -96,10 +97,10 @@ struct BucketArgs {
     int64_t n_rows;
     int64_t n_cols;
     int width_log, buckets;
-    int64_t tiles;
+    int64_t tiles;               // of kBucketTile entries
     int32_t* hist;               // [bucket][tile] counts, then their prefix sums (+ 1 entry: the total)
     int32_t* tile_row;           // [tile] the row that holds the tile's first entry
-    int32_t* b_col;              // entries by bucket: column, row, position in ids
+    uint16_t* b_col;             // entries by bucket: column within the bucket, row, position in ids
     int32_t* b_row;
     int32_t* b_edge;
     int32_t* segments;           // [0] = how many, then per segment {bucket, first entry, entries}
@@ -117,6 +118,16 @@ __device__ __forceinline__ int64_t bucket_entries(const BucketArgs& g)
     return n < g.n_max ? n : g.n_max;
 }
 
+// Workgroup -> tile (the grid is a multiple of eight): every XCD takes a contiguous eighth, in order.  Workgroups go to the
+// XCDs in turn and each XCD has its own L2: neighbouring tiles write next to each other (a histogram's row, a bucket's next
+// entries), and only in one L2 do their pieces become whole lines.
+__device__ __forceinline__ int64_t xcd_tile(int64_t n)
+{
+    const int64_t per = (n + 7) / 8;
+    const int64_t i = (int64_t)(blockIdx.x / 8), at = (int64_t)(blockIdx.x % 8) * per + i;
+    return i < per && at < n ? at : -1;
+}
+
 // counters to zero; the row of every tile's first entry (each row names the tiles that begin inside it)
 __global__ __launch_bounds__(kBlock) void bucket_init_kernel(const BucketArgs g)
 {
@@ -128,54 +139,136 @@ __global__ __launch_bounds__(kBlock) void bucket_init_kernel(const BucketArgs g)
     for (int64_t r = first; r < g.n_rows; r += stride) mark_tile_rows<kBucketTile>(g.indptr, r, g.tiles, g.tile_row);
 }
 
+// the bucket of each of a lane's neighbouring entries (-1: no such entry, or no such column)
+__device__ __forceinline__ void load_columns(const BucketArgs& g, int64_t first, int64_t n, int32_t (&c)[kBucketItems])
+{
+    typedef int32_t I4 __attribute__((ext_vector_type(4), aligned(4)));
+    if (first + kBucketItems <= n) {
+#pragma unroll
+        for (int q = 0; q < kBucketItems / 4; ++q) {
+            const I4 v = *reinterpret_cast<const I4*>(g.ids + first + 4 * q);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) c[4 * q + j] = v[j];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j) c[j] = first + j < n ? g.ids[first + j] : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j)
+        if (c[j] >= g.n_cols) c[j] = -1;
+}
+
+// (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's rows -- would otherwise be 64
+// updates of one counter at a time, one after the other.)
 __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
 {
     __shared__ int s_cnt[kMaxBuckets];
     const int64_t n = bucket_entries(g);
-    const int64_t tile = blockIdx.x, e0 = tile * kBucketTile;
+    const int64_t tile = xcd_tile(g.tiles);
+    if (tile < 0) return;
     for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) s_cnt[b] = 0;
     __syncthreads();
     int32_t c[kBucketItems];
+    load_columns(g, tile * kBucketTile + (int64_t)threadIdx.x * kBucketItems, n, c);
+    int run = 0;
 #pragma unroll
     for (int j = 0; j < kBucketItems; ++j) {
-        const int64_t e = e0 + j * kBucketBlock + threadIdx.x;
-        c[j] = e < n ? g.ids[e] : -1;
+        ++run;
+        const int b = c[j] >> g.width_log;  // (-1 stays -1)
+        if (j + 1 < kBucketItems && c[j + 1] >> g.width_log == b) continue;
+        if (b >= 0) atomicAdd(&s_cnt[b], run);
+        run = 0;
     }
-#pragma unroll
-    for (int j = 0; j < kBucketItems; ++j)
-        if (c[j] >= 0 && c[j] < g.n_cols) atomicAdd(&s_cnt[c[j] >> g.width_log], 1);
     __syncthreads();
     for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) g.hist[(int64_t)b * g.tiles + tile] = s_cnt[b];
 }
 
-// every entry to its bucket's place
+// Every entry to its bucket's place.  A tile is put in order in LDS first, so that a bucket's entries leave as runs (7 of a tile over
+// 1172 buckets), which the neighbouring tiles of the XCD complete to lines: stored one by one they were as many requests
+// to L2 as entries.  (54 M entries, columns and rows: 472 -> 231 us; columns only 227 -> 113.  Tiles of 16384: 254 and 147, a
+// workgroup per CU less; two tiles a workgroup, for half the histogram: 264 and 140.)
 template <bool ROWS, bool EDGES>
 __global__ __launch_bounds__(kBucketBlock) void bucket_scatter_kernel(const BucketArgs g)
 {
-    __shared__ int s_next[kMaxBuckets];
-    __shared__ __align__(16) int s_row[ROWS ? kBucketTile : 4];
-    __shared__ int s_wave[kBucketBlock / kWave];
+    constexpr int NT = kBucketBlock, kPer = kMaxBuckets / NT;
+    __shared__ __align__(16) int s_buf[kBucketTile];
+    __shared__ int s_start[kMaxBuckets];
+    __shared__ int s_delta[kMaxBuckets];  // (and, before it is filled, the scratch of the scans)
     const int64_t n = bucket_entries(g);
-    const int64_t tile = blockIdx.x, e0 = tile * kBucketTile;
-    if (e0 >= n) return;  // (uniform over the workgroup)
-    int32_t c[kBucketItems];
+    const int64_t tile = xcd_tile(g.tiles), e0 = tile * kBucketTile;
+    if (tile < 0 || e0 >= n) return;  // (uniform over the workgroup)
+    const int tid = (int)threadIdx.x, at = tid * kBucketItems;
+    int32_t c[kBucketItems], r[ROWS ? kBucketItems : 1];
+    load_columns(g, e0 + at, n, c);
+    if constexpr (ROWS) {
+        tile_rows<NT, kBucketItems>(g.indptr, g.n_rows, g.tile_row, tile, n, s_buf, s_delta);
+#pragma unroll
+        for (int q = 0; q < kBucketItems / 4; ++q) {
+            const int4 v = reinterpret_cast<const int4*>(s_buf + at)[q];
+            r[4 * q] = v.x; r[4 * q + 1] = v.y; r[4 * q + 2] = v.z; r[4 * q + 3] = v.w;
+        }
+    }
+    for (int b = tid; b < kMaxBuckets; b += NT) s_start[b] = 0;
+    __syncthreads();
+    // places within the tile: a run of equal buckets takes its places with one update
+    int place[kBucketItems], len[kBucketItems];
+#pragma unroll
+    for (int j = kBucketItems - 1; j >= 0; --j)
+        len[j] = j + 1 < kBucketItems && c[j] >> g.width_log == c[(j + 1) % kBucketItems] >> g.width_log ? len[(j + 1) % kBucketItems] + 1 : 1;
 #pragma unroll
     for (int j = 0; j < kBucketItems; ++j) {
-        const int64_t e = e0 + j * kBucketBlock + threadIdx.x;
-        c[j] = e < n ? g.ids[e] : -1;
+        const int b = c[j] >> g.width_log;
+        place[j] = 0;
+        if (j > 0 && b == c[(j + kBucketItems - 1) % kBucketItems] >> g.width_log) place[j] = place[(j + kBucketItems - 1) % kBucketItems] + 1;
+        else if (b >= 0) place[j] = atomicAdd(&s_start[b], len[j]);
     }
-    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) s_next[b] = g.hist[(int64_t)b * g.tiles + tile];
-    if constexpr (ROWS) tile_rows<kBucketBlock, kBucketItems>(g.indptr, g.n_rows, g.tile_row, tile, n, s_row, s_wave);
-    else __syncthreads();
+    __syncthreads();
+    int cnt[kPer], sum = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        cnt[q] = s_start[tid * kPer + q];
+        sum += cnt[q];
+    }
+    int total;
+    int run = block_exclusive_scan<NT>(sum, s_delta, &total);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        s_start[tid * kPer + q] = run;
+        if (tid * kPer + q < g.buckets) s_delta[tid * kPer + q] = g.hist[(int64_t)(tid * kPer + q) * g.tiles + tile] - run;
+        run += cnt[q];
+    }
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < kBucketItems; ++j) {
-        if (c[j] < 0 || c[j] >= g.n_cols) continue;
-        const int at = j * kBucketBlock + (int)threadIdx.x;
-        const int pos = atomicAdd(&s_next[c[j] >> g.width_log], 1);
-        g.b_col[pos] = c[j];
-        if constexpr (ROWS) g.b_row[pos] = s_row[at];
-        if constexpr (EDGES) g.b_edge[pos] = (int32_t)(e0 + at);
+        if (c[j] < 0) continue;
+        place[j] += s_start[c[j] >> g.width_log];
+        s_buf[place[j]] = c[j];
     }
+    __syncthreads();
+    int to[kBucketItems];
+#pragma unroll
+    for (int j = 0; j < kBucketItems; ++j) {
+        const int i = tid + j * NT;
+        to[j] = 0;
+        if (i < total) {
+            const int col = s_buf[i], b = col >> g.width_log;
+            to[j] = i + s_delta[b];
+            g.b_col[to[j]] = (uint16_t)(col - (b << g.width_log));
+        }
+    }
+    auto send = [&](int32_t* out, auto value) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j)
+            if (c[j] >= 0) s_buf[place[j]] = value(j);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j)
+            if (tid + j * NT < total) out[to[j]] = s_buf[tid + j * NT];
+    };
+    if constexpr (ROWS) send(g.b_row, [&](int j) { return r[j]; });
+    if constexpr (EDGES) send(g.b_edge, [&](int j) { return (int)(e0 + at + j); });
 }
 
 // One workgroup: the buckets cut into segments of at most kSegment entries.
@@ -216,16 +309,25 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_count_kernel(const Bucket
     const int col0 = bucket << g.width_log;
     for (int c = (int)threadIdx.x; c < width; c += kBucketBlock) s_cnt[c] = 0;
     __syncthreads();
-    constexpr int kInFlight = 8;
-    int i = (int)threadIdx.x;
-    for (; i + (kInFlight - 1) * kBucketBlock < size; i += kInFlight * kBucketBlock) {
-        int32_t c[kInFlight];
+    // eight neighbours a lane, from whole 16-byte pieces of the array (which is padded to them); equal ones counted together
+    const int64_t g0 = first / 8, g1 = ((int64_t)first + size + 7) / 8;
+    for (int64_t q = g0 + threadIdx.x; q < g1; q += kBucketBlock) {
+        const uint4 v = reinterpret_cast<const uint4*>(g.b_col)[q];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        int c[8], run = 0;
 #pragma unroll
-        for (int j = 0; j < kInFlight; ++j) c[j] = g.b_col[(int64_t)first + i + j * kBucketBlock];
+        for (int j = 0; j < 8; ++j) {
+            const int64_t i = q * 8 + j;
+            c[j] = i >= first && i < (int64_t)first + size ? (int)((w[j / 2] >> (16 * (j % 2))) & 0xFFFFu) : -1;
+        }
 #pragma unroll
-        for (int j = 0; j < kInFlight; ++j) atomicAdd(&s_cnt[c[j] - col0], 1);
+        for (int j = 0; j < 8; ++j) {
+            ++run;
+            if (j + 1 < 8 && c[(j + 1) % 8] == c[j]) continue;
+            if (c[j] >= 0) atomicAdd(&s_cnt[c[j]], run);
+            run = 0;
+        }
     }
-    for (; i < size; i += kBucketBlock) atomicAdd(&s_cnt[g.b_col[(int64_t)first + i] - col0], 1);
     __syncthreads();
     for (int c = (int)threadIdx.x; c < width; c += kBucketBlock) {
         const int v = s_cnt[c];
@@ -235,39 +337,87 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_count_kernel(const Bucket
     }
 }
 
-// ... and, once the counts have become offsets, every entry into its column's row of the transposed block
-template <bool EDGES>
+// ... and, once the counts have become offsets, every entry into its column's row of the transposed block.  A chunk of the segment
+// is put in order by column in LDS and leaves as runs: stored one by one, a segment's entries go all over its bucket's 200 KB of
+// the output, a thousand segments' worth of which no L2 holds.  (54 M entries: 737 -> 207 us.)
+template <int WIDTH_LOG, bool EDGES>
 __global__ __launch_bounds__(kBucketBlock) void bucket_fill_kernel(const BucketArgs g)
 {
-    __shared__ int s_next[1 << kMaxWidthLog];
+    constexpr int kWidth = 1 << WIDTH_LOG, kPer = kWidth / kBucketBlock;
+    __shared__ int s_buf[kBucketTile];
+    __shared__ int s_start[kWidth];
+    __shared__ int s_delta[kWidth];  // (and, before it is filled, the scratch of the scan)
     const int seg = (int)blockIdx.x;
     if (seg >= g.segments[0]) return;
-    const int width = 1 << g.width_log;
     const int bucket = g.segments[1 + 3 * seg], first = g.segments[2 + 3 * seg], size = g.segments[3 + 3 * seg];
-    const int col0 = bucket << g.width_log;
-    for (int c = (int)threadIdx.x; c < width; c += kBucketBlock)  // (columns that the segment does not mention: never used)
-        if (col0 + c < g.n_cols) s_next[c] = g.counts[(int64_t)col0 + c] + g.seg_base[((int64_t)seg << g.width_log) + c];
-    __syncthreads();
-    constexpr int kInFlight = 4;
-    for (int i0 = (int)threadIdx.x; i0 < size; i0 += kInFlight * kBucketBlock) {
-        int32_t c[kInFlight], r[kInFlight], e[kInFlight];
+    const int tid = (int)threadIdx.x;
+    // the segment's next place in each of the lane's columns (columns that it does not mention: never used)
+    int next[kPer];
 #pragma unroll
-        for (int j = 0; j < kInFlight; ++j) {
-            const int i = i0 + j * kBucketBlock;
-            if (i < size) {
-                c[j] = g.b_col[(int64_t)first + i];
-                r[j] = g.b_row[(int64_t)first + i];
-                if constexpr (EDGES) e[j] = g.b_edge[(int64_t)first + i];
-            }
-        }
+    for (int q = 0; q < kPer; ++q) {
+        const int c = tid * kPer + q;
+        const int64_t col = ((int64_t)bucket << g.width_log) + c;
+        next[q] = c < 1 << g.width_log && col < g.n_cols ? g.counts[col] + g.seg_base[((int64_t)seg << g.width_log) + c] : 0;
+    }
+    for (int from = 0; from < size; from += kBucketTile) {
+        const int here = size - from < kBucketTile ? size - from : kBucketTile;
+        const int64_t e0 = (int64_t)first + from;
+        int c[kBucketItems], place[kBucketItems];
 #pragma unroll
-        for (int j = 0; j < kInFlight; ++j) {
-            if (i0 + j * kBucketBlock < size) {
-                const int pos = atomicAdd(&s_next[c[j] - col0], 1);
-                g.t_indices[pos] = r[j];
-                if constexpr (EDGES) g.t_edge[pos] = e[j];
-            }
+        for (int j = 0; j < kBucketItems; ++j) {
+            const int i = tid + j * kBucketBlock;
+            c[j] = i < here ? (int)g.b_col[e0 + i] : -1;
         }
+        for (int q = tid; q < kWidth; q += kBucketBlock) s_start[q] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j) place[j] = c[j] >= 0 ? atomicAdd(&s_start[c[j]], 1) : 0;
+        __syncthreads();
+        int cnt[kPer], sum = 0;
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            cnt[q] = s_start[tid * kPer + q];
+            sum += cnt[q];
+        }
+        int total;
+        int run = block_exclusive_scan<kBucketBlock>(sum, s_delta, &total);
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            s_start[tid * kPer + q] = run;
+            s_delta[tid * kPer + q] = next[q] - run;
+            next[q] += cnt[q];
+            run += cnt[q];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j) {
+            if (c[j] < 0) continue;
+            place[j] += s_start[c[j]];
+            s_buf[place[j]] = c[j];
+        }
+        __syncthreads();
+        int to[kBucketItems];
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j) {
+            const int i = tid + j * kBucketBlock;
+            to[j] = i < here ? i + s_delta[s_buf[i]] : 0;
+        }
+        auto send = [&](int32_t* out, const int32_t* in) {  // (one array after the other: registers)
+            int v[kBucketItems];
+#pragma unroll
+            for (int j = 0; j < kBucketItems; ++j) v[j] = tid + j * kBucketBlock < here ? in[e0 + tid + j * kBucketBlock] : 0;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kBucketItems; ++j)
+                if (tid + j * kBucketBlock < here) s_buf[place[j]] = v[j];
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < kBucketItems; ++j)
+                if (tid + j * kBucketBlock < here) out[to[j]] = s_buf[tid + j * kBucketBlock];
+        };
+        send(g.t_indices, g.b_row);
+        if constexpr (EDGES) send(g.t_edge, g.b_edge);
+        __syncthreads();
     }
 }
 
@@ -284,8 +434,8 @@ static int range_slices(int64_t n_ids, int64_t n_counters)
 // What the forms measured (us, MI355X, replayed from a graph; atomics / ranges / buckets), counting:
 //   75 K ids, 27 K counters, R-MAT          24 /   7 /  -           205 K, 200 K, uniform    11.5 / 14 / 23
 //   144 K, 400 K, uniform                    9 /  15 /  -           251 K, 27 K, R-MAT         60 /  9 / 29
-//   2.5 M, 100 K, R-MAT                    314 /  24 / 45           3.1 M, 2.4 M, R-MAT       433 /  - / 60
-//   54 M, 2.4 M, R-MAT                    5900 /   - / 499          54 M, 2.4 M, sorted     13200 /  - / 674
+//   2.5 M, 100 K, R-MAT                    314 /  24 / 45           3.1 M, 2.4 M, R-MAT       433 /  - / 45
+//   54 M, 2.4 M, R-MAT                    5900 /   - / 310          54 M, 2.4 M, sorted     13200 /  - / 270
 // Ranges read every id once per range and store every counter once per slice: they are kept to half a million counters (32
 // ranges) and four million ids, and small inputs take them where a counter is mentioned twice on average.
 static bool count_by_ranges(int64_t n_ids, int64_t n_counters)
@@ -300,14 +450,14 @@ static bool count_by_buckets(int64_t n_ids, int64_t n_counters)
 }
 // Transposing (atomics with the fill by entries / buckets): 205 K entries, 200 K columns, uniform 26 / 43; 251 K, 27 K, R-MAT 88 / 72;
 // 434 K, a sampled block 93 / 75; 600 K, 200 K, uniform 47 / 50; 1.15 M, a sampled block 113 / 91; 2.5 M, 100 K, R-MAT 335 / 108;
-// 54 M, 2.4 M, R-MAT 24700 (sixteen lanes per row) / 1550.  Columns of graphs are skewed: the line is where those gain, and uniform
+// 54 M, 2.4 M, R-MAT 24700 (sixteen lanes per row) / 700.  Columns of graphs are skewed: the line is where those gain, and uniform
 // ones pay up to twice the time there (300 K entries, 30 K columns 31 / 57, columns drawn as u^4 319 / 67; 600 K, 30 K 47 / 70, 591 / 71;
 // 300 K, 300 K 32 / 47, 207 / 70); from 1.2 M on neither does.
 bool bucket_transpose_form(int64_t n_entries, int64_t n_cols) { return n_entries >= ((int64_t)1 << 18) && fits_buckets(n_entries, n_cols); }
 
 static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edges, void* ws, BucketArgs* g, size_t* bytes)
 {
-    int w = 11;
+    int w = kMinWidthLog;
     while ((n_cols + ((int64_t)1 << w) - 1) >> w > kMaxBuckets) ++w;
     g->width_log = w;
     g->buckets = (int)((n_cols + ((int64_t)1 << w) - 1) >> w);
@@ -316,7 +466,7 @@ static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edg
     Carver c(ws);
     g->hist = c.take<int32_t>((size_t)(g->buckets * g->tiles + 1));
     g->segments = c.take<int32_t>((size_t)(1 + 3 * max_segments));
-    g->b_col = c.take<int32_t>((size_t)n_entries);
+    g->b_col = c.take<uint16_t>(align_up((size_t)n_entries, 8));  // (read in 16-byte pieces)
     if (rows) {
         g->tile_row = c.take<int32_t>((size_t)g->tiles);
         g->b_row = c.take<int32_t>((size_t)n_entries);
@@ -340,16 +490,17 @@ static int launch_partition(const BucketArgs& g, bool rows, bool edges, hipStrea
     if (rows && g.n_rows > init_items) init_items = g.n_rows;
     int64_t blocks = ceil_div(init_items, kBlock);
     if (blocks > 8192) blocks = 8192;
+    const unsigned tiles = (unsigned)align_up(g.tiles, 8);
     hipLaunchKernelGGL(bucket_init_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
-    hipLaunchKernelGGL(bucket_hist_kernel, dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    hipLaunchKernelGGL(bucket_hist_kernel, dim3(tiles), dim3(kBucketBlock), 0, stream, g);
     FGL_CHECK_LAUNCH("bucket_hist_kernel");
     const int64_t n_hist = g.buckets * g.tiles;
-    char* scan_ws = reinterpret_cast<char*>(g.b_edge ? g.b_edge : g.b_col);  // (not written yet: the scan's scratch fits into any of the entry arrays)
-    int rc = launch_exclusive_sum(g.hist, n_hist, nullptr, g.hist, nullptr, scan_ws, scan_workspace_bytes(n_hist), stream);
+    // (the entries are not written yet: the scan's scratch -- a few words per tile -- fits where they go)
+    int rc = launch_exclusive_sum(g.hist, n_hist, nullptr, g.hist, nullptr, g.b_col, scan_workspace_bytes(n_hist), stream);
     if (rc != FGL_OK) return rc;
-    if (rows && edges) hipLaunchKernelGGL((bucket_scatter_kernel<true, true>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
-    else if (rows) hipLaunchKernelGGL((bucket_scatter_kernel<true, false>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
-    else hipLaunchKernelGGL((bucket_scatter_kernel<false, false>), dim3((unsigned)g.tiles), dim3(kBucketBlock), 0, stream, g);
+    if (rows && edges) hipLaunchKernelGGL((bucket_scatter_kernel<true, true>), dim3(tiles), dim3(kBucketBlock), 0, stream, g);
+    else if (rows) hipLaunchKernelGGL((bucket_scatter_kernel<true, false>), dim3(tiles), dim3(kBucketBlock), 0, stream, g);
+    else hipLaunchKernelGGL((bucket_scatter_kernel<false, false>), dim3(tiles), dim3(kBucketBlock), 0, stream, g);
     hipLaunchKernelGGL(bucket_segments_kernel, dim3(1), dim3(1024), 0, stream, g);
     const unsigned segs = (unsigned)(g.buckets + g.n_max / kSegment + 1);
     if (rows) hipLaunchKernelGGL(bucket_count_kernel<true>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
@@ -411,8 +562,13 @@ int launch_bucket_transpose(const int32_t* d_indptr, const int32_t* d_indices, i
     rc = launch_exclusive_sum(d_t_indptr, n_cols, nullptr, d_t_indptr, nullptr, g.hist, scan_workspace_bytes(n_cols), stream);
     if (rc != FGL_OK) return rc;
     const unsigned segs = (unsigned)(g.buckets + n_edges / kSegment + 1);
-    if (edges) hipLaunchKernelGGL(bucket_fill_kernel<true>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
-    else hipLaunchKernelGGL(bucket_fill_kernel<false>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    if (g.width_log == kMinWidthLog) {
+        if (edges) hipLaunchKernelGGL((bucket_fill_kernel<kMinWidthLog, true>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
+        else hipLaunchKernelGGL((bucket_fill_kernel<kMinWidthLog, false>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    } else {
+        if (edges) hipLaunchKernelGGL((bucket_fill_kernel<kMaxWidthLog, true>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
+        else hipLaunchKernelGGL((bucket_fill_kernel<kMaxWidthLog, false>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
+    }
     FGL_CHECK_LAUNCH("bucket_fill_kernel");
     return FGL_OK;
 }
