@@ -104,13 +104,18 @@ struct RpCols<uint16_t, VB> {
     __device__ __forceinline__ Bf16x8 operand(int c) const { return bf16_column(r, c); }
 };
 
-struct RowProductArgs {
+struct RowProductSide {
     const void* a;
     const void* b;
+    int64_t lda, ldb;
+    int k;  // 0: no such pair
+};
+struct RowProductArgs {
+    RowProductSide side[2];  // C = A0 B0 + A1 B1
     const void* bias;
     void* c;
-    int64_t lda, ldb, ldc, m;
-    int n, k;
+    int64_t ldc, m;
+    int n;
     int tiles_n;          // tiles of C along n
     int64_t row_blocks;   // workgroups along m
 };
@@ -178,6 +183,27 @@ struct RpStep {
     }
 };
 
+__device__ __forceinline__ uint32_t rp_bf16_bits(float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v); }
+
+// v += what p holds
+template <typename T, int VB>
+__device__ __forceinline__ void rp_add(const T* p, float (&v)[VB])
+{
+    if constexpr (sizeof(T) == 4) {
+        typedef float Vec __attribute__((ext_vector_type(VB), aligned(4)));
+        const Vec o = *reinterpret_cast<const Vec*>(p);
+#pragma unroll
+        for (int t = 0; t < VB; ++t) v[t] += o[t];
+    } else if constexpr (VB == 1) {
+        v[0] += __uint_as_float((uint32_t)*p << 16);
+    } else {
+        typedef uint32_t Vec __attribute__((ext_vector_type(VB / 2), aligned(4)));
+        const Vec o = *reinterpret_cast<const Vec*>(p);
+#pragma unroll
+        for (int t = 0; t < VB; ++t) v[t] += __uint_as_float(t & 1 ? o[t / 2] & 0xFFFF0000u : o[t / 2] << 16);
+    }
+}
+
 template <typename T, int VB>
 __device__ __forceinline__ void rp_store(T* p, const float (&v)[VB])
 {
@@ -198,10 +224,48 @@ __device__ __forceinline__ void rp_store(T* p, const float (&v)[VB])
     }
 }
 
+// acc += the products of one pair of operands.  row0: the wave's first row; col: the lane's first column.
 template <typename T, int VA, int VB, bool BT>
-__global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kernel(const RowProductArgs g)
+__device__ __forceinline__ void rp_side(const RowProductSide& side, int64_t row0, int64_t m, int col, RpF32x16 (&acc)[VA * VB])
 {
     constexpr int kLane = RpRow<T>::kLane, kStep = 2 * kLane;
+    const int lane = lane_id(), half = lane / 32, k = side.k;
+    const T* pa[VA];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) {
+        const int64_t row = row0 + 32 * i + lane % 32;
+        pa[i] = static_cast<const T*>(side.a) + (row < m ? row : m - 1) * side.lda;
+    }
+    const T* pb = static_cast<const T*>(side.b) + (BT ? (int64_t)col * side.ldb : (int64_t)col);
+    // Steps before the last one are whole.  As in wgrad_kernel nothing branches between the last products and the first reads of
+    // the accumulators, and every branch around a product is one of the whole wave.
+    const int whole = (k - 1) / kStep;
+    RpStep<T, VA, VB, BT> cur, next;
+    int k0 = half * kLane;
+    if (whole > 0) cur.load(pa, pb, side.ldb, k0);
+    else cur.load_tail(pa, pb, side.ldb, k0, 0);  // (zeros)
+    for (int s = 1; s < whole; ++s) {
+        k0 += kStep;
+        next.load(pa, pb, side.ldb, k0);
+        __builtin_amdgcn_sched_barrier(0);  // (left alone, the compiler moves the loads behind the products to save registers)
+        cur.multiply(acc);
+        cur = next;
+    }
+    k0 = whole * kStep + half * kLane;
+    if (k % kStep == 0) next.load(pa, pb, side.ldb, k0);
+    else next.load_tail(pa, pb, side.ldb, k0, k - k0);
+    cur.multiply(acc);
+    next.multiply(acc);
+}
+
+// FORM: one product (kRpOne), two of them and their sum (kRpSum: a layer's own rows with one weight and its gathered rows with another, in one
+// pass over C where the products and their sum were five), or a product added to what C holds (kRpAdd).  In bf16 a product is rounded to
+// bf16 before it is added to another or to C, as it would be if it were stored in between.
+constexpr int kRpOne = 0, kRpSum = 1, kRpAdd = 2;
+
+template <typename T, int VA, int VB, bool BT, int FORM>
+__global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kernel(const RowProductArgs g)
+{
     const int lane = lane_id();
     const int half = lane / 32;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
@@ -212,15 +276,8 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
     const int64_t row0 = (rb * (kBlock / kWave) + wave) * (32 * VA);
     if (rb >= g.row_blocks || row0 >= g.m) return;  // (uniform over the wave)
 
-    const T* pa[VA];
-#pragma unroll
-    for (int i = 0; i < VA; ++i) {
-        const int64_t row = row0 + 32 * i + lane % 32;
-        pa[i] = static_cast<const T*>(g.a) + (row < g.m ? row : g.m - 1) * g.lda;
-    }
     int col = (tn * 32 + lane % 32) * VB;
     if (col + VB > g.n) col = g.n - VB;
-    const T* pb = static_cast<const T*>(g.b) + (BT ? (int64_t)col * g.ldb : (int64_t)col);
     RpF32x16 acc[VA * VB];
 #pragma unroll
     for (int t = 0; t < VA * VB; ++t)
@@ -236,25 +293,26 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
         }
     }
 
-    // Steps before the last one are whole.  As in wgrad_kernel nothing branches between the last products and the first reads of
-    // the accumulators, and every branch around a product is one of the whole wave.
-    const int whole = (g.k - 1) / kStep;
-    RpStep<T, VA, VB, BT> cur, next;
-    int k0 = half * kLane;
-    if (whole > 0) cur.load(pa, pb, g.ldb, k0);
-    else cur.load_tail(pa, pb, g.ldb, k0, 0);  // (zeros)
-    for (int s = 1; s < whole; ++s) {
-        k0 += kStep;
-        next.load(pa, pb, g.ldb, k0);
-        __builtin_amdgcn_sched_barrier(0);  // (left alone, the compiler moves the loads behind the products to save registers)
-        cur.multiply(acc);
-        cur = next;
+    rp_side<T, VA, VB, BT>(g.side[0], row0, g.m, col, acc);
+    constexpr bool kKeep = FORM == kRpSum && sizeof(T) == 2;
+    uint32_t kept[kKeep ? VA * VB : 1][8];  // the first product's values, two to a word
+    if constexpr (FORM == kRpSum) {
+        if constexpr (kKeep) {
+#pragma unroll
+            for (int t = 0; t < VA * VB; ++t)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    uint32_t w = rp_bf16_bits(acc[t][2 * i]) | rp_bf16_bits(acc[t][2 * i + 1]) << 16;
+                    asm volatile("" : "+v"(w));
+                    kept[t][i] = w;
+                }
+#pragma unroll
+            for (int t = 0; t < VA * VB; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+        }
+        rp_side<T, VA, VB, BT>(g.side[1], row0, g.m, col, acc);
     }
-    k0 = whole * kStep + half * kLane;
-    if (g.k % kStep == 0) next.load(pa, pb, g.ldb, k0);
-    else next.load_tail(pa, pb, g.ldb, k0, g.k - k0);
-    cur.multiply(acc);
-    next.multiply(acc);
 
     // Every sum leaves the accumulators here, before the branches around the stores: the empty statement keeps the compiler from moving
     // the additions behind them, which it did.  (fp32 107 K x 256 x 256: 149 us with them behind, 144 here; other sizes alike.)
@@ -265,6 +323,8 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float s = acc[i * VB + t][r] + add[t];
+                if constexpr (FORM != kRpOne && sizeof(T) == 2) s = __uint_as_float(rp_bf16_bits(s) << 16);
+                if constexpr (kKeep) s += __uint_as_float(r & 1 ? kept[i * VB + t][r / 2] & 0xFFFF0000u : kept[i * VB + t][r / 2] << 16);
                 asm volatile("" : "+v"(s));
                 acc[i * VB + t][r] = s;
             }
@@ -278,24 +338,28 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
             float v[VB];
 #pragma unroll
             for (int t = 0; t < VB; ++t) v[t] = acc[i * VB + t][r];
-            if (row < g.m) rp_store<T, VB>(static_cast<T*>(g.c) + row * g.ldc + col, v);
+            if (row < g.m) {
+                T* p = static_cast<T*>(g.c) + row * g.ldc + col;
+                if constexpr (FORM == kRpAdd) rp_add<T, VB>(p, v);
+                rp_store<T, VB>(p, v);
+            }
         }
 }
 
-template <typename T, int VA, int VB, bool BT>
+template <typename T, int VA, int VB, bool BT, int FORM>
 static int launch_row_product(RowProductArgs g, hipStream_t stream)
 {
     g.tiles_n = (int)ceil_div(g.n, 32 * VB);
     g.row_blocks = ceil_div(g.m, (int64_t)(kBlock / kWave) * 32 * VA);
     const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
     FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");
-    hipLaunchKernelGGL((row_product_kernel<T, VA, VB, BT>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
+    hipLaunchKernelGGL((row_product_kernel<T, VA, VB, BT, FORM>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
     FGL_CHECK_LAUNCH("row_product_kernel");
     return FGL_OK;
 }
 
 // Tile: what pads n least, wide tiles where they still make a thousand waves (four per CU).
-template <typename T, bool BT>
+template <typename T, bool BT, int FORM>
 static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStream_t stream)
 {
     const int64_t pad1 = ceil_div(g.n, 32) * 32;
@@ -305,32 +369,67 @@ static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStre
         const int64_t waves = ceil_div(g.m, 32) * (p / (32 * v));
         if (g.n >= v && p * 10 <= pad1 * 12 && waves >= 1024) vb = v;
     }
-    const bool tall = vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048;
-    if (vb == 4) return tall ? launch_row_product<T, 2, 4, BT>(g, stream) : launch_row_product<T, 1, 4, BT>(g, stream);
-    if (vb == 2) return tall ? launch_row_product<T, 2, 2, BT>(g, stream) : launch_row_product<T, 1, 2, BT>(g, stream);
-    return launch_row_product<T, 1, 1, BT>(g, stream);
+    // (a sum keeps the first product's values besides the accumulators: no tall tiles)
+    const bool tall = FORM != kRpSum && vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048;
+    if constexpr (FORM != kRpSum) {
+        if (vb == 4 && tall) return launch_row_product<T, 2, 4, BT, FORM>(g, stream);
+        if (vb == 2 && tall) return launch_row_product<T, 2, 2, BT, FORM>(g, stream);
+    }
+    if (vb == 4) return launch_row_product<T, 1, 4, BT, FORM>(g, stream);
+    if (vb == 2) return launch_row_product<T, 1, 2, BT, FORM>(g, stream);
+    return launch_row_product<T, 1, 1, BT, FORM>(g, stream);
 }
 
 }  // namespace fgl
 
 using namespace fgl;
 
+template <int FORM>
+static int row_product(const RowProductSide& one, const RowProductSide& two, int b_transposed, int64_t m, int n, int dtype, const void* d_bias,
+                       void* d_c, int64_t ldc, void* stream)
+{
+    FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "row_product: unknown dtype %d", dtype);
+    FGL_REQUIRE(m >= 0 && n >= 1 && n <= 65536 && ldc >= n, "row_product: %lld rows of %d columns, %lld apart", (long long)m, n, (long long)ldc);
+    RowProductArgs g;
+    memset(&g, 0, sizeof(g));
+    g.side[0] = one; g.side[1] = two; g.bias = d_bias; g.c = d_c; g.ldc = ldc; g.m = m; g.n = n;
+    bool vectors = true;
+    for (int i = 0; i < (FORM == kRpSum ? 2 : 1); ++i) {
+        const RowProductSide& x = g.side[i];
+        FGL_REQUIRE(x.k >= 1 && x.k <= 65536, "row_product: sizes %lld x %d x %d", (long long)m, x.k, n);
+        FGL_REQUIRE(x.lda >= x.k && x.ldb >= (b_transposed ? x.k : n), "row_product: row stride smaller than the row length");
+        if (m == 0) continue;
+        FGL_REQUIRE(x.a && x.b && d_c, "row_product: null pointer");
+        if (dtype == FGL_F32) continue;
+        // bf16 moves in words: every row that is read along k starts on one, and so does every vector of C (and of an untransposed B)
+        FGL_REQUIRE(x.lda % 2 == 0 && (uintptr_t)x.a % 4 == 0 && (!b_transposed || (x.ldb % 2 == 0 && (uintptr_t)x.b % 4 == 0)),
+                    "row_product: bf16 rows must start on 4-byte boundaries");
+        vectors = vectors && n % 2 == 0 && ldc % 2 == 0 && (uintptr_t)d_c % 4 == 0 && (b_transposed || (x.ldb % 2 == 0 && (uintptr_t)x.b % 4 == 0));
+    }
+    if (m == 0) return FGL_OK;
+    hipStream_t s = as_stream(stream);
+    if (dtype == FGL_F32) return b_transposed ? launch_row_product_any<float, true, FORM>(g, true, s) : launch_row_product_any<float, false, FORM>(g, true, s);
+    return b_transposed ? launch_row_product_any<uint16_t, true, FORM>(g, vectors, s) : launch_row_product_any<uint16_t, false, FORM>(g, vectors, s);
+}
+
 FGL_EXPORT int fgl_row_product(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
                                const void* d_bias, void* d_c, int64_t ldc, void* stream)
 {
-    FGL_REQUIRE(m >= 0 && k >= 1 && n >= 1 && k <= 65536 && n <= 65536, "row_product: sizes %lld x %d x %d", (long long)m, k, n);
-    FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "row_product: unknown dtype %d", dtype);
-    FGL_REQUIRE(lda >= k && ldb >= (b_transposed ? k : n) && ldc >= n, "row_product: row stride smaller than the row length");
-    if (m == 0) return FGL_OK;
-    FGL_REQUIRE(d_a && d_b && d_c, "row_product: null pointer");
-    RowProductArgs g;
-    g.a = d_a; g.b = d_b; g.bias = d_bias; g.c = d_c; g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.m = m; g.n = n; g.k = k;
-    g.tiles_n = 0; g.row_blocks = 0;
-    hipStream_t s = as_stream(stream);
-    if (dtype == FGL_F32) return b_transposed ? launch_row_product_any<float, true>(g, true, s) : launch_row_product_any<float, false>(g, true, s);
-    // bf16 moves in words: every row that is read along k starts on one, and so does every vector of C (and of an untransposed B)
-    FGL_REQUIRE(lda % 2 == 0 && (uintptr_t)d_a % 4 == 0 && (!b_transposed || (ldb % 2 == 0 && (uintptr_t)d_b % 4 == 0)),
-                "row_product: bf16 rows must start on 4-byte boundaries");
-    const bool vectors = n % 2 == 0 && ldc % 2 == 0 && (uintptr_t)d_c % 4 == 0 && (b_transposed || (ldb % 2 == 0 && (uintptr_t)d_b % 4 == 0));
-    return b_transposed ? launch_row_product_any<uint16_t, true>(g, vectors, s) : launch_row_product_any<uint16_t, false>(g, vectors, s);
+    return row_product<kRpOne>(RowProductSide{d_a, d_b, lda, ldb, k}, RowProductSide{nullptr, nullptr, 0, 0, 0}, b_transposed, m, n, dtype, d_bias, d_c,
+                               ldc, stream);
+}
+
+FGL_EXPORT int fgl_row_product_sum(const void* d_a0, int64_t lda0, const void* d_b0, int64_t ldb0, int k0, const void* d_a1, int64_t lda1,
+                                   const void* d_b1, int64_t ldb1, int k1, int b_transposed, int64_t m, int n, int dtype, const void* d_bias,
+                                   void* d_c, int64_t ldc, void* stream)
+{
+    return row_product<kRpSum>(RowProductSide{d_a0, d_b0, lda0, ldb0, k0}, RowProductSide{d_a1, d_b1, lda1, ldb1, k1}, b_transposed, m, n, dtype, d_bias,
+                               d_c, ldc, stream);
+}
+
+FGL_EXPORT int fgl_row_product_add(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
+                                   void* d_c, int64_t ldc, void* stream)
+{
+    return row_product<kRpAdd>(RowProductSide{d_a, d_b, lda, ldb, k}, RowProductSide{nullptr, nullptr, 0, 0, 0}, b_transposed, m, n, dtype, nullptr, d_c,
+                               ldc, stream);
 }

@@ -431,6 +431,73 @@ class MA_Function_Mean(torch.autograd.Function):
         return None, d_feat, None
 
 
+class _SageFunction(torch.autograd.Function):
+    """A ``SAGEConv`` layer as a whole: the two products and their sum are one pass over the output, and in the backward pass the
+    gradient of a node's own row is added to its row of the gathered gradient, where autograd would write it into a cleared array of all
+    source rows and add that.  (GraphSAGE in bf16, 87 K and 41 K rows of 256 columns: 20 of a training step's 57 launches.)
+    ``feat_dst`` is ``None`` where the destination rows are the first rows of ``feat_src``."""
+
+    @staticmethod
+    def run(block, feat_src, feat_dst, w_self, w_neigh, bias, use_global):
+        n_dst = block.num_dst_nodes()
+        h = ops.aggregate(block.edge_ptr, block.src_global if use_global else block.src_local, feat_src, mode="mean", zero_policy="zeros", n_rows=n_dst)
+        x = feat_src[:n_dst] if feat_dst is None else feat_dst
+        out = ops.row_product_sum(x, w_self, h, w_neigh, bias)
+        if out is None:  # (sizes that are the library's)
+            out = ops.row_product(x, w_self, transposed=True) + ops.row_product(h, w_neigh, transposed=True, bias=bias)
+        return out, x, h
+
+    @staticmethod
+    def forward(ctx, block, feat_src, feat_dst, w_self, w_neigh, bias, use_global):
+        out, x, h = _SageFunction.run(block, feat_src, feat_dst, w_self, w_neigh, bias, use_global)
+        ctx.block, ctx.use_global, ctx.own_rows = block, use_global, feat_dst is None
+        ctx.n_src = block.num_src_nodes()
+        ctx.save_for_backward(x, h, w_self, w_neigh)
+        return out
+
+    @staticmethod
+    def backward(ctx, d_out):
+        x, h, w_self, w_neigh = ctx.saved_tensors
+        _, need_src, need_dst, need_self, need_neigh, need_bias, _ = ctx.needs_input_grad
+        d_src = d_dst = d_self = d_neigh = d_bias = None
+        recorded = torch.is_grad_enabled()  # (a graph of the gradients is being built: operators that have gradients themselves)
+        if recorded:
+            d_self = torch.mm(d_out.transpose(0, 1), x) if need_self else None
+            d_neigh = torch.mm(d_out.transpose(0, 1), h) if need_neigh else None
+            d_bias = d_out.sum(0) if need_bias else None
+        else:
+            if need_neigh and need_bias:
+                d_neigh, d_bias = ops.weight_grad(d_out, h, column_sums=True)
+            elif need_neigh:
+                d_neigh = ops.weight_grad(d_out, h)
+            elif need_bias:
+                d_bias = d_out.sum(0)
+            if need_self:
+                d_self = ops.weight_grad(d_out, x)
+        if need_src and not ctx.use_global:
+            t_ptr, t_idx = ctx.block.transposed()
+            d_src = ops.aggregate(t_ptr, t_idx, ops.row_product(d_out, w_neigh).contiguous(), mode="colmean_ptr", zero_policy="zeros",
+                                  col_norm=ctx.block.edge_ptr, n_rows=ctx.n_src)
+            if ctx.own_rows and recorded:
+                n_dst = int(d_out.size(0))
+                d_src = torch.cat([d_src[:n_dst] + torch.mm(d_out, w_self), d_src[n_dst:]])
+            elif ctx.own_rows:
+                ops.row_product_add_(d_src, d_out, w_self)
+        if need_dst:
+            d_dst = ops.row_product(d_out, w_self)
+        return None, d_src, d_dst, d_self, d_neigh, d_bias, None
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _called_plainly(module):
+    """Whether calling ``module`` runs its class's ``forward`` and nothing else."""
+    d = module.__dict__
+    return not any(d[k] for k in _HOOKS) and "forward" not in d and d.get("_compiled_call_impl") is None and not any(
+        getattr(torch.nn.modules.module, "_global" + k) for k in _HOOKS)
+
+
 class SAGEConv(nn.Module):
     """``h_dst W_self + mean(h_src) W_neigh + b`` (the mean aggregator of GraphSAGE)."""
 
@@ -439,7 +506,25 @@ class SAGEConv(nn.Module):
         self.fc_self = _Linear(input_dim, output_dim, bias=False)
         self.fc_neigh = _Linear(input_dim, output_dim, bias=bias)
 
+    def _as_one(self, feat_src, feat_dst, use_global):
+        """Whether the layer may be formed as a whole: both parts are what ``__init__`` made them, called by nobody but this layer, and their
+        inputs the ones that ``_Linear`` takes to the kernels."""
+        if torch.compiler.is_compiling() or torch.jit.is_tracing():
+            return False
+        a, b = self.fc_self, self.fc_neigh
+        if type(a) is not _Linear or type(b) is not _Linear or a.bias is not None or not _called_plainly(a) or not _called_plainly(b):
+            return False
+        own = feat_src if feat_dst is None else feat_dst
+        used = (feat_src, own, a.weight, b.weight) if b.bias is None else (feat_src, own, a.weight, b.weight, b.bias)
+        return (feat_src.is_cuda and feat_src.dim() == 2 and own.dim() == 2 and feat_src.dtype in ops._FEAT and
+                (feat_dst is not None or not use_global) and all(t.dtype == feat_src.dtype and t.device == feat_src.device for t in used) and
+                not any(map(_watched, used)) and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0 and
+                not ops._followed())
+
     def forward(self, block, feat_src, feat_dst=None, use_global=False):
+        if isinstance(block, Block) and self._as_one(feat_src, feat_dst, use_global):
+            args = (block, feat_src, feat_dst, self.fc_self.weight, self.fc_neigh.weight, self.fc_neigh.bias, use_global)
+            return _SageFunction.apply(*args) if torch.is_grad_enabled() else _SageFunction.run(*args)[0]
         h_neigh = MA_Function_Mean.apply(block, feat_src, use_global)
         if feat_dst is None:
             feat_dst = feat_src[:block.num_dst_nodes()]
@@ -462,7 +547,9 @@ class SAGE(nn.Module):
             if i == 0 and input_nodes is not None:
                 if block.src_global is None:
                     raise RuntimeError("the outermost block does not carry graph ids")
-                dst_ids = input_nodes[:block.num_dst_nodes()].long()
+                dst_ids = input_nodes[:block.num_dst_nodes()]
+                if dst_ids.dtype != torch.int32 or features.requires_grad:
+                    dst_ids = dst_ids.long()
                 h = layer(block, features, feat_dst=features.index_select(0, dst_ids), use_global=True)
             else:
                 h = layer(block, h)

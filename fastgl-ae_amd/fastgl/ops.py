@@ -408,6 +408,37 @@ def row_product(a, b, transposed=False, bias=None):
     return out
 
 
+def row_product_sum(a0, b0, a1, b1, bias=None):
+    """``a0 b0^T + (a1 b1^T + bias)`` in one pass over the result, rounded as the two products and their sum would be, for the operands
+    that ``row_product`` takes to the kernel; ``None`` for all others."""
+    m, n = int(a0.size(0)), int(b0.size(0))
+    k0, k1 = int(a0.size(1)), int(a1.size(1))
+    if int(a1.size(0)) != m or int(b1.size(0)) != n or a1.dtype != a0.dtype or a1.device != a0.device or int(b0.size(1)) != k0 or int(b1.size(1)) != k1:
+        return None
+    at0, at1 = _forms_row_product(a0, b0, True, m, k0, n), _forms_row_product(a1, b1, True, m, k1, n)
+    if at0 is None or at1 is None or not (bias is None or (bias.device == a0.device and bias.dtype == a0.dtype and bias.is_contiguous() and
+                                                           bias.numel() == n and not (torch.is_grad_enabled() and bias.requires_grad))):
+        return None
+    dev = a0.device
+    with _on_device(dev):
+        out = torch.empty((m, n), dtype=a0.dtype, device=dev)
+        L.check(L.lib().fgl_row_product_sum(*at0, k0, *at1, k1, 1, m, n, L.F32 if a0.dtype == torch.float32 else L.BF16, L.ptr(bias),
+                                            out.data_ptr(), n, L.stream_handle()))
+    return out
+
+
+def row_product_add_(out, a, b):
+    """``out[:len(a)] += a b``, the product rounded before it is added; ``out`` is contiguous and nobody else's."""
+    m, k, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
+    at = _forms_row_product(a, b, False, m, k, n) if out.dtype == a.dtype and out.device == a.device and out.is_contiguous() else None
+    if at is None:
+        out[:m].add_(row_product(a, b))
+        return out
+    with _on_device(a.device):
+        L.check(L.lib().fgl_row_product_add(*at, 0, m, k, n, L.F32 if a.dtype == torch.float32 else L.BF16, out.data_ptr(), n, L.stream_handle()))
+    return out
+
+
 def weight_grad(a, b, column_sums=False):
     """``a^T b`` for ``a`` [k, m] and ``b`` [k, n]: a dense layer's weight gradient from its input rows and the gradient of
     its output (fp32 sums, result in the operands' dtype).  ``column_sums=True``: ``(a^T b, a.sum(0))``, with ``a`` the

@@ -418,6 +418,16 @@ int fgl_head_scores(const float* d_x, int64_t ldx, int64_t n_rows, int64_t n_er,
 int fgl_row_product(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
                     const void* d_bias, void* d_c, int64_t ldc, void* stream);
 
+/* C = A0 B0 + (A1 B1 + bias): two products as above, of the same rows, columns and b_transposed, and their sum, in one pass over C -- a layer
+ * that adds a node's own row times one weight to its gathered row times another.  bf16: each of the two is rounded before they are added. */
+int fgl_row_product_sum(const void* d_a0, int64_t lda0, const void* d_b0, int64_t ldb0, int k0, const void* d_a1, int64_t lda1,
+                        const void* d_b1, int64_t ldb1, int k1, int b_transposed, int64_t m, int n, int dtype, const void* d_bias,
+                        void* d_c, int64_t ldc, void* stream);
+
+/* C += A B, with the operands of fgl_row_product; bf16: the product is rounded before it is added. */
+int fgl_row_product_add(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int b_transposed, int64_t m, int k, int n, int dtype,
+                        void* d_c, int64_t ldc, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * Weight gradient of a dense layer: C[i, j] = sum over r < k of A[r, i] * B[r, j] -- the d_w = X^T G of backward_gcn /
  * backward_gin (aggregate_acc.cpp:371-374,402-405, torch::mm on a transposed view there).  A: [k, m] with row stride
