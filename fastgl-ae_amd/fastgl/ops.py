@@ -365,6 +365,17 @@ def _splits_k(k, m, n):
     return m * n <= 65536 or k * k >= 256 * m * n
 
 
+def _long_product_is_the_kernels(dtype, transposed, k, n):
+    """Beyond 8e9 multiplications: whether the kernel is ahead of the library for a product of k x n.  A short k leaves little to multiply for each
+    row that moves, and the library moves rows at half the memory's rate, less where a row of the result is no whole number of lines.
+    2.4 M rows, us, library / kernel (transposed): fp32 16 x 64 293 / 151 (191 / 153), 50 x 50 503 / 334 (456 / 356), 64 x 100 627 / 449 (621 / 510),
+    100 x 100 826 / 709 (1933 / 886), but 64 x 64 327 / 345, 100 x 16 345 / 373, 100 x 64 510 / 550, 128 x 64 460 / 559; bf16 64 x 64 202 / 123 (194 / 135),
+    64 x 100 525 / 164 (465 / 182), 100 x 64 360 / 238 (355 / 277), 128 x 128 309 / 264 (but 298 / 359)."""
+    if dtype == torch.bfloat16:
+        return k <= (100 if transposed else 128)
+    return k <= 32 or (k <= 100 and n > 32 and n % 32 != 0)
+
+
 def _forms_row_product(a, b, transposed, m, k, n):
     """Whether ``row_product`` is the kernel's: plain matrices on one GPU of one type, nobody recording a graph of the call or following it,
     no autocast to change the types, and a size where steps over fresh blocks gain.  The library looks for a kernel on every call with sizes
@@ -375,10 +386,10 @@ def _forms_row_product(a, b, transposed, m, k, n):
     transposed 27 / 52; 256 x 384 and 300 x 300 are no worse): a caller of ever the same sizes whom the GPU keeps waiting loses that much.  Steps
     over fresh blocks gain all the same: drawing the line for k > 128 at 2e9 instead made GCN inference of 256 x 256 (60 K rows) 330 -> 349 us, GraphSAGE in
     bf16, 87 K rows of 256 x 256, 996 -> 1294 us a training step and 360 -> 423 in inference, and 3 % better at most (in fp32, 1663 -> 1625).  Products beyond the
-    line keep the GPU busy for longer than the host takes, and there the library is ahead (fp32 2.4 M x 64 x 100, transposed: 534 / 640; a GIN layer of
-    602 x 256 over 8192 rows, forward and backward, 394 / 418 in all).
+    line keep the GPU busy for longer than the host takes, and there it depends on the size (a GIN layer of 602 x 256 over 8192 rows, forward and backward, is the
+    library's: 394 / 418 in all), see ``_long_product_is_the_kernels``.
     Returns the operands' addresses and row strides if so, else None."""
-    if not (m * k * n <= 8 * 10 ** 9 and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
+    if not ((m * k * n <= 8 * 10 ** 9 or _long_product_is_the_kernels(a.dtype, transposed, k, n)) and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
             0 < n <= 65536 and a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
             not torch.is_autocast_enabled() and not _followed()):
         return None
