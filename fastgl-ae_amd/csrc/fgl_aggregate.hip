@@ -392,6 +392,13 @@ __device__ __forceinline__ void gather_row_edge(const AggArgs& g, const LaneSlic
 // here, 250 us with lists beyond 256 entries handed over, less with 128.)  Sampled blocks stay below it
 // for fanouts up to 128.
 constexpr int kLongRowEntries = 128;
+// Where rows are bundled -- a transposed block of at most a few entries a row -- a list is left to the other launch from this many entries on:
+// the bundles are done in the time of some ten accesses, and one list of a hundred entries, four rows in flight, takes thirty.
+// (us, rows of 64 / 128 / 300 fp32 and 256 bf16 columns, lists beyond 128 -> beyond 48 handed over: 87 K rows, 145 K entries, longest 286
+// 63 / 62 / 143 / 65 -> 43 / 42 / 80 / 43; 91 K, 161 K, 304 51 / 47 / 125 / 50 -> 41 / 41 / 84 / 44; 16 K, 23 K, 172 36 / 29 / 67 / 32 ->
+// 27 / 27 / 39 / 30.  64 instead of 48 leaves the last as it was.  Denser blocks keep 128: they have many such lists, and that launch
+// takes a workgroup for each -- 70 K rows of 446 K entries 46 / 61 / 144 / 66 -> 64 / 94 / 196 / 111.)
+constexpr int kBundleLongEntries = 48;
 
 // Rows in order of length, tile by tile (ORDERED below).  The lane groups of a wave walk their lists together, and a wave is done when its
 // longest list is: with rows that differ by an order of magnitude from one to the next -- a whole graph's -- the others wait. Here
@@ -684,9 +691,11 @@ __global__ __launch_bounds__(kBlock) void aggregate_bundle_kernel(const AggArgs 
     int skip = g.skip_rows_longer_than;  // as in aggregate_kernel
     if (g.longest_row != nullptr && *g.longest_row <= skip) skip = 0x7FFFFFFF;
     const int total = off[R] - off[0];
+    bool left_out = false;  // a row of the bundle is long enough to be left to the long-row launch
+#pragma unroll
+    for (int j = 0; j < R; ++j) left_out |= off[j + 1] - off[j] > skip;
 
-    if (total <= kLongRowEntries) {
-        // (no row of the bundle is long enough to be left to the long-row launch)
+    if (total <= kLongRowEntries && !left_out) {
         float acc[VEC];
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
@@ -907,8 +916,11 @@ __global__ __launch_bounds__(kBlock) void aggregate_flat_bundle_kernel(const Agg
     int skip = g.skip_rows_longer_than;  // as in aggregate_kernel
     if (g.longest_row != nullptr && *g.longest_row <= skip) skip = 0x7FFFFFFF;
     const int total = off[R] - off[0];
+    bool left_out = false;
+#pragma unroll
+    for (int j = 0; j < R; ++j) left_out |= off[j + 1] - off[j] > skip;
 
-    if (total <= kLongRowEntries) {
+    if (total <= kLongRowEntries && !left_out) {
         float acc[VEC];
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
@@ -1508,6 +1520,9 @@ constexpr int64_t kOrderMinRows = (int64_t)1 << 17;
 constexpr int kLongRowBlocks = 1021;  // a prime: rows are dealt round robin, and ids that agree in their low bits are
                                        // alike in synthetic (R-MAT) graphs -- a power of two would hand all hubs to a few workgroups
 
+// Lists with more entries than this are the second launch's (segments are sized for the one limit).
+static inline int long_row_limit(bool bundle, const AggArgs& g) { return bundle && g.ws == nullptr ? kBundleLongEntries : kLongRowEntries; }
+
 // The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
 // for large inputs), else a workgroup per row.
 template <typename T, int VEC, int LPR, int MODE>
@@ -1588,9 +1603,11 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
 
 // Flat mapping (aggregate_flat_kernel) for the short rows, the usual second launch for the long ones.
 template <typename T, int VEC>
-static int launch_agg_flat(int mode, bool long_rows_possible, int lanes, bool bundle, hipStream_t stream, AggArgs g)
+static int launch_agg_flat(int mode, int64_t longest_row_max, int lanes, bool bundle, hipStream_t stream, AggArgs g)
 {
-    g.skip_rows_longer_than = long_rows_possible ? kLongRowEntries : 0x7FFFFFFF;
+    const int limit = long_row_limit(bundle, g);
+    const bool long_rows_possible = longest_row_max < 0 || longest_row_max > limit;
+    g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;
     note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible, g.ws != nullptr);
     const int64_t blocks = ceil_div((bundle ? ceil_div(g.n_rows_max, kBundleRows) : g.n_rows_max) * lanes, kBlock);
     if (blocks > 0x7FFFFFFF) {
@@ -1650,9 +1667,13 @@ static int launch_agg_split(int mode, unsigned gy, hipStream_t stream, AggArgs g
 }
 
 template <typename T, int VEC, int LPR>
-static int launch_agg_bundle(int mode, bool long_rows_possible, unsigned gy, hipStream_t stream, AggArgs g)
+static int launch_agg_bundle(int mode, int64_t longest_row_max, unsigned gy, hipStream_t stream, AggArgs g)
 {
-    g.skip_rows_longer_than = long_rows_possible ? kLongRowEntries : 0x7FFFFFFF;
+    // (a longest row of 49 .. 128 entries known on the host: no second launch, whose 8 us are more than that row takes -- 12 K rows, longest
+    // 101, 256 columns 19 us without and 27 with; the wide rows of launch_agg_flat gain all the same, 54 -> 42)
+    const bool long_rows_possible = longest_row_max < 0 || longest_row_max > kLongRowEntries;
+    const int limit = long_row_limit(true, g);
+    g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;
     note_mapping("aggregate_bundle_kernel", LPR, 100, long_rows_possible, g.ws != nullptr);
     const int64_t gx = ceil_div(ceil_div(g.n_rows_max, kBundleRows), kBlock / LPR);
 #define FGL_LAUNCH_BUNDLE(M)                                                                                          \
@@ -1702,8 +1723,7 @@ static int launch_agg_vec(int mode, int64_t longest_row_max, int64_t n_entries_m
     // rows wider than one 64-lane group that fill their groups to less than 90 %: flat mapping
     // (602 fp32 columns: 100 -> 80 us; 602 bf16: 59 -> 44 us forward, 135 -> 84 us on the transposed block)
     if (lanes_needed > 64 && mode != FGL_AGG_EDGE && lanes_needed * 10 < ceil_div(lanes_needed, 64) * 64 * 9)
-        return launch_agg_flat<T, VEC>(mode, longest_row_max < 0 || longest_row_max > kLongRowEntries, lanes_needed,
-                                       short_lists, stream, g);
+        return launch_agg_flat<T, VEC>(mode, longest_row_max, lanes_needed, short_lists, stream, g);
     const int64_t groups = kBlock / lpr;
     const int64_t gx = ceil_div(g.n_rows_max, groups);
     const int64_t gy = ceil_div(lanes_needed, lpr);
@@ -1733,9 +1753,9 @@ static int launch_agg_vec(int mode, int64_t longest_row_max, int64_t n_entries_m
         // (not for rows of eight lanes -- 128 bytes, one cache line: there the bundle's bookkeeping costs what it saves)
         if (short_lists && lpr >= 16) {
             switch (lpr) {
-                case 16: return launch_agg_bundle<T, VEC, 16>(mode, long_rows_possible, grid.y, stream, g);
-                case 32: return launch_agg_bundle<T, VEC, 32>(mode, long_rows_possible, grid.y, stream, g);
-                default: return launch_agg_bundle<T, VEC, 64>(mode, long_rows_possible, grid.y, stream, g);
+                case 16: return launch_agg_bundle<T, VEC, 16>(mode, longest_row_max, grid.y, stream, g);
+                case 32: return launch_agg_bundle<T, VEC, 32>(mode, longest_row_max, grid.y, stream, g);
+                default: return launch_agg_bundle<T, VEC, 64>(mode, longest_row_max, grid.y, stream, g);
             }
         }
     }
