@@ -253,12 +253,18 @@ __global__ __launch_bounds__(kBlock) void transpose_sort_rows_kernel(const SortJ
     tjob_sort_rows<kBlock>(jobs, (int)blockIdx.y);
 }
 
-// ... and the rows of more than 64 entries that it listed, a workgroup per row
+// ... and the rows of more than 64 entries that it listed, a workgroup per piece of a row
 __global__ __launch_bounds__(kSortBlock) void transpose_sort_long_rows_kernel(const SortJobs jobs)
 {
-    __shared__ int s_key[kSortLds];
-    __shared__ int s_val[kSortLds];
+    __shared__ int s_key[kSortPiece];
+    __shared__ int s_val[kSortPiece];
     tjob_sort_long_rows<kSortBlock>(jobs, s_key, s_val);
+}
+
+__global__ __launch_bounds__(kSortBlock) void transpose_merge_long_rows_kernel(const SortJobs jobs)
+{
+    __shared__ int s_key[kSortPiece];
+    tjob_merge_long_rows<kSortBlock>(jobs, s_key);
 }
 
 // ---- R-MAT -------------------------------------------------------------------------
@@ -518,17 +524,18 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
     }
     if (sort_rows && transpose_hops != 0) {
         // rows of the transposed blocks in a fixed order: two more launches per eight blocks -- every row of up to
-        // 64 entries, then the longer ones that the first launch has listed
+        // 64 entries, then the longer ones that the first launch has listed -- and a third one where a row may have several pieces
         SortJobs jobs;
         memset(&jobs, 0, sizeof(jobs));
         jobs.long_rows = ws.sort_long_rows;
         jobs.long_max = p.sort_long_max;
         int n_jobs = 0, round = 0;
-        int64_t most_cols = 1;
+        int64_t most_cols = 1, most_edges = 0;
         for (int h = 0; h <= n_hops; ++h) {
             if (h < n_hops && ((transpose_hops >> h) & 1u)) {
                 jobs.job[n_jobs++] = make_job(h);
                 if (p.cap_src[h] > most_cols) most_cols = p.cap_src[h];
+                if (p.cap_edges[h] > most_edges) most_edges = p.cap_edges[h];
             }
             if (n_jobs == 8 || (h == n_hops && n_jobs > 0)) {
                 jobs.n_long = ws.sort_n_long + round++;
@@ -536,9 +543,12 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
                 hipLaunchKernelGGL(transpose_sort_rows_kernel, dim3((unsigned)gx, (unsigned)n_jobs), dim3(kBlock), 0, s, jobs);
                 const int64_t gl = p.sort_long_max < 2048 ? p.sort_long_max : 2048;
                 hipLaunchKernelGGL(transpose_sort_long_rows_kernel, dim3((unsigned)(gl > 0 ? gl : 1)), dim3(kSortBlock), 0, s, jobs);
+                if (most_edges > kSortPiece)
+                    hipLaunchKernelGGL(transpose_merge_long_rows_kernel, dim3((unsigned)(gl > 0 ? gl : 1)), dim3(kSortBlock), 0, s, jobs);
                 FGL_CHECK_LAUNCH("transpose_sort_rows_kernel");
                 n_jobs = 0;
                 most_cols = 1;
+                most_edges = 0;
                 memset(jobs.job, 0, sizeof(jobs.job));
             }
         }

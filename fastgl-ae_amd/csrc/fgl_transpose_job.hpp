@@ -181,17 +181,21 @@ __device__ __forceinline__ void tjob_fill(const TransposeJob& j)
 //   up to 64            the row's wave, one entry per lane, by shuffles;
 //   longer rows         are listed by that pass and dealt out, one workgroup per row, by a second launch (hubs sit
 //                       next to each other in the numbering: left to the workgroup that finds them they would queue
-//                       up behind each other): up to kSortLds entries in LDS, beyond that kSortLds / 2 entries at a
-//                       time and then odd-even rounds of merging neighbouring pieces (as many rounds as pieces: a
-//                       hub of a whole graph taken as one block).
+//                       up behind each other): up to kSortPiece entries in LDS;
+//   beyond that         (a hub of a large mini-batch, or of a whole graph taken as one block) a workgroup per piece of kSortPiece
+//                       entries: the second launch puts the pieces' keys in order, and a third one finds every key's place, which
+//                       is its place in its piece plus the number of smaller keys in each of the others. (One workgroup per
+//                       row, 4096 entries in LDS and then rounds of merging neighbours, took as many rounds as pieces, one behind the
+//                       other: a row of 6000 / 20 000 / 100 000 entries sampled and put in order in 265 / 1042 / 14 633 us; now
+//                       198 / 395 / 1548.  The five-hop mini-batch below: 66 -> 59 us, of which the third launch 27.)
 // Keys are distinct (positions), or -- without t_edge -- destination rows, whose ties are interchangeable.
-constexpr int kSortLds = 4096;
-constexpr int kSortBlock = 512;  // threads of a workgroup of the second launch
+constexpr int kSortPiece = 2048;
+constexpr int kSortBlock = 512;  // threads of a workgroup of the second and third launch
 constexpr int kSortMax = 0x7FFFFFFF;
 
 struct SortJobs {
     TransposeJob job[8];
-    int32_t* long_rows;   // pairs (job, row) of the rows left to the second launch
+    int32_t* long_rows;   // pairs (job + 8 * piece, row) of the rows left to the second launch
     int32_t* n_long;      // how many (zero when the first launch starts; may exceed long_max: then rows were dropped
     int64_t long_max;     //   from the list -- which its size, one per 65 entries, rules out)
 };
@@ -221,34 +225,21 @@ __device__ __forceinline__ void sort_lanes(int& k, int& v, int first, bool up)
     }
 }
 
-// bitonic sort of n (a power of two, 128 <= n <= kSortLds) pairs in LDS by the whole workgroup; `merge_only`: the two
-// halves are sorted already (ascending), only the last merge is needed.  What bounds it is the chain of steps (78 for 4096
-// pairs), each a pass over LDS and a barrier: the 57 at distances below a wave are done in registers, a wave per 64 neighbours,
-// which leaves 21 barriers of that kind and 7 around the register passes.  The long rows of a five-hop mini-batch (1000 seeds,
-// 2.4 M nodes), with 512 threads a row instead of 256: 98 -> 67 us (1024 threads: 65, and half as many rows at a time).
+// bitonic sort of n (a power of two, 128 <= n <= kSortPiece) pairs in LDS by the whole workgroup.  What bounds it is the chain of
+// steps (66 for 2048 pairs), each a pass over LDS and a barrier: the 51 at distances below a wave are done in registers, a wave per 64
+// neighbours, which leaves 15 barriers of that kind and 6 around the register passes.  The long rows of a five-hop mini-batch (1000 seeds,
+// 2.4 M nodes), with 512 threads a piece instead of 256: 98 -> 67 us (1024 threads: 65, and half as many pieces at a time).
 template <int NT>
-__device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n, bool merge_only)
+__device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n)
 {
-    if (merge_only) {  // (a bitonic merge wants the second half descending)
-        for (int i = threadIdx.x; i < n / 4; i += NT) {
-            const int a = n / 2 + i, b = n - 1 - i;
-            const int k = s_key[a], v = s_val[a];
-            s_key[a] = s_key[b];
-            s_val[a] = s_val[b];
-            s_key[b] = k;
-            s_val[b] = v;
-        }
-        __syncthreads();
-    } else {
-        for (int i = threadIdx.x; i < n; i += NT) {  // (n and NT are multiples of a wave)
-            int k = s_key[i], v = s_val[i];
-            for (int run = 2; run <= kWave; run <<= 1) sort_lanes(k, v, run >> 1, (i & run) == 0);
-            s_key[i] = k;
-            s_val[i] = v;
-        }
-        __syncthreads();
+    for (int i = threadIdx.x; i < n; i += NT) {  // (n and NT are multiples of a wave)
+        int k = s_key[i], v = s_val[i];
+        for (int run = 2; run <= kWave; run <<= 1) sort_lanes(k, v, run >> 1, (i & run) == 0);
+        s_key[i] = k;
+        s_val[i] = v;
     }
-    for (int k = merge_only ? n : 2 * kWave; k <= n; k <<= 1) {
+    __syncthreads();
+    for (int k = 2 * kWave; k <= n; k <<= 1) {
         for (int jj = k >> 1; jj >= kWave; jj >>= 1) {
             for (int t = threadIdx.x; t < n / 2; t += NT) {
                 const int i = 2 * t - (t & (jj - 1));  // the lower index of the t-th pair at distance jj
@@ -275,62 +266,20 @@ __device__ __forceinline__ void sort_lds(int* s_key, int* s_val, int n, bool mer
 }
 
 template <int NT>
-__device__ __forceinline__ void sort_load(int* s_key, int* s_val, int at, const int32_t* key, const int32_t* val, int64_t a,
-                                          int64_t first, int64_t len, int n)
+__device__ __forceinline__ void sort_load(int* s_key, int* s_val, const int32_t* key, const int32_t* val, int64_t a, int len, int n)
 {
     for (int i = threadIdx.x; i < n; i += NT) {
-        const int64_t e = first + i;
-        s_key[at + i] = e < len ? key[a + e] : kSortMax;
-        s_val[at + i] = (val != nullptr && e < len) ? val[a + e] : 0;
+        s_key[i] = i < len ? key[a + i] : kSortMax;
+        s_val[i] = (val != nullptr && i < len) ? val[a + i] : 0;
     }
 }
 
 template <int NT>
-__device__ __forceinline__ void sort_store(const int* s_key, const int* s_val, int at, int32_t* key, int32_t* val, int64_t a,
-                                           int64_t first, int64_t len, int n)
+__device__ __forceinline__ void sort_store(const int* s_key, const int* s_val, int32_t* key, int32_t* val, int64_t a, int len)
 {
-    for (int i = threadIdx.x; i < n; i += NT) {
-        const int64_t e = first + i;
-        if (e < len) {
-            key[a + e] = s_key[at + i];
-            if (val != nullptr) val[a + e] = s_val[at + i];
-        }
-    }
-}
-
-// one row of more than 64 entries, by the whole workgroup
-template <int NT>
-__device__ __forceinline__ void sort_row_block(int* s_key, int* s_val, int32_t* key, int32_t* val, int64_t a, int64_t len)
-{
-    if (len <= kSortLds) {
-        int n = 128;
-        while (n < len) n <<= 1;
-        sort_load<NT>(s_key, s_val, 0, key, val, a, 0, len, n);
-        __syncthreads();
-        sort_lds<NT>(s_key, s_val, n, false);
-        sort_store<NT>(s_key, s_val, 0, key, val, a, 0, len, n);
-        __syncthreads();
-        return;
-    }
-    constexpr int kPiece = kSortLds / 2;
-    const int64_t pieces = (len + kPiece - 1) / kPiece;
-    for (int64_t p = 0; p < pieces; ++p) {
-        sort_load<NT>(s_key, s_val, 0, key, val, a, p * kPiece, len, kPiece);
-        __syncthreads();
-        sort_lds<NT>(s_key, s_val, kPiece, false);
-        sort_store<NT>(s_key, s_val, 0, key, val, a, p * kPiece, len, kPiece);
-        __syncthreads();
-    }
-    // odd-even rounds: neighbouring pieces are merged and split again, smaller half first; the padding of the last
-    // piece sorts to its end, which is never stored
-    for (int64_t round = 0; round < pieces; ++round) {
-        for (int64_t p = round & 1; p + 1 < pieces; p += 2) {
-            sort_load<NT>(s_key, s_val, 0, key, val, a, p * kPiece, len, kSortLds);
-            __syncthreads();
-            sort_lds<NT>(s_key, s_val, kSortLds, true);
-            sort_store<NT>(s_key, s_val, 0, key, val, a, p * kPiece, len, kSortLds);
-            __syncthreads();
-        }
+    for (int i = threadIdx.x; i < len; i += NT) {
+        key[a + i] = s_key[i];
+        if (val != nullptr) val[a + i] = s_val[i];
     }
 }
 
@@ -411,30 +360,116 @@ __device__ __forceinline__ void tjob_sort_rows(const SortJobs& jobs, int job_ind
                 if (val != nullptr) val[ra + lane] = vv;
             }
         }
-        // longer rows: listed for the second launch
+        // longer rows: listed for the second launch, piece by piece
         if (len > kWave) {
-            const int64_t at = atomicAdd(jobs.n_long, 1);
-            if (at < jobs.long_max) {
-                jobs.long_rows[2 * at] = job_index;
-                jobs.long_rows[2 * at + 1] = (int32_t)c;
+            const int pieces = (int)((len + kSortPiece - 1) / kSortPiece);
+            const int64_t at = atomicAdd(jobs.n_long, pieces);
+            for (int p = 0; p < pieces; ++p) {
+                if (at + p >= jobs.long_max) break;
+                jobs.long_rows[2 * (at + p)] = job_index + 8 * p;
+                jobs.long_rows[2 * (at + p) + 1] = (int32_t)c;
             }
         }
     }
 }
 
+// the piece that entry q of the list names: its first entry and its length, and those of its row
+struct SortPiece {
+    int64_t row_a, row_len, a;
+    int len;
+};
+__device__ __forceinline__ SortPiece sort_piece(const SortJobs& jobs, const TransposeJob& j, int64_t q)
+{
+    const int64_t c = jobs.long_rows[2 * q + 1];
+    const int64_t n_edges = actual_count(j.edges_max, j.d_n_edges);
+    int64_t a = j.t_ptr[c], b = j.t_ptr[c + 1];
+    if (b > n_edges) b = n_edges;
+    if (a > b) a = b;
+    SortPiece p;
+    p.row_a = a;
+    p.row_len = b - a;
+    const int64_t from = (int64_t)(jobs.long_rows[2 * q] >> 3) * kSortPiece;
+    p.a = a + from;
+    const int64_t left = b - p.a;
+    p.len = left <= 0 ? 0 : left < kSortPiece ? (int)left : kSortPiece;
+    return p;
+}
+
+// second launch: rows of one piece in place; the keys of the others' pieces, in order, to where the ranks were
 template <int NT>
 __device__ __forceinline__ void tjob_sort_long_rows(const SortJobs& jobs, int* s_key, int* s_val)
 {
-    int64_t n = *jobs.n_long;
-    if (n > jobs.long_max) n = jobs.long_max;
-    for (int64_t q = blockIdx.x; q < n; q += gridDim.x) {
+    int64_t total = *jobs.n_long;
+    if (total > jobs.long_max) total = jobs.long_max;
+    for (int64_t q = blockIdx.x; q < total; q += gridDim.x) {
         const TransposeJob& j = jobs.job[jobs.long_rows[2 * q] & 7];
-        const int64_t c = jobs.long_rows[2 * q + 1];
-        const int64_t n_edges = actual_count(j.edges_max, j.d_n_edges);
-        int64_t a = j.t_ptr[c], b = j.t_ptr[c + 1];
-        if (b > n_edges) b = n_edges;
-        if (a > b) a = b;
-        sort_row_block<NT>(s_key, s_val, j.t_edge ? j.t_edge : j.t_dst, j.t_edge ? j.t_dst : nullptr, a, b - a);
+        const SortPiece p = sort_piece(jobs, j, q);
+        const bool alone = p.row_len <= kSortPiece;
+        int32_t* key = j.t_edge ? j.t_edge : j.t_dst;
+        int32_t* val = alone && j.t_edge ? j.t_dst : nullptr;
+        int n = 128;
+        while (n < p.len) n <<= 1;
+        sort_load<NT>(s_key, s_val, key, val, p.a, p.len, n);
+        __syncthreads();
+        sort_lds<NT>(s_key, s_val, n);
+        sort_store<NT>(s_key, s_val, alone ? key : j.rank, val, p.a, p.len);
+        __syncthreads();
+    }
+}
+
+// third launch: the keys of rows of several pieces to their places; an entry's destination row is the block's row that holds its
+// position, looked up again (the pieces moved without it)
+template <int NT>
+__device__ __forceinline__ void tjob_merge_long_rows(const SortJobs& jobs, int* s_key)
+{
+    constexpr int kItems = kSortPiece / NT;
+    int64_t total = *jobs.n_long;
+    if (total > jobs.long_max) total = jobs.long_max;
+    for (int64_t q = blockIdx.x; q < total; q += gridDim.x) {
+        const TransposeJob& j = jobs.job[jobs.long_rows[2 * q] & 7];
+        const SortPiece p = sort_piece(jobs, j, q);
+        if (p.row_len <= kSortPiece) continue;  // (uniform over the workgroup)
+        int key[kItems];
+        int64_t at[kItems];
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            const int i = (int)threadIdx.x + u * NT;
+            key[u] = i < p.len ? j.rank[p.a + i] : kSortMax;
+            at[u] = p.row_a + i;
+        }
+        for (int64_t o = p.row_a; o < p.row_a + p.row_len; o += kSortPiece) {
+            if (o == p.a) continue;
+            const int64_t left = p.row_a + p.row_len - o;
+            const int len = left < kSortPiece ? (int)left : kSortPiece;
+            for (int i = threadIdx.x; i < len; i += NT) s_key[i] = j.rank[o + i];
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kItems; ++u) {
+                int lo = 0, hi = len;  // (equal keys -- only without positions -- stay in the order of their pieces)
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (o < p.a ? s_key[mid] <= key[u] : s_key[mid] < key[u]) lo = mid + 1; else hi = mid;
+                }
+                at[u] += lo;
+            }
+            __syncthreads();
+        }
+        const int64_t n_rows = actual_count(j.rows_max, j.d_n_rows);
+#pragma unroll
+        for (int u = 0; u < kItems; ++u) {
+            if ((int)threadIdx.x + u * NT >= p.len) continue;
+            if (j.t_edge == nullptr) {
+                j.t_dst[at[u]] = key[u];
+                continue;
+            }
+            j.t_edge[at[u]] = key[u];
+            int64_t lo = 0, hi = n_rows;  // block_ptr[lo] <= key < block_ptr[hi]
+            while (hi - lo > 1) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (j.block_ptr[mid] <= key[u]) lo = mid; else hi = mid;
+            }
+            j.t_dst[at[u]] = (int32_t)lo;
+        }
     }
 }
 
