@@ -96,7 +96,7 @@ struct BlocksPlan {
     uint32_t transpose_hops;
     int64_t cap_src[32];  // max source nodes (= columns) of hop h
     int split[32];        // counters per column while hop h's transposed rows are being counted
-    int64_t sort_long_max;  // rows of more than 64 entries that the transposed blocks can hold between them
+    int64_t sort_long_max;  // pieces of rows of more than 64 entries that the transposed blocks can hold between them (one per 65)
 };
 
 struct BlocksScratch {
@@ -110,7 +110,7 @@ struct BlocksScratch {
     int32_t* t_rank[32];
     int32_t* t_tile_sums[32];
     int32_t* t_split_cnt[32];  // split counters (hops that count with several counters per column)
-    int32_t* sort_long_rows;   // rows left to the second launch of the row sort: pairs (job, row)
+    int32_t* sort_long_rows;   // rows left to the second launch of the row sort: pairs (job + 8 * piece, row)
     int32_t* sort_n_long;      // their number, one counter per group of eight transposed blocks (zeroed by the first launch of a call)
 };
 
@@ -524,7 +524,8 @@ FGL_EXPORT int fgl_sample_blocks(const void* d_indptr, int indptr_is64, const in
     }
     if (sort_rows && transpose_hops != 0) {
         // rows of the transposed blocks in a fixed order: two more launches per eight blocks -- every row of up to
-        // 64 entries, then the longer ones that the first launch has listed -- and a third one where a row may have several pieces
+        // 64 entries, then the longer ones that the first launch has listed -- and a third one where
+        // an edge count allows a row of several pieces
         SortJobs jobs;
         memset(&jobs, 0, sizeof(jobs));
         jobs.long_rows = ws.sort_long_rows;

@@ -89,7 +89,7 @@ enum fgl_zero_policy {
 #define FGL_BLOCKS_SORT_TRANSPOSED 16  /* the rows of the transposed blocks that the call builds come out sorted by the
                                           position of their entries in the block (= by destination row), instead of in the
                                           order in which the entries' atomics landed: the same arrays from run to run, and
-                                          with them the same fp32 sums in every gather over them; one more launch per call */
+                                          with them the same fp32 sums in every gather over them; two or three more launches per call */
 #define FGL_MAX_FANOUT 192
 
 int fgl_abi_version(void);
