@@ -277,6 +277,7 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
     if (rb >= g.row_blocks || row0 >= g.m) return;  // (uniform over the wave)
 
     int col = (tn * 32 + lane % 32) * VB;
+    const bool past_end = FORM == kRpAdd && col >= g.n;  // (adds nothing: the columns that it repeats are another lane's)
     if (col + VB > g.n) col = g.n - VB;
     RpF32x16 acc[VA * VB];
 #pragma unroll
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kern
             float v[VB];
 #pragma unroll
             for (int t = 0; t < VB; ++t) v[t] = acc[i * VB + t][r];
-            if (row < g.m) {
+            if (row < g.m && !past_end) {
                 T* p = static_cast<T*>(g.c) + row * g.ldc + col;
                 if constexpr (FORM == kRpAdd) rp_add<T, VB>(p, v);
                 rp_store<T, VB>(p, v);
@@ -358,7 +359,9 @@ static int launch_row_product(RowProductArgs g, hipStream_t stream)
     return FGL_OK;
 }
 
-// Tile: what pads n least, wide tiles where they still make a thousand waves (four per CU).
+// Tile: what pads n least, wide tiles where they still make a thousand waves (four per CU).  The last vector of a row is moved back to end with
+// it and repeats columns of its neighbour, which for 129 columns in twos, or 514 in fours, is another workgroup's: harmless where both store
+// the same values, but a sum would be added twice, so sums go to C in vectors only if a row is a whole number of them.
 template <typename T, bool BT, int FORM>
 static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStream_t stream)
 {
@@ -367,7 +370,7 @@ static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStre
     for (int v = 2; v <= 4 && vectors; v *= 2) {
         const int64_t p = ceil_div(g.n, 32 * v) * 32 * v;
         const int64_t waves = ceil_div(g.m, 32) * (p / (32 * v));
-        if (g.n >= v && p * 10 <= pad1 * 12 && waves >= 1024) vb = v;
+        if (g.n >= v && p * 10 <= pad1 * 12 && waves >= 1024 && (FORM != kRpAdd || g.n % v == 0)) vb = v;
     }
     // (a sum keeps the first product's values besides the accumulators: no tall tiles)
     const bool tall = FORM != kRpSum && vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048;

@@ -37,6 +37,20 @@ def test_two_products_in_one_pass(cuda, dtype, rel, m, k0, k1, n):
         assert float((got.cpu().double() - want).norm() / want.norm()) < rel
 
 
+# wide vectors need a thousand waves; rows that are no whole number of them, whose last vector lies across two tiles (129, 514) or two lanes
+@pytest.mark.parametrize("dtype,rel", [(torch.float32, 1e-6), (torch.bfloat16, 6e-3)])
+@pytest.mark.parametrize("m,k,n", [(12_000, 8, 129), (9_000, 8, 514), (9_000, 16, 130), (12_000, 8, 98), (12_000, 8, 256)])
+def test_sums_are_added_once(cuda, dtype, rel, m, k, n):
+    print("add", dtype, m, k, n, flush=True)
+    gen = torch.Generator().manual_seed(n)
+    a, b, base = (torch.randn(s, generator=gen).to(dtype) for s in ((m, k), (k, n), (m + 1, n)))
+    with torch.no_grad():
+        got = ops.row_product_add_(base.to(cuda), a.to(cuda), b.to(cuda)).cpu().double()
+    want = base.double()
+    want[:m] += a.double() @ b.double()
+    assert float(((got - want).norm(dim=0) / want.norm(dim=0)).max()) < rel  # (column by column: a sum of one column added twice is seen)
+
+
 def _setup(cuda, dtype, dim, hidden, classes):
     edge_ptr, edge_src = fastgl.graph.rmat_csr(20_000, 200_000, seed=3, device=cuda)
     sampler = fastgl.FusedMapSampler([10, 8], rng_seed=1, deterministic=True).set_graph(edge_ptr, edge_src)
