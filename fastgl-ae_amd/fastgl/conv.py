@@ -506,23 +506,27 @@ class SAGEConv(nn.Module):
         self.fc_self = _Linear(input_dim, output_dim, bias=False)
         self.fc_neigh = _Linear(input_dim, output_dim, bias=bias)
 
-    def _as_one(self, feat_src, feat_dst, use_global):
-        """Whether the layer may be formed as a whole: both parts are what ``__init__`` made them, called by nobody but this layer, and their
-        inputs the ones that ``_Linear`` takes to the kernels."""
+    def _as_one(self, block, feat_src, feat_dst, use_global):
+        """Whether the layer may be formed as a whole: both parts are what ``__init__`` made them, called by nobody but this layer, their
+        inputs the ones that ``_Linear`` takes to the kernels, and there is one own row for each destination (a single one that stands for
+        all of them is repeated by the operators' sum) and, if they are taken from the source rows, a row of their gradient for each."""
         if torch.compiler.is_compiling() or torch.jit.is_tracing():
             return False
         a, b = self.fc_self, self.fc_neigh
         if type(a) is not _Linear or type(b) is not _Linear or a.bias is not None or not _called_plainly(a) or not _called_plainly(b):
             return False
         own = feat_src if feat_dst is None else feat_dst
+        n_dst = block.num_dst_nodes()
+        if own.dim() != 2 or (n_dst > min(own.size(0), block.num_src_nodes()) if feat_dst is None else own.size(0) != n_dst):
+            return False
         used = (feat_src, own, a.weight, b.weight) if b.bias is None else (feat_src, own, a.weight, b.weight, b.bias)
-        return (feat_src.is_cuda and feat_src.dim() == 2 and own.dim() == 2 and feat_src.dtype in ops._FEAT and
+        return (feat_src.is_cuda and feat_src.dim() == 2 and feat_src.dtype in ops._FEAT and
                 (feat_dst is not None or not use_global) and all(t.dtype == feat_src.dtype and t.device == feat_src.device for t in used) and
                 not any(map(_watched, used)) and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0 and
                 not ops._followed())
 
     def forward(self, block, feat_src, feat_dst=None, use_global=False):
-        if isinstance(block, Block) and self._as_one(feat_src, feat_dst, use_global):
+        if isinstance(block, Block) and self._as_one(block, feat_src, feat_dst, use_global):
             args = (block, feat_src, feat_dst, self.fc_self.weight, self.fc_neigh.weight, self.fc_neigh.bias, use_global)
             return _SageFunction.apply(*args) if torch.is_grad_enabled() else _SageFunction.run(*args)[0]
         h_neigh = MA_Function_Mean.apply(block, feat_src, use_global)

@@ -441,7 +441,8 @@ def row_product_sum(a0, b0, a1, b1, bias=None):
 def row_product_add_(out, a, b):
     """``out[:len(a)] += a b``, the product rounded before it is added; ``out`` is contiguous and nobody else's."""
     m, k, n = int(a.size(0)), int(a.size(1)), int(b.size(1))
-    at = _forms_row_product(a, b, False, m, k, n) if out.dtype == a.dtype and out.device == a.device and out.is_contiguous() else None
+    fits = out.dim() == 2 and out.size(0) >= m and out.size(1) == n and int(b.size(0)) == k
+    at = _forms_row_product(a, b, False, m, k, n) if fits and out.dtype == a.dtype and out.device == a.device and out.is_contiguous() else None
     if at is None:
         out[:m].add_(row_product(a, b))
         return out

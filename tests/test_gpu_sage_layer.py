@@ -119,6 +119,34 @@ def test_what_calls_the_parts_still_does(cuda):
     assert torch.allclose(model(blocks, x), whole, rtol=1e-4, atol=1e-5)
 
 
+def test_layers_whose_own_rows_are_not_one_for_each_destination(cuda):
+    """One row that stands for all destinations is repeated, and its gradient summed; other numbers of rows are refused."""
+    model, nodes, blocks, feat = _setup(cuda, torch.float32, 32, 16, 8)
+    layer, block, x = model.layers[0], blocks[0], feat[nodes.long()]
+    def step(hooked):
+        handle = layer.fc_self.register_forward_hook(lambda *a: None) if hooked else None
+        one = x[:1].clone().requires_grad_()
+        out = layer(block, x, feat_dst=one)
+        grads = torch.autograd.grad((out ** 2).mean(), [one] + list(layer.parameters()))
+        if handle is not None:
+            handle.remove()
+        return [out.detach()] + list(grads)
+    for a, b in zip(step(False), step(True)):
+        assert a.shape == b.shape and float((a - b).norm() / b.norm()) < 2e-6
+    with pytest.raises(RuntimeError):
+        layer(block, x, feat_dst=x[:2])
+    # (two destinations of one source, whose only row stands for both)
+    ptr, ids = torch.tensor([0, 1, 2], dtype=torch.int32, device=cuda), torch.zeros(2, dtype=torch.int32, device=cuda)
+    few = fastgl.Block(ptr, ids, 1, 2)
+    one = x[:1].clone().requires_grad_()
+    out = layer(few, one)
+    got, = torch.autograd.grad(out.sum(), one)
+    want = 2 * (layer.fc_self.weight + layer.fc_neigh.weight).detach().sum(0)
+    assert out.shape == (2, 16) and float((got[0] - want).norm() / want.norm()) < 2e-6
+    with pytest.raises(RuntimeError):
+        ops.row_product_add_(torch.zeros((1, 32), device=cuda), torch.zeros((2, 16), device=cuda), layer.fc_self.weight.detach())
+
+
 def test_gradients_of_gradients_of_the_weights(cuda):
     model, nodes, blocks, feat = _setup(cuda, torch.float32, 16, 8, 4)
     x, layer = feat[nodes.long()], model.layers[0]
