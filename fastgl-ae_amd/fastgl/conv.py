@@ -435,7 +435,8 @@ class _SageFunction(torch.autograd.Function):
     """A ``SAGEConv`` layer as a whole: the two products and their sum are one pass over the output, and in the backward pass the
     gradient of a node's own row is added to its row of the gathered gradient, where autograd would write it into a cleared array of all
     source rows and add that.  (GraphSAGE in bf16, 87 K and 41 K rows of 256 columns: 20 of a training step's 57 launches.)
-    ``feat_dst`` is ``None`` where the destination rows are the first rows of ``feat_src``."""
+    ``feat_dst`` is ``None`` where the destination rows are the first rows of ``feat_src``; otherwise ``feat_src`` gets no gradient (it is
+    the whole table, or wants none)."""
 
     @staticmethod
     def run(block, feat_src, feat_dst, w_self, w_neigh, bias, use_global):
@@ -445,23 +446,27 @@ class _SageFunction(torch.autograd.Function):
         out = ops.row_product_sum(x, w_self, h, w_neigh, bias)
         if out is None:  # (sizes that are the library's)
             out = ops.row_product(x, w_self, transposed=True) + ops.row_product(h, w_neigh, transposed=True, bias=bias)
-        return out, x, h
+        return out, h
 
     @staticmethod
     def forward(ctx, block, feat_src, feat_dst, w_self, w_neigh, bias, use_global):
-        out, x, h = _SageFunction.run(block, feat_src, feat_dst, w_self, w_neigh, bias, use_global)
-        ctx.block, ctx.use_global, ctx.own_rows = block, use_global, feat_dst is None
-        ctx.n_src = block.num_src_nodes()
-        ctx.save_for_backward(x, h, w_self, w_neigh)
+        out, h = _SageFunction.run(block, feat_src, feat_dst, w_self, w_neigh, bias, use_global)
+        ctx.block, ctx.own_rows = block, feat_dst is None
+        # (the input that the own rows come from, not the slice of it: what is saved of an input has its history when it comes back)
+        ctx.save_for_backward(feat_src if feat_dst is None else feat_dst, h, w_self, w_neigh)
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        x, h, w_self, w_neigh = ctx.saved_tensors
+        own, h, w_self, w_neigh = ctx.saved_tensors
         _, need_src, need_dst, need_self, need_neigh, need_bias, _ = ctx.needs_input_grad
+        need_src = need_src and ctx.own_rows
         d_src = d_dst = d_self = d_neigh = d_bias = None
+        x = own[:ctx.block.num_dst_nodes()] if ctx.own_rows else own
         recorded = torch.is_grad_enabled()  # (a graph of the gradients is being built: operators that have gradients themselves)
         if recorded:
+            if need_src and need_neigh:
+                h = MA_Function_Mean.apply(ctx.block, own, False)  # (the saved one was formed inside this function: no history)
             d_self = torch.mm(d_out.transpose(0, 1), x) if need_self else None
             d_neigh = torch.mm(d_out.transpose(0, 1), h) if need_neigh else None
             d_bias = d_out.sum(0) if need_bias else None
@@ -474,14 +479,14 @@ class _SageFunction(torch.autograd.Function):
                 d_bias = d_out.sum(0)
             if need_self:
                 d_self = ops.weight_grad(d_out, x)
-        if need_src and not ctx.use_global:
+        if need_src:
             t_ptr, t_idx = ctx.block.transposed()
             d_src = ops.aggregate(t_ptr, t_idx, ops.row_product(d_out, w_neigh).contiguous(), mode="colmean_ptr", zero_policy="zeros",
-                                  col_norm=ctx.block.edge_ptr, n_rows=ctx.n_src)
-            if ctx.own_rows and recorded:
+                                  col_norm=ctx.block.edge_ptr, n_rows=ctx.block.num_src_nodes())
+            if recorded:
                 n_dst = int(d_out.size(0))
                 d_src = torch.cat([d_src[:n_dst] + torch.mm(d_out, w_self), d_src[n_dst:]])
-            elif ctx.own_rows:
+            else:
                 ops.row_product_add_(d_src, d_out, w_self)
         if need_dst:
             d_dst = ops.row_product(d_out, w_self)
@@ -509,8 +514,13 @@ class SAGEConv(nn.Module):
     def _as_one(self, block, feat_src, feat_dst, use_global):
         """Whether the layer may be formed as a whole: both parts are what ``__init__`` made them, called by nobody but this layer, their
         inputs the ones that ``_Linear`` takes to the kernels, and there is one own row for each destination (a single one that stands for
-        all of them is repeated by the operators' sum) and, if they are taken from the source rows, a row of their gradient for each."""
+        all of them is repeated by the operators' sum) and, if they are taken from the source rows, a row of their gradient for each.
+        Source rows that have a gradient are saved for gradients of the gradients; the parts save their products' inputs, no more, so where
+        the own rows come from elsewhere, or a hook is handed what is saved, the layer is formed part by part."""
         if torch.compiler.is_compiling() or torch.jit.is_tracing():
+            return False
+        if torch.is_grad_enabled() and ((feat_dst is not None and not use_global and feat_src.requires_grad) or
+                                        torch._C._autograd._top_saved_tensors_default_hooks(False) is not None):
             return False
         a, b = self.fc_self, self.fc_neigh
         if type(a) is not _Linear or type(b) is not _Linear or a.bias is not None or not _called_plainly(a) or not _called_plainly(b):

@@ -160,3 +160,47 @@ def test_gradients_of_gradients_of_the_weights(cuda):
         return second
     for a, b in zip(penalty(False), penalty(True)):
         assert float((a - b).norm() / b.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("own_rows", [True, False])
+def test_gradients_of_gradients_reach_what_lies_below(cuda, own_rows):
+    """A penalty on the second layer's weight gradients, differentiated by the input and by every weight, the first layer's among them."""
+    model, nodes, blocks, feat = _setup(cuda, torch.float32, 16, 8, 4)
+    x = feat[nodes.long()].requires_grad_()
+    params = list(model.parameters())
+    def penalty(hooked):
+        handles = [layer.fc_self.register_forward_hook(lambda *a: None) for layer in model.layers] if hooked else []
+        h = model.layers[0](blocks[0], x)
+        out = model.layers[1](blocks[1], h) if own_rows else model.layers[1](blocks[1], h, feat_dst=h[:blocks[1].num_dst_nodes()] * 2)
+        g = torch.autograd.grad((out ** 3).sum(), list(model.layers[1].parameters()), create_graph=True)
+        second = torch.autograd.grad(sum((t ** 2).sum() for t in g), [x] + params)
+        for handle in handles:
+            handle.remove()
+        return second
+    for a, b in zip(penalty(False), penalty(True)):
+        assert float(b.norm()) > 0 and float((a - b).norm() / b.norm()) < 1e-5
+
+
+def test_what_is_saved_is_what_the_products_save(cuda):
+    """Saved-tensor hooks see the inputs of the products, of as many rows, and rows that only the aggregation reads may change in place."""
+    model, nodes, blocks, feat = _setup(cuda, torch.float32, 16, 8, 4)
+    layer, block = model.layers[0], blocks[0]
+    x, n_dst = feat[nodes.long()].requires_grad_(), block.num_dst_nodes()
+    def saved(hooked):
+        shapes = []
+        handle = layer.fc_self.register_forward_hook(lambda *a: None) if hooked else None
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: shapes.append(tuple(t.shape)) or t, lambda t: t):
+            layer(block, x).sum().backward()
+        if handle is not None:
+            handle.remove()
+        return sorted(shapes)
+    assert saved(False) == saved(True) and saved(False).count((n_dst, 16)) == 2
+    src, own = (t.detach().clone().requires_grad_() for t in (x, x[:n_dst]))
+    with torch.no_grad():
+        want = layer(block, src, feat_dst=own)
+    out = layer(block, src, feat_dst=own)
+    with torch.no_grad():
+        src.zero_()
+    out.sum().backward()
+    assert torch.equal(out.detach(), want) or torch.allclose(out, want, rtol=1e-5, atol=1e-5)
+    assert src.grad.shape == src.shape and own.grad.shape == own.shape
