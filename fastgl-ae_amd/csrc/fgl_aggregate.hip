@@ -147,7 +147,8 @@ struct AggArgs {
     int col_norm_is_ptr;        // col_norm is an offsets array, the counts are its differences
     void* ws;                   // scratch of aggregate_workspace_bytes(n_entries_max, D) bytes: long rows go in segments (NULL: row by row)
     int64_t n_entries_max;      // (with ws) no fewer entries than the rows hold
-    const int32_t* order;       // aggregate_kernel<.., ORDERED>: lane group i takes row order[i]
+    const int32_t* order;       // aggregate_kernel<.., ORDERED>: lane group i takes row order[i] ...
+    const int32_t* in_order;    // ... in the tiles of kSegTile rows that are marked here
 };
 
 // per-edge weight, evaluated by the lane that loaded the neighbour id
@@ -400,54 +401,17 @@ constexpr int kLongRowEntries = 128;
 // takes a workgroup for each -- 70 K rows of 446 K entries 46 / 61 / 144 / 66 -> 64 / 94 / 196 / 111.)
 constexpr int kBundleLongEntries = 48;
 
-// Rows in order of length, tile by tile (ORDERED below).  The lane groups of a wave walk their lists together, and a wave is done when its
-// longest list is: with rows that differ by an order of magnitude from one to the next -- a whole graph's -- the others wait. Here
-// a tile's rows are listed by length, longest first, so that neighbours in the list are alike, and the gather takes the rows in that
-// order; a row's sum is the same, bit for bit.  (2.4 M rows of 0..128 entries, 5.6 on average, 64 fp32 columns, four rows to a wave:
-// 1080 us as they come, 750 in order and 40 for the lists.)
-constexpr int kOrderBlock = 1024, kOrderRows = 8, kOrderTile = kOrderBlock * kOrderRows;
-__global__ __launch_bounds__(kOrderBlock) void row_order_kernel(const AggArgs g, int32_t* __restrict__ order)
+constexpr int kSegBlock = 1024, kSegRows = 8, kSegTile = kSegBlock * kSegRows;  // rows that seg_lists_kernel looks at, a workgroup
+
+// Workgroup -> place among the n of a launch that takes rows in sequence.  Workgroups go to the eight XCDs in turn, so row numbers with the same
+// few low bits are one XCD's work; where those bits say how long rows are -- R-MAT graphs: 0.76 of the entries for every bit that is zero -- one
+// XCD had almost half of all, and the others waited for it.  Every eight neighbouring workgroups are turned by as many places as a hash of
+// their number says.  (1 M R-MAT rows, us, as they come -> turned: 64 / 128 fp32 columns, 4 M draws 547 / 955 -> 368 / 658, 15 M 1196 / 2264 -> 1001 /
+// 1947; 64 / 128 bf16 columns 351 / 581 -> 233 / 385.  Rows of even lengths, or of uneven ones anywhere, are the same within the runs' 1 %.)
+__device__ __forceinline__ unsigned turned_block(unsigned b, unsigned n)
 {
-    constexpr int kBins = 256;  // lengths 0 .. 254, and all above (which the gather leaves out or are its last)
-    __shared__ int s_bin[kBins];
-    __shared__ int s_scan[kOrderBlock / kWave + 1];
-    const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
-    const int64_t r0 = (int64_t)blockIdx.x * kOrderTile;
-    if (r0 >= n_rows) return;  // (uniform over the workgroup)
-    const int tid = (int)threadIdx.x, lane = lane_id();
-    int key[kOrderRows], place[kOrderRows];
-#pragma unroll
-    for (int i = 0; i < kOrderRows; ++i) {
-        const int64_t row = r0 + i * kOrderBlock + tid;
-        key[i] = -1;
-        if (row < n_rows) {
-            const int n = g.indptr[row + 1] - g.indptr[row];
-            key[i] = kBins - 1 - (n < 0 ? 0 : n < kBins - 1 ? n : kBins - 1);  // (longest first)
-        }
-    }
-    if (tid < kBins) s_bin[tid] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kOrderRows; ++i) {
-        // (empty rows, a third of them and more: one update per wave)
-        const bool empty = key[i] == kBins - 1;
-        const unsigned long long who = __ballot(empty);
-        int base = 0;
-        if (who != 0) {
-            if (lane == __ffsll((long long)who) - 1) base = atomicAdd(&s_bin[kBins - 1], __popcll(who));
-            base = __shfl(base, __ffsll((long long)who) - 1, kWave);
-        }
-        if (empty) place[i] = base + __popcll(who & ((1ull << lane) - 1ull));
-        else place[i] = key[i] >= 0 ? atomicAdd(&s_bin[key[i]], 1) : 0;
-    }
-    __syncthreads();
-    int total;
-    const int first = block_exclusive_scan<kOrderBlock>(tid < kBins ? s_bin[tid] : 0, s_scan, &total);
-    if (tid < kBins) s_bin[tid] = first;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kOrderRows; ++i)
-        if (key[i] >= 0) order[r0 + s_bin[key[i]] + place[i]] = (int32_t)(r0 + i * kOrderBlock + tid);
+    const unsigned eight = b / 8;
+    return (eight + 1) * 8 > n ? b : eight * 8 + ((b + ((eight * 0x9E3779B1u) >> 29)) & 7u);
 }
 
 template <typename T, int VEC, int LPR, int MODE, bool ORDERED>
@@ -463,14 +427,21 @@ __global__ __launch_bounds__(kBlock) void aggregate_kernel(const AggArgs g)
 
     const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
     const int gl = (int)threadIdx.x % LPR;  // lane within the group
-    int64_t row = (int64_t)blockIdx.x * kGroups + (int)threadIdx.x / LPR;
+    const int64_t row0 = (int64_t)turned_block(blockIdx.x, gridDim.x) * kGroups;
+    int64_t row = row0 + (int)threadIdx.x / LPR;
     if (row >= n_rows) return;  // uniform per group: the cross-lane reads below stay inside the group
-    if constexpr (ORDERED) row = g.order[row];
+    int a = indptr[row], b = indptr[row + 1];
+    if constexpr (ORDERED) {
+        if (g.in_order[row0 / kSegTile]) {  // (a workgroup's rows are one tile's; in a tile that keeps its order nothing waits for the mark)
+            row = g.order[row];
+            a = indptr[row];
+            b = indptr[row + 1];
+        }
+    }
     const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, gl, D);
     const int col0 = ls.col0;
     const bool live = ls.live;
 
-    const int a = indptr[row], b = indptr[row + 1];
     {
         // rows left to aggregate_long_rows_kernel -- unless the caller's device-side count rules long
         // rows out, in which case that kernel ends at once and every row is summed here
@@ -1190,19 +1161,100 @@ __global__ void seg_init_kernel(int32_t* __restrict__ counts)
     if (threadIdx.x < 3) counts[threadIdx.x] = 0;
 }
 
+// Rows in order of length, tile by tile (ORDERED in aggregate_kernel).  The lane groups of a wave walk their lists together, and a wave is
+// done when its longest list is: with rows that differ by an order of magnitude from one to the next -- a whole graph's -- the others wait.  Such a
+// tile's rows are listed by length, longest first, so that neighbours in the list are alike, and the gather takes the rows in that
+// order; a row's sum is the same, bit for bit.  Rows that are not as unlike keep their order: there the gather, and the stores of
+// narrow rows, go through memory as they lie in it, which is worth more.  A tile is judged by the accesses that its waves wait for -- a
+// row's is one for up to kInFlight entries -- against those that its rows make: R-MAT rows wait for 1.4 / 1.8 / 2.6 times as many, two / four / eight
+// rows to a wave, log-normal ones (median 4.5, sigma 1) for 1.2 / 1.4 / 2.3, rows of 0 .. 64 entries drawn evenly for 1.3 / 1.5 / 1.7, of 8 on average
+// (Poisson) for 1.0 / 1.0 / 1.4; the lines lie between those that gain and those that do not.
+// (us, 64 fp32 columns, the rows as they come / all tiles in order, listed by a launch of their own / this way: 300 K rows, R-MAT 151 / 94 / 93 -- the turned
+// workgroups above are half of that -- log-normal 114 / 128 / 117, all of 8 entries 110 / 120 / 110; 140 K rows of 8 entries, 64 bf16 columns 33 / 45 / 35.)
+// PER_WAVE rows to a wave; every lane has the entries of rows row0 + i * kSegBlock, -1: no such row.
+template <int PER_WAVE>
+__device__ __forceinline__ void order_rows(const int (&entries)[kSegRows], int64_t row0, int limit, int* s_scan, int* s_bin, int32_t* __restrict__ order,
+                                           int32_t* __restrict__ in_order)
+{
+    constexpr int kInFlight = PER_WAVE == 8 ? 8 : 16;
+    constexpr int kLine = PER_WAVE == 8 ? 15 : PER_WAVE == 4 ? 10 : 8;  // sixths
+    constexpr int kBins = 256;  // lengths 0 .. 254, and all above (which the gather leaves out or are its last)
+    const int tid = (int)threadIdx.x, lane = lane_id();
+    // (a quarter of the tile's rows stands for it; both sums in one word: 2048 rows of at most 16 accesses each)
+    uint32_t both = 0;
+#pragma unroll
+    for (int i = 0; i < kSegRows; i += kSegRows / 2) {
+        int n = entries[i] > 0 && entries[i] <= limit ? 1 + (entries[i] - 1) / kInFlight : 0;
+        if (n > 16) n = 16;
+        both += (uint32_t)n;
+#pragma unroll
+        for (int d = 1; d < PER_WAVE; d <<= 1) {
+            const int o = __shfl_xor(n, d, kWave);
+            n = o > n ? o : n;
+        }
+        both += (uint32_t)n << 16;
+    }
+    both = (uint32_t)block_sum_of_lanes<kSegBlock>((int)both, s_scan);
+    const uint32_t made = both & 0xFFFFu, waited = both >> 16;
+    const bool unlike = 6u * waited > (uint32_t)kLine * made;  // (the same for the whole workgroup)
+    if (tid == 0) in_order[blockIdx.x] = unlike;
+    if (!unlike) return;
+    if (tid < kBins) s_bin[tid] = 0;
+    __syncthreads();
+    int key[kSegRows], place[kSegRows];
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i) {
+        key[i] = entries[i] < 0 ? -1 : kBins - 1 - (entries[i] < kBins - 1 ? entries[i] : kBins - 1);  // (longest first)
+        // (empty rows, a third of them and more: one update per wave)
+        const bool empty = key[i] == kBins - 1;
+        const unsigned long long who = __ballot(empty);
+        int base = 0;
+        if (who != 0) {
+            if (lane == __ffsll((long long)who) - 1) base = atomicAdd(&s_bin[kBins - 1], __popcll(who));
+            base = __shfl(base, __ffsll((long long)who) - 1, kWave);
+        }
+        if (empty) place[i] = base + __popcll(who & ((1ull << lane) - 1ull));
+        else place[i] = key[i] >= 0 ? atomicAdd(&s_bin[key[i]], 1) : 0;
+    }
+    __syncthreads();
+    int total;
+    const int first = block_exclusive_scan<kSegBlock>(tid < kBins ? s_bin[tid] : 0, s_scan, &total);
+    if (tid < kBins) s_bin[tid] = first;
+    __syncthreads();
+    const int64_t tile0 = row0 - tid;
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i)
+        if (key[i] >= 0) order[tile0 + s_bin[key[i]] + place[i]] = (int32_t)(row0 + (int64_t)i * kSegBlock);
+}
+
 // The lists.  Their order is up to scheduling, the sums are not: a row's segments are cut and added the same way on every run.
 // A workgroup looks through kSegRows rows per lane and takes its places in the lists with three atomics (one address each:
-// their updates run one after the other, so there are few of them).
-constexpr int kSegBlock = 1024, kSegRows = 8;
-__global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, const SegLists l)
+// their updates run one after the other, so there are few of them).  PER_WAVE: the gather's order of the rows as well (0: no order).
+template <int PER_WAVE>
+__global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, const SegLists l, int32_t* __restrict__ order,
+                                                              int32_t* __restrict__ in_order)
 {
     __shared__ int s_scan[kSegBlock / kWave + 1];
     __shared__ int s_base[3];
-    const int threshold = g.skip_rows_longer_than;
-    if (g.longest_row != nullptr && *g.longest_row <= threshold) return;
+    int threshold = g.skip_rows_longer_than;
+    const bool none_left_out = g.longest_row != nullptr && *g.longest_row <= threshold;
+    if (none_left_out && PER_WAVE == 0) return;
+    if (none_left_out) threshold = 0x7FFFFFFF;
     const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
-    const int64_t row0 = (int64_t)blockIdx.x * kSegBlock * kSegRows + threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * kSegTile + threadIdx.x;
     int first[kSegRows], entries[kSegRows];
+#pragma unroll
+    for (int i = 0; i < kSegRows; ++i) {
+        const int64_t row = row0 + (int64_t)i * kSegBlock;
+        first[i] = row < n_rows ? g.indptr[row] : 0;
+        entries[i] = row < n_rows ? g.indptr[row + 1] - first[i] : -1;
+        if (row < n_rows && entries[i] < 0) entries[i] = 0;
+    }
+    if constexpr (PER_WAVE > 0) {
+        __shared__ int s_bin[256];
+        order_rows<PER_WAVE>(entries, row0, threshold, s_scan, s_bin, order, in_order);
+        if (none_left_out) return;
+    }
     int segs = 0, ones = 0, many = 0;
 #pragma unroll
     for (int i = 0; i < kSegRows; ++i) {
@@ -1220,6 +1272,7 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
             segs += (entries[i] + kSegEntries - 1) / kSegEntries;
         }
     }
+    if (__syncthreads_or(ones | many) == 0) return;
     int total_segs, total_ones, total_many;
     int at_seg = block_exclusive_scan<kSegBlock>(segs, s_scan, &total_segs);
     int at_one = block_exclusive_scan<kSegBlock>(ones, s_scan, &total_ones);
@@ -1510,10 +1563,9 @@ static void note_mapping(const char* kernel, int lpr, int extra, bool second_pas
              !second_pass ? "" : segments ? " + segments" : " + long_rows");
 }
 
-// From this many rows on, rows of a large block with long ones among them are gathered in order of length (rows of up to 32 lanes: a 64-lane
-// row has its wave to itself).  Whole R-MAT graphs, us, as they come -> in order: 2.4 M rows of 64 fp32 columns, 54 M entries 2956 -> 2644,
-// 18 M entries 1377 -> 970; 1 M rows 818 -> 613; 500 K rows 397 -> 317, of 64 bf16 columns 277 -> 194; 200 K rows 173 -> 124, 152 -> 99;
-// 50 K rows 74 -> 76, 73 -> 76 (one more launch, and the chip no longer full).
+// From this many rows on, the tiles of a large block with long rows among them are looked at for an order by length (rows of up to 32 lanes: a
+// 64-lane row has its wave to itself).  R-MAT graphs, us, with the workgroups turned only / with the order: 1 M rows of 64 bf16 columns 535 / 423,
+// 64 fp32 columns 1001 / 983; 150 K rows 90 / 77, 109 / 99; 50 K rows, as they come / in order, 73 / 76 (the chip is no longer full).
 constexpr int64_t kOrderMinRows = (int64_t)1 << 17;
 
 // Workgroups of the long-row pass: each looks through an equal share of the row offsets.
@@ -1523,6 +1575,14 @@ constexpr int kLongRowBlocks = 1021;  // a prime: rows are dealt round robin, an
 // Lists with more entries than this are the second launch's (segments are sized for the one limit).
 static inline int long_row_limit(bool bundle, const AggArgs& g) { return bundle && g.ws == nullptr ? kBundleLongEntries : kLongRowEntries; }
 
+template <int PER_WAVE>
+static void launch_seg_lists(const SegLists& l, hipStream_t stream, const AggArgs& g, int32_t* order, int32_t* in_order)
+{
+    hipLaunchKernelGGL(seg_init_kernel, dim3(1), dim3(kWave), 0, stream, l.counts);
+    hipLaunchKernelGGL(seg_lists_kernel<PER_WAVE>, dim3((unsigned)ceil_div(g.n_rows_max, kSegTile)), dim3(kSegBlock), 0, stream, g, l, order,
+                       in_order);
+}
+
 // The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
 // for large inputs), else a workgroup per row.
 template <typename T, int VEC, int LPR, int MODE>
@@ -1531,8 +1591,7 @@ static void launch_long_rows(unsigned gy, hipStream_t stream, const AggArgs& g)
     if constexpr (MODE != FGL_AGG_EDGE) {
         if (g.ws != nullptr) {
             const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
-            hipLaunchKernelGGL(seg_init_kernel, dim3(1), dim3(kWave), 0, stream, l.counts);
-            hipLaunchKernelGGL(seg_lists_kernel, dim3((unsigned)ceil_div(g.n_rows_max, kSegBlock * kSegRows)), dim3(kSegBlock), 0, stream, g, l);
+            if (g.order == nullptr) launch_seg_lists<0>(l, stream, g, nullptr, nullptr);  // (else listed with the rows' order)
             // (a unit has more than kLongRowEntries entries, or is one of at most two per kSegEntries > 2 * kLongRowEntries of them)
             static_assert(kSegEntries > 2 * kLongRowEntries, "the bound on the number of units");
             hipLaunchKernelGGL((aggregate_segments_kernel<T, VEC, LPR, MODE>), dim3((unsigned)ceil_div(l.cap_one, kBlock / kWave), gy),
@@ -1571,12 +1630,13 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
     bool ordered = false;
     if constexpr (LPR <= 32) {
         if (second_pass && g.ws != nullptr && mode != FGL_AGG_EDGE && g.n_rows_max >= kOrderMinRows) {
-            // (in the place of the partial sums, which the launches behind this one fill)
+            // (in the place of the partial sums, which the launches behind the gather fill; the launch that lists the long rows finds the order)
             const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
-            if ((int64_t)l.cap_seg * l.ldp >= g.n_rows_max) {
+            if ((int64_t)l.cap_seg * l.ldp >= g.n_rows_max + ceil_div(g.n_rows_max, kSegTile)) {
                 int32_t* order = reinterpret_cast<int32_t*>(l.partial);
-                hipLaunchKernelGGL(row_order_kernel, dim3((unsigned)ceil_div(g.n_rows_max, kOrderTile)), dim3(kOrderBlock), 0, stream, g, order);
+                launch_seg_lists<kWave / LPR>(l, stream, g, order, order + g.n_rows_max);
                 g.order = order;
+                g.in_order = order + g.n_rows_max;
                 ordered = true;
             }
         }
@@ -1856,6 +1916,7 @@ FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indice
     g.ws = ws_needed > 0 && d_ws != nullptr && ws_bytes >= ws_needed ? d_ws : nullptr;
     g.n_entries_max = n_entries_max;
     g.order = nullptr;
+    g.in_order = nullptr;
     hipStream_t s = as_stream(stream);
     if (dtype == FGL_F32) return launch_agg_vec<float, 4>(mode, longest_row_max, n_entries_max, s, g);
     if (bf16_rows_dword_aligned(ldx, ldo, d_x, d_out)) return launch_agg_vec<uint16_t, 8>(mode, longest_row_max, n_entries_max, s, g);

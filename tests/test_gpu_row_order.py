@@ -1,5 +1,5 @@
-"""Rows gathered in order of length (large blocks with long rows among them) against the same rows as they come -- a row of up to 128
-entries is the same sum, bit for bit -- and, for the longer ones, against float64; at the sizes where the order starts and a tile ends."""
+"""Rows gathered in order of length (large blocks with long rows among them) against the same rows as they come: a row of up to 128
+entries is the same sum, bit for bit, a longer one the same up to the order of its sum; at the sizes where the order starts and a tile ends."""
 import pytest
 import torch
 
