@@ -87,7 +87,7 @@ constexpr int kBucketItems = 16;  // entries per lane
 constexpr int kBucketTile = kBucketBlock * kBucketItems;  // entries that are put in order in LDS together
 constexpr int kMaxBuckets = 2048;
 constexpr int kMinWidthLog = 11, kMaxWidthLog = 13;
-constexpr int kSegment = 32768;  // entries per workgroup of the passes over buckets
+constexpr int kSegment = 32768, kMinSegment = 8192;  // entries per workgroup of the passes over buckets: BucketArgs::segment, between these
 
 struct BucketArgs {
     const int32_t* ids;          // column of every entry
@@ -96,7 +96,7 @@ struct BucketArgs {
     const int32_t* indptr;       // transpose only: rows of the entries
     int64_t n_rows;
     int64_t n_cols;
-    int width_log, buckets;
+    int width_log, buckets, segment;
     int64_t tiles;               // of kBucketTile entries
     int32_t* hist;               // [bucket][tile] counts, then their prefix sums (+ 1 entry: the total)
     int32_t* tile_row;           // [tile] the row that holds the tile's first entry
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_scatter_kernel(const Buck
     if constexpr (EDGES) send(g.b_edge, [&](int j) { return (int)(e0 + at + j); });
 }
 
-// One workgroup: the buckets cut into segments of at most kSegment entries.
+// One workgroup: the buckets cut into segments of at most g.segment entries.
 __global__ __launch_bounds__(1024) void bucket_segments_kernel(const BucketArgs g)
 {
     __shared__ int smem[1024 / kWave + 1];
@@ -283,14 +283,14 @@ __global__ __launch_bounds__(1024) void bucket_segments_kernel(const BucketArgs 
             first = g.hist[(int64_t)b * g.tiles];
             size = g.hist[(int64_t)(b + 1) * g.tiles] - first;
         }
-        const int segs = (size + kSegment - 1) / kSegment;
+        const int segs = (size + g.segment - 1) / g.segment;
         int total;
         const int at = carry + block_exclusive_scan<1024>(segs, smem, &total);
         for (int q = 0; q < segs; ++q) {
             int32_t* s = g.segments + 1 + 3 * (at + q);
             s[0] = b;
-            s[1] = first + q * kSegment;
-            s[2] = size - q * kSegment < kSegment ? size - q * kSegment : kSegment;
+            s[1] = first + q * g.segment;
+            s[2] = size - q * g.segment < g.segment ? size - q * g.segment : g.segment;
         }
         carry += total;
     }
@@ -340,24 +340,83 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_count_kernel(const Bucket
 // ... and, once the counts have become offsets, every entry into its column's row of the transposed block.  A chunk of the segment
 // is put in order by column in LDS and leaves as runs: stored one by one, a segment's entries go all over its bucket's 200 KB of
 // the output, a thousand segments' worth of which no L2 holds.  (54 M entries: 737 -> 207 us.)
+// Entries that are next to each other in the output already -- those of sorted ids, and of a graph whose rows keep to a band -- and segments
+// of buckets with fewer entries than columns are stored as they are met: ordering them only lengthens the chain.  (This launch, all segments in order ->
+// now, as it was when all were stored: 300 K entries, 6 M columns 55 -> 10, 11; 5 M in a band of 14 M columns 114 -> 35, 31; whole transposes with edge ids, 1.2 M
+// sorted entries of 300 K columns 71 -> 61, 60; 30 M of 2.4 M columns, sorted 505 -> 453, 572, in a band 64 wide 480 -> 482, 749, uniform 577 -> 575, 2061.)
+constexpr int kLook = 4;    // entries of a lane that a segment is judged by
+constexpr int kNear = 200;  // entries of the output that neighbours may lie apart on average: bands 64 wide cross at some ten entries a column
 template <int WIDTH_LOG, bool EDGES>
 __global__ __launch_bounds__(kBucketBlock) void bucket_fill_kernel(const BucketArgs g)
 {
     constexpr int kWidth = 1 << WIDTH_LOG, kPer = kWidth / kBucketBlock;
     __shared__ int s_buf[kBucketTile];
-    __shared__ int s_start[kWidth];
-    __shared__ int s_delta[kWidth];  // (and, before it is filled, the scratch of the scan)
+    __shared__ int s_at[kWidth + kBucketBlock];  // by column: entries, their first place in the chunk, what leads from there to the output
+    __shared__ int s_scan[kBucketBlock / kWave + 1];
+    auto slot = [](int c) { return c + c / kPer; };  // (a lane's columns are neighbours: no two lanes meet in a bank)
     const int seg = (int)blockIdx.x;
     if (seg >= g.segments[0]) return;
     const int bucket = g.segments[1 + 3 * seg], first = g.segments[2 + 3 * seg], size = g.segments[3 + 3 * seg];
     const int tid = (int)threadIdx.x;
     // the segment's next place in each of the lane's columns (columns that it does not mention: never used)
     int next[kPer];
+    {
+        const int64_t col0 = (int64_t)bucket * kWidth + tid * kPer;
+        const int32_t* base = g.seg_base + (int64_t)seg * kWidth + tid * kPer;
+        if (col0 + kPer <= g.n_cols) {
+            typedef int32_t I4 __attribute__((ext_vector_type(4), aligned(4)));
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const int c = tid * kPer + q;
-        const int64_t col = ((int64_t)bucket << g.width_log) + c;
-        next[q] = c < 1 << g.width_log && col < g.n_cols ? g.counts[col] + g.seg_base[((int64_t)seg << g.width_log) + c] : 0;
+            for (int q = 0; q < kPer / 4; ++q) {
+                const I4 a = reinterpret_cast<const I4*>(g.counts + col0)[q], b = reinterpret_cast<const I4*>(base)[q];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) next[4 * q + j] = a[j] + b[j];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) next[q] = col0 + q < g.n_cols ? g.counts[col0 + q] + base[q] : 0;
+        }
+    }
+    // how far apart neighbouring entries' columns lie, from the segment's first entries, and how many entries the bucket's columns have
+    const int64_t bucket0 = (int64_t)bucket * kWidth;
+    const int64_t entries = (bucket0 + kWidth < g.n_cols ? g.counts[bucket0 + kWidth] : g.n_max) - g.counts[bucket0];
+    bool direct = entries < kWidth;
+    if (!direct && size >= kLook * kBucketBlock) {  // (uniform over the workgroup)
+        int apart = 0;
+#pragma unroll
+        for (int j = 0; j < kLook; ++j) {
+            const int c = g.b_col[(int64_t)first + tid + j * kBucketBlock];
+            const int d = c - __shfl_xor(c, 1, kWave);
+            apart += d < 0 ? -d : d;
+        }
+        apart = block_sum_of_lanes<kBucketBlock>(apart, s_scan);
+        direct = (int64_t)apart * entries < (int64_t)kNear * kWidth * (kLook * kBucketBlock);
+    }
+    if (direct) {
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) s_at[slot(tid * kPer + q)] = next[q];
+        __syncthreads();
+        constexpr int kInFlight = 4;
+        for (int i0 = tid; i0 < size; i0 += kInFlight * kBucketBlock) {
+            int c[kInFlight], r[kInFlight], e[kInFlight];
+#pragma unroll
+            for (int j = 0; j < kInFlight; ++j) {
+                const int64_t i = i0 + j * kBucketBlock;
+                c[j] = -1;
+                if (i < size) {
+                    c[j] = g.b_col[first + i];
+                    r[j] = g.b_row[first + i];
+                    if constexpr (EDGES) e[j] = g.b_edge[first + i];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kInFlight; ++j) {
+                if (c[j] < 0) continue;
+                const int at = atomicAdd(&s_at[slot(c[j])], 1);
+                g.t_indices[at] = r[j];
+                if constexpr (EDGES) g.t_edge[at] = e[j];
+            }
+        }
+        return;
     }
     for (int from = 0; from < size; from += kBucketTile) {
         const int here = size - from < kBucketTile ? size - from : kBucketTile;
@@ -368,39 +427,43 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_fill_kernel(const BucketA
             const int i = tid + j * kBucketBlock;
             c[j] = i < here ? (int)g.b_col[e0 + i] : -1;
         }
-        for (int q = tid; q < kWidth; q += kBucketBlock) s_start[q] = 0;
+        for (int q = tid; q < kWidth + kBucketBlock; q += kBucketBlock) s_at[q] = 0;
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kBucketItems; ++j) place[j] = c[j] >= 0 ? atomicAdd(&s_start[c[j]], 1) : 0;
+        for (int j = 0; j < kBucketItems; ++j) place[j] = c[j] >= 0 ? atomicAdd(&s_at[slot(c[j])], 1) : 0;
         __syncthreads();
         int cnt[kPer], sum = 0;
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            cnt[q] = s_start[tid * kPer + q];
+            cnt[q] = s_at[slot(tid * kPer + q)];
             sum += cnt[q];
         }
         int total;
-        int run = block_exclusive_scan<kBucketBlock>(sum, s_delta, &total);
+        int run = block_exclusive_scan<kBucketBlock>(sum, s_scan, &total);
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
-            s_start[tid * kPer + q] = run;
-            s_delta[tid * kPer + q] = next[q] - run;
-            next[q] += cnt[q];
-            run += cnt[q];
+            s_at[slot(tid * kPer + q)] = run;
+            const int n = cnt[q];
+            cnt[q] = next[q] - run;
+            next[q] += n;
+            run += n;
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < kBucketItems; ++j) {
             if (c[j] < 0) continue;
-            place[j] += s_start[c[j]];
+            place[j] += s_at[slot(c[j])];
             s_buf[place[j]] = c[j];
         }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) s_at[slot(tid * kPer + q)] = cnt[q];
         __syncthreads();
         int to[kBucketItems];
 #pragma unroll
         for (int j = 0; j < kBucketItems; ++j) {
             const int i = tid + j * kBucketBlock;
-            to[j] = i < here ? i + s_delta[s_buf[i]] : 0;
+            to[j] = i < here ? i + s_at[slot(s_buf[i])] : 0;
         }
         auto send = [&](int32_t* out, const int32_t* in) {  // (one array after the other: registers)
             int v[kBucketItems];
@@ -455,6 +518,17 @@ static bool count_by_buckets(int64_t n_ids, int64_t n_counters)
 // 300 K, 300 K 32 / 47, 207 / 70); from 1.2 M on neither does.
 bool bucket_transpose_form(int64_t n_entries, int64_t n_cols) { return n_entries >= ((int64_t)1 << 18) && fits_buckets(n_entries, n_cols); }
 
+// Up to two million entries, segments are shorter: those of 32768 are so few that most of the chip waits for them, the longer the more is done for
+// each chunk of them.  From 128 buckets on, half as many entries again as a bucket holds on average, so that buckets that are alike are not cut.
+// (Transposes with edge ids, us, segments of 32768 / these: 300 K entries, 30 K columns, uniform 69 / 53, in a band 72 / 55; 1.2 M entries, 30 K columns 99 / 70,
+// 300 K columns, uniform 66 / 65, drawn as u^3 96 / 73.)
+static int segment_entries(int64_t n_entries, int64_t buckets)
+{
+    if (n_entries > ((int64_t)1 << 21)) return kSegment;
+    const int64_t s = buckets < 128 ? kMinSegment : (int64_t)align_up((size_t)(n_entries * 3 / (2 * buckets)), 512);
+    return (int)(s < kMinSegment ? kMinSegment : s > kSegment ? kSegment : s);
+}
+
 static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edges, void* ws, BucketArgs* g, size_t* bytes)
 {
     int w = kMinWidthLog;
@@ -462,7 +536,8 @@ static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edg
     g->width_log = w;
     g->buckets = (int)((n_cols + ((int64_t)1 << w) - 1) >> w);
     g->tiles = ceil_div(n_entries, kBucketTile);
-    const int64_t max_segments = g->buckets + n_entries / kSegment + 1;
+    g->segment = segment_entries(n_entries, g->buckets);
+    const int64_t max_segments = g->buckets + n_entries / g->segment + 1;
     Carver c(ws);
     g->hist = c.take<int32_t>((size_t)(g->buckets * g->tiles + 1));
     g->segments = c.take<int32_t>((size_t)(1 + 3 * max_segments));
@@ -502,7 +577,7 @@ static int launch_partition(const BucketArgs& g, bool rows, bool edges, hipStrea
     else if (rows) hipLaunchKernelGGL((bucket_scatter_kernel<true, false>), dim3(tiles), dim3(kBucketBlock), 0, stream, g);
     else hipLaunchKernelGGL((bucket_scatter_kernel<false, false>), dim3(tiles), dim3(kBucketBlock), 0, stream, g);
     hipLaunchKernelGGL(bucket_segments_kernel, dim3(1), dim3(1024), 0, stream, g);
-    const unsigned segs = (unsigned)(g.buckets + g.n_max / kSegment + 1);
+    const unsigned segs = (unsigned)(g.buckets + g.n_max / g.segment + 1);
     if (rows) hipLaunchKernelGGL(bucket_count_kernel<true>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
     else hipLaunchKernelGGL(bucket_count_kernel<false>, dim3(segs), dim3(kBucketBlock), 0, stream, g);
     FGL_CHECK_LAUNCH("bucket_count_kernel");
@@ -561,14 +636,17 @@ int launch_bucket_transpose(const int32_t* d_indptr, const int32_t* d_indices, i
     // (the histogram is no longer needed: scratch of this scan)
     rc = launch_exclusive_sum(d_t_indptr, n_cols, nullptr, d_t_indptr, nullptr, g.hist, scan_workspace_bytes(n_cols), stream);
     if (rc != FGL_OK) return rc;
-    const unsigned segs = (unsigned)(g.buckets + n_edges / kSegment + 1);
-    if (g.width_log == kMinWidthLog) {
-        if (edges) hipLaunchKernelGGL((bucket_fill_kernel<kMinWidthLog, true>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
-        else hipLaunchKernelGGL((bucket_fill_kernel<kMinWidthLog, false>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
-    } else {
-        if (edges) hipLaunchKernelGGL((bucket_fill_kernel<kMaxWidthLog, true>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
-        else hipLaunchKernelGGL((bucket_fill_kernel<kMaxWidthLog, false>), dim3(segs), dim3(kBucketBlock), 0, stream, g);
-    }
+    const unsigned segs = (unsigned)(g.buckets + n_edges / g.segment + 1);
+#define FGL_LAUNCH_FILL(W)                                                                                                   \
+    do {                                                                                                                      \
+        if (edges) hipLaunchKernelGGL((bucket_fill_kernel<W, true>), dim3(segs), dim3(kBucketBlock), 0, stream, g);             \
+        else hipLaunchKernelGGL((bucket_fill_kernel<W, false>), dim3(segs), dim3(kBucketBlock), 0, stream, g);                  \
+    } while (0)
+    static_assert(kMaxWidthLog == kMinWidthLog + 2, "a form of the kernel for each width");
+    if (g.width_log == kMinWidthLog) FGL_LAUNCH_FILL(kMinWidthLog);
+    else if (g.width_log == kMinWidthLog + 1) FGL_LAUNCH_FILL(kMinWidthLog + 1);
+    else FGL_LAUNCH_FILL(kMaxWidthLog);
+#undef FGL_LAUNCH_FILL
     FGL_CHECK_LAUNCH("bucket_fill_kernel");
     return FGL_OK;
 }

@@ -1,5 +1,6 @@
 """The partition behind large counts and transposes, at the edges of what it puts in order in LDS: tiles of 8192 entries, segments of
-32768, buckets of 2^11 and 2^12 columns; sorted ids (runs of equal ones), ids that start on any word, and ids that are none.
+8192 to 32768, buckets of 2^11 to 2^13 columns, entries stored in order or as they are met; sorted ids (runs of equal ones), ids in a band, ids that
+start on any word, and ids that are none.
 Whole numbers, equal to torch.bincount and to the sorted pairs."""
 import pytest
 import torch
@@ -14,6 +15,9 @@ M = 1 << 20
 def _ids(kind, n, bins, gen, device):
     if kind == "sorted":
         return (torch.arange(n, device=device) * bins // max(n, 1)).int()
+    if kind == "band":
+        at = torch.arange(n, device=device) * bins // max(n, 1) + torch.randint(0, 64, (n,), generator=gen, device=device)
+        return at.clamp(max=bins - 1).int()
     ids = torch.randint(0, bins, (n,), generator=gen, device=device, dtype=torch.int32)
     if kind == "runs":  # runs of 1..40 equal ids, none of them at the same place in a lane's sixteen
         ids = torch.repeat_interleave(ids, torch.randint(1, 41, (n,), generator=gen, device=device))[:n].contiguous()
@@ -36,8 +40,9 @@ def test_counts(cuda, kind, n, bins, first):
 
 
 @pytest.mark.parametrize("edge_ids", [False, True])
-@pytest.mark.parametrize("kind", ["sorted", "runs", "hub"])
-@pytest.mark.parametrize("n,cols", [((1 << 18), 2048), ((1 << 18) + 1, 2049), (32 * 8192 + 8191, 4 * M + 1), (300_000, 1), (M + 8193, 100_000)])
+@pytest.mark.parametrize("kind", ["sorted", "runs", "hub", "band"])
+@pytest.mark.parametrize("n,cols", [((1 << 18), 2048), ((1 << 18) + 1, 2049), (32 * 8192 + 8191, 4 * M + 1), (300_000, 1), (M + 8193, 100_000),
+                                    ((1 << 18) + 1, 9 * M), (2 * M, 127 * 2048), (2 * M, 128 * 2048), (2 * M + 1, 300_000), (6 * M, 5 * M), (4 * M, 2047)])
 def test_transposes(cuda, kind, n, cols, edge_ids):
     print("transposes", kind, n, cols, edge_ids, flush=True)
     gen = torch.Generator(device=cuda).manual_seed(n + cols)
