@@ -367,13 +367,25 @@ def _splits_k(k, m, n):
 
 def _long_product_is_the_kernels(dtype, transposed, k, n):
     """Beyond 8e9 multiplications: whether the kernel is ahead of the library for a product of k x n.  A short k leaves little to multiply for each
-    row that moves, and the library moves rows at half the memory's rate, less where a row of the result is no whole number of lines.
-    2.4 M rows, us, library / kernel (transposed): fp32 16 x 64 293 / 151 (191 / 153), 50 x 50 503 / 334 (456 / 356), 64 x 100 627 / 449 (621 / 510),
-    100 x 100 826 / 709 (1933 / 886), but 64 x 64 327 / 345, 100 x 16 345 / 373, 100 x 64 510 / 550, 128 x 64 460 / 559; bf16 64 x 64 202 / 123 (194 / 135),
-    64 x 100 525 / 164 (465 / 182), 100 x 64 360 / 238 (355 / 277), 128 x 128 309 / 264 (but 298 / 359)."""
+    row that moves, and the library moves rows at half the memory's rate: up to k = 32 in fp32, and in bf16 up to 128 (transposed: 100), the kernel is
+    ahead.  For a longer k in fp32 it depends on what either pads.  The library is slow where a row is no whole number of 64-byte lines (a
+    sixteenth of the sizes is its own, then); the kernel works in 32 columns a wave, one vector of two or four a lane where that pads little, so
+    that 65 .. 80 columns cost it as much as 96, one by one, and 129 .. 160 as much as 192.  The lines lie where sweeps of n = 33 .. 330 cross, k = 36 .. 128.
+    Kernel's time over the library's, 9e9 multiplications (transposed), k = 64 / 100 / 128: 40 columns 0.96 / 1.01 / 1.19 (0.61 / 0.62 / 0.69), 50 columns
+    0.78 / 0.76 / 0.94 (0.85 / 0.87 / 1.01), 72 columns 1.06 / 1.44 / 1.48 (1.13 / 0.79 / 0.86), 80 columns 1.38 / 1.50 / - (1.49 / 1.66 / -), 90 columns 0.87 /
+    0.95 / 1.01 (0.93 / 1.11 / 1.18), 100 columns 0.62 / 0.87 / 0.82 (0.70 / 0.47 / 0.88), 120 columns 0.58 / 0.76 / 0.82 (0.66 / 0.91 / 0.89), 130 columns 1.21 /
+    1.35 / 1.29 (1.09 / 0.56 / 0.62), 250 columns 0.47 / 0.82 / 0.51 (0.68 / 0.81 / 0.86), 300 columns 0.66 / 0.89 / 0.98 (0.72 / 0.84 / 1.08); 128 x 64 is
+    the library's in both layouts.  bf16, k = 64 / 100 / 128: 64 columns 0.61 / 0.62 / 0.86, 100 columns 0.30 / 0.36 / 0.43, but 96 columns, one by one again,
+    0.78 / 0.86 / 1.09 and with k = 96 1.12 (1.19); transposed odd columns beyond 192, stored one by one, 0.83 / 1.06 / 1.33."""
     if dtype == torch.bfloat16:
-        return k <= (100 if transposed else 128)
-    return k <= 32 or (k <= 100 and n > 32 and n % 32 != 0)
+        return k <= (100 if transposed else 128) and not (64 < n <= 96 and n % 16 == 0) and not (transposed and n > 192 and n % 2 == 1)
+    if k <= 32:
+        return True
+    if k > 128 or n % 16 == 0:
+        return False
+    if n <= 192:
+        return (32 if transposed else 48) < n < 64 or (96 if transposed else 80) < n < 128
+    return k <= (100 if transposed else 128) and -(-n // 64) * 64 <= 1.15 * (-(-n // 16) * 16)
 
 
 def _forms_row_product(a, b, transposed, m, k, n):
@@ -389,8 +401,9 @@ def _forms_row_product(a, b, transposed, m, k, n):
     line keep the GPU busy for longer than the host takes, and there it depends on the size (a GIN layer of 602 x 256 over 8192 rows, forward and backward, is the
     library's: 394 / 418 in all), see ``_long_product_is_the_kernels``.
     Returns the operands' addresses and row strides if so, else None."""
-    if not ((m * k * n <= 8 * 10 ** 9 or _long_product_is_the_kernels(a.dtype, transposed, k, n)) and k * n <= 100000 and a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and
-            0 < n <= 65536 and a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
+    if not (k * n <= 100000 and (m * k * n <= 8 * 10 ** 9 or _long_product_is_the_kernels(a.dtype, transposed, k, n)) and
+            a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
+            a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
             not torch.is_autocast_enabled() and not _followed()):
         return None
     (lda, unit_a), (ldb, unit_b), at = a.stride(), b.stride(), _addresses(a, b)
