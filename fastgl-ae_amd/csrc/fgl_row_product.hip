@@ -372,9 +372,13 @@ static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStre
         const int64_t waves = ceil_div(g.m, 32) * (p / (32 * v));
         if (g.n >= v && p * 10 <= pad1 * 12 && waves >= 1024 && (FORM != kRpAdd || g.n % v == 0)) vb = v;
     }
-    // (a sum keeps the first product's values besides the accumulators: no tall tiles)
-    const bool tall = FORM != kRpSum && vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048;
-    if constexpr (FORM != kRpSum) {
+    // A bf16 sum keeps the first product's values besides the accumulators: no tall tiles.  An fp32 one goes on in the same accumulators; it gains by
+    // tall tiles where there is enough to multiply (us, tiles of 32 / 64 rows: 87 K rows of 2 x 256 x 256 276 / 242, 2 x 100 x 256 128 / 115, 200 K of 2 x 256 x 64
+    // 235 / 200, 2 x 128 x 128 192 / 180; but 2 x 100 x 100 146 / 150, 2 x 64 x 64 51 / 53, 2 x 50 x 47 45 / 49).
+    constexpr bool kTall = FORM != kRpSum || sizeof(T) == 4;
+    const bool tall = kTall && vb >= 2 && ceil_div(g.m, 64) * ceil_div(g.n, 32 * vb) >= 2048 &&
+                      (FORM != kRpSum || (int64_t)(g.side[0].k + g.side[1].k) * g.n >= 32768);
+    if constexpr (kTall) {
         if (vb == 4 && tall) return launch_row_product<T, 2, 4, BT, FORM>(g, stream);
         if (vb == 2 && tall) return launch_row_product<T, 2, 2, BT, FORM>(g, stream);
     }

@@ -433,8 +433,8 @@ def row_product(a, b, transposed=False, bias=None):
 
 
 def row_product_sum(a0, b0, a1, b1, bias=None):
-    """``a0 b0^T + (a1 b1^T + bias)`` in one pass over the result, rounded as the two products and their sum would be, for the operands
-    that ``row_product`` takes to the kernel; ``None`` for all others."""
+    """``a0 b0^T + (a1 b1^T + bias)`` in one pass over the result, for the operands that ``row_product`` takes to the kernel; ``None`` for all
+    others.  bf16: rounded where the two products and their sum would be; fp32: one sum over both products' terms, the bias added last."""
     m, n = int(a0.size(0)), int(b0.size(0))
     k0, k1 = int(a0.size(1)), int(a1.size(1))
     if int(a1.size(0)) != m or int(b1.size(0)) != n or a1.dtype != a0.dtype or a1.device != a0.device or int(b0.size(1)) != k0 or int(b1.size(1)) != k1:

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # two operands' k around a step (8 / 16), m around a tile (32, 64, 128), n around a vector and a tile
 @pytest.mark.parametrize("dtype,rel", [(torch.float32, 1e-6), (torch.bfloat16, 6e-3)])  # (bf16: two values and their sum rounded, 2^-9 each)
 @pytest.mark.parametrize("m,k0,k1,n", [(1, 2, 2, 1), (33, 8, 16, 32), (64, 34, 2, 66), (127, 100, 256, 47), (200, 16, 130, 128), (1025, 64, 62, 256),
-                                       (70_000, 32, 48, 96)])
+                                       (70_000, 32, 48, 96), (65_537, 60, 70, 256), (65_537, 64, 62, 256), (131_009, 258, 254, 64)])
 def test_two_products_in_one_pass(cuda, dtype, rel, m, k0, k1, n):
     print("pair", dtype, m, k0, k1, n, flush=True)
     gen = torch.Generator().manual_seed(m + n)
