@@ -376,8 +376,7 @@ __global__ __launch_bounds__(kBlock) void sample_insert_kernel(const int32_t* __
                                                                const int32_t* __restrict__ d_n, int fanout,
                                                                const int64_t* __restrict__ row_start,
                                                                const int32_t* __restrict__ deg_arr,
-                                                               const int32_t* __restrict__ tile_sums,
-                                                               const int32_t* __restrict__ tile_prefix, uint32_t seed_lo,
+                                                               const int32_t* __restrict__ tile_sums, uint32_t seed_lo,
                                                                uint32_t seed_hi, uint32_t stream_id,
                                                                const uint32_t* __restrict__ d_stream_add, int32_t* src_out,
                                                                int32_t* __restrict__ block_ptr, int32_t* __restrict__ n_edges_out,
@@ -401,7 +400,7 @@ __global__ __launch_bounds__(kBlock) void sample_insert_kernel(const int32_t* __
     const int64_t e_max = n_max * fanout;
     const int64_t n = actual_count(n_max, d_n);
     const int64_t n_tiles = (n + TS - 1) / TS;
-    publish_empty(tile_prefix, n_tiles, block_ptr, n_edges_out, nullptr, d_status);
+    publish_empty(nullptr, n_tiles, block_ptr, n_edges_out, nullptr, d_status);
     for (int64_t sub = blockIdx.x; sub < n_tiles * kParts; sub += gridDim.x) {
         const int64_t tile = sub / kParts;
         const int part = (int)(sub % kParts);
@@ -414,7 +413,7 @@ __global__ __launch_bounds__(kBlock) void sample_insert_kernel(const int32_t* __
             seed = seeds[i];
         }
         // (the earlier tiles' sums are fetched while the seed's own three loads are still under way)
-        const int sum_before = tile_prefix ? 0 : lane_sum_before<kBlock>(tile_sums, tile);
+        const int sum_before = lane_sum_before<kBlock>(tile_sums, tile);
         if (wave == 0 && part == 0) {
             seed_checks_and_next_hop<TS>(i < n, tile, row, deg, d_status, next_fanout, next_tile_seeds, next_tile_sums);
         } else if (row < 0) {
@@ -447,8 +446,7 @@ __global__ __launch_bounds__(kBlock) void sample_insert_kernel(const int32_t* __
             }
         }
         // (barriers: the draws are in place behind them)
-        const int base = tile_base<kBlock>(sum_before, tile_prefix, tile, n_tiles, n, total, s_scan, block_ptr, n_edges_out, nullptr, d_status);
-        if (tile_prefix) __syncthreads();
+        const int base = tile_base<kBlock>(sum_before, nullptr, tile, n_tiles, n, total, s_scan, block_ptr, n_edges_out, nullptr, d_status);
         if (wave == 1 && part == 0 && i < n) block_ptr[i] = base + ex_tile;
         // Floyd: for j = deg-k .. deg-1 draw t in [0, j]; take t unless already taken, else j.  (deg <= fanout: the whole row, in
         // CSR order)
@@ -577,10 +575,11 @@ static int launch_edges_ts(const int32_t* d_indices, const int32_t* d_seeds, int
     const int next_ts = next ? next->tile_seeds : TS;
     int32_t* next_sums = next ? next->tile_sums : nullptr;
     if (insert != nullptr) {
-        FGL_REQUIRE(TS == kInsertTile && d_dst_out == nullptr && d_readback == nullptr && fanout <= 32, "sample_edges: this form does not insert");
+        FGL_REQUIRE(TS == kInsertTile && d_dst_out == nullptr && d_readback == nullptr && fanout <= 32 && prefix == nullptr,
+                    "sample_edges: this form does not insert");
 #define FGL_LAUNCH_INSERT(F)                                                                                                  \
     hipLaunchKernelGGL((sample_insert_kernel<F>), dim3(grid), dim3(kBlock), 0, stream, d_indices, d_seeds,                \
-                       n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, prefix, (uint32_t)rng_seed,                   \
+                       n_seeds_max, d_n_seeds, fanout, row_start, deg, sums, (uint32_t)rng_seed,                           \
                        (uint32_t)(rng_seed >> 32), stream_id, d_stream_add, d_src_out, d_block_ptr, d_n_edges_out, d_status,  \
                        next_fanout, next_ts, next_sums, steps, *insert)
         if (fanout <= 8) FGL_LAUNCH_INSERT(8);

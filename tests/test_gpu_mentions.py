@@ -34,15 +34,19 @@ def test_numbering_at_the_edges_of_lines_and_tiles(cuda, oracle, n_edges, order)
     assert np.array_equal(got[2].cpu().numpy(), w_uniq)
 
 
-# hops of up to 65536 seeds insert while they sample (64 seeds a workgroup), larger ones and fanouts beyond 32 do not
-@pytest.mark.parametrize("n_seeds,fanouts", [(1, [3, 2]), (64, [8, 9]), (65, [16, 17]), (63, [32, 1]), (640, [33, 5]), (65_536, [4]), (65_537, [4]),
-                                             (100, [6, 6, 6, 6])])
+# hops of up to 262144 seeds (in the plan's bounds) and fanout 32 insert while they sample, 16 seeds a workgroup and 64 to an entry of the tile
+# sums; fanouts beyond 32 do not, with 64 seeds a tile, nor do larger hops, with 256 (64 beyond fanout 48).  120000 seeds: the second hop's tiles are
+# others than the first's
+@pytest.mark.parametrize("n_seeds,fanouts", [(1, [3, 2]), (15, [5, 8]), (16, [9, 8]), (17, [9, 8]), (64, [8, 9]), (65, [16, 17]), (63, [32, 1]), (640, [33, 5]),
+                                             (65_536, [4]), (65_537, [4]), (262_144, [4]), (262_145, [4]), (120_000, [2, 4]), (120_000, [33, 4]),
+                                             (120_000, [49, 4]), (100, [6, 6, 6, 6])])
 @pytest.mark.parametrize("transposed", ["none", "inner", "all"])
 def test_hops_on_both_sides_of_the_line(cuda, oracle, n_seeds, fanouts, transposed):
     import fastgl
     print("hops %d %s %s" % (n_seeds, fanouts, transposed), flush=True)
-    indptr, indices = oracle.rmat_csr(70_000, 700_000, seed=3)
-    seeds = np.random.default_rng(n_seeds).permutation(70_000)[:n_seeds].astype(np.int32)
+    n_nodes = 70_000 if n_seeds <= 65_537 else 300_000
+    indptr, indices = oracle.rmat_csr(n_nodes, 10 * n_nodes, seed=3)
+    seeds = np.random.default_rng(n_seeds).permutation(n_nodes)[:n_seeds].astype(np.int32)
     sampler = fastgl.FusedMapSampler(fanouts, rng_seed=5, deterministic=True, transposed=transposed).set_graph(
         torch.from_numpy(indptr).to(cuda), torch.from_numpy(indices).to(cuda))
     for it in range(3):
