@@ -627,8 +627,8 @@ __global__ __launch_bounds__(kBlock) void aggregate_split_kernel(const AggArgs g
 // consecutive rows: their offsets are one read, their entries are consecutive in `indices` and are read
 // (with their weights and the row each belongs to) in one coalesced chunk, and the data rows of all of
 // them are in flight together, four at a time; the running sum is stored and cleared whenever an entry is
-// the last of its row.  A bundle that holds a hub (more than 128 entries in all) falls back to one row
-// after the other.  Sums are in CSR order, as in aggregate_kernel.
+// the last of its row.  A bundle that holds a hub (more than 128 entries in all, or a row that is left to
+// the long rows' launch) falls back to one row after the other.  Sums are in CSR order, as in aggregate_kernel.
 #ifndef FGL_BUNDLE_ROWS
 #define FGL_BUNDLE_ROWS 4
 #endif

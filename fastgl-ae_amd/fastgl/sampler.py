@@ -220,12 +220,12 @@ class FusedMapSampler:
             raise ValueError("id_order must be 'first' or 'arrival'")
         self.id_order = id_order  # numbering of new node ids (fused path): see ops.sample_blocks_fused
         # deterministic=True also fixes the order inside each block's transposed lists, so that the
-        # fp32 sums of the backward pass are reproducible bit for bit (one more launch per mini-batch for the transposed
+        # fp32 sums of the backward pass are reproducible bit for bit (two or three more launches per mini-batch for the transposed
         # blocks that the sampling call builds, a stable sort for those built on demand)
         self.deterministic = bool(deterministic)
         if self.deterministic and id_order != "first":
             raise ValueError("deterministic=True needs id_order='first'")
-        # graph_slots = R > 0: the fused path's launch sequence (8 kernels for three hops) is captured once in a
+        # graph_slots = R > 0: the fused path's launch sequence (8 kernels for three small hops, one more for each hop of more than 262144 seeds or fanout 32) is captured once in a
         # HIP graph per output slot and replayed, which takes the host's launch cost out of the small hops.  It
         # pays off where the GPU would otherwise wait for the host -- one mini-batch at a time from an idle GPU:
         # -11 % at batch 8192, -26 % at batch 1024 -- and not in a loop that keeps the GPU busy, where the launches
@@ -236,7 +236,7 @@ class FusedMapSampler:
         # transposed: which blocks come with their transposed form (what the backward pass of a layer gathers over),
         # built inside the fused sampling call at next to no cost: "inner" = every block but the outermost (the first
         # layer's input needs no gradient), "all", or "none" (built on demand, Block.transposed()).  A deterministic
-        # sampler has the call sort their rows as well (one more launch); blocks whose transposed form is built on
+        # sampler has the call sort their rows as well (two or three more launches); blocks whose transposed form is built on
         # demand get theirs from a stable sort.
         if transposed not in ("inner", "all", "none"):
             raise ValueError("transposed must be 'inner', 'all' or 'none'")
