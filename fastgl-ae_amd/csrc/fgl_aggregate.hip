@@ -148,7 +148,8 @@ struct AggArgs {
     void* ws;                   // scratch of aggregate_workspace_bytes(n_entries_max, D) bytes: long rows go in segments (NULL: row by row)
     int64_t n_entries_max;      // (with ws) no fewer entries than the rows hold
     const int32_t* order;       // aggregate_kernel<.., ORDERED>: lane group i takes row order[i] ...
-    const int32_t* in_order;    // ... in the tiles of kSegTile rows that are marked here
+    const int32_t* in_order;    // ... in the tiles of 2^tile_log rows that are marked here
+    int tile_log;
 };
 
 // per-edge weight, evaluated by the lane that loaded the neighbour id
@@ -401,7 +402,11 @@ constexpr int kLongRowEntries = 128;
 // takes a workgroup for each -- 70 K rows of 446 K entries 46 / 61 / 144 / 66 -> 64 / 94 / 196 / 111.)
 constexpr int kBundleLongEntries = 48;
 
-constexpr int kSegBlock = 1024, kSegRows = 8, kSegTile = kSegBlock * kSegRows;  // rows that seg_lists_kernel looks at, a workgroup
+// Rows that seg_lists_kernel looks at: a workgroup takes kSegBlock of them eight times, or, below half a million rows, where that would be a few dozen workgroups,
+// each a chain of as many steps, twice.  (The launch, 312 K rows of a transposed block, 15 -> 9 us; the gather with it, 128 fp32 columns 134 -> 127, 128 bf16 columns
+// 84 -> 78, R-MAT 150 K rows of 64 fp32 columns 90 -> 83, but 1 M rows of it 285 -> 302: tiles of 2048 rows sort less well.)
+constexpr int kSegBlock = 1024, kSegRows = 8, kSegFewRows = 2;
+static inline int seg_tile(int64_t n_rows_max) { return kSegBlock * (n_rows_max >= ((int64_t)1 << 19) ? kSegRows : kSegFewRows); }
 
 // Workgroup -> place among the n of a launch that takes rows in sequence.  Workgroups go to the eight XCDs in turn, so row numbers with the same
 // few low bits are one XCD's work; where those bits say how long rows are -- R-MAT graphs: 0.76 of the entries for every bit that is zero -- one
@@ -432,7 +437,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_kernel(const AggArgs g)
     if (row >= n_rows) return;  // uniform per group: the cross-lane reads below stay inside the group
     int a = indptr[row], b = indptr[row + 1];
     if constexpr (ORDERED) {
-        if (g.in_order[row0 / kSegTile]) {  // (a workgroup's rows are one tile's; in a tile that keeps its order nothing waits for the mark)
+        if (g.in_order[row0 >> g.tile_log]) {  // (a workgroup's rows are one tile's; in a tile that keeps its order nothing waits for the mark)
             row = g.order[row];
             a = indptr[row];
             b = indptr[row + 1];
@@ -1172,18 +1177,18 @@ __global__ void seg_init_kernel(int32_t* __restrict__ counts)
 // (us, 64 fp32 columns, the rows as they come / all tiles in order, listed by a launch of their own / this way: 300 K rows, R-MAT 151 / 94 / 93 -- the turned
 // workgroups above are half of that -- log-normal 114 / 128 / 117, all of 8 entries 110 / 120 / 110; 140 K rows of 8 entries, 64 bf16 columns 33 / 45 / 35.)
 // PER_WAVE rows to a wave; every lane has the entries of rows row0 + i * kSegBlock, -1: no such row.
-template <int PER_WAVE>
-__device__ __forceinline__ void order_rows(const int (&entries)[kSegRows], int64_t row0, int limit, int* s_scan, int* s_bin, int32_t* __restrict__ order,
+template <int PER_WAVE, int ROWS>
+__device__ __forceinline__ void order_rows(const int (&entries)[ROWS], int64_t row0, int limit, int* s_scan, int* s_bin, int32_t* __restrict__ order,
                                            int32_t* __restrict__ in_order)
 {
     constexpr int kInFlight = PER_WAVE == 8 ? 8 : 16;
     constexpr int kLine = PER_WAVE == 8 ? 15 : PER_WAVE == 4 ? 10 : 8;  // sixths
     constexpr int kBins = 256;  // lengths 0 .. 254, and all above (which the gather leaves out or are its last)
     const int tid = (int)threadIdx.x, lane = lane_id();
-    // (a quarter of the tile's rows stands for it; both sums in one word: 2048 rows of at most 16 accesses each)
+    // (two of a lane's rows stand for the tile; both sums in one word: 2048 rows of at most 16 accesses each)
     uint32_t both = 0;
 #pragma unroll
-    for (int i = 0; i < kSegRows; i += kSegRows / 2) {
+    for (int i = 0; i < ROWS; i += ROWS / 2) {
         int n = entries[i] > 0 && entries[i] <= limit ? 1 + (entries[i] - 1) / kInFlight : 0;
         if (n > 16) n = 16;
         both += (uint32_t)n;
@@ -1201,9 +1206,9 @@ __device__ __forceinline__ void order_rows(const int (&entries)[kSegRows], int64
     if (!unlike) return;
     if (tid < kBins) s_bin[tid] = 0;
     __syncthreads();
-    int key[kSegRows], place[kSegRows];
+    int key[ROWS], place[ROWS];
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
         key[i] = entries[i] < 0 ? -1 : kBins - 1 - (entries[i] < kBins - 1 ? entries[i] : kBins - 1);  // (longest first)
         // (empty rows, a third of them and more: one update per wave)
         const bool empty = key[i] == kBins - 1;
@@ -1223,14 +1228,14 @@ __device__ __forceinline__ void order_rows(const int (&entries)[kSegRows], int64
     __syncthreads();
     const int64_t tile0 = row0 - tid;
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i)
+    for (int i = 0; i < ROWS; ++i)
         if (key[i] >= 0) order[tile0 + s_bin[key[i]] + place[i]] = (int32_t)(row0 + (int64_t)i * kSegBlock);
 }
 
 // The lists.  Their order is up to scheduling, the sums are not: a row's segments are cut and added the same way on every run.
-// A workgroup looks through kSegRows rows per lane and takes its places in the lists with three atomics (one address each:
+// A workgroup looks through ROWS rows per lane and takes its places in the lists with three atomics (one address each:
 // their updates run one after the other, so there are few of them).  PER_WAVE: the gather's order of the rows as well (0: no order).
-template <int PER_WAVE>
+template <int PER_WAVE, int ROWS>
 __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, const SegLists l, int32_t* __restrict__ order,
                                                               int32_t* __restrict__ in_order)
 {
@@ -1241,10 +1246,10 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
     if (none_left_out && PER_WAVE == 0) return;
     if (none_left_out) threshold = 0x7FFFFFFF;
     const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
-    const int64_t row0 = (int64_t)blockIdx.x * kSegTile + threadIdx.x;
-    int first[kSegRows], entries[kSegRows];
+    const int64_t row0 = (int64_t)blockIdx.x * (kSegBlock * ROWS) + threadIdx.x;
+    int first[ROWS], entries[ROWS];
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
         const int64_t row = row0 + (int64_t)i * kSegBlock;
         first[i] = row < n_rows ? g.indptr[row] : 0;
         entries[i] = row < n_rows ? g.indptr[row + 1] - first[i] : -1;
@@ -1252,18 +1257,18 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
     }
     if constexpr (PER_WAVE > 0) {
         __shared__ int s_bin[256];
-        order_rows<PER_WAVE>(entries, row0, threshold, s_scan, s_bin, order, in_order);
+        order_rows<PER_WAVE, ROWS>(entries, row0, threshold, s_scan, s_bin, order, in_order);
         if (none_left_out) return;
     }
     int segs = 0, ones = 0, many = 0;
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
         const int64_t row = row0 + (int64_t)i * kSegBlock;
         first[i] = row < n_rows ? g.indptr[row] : 0;
         entries[i] = row < n_rows ? g.indptr[row + 1] - first[i] : 0;
     }
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
         if (entries[i] <= threshold) continue;
         if (entries[i] <= kSegEntries) {
             ++ones;
@@ -1286,7 +1291,7 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
     at_one += s_base[1];
     at_many += s_base[2];
 #pragma unroll
-    for (int i = 0; i < kSegRows; ++i) {
+    for (int i = 0; i < ROWS; ++i) {
         if (entries[i] <= threshold) continue;
         const int row = (int)(row0 + (int64_t)i * kSegBlock);
         if (entries[i] <= kSegEntries) {
@@ -1579,8 +1584,12 @@ template <int PER_WAVE>
 static void launch_seg_lists(const SegLists& l, hipStream_t stream, const AggArgs& g, int32_t* order, int32_t* in_order)
 {
     hipLaunchKernelGGL(seg_init_kernel, dim3(1), dim3(kWave), 0, stream, l.counts);
-    hipLaunchKernelGGL(seg_lists_kernel<PER_WAVE>, dim3((unsigned)ceil_div(g.n_rows_max, kSegTile)), dim3(kSegBlock), 0, stream, g, l, order,
-                       in_order);
+    const int tile = seg_tile(g.n_rows_max);
+    const dim3 grid((unsigned)ceil_div(g.n_rows_max, tile));
+    if (tile == kSegBlock * kSegRows)
+        hipLaunchKernelGGL((seg_lists_kernel<PER_WAVE, kSegRows>), grid, dim3(kSegBlock), 0, stream, g, l, order, in_order);
+    else
+        hipLaunchKernelGGL((seg_lists_kernel<PER_WAVE, kSegFewRows>), grid, dim3(kSegBlock), 0, stream, g, l, order, in_order);
 }
 
 // The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
@@ -1632,11 +1641,13 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
         if (second_pass && g.ws != nullptr && mode != FGL_AGG_EDGE && g.n_rows_max >= kOrderMinRows) {
             // (in the place of the partial sums, which the launches behind the gather fill; the launch that lists the long rows finds the order)
             const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
-            if ((int64_t)l.cap_seg * l.ldp >= g.n_rows_max + ceil_div(g.n_rows_max, kSegTile)) {
+            const int tile = seg_tile(g.n_rows_max);
+            if ((int64_t)l.cap_seg * l.ldp >= g.n_rows_max + ceil_div(g.n_rows_max, tile)) {
                 int32_t* order = reinterpret_cast<int32_t*>(l.partial);
                 launch_seg_lists<kWave / LPR>(l, stream, g, order, order + g.n_rows_max);
                 g.order = order;
                 g.in_order = order + g.n_rows_max;
+                g.tile_log = __builtin_ctz((unsigned)tile);
                 ordered = true;
             }
         }
@@ -1917,6 +1928,7 @@ FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indice
     g.n_entries_max = n_entries_max;
     g.order = nullptr;
     g.in_order = nullptr;
+    g.tile_log = 0;
     hipStream_t s = as_stream(stream);
     if (dtype == FGL_F32) return launch_agg_vec<float, 4>(mode, longest_row_max, n_entries_max, s, g);
     if (bf16_rows_dword_aligned(ldx, ldo, d_x, d_out)) return launch_agg_vec<uint16_t, 8>(mode, longest_row_max, n_entries_max, s, g);

@@ -1,5 +1,5 @@
-"""Blocks whose tiles of 8192 rows are partly alike (taken as they come) and partly not (taken in order of length), with two, four and eight rows
-to a wave: rows of up to 128 entries against the same rows in one launch, bit for bit, the longer ones against float64 sums."""
+"""Blocks whose tiles (of 8192 rows from 524288 rows on, 2048 below) are partly alike (taken as they come) and partly not (taken in order of
+length), with two, four and eight rows to a wave: rows of up to 128 entries against the same rows in one launch, bit for bit, the longer ones against float64 sums."""
 import pytest
 import torch
 
@@ -25,11 +25,11 @@ def _lens(kinds, tail, gen):
 
 
 @pytest.mark.parametrize("dim,dtype", [(128, torch.float32), (64, torch.float32), (40, torch.bfloat16), (200, torch.bfloat16), (33, torch.float32)])
-@pytest.mark.parametrize("tail", [0, 1, TILE - 1])
-def test_tiles_in_order_and_as_they_come(cuda, dim, dtype, tail):
-    print("row tiles", dim, dtype, tail, flush=True)
+@pytest.mark.parametrize("tail,times", [(0, 3), (1, 3), (2047, 3), (TILE - 1, 3), (1, 11)])
+def test_tiles_in_order_and_as_they_come(cuda, dim, dtype, tail, times):
+    print("row tiles", dim, dtype, tail, times, flush=True)
     gen = torch.Generator().manual_seed(dim + tail)
-    lens = _lens(["alike", "skewed", "empty", "skewed", "alike", "alike"] * 3 + ["skewed"], tail, gen)
+    lens = _lens(["alike", "skewed", "empty", "skewed", "alike", "alike"] * times + ["skewed"], tail, gen)
     n, n_cols = lens.numel(), 60_000
     ptr = torch.zeros(n + 1, dtype=torch.int64)
     ptr[1:] = torch.cumsum(lens, 0)
@@ -44,7 +44,7 @@ def test_tiles_in_order_and_as_they_come(cuda, dim, dtype, tail):
         out = torch.full((n, dim), 7.0, dtype=dtype, device=cuda)
         ops.aggregate(d_ptr, d_idx, d_x, mode="sum", zero_policy="zeros", n_rows=n, out=out, **kw)
         assert torch.equal(out[short], plain[short])
-        for r in torch.nonzero(lens > 128).flatten()[::7].tolist():
+        for r in torch.nonzero(lens > 128).flatten()[::7 * times].tolist():
             rows = x[idx[ptr[r]:ptr[r + 1]].long()].double()
             # (sums of up to 700 entries in two levels: far below n 2^-24 of the sum of magnitudes; bf16 results are rounded once more)
             bound = int(lens[r]) * 2.0 ** -24 * rows.abs().sum(0) + (rows.sum(0).abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
