@@ -434,7 +434,7 @@ class MA_Function_Mean(torch.autograd.Function):
 class _SageFunction(torch.autograd.Function):
     """A ``SAGEConv`` layer as a whole: the two products and their sum are one pass over the output, and in the backward pass the
     gradient of a node's own row is added to its row of the gathered gradient, where autograd would write it into a cleared array of all
-    source rows and add that.  (GraphSAGE in bf16, 87 K and 41 K rows of 256 columns: 20 of a training step's 57 launches.)
+    source rows and add that.  (GraphSAGE in bf16, 87 K and 41 K rows of 256 columns: 12 of a training step's 61 launches.)
     ``feat_dst`` is ``None`` where the destination rows are the first rows of ``feat_src``; otherwise ``feat_src`` gets no gradient (it is
     the whole table, or wants none)."""
 

@@ -228,7 +228,7 @@ class FusedMapSampler:
         # graph_slots = R > 0: the fused path's launch sequence (8 kernels for three small hops, one more for each hop of more than 262144 seeds or fanout 32) is captured once in a
         # HIP graph per output slot and replayed, which takes the host's launch cost out of the small hops.  It
         # pays off where the GPU would otherwise wait for the host -- one mini-batch at a time from an idle GPU:
-        # -11 % at batch 8192, -26 % at batch 1024 -- and not in a loop that keeps the GPU busy, where the launches
+        # -10 % at batch 8192, -15 % at batch 1024 -- and not in a loop that keeps the GPU busy, where the launches
         # are hidden behind the previous step's kernels anyway.  The price: outputs live in R fixed slots used in
         # turn, so the tensors of a mini-batch are overwritten when the R-th mini-batch after it is sampled (with
         # iter_batches: the R-th after it on the same lane, i.e. R * prefetch mini-batches later) -- consume (or
