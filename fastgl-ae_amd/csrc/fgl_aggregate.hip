@@ -150,6 +150,7 @@ struct AggArgs {
     const int32_t* order;       // aggregate_kernel<.., ORDERED>: lane group i takes row order[i] ...
     const int32_t* in_order;    // ... in the tiles of 2^tile_log rows that are marked here
     int tile_log;
+    int turn;                   // the workgroups of aggregate_kernel take their rows as turned_block deals them out
 };
 
 // per-edge weight, evaluated by the lane that loaded the neighbour id
@@ -411,7 +412,9 @@ static inline int seg_tile(int64_t n_rows_max) { return kSegBlock * (n_rows_max 
 // Workgroup -> place among the n of a launch that takes rows in sequence.  Workgroups go to the eight XCDs in turn, so row numbers with the same
 // few low bits are one XCD's work; where those bits say how long rows are -- R-MAT graphs: 0.76 of the entries for every bit that is zero -- one
 // XCD had almost half of all, and the others waited for it.  Every eight neighbouring workgroups are turned by as many places as a hash of
-// their number says.  (1 M R-MAT rows, us, as they come -> turned: 64 / 128 fp32 columns, 4 M draws 547 / 955 -> 368 / 658, 15 M 1196 / 2264 -> 1001 /
+// their number says, where long rows are possible: where the caller rules them out -- a sampled block, whose rows are numbered as they are met -- rows are dealt
+// out evenly as they come (the outermost block of a batch on 111 M nodes, 110 K rows of 13.5 entries, 128 fp32 columns, four batches, us: 162.8 / 159.7 / 162.5 /
+// 156.9 as they come, 165.5 / 159.6 / 162.0 / 159.3 turned).  (1 M R-MAT rows, us, as they come -> turned: 64 / 128 fp32 columns, 4 M draws 547 / 955 -> 368 / 658, 15 M 1196 / 2264 -> 1001 /
 // 1947; 64 / 128 bf16 columns 351 / 581 -> 233 / 385.  Rows of even lengths, or of uneven ones anywhere, are the same within the runs' 1 %.)
 __device__ __forceinline__ unsigned turned_block(unsigned b, unsigned n)
 {
@@ -432,7 +435,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_kernel(const AggArgs g)
 
     const int64_t n_rows = actual_count(g.n_rows_max, g.d_n_rows);
     const int gl = (int)threadIdx.x % LPR;  // lane within the group
-    const int64_t row0 = (int64_t)turned_block(blockIdx.x, gridDim.x) * kGroups;
+    const int64_t row0 = (int64_t)(g.turn ? turned_block(blockIdx.x, gridDim.x) : blockIdx.x) * kGroups;
     int64_t row = row0 + (int)threadIdx.x / LPR;
     if (row >= n_rows) return;  // uniform per group: the cross-lane reads below stay inside the group
     int a = indptr[row], b = indptr[row + 1];
@@ -1636,6 +1639,7 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
       }
     }
     note_mapping("aggregate_kernel", LPR, 1, second_pass, g.ws != nullptr);
+    g.turn = second_pass;
     bool ordered = false;
     if constexpr (LPR <= 32) {
         if (second_pass && g.ws != nullptr && mode != FGL_AGG_EDGE && g.n_rows_max >= kOrderMinRows) {
@@ -1929,6 +1933,7 @@ FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indice
     g.order = nullptr;
     g.in_order = nullptr;
     g.tile_log = 0;
+    g.turn = 0;
     hipStream_t s = as_stream(stream);
     if (dtype == FGL_F32) return launch_agg_vec<float, 4>(mode, longest_row_max, n_entries_max, s, g);
     if (bf16_rows_dword_aligned(ldx, ldo, d_x, d_out)) return launch_agg_vec<uint16_t, 8>(mode, longest_row_max, n_entries_max, s, g);
