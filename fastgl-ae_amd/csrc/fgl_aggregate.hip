@@ -402,6 +402,7 @@ constexpr int kLongRowEntries = 128;
 // 27 / 27 / 39 / 30.  64 instead of 48 leaves the last as it was.  Denser blocks keep 128: they have many such lists, and that launch
 // takes a workgroup for each -- 70 K rows of 446 K entries 46 / 61 / 144 / 66 -> 64 / 94 / 196 / 111.)
 constexpr int kBundleLongEntries = 48;
+constexpr int kBundleKnownEntries = 72;  // wide rows: a longest row of up to this many known on the host is no reason for that launch
 
 // Rows that seg_lists_kernel looks at: a workgroup takes kSegBlock of them eight times, or, below half a million rows, where that would be a few dozen workgroups,
 // each a chain of as many steps, twice.  (The launch, 312 K rows of a transposed block, 15 -> 9 us; the gather with it, 128 fp32 columns 134 -> 127, 128 bf16 columns
@@ -1680,8 +1681,12 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
 template <typename T, int VEC>
 static int launch_agg_flat(int mode, int64_t longest_row_max, int lanes, bool bundle, hipStream_t stream, AggArgs g)
 {
+    // (a longest row of 49 .. 72 entries known on the host: no second launch, which costs more than walking that row does.  300 fp32 columns, us, without / with:
+    // 20 K rows, longest 49 / 64 / 80 / 101 20.6 / 22.6, 25.2 / 23.2, 29.8 / 24.2, 35.8 / 24.2; 87 K rows, longest 56 / 64 / 72 / 80 50.0 / 60.5, 53.7 / 56.1, 56.8 / 56.3,
+    // 59.1 / 55.7)
     const int limit = long_row_limit(bundle, g);
-    const bool long_rows_possible = longest_row_max < 0 || longest_row_max > limit;
+    const int known = bundle && limit < kBundleKnownEntries ? kBundleKnownEntries : limit;
+    const bool long_rows_possible = longest_row_max < 0 || longest_row_max > known;
     g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;
     note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible, g.ws != nullptr);
     const int64_t blocks = ceil_div((bundle ? ceil_div(g.n_rows_max, kBundleRows) : g.n_rows_max) * lanes, kBlock);
@@ -1745,7 +1750,7 @@ template <typename T, int VEC, int LPR>
 static int launch_agg_bundle(int mode, int64_t longest_row_max, unsigned gy, hipStream_t stream, AggArgs g)
 {
     // (a longest row of 49 .. 128 entries known on the host: no second launch, whose 8 us are more than that row takes -- 12 K rows, longest
-    // 101, 256 columns 19 us without and 27 with; the wide rows of launch_agg_flat gain all the same, 54 -> 42)
+    // 101, 256 columns 19 us without and 27 with; the wide rows of launch_agg_flat gain from 72 entries on)
     const bool long_rows_possible = longest_row_max < 0 || longest_row_max > kLongRowEntries;
     const int limit = long_row_limit(true, g);
     g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;

@@ -43,3 +43,24 @@ def test_lists_at_the_limit(cuda, mode, dim, dtype):
         got = ops.aggregate(ptr.int().to(cuda), idx.to(cuda), x.to(cuda), mode=mode, zero_policy="zeros", n_rows=n_rows, longest_row=longest, **kw)
         assert b"bundled" in L.lib().fgl_aggregate_last_mapping() and b"long_rows" in L.lib().fgl_aggregate_last_mapping()
         assert bool(((got.cpu().double() - want).abs() <= eps).all())
+
+
+@pytest.mark.parametrize("dim,dtype", [(300, torch.float32), (600, torch.bfloat16)])
+@pytest.mark.parametrize("longest,second", [(49, False), (72, False), (73, True), (129, True)])
+def test_wide_rows_with_a_longest_row_known_to_the_host(cuda, dim, dtype, longest, second):
+    print("known longest", dim, dtype, longest, flush=True)
+    gen = torch.Generator().manual_seed(longest)
+    n_rows, n_cols = 16_385, 3000
+    lens = torch.randint(0, 3, (n_rows,), generator=gen)
+    lens[5::3001] = longest
+    lens[-1] = longest
+    ptr = torch.zeros(n_rows + 1, dtype=torch.int64)
+    ptr[1:] = torch.cumsum(lens, 0)
+    idx = torch.randint(0, n_cols, (int(ptr[-1]),), generator=gen, dtype=torch.int32)
+    x = torch.randn((n_cols, dim), generator=gen).to(dtype)
+    rows = torch.repeat_interleave(torch.arange(n_rows), lens)
+    want, size = (torch.zeros((n_rows, dim), dtype=torch.float64).index_add_(0, rows, v) for v in (x[idx.long()].double(), x[idx.long()].double().abs()))
+    got = ops.aggregate(ptr.int().to(cuda), idx.to(cuda), x.to(cuda), mode="sum", zero_policy="zeros", n_rows=n_rows, longest_row=longest)
+    assert (b"long_rows" in L.lib().fgl_aggregate_last_mapping()) == second
+    eps = 2.0 ** -24 * 73 * size + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)  # (72 additions in a chain at most)
+    assert bool(((got.cpu().double() - want).abs() <= eps).all())
