@@ -7,7 +7,8 @@
 // 890..940, GraphSAGE in bf16 1430..1630 -> 1110..1140 (three runs; the autograd thread makes two of them uneven).  Where such products
 // gain is ops._forms_row_product's rule.
 //
-// What bounds it: in fp32 the matrix cores, in bf16 the one pass over A and C.
+// What bounds it: in fp32 the matrix cores, in bf16 the one pass over A and C.  Large fp32 products go to fgl_split_product.hip, which forms them on the bf16
+// matrix cores; the line is split_product_pays.
 //
 // Tile: a wave holds (32 VA) x (32 VB) outputs in its accumulators.  Nothing goes through LDS: the order of the k within a step
 // is free, so lane i of a half-wave reads its own row of A with one 16-byte load along k (half 0 the step's first values, half 1 the rest) and
@@ -26,6 +27,7 @@
 // (bit-equal copies of its neighbour's); k past the end is zero in both operands.  No access leaves the operands.
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
+#include "fgl_row_product.hpp"
 
 namespace fgl {
 
@@ -104,22 +106,6 @@ struct RpCols<uint16_t, VB> {
     __device__ __forceinline__ Bf16x8 operand(int c) const { return bf16_column(r, c); }
 };
 
-struct RowProductSide {
-    const void* a;
-    const void* b;
-    int64_t lda, ldb;
-    int k;  // 0: no such pair
-};
-struct RowProductArgs {
-    RowProductSide side[2];  // C = A0 B0 + A1 B1
-    const void* bias;
-    void* c;
-    int64_t ldc, m;
-    int n;
-    int tiles_n;          // tiles of C along n
-    int64_t row_blocks;   // workgroups along m
-};
-
 template <typename T, int VA, int VB, bool BT>
 struct RpStep {
     static constexpr int kLane = RpRow<T>::kLane;
@@ -183,47 +169,6 @@ struct RpStep {
     }
 };
 
-__device__ __forceinline__ uint32_t rp_bf16_bits(float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v); }
-
-// v += what p holds
-template <typename T, int VB>
-__device__ __forceinline__ void rp_add(const T* p, float (&v)[VB])
-{
-    if constexpr (sizeof(T) == 4) {
-        typedef float Vec __attribute__((ext_vector_type(VB), aligned(4)));
-        const Vec o = *reinterpret_cast<const Vec*>(p);
-#pragma unroll
-        for (int t = 0; t < VB; ++t) v[t] += o[t];
-    } else if constexpr (VB == 1) {
-        v[0] += __uint_as_float((uint32_t)*p << 16);
-    } else {
-        typedef uint32_t Vec __attribute__((ext_vector_type(VB / 2), aligned(4)));
-        const Vec o = *reinterpret_cast<const Vec*>(p);
-#pragma unroll
-        for (int t = 0; t < VB; ++t) v[t] += __uint_as_float(t & 1 ? o[t / 2] & 0xFFFF0000u : o[t / 2] << 16);
-    }
-}
-
-template <typename T, int VB>
-__device__ __forceinline__ void rp_store(T* p, const float (&v)[VB])
-{
-    if constexpr (sizeof(T) == 4) {
-        typedef float Vec __attribute__((ext_vector_type(VB), aligned(4)));
-        Vec o;
-#pragma unroll
-        for (int t = 0; t < VB; ++t) o[t] = v[t];
-        *reinterpret_cast<Vec*>(p) = o;
-    } else if constexpr (VB == 1) {
-        *reinterpret_cast<__bf16*>(p) = (__bf16)v[0];
-    } else {
-        typedef __bf16 Vec __attribute__((ext_vector_type(VB), aligned(4)));
-        Vec o;
-#pragma unroll
-        for (int t = 0; t < VB; ++t) o[t] = (__bf16)v[t];
-        *reinterpret_cast<Vec*>(p) = o;
-    }
-}
-
 // acc += the products of one pair of operands.  row0: the wave's first row; col: the lane's first column.
 template <typename T, int VA, int VB, bool BT>
 __device__ __forceinline__ void rp_side(const RowProductSide& side, int64_t row0, int64_t m, int col, RpF32x16 (&acc)[VA * VB])
@@ -257,11 +202,6 @@ __device__ __forceinline__ void rp_side(const RowProductSide& side, int64_t row0
     cur.multiply(acc);
     next.multiply(acc);
 }
-
-// FORM: one product (kRpOne), two of them and their sum (kRpSum: a layer's own rows with one weight and its gathered rows with another, in one
-// pass over C where the products and their sum were five), or a product added to what C holds (kRpAdd).  In bf16 a product is rounded to
-// bf16 before it is added to another or to C, as it would be if it were stored in between.
-constexpr int kRpOne = 0, kRpSum = 1, kRpAdd = 2;
 
 template <typename T, int VA, int VB, bool BT, int FORM>
 __global__ __launch_bounds__(kBlock, VA * VB >= 4 ? 2 : 4) void row_product_kernel(const RowProductArgs g)
@@ -415,6 +355,7 @@ static int row_product(const RowProductSide& one, const RowProductSide& two, int
     }
     if (m == 0) return FGL_OK;
     hipStream_t s = as_stream(stream);
+    if (dtype == FGL_F32 && split_product_pays(g)) return split_product(g, b_transposed != 0, FORM, s);
     if (dtype == FGL_F32) return b_transposed ? launch_row_product_any<float, true, FORM>(g, true, s) : launch_row_product_any<float, false, FORM>(g, true, s);
     return b_transposed ? launch_row_product_any<uint16_t, true, FORM>(g, vectors, s) : launch_row_product_any<uint16_t, false, FORM>(g, vectors, s);
 }

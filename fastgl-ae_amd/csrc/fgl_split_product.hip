@@ -1,0 +1,449 @@
+// Products over the rows of a block in fp32 (what fgl_row_product.hip forms, which see), on the bf16 matrix cores: C[m, n] = A[m, k] B[k, n].
+//
+// Why: the fp32 matrix instructions reach 157 TFLOP/s, the bf16 ones 2500.  An fp32 value is the sum of three bf16 values, exactly, so a product is six
+// bf16 products and loses only terms below 2^-26 of it: a2 b0, a0 b2, a1 b1, a1 b0, a0 b1, a0 b0 of a = a0 + a1 + a2, b = b0 + b1 + b2, 2.6 times the rate.
+//
+// How exact.  Every product of two parts is exact, and what a matrix instruction adds up is cut to 26 bits of its largest term.  So the 32 k of a chunk are
+// added up from zero, the small products first, and only their sum is added to the accumulators, in fp32: errors of a sum of k terms grow with k / 32 where they
+// grew with k.  Against 64-bit sums, 2-norm, normal / non-negative operands (the fp32 instructions in brackets): k = 100 5.8e-8 / 4.7e-8 (1.8e-7 / 1.4e-7),
+// k = 256 7.0e-8 / 5.1e-8 (2.9e-7 / 2.5e-7), k = 800 1.1e-7 / 7.1e-8 (5.1e-7 / 3.8e-7).  Added to the accumulators directly the errors of k = 602 were
+// those of the fp32 instructions and larger, because the cut then is at the accumulator's 26 bits.
+// Values without such parts: infinite, not a number or rounded to infinity ones make results that are no finite numbers, and bits below 2^-133, bf16's last, matter
+// only to a row of A or a column of B whose largest value is below 2^-85.  A tile with such a result, row or column is formed again in fp32 matrix instructions.
+//
+// What bounds it: for short k and few columns the pass over A and C, beyond that the matrix cores and the vector unit beside them.
+//
+// Split: a workgroup keeps its 32 NT columns of B in LDS, already in parts and in the order in which the lanes take them, and its waves go over the rows of
+// A in tiles of 32, each by itself: no barrier after the first.  A lane reads its row of A straight to registers, a chunk ahead, and splits it; so the
+// splitting costs each wave once for NT tiles, and no row is staged.  B is staged once for as many rows as there are, which is what a row tile a workgroup cannot do (both
+// operands through LDS by tiles of 128 x 128: 107 K x 100 x 256 60 us where this takes 49).
+// Beside each matrix instruction (32 cycles) the vector unit has room for about six others: the splitting of the next step (44 a step) and the addition of the last
+// round's sums (16 a tile) are dealt out between them, which the compiler does not do by itself.  Left to its order, with the same instructions, 107 K x 256 x 256 takes 96 us.
+//
+// Measured (MI355X, us: the fp32 instructions / the library / this; a transposed B costs no more here): 2.4 M x 100 x 64 550 / 512 / 338 (4.7 TB/s),
+// 2.4 M x 64 x 100 450 / 627 / 325 (4.8 TB/s), 107 K x 100 x 256 77 / 80 / 49, 107 K x 256 x 256 142 / 137 / 85, 17 K x 256 x 256 42 / 24 / 18,
+// 200 K x 128 x 128 85 / 80 / 47, 8192 x 602 x 256 29 / 28 / 25, 8192 x 256 x 602 43 / 36 / 29.
+//
+// Rows past the end repeat the last one and are not stored, nor are columns past the end, which repeat the last one too; the last step of k ends with k, and what the step before has
+// of it is zero in LDS.  No access leaves the operands.
+#include "fgl_common.hpp"
+#include "fgl_kernels.hpp"
+#include "fgl_row_product.hpp"
+
+namespace fgl {
+
+typedef float SpF32x16 __attribute__((ext_vector_type(16)));
+typedef float SpF4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t SpU4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSpLds = 158 * 1024;  // of a CU, for B (the rest: the largest of each column)
+
+// Eight fp32 values as three bf16 operands: v = p[0] + p[1] + p[2] to the last bit (while v's last bit is no smaller than bf16's, 2^-133).  (v_dot2 with
+// (-1, 0) and (0, -1) would take a part off in one instruction instead of two, but does not run beside a matrix instruction: one a MFMA takes 34 cycles to 45.)
+__device__ __forceinline__ void sp_split(const float (&v)[8], SpU4 (&p)[3])
+{
+    typedef __bf16 B2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float x = v[2 * j], y = v[2 * j + 1];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            B2 h;
+            h[0] = (__bf16)x;
+            h[1] = (__bf16)y;
+            uint32_t w = __builtin_bit_cast(uint32_t, h);
+            p[s][j] = w;
+            if (s == 2) break;
+            x -= __uint_as_float(w << 16);
+            y -= __uint_as_float(w & 0xFFFF0000u);
+        }
+    }
+}
+
+// m = the largest magnitude of m and eight values (what is not a number is passed over)
+__device__ __forceinline__ void sp_most(const float (&v)[8], float& m)
+{
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(v[j]), "v"(v[j + 1]));
+}
+// Whether a row or a column whose largest magnitude is m may lose bits to bf16's range: its values are off by 2^-134 at most, 2^-49 of anything from here on.
+__device__ __forceinline__ bool sp_small(float m) { return m > 0.0f && m < 0x1p-85f; }
+
+// Eight values of a row of A, from its k number k0 on; only the first n of them exist.
+__device__ __forceinline__ void sp_load(const float* p, float (&v)[8])
+{
+    const SpF4 a = *reinterpret_cast<const SpF4*>(p), b = *reinterpret_cast<const SpF4*>(p + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] = a[j];
+        v[4 + j] = b[j];
+    }
+}
+__device__ __forceinline__ void sp_load_tail(const float* p, int n, float (&v)[8])
+{
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        v[j] = 0.0f;
+        if (j < n) v[j] = p[j];
+    }
+}
+
+// Where step s starts: the last one ends with k (where k has 16 values at all), and B's image in LDS is zero for what the step before had.
+__device__ __forceinline__ int sp_first(int s, int k)
+{
+    const int at = 16 * s;
+    return k >= 16 && at + 16 > k ? k - 16 : at;
+}
+
+
+// The k of one product in steps of 16, two steps to a chunk.  (Where the steps are odd in number the last is one of zeros.)
+__device__ __host__ __forceinline__ int sp_chunks(int k) { return (k + 31) / 32; }
+
+// Column of tile t, lane i (of 32), from the workgroup's first one: a lane's columns are neighbours by fours
+template <int NT>
+__device__ __forceinline__ int sp_column(int t, int i)
+{
+    constexpr int kVec = NT < 4 ? NT : 4;
+    return t / kVec * 32 * kVec + i * kVec + t % kVec;
+}
+
+// The steps of B's columns from col0 on -> img[step * NT + tile][part][lane], and the largest magnitude of each (magnitudes are in order as whole numbers too).  Four eights of k of one column a thread at a time, so that
+// their loads are in flight together.
+template <int NT, bool BT, int THREADS>
+__device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, SpU4* img, float* most)
+{
+    constexpr int kVec = NT < 4 ? NT : 4, kCols = 32 * NT, kBatch = 4;
+    const float* b = static_cast<const float*>(x.b);
+    const int items = steps * 2 * kCols;
+    for (int first = (int)threadIdx.x; first < items; first += THREADS * kBatch) {
+        float v[kBatch][8];
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const int at = first + i * THREADS < items ? first + i * THREADS : items - 1, oct = at / kCols;
+            const int col = col0 + at % kCols < n ? col0 + at % kCols : n - 1;  // (columns past the end repeat the last one)
+            const int own = 16 * (oct / 2) + oct % 2 * 8, k0 = sp_first(oct / 2, x.k) + oct % 2 * 8;
+            const float* p = BT ? b + (int64_t)col * x.ldb + k0 : b + k0 * x.ldb + col;
+            if (k0 == own && k0 + 8 <= x.k) {
+                if constexpr (BT) {
+                    sp_load(p, v[i]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[i][j] = p[j * x.ldb];
+                }
+            } else {  // the last step: what the step before has of it, and what lies past the end, is zero
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    v[i][j] = 0.0f;
+                    if (k0 + j >= own - oct % 2 * 8 && k0 + j < x.k) v[i][j] = BT ? p[j] : p[j * x.ldb];
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+            const int at = first + i * THREADS, oct = at / kCols, col = at % kCols;
+            if (at >= items) break;
+            const int in_group = col % (32 * kVec), t = col / (32 * kVec) * kVec + in_group % kVec;
+            float m = 0.0f;
+            sp_most(v[i], m);
+            atomicMax(reinterpret_cast<int*>(most + col), __float_as_int(m));
+            SpU4 p[3];
+            sp_split(v[i], p);
+            SpU4* to = img + ((oct / 2) * NT + t) * 3 * kWave + oct % 2 * 32 + in_group / kVec;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) to[q * kWave] = p[q];
+        }
+    }
+}
+
+// What a wave multiplies and what it has on the way.  A step of 16 k takes P = NT / 2 rounds of two tiles (one, where NT is 1); a round is six matrix
+// instructions a tile, and the vector unit meanwhile adds the round before's sums to the accumulators and splits the step after's values of A.
+template <int NT>
+struct SpWave {
+    static constexpr int kTiles = NT < 2 ? 1 : 2, kRounds = NT / kTiles;
+    SpF32x16 acc[NT];
+    SpF32x16 sum[2][kTiles];  // of this round and the one before
+    SpU4 b[2][kTiles][3];     // B's values of this round and the next
+    SpU4 a[2][3];             // A's of this step and the next
+    float x[8], y[2][8];      // A's as loaded: the chunk's second step, the next chunk
+    float most, next_most;    // the largest magnitude of the row as far as it is split, and of the next chunk's first step
+
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = SpF32x16{};
+        most = 0.0f;
+    }
+    template <int BUF>
+    __device__ __forceinline__ void read_b(const SpU4* img)
+    {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) b[BUF][t][p] = img[(t * 3 + p) * kWave];
+    }
+    // step U of a chunk; img: its B (of the lane), after: the next step's; r: the next step's values of A
+    template <int U>
+    __device__ __forceinline__ void step(const SpU4* img, const SpU4* after, const float (&r)[8])
+    {
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            constexpr int kPa[6] = {2, 0, 1, 1, 0, 0}, kPb[6] = {0, 2, 1, 0, 1, 0};
+            const int buf = kRounds % 2 ? (U + j) & 1 : j & 1;
+            const SpU4* ahead = j + 1 < kRounds ? img + (j + 1) * kTiles * 3 * kWave : after;
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) b[buf ^ 1][t][p] = ahead[(t * 3 + p) * kWave];
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int t = 0; t < kTiles; ++t)
+                    sum[buf][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(Bf16x8, a[U & 1][kPa[q]]), __builtin_bit_cast(Bf16x8, b[buf][t][kPb[q]]),
+                                                                          q == 0 ? SpF32x16{} : sum[buf][t], 0, 0, 0);
+            const int before = (j + kRounds - 1) % kRounds * kTiles;
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[before + t][i] += sum[buf ^ 1][t][i];
+            if (j == kRounds - 1) {
+                sp_split(r, a[(U + 1) & 1]);
+                sp_most(r, U == 0 ? most : next_most);
+            }
+#pragma unroll
+            for (int i = 0; i < 6 * kTiles; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, kTiles == 1 ? 10 : kRounds == 1 ? 7 : 5, 0);
+                if (i < 3 * kTiles) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // after the last step of a tile, which had ring position U
+    template <int U>
+    __device__ __forceinline__ void flush()
+    {
+        constexpr int kBuf = kRounds % 2 ? (U + kRounds - 1) & 1 : (kRounds - 1) & 1;
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[NT - kTiles + t][i] += sum[kBuf][t][i];
+        sum[kBuf][0] = SpF32x16{};
+        if constexpr (kTiles == 2) sum[kBuf][1] = SpF32x16{};
+    }
+};
+
+// One pair of operands in fp32 matrix instructions
+template <int NT, bool BT>
+__device__ __forceinline__ void sp_plain(const RowProductSide& x, const float* a, int col0, int n, SpF32x16 (&acc)[NT])
+{
+    const int lane = lane_id(), half = lane / 32;
+    const float* b = static_cast<const float*>(x.b);
+    for (int k0 = 0; k0 < x.k; k0 += 2) {
+        const int k = k0 + half;
+        const bool in = k < x.k;
+        const float va = in ? a[k] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int col = col0 + sp_column<NT>(t, lane % 32);
+            float vb = 0.0f;
+            if (in && col < n) vb = BT ? b[(int64_t)col * x.ldb + k] : b[(int64_t)k * x.ldb + col];
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, vb, acc[t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(0.0f, 0.0f, acc[t], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float s = acc[t][i] + 0.0f;
+            asm volatile("" : "+v"(s));
+            acc[t][i] = s;
+        }
+    }
+}
+
+template <int NT, int W, bool BT, int FORM>
+__global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowProductArgs g)
+{
+    constexpr int kVec = NT < 4 ? NT : 4, kThreads = W * kWave;
+    extern __shared__ SpU4 s_img[];
+    __shared__ float s_most[2][32 * NT];
+    const int lane = lane_id(), half = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const unsigned per_group = 8u * (unsigned)g.tiles_n;
+    const int64_t rb = (int64_t)(blockIdx.x / per_group) * 8 + blockIdx.x % per_group % 8;
+    const int col0 = (int)(blockIdx.x % per_group / 8) * 32 * NT;
+    if (rb >= g.row_blocks) return;  // (uniform over the workgroup)
+    const int chunks0 = sp_chunks(g.side[0].k), chunks = chunks0 + (FORM == kRpSum ? sp_chunks(g.side[1].k) : 0);
+    const int64_t row_tiles = (g.m + 31) / 32, stride = g.row_blocks * W;
+    int64_t tile = rb * W + wave;
+
+    // the lane's row of a tile, from its half-wave's first k on
+    auto row_of = [&](const RowProductSide& x, int64_t t) {
+        int64_t row = t * 32 + lane % 32;
+        if (row >= g.m) row = g.m - 1;
+        return static_cast<const float*>(x.a) + row * x.lda + half * 8;
+    };
+    // what is loaded next: chunk `at` of tile `ahead`, whose rows begin at p0 and p1
+    int64_t ahead = tile;
+    int at = 0;
+    const float* p0 = row_of(g.side[0], ahead);
+    const float* p1 = FORM == kRpSum ? row_of(g.side[1], ahead) : nullptr;
+    auto load = [&](float (&r)[2][8]) {
+        const bool second = FORM == kRpSum && at >= chunks0;
+        const float* p = second ? p1 : p0;
+        const int k = second ? g.side[1].k : g.side[0].k, first = 32 * (second ? at - chunks0 : at);
+        if (k >= 16) {
+            sp_load(p + (first < k - 16 ? first : k - 16), r[0]);
+            sp_load(p + (first + 16 < k - 16 ? first + 16 : k - 16), r[1]);
+        } else {
+            sp_load_tail(p, k - half * 8, r[0]);
+            sp_load_tail(p, 0, r[1]);
+        }
+        if (++at == chunks) {
+            at = 0;
+            if (ahead + stride < row_tiles) ahead += stride;
+            p0 = row_of(g.side[0], ahead);
+            if constexpr (FORM == kRpSum) p1 = row_of(g.side[1], ahead);
+        }
+    };
+    SpWave<NT> w;
+    load(w.y);
+    if (threadIdx.x < 64 * NT) (&s_most[0][0])[threadIdx.x] = 0.0f;  // (64 NT <= kThreads)
+    __syncthreads();
+    sp_stage<NT, BT, kThreads>(g.side[0], 2 * chunks0, col0, g.n, s_img, s_most[0]);
+    if constexpr (FORM == kRpSum) sp_stage<NT, BT, kThreads>(g.side[1], 2 * (chunks - chunks0), col0, g.n, s_img + chunks0 * 2 * NT * 3 * kWave, s_most[1]);
+    __syncthreads();
+    if (tile >= row_tiles) return;  // (uniform over the wave; no barrier follows)
+    bool small_column = false;
+    for (int i = lane; i < 64 * NT; i += kWave) small_column |= sp_small((&s_most[0][0])[i]);
+    small_column = __any(small_column);
+    w.clear();
+#pragma unroll
+    for (int t = 0; t < SpWave<NT>::kTiles; ++t) w.sum[1][t] = SpF32x16{};
+    sp_split(w.y[0], w.a[0]);
+    w.next_most = 0.0f;
+    sp_most(w.y[0], w.next_most);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w.x[j] = w.y[1][j];
+    const SpU4* img = s_img + lane;
+    w.template read_b<0>(img);
+    for (;;) {
+        for (int c = 0; c < chunks; ++c) {
+            load(w.y);
+            w.most = w.most < w.next_most ? w.next_most : w.most;
+            w.next_most = 0.0f;
+            const SpU4* after = c + 1 == chunks ? s_img + lane : img + 2 * NT * 3 * kWave;
+            __builtin_amdgcn_sched_barrier(0);
+            w.template step<0>(img, img + NT * 3 * kWave, w.x);
+            w.template step<1>(img + NT * 3 * kWave, after, w.y[0]);
+            img = after;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w.x[j] = w.y[1][j];
+        }
+        w.template flush<1>();
+        SpF32x16 (&acc)[NT] = w.acc;
+        const int64_t row0 = tile * 32;
+        bool odd = small_column || sp_small(fmaxf(w.most, __shfl_xor(w.most, 32, kWave)));
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) odd |= __builtin_amdgcn_classf(acc[t][i], 0x207);  // (infinite or not a number)
+        if (__any(odd)) {
+            w.clear();
+            sp_plain<NT, BT>(g.side[0], row_of(g.side[0], tile) - half * 8, col0, g.n, acc);
+            if constexpr (FORM == kRpSum) sp_plain<NT, BT>(g.side[1], row_of(g.side[1], tile) - half * 8, col0, g.n, acc);
+        }
+        float* out = static_cast<float*>(g.c) + (row0 + 4 * half) * g.ldc + col0;
+        const bool rows = row0 + 32 <= g.m;  // (uniform)
+#pragma unroll
+        for (int q = 0; q < NT / kVec; ++q) {
+            const int at = sp_column<NT>(q * kVec, lane % 32), left = g.n - col0 - at;
+            float add[kVec];
+#pragma unroll
+            for (int t = 0; t < kVec; ++t) {
+                add[t] = 0.0f;
+                if (g.bias != nullptr && t < left) add[t] = static_cast<const float*>(g.bias)[col0 + at + t];
+            }
+            if (rows && left >= kVec) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float* p = out + at + (8 * (r / 4) + r % 4) * g.ldc;
+                    float v[kVec];
+#pragma unroll
+                    for (int t = 0; t < kVec; ++t) v[t] = acc[q * kVec + t][r] + add[t];
+                    if constexpr (FORM == kRpAdd) rp_add<float, kVec>(p, v);
+                    rp_store<float, kVec>(p, v);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float* p = out + at + (8 * (r / 4) + r % 4) * g.ldc;
+                    const bool in = row0 + 8 * (r / 4) + 4 * half + r % 4 < g.m;
+#pragma unroll
+                    for (int t = 0; t < kVec; ++t)
+                        if (in && t < left) p[t] = (acc[q * kVec + t][r] + add[t]) + (FORM == kRpAdd ? p[t] : 0.0f);
+                }
+            }
+        }
+        tile += stride;
+        if (tile >= row_tiles) return;
+        w.clear();
+    }
+}
+
+static size_t sp_lds(const RowProductArgs& g, int nt) { return (size_t)(sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)) * 2 * nt * 3 * kWave * sizeof(SpU4); }
+
+template <int NT, int W, bool BT, int FORM>
+static int launch_split_product(RowProductArgs g, hipStream_t stream)
+{
+    const size_t lds = sp_lds(g, NT);
+    g.tiles_n = (int)ceil_div(g.n, 32 * NT);
+    // eight waves a CU (two a SIMD, as the registers allow), in as many workgroups as their LDS allows
+    int64_t per_cu = kSpLds / (int64_t)lds;
+    if (per_cu > 8 / W) per_cu = 8 / W;
+    const int64_t want = ceil_div(ceil_div(g.m, 32), W), slots = ceil_div(256 * per_cu / g.tiles_n, 8) * 8;
+    g.row_blocks = want < slots ? want : slots;
+    const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
+    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");
+    hipLaunchKernelGGL((split_product_kernel<NT, W, BT, FORM>), dim3((unsigned)blocks), dim3(W * kWave), lds, stream, g);
+    FGL_CHECK_LAUNCH("split_product_kernel");
+    return FGL_OK;
+}
+
+// Columns of a workgroup: 64, so that a split value of A serves two tiles and B fits up to k = 416; 32 for fewer columns or a longer k; 128 where k is short
+// and the pass over A is what counts (2.4 M x 64 x 100: 325 us against 404; 200 K x 128 x 128, with one workgroup of four waves left a CU, 50 against 46).
+static int sp_tiles(const RowProductArgs& g)
+{
+    const int steps = 2 * (sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k));
+    if (g.n > 64 && steps <= 4) return 4;
+    return g.n > 32 && sp_lds(g, 2) <= (size_t)kSpLds ? 2 : 1;
+}
+
+// Whether the split pays.  Below the line the fp32 instructions' kernel is ahead, which has nothing to stage first: us, that one / this, 64 x 64: 32 K rows 7 / 8,
+// 64 K 12 / 10; 100 x 64: 16 K 6 / 8, 32 K 9 / 9; 100 x 256: 4000 6 / 8, 8000 9 / 9, 16 K 15 / 12; 128 x 128: 8000 6 / 8, 16 K 10 / 9; 256 x 256: 4000 9 / 13, 8000 16 / 14;
+// 300 x 64: 16 K 11 / 17, 32 K 19 / 18; 602 x 256: 4000 16 / 21, 8000 32 / 25; 256 x 602: 2000 15 / 15, 4000 25 / 16.
+bool split_product_pays(const RowProductArgs& g)
+{
+    const double outputs = (double)g.m * g.n;
+    return sp_lds(g, 1) <= (size_t)kSpLds && outputs >= 1.6e6 && outputs * (g.side[0].k + g.side[1].k) >= 2e8;
+}
+
+template <bool BT, int FORM>
+static int launch_split_product_any(const RowProductArgs& g, hipStream_t stream)
+{
+    const int nt = sp_tiles(g);
+    const bool one_a_cu = sp_lds(g, nt) * 2 > (size_t)kSpLds;  // then of eight waves, otherwise two of four
+    if (nt == 4) return launch_split_product<4, 4, BT, FORM>(g, stream);
+    if (nt == 2) return one_a_cu ? launch_split_product<2, 8, BT, FORM>(g, stream) : launch_split_product<2, 4, BT, FORM>(g, stream);
+    return one_a_cu ? launch_split_product<1, 8, BT, FORM>(g, stream) : launch_split_product<1, 4, BT, FORM>(g, stream);
+}
+
+int split_product(const RowProductArgs& g, bool b_transposed, int form, hipStream_t stream)
+{
+    if (form == kRpSum) return b_transposed ? launch_split_product_any<true, kRpSum>(g, stream) : launch_split_product_any<false, kRpSum>(g, stream);
+    if (form == kRpAdd) return b_transposed ? launch_split_product_any<true, kRpAdd>(g, stream) : launch_split_product_any<false, kRpAdd>(g, stream);
+    return b_transposed ? launch_split_product_any<true, kRpOne>(g, stream) : launch_split_product_any<false, kRpOne>(g, stream);
+}
+
+}  // namespace fgl

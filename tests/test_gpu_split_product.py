@@ -1,0 +1,73 @@
+"""fp32 products over rows on the bf16 matrix cores (csrc/fgl_split_product.hip) against float64, at the edges of their tiles: row tiles of 32, 32, 64 and 128
+columns a workgroup, steps of 16 k that are odd or even in number and end with k, k too long for one width of B in LDS; and values that have no three bf16 parts."""
+import pytest
+import torch
+
+from fastgl import ops
+
+pytestmark = pytest.mark.gpu
+
+# all large enough for the split (1.6e6 outputs, 2e8 multiplications): (rows, k, columns)
+SHAPES = [(1_600_001, 1, 128), (450_017, 7, 65), (210_031, 15, 64), (210_001, 16, 64), (400_033, 17, 31), (97_001, 33, 63), (50_001, 64, 129), (26_001, 100, 256),
+          (32_003, 96, 66), (6_417, 256, 300), (6_500, 416, 250), (6_500, 417, 250), (50_001, 832, 33), (50_001, 833, 33)]
+
+
+def _check(got, want, bound):
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_split_product(cuda, m, k, n, transposed):
+    print("split product", m, k, n, transposed, flush=True)
+    gen = torch.Generator(device=cuda).manual_seed(m + k + n)
+    a = torch.full((m, k + 3), float("nan"), device=cuda)[:, 1:k + 1]  # (rows that start on no vector's boundary; what lies around must not be read into the sums)
+    a.copy_(torch.randn((m, k), generator=gen, device=cuda))
+    b = torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
+    bias = torch.randn(n, generator=gen, device=cuda)
+    w = (b.t() if transposed else b).double()
+    got, plus = ops.row_product(a, b, transposed), ops.row_product(a, b, transposed, bias)
+    for rows in (slice(0, 5000), slice(m // 2, m // 2 + 5000), slice(max(m - 5000, 0), m)):
+        x = a[rows].double()
+        # three parts of eight bits each: the products that are left out are below 2^-26, what a matrix instruction cuts off below 2^-25 of a chunk's sum, and k / 32
+        # sums are rounded: within the (k + 2) 2^-24 of the magnitudes that k fp32 products and sums are given
+        want, bound = x @ w, (k + 2) * 2.0 ** -24 * (x.abs() @ w.abs() + bias.double().abs())
+        _check(got[rows], want, bound)
+        _check(plus[rows], want + bias.double(), bound)
+
+
+@pytest.mark.parametrize("m,k0,k1,n", [(40_001, 100, 33, 65), (13_001, 256, 128, 128), (30_001, 16, 400, 64)])
+def test_sums_and_additions(cuda, m, k0, k1, n):
+    gen = torch.Generator(device=cuda).manual_seed(m)
+    a0, a1 = (torch.randn((m, k), generator=gen, device=cuda) for k in (k0, k1))
+    b0, b1 = (torch.randn((n, k), generator=gen, device=cuda) for k in (k0, k1))
+    bias, base = torch.randn(n, generator=gen, device=cuda), torch.randn((m + 5, n), generator=gen, device=cuda)
+    want, size = a0.double() @ b0.double().t() + a1.double() @ b1.double().t() + bias.double(), a0.double().abs() @ b0.double().abs().t() + a1.double().abs() @ b1.double().abs().t()
+    _check(ops.row_product_sum(a0, b0, a1, b1, bias), want, (k0 + k1 + 2) * 2.0 ** -24 * (size + bias.double().abs()))
+    w = b0.t().contiguous()
+    got = ops.row_product_add_(base.clone(), a0, w)
+    assert torch.equal(got[m:], base[m:])
+    size = a0.double().abs() @ w.double().abs() + base[:m].double().abs()
+    _check(got[:m], a0.double() @ w.double() + base[:m].double(), (k0 + 2) * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_values_without_three_parts(cuda, transposed):
+    m, k, n = 40_000, 100, 64
+    gen = torch.Generator(device=cuda).manual_seed(5)
+    a, b = torch.randn((m, k), generator=gen, device=cuda), torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
+    clean = ops.row_product(a, b, transposed)
+    a[70, 3], a[1000, 99], a[1000, 5], a[5000, 0], a[5001, 98] = float("inf"), float("inf"), float("-inf"), float("nan"), float("-inf")
+    a[9000] = 3.4e38 * torch.rand(k, generator=gen, device=cuda) ** 0.01  # (rounds to infinity in bf16)
+    b.mul_(0.01)
+    a[20000] *= 1e-36  # (bits below bf16's last)
+    a[30000] *= 1e-42
+    got, w = ops.row_product(a, b, transposed), (b.t() if transposed else b).double()
+    want = a.double() @ w
+    for r in (70, 1000, 5000, 5001):  # (row 1000: inf * w - inf * w', infinite or not a number by the weights' signs)
+        assert not bool(torch.isfinite(got[r]).any()) and torch.allclose(got[r].double(), want[r], rtol=0, atol=0, equal_nan=True)
+    rest = torch.tensor([r for r in range(m) if r not in (70, 1000, 5000, 5001)], device=cuda)
+    # (subnormal operands and results: each rounded to a multiple of 2^-149 at most once a term)
+    _check(got[rest], want[rest], (k + 2) * 2.0 ** -24 * (a[rest].double().abs() @ w.abs()) + (k + 2) * 2.0 ** -149)
+    neighbours = torch.cat((torch.arange(0, 70), torch.arange(1024, 4992), torch.arange(31000, m))).to(cuda)
+    _check(got[neighbours], clean[neighbours].double() * 0.01, (k + 4) * 2.0 ** -23 * (a[neighbours].double().abs() @ w.abs()))
