@@ -401,8 +401,14 @@ def _forms_row_product(a, b, transposed, m, k, n):
     line keep the GPU busy for longer than the host takes, and there it depends on the size (a GIN layer of 602 x 256 over 8192 rows, forward and backward, is the
     library's: 394 / 418 in all), see ``_long_product_is_the_kernels``.
     Returns the operands' addresses and row strides if so, else None."""
-    if not (k * n <= 100000 and (m * k * n <= 8 * 10 ** 9 or _long_product_is_the_kernels(a.dtype, transposed, k, n)) and
-            a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
+    if not (k * n <= 100000 and (m * k * n <= 8 * 10 ** 9 or _long_product_is_the_kernels(a.dtype, transposed, k, n))):
+        return None
+    return _product_operands(a, b, transposed, m, k, n)
+
+
+def _product_operands(a, b, transposed, m, k, n):
+    """The operands' addresses and row strides where fgl_row_product can take them, else None (see ``_forms_row_product``)."""
+    if not (a.is_cuda and a.dtype == b.dtype and a.dtype in _FEAT and m > 0 and 0 < k <= 65536 and 0 < n <= 65536 and
             a.get_device() == b.get_device() and not (torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)) and
             not torch.is_autocast_enabled() and not _followed()):
         return None
@@ -413,13 +419,26 @@ def _forms_row_product(a, b, transposed, m, k, n):
     return None
 
 
+def _forms_split_product(a, b, transposed, m, k, n):
+    """What ``_forms_row_product`` leaves, and the fp32 kernel on the bf16 matrix cores (csrc/fgl_split_product.hip) forms ahead of the library: more than 8e9
+    multiplications, or weights of more than 100000 values.  GPU time over the library's (N: plain, T: transposed weight), 9e9 multiplications: k = 64 .. 256
+    and n = 64, 100, 128, 256, 300 0.5 .. 0.95 in both layouts (2.4 M x 100 x 64 338 / 512 us, x 64 x 100 325 / 627); but n = 66, which takes two workgroups' columns, 1.03 .. 1.09, n = 160,
+    which takes three and is whole vectors to the library, 1.06 .. 1.18 from k = 200 on, and n = 33 and 47 1.02 .. 1.11 from k = 384 on.  Wide weights: 256 x 602
+    N 0.84 / 0.76 / 0.58, T 0.98 / 0.71 / 0.71 (8192 / 20 K / 60 K rows), 400 x 300 0.61 / 0.49 / 0.77, 300 x 400 0.85 / 0.88 / 0.80; but 4000 rows of these two, fewer
+    than 2e6 results, 1.01 .. 1.16, and a k beyond 400, of which only 32 columns at a time fit, 0.9 .. 1.2 (602 x 256: 0.96 .. 1.10)."""
+    if not (a.dtype == torch.float32 and 32 < k <= 400 and m * n >= 2 * 10 ** 6 and not 64 < n < 72 and not (k > 128 and 128 < n <= 160) and
+            not (k > 256 and n <= 48)):
+        return None
+    return _product_operands(a, b, transposed, m, k, n)
+
+
 def row_product(a, b, transposed=False, bias=None):
     """``a b`` (``transposed``: ``a b^T``) ``+ bias`` for the rows ``a`` [m, k] of a block and a layer's weight ``b`` [k, n]
     (transposed: [n, k]); fp32 sums, result in the operands' dtype."""
     if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(1 if transposed else 0):
         raise RuntimeError("row_product: shapes %s and %s do not match" % (tuple(a.shape), tuple(b.shape)))
     m, k, n = int(a.size(0)), int(a.size(1)), int(b.size(0 if transposed else 1))
-    at = _forms_row_product(a, b, transposed, m, k, n)
+    at = _forms_row_product(a, b, transposed, m, k, n) or _forms_split_product(a, b, transposed, m, k, n)
     if at is None or not (bias is None or (bias.device == a.device and bias.dtype == a.dtype and bias.is_contiguous() and bias.numel() == n and
                                            not (torch.is_grad_enabled() and bias.requires_grad))):
         w = b.transpose(0, 1) if transposed else b

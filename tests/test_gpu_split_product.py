@@ -71,3 +71,19 @@ def test_values_without_three_parts(cuda, transposed):
     _check(got[rest], want[rest], (k + 2) * 2.0 ** -24 * (a[rest].double().abs() @ w.abs()) + (k + 2) * 2.0 ** -149)
     neighbours = torch.cat((torch.arange(0, 70), torch.arange(1024, 4992), torch.arange(31000, m))).to(cuda)
     _check(got[neighbours], clean[neighbours].double() * 0.01, (k + 4) * 2.0 ** -23 * (a[neighbours].double().abs() @ w.abs()))
+
+
+@pytest.mark.parametrize("m,k,n,split", [(1_300_001, 100, 64, True), (1_300_001, 100, 66, False), (8192, 256, 602, True), (3000, 256, 602, False), (8192, 602, 256, False),
+                                         (300_001, 200, 160, False), (600_001, 384, 40, False)])
+def test_products_beyond_the_general_line(cuda, m, k, n, split):
+    print("long or wide product", m, k, n, flush=True)
+    gen = torch.Generator(device=cuda).manual_seed(m)
+    a = torch.randn((m, k), generator=gen, device=cuda)
+    for transposed in (False, True):
+        b = torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
+        assert ops._forms_row_product(a, b, transposed, m, k, n) is None
+        assert (ops._forms_split_product(a, b, transposed, m, k, n) is not None) == split
+        got, w = ops.row_product(a, b, transposed), (b.t() if transposed else b).double()
+        for rows in (slice(0, 1000), slice(m - 1000, m)):
+            x = a[rows].double()
+            _check(got[rows], x @ w, (k + 2) * 2.0 ** -24 * (x.abs() @ w.abs()))
