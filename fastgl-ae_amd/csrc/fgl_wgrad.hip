@@ -25,10 +25,21 @@
 // 602 x 256, k = 8192: 57 -> 42 us; bf16 100 x 256, k = 105 K: 245 -> 25 us, 100 x 64, k = 2.4 M: 2745 -> 148 us (5.3 TB/s).
 // Eight rows a step and one step ahead: 16 and 24 rows measured the same within 3 %.
 //
+// The split form of fp32: the fp32 matrix instructions' rate is what the wide tiles wait for, and their 256 accumulators a lane leave one wave a SIMD, which nothing
+// covers while it waits for rows.  Each value is three bf16 parts instead, a product six bf16 products (fgl_split_product.hip says which and how exact that is), in
+// tiles of 64 x 64, two waves a SIMD: one splits (88 instructions for a step's 64 columns) while the other multiplies.  Every step's products are added up from
+// zero before they are added to the accumulators; and since what a matrix instruction cuts off is cut downwards, which over 10^4 .. 10^6 rows adds up (7e-7 of the
+// result's 2-norm for k = 107 K where the fp32 form has 2.8e-7), every other step is formed of A's negative and subtracted: 1.4e-7.
+// us, fp32 / split: 100 x 256 k = 107 K 75 / 68, k = 16 K 33 / 21, k = 2000 26 / 12; 256 x 256 k = 17 K 36 / 29, k = 5000 31 / 16; 128 x 128 k = 60 K 37 / 28;
+// 602 x 256 k = 8192 41 / 38; 256 x 47 k = 20 K 20 / 16.  What it waits for now is the rows: one step ahead is half a microsecond at these rates.
+// Tried: blocks of 128 x 128 through LDS, in which every value is split once (65 us for the first of these, but 34 and 41 for 256 x 256 and 602 x 256), and two steps ahead, for
+// which the registers do not suffice (89).
+//
 // A lane whose columns would leave the row takes the row's last VA columns instead (its sums are then bit-equal copies of
 // its neighbour's); rows past the end are replaced by zeros.  No access leaves the operands.
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
+#include "fgl_split.hpp"
 
 namespace fgl {
 
@@ -142,6 +153,42 @@ __device__ __forceinline__ void wgrad_multiply(const WgradRows<uint16_t, VA>& a,
     }
 }
 
+// The rows of a step of the split form as loaded: eight per half-wave, V neighbouring columns a lane.
+template <int V>
+struct WgradEights {
+    typedef float Vec __attribute__((ext_vector_type(V), aligned(4)));
+    Vec r[8];
+    static __device__ __forceinline__ uint32_t lane_offset(int col, int64_t ld, int half) { return (uint32_t)(8 * half * ld) + (uint32_t)col; }
+    __device__ __forceinline__ void load(const float* p, int64_t ld, uint32_t off)
+    {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = *reinterpret_cast<const Vec*>(p + (int64_t)i * ld + off);
+    }
+    __device__ __forceinline__ void load_tail(const float* p, int64_t ld, uint32_t off, int half, int n)
+    {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            Vec z = {};
+            r[i] = z;
+            if (8 * half + i < n) r[i] = *reinterpret_cast<const Vec*>(p + (int64_t)i * ld + off);
+        }
+    }
+    // sign times column c in three parts, and the largest magnitude of it so far
+    __device__ __forceinline__ void split(int c, float sign, SpU4 (&p)[3], float& most) const
+    {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = r[i][c] * sign;
+        sp_split(v, p);
+        sp_most(v, most);
+    }
+    __device__ __forceinline__ void add_columns(float (&sum)[V]) const
+    {
+#pragma unroll
+        for (int c = 0; c < V; ++c) sum[c] += ((r[0][c] + r[1][c]) + (r[2][c] + r[3][c])) + ((r[4][c] + r[5][c]) + (r[6][c] + r[7][c]));
+    }
+};
+
 struct WgradArgs {
     const void* a;
     const void* b;
@@ -166,45 +213,20 @@ __device__ __forceinline__ int wgrad_column(int tile, int i, int n)
     return c + V <= n ? c : n - V;
 }
 
+// acc += the products of the wave's rows between k0 and k1, and sum += the column sums of A's.  col_a, col_b: the lane's first column of either.
 template <typename T, int VA, int VB>
-__global__ __launch_bounds__(kBlock, VA * VB >= 16 ? 1 : 2) void wgrad_kernel(const WgradArgs g)
+__device__ __forceinline__ void wgrad_rows(const WgradArgs& g, int64_t k0, int64_t k1, int wave, int col_a, int col_b, bool sums, F32x16 (&acc)[VA * VB], float (&sum)[VA])
 {
-    constexpr int kRows = WgradRows<T, VA>::kRows;
-    constexpr int kTiles = VA * VB;                    // 32x32 tiles of a wave
-    constexpr int kChunk = kTiles < 4 ? kTiles : 4;    // of them added through LDS at a time
-    constexpr int kWaves = kBlock / kWave;
-    __shared__ float s_acc[kWaves][kChunk * 16][kWave];
-    const int lane = lane_id();
-    // The wave's number as a scalar: every branch around the matrix instructions below has to be a branch of the whole wave,
-    // since they multiply in all lanes whatever the execution mask says.
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    // workgroup -> (split, tile): eight neighbouring splits (one per XCD) take turns, so the tiles of a split share an XCD
-    const int group = (int)(blockIdx.x / (8u * (unsigned)g.tiles)), in_group = (int)(blockIdx.x % (8u * (unsigned)g.tiles));
-    const int split = group * 8 + in_group % 8, tile = in_group / 8;
-    if (split >= g.splits) return;  // (uniform over the workgroup)
-    const int tm = tile / g.tiles_n, tn = tile % g.tiles_n;
-    const int64_t k0 = (int64_t)split * g.k_per_split;
-    const int64_t k1 = k0 + g.k_per_split < g.k ? k0 + g.k_per_split : g.k;
-    const int half = lane / 32;
+    const int half = lane_id() / 32;
     const T* pa = static_cast<const T*>(g.a);
     const T* pb = static_cast<const T*>(g.b);
-    const uint32_t off_a = WgradRows<T, VA>::lane_offset(wgrad_column<VA>(tm, lane % 32, g.m), g.lda, half);
-    const uint32_t off_b = WgradRows<T, VB>::lane_offset(wgrad_column<VB>(tn, lane % 32, g.n), g.ldb, half);
-    F32x16 acc[kTiles];
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
-    // (the column sums of A ride on the workgroups of C's first column of tiles)
-    const bool sums = g.sum_a != nullptr && tn == 0;
-    float sum[VA];
-#pragma unroll
-    for (int i = 0; i < VA; ++i) sum[i] = 0.0f;
-
+    const uint32_t off_a = WgradRows<T, VA>::lane_offset(col_a, g.lda, half);
+    const uint32_t off_b = WgradRows<T, VB>::lane_offset(col_b, g.ldb, half);
     // The wave's steps: rows k .. k + kRows - 1, then four steps (one per wave) further on; only the last may be short (or
     // empty).  The next step's rows are requested before the current ones are multiplied.  Nothing branches between the last
     // products and the first reads of the accumulators: a matrix instruction's results may be read a fixed number of
     // cycles later only, which the compiler (clang 22) was seen not to keep across such a branch.
+    constexpr int kRows = WgradRows<T, VA>::kRows, kWaves = kBlock / kWave;
     constexpr int64_t kStep = (int64_t)kRows * kWaves;
     const int64_t first = k0 + (int64_t)wave * kRows;
     const int whole = k1 > first ? (int)((k1 - first - 1) / kStep) : 0;  // steps before the last one
@@ -240,6 +262,130 @@ __global__ __launch_bounds__(kBlock, VA * VB >= 16 ? 1 : 2) void wgrad_kernel(co
     }
     wgrad_multiply<VA, VB>(a0, b0, acc);
     wgrad_multiply<VA, VB>(a1, b1, acc);
+}
+
+// The same in three bf16 parts a value, the wave's rows being others; true where the lane met values that have none (then acc is not the sum)
+template <int VA, int VB>
+__device__ __forceinline__ bool wgrad_split_rows(const WgradArgs& g, int64_t k0, int64_t k1, int wave, int col_a, int col_b, bool sums, F32x16 (&acc)[VA * VB],
+                                                 float (&sum)[VA])
+{
+    constexpr int kRows = 16, kWaves = kBlock / kWave;
+    constexpr int64_t kStep = (int64_t)kRows * kWaves;
+    constexpr int kPa[6] = {2, 0, 1, 1, 0, 0}, kPb[6] = {0, 2, 1, 0, 1, 0};  // (the small products first)
+    const int half = lane_id() / 32;
+    const uint32_t off_a = WgradEights<VA>::lane_offset(col_a, g.lda, half);
+    const uint32_t off_b = WgradEights<VB>::lane_offset(col_b, g.ldb, half);
+    const int64_t first = k0 + (int64_t)wave * kRows;
+    const int whole = k1 > first ? (int)((k1 - first - 1) / kStep) : 0;  // steps before the last one, which may be short or empty
+    const float* ra = static_cast<const float*>(g.a) + first * g.lda;
+    const float* rb = static_cast<const float*>(g.b) + first * g.ldb;
+    const int64_t last = first + whole * kStep;
+    const int n = k1 - last < kRows ? (k1 > last ? (int)(k1 - last) : 0) : kRows;
+    WgradEights<VA> a;
+    WgradEights<VB> b;
+    float most_a[VA], most_b[VB];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) most_a[i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VB; ++j) most_b[j] = 0.0f;
+    auto load = [&](int i) {
+        if (i < whole) {
+            a.load(ra, g.lda, off_a);
+            b.load(rb, g.ldb, off_b);
+        } else {
+            a.load_tail(ra, g.lda, off_a, half, n);
+            b.load_tail(rb, g.ldb, off_b, half, n);
+        }
+        ra += kStep * g.lda;
+        rb += kStep * g.ldb;
+    };
+    load(0);
+    float sign = 1.0f;
+    for (int s = 0; s <= whole; ++s) {
+        if (sums) a.add_columns(sum);
+        SpU4 pa[VA][3], pb[VB][3];
+#pragma unroll
+        for (int i = 0; i < VA; ++i) a.split(i, sign, pa[i], most_a[i]);
+#pragma unroll
+        for (int j = 0; j < VB; ++j) b.split(j, 1.0f, pb[j], most_b[j]);
+        if (s < whole) load(s + 1);  // (on the way while these are multiplied)
+        __builtin_amdgcn_sched_barrier(0);
+        F32x16 part[VA * VB];
+#pragma unroll
+        for (int i = 0; i < VA; ++i)
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int j = 0; j < VB; ++j)
+                    part[i * VB + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(Bf16x8, pa[i][kPa[q]]), __builtin_bit_cast(Bf16x8, pb[j][kPb[q]]),
+                                                                               q == 0 ? F32x16{} : part[i * VB + j], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < VA * VB; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[t][i] = fmaf(part[t][i], sign, acc[t][i]);
+        sign = -sign;
+    }
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < VA; ++i) odd |= sp_small(fmaxf(most_a[i], __shfl_xor(most_a[i], 32, kWave)));
+#pragma unroll
+    for (int j = 0; j < VB; ++j) odd |= sp_small(fmaxf(most_b[j], __shfl_xor(most_b[j], 32, kWave)));
+#pragma unroll
+    for (int t = 0; t < VA * VB; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) odd |= __builtin_amdgcn_classf(acc[t][i], 0x207);  // (infinite or not a number)
+    return odd;
+}
+
+template <typename T, int VA, int VB, bool SPLIT>
+__global__ __launch_bounds__(kBlock, VA * VB >= 16 ? 1 : 2) void wgrad_kernel(const WgradArgs g)
+{
+    constexpr int kTiles = VA * VB;                    // 32x32 tiles of a wave
+    constexpr int kChunk = kTiles < 4 ? kTiles : 4;    // of them added through LDS at a time
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ float s_acc[kWaves][kChunk * 16][kWave];
+    const int lane = lane_id();
+    // The wave's number as a scalar: every branch around the matrix instructions below has to be a branch of the whole wave,
+    // since they multiply in all lanes whatever the execution mask says.
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    // workgroup -> (split, tile): eight neighbouring splits (one per XCD) take turns, so the tiles of a split share an XCD
+    const int group = (int)(blockIdx.x / (8u * (unsigned)g.tiles)), in_group = (int)(blockIdx.x % (8u * (unsigned)g.tiles));
+    const int split = group * 8 + in_group % 8, tile = in_group / 8;
+    if (split >= g.splits) return;  // (uniform over the workgroup)
+    const int tm = tile / g.tiles_n, tn = tile % g.tiles_n;
+    const int64_t k0 = (int64_t)split * g.k_per_split;
+    const int64_t k1 = k0 + g.k_per_split < g.k ? k0 + g.k_per_split : g.k;
+    const int col_a = wgrad_column<VA>(tm, lane % 32, g.m), col_b = wgrad_column<VB>(tn, lane % 32, g.n);
+    F32x16 acc[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+    // (the column sums of A ride on the workgroups of C's first column of tiles)
+    const bool sums = g.sum_a != nullptr && tn == 0;
+    float sum[VA];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) sum[i] = 0.0f;
+
+    if constexpr (SPLIT) {
+        // (all waves of a workgroup or none; the sums of columns are right all the same)
+        if (__syncthreads_or(wgrad_split_rows<VA, VB>(g, k0, k1, wave, col_a, col_b, sums, acc, sum))) {
+            float unused[VA];
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) acc[t] = F32x16{};
+            wgrad_rows<T, VA, VB>(g, k0, k1, wave, col_a, col_b, false, acc, unused);
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {  // (read before the branch ends, see wgrad_rows)
+                    float v = acc[t][i] + 0.0f;
+                    asm volatile("" : "+v"(v));
+                    acc[t][i] = v;
+                }
+        }
+    } else {
+        wgrad_rows<T, VA, VB>(g, k0, k1, wave, col_a, col_b, sums, acc, sum);
+    }
 
     float* out = g.partial + ((int64_t)split * g.tiles + tile) * (kTiles * 16) * kWave;
 #pragma unroll
@@ -317,12 +463,12 @@ __global__ __launch_bounds__(kBlock) void wgrad_reduce_kernel(const WgradArgs g)
 }
 
 // Columns per lane along one side of C: what pads the least, the wider of two that pad alike.
-static inline int wgrad_vec(int n, bool vectors)
+static inline int wgrad_vec(int n, bool vectors, int widest)
 {
     if (!vectors || n <= 32) return 1;
     int best = 1;
     int64_t pad = ceil_div(n, 32) * 32;
-    for (int v = 2; v <= 4; v *= 2) {
+    for (int v = 2; v <= widest; v *= 2) {
         const int64_t p = ceil_div(n, 32 * v) * 32 * v;
         if (n >= v && p * 10 <= pad * 12) {  // (a fifth more columns is a fair price for a vector load twice as wide)
             best = v;
@@ -340,19 +486,34 @@ struct WgradPlan {
     size_t ws_bytes;
 };
 
-static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok)
+// Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
+// faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
+// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 75 / 68, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237).
+static bool wgrad_split_pays(int64_t k, int m, int n)
+{
+    return wgrad_vec(m, true, 4) * wgrad_vec(n, true, 4) >= 8 && (double)k * m * n <= 9e9;
+}
+
+static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, bool split)
 {
     WgradPlan p;
-    p.va = wgrad_vec(m, va_ok);
-    p.vb = wgrad_vec(n, vb_ok);
+    p.va = wgrad_vec(m, va_ok, split ? 2 : 4);
+    p.vb = wgrad_vec(n, vb_ok, split ? 2 : 4);
     p.tiles_n = (int)ceil_div(n, 32 * p.vb);
     p.tiles = p.tiles_n * (int)ceil_div(m, 32 * p.va);
     // workgroups: one per CU with 16 tiles a wave (256 accumulators a lane), more of the smaller ones
-    const int per_cu = p.va * p.vb >= 16 ? 1 : p.va * p.vb >= 8 ? 2 : 4;
+    const int per_cu = p.va * p.vb >= 16 ? 1 : p.va * p.vb >= 8 || split ? 2 : 4;
     int64_t splits = 256 * per_cu / p.tiles;
     const int64_t most = ceil_div(k, 256);  // 256 rows and more per split: the sum over the splits costs as much as they do otherwise
     if (splits > most) splits = most;
     if (splits > 8) splits = splits / 8 * 8;
+    // With many tiles eights of splits fill the chip badly (602 x 256 in 40 tiles: 320 workgroups of 512 places): the first number of them that leaves less than an
+    // eighth of the places empty, also if it takes two rounds
+    for (int64_t s = 8; split && splits < 32 && s <= 32 && s <= most; s += 8) {
+        const int64_t rounds = ceil_div(s * p.tiles, 512) * 512;
+        splits = s;
+        if (s * p.tiles * 8 >= rounds * 7) break;
+    }
     if (splits < 1) splits = 1;
     p.k_per_split = ceil_div(ceil_div(k, splits), 64) * 64;
     if (p.k_per_split < 64) p.k_per_split = 64;
@@ -368,11 +529,11 @@ static bool wgrad_vectors(int dtype, int cols, int64_t ld, const void* ptr)
     return dtype == FGL_F32 || (cols % 2 == 0 && ld % 2 == 0 && ((uintptr_t)ptr & 3) == 0);
 }
 
-template <typename T, int VA, int VB>
+template <typename T, int VA, int VB, bool SPLIT>
 static int launch_wgrad(const WgradArgs& g, hipStream_t stream)
 {
     const int64_t blocks = ceil_div(g.splits, 8) * 8 * g.tiles;
-    hipLaunchKernelGGL((wgrad_kernel<T, VA, VB>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
+    hipLaunchKernelGGL((wgrad_kernel<T, VA, VB, SPLIT>), dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
     const int64_t sum_blocks = g.sum_a != nullptr ? ceil_div((int64_t)(g.tiles / g.tiles_n) * 32 * VA, kWave) : 0;
     hipLaunchKernelGGL((wgrad_reduce_kernel<T, VA, VB>), dim3((unsigned)(g.tiles * VA * VB * 16 + sum_blocks)), dim3(kBlock), 0, stream, g);
     FGL_CHECK_LAUNCH("wgrad_kernel");
@@ -382,7 +543,7 @@ static int launch_wgrad(const WgradArgs& g, hipStream_t stream)
 template <typename T>
 static int launch_wgrad_any(const WgradPlan& p, const WgradArgs& g, hipStream_t s)
 {
-#define FGL_WGRAD_CASE(A_, B_) if (p.va == A_ && p.vb == B_) return launch_wgrad<T, A_, B_>(g, s)
+#define FGL_WGRAD_CASE(A_, B_) if (p.va == A_ && p.vb == B_) return launch_wgrad<T, A_, B_, false>(g, s)
     FGL_WGRAD_CASE(4, 4);
     FGL_WGRAD_CASE(4, 2);
     FGL_WGRAD_CASE(4, 1);
@@ -392,7 +553,7 @@ static int launch_wgrad_any(const WgradPlan& p, const WgradArgs& g, hipStream_t 
     FGL_WGRAD_CASE(1, 4);
     FGL_WGRAD_CASE(1, 2);
 #undef FGL_WGRAD_CASE
-    return launch_wgrad<T, 1, 1>(g, s);
+    return launch_wgrad<T, 1, 1, false>(g, s);
 }
 
 }  // namespace fgl
@@ -404,9 +565,11 @@ FGL_EXPORT size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n)
     if (k < 0 || m < 1 || n < 1) return 0;
     size_t most = 0;
     for (int i = 0; i < 4; ++i) {
-        const size_t b = wgrad_plan(k, m, n, (i & 1) != 0, (i & 2) != 0).ws_bytes;
+        const size_t b = wgrad_plan(k, m, n, (i & 1) != 0, (i & 2) != 0, false).ws_bytes;
         if (b > most) most = b;
     }
+    const size_t b = wgrad_plan(k, m, n, true, true, true).ws_bytes;
+    if (b > most) most = b;
     return most;
 }
 
@@ -418,7 +581,8 @@ FGL_EXPORT int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, in
     FGL_REQUIRE(lda >= m && ldb >= n && ldc >= n, "weight_grad: row stride smaller than the row length");
     FGL_REQUIRE(lda < (1 << 24) && ldb < (1 << 24), "weight_grad: row stride too large");  // (eight rows are spanned by 32-bit offsets)
     FGL_REQUIRE(d_c != nullptr && (k == 0 || (d_a && d_b)), "weight_grad: null pointer");
-    const WgradPlan p = wgrad_plan(k, m, n, wgrad_vectors(dtype, m, lda, d_a), wgrad_vectors(dtype, n, ldb, d_b));
+    const bool split = dtype == FGL_F32 && wgrad_split_pays(k, m, n);
+    const WgradPlan p = wgrad_plan(k, m, n, wgrad_vectors(dtype, m, lda, d_a), wgrad_vectors(dtype, n, ldb, d_b), split);
     if (d_ws == nullptr || ws_bytes < p.ws_bytes) {
         set_error("weight_grad: workspace too small (%zu < %zu)", ws_bytes, p.ws_bytes);
         return FGL_ERR_WORKSPACE;
@@ -428,6 +592,7 @@ FGL_EXPORT int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, in
     g.splits = p.splits; g.k_per_split = p.k_per_split; g.partial = static_cast<float*>(d_ws); g.c = d_c; g.ldc = ldc;
     g.sum_a = d_sum_a; g.partial_sum = reinterpret_cast<float*>(static_cast<char*>(d_ws) + p.sum_offset);
     hipStream_t s = as_stream(stream);
+    if (split) return launch_wgrad<float, 2, 2, true>(g, s);  // (whoever is 128 wide in fours or 64 in twos is whole in twos)
     if (dtype == FGL_F32) return launch_wgrad_any<float>(p, g, s);
     return launch_wgrad_any<uint16_t>(p, g, s);
 }

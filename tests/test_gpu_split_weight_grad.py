@@ -1,0 +1,48 @@
+"""The weight gradient in three bf16 parts a value (csrc/fgl_wgrad.hip) against float64: short and odd numbers of steps, tiles that the columns do not fill, many tiles
+with several rounds of workgroups, strided rows with their column sums, and values that have no three parts."""
+import pytest
+import torch
+
+from fastgl import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n", [(100, 64), (65, 200), (256, 47), (127, 129), (602, 256)])
+def test_against_float64(cuda, m, n):
+    gen = torch.Generator(device=cuda).manual_seed(m + n)
+    for k in (1, 15, 16, 17, 63, 65, 127, 129, 1001, 8192, 30011):
+        print("weight gradient", m, n, k, flush=True)
+        a = torch.full((k, m + 3), float("nan"), device=cuda)[:, 1:m + 1]  # (what lies around the rows must not be read into the sums)
+        a.copy_(torch.randn((k, m), generator=gen, device=cuda))
+        b = torch.randn((k, n), generator=gen, device=cuda)
+        got, sums = ops.weight_grad(a, b, column_sums=True)
+        want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+        # a step of 16 rows is right to 2^-24 of its largest sum or so, and k / 16 of them are added up in fp32: within (k / 16 + 16) 2^-24 of the magnitudes
+        assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
+        assert bool(((sums.double() - a.double().sum(0)).abs() <= (k / 16 + 16) * 2.0 ** -24 * a.double().abs().sum(0)).all())
+        again = ops.weight_grad(a, b)
+        assert torch.equal(got, again)
+
+
+def test_errors_do_not_add_up_over_the_rows(cuda):
+    """2-norm of the error over the result's: with the cut of the matrix instructions on one side it was 7e-7 here, that of fp32 sums is 3e-7."""
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    a, b = torch.randn((107_000, 100), generator=gen, device=cuda), torch.randn((107_000, 256), generator=gen, device=cuda)
+    want = a.double().t() @ b.double()
+    assert (ops.weight_grad(a, b).double() - want).norm() <= 2.8e-7 * want.norm()
+
+
+def test_values_without_three_parts(cuda):
+    k, m, n = 5000, 100, 128
+    gen = torch.Generator(device=cuda).manual_seed(5)
+    a, b = torch.randn((k, m), generator=gen, device=cuda), torch.randn((k, n), generator=gen, device=cuda) * 0.01
+    a[70, 3], a[4000, 9], b[4999, 100] = float("inf"), float("nan"), float("-inf")
+    a[:, 20] *= 1e-36      # (bits below bf16's last)
+    a[17, 30] = 3.4e38     # (rounds to infinity in bf16)
+    got, want = ops.weight_grad(a, b), a.double().t() @ b.double()
+    odd = ~torch.isfinite(want)
+    assert bool(odd[3].all()) and bool(odd[9].all()) and bool(odd[:, 100].all()) and int(odd.sum()) == 2 * n + m - 2
+    assert torch.allclose(got[odd].double(), want[odd], rtol=0, atol=0, equal_nan=True)
+    size = a.double().abs().t() @ b.double().abs()
+    assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size + k * 2.0 ** -149)[~odd].all())
