@@ -1133,6 +1133,9 @@ __global__ __launch_bounds__(kLongBlock) void aggregate_long_rows_kernel(const A
 // Measured (that graph, 64 fp32 columns, gcn weights, MI355X): 54 M entries 3403 -> 3137 us
 // in all (4.4 TB/s of gathered rows, the memory's bound; 100 columns 5154 -> 4307); 100 K nodes, 2.5 M entries: 274 -> 117 us.
 constexpr int kSegEntries = 512;
+struct ClassEnds {
+    uint16_t end[8];  // of each class in its segment
+};
 struct SegLists {
     int32_t* counts;    // [0] segments of rows of several, [1] rows of one segment, [2] rows of several segments
     int32_t* seg_row;   // segments of rows of several: the row ...
@@ -1140,19 +1143,47 @@ struct SegLists {
     int32_t* one_row;   // rows of one segment
     int32_t* many_row;  // rows of several segments: the row ...
     int32_t* many_seg;  // ... and its first segment's number (a row's segments are neighbours)
-    float* partial;     // [seg][ldp]
+    float* partial;     // [seg][ldp]; in classes: [seg][class][ldp]
     int ldp;
     int32_t cap_seg, cap_one, cap_many;
+    int one_entries;    // rows of up to so many entries are rows of one segment, which need no second sum
+    int classes;        // 1, or kClasses: segments are gathered class by class (see below)
+    int32_t* class_ids; // then: the segments' neighbour ids, class after class within each, at the places where its entries lie in `indices`
+    ClassEnds* class_ends;
 };
 
-// A row of n > kSegEntries entries has at most 2 n / kSegEntries segments.
-static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, size_t* bytes)
+// ---- segments in classes ---------------------------------------------------------------
+// Each XCD has its own L2 of 4 MB, 16 K rows of 256 bytes, and a gather that runs on all of them has the same 16 K most mentioned rows in every one.  Here the
+// neighbours are in eight classes by a hash of their ids, an XCD gathers one class of every segment, and its L2 has to hold an eighth of
+// the rows: 128 K different ones on the chip.  On an R-MAT graph of 2.4 M nodes and 54 M entries the 16 K most mentioned rows are 44 % of all mentions and the 128 K
+// most mentioned 78 %; a third of the accesses hit the L2 before, and what missed came through the fabric at 6.2 TB/s, which is what it gives.
+// A launch puts every segment's ids in order of class (a wave a segment, by ballots: the sums' order does not depend on scheduling), the next takes (segment, class)
+// by lane group, workgroup w the class w mod 8 -- workgroups go to the XCDs in turn -- and a row's sums are added up in their order.  32 neighbouring ids are of one class,
+// so that a line of their entry counts is read by one XCD as well.  Right on any mapping of workgroups; only the speed depends on it.
+// MI355X, gcn weights, us, segments as they come / in classes: that graph, 64 fp32 columns 2455 / 1935 -- of it the rows of more than 256 entries 1300 / 800: 655 gathering (11 TB/s of
+// rows), 86 the ids' order, 54 the sums -- 100 columns 3730 / 3120, 128 4800 / 4000, 128 bf16 columns 2560 / 2065; 1.2 M nodes, 27 M entries, 100 fp32 columns 1700 / 1420;
+// 600 K, 13 M, 64 columns 525 / 470, in another place of memory 413 / 413.  The lines: 600 K, 9 M 335 / 330, 1.2 M, 9 M 423 / 434, 300 K, 6.5 M 199 / 218; rows of 128 bytes, of which an L2 holds twice as
+// many, 1165 / 1250.  Graphs without long rows pay two launches more that end at once (600 K rows of 40 entries 1106 / 1106).  Marking the loads of little-mentioned rows
+// as non-temporal instead changed nothing.
+constexpr int kClasses = 8;
+constexpr int kClassEntries = 256;                       // rows of fewer entries have too few a class to be worth eight sums
+constexpr int64_t kClassMinEntries = (int64_t)3 << 22;
+constexpr int kClassMinRow = 256;                        // bytes of a gathered row: of shorter ones an L2 holds enough as it is
+constexpr int64_t kClassMinBytes = (int64_t)64 << 20;    // of the gathered rows: twice what the L2s hold together
+constexpr size_t kClassMaxBytes = (size_t)4 << 30;       // of scratch
+__device__ __forceinline__ int neighbour_class(int id) { return (int)(((uint32_t)id >> 5) * 0x9E3779B1u >> 29); }
+
+// A row of n > kSegEntries entries has at most 2 n / kSegEntries segments, one of kClassEntries < n <= kSegEntries has one.
+static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, bool classes, size_t* bytes)
 {
     SegLists l;
     l.cap_seg = (int32_t)(2 * n_entries_max / kSegEntries + 1);
+    static_assert(kSegEntries <= 2 * kClassEntries, "the bound on the number of segments");
     l.cap_one = (int32_t)(n_entries_max / kLongRowEntries + 1);
-    l.cap_many = (int32_t)(n_entries_max / kSegEntries + 1);
+    l.cap_many = (int32_t)(n_entries_max / (classes ? kClassEntries : kSegEntries) + 1);
     l.ldp = (D + 7) / 8 * 8;
+    l.one_entries = classes ? kClassEntries : kSegEntries;
+    l.classes = classes ? kClasses : 1;
     Carver c(ws);
     l.counts = c.take<int32_t>(3);
     l.seg_row = c.take<int32_t>((size_t)l.cap_seg);
@@ -1160,9 +1191,26 @@ static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, size_t* bytes)
     l.one_row = c.take<int32_t>((size_t)l.cap_one);
     l.many_row = c.take<int32_t>((size_t)l.cap_many);
     l.many_seg = c.take<int32_t>((size_t)l.cap_many);
-    l.partial = c.take<float>((size_t)l.cap_seg * (size_t)l.ldp);
+    l.partial = c.take<float>((size_t)l.cap_seg * (size_t)l.ldp * (size_t)l.classes);
+    l.class_ids = classes ? c.take<int32_t>((size_t)n_entries_max) : nullptr;
+    l.class_ends = classes ? c.take<ClassEnds>((size_t)l.cap_seg) : nullptr;
     if (bytes) *bytes = c.used();
     return l;
+}
+
+// Scratch for classes, where there may be any: the caller's sizes decide, and the launch among those by what it also knows.
+static size_t class_bytes(int64_t n_entries_max, int D)
+{
+    if (n_entries_max < kClassMinEntries || D * (int64_t)sizeof(float) < kClassMinRow) return 0;
+    size_t bytes = 0;
+    (void)seg_lists(nullptr, n_entries_max, D, true, &bytes);
+    return bytes <= kClassMaxBytes ? bytes : 0;
+}
+static SegLists seg_lists_of(const AggArgs& g, size_t element)
+{
+    const int64_t row = g.D * (int64_t)element;
+    const bool classes = class_bytes(g.n_entries_max, g.D) > 0 && row >= kClassMinRow && g.n_rows_max * row >= kClassMinBytes;
+    return seg_lists(g.ws, g.n_entries_max, g.D, classes, nullptr);
 }
 
 __global__ void seg_init_kernel(int32_t* __restrict__ counts)
@@ -1274,7 +1322,7 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
 #pragma unroll
     for (int i = 0; i < ROWS; ++i) {
         if (entries[i] <= threshold) continue;
-        if (entries[i] <= kSegEntries) {
+        if (entries[i] <= l.one_entries) {
             ++ones;
         } else {
             ++many;
@@ -1298,7 +1346,7 @@ __global__ __launch_bounds__(kSegBlock) void seg_lists_kernel(const AggArgs g, c
     for (int i = 0; i < ROWS; ++i) {
         if (entries[i] <= threshold) continue;
         const int row = (int)(row0 + (int64_t)i * kSegBlock);
-        if (entries[i] <= kSegEntries) {
+        if (entries[i] <= l.one_entries) {
             if (at_one < l.cap_one) l.one_row[at_one] = row;
             ++at_one;
             continue;
@@ -1324,7 +1372,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_segments_kernel(const AggArg
     using IO = RowIO<T, VEC>;
     typedef float Vec __attribute__((ext_vector_type(VEC), aligned(4)));
     constexpr int kInFlight = LPR < 16 ? LPR : 16;
-    const int n_seg = l.counts[0] < l.cap_seg ? l.counts[0] : l.cap_seg;
+    const int n_seg = l.classes > 1 ? 0 : l.counts[0] < l.cap_seg ? l.counts[0] : l.cap_seg;  // (in classes: the launches below)
     const int n_one = l.counts[1] < l.cap_one ? l.counts[1] : l.cap_one;
     const int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
     if (unit >= (int64_t)n_seg + n_one) return;
@@ -1398,37 +1446,143 @@ __global__ __launch_bounds__(kBlock) void aggregate_segments_kernel(const AggArg
     *reinterpret_cast<Vec*>(l.partial + unit * l.ldp + col0) = v;
 }
 
-// The rows of several segments: a lane group adds a row's partial sums in order.
+// A segment's ids, class after class, each class's in their order: a wave a segment.
+__global__ __launch_bounds__(kBlock) void seg_classes_kernel(const AggArgs g, const SegLists l)
+{
+    constexpr int kRounds = kSegEntries / kWave;
+    const int n_seg = l.counts[0] < l.cap_seg ? l.counts[0] : l.cap_seg;
+    const int lane = lane_id();
+    for (int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; unit < n_seg; unit += (int64_t)gridDim.x * (kBlock / kWave)) {
+        const int a = l.seg_first[unit], row_b = g.indptr[l.seg_row[unit] + 1];
+        const int n = row_b - a < kSegEntries ? row_b - a : kSegEntries;
+        const int rounds = __builtin_amdgcn_readfirstlane((n + kWave - 1) / kWave);
+        int id[kRounds];
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) id[j] = j * kWave + lane < n ? g.indices[a + j * kWave + lane] : 0;
+        // which lanes of a round are of class c: from the three bits of their classes
+        uint64_t bits[kRounds][3], there[kRounds];
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            there[j] = bits[j][0] = bits[j][1] = bits[j][2] = 0;
+            if (j >= rounds) continue;
+            const int c = neighbour_class(id[j]);
+            there[j] = __ballot(j * kWave + lane < n);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) bits[j][b] = __ballot(c >> b & 1);
+        }
+        auto of_class = [&](int j, int c) {
+            uint64_t m = there[j];
+#pragma unroll
+            for (int b = 0; b < 3; ++b) m &= c >> b & 1 ? bits[j][b] : ~bits[j][b];
+            return m;
+        };
+        int total = 0;  // lane c: class c's entries
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j)
+            if (j < rounds) total += __popcll(of_class(j, lane & 7));
+        int end = total;
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) {
+            const int t = __shfl_up(end, d, 8);
+            if ((lane & 7) >= d) end += t;
+        }
+        int first = end - total;  // lane c: where the class's next entry goes
+        if (lane < 8) l.class_ends[unit].end[lane] = (uint16_t)end;
+        const uint64_t before = ((uint64_t)1 << lane) - 1;
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            if (j >= rounds) continue;
+            const int c = neighbour_class(id[j]);
+            const int at = __shfl(first, c, 8) + __popcll(of_class(j, c) & before);
+            if (j * kWave + lane < n) l.class_ids[a + at] = id[j];
+            first += __popcll(of_class(j, lane & 7));
+        }
+    }
+}
+
+// One lane group, the entries of one class of a segment.
+template <typename T, int VEC, int LPR, int MODE>
+__global__ __launch_bounds__(kBlock) void aggregate_classes_kernel(const AggArgs g, const SegLists l)
+{
+    typedef float Vec __attribute__((ext_vector_type(VEC), aligned(4)));
+    const int n_seg = l.counts[0] < l.cap_seg ? l.counts[0] : l.cap_seg;
+    const int cls = (int)(blockIdx.x % kClasses);
+    const int gl = (int)threadIdx.x % LPR;
+    const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, gl, g.D);
+    const T* __restrict__ X = static_cast<const T*>(g.x);
+    const bool all_full = all_lanes_full<T, VEC>(g.D);
+    // (a unit is a group's: all its lanes take the same turns)
+    for (int64_t unit = (int64_t)(blockIdx.x / kClasses) * (kBlock / LPR) + threadIdx.x / LPR; unit < n_seg; unit += (int64_t)(gridDim.x / kClasses) * (kBlock / LPR)) {
+        const int row = l.seg_row[unit];
+        const int entries = g.indptr[row + 1] - g.indptr[row];
+        const int first = l.seg_first[unit];
+        const int a = first + (cls > 0 ? l.class_ends[unit].end[cls - 1] : 0), b = first + l.class_ends[unit].end[cls];
+        float acc[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
+        const float row_factor = row_weight<MODE>(g.row_norm, row, entries);
+        int next_col = a + gl < b ? l.class_ids[a + gl] : 0;
+        for (int base = a; base < b; base += LPR) {
+            const int cnt = b - base < LPR ? b - base : LPR;
+            const int my_col = next_col;
+            const float my_w = gl < cnt ? edge_weight<MODE>(my_col, row_factor, g.col_norm, g.col_norm_is_ptr) : 0.0f;
+            next_col = base + LPR + gl < b ? l.class_ids[base + LPR + gl] : 0;
+            float part[VEC];  // two-level summation, as in gather_row
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) part[k] = 0.0f;
+            if (all_full) accumulate_chunk<T, VEC, LPR, true>(ls, X, g.ldx, my_col, my_w, cnt, part);
+            else accumulate_chunk<T, VEC, LPR, false>(ls, X, g.ldx, my_col, my_w, cnt, part);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) acc[k] += part[k];
+        }
+        Vec v;  // (whole vectors also where the row ends inside one: ldp is padded)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) v[k] = acc[k];
+        if (ls.live) *reinterpret_cast<Vec*>(l.partial + (unit * kClasses + cls) * l.ldp + ls.col0) = v;
+    }
+}
+
+// The rows of several segments: a wave adds a row's partial sums, its lane groups every second, fourth or eighth run of eight of them, and then their sums by a
+// __shfl_xor tree -- an order that depends on the row's length alone.  (A lane group a row, one run after the other, waited 110 us for the 1328 sums in classes of an 85 K-entry row.)
 template <typename T, int VEC, int LPR>
 __global__ __launch_bounds__(kBlock) void seg_reduce_kernel(const AggArgs g, const SegLists l)
 {
     typedef float Vec __attribute__((ext_vector_type(VEC), aligned(4)));
+    constexpr int kRun = 8;
     const int n_many = l.counts[2] < l.cap_many ? l.counts[2] : l.cap_many;
-    const int64_t i = (int64_t)blockIdx.x * (kBlock / LPR) + threadIdx.x / LPR;
-    if (i >= n_many) return;
-    const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, (int)threadIdx.x % LPR, g.D);
-    if (!ls.live) return;
-    const int64_t row = l.many_row[i];
-    const int n = (g.indptr[row + 1] - g.indptr[row] + kSegEntries - 1) / kSegEntries;
-    int64_t seg = l.many_seg[i];
-    const int64_t end = seg + n < l.cap_seg ? seg + n : l.cap_seg;
-    float acc[VEC];
+    const int lane = lane_id(), grp = lane / LPR;
+    const LaneSlice<T, VEC> ls((int)blockIdx.y, LPR, lane % LPR, g.D);
+    for (int64_t i = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; i < n_many; i += (int64_t)gridDim.x * (kBlock / kWave)) {
+        const int64_t row = l.many_row[i];
+        const int n = (g.indptr[row + 1] - g.indptr[row] + kSegEntries - 1) / kSegEntries;
+        const int64_t seg = l.many_seg[i], last = seg + n < l.cap_seg ? seg + n : l.cap_seg, end = last * l.classes;
+        float acc[VEC];
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
-    auto add = [&](const Vec& v) {
+        for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
+        auto add = [&](const Vec& v) {
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) acc[k] += v[k];
-    };
-    const float* p = l.partial + ls.col0;
-    for (; seg + 8 <= end; seg += 8) {
-        Vec v[8];
+            for (int k = 0; k < VEC; ++k) acc[k] += v[k];
+        };
+        const float* p = l.partial + ls.col0;
+        if (ls.live) {
+            for (int64_t at = seg * l.classes + grp * kRun; at < end; at += kWave / LPR * kRun) {
+                if (at + kRun <= end) {
+                    Vec v[kRun];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const Vec*>(p + (seg + j) * l.ldp);
+                    for (int j = 0; j < kRun; ++j) v[j] = *reinterpret_cast<const Vec*>(p + (at + j) * l.ldp);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) add(v[j]);
+                    for (int j = 0; j < kRun; ++j) add(v[j]);
+                } else {
+                    for (int64_t k = at; k < end; ++k) add(*reinterpret_cast<const Vec*>(p + k * l.ldp));
+                }
+            }
+        }
+#pragma unroll
+        for (int d = LPR; d < kWave; d <<= 1)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) acc[k] += __shfl_xor(acc[k], d, kWave);
+        if (grp == 0 && ls.live) ls.store(static_cast<T*>(g.out) + row * g.ldo + ls.col0, acc);
     }
-    for (; seg < end; ++seg) add(*reinterpret_cast<const Vec*>(p + seg * l.ldp));
-    ls.store(static_cast<T*>(g.out) + row * g.ldo + ls.col0, acc);
 }
 
 
@@ -1598,18 +1752,26 @@ static void launch_seg_lists(const SegLists& l, hipStream_t stream, const AggArg
 
 // The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
 // for large inputs), else a workgroup per row.
+// Workgroups for what the device counts: as many as there may be, up to so many, which then take turns (empty launches of 32 K and twice 8 K workgroups took 20 us, of 8 K and twice 4 K within the runs' differences)
+static unsigned at_most(int64_t blocks, int64_t most) { return (unsigned)(blocks < most ? blocks : most); }
+
 template <typename T, int VEC, int LPR, int MODE>
 static void launch_long_rows(unsigned gy, hipStream_t stream, const AggArgs& g)
 {
     if constexpr (MODE != FGL_AGG_EDGE) {
         if (g.ws != nullptr) {
-            const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
+            const SegLists l = seg_lists_of(g, sizeof(T));
             if (g.order == nullptr) launch_seg_lists<0>(l, stream, g, nullptr, nullptr);  // (else listed with the rows' order)
             // (a unit has more than kLongRowEntries entries, or is one of at most two per kSegEntries > 2 * kLongRowEntries of them)
             static_assert(kSegEntries > 2 * kLongRowEntries, "the bound on the number of units");
             hipLaunchKernelGGL((aggregate_segments_kernel<T, VEC, LPR, MODE>), dim3((unsigned)ceil_div(l.cap_one, kBlock / kWave), gy),
                                dim3(kBlock), 0, stream, g, l);
-            hipLaunchKernelGGL((seg_reduce_kernel<T, VEC, LPR>), dim3((unsigned)ceil_div(l.cap_many, kBlock / LPR), gy), dim3(kBlock), 0, stream, g, l);
+            if (l.classes > 1) {
+                hipLaunchKernelGGL(seg_classes_kernel, dim3(at_most(ceil_div(l.cap_seg, kBlock / kWave), 4096)), dim3(kBlock), 0, stream, g, l);
+                hipLaunchKernelGGL((aggregate_classes_kernel<T, VEC, LPR, MODE>), dim3(at_most(ceil_div(l.cap_seg, kBlock / LPR), 1024) * kClasses, gy), dim3(kBlock), 0,
+                                   stream, g, l);
+            }
+            hipLaunchKernelGGL((seg_reduce_kernel<T, VEC, LPR>), dim3(at_most(ceil_div(l.cap_many, kBlock / kWave), 4096), gy), dim3(kBlock), 0, stream, g, l);
             return;
         }
     }
@@ -1645,9 +1807,9 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
     if constexpr (LPR <= 32) {
         if (second_pass && g.ws != nullptr && mode != FGL_AGG_EDGE && g.n_rows_max >= kOrderMinRows) {
             // (in the place of the partial sums, which the launches behind the gather fill; the launch that lists the long rows finds the order)
-            const SegLists l = seg_lists(g.ws, g.n_entries_max, g.D, nullptr);
+            const SegLists l = seg_lists_of(g, sizeof(T));
             const int tile = seg_tile(g.n_rows_max);
-            if ((int64_t)l.cap_seg * l.ldp >= g.n_rows_max + ceil_div(g.n_rows_max, tile)) {
+            if ((int64_t)l.cap_seg * l.ldp * l.classes >= g.n_rows_max + ceil_div(g.n_rows_max, tile)) {
                 int32_t* order = reinterpret_cast<int32_t*>(l.partial);
                 launch_seg_lists<kWave / LPR>(l, stream, g, order, order + g.n_rows_max);
                 g.order = order;
@@ -1896,8 +2058,9 @@ FGL_EXPORT size_t fgl_aggregate_workspace_bytes(int64_t n_entries_max, int D, in
     if (n_entries_max < kSegMinEntries || n_entries_max > 0x7FFFFFFF || D < 1 || mode == FGL_AGG_EDGE) return 0;
     if (longest_row_max >= 0 && longest_row_max <= kLongRowEntries) return 0;
     size_t bytes = 0;
-    (void)seg_lists(nullptr, n_entries_max, D, &bytes);
-    return bytes;
+    (void)seg_lists(nullptr, n_entries_max, D, false, &bytes);
+    const size_t in_classes = class_bytes(n_entries_max, D);
+    return bytes > in_classes ? bytes : in_classes;
 }
 
 FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indices, int64_t n_rows_max,

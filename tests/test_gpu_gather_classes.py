@@ -1,0 +1,58 @@
+"""Long rows of large graphs, gathered class by class of their neighbours (csrc/fgl_aggregate.hip): rows around the limits of the long row, the row in classes and
+the segment, in every mode, against float64; the sizes on either side of the rule; the same bits on every run."""
+import pytest
+import torch
+
+from fastgl import ops
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [0, 1, 127, 128, 129, 255, 256, 257, 300, 511, 512, 513, 1023, 1024, 1025, 4097, 9000, 85_000]
+
+
+def _graph(cuda, n_rows, rest, seed):
+    """The lengths above at both ends of the rows and `rest` entries in every other one; half of the neighbours are among a few hundred ids."""
+    gen = torch.Generator(device=cuda).manual_seed(seed)
+    lengths = torch.full((n_rows,), rest, dtype=torch.int64)
+    lengths[:len(LENGTHS)] = torch.tensor(LENGTHS)
+    lengths[-len(LENGTHS):] = torch.tensor(LENGTHS[::-1])
+    ptr = torch.zeros(n_rows + 1, dtype=torch.int64)
+    ptr[1:] = lengths.cumsum(0)
+    n = int(ptr[-1])
+    idx = torch.randint(0, n_rows, (n,), generator=gen, device=cuda)
+    few = torch.randint(0, 300, (n,), generator=gen, device=cuda)
+    idx = torch.where(torch.rand(n, generator=gen, device=cuda) < 0.5, few, idx).int()
+    return ptr.int().to(cuda), idx, lengths
+
+
+@pytest.mark.parametrize("n_rows,rest,D,dtype", [(280_000, 46, 64, torch.float32), (260_000, 50, 65, torch.float32), (270_000, 47, 130, torch.float32),
+                                                 (280_000, 46, 602, torch.float32), (270_000, 48, 128, torch.bfloat16),
+                                                 (280_000, 40, 64, torch.float32), (280_000, 46, 60, torch.float32), (280_000, 46, 64, torch.bfloat16)])
+def test_against_float64(cuda, n_rows, rest, D, dtype):
+    print("classes", n_rows, rest, D, dtype, flush=True)
+    ptr, idx, lengths = _graph(cuda, n_rows, rest, D)
+    gen = torch.Generator(device=cuda).manual_seed(D + 1)
+    x = torch.randn((n_rows, D), generator=gen, device=cuda).to(dtype)
+    row_norm, col_norm = (torch.randint(1, 50, (n_rows,), generator=gen, device=cuda, dtype=torch.int32) for _ in range(2))
+    rows = torch.cat((torch.arange(len(LENGTHS) + 5), torch.arange(n_rows - len(LENGTHS), n_rows)))
+    first, n = ptr.cpu().long()[rows], lengths[rows]
+    at = torch.cat([torch.arange(f, f + k) for f, k in zip(first.tolist(), n.tolist())]).to(cuda)  # the rows' entries
+    which = torch.repeat_interleave(torch.arange(rows.numel()), n).to(cuda)
+    n, rows, c = n.to(cuda), rows.to(cuda), idx[at].long()
+    for mode in ("sum", "mean", "gcn", "colmean"):
+        norms = dict(row_norm=row_norm if mode == "gcn" else None, col_norm=col_norm if mode in ("gcn", "colmean") else None)
+        got = ops.aggregate(ptr, idx, x, mode=mode, zero_policy="zeros", **norms)
+        assert torch.equal(got, ops.aggregate(ptr, idx, x, mode=mode, zero_policy="zeros", **norms))
+        w = torch.ones(at.numel(), dtype=torch.float64, device=cuda)
+        if mode == "mean":
+            w = 1 / n[which].double()
+        elif mode == "gcn":
+            w = (1 / col_norm[c].double()).sqrt() / row_norm[rows][which].double().sqrt()
+        elif mode == "colmean":
+            w = 1 / col_norm[c].double()
+        terms = w[:, None] * x[c].double()
+        want = torch.stack([t.sum(0) for t in terms.split(n.tolist())])
+        size = torch.stack([t.abs().sum(0) for t in terms.split(n.tolist())])
+        # a weight is three roundings, a term one, and a sum at most 64 in a chunk, n / 16 chunks, eight classes and n / 512 segments deep
+        bound = (80 + n.double()[:, None] / 16) * 2.0 ** -24 * size + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+        assert bool(((got[rows].double() - want).abs() <= bound).all()), mode
