@@ -22,7 +22,7 @@
 //     Within a bucket a column is 16 bits.  Traffic: 2 reads of the ids, 2 writes and reads of the rows, 1 write and 2 reads of
 //     half the columns.
 //     (54 M entries of a 2.4 M-node graph, hubs of 85 K, us: counts, with an atomic per entry 5900 / 13200 -- unordered / sorted
-//     ids --, with 4-byte stores all over the buckets 499 / 674, now 310 / 270; transpose 24700, 1550, now 700.)
+//     ids --, with 4-byte stores all over the buckets 499 / 674, now 276 / 177; transpose 24700, 1550, now 700.)
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_tile_rows.hpp"
@@ -100,6 +100,7 @@ struct BucketArgs {
     int64_t tiles;               // of kBucketTile entries
     int32_t* hist;               // [bucket][tile] counts, then their prefix sums (+ 1 entry: the total)
     int32_t* tile_row;           // [tile] the row that holds the tile's first entry
+    int32_t* direct;             // [tile] counting only: 1 where bucket_hist_kernel has counted the tile's entries already
     uint16_t* b_col;             // entries by bucket: column within the bucket, row, position in ids
     int32_t* b_row;
     int32_t* b_edge;
@@ -159,29 +160,88 @@ __device__ __forceinline__ void load_columns(const BucketArgs& g, int64_t first,
         if (c[j] >= g.n_cols) c[j] = -1;
 }
 
-// (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's rows -- would otherwise be 64
+// A tile's entries by bucket.  (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's rows -- would otherwise be 64
 // updates of one counter at a time, one after the other.)
+// DIRECT (counting only): a tile that is runs of equal ids -- at most four begin inside the sixteen entries of seven lanes in eight of its first wave: the destinations of an edge list in order -- is
+// counted here,
+// one atomic a run in device memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.  (Whole counts, us, before / with it: 54 M ids
+// over 2.4 M counters, sorted 276 / 177, in no order 275 / 276; 20 M over 100 K, sorted 82 / 42; 5 M over 600 K, sorted 42 / 37, in no order 38.3 / 38.8; 8 M over 2.4 M, sorted,
+// three and a third a run and so not direct, 67.7 / 68.7.)
+template <bool DIRECT>
 __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
 {
     __shared__ int s_cnt[kMaxBuckets];
     const int64_t n = bucket_entries(g);
     const int64_t tile = xcd_tile(g.tiles);
     if (tile < 0) return;
-    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) s_cnt[b] = 0;
-    __syncthreads();
+    const int tid = (int)threadIdx.x;
+    for (int b = tid; b < g.buckets; b += kBucketBlock) s_cnt[b] = 0;
     int32_t c[kBucketItems];
-    load_columns(g, tile * kBucketTile + (int64_t)threadIdx.x * kBucketItems, n, c);
-    int run = 0;
+    load_columns(g, tile * kBucketTile + (int64_t)tid * kBucketItems, n, c);
+    bool direct = false;
+    if constexpr (DIRECT) {
+        // one wave looks at its 1024 entries, for all: what the others would see costs an input in no order 2 % of the whole count
+        __shared__ int s_direct;
+        if (tid < kWave) {
+            int begin = 0;
 #pragma unroll
-    for (int j = 0; j < kBucketItems; ++j) {
-        ++run;
-        const int b = c[j] >> g.width_log;  // (-1 stays -1)
-        if (j + 1 < kBucketItems && c[j + 1] >> g.width_log == b) continue;
-        if (b >= 0) atomicAdd(&s_cnt[b], run);
-        run = 0;
+            for (int j = 1; j < kBucketItems; ++j) begin += c[j] != c[j - 1];
+            const int few = __popcll(__ballot(begin <= kBucketItems / 4));
+            if (tid == 0) {
+                s_direct = few >= kWave / 8 * 7;
+                g.direct[tile] = few >= kWave / 8 * 7;
+            }
+        }
+        __syncthreads();
+        direct = s_direct != 0;
+        if (direct) {  // (the whole workgroup)
+            constexpr int kWaves = kBucketBlock / kWave;
+            __shared__ int s_last[kBucketBlock], s_first[kWaves];
+            const int lane = lane_id(), wave = tid / kWave;
+            s_last[tid] = c[kBucketItems - 1];
+            __syncthreads();
+            uint32_t heads = 0;  // where runs begin: bit j for the lane's entry j
+#pragma unroll
+            for (int j = 1; j < kBucketItems; ++j) heads |= c[j] != c[j - 1] ? 1u << j : 0u;
+            if (tid == 0 || c[0] != s_last[tid - 1]) heads |= 1u;
+            // the first of them, as a place in the tile, in this lane or behind it in the wave
+            int first = heads != 0 ? tid * kBucketItems + __ffs((int)heads) - 1 : kBucketTile;
+#pragma unroll
+            for (int d = 1; d < kWave; d <<= 1) {
+                const int t = __shfl_down(first, d, kWave);
+                if (lane + d < kWave && t < first) first = t;
+            }
+            if (lane == 0) s_first[wave] = first;
+            __syncthreads();
+            int next = __shfl_down(first, 1, kWave);
+            if (lane == kWave - 1) next = kBucketTile;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w)
+                if (w > wave && s_first[w] < next) next = s_first[w];
+#pragma unroll
+            for (int j = kBucketItems - 1; j >= 0; --j) {
+                if ((heads >> j & 1) == 0) continue;
+                const int at = tid * kBucketItems + j;
+                if (c[j] >= 0) atomicAdd(&g.counts[c[j]], next - at);
+                next = at;
+            }
+        }
+    } else {
+        __syncthreads();
+    }
+    if (!direct) {
+        int run = 0;
+#pragma unroll
+        for (int j = 0; j < kBucketItems; ++j) {
+            ++run;
+            const int b = c[j] >> g.width_log;  // (-1 stays -1)
+            if (j + 1 < kBucketItems && c[j + 1] >> g.width_log == b) continue;
+            if (b >= 0) atomicAdd(&s_cnt[b], run);
+            run = 0;
+        }
     }
     __syncthreads();
-    for (int b = (int)threadIdx.x; b < g.buckets; b += kBucketBlock) g.hist[(int64_t)b * g.tiles + tile] = s_cnt[b];
+    for (int b = tid; b < g.buckets; b += kBucketBlock) g.hist[(int64_t)b * g.tiles + tile] = s_cnt[b];
 }
 
 // Every entry to its bucket's place.  A tile is put in order in LDS first, so that a bucket's entries leave as runs (7 of a tile over
@@ -198,9 +258,11 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_scatter_kernel(const Buck
     const int64_t n = bucket_entries(g);
     const int64_t tile = xcd_tile(g.tiles), e0 = tile * kBucketTile;
     if (tile < 0 || e0 >= n) return;  // (uniform over the workgroup)
+    const int direct = ROWS ? 0 : g.direct[tile];
     const int tid = (int)threadIdx.x, at = tid * kBucketItems;
     int32_t c[kBucketItems], r[ROWS ? kBucketItems : 1];
     load_columns(g, e0 + at, n, c);
+    if (direct) return;  // (counted already; asked for together with the entries, so that the others do not wait twice)
     if constexpr (ROWS) {
         tile_rows<NT, kBucketItems>(g.indptr, g.n_rows, g.tile_row, tile, n, s_buf, s_delta);
 #pragma unroll
@@ -542,6 +604,7 @@ static void bucket_layout(int64_t n_entries, int64_t n_cols, bool rows, bool edg
     g->hist = c.take<int32_t>((size_t)(g->buckets * g->tiles + 1));
     g->segments = c.take<int32_t>((size_t)(1 + 3 * max_segments));
     g->b_col = c.take<uint16_t>(align_up((size_t)n_entries, 8));  // (read in 16-byte pieces)
+    g->direct = rows ? nullptr : c.take<int32_t>((size_t)g->tiles);
     if (rows) {
         g->tile_row = c.take<int32_t>((size_t)g->tiles);
         g->b_row = c.take<int32_t>((size_t)n_entries);
@@ -567,7 +630,8 @@ static int launch_partition(const BucketArgs& g, bool rows, bool edges, hipStrea
     if (blocks > 8192) blocks = 8192;
     const unsigned tiles = (unsigned)align_up(g.tiles, 8);
     hipLaunchKernelGGL(bucket_init_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, g);
-    hipLaunchKernelGGL(bucket_hist_kernel, dim3(tiles), dim3(kBucketBlock), 0, stream, g);
+    if (rows) hipLaunchKernelGGL(bucket_hist_kernel<false>, dim3(tiles), dim3(kBucketBlock), 0, stream, g);
+    else hipLaunchKernelGGL(bucket_hist_kernel<true>, dim3(tiles), dim3(kBucketBlock), 0, stream, g);
     FGL_CHECK_LAUNCH("bucket_hist_kernel");
     const int64_t n_hist = g.buckets * g.tiles;
     // (the entries are not written yet: the scan's scratch -- a few words per tile -- fits where they go)
