@@ -1037,8 +1037,13 @@ __global__ __launch_bounds__(kLongBlock) void aggregate_long_rows_kernel(const A
             float acc[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
-            for (int64_t base = (int64_t)a + (int64_t)grp * LPR; base < b; base += (int64_t)kGroups * LPR) {
-                const int cnt = (b - base) < LPR ? (int)(b - base) : LPR;
+            // chunks of at most LPR entries, of one length so that the groups share the list evenly: 140 entries for eight groups of 64 lanes are five
+            // chunks of 32, two loads of sixteen rows after each other instead of the four of three chunks of 64
+            // (the hubs of a sampled block's transpose: 256 fp32 columns 17.1 -> 11.7 us, with weights 17.8 -> 14.0, bf16 13.7 -> 11.1)
+            const int rounds = (b - a - 1) / kLongBlock + 1;
+            const int chunk = LPR <= kInFlight ? LPR : ((b - a - 1) / (kGroups * rounds) + kInFlight) / kInFlight * kInFlight;
+            for (int64_t base = (int64_t)a + (int64_t)grp * chunk; base < b; base += (int64_t)kGroups * chunk) {
+                const int cnt = (b - base) < chunk ? (int)(b - base) : chunk;
                 int my_col = 0;
                 int my_eid = 0;     // FGL_AGG_EDGE: which row of edge_w the entry uses
                 float my_w = 0.0f;  // the other modes: the entry's weight
