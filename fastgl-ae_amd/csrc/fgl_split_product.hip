@@ -370,7 +370,9 @@ static int launch_split_product(RowProductArgs g, hipStream_t stream)
     // eight waves a CU (two a SIMD, as the registers allow), in as many workgroups as their LDS allows
     int64_t per_cu = kSpLds / (int64_t)lds;
     if (per_cu > 8 / W) per_cu = 8 / W;
-    const int64_t want = ceil_div(ceil_div(g.m, 32), W), slots = ceil_div(256 * per_cu / g.tiles_n, 8) * 8;
+    const int64_t want = ceil_div(ceil_div(g.m, 32), W);
+    int64_t slots = ceil_div(256 * per_cu / g.tiles_n, 8) * 8;
+    if (slots < 8) slots = 8;  // (more tiles along n than there is room for at once)
     g.row_blocks = want < slots ? want : slots;
     const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
     FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");

@@ -3,6 +3,7 @@ columns a workgroup, steps of 16 k that are odd or even in number and end with k
 import pytest
 import torch
 
+from fastgl import _lib as L
 from fastgl import ops
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +88,22 @@ def test_products_beyond_the_general_line(cuda, m, k, n, split):
         for rows in (slice(0, 1000), slice(m - 1000, m)):
             x = a[rows].double()
             _check(got[rows], x @ w, (k + 2) * 2.0 ** -24 * (x.abs() @ w.abs()))
+
+
+@pytest.mark.parametrize("m,k,n", [(2000, 256, 16384), (2000, 256, 16385), (2037, 256, 20000), (2000, 100, 32768), (2000, 100, 32769), (2048, 100, 40000),
+                                   (2000, 832, 8192), (2000, 832, 8193), (2000, 500, 20000), (2000, 100, 65536)])
+def test_more_tiles_along_n_than_the_chip_holds(cuda, m, k, n):
+    """Products with so many columns that the workgroups of one row tile each are more than the chip takes at a time."""
+    print("wide product", m, k, n, flush=True)
+    gen = torch.Generator(device=cuda).manual_seed(n)
+    a = torch.randn((m, k), generator=gen, device=cuda)
+    lib = L.lib()
+    for transposed in (False, True):
+        b = torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
+        w = (b.t() if transposed else b).double()
+        want, bound = a.double() @ w, (k + 2) * 2.0 ** -24 * (a.double().abs() @ w.abs())
+        _check(ops.row_product(a, b, transposed), want, bound)
+        got = torch.full((m, n), float("nan"), device=cuda)  # (the C entry itself: from Python some of these are the library's)
+        L.check(lib.fgl_row_product(a.data_ptr(), k, b.data_ptr(), k if transposed else n, int(transposed), m, k, n, L.F32, None, got.data_ptr(), n,
+                                    L.stream_handle()))
+        _check(got, want, bound)
