@@ -1153,7 +1153,8 @@ struct SegLists {
     int32_t cap_seg, cap_one, cap_many;
     int one_entries;    // rows of up to so many entries are rows of one segment, which need no second sum
     int classes;        // 1, or kClasses: segments are gathered class by class (see below)
-    int32_t* class_ids; // then: the segments' neighbour ids, class after class within each, at the places where its entries lie in `indices`
+    int32_t* class_ids; // then: the segments' neighbour ids, class after class within each, where its entries lie among those of the rows (indptr[0] on)
+    int64_t class_cap;  // of them
     ClassEnds* class_ends;
 };
 
@@ -1198,6 +1199,7 @@ static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, bool classes, 
     l.many_seg = c.take<int32_t>((size_t)l.cap_many);
     l.partial = c.take<float>((size_t)l.cap_seg * (size_t)l.ldp * (size_t)l.classes);
     l.class_ids = classes ? c.take<int32_t>((size_t)n_entries_max) : nullptr;
+    l.class_cap = classes ? n_entries_max : 0;
     l.class_ends = classes ? c.take<ClassEnds>((size_t)l.cap_seg) : nullptr;
     if (bytes) *bytes = c.used();
     return l;
@@ -1459,7 +1461,9 @@ __global__ __launch_bounds__(kBlock) void seg_classes_kernel(const AggArgs g, co
     const int lane = lane_id();
     for (int64_t unit = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; unit < n_seg; unit += (int64_t)gridDim.x * (kBlock / kWave)) {
         const int a = l.seg_first[unit], row_b = g.indptr[l.seg_row[unit] + 1];
-        const int n = row_b - a < kSegEntries ? row_b - a : kSegEntries;
+        const int64_t place = (int64_t)a - g.indptr[0];  // (the rows may be a stretch of a larger CSR)
+        int n = row_b - a < kSegEntries ? row_b - a : kSegEntries;
+        if (place + n > l.class_cap) n = 0;  // (more entries than the caller's bound says: nothing is written past it)
         const int rounds = __builtin_amdgcn_readfirstlane((n + kWave - 1) / kWave);
         int id[kRounds];
 #pragma unroll
@@ -1499,7 +1503,7 @@ __global__ __launch_bounds__(kBlock) void seg_classes_kernel(const AggArgs g, co
             if (j >= rounds) continue;
             const int c = neighbour_class(id[j]);
             const int at = __shfl(first, c, 8) + __popcll(of_class(j, c) & before);
-            if (j * kWave + lane < n) l.class_ids[a + at] = id[j];
+            if (j * kWave + lane < n) l.class_ids[place + at] = id[j];
             first += __popcll(of_class(j, lane & 7));
         }
     }
@@ -1520,7 +1524,7 @@ __global__ __launch_bounds__(kBlock) void aggregate_classes_kernel(const AggArgs
     for (int64_t unit = (int64_t)(blockIdx.x / kClasses) * (kBlock / LPR) + threadIdx.x / LPR; unit < n_seg; unit += (int64_t)(gridDim.x / kClasses) * (kBlock / LPR)) {
         const int row = l.seg_row[unit];
         const int entries = g.indptr[row + 1] - g.indptr[row];
-        const int first = l.seg_first[unit];
+        const int first = l.seg_first[unit] - g.indptr[0];  // (of class_ids, as seg_classes_kernel has placed them)
         const int a = first + (cls > 0 ? l.class_ends[unit].end[cls - 1] : 0), b = first + l.class_ends[unit].end[cls];
         float acc[VEC];
 #pragma unroll

@@ -3,6 +3,7 @@ the segment, in every mode, against float64; the sizes on either side of the rul
 import pytest
 import torch
 
+from fastgl import _lib as L
 from fastgl import ops
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,21 @@ def test_against_float64(cuda, n_rows, rest, D, dtype):
         # a weight is three roundings, a term one, and a sum at most 64 in a chunk, n / 16 chunks, eight classes and n / 512 segments deep
         bound = (80 + n.double()[:, None] / 16) * 2.0 ** -24 * size + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
         assert bool(((got[rows].double() - want).abs() <= bound).all()), mode
+
+
+def test_rows_of_a_larger_csr(cuda):
+    """The C entry over a stretch of a CSR's rows, with the entries of that stretch as their bound: offsets that begin far beyond the scratch's ids."""
+    lib, D, first = L.lib(), 64, 270_000
+    ptr, idx, lengths = _graph(cuda, 2 * first, 48, 5)
+    x = torch.randn((2 * first, D), generator=torch.Generator(device=cuda).manual_seed(6), device=cuda)
+    rows, n = ptr[first:], int(ptr[-1] - ptr[first])
+    assert n < int(ptr[first]) + 100_000 and n > 12_582_912
+    out = torch.empty((first, D), device=cuda)
+    ws_bytes = lib.fgl_aggregate_workspace_bytes(n, D, L.AGG_SUM, -1)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=cuda)
+    L.check(lib.fgl_aggregate_ws(rows.data_ptr(), idx.data_ptr(), first, None, x.data_ptr(), D, D, L.F32, L.AGG_SUM, L.ZERO_ZEROS, None, None, None, 1, None,
+                                 -1, None, n, out.data_ptr(), D, ws.data_ptr(), ws_bytes, L.stream_handle()))
+    for r in range(2 * first - len(LENGTHS), 2 * first):
+        terms = x[idx[int(ptr[r]):int(ptr[r + 1])].long()].double()
+        bound = (80 + lengths[r].item() / 16) * 2.0 ** -24 * terms.abs().sum(0)
+        assert bool(((out[r - first].double() - terms.sum(0)).abs() <= bound).all())
