@@ -16,6 +16,9 @@ int launch_tile_prefix(const int32_t* tile_sums, int n_tiles, int32_t* tile_pref
                        hipStream_t stream, int32_t* readback = nullptr, const uint32_t* d_status = nullptr);
 int launch_fill_u32(uint32_t* p, int64_t n, uint32_t value, hipStream_t stream);
 
+// which kernel the calling thread's last dense product was formed by (fgl_product_last_kernel)
+void note_product(const char* kernel);
+
 // Row start of a node whose id lies outside the graph / whose insert found the table full: how a launch that
 // must not touch the status word hands the error to the next one that reads the entry.
 constexpr int64_t kRowBadId = -1;

@@ -331,6 +331,10 @@ static int launch_row_product_any(const RowProductArgs& g, bool vectors, hipStre
 
 using namespace fgl;
 
+static thread_local const char* g_product = "";
+void fgl::note_product(const char* kernel) { g_product = kernel; }
+FGL_EXPORT const char* fgl_product_last_kernel(void) { return g_product; }
+
 template <int FORM>
 static int row_product(const RowProductSide& one, const RowProductSide& two, int b_transposed, int64_t m, int n, int dtype, const void* d_bias,
                        void* d_c, int64_t ldc, void* stream)
@@ -355,7 +359,9 @@ static int row_product(const RowProductSide& one, const RowProductSide& two, int
     }
     if (m == 0) return FGL_OK;
     hipStream_t s = as_stream(stream);
-    if (dtype == FGL_F32 && split_product_pays(g)) return split_product(g, b_transposed != 0, FORM, s);
+    const bool split = dtype == FGL_F32 && split_product_pays(g);
+    note_product(split ? "split_product_kernel" : "row_product_kernel");
+    if (split) return split_product(g, b_transposed != 0, FORM, s);
     if (dtype == FGL_F32) return b_transposed ? launch_row_product_any<float, true, FORM>(g, true, s) : launch_row_product_any<float, false, FORM>(g, true, s);
     return b_transposed ? launch_row_product_any<uint16_t, true, FORM>(g, vectors, s) : launch_row_product_any<uint16_t, false, FORM>(g, vectors, s);
 }

@@ -390,13 +390,21 @@ static int sp_tiles(const RowProductArgs& g)
     return g.n > 32 && sp_lds(g, 2) <= (size_t)kSpLds ? 2 : 1;
 }
 
-// Whether the split pays.  Below the line the fp32 instructions' kernel is ahead, which has nothing to stage first: us, that one / this, 64 x 64: 32 K rows 7 / 8,
-// 64 K 12 / 10; 100 x 64: 16 K 6 / 8, 32 K 9 / 9; 100 x 256: 4000 6 / 8, 8000 9 / 9, 16 K 15 / 12; 128 x 128: 8000 6 / 8, 16 K 10 / 9; 256 x 256: 4000 9 / 13, 8000 16 / 14;
-// 300 x 64: 16 K 11 / 17, 32 K 19 / 18; 602 x 256: 4000 16 / 21, 8000 32 / 25; 256 x 602: 2000 15 / 15, 4000 25 / 16.
+// Whether the split pays, against the fp32 instructions' kernel, which has nothing to stage first and pads less.  A step here is 32 k and 32 to 128 columns: what they
+// pad makes the line higher (us, that kernel / this: 909 K x 8 x 33 42 / 70, 454 K x 8 x 66 31 / 60, 234 K x 16 x 128 27 / 29, 106 K x 33 x 66 18 / 28, but 140 K x 33 x 100
+// 30 / 24), and up to two steps it is higher by another quarter (54 K x 64 x 128 17 / 21, 109 K x 64 x 128 30 / 27).  Otherwise it lies at 4.3e8 multiplications: 100 x 64:
+// 39 K rows 13 / 14, 62 K 15 / 13; 100 x 256: 9800 13 / 12, 27 K 22 / 20; 200 x 128: 13 K 12 / 14, 20 K 21 / 15; 256 x 66: 25 K 21 / 18; 602 x 256: 6400 30 / 24.
+// Workgroups of one row block go to one XCD, eight blocks at a time, so that fewer than 2000 rows leave XCDs idle: 1000 x 256 x 4000 22 / 36, 500 x 602 x 16000 192 / 356,
+// 250 x 832 x 30000 521 / 909, 2000 x 256 x 4000 44 / 40.  Results as few as 1.6e6 take that many rows' worth twice: 3000 x 602 x 602 31 / 44, 4000 x 400 x 400 19 / 21.
 bool split_product_pays(const RowProductArgs& g)
 {
+    const int k = g.side[0].k + g.side[1].k;
+    if (sp_lds(g, 1) > (size_t)kSpLds || k <= 32 || g.m < 2000) return false;
     const double outputs = (double)g.m * g.n;
-    return sp_lds(g, 1) <= (size_t)kSpLds && outputs >= 1.6e6 && outputs * (g.side[0].k + g.side[1].k) >= 2e8;
+    if (outputs < (g.m < 5000 ? 2.1e6 : 1.6e6)) return false;
+    const int nt = sp_tiles(g);
+    const double padded_k = 32.0 * (sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)), wide = (double)(ceil_div(g.n, 32 * nt) * 32 * nt), narrow = (double)(ceil_div(g.n, 32) * 32);
+    return outputs * k >= (k <= 64 ? 5e8 : 4.3e8) * (padded_k / k) * (wide / narrow);
 }
 
 template <bool BT, int FORM>

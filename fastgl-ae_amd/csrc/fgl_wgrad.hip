@@ -592,6 +592,7 @@ FGL_EXPORT int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, in
     g.splits = p.splits; g.k_per_split = p.k_per_split; g.partial = static_cast<float*>(d_ws); g.c = d_c; g.ldc = ldc;
     g.sum_a = d_sum_a; g.partial_sum = reinterpret_cast<float*>(static_cast<char*>(d_ws) + p.sum_offset);
     hipStream_t s = as_stream(stream);
+    note_product(split ? "wgrad_kernel in parts" : "wgrad_kernel");
     if (split) return launch_wgrad<float, 2, 2, true>(g, s);  // (whoever is 128 wide in fours or 64 in twos is whole in twos)
     if (dtype == FGL_F32) return launch_wgrad_any<float>(p, g, s);
     return launch_wgrad_any<uint16_t>(p, g, s);

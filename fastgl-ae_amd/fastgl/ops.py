@@ -425,9 +425,14 @@ def _forms_split_product(a, b, transposed, m, k, n):
     and n = 64, 100, 128, 256, 300 0.5 .. 0.95 in both layouts (2.4 M x 100 x 64 338 / 512 us, x 64 x 100 325 / 627); but n = 66, which takes two workgroups' columns, 1.03 .. 1.09, n = 160,
     which takes three and is whole vectors to the library, 1.06 .. 1.18 from k = 200 on, and n = 33 and 47 1.02 .. 1.11 from k = 384 on.  Wide weights: 256 x 602
     N 0.84 / 0.76 / 0.58, T 0.98 / 0.71 / 0.71 (8192 / 20 K / 60 K rows), 400 x 300 0.61 / 0.49 / 0.77, 300 x 400 0.85 / 0.88 / 0.80; but 4000 rows of these two, fewer
-    than 2e6 results, 1.01 .. 1.16, and a k beyond 400, of which only 32 columns at a time fit, 0.9 .. 1.2 (602 x 256: 0.96 .. 1.10)."""
-    if not (a.dtype == torch.float32 and 32 < k <= 400 and m * n >= 2 * 10 ** 6 and not 64 < n < 72 and not (k > 128 and 128 < n <= 160) and
+    than 2.1e6 results, 1.01 .. 1.16, and a k beyond 400, of which only 32 columns at a time fit, 0.9 .. 1.2 (602 x 256: 0.96 .. 1.10).  From 4000 rows on, up to 30000 columns,
+    0.5 .. 0.83; fewer where they fill the XCDs' turns, 2048 rows each, 1024 up to k = 192 (2000 rows: k = 33 .. 400 0.6 .. 0.95; 3000 rows: k = 33 .. 100 0.56 .. 0.9, but
+    200 and 256 up to 1.1; 1500 rows up to 1.3, 1000 rows up to 1.5, 250 rows 3 .. 6)."""
+    if not (a.dtype == torch.float32 and 32 < k <= 400 and m * n >= 2.1e6 and not 64 < n < 72 and not (k > 128 and 128 < n <= 160) and
             not (k > 256 and n <= 48)):
+        return None
+    turn = 1024 if k <= 192 else 2048
+    if m < 2000 or (m < 4000 and 5 * m < 4 * turn * -(-m // turn)):
         return None
     return _product_operands(a, b, transposed, m, k, n)
 

@@ -440,6 +440,10 @@ size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n);
 int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int64_t k, int m, int n, int dtype,
                     void* d_c, int64_t ldc, void* d_sum_a, void* d_ws, size_t ws_bytes, void* stream);
 
+/* Which kernel formed the calling thread's last fgl_row_product*, fgl_weight_grad result, as text ("split_product_kernel",
+ * "row_product_kernel", "wgrad_kernel in parts", "wgrad_kernel"): for benchmark records and bug reports. */
+const char* fgl_product_last_kernel(void);
+
 /* ---------------------------------------------------------------------------------
  * Seeded R-MAT key generator for the synthetic graphs (a=.57 b=.19 c=.19 d=.05).
  * For draw e in [first_edge, first_edge+n_edges): writes the two symmetrised keys

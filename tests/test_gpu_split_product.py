@@ -8,9 +8,15 @@ from fastgl import ops
 
 pytestmark = pytest.mark.gpu
 
-# all large enough for the split (1.6e6 outputs, 2e8 multiplications): (rows, k, columns)
-SHAPES = [(1_600_001, 1, 128), (450_017, 7, 65), (210_031, 15, 64), (210_001, 16, 64), (400_033, 17, 31), (97_001, 33, 63), (50_001, 64, 129), (26_001, 100, 256),
-          (32_003, 96, 66), (6_417, 256, 300), (6_500, 416, 250), (6_500, 417, 250), (50_001, 832, 33), (50_001, 833, 33)]
+# (rows, k, columns) on both sides of the line between the kernels: those that are in parts, and those that the fp32 instructions form
+IN_PARTS = [(480_001, 33, 63), (180_001, 48, 129), (440_001, 49, 31), (100_001, 64, 129), (26_001, 100, 256), (95_003, 96, 66), (6_417, 256, 300), (6_500, 416, 250),
+            (6_500, 417, 250), (50_001, 832, 33), (2000, 256, 1100)]
+PLAIN = [(1_600_001, 1, 128), (450_017, 7, 65), (210_031, 15, 64), (210_001, 16, 64), (400_033, 17, 31), (97_001, 33, 63), (909_001, 8, 33), (50_001, 833, 33),
+         (1990, 256, 1200), (4000, 400, 400), (32_003, 96, 66)]
+
+
+def _kernel():
+    return L.lib().fgl_product_last_kernel()
 
 
 def _check(got, want, bound):
@@ -18,7 +24,7 @@ def _check(got, want, bound):
 
 
 @pytest.mark.parametrize("transposed", [False, True])
-@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("m,k,n", IN_PARTS + PLAIN)
 def test_split_product(cuda, m, k, n, transposed):
     print("split product", m, k, n, transposed, flush=True)
     gen = torch.Generator(device=cuda).manual_seed(m + k + n)
@@ -27,26 +33,33 @@ def test_split_product(cuda, m, k, n, transposed):
     b = torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
     bias = torch.randn(n, generator=gen, device=cuda)
     w = (b.t() if transposed else b).double()
-    got, plus = ops.row_product(a, b, transposed), ops.row_product(a, b, transposed, bias)
+    got, plus, through_c = ops.row_product(a, b, transposed), ops.row_product(a, b, transposed, bias), torch.empty((m, n), device=cuda)
+    L.check(L.lib().fgl_row_product(a.data_ptr(), k + 3, b.data_ptr(), b.size(1), int(transposed), m, k, n, L.F32, None, through_c.data_ptr(), n, L.stream_handle()))
+    assert _kernel() == (b"split_product_kernel" if (m, k, n) in IN_PARTS else b"row_product_kernel")
     for rows in (slice(0, 5000), slice(m // 2, m // 2 + 5000), slice(max(m - 5000, 0), m)):
         x = a[rows].double()
         # three parts of eight bits each: the products that are left out are below 2^-26, what a matrix instruction cuts off below 2^-25 of a chunk's sum, and k / 32
         # sums are rounded: within the (k + 2) 2^-24 of the magnitudes that k fp32 products and sums are given
         want, bound = x @ w, (k + 2) * 2.0 ** -24 * (x.abs() @ w.abs() + bias.double().abs())
         _check(got[rows], want, bound)
+        _check(through_c[rows], want, bound)
         _check(plus[rows], want + bias.double(), bound)
 
 
-@pytest.mark.parametrize("m,k0,k1,n", [(40_001, 100, 33, 65), (13_001, 256, 128, 128), (30_001, 16, 400, 64)])
+@pytest.mark.parametrize("m,k0,k1,n", [(120_001, 100, 33, 65), (13_501, 256, 128, 128), (30_001, 16, 400, 64), (160_001, 7, 100, 65), (150_001, 100, 1, 65),
+                                       (250_003, 15, 40, 64)])
 def test_sums_and_additions(cuda, m, k0, k1, n):
     gen = torch.Generator(device=cuda).manual_seed(m)
     a0, a1 = (torch.randn((m, k), generator=gen, device=cuda) for k in (k0, k1))
     b0, b1 = (torch.randn((n, k), generator=gen, device=cuda) for k in (k0, k1))
     bias, base = torch.randn(n, generator=gen, device=cuda), torch.randn((m + 5, n), generator=gen, device=cuda)
     want, size = a0.double() @ b0.double().t() + a1.double() @ b1.double().t() + bias.double(), a0.double().abs() @ b0.double().abs().t() + a1.double().abs() @ b1.double().abs().t()
-    _check(ops.row_product_sum(a0, b0, a1, b1, bias), want, (k0 + k1 + 2) * 2.0 ** -24 * (size + bias.double().abs()))
+    got = ops.row_product_sum(a0, b0, a1, b1, bias)
+    assert _kernel() == b"split_product_kernel"
+    _check(got, want, (k0 + k1 + 2) * 2.0 ** -24 * (size + bias.double().abs()))
     w = b0.t().contiguous()
     got = ops.row_product_add_(base.clone(), a0, w)
+    assert (_kernel() == b"split_product_kernel") == (k0 >= 100)
     assert torch.equal(got[m:], base[m:])
     size = a0.double().abs() @ w.double().abs() + base[:m].double().abs()
     _check(got[:m], a0.double() @ w.double() + base[:m].double(), (k0 + 2) * 2.0 ** -24 * size)
@@ -54,10 +67,11 @@ def test_sums_and_additions(cuda, m, k0, k1, n):
 
 @pytest.mark.parametrize("transposed", [False, True])
 def test_values_without_three_parts(cuda, transposed):
-    m, k, n = 40_000, 100, 64
+    m, k, n = 90_000, 100, 64
     gen = torch.Generator(device=cuda).manual_seed(5)
     a, b = torch.randn((m, k), generator=gen, device=cuda), torch.randn((n, k) if transposed else (k, n), generator=gen, device=cuda)
     clean = ops.row_product(a, b, transposed)
+    assert _kernel() == b"split_product_kernel"
     a[70, 3], a[1000, 99], a[1000, 5], a[5000, 0], a[5001, 98] = float("inf"), float("inf"), float("-inf"), float("nan"), float("-inf")
     a[9000] = 3.4e38 * torch.rand(k, generator=gen, device=cuda) ** 0.01  # (rounds to infinity in bf16)
     b.mul_(0.01)
@@ -75,6 +89,7 @@ def test_values_without_three_parts(cuda, transposed):
 
 
 @pytest.mark.parametrize("m,k,n,split", [(1_300_001, 100, 64, True), (1_300_001, 100, 66, False), (8192, 256, 602, True), (3000, 256, 602, False), (8192, 602, 256, False),
+                                         (2048, 256, 2000, True), (1999, 256, 2000, False), (3000, 256, 1000, False), (3000, 100, 2000, True), (200, 256, 20000, False),
                                          (300_001, 200, 160, False), (600_001, 384, 40, False)])
 def test_products_beyond_the_general_line(cuda, m, k, n, split):
     print("long or wide product", m, k, n, flush=True)
@@ -85,7 +100,8 @@ def test_products_beyond_the_general_line(cuda, m, k, n, split):
         assert ops._forms_row_product(a, b, transposed, m, k, n) is None
         assert (ops._forms_split_product(a, b, transposed, m, k, n) is not None) == split
         got, w = ops.row_product(a, b, transposed), (b.t() if transposed else b).double()
-        for rows in (slice(0, 1000), slice(m - 1000, m)):
+        assert not split or _kernel() == b"split_product_kernel"
+        for rows in (slice(0, 1000), slice(max(m - 1000, 0), m)):
             x = a[rows].double()
             _check(got[rows], x @ w, (k + 2) * 2.0 ** -24 * (x.abs() @ w.abs()))
 
@@ -106,4 +122,5 @@ def test_more_tiles_along_n_than_the_chip_holds(cuda, m, k, n):
         got = torch.full((m, n), float("nan"), device=cuda)  # (the C entry itself: from Python some of these are the library's)
         L.check(lib.fgl_row_product(a.data_ptr(), k, b.data_ptr(), k if transposed else n, int(transposed), m, k, n, L.F32, None, got.data_ptr(), n,
                                     L.stream_handle()))
+        assert _kernel() == b"split_product_kernel"
         _check(got, want, bound)
