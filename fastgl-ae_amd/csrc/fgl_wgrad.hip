@@ -489,9 +489,11 @@ struct WgradPlan {
 // Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
 // faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
 // reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 75 / 68, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237).
+// Fewer rows than a step has are the fp32 form's, whose sums of one and two products are the more exact ones: rms errors against 64 bits, fp32 / split, k = 1
+// 2.5e-8 / 3.5e-8, k = 2 3.1e-8 / 3.4e-8, k = 16 6.1e-8 / 3.4e-8, k = 17 6.5e-8 / 4.3e-8, k = 64 8.6e-8 / 5.5e-8.
 static bool wgrad_split_pays(int64_t k, int m, int n)
 {
-    return wgrad_vec(m, true, 4) * wgrad_vec(n, true, 4) >= 8 && (double)k * m * n <= 9e9;
+    return k >= 16 && wgrad_vec(m, true, 4) * wgrad_vec(n, true, 4) >= 8 && (double)k * m * n <= 9e9;
 }
 
 static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, bool split)

@@ -46,6 +46,12 @@ def test_split_product(cuda, m, k, n, transposed):
         _check(plus[rows], want + bias.double(), bound)
 
 
+def test_one_term_is_rounded_once(cuda):
+    gen = torch.Generator(device=cuda).manual_seed(2)
+    a, b = torch.randn((1_700_001, 1), generator=gen, device=cuda), torch.randn((1, 128), generator=gen, device=cuda)
+    assert torch.equal(ops.row_product(a, b), a * b)
+
+
 @pytest.mark.parametrize("m,k0,k1,n", [(120_001, 100, 33, 65), (13_501, 256, 128, 128), (30_001, 16, 400, 64), (160_001, 7, 100, 65), (150_001, 100, 1, 65),
                                        (250_003, 15, 40, 64)])
 def test_sums_and_additions(cuda, m, k0, k1, n):

@@ -3,12 +3,13 @@ with several rounds of workgroups, strided rows with their column sums, and valu
 import pytest
 import torch
 
+from fastgl import _lib as L
 from fastgl import ops
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n", [(100, 64), (65, 200), (256, 47), (127, 129), (602, 256)])
+@pytest.mark.parametrize("m,n", [(100, 64), (97, 200), (256, 47), (127, 129), (602, 256)])
 def test_against_float64(cuda, m, n):
     gen = torch.Generator(device=cuda).manual_seed(m + n)
     for k in (1, 15, 16, 17, 63, 65, 127, 129, 1001, 8192, 30011):
@@ -17,6 +18,8 @@ def test_against_float64(cuda, m, n):
         a.copy_(torch.randn((k, m), generator=gen, device=cuda))
         b = torch.randn((k, n), generator=gen, device=cuda)
         got, sums = ops.weight_grad(a, b, column_sums=True)
+        if m * n <= 65536 or k * k >= 256 * m * n:  # (else the library's)
+            assert L.lib().fgl_product_last_kernel() == (b"wgrad_kernel in parts" if k >= 16 else b"wgrad_kernel")
         want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
         # a step of 16 rows is right to 2^-24 of its largest sum or so, and k / 16 of them are added up in fp32: within (k / 16 + 16) 2^-24 of the magnitudes
         assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
@@ -25,11 +28,23 @@ def test_against_float64(cuda, m, n):
         assert torch.equal(got, again)
 
 
+@pytest.mark.parametrize("m,n", [(100, 256), (256, 47), (64, 128)])
+def test_few_rows_are_as_exact_as_fp32(cuda, m, n):
+    gen = torch.Generator(device=cuda).manual_seed(m)
+    a, b = torch.randn((15, m), generator=gen, device=cuda), torch.randn((15, n), generator=gen, device=cuda)
+    assert torch.equal(ops.weight_grad(a[:1], b[:1]), a[0][:, None] * b[0])  # one product, rounded once
+    for k in (2, 3, 15):
+        want, size = a[:k].double().t() @ b[:k].double(), a[:k].double().abs().t() @ b[:k].double().abs()
+        assert bool(((ops.weight_grad(a[:k], b[:k]).double() - want).abs() <= k * 2.0 ** -24 * size).all())  # (k products and k - 1 sums, each rounded once)
+
+
 def test_errors_do_not_add_up_over_the_rows(cuda):
     """2-norm of the error over the result's: with the cut of the matrix instructions on one side it was 7e-7 here, that of fp32 sums is 3e-7."""
     gen = torch.Generator(device=cuda).manual_seed(3)
     a, b = torch.randn((107_000, 100), generator=gen, device=cuda), torch.randn((107_000, 256), generator=gen, device=cuda)
     want = a.double().t() @ b.double()
+    ops.weight_grad(a, b)
+    assert L.lib().fgl_product_last_kernel() == b"wgrad_kernel in parts"
     assert (ops.weight_grad(a, b).double() - want).norm() <= 2.8e-7 * want.norm()
 
 
@@ -41,6 +56,7 @@ def test_values_without_three_parts(cuda):
     a[:, 20] *= 1e-36      # (bits below bf16's last)
     a[17, 30] = 3.4e38     # (rounds to infinity in bf16)
     got, want = ops.weight_grad(a, b), a.double().t() @ b.double()
+    assert L.lib().fgl_product_last_kernel() == b"wgrad_kernel in parts"
     odd = ~torch.isfinite(want)
     assert bool(odd[3].all()) and bool(odd[9].all()) and bool(odd[:, 100].all()) and int(odd.sum()) == 2 * n + m - 2
     assert torch.allclose(got[odd].double(), want[odd], rtol=0, atol=0, equal_nan=True)
