@@ -486,16 +486,6 @@ struct WgradPlan {
     size_t ws_bytes;
 };
 
-// Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
-// faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
-// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 75 / 68, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237).
-// Fewer rows than a step has are the fp32 form's, whose sums of one and two products are the more exact ones: rms errors against 64 bits, fp32 / split, k = 1
-// 2.5e-8 / 3.5e-8, k = 2 3.1e-8 / 3.4e-8, k = 16 6.1e-8 / 3.4e-8, k = 17 6.5e-8 / 4.3e-8, k = 64 8.6e-8 / 5.5e-8.
-static bool wgrad_split_pays(int64_t k, int m, int n)
-{
-    return k >= 16 && wgrad_vec(m, true, 4) * wgrad_vec(n, true, 4) >= 8 && (double)k * m * n <= 9e9;
-}
-
 static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, bool split)
 {
     WgradPlan p;
@@ -524,6 +514,22 @@ static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, boo
     p.sum_offset = align_up((size_t)p.splits * p.tiles * p.va * p.vb * 16 * kWave * sizeof(float), 256);
     p.ws_bytes = p.sum_offset + align_up((size_t)p.splits * (p.tiles / p.tiles_n) * 32 * p.va * sizeof(float), 256);
     return p;
+}
+
+// Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
+// faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
+// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 75 / 68, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237;
+// with 65 to 128 columns on one side, two tiles, 100 x 4000 k = 20 K 174 / 203, 100 x 602 k = 110 K 159 / 166, 100 x 1000 k = 60 K 142 / 136).  A split's workgroups are one XCD's,
+// so that fewer than eight splits leave XCDs idle; four times the tiles leave room for fewer of them where k allows few: k = 1000, 1000 x 1000 61 / 83 (four splits / two),
+// 2000 x 602 104 / 162, 256 x 4000 61 / 82; k = 3000 119 / 79, 214 / 97, 120 / 77.
+// Fewer rows than a step has are the fp32 form's, whose sums of one and two products are the more exact ones: rms errors against 64 bits, fp32 / split, k = 1
+// 2.5e-8 / 3.5e-8, k = 2 3.1e-8 / 3.4e-8, k = 16 6.1e-8 / 3.4e-8, k = 17 6.5e-8 / 4.3e-8, k = 64 8.6e-8 / 5.5e-8.
+static bool wgrad_split_pays(int64_t k, int m, int n)
+{
+    const int least = m < n ? m : n;
+    if (k < 16 || wgrad_vec(m, true, 4) * wgrad_vec(n, true, 4) < 8 || (double)k * m * n > (least > 64 && least <= 128 ? 6e9 : 9e9)) return false;
+    const int splits = wgrad_plan(k, m, n, true, true, true).splits;
+    return splits >= 8 || splits >= wgrad_plan(k, m, n, true, true, false).splits;
 }
 
 static bool wgrad_vectors(int dtype, int cols, int64_t ld, const void* ptr)

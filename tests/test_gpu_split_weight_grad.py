@@ -62,3 +62,25 @@ def test_values_without_three_parts(cuda):
     assert torch.allclose(got[odd].double(), want[odd], rtol=0, atol=0, equal_nan=True)
     size = a.double().abs().t() @ b.double().abs()
     assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size + k * 2.0 ** -149)[~odd].all())
+
+
+def _through_c(a, b, ws_bytes):
+    """The C entry on a workspace of so many bytes: status, result."""
+    lib, (k, m), n = L.lib(), a.shape, b.size(1)
+    out, ws = torch.empty((m, n), dtype=a.dtype, device=a.device), torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
+    dtype = L.F32 if a.dtype == torch.float32 else L.BF16
+    rc = lib.fgl_weight_grad(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), k, m, n, dtype, out.data_ptr(), n, None, ws.data_ptr(), ws_bytes, L.stream_handle())
+    return rc, out
+
+
+@pytest.mark.parametrize("k,m,n,kernel", [(1000, 1000, 1000, b"wgrad_kernel"), (3000, 1000, 1000, b"wgrad_kernel in parts"), (1000, 602, 2000, b"wgrad_kernel"),
+                                          (3000, 602, 2000, b"wgrad_kernel in parts"), (20_000, 100, 4000, b"wgrad_kernel"), (8000, 100, 4000, b"wgrad_kernel in parts"),
+                                          (1000, 256, 256, b"wgrad_kernel in parts")])
+def test_line_between_the_forms(cuda, k, m, n, kernel):
+    """Few splits of k leave XCDs idle: many tiles and a short k are the fp32 form's."""
+    gen = torch.Generator(device=cuda).manual_seed(k)
+    a, b = torch.randn((k, m), generator=gen, device=cuda), torch.randn((k, n), generator=gen, device=cuda)
+    rc, got = _through_c(a, b, L.lib().fgl_weight_grad_workspace_bytes(k, m, n))
+    assert rc == 0 and L.lib().fgl_product_last_kernel() == kernel
+    want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+    assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
