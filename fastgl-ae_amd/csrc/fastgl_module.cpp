@@ -151,7 +151,7 @@ torch::Tensor weight_grad(const torch::Tensor& a, const torch::Tensor& b)
         a.stride(0) >= (1 << 24) || b.stride(0) >= (1 << 24))
         return torch::mm(a.transpose(0, 1), b);
     auto out = torch::empty({m, n}, a.options());
-    auto ws = scratch(fgl_weight_grad_workspace_bytes(k, (int)m, (int)n), a);
+    auto ws = scratch(fgl_weight_grad_workspace_bytes_for(k, (int)m, (int)n, dtype_of(a)), a);
     ok(fgl_weight_grad(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), k, (int)m, (int)n, dtype_of(a), out.data_ptr(), n, nullptr,
                        ws.data_ptr(), (size_t)ws.numel(), stream_of(a)));
     return out;

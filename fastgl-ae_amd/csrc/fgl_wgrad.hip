@@ -568,7 +568,7 @@ static int launch_wgrad_any(const WgradPlan& p, const WgradArgs& g, hipStream_t 
 
 using namespace fgl;
 
-FGL_EXPORT size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n)
+FGL_EXPORT size_t fgl_weight_grad_workspace_bytes_for(int64_t k, int m, int n, int dtype)
 {
     if (k < 0 || m < 1 || n < 1) return 0;
     size_t most = 0;
@@ -576,10 +576,11 @@ FGL_EXPORT size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n)
         const size_t b = wgrad_plan(k, m, n, (i & 1) != 0, (i & 2) != 0, false).ws_bytes;
         if (b > most) most = b;
     }
-    const size_t b = wgrad_plan(k, m, n, true, true, true).ws_bytes;
-    if (b > most) most = b;
-    return most;
+    const size_t b = dtype == FGL_F32 && wgrad_split_pays(k, m, n) ? wgrad_plan(k, m, n, true, true, true).ws_bytes : 0;
+    return b > most ? b : most;
 }
+
+FGL_EXPORT size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n) { return fgl_weight_grad_workspace_bytes_for(k, m, n, FGL_F32); }
 
 FGL_EXPORT int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int64_t k, int m, int n, int dtype,
                                void* d_c, int64_t ldc, void* d_sum_a, void* d_ws, size_t ws_bytes, void* stream)
@@ -589,8 +590,13 @@ FGL_EXPORT int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, in
     FGL_REQUIRE(lda >= m && ldb >= n && ldc >= n, "weight_grad: row stride smaller than the row length");
     FGL_REQUIRE(lda < (1 << 24) && ldb < (1 << 24), "weight_grad: row stride too large");  // (eight rows are spanned by 32-bit offsets)
     FGL_REQUIRE(d_c != nullptr && (k == 0 || (d_a && d_b)), "weight_grad: null pointer");
-    const bool split = dtype == FGL_F32 && wgrad_split_pays(k, m, n);
-    const WgradPlan p = wgrad_plan(k, m, n, wgrad_vectors(dtype, m, lda, d_a), wgrad_vectors(dtype, n, ldb, d_b), split);
+    const bool va = wgrad_vectors(dtype, m, lda, d_a), vb = wgrad_vectors(dtype, n, ldb, d_b);
+    bool split = dtype == FGL_F32 && wgrad_split_pays(k, m, n);
+    WgradPlan p = wgrad_plan(k, m, n, va, vb, split);
+    if (split && ws_bytes < p.ws_bytes) {  // (a workspace for a longer k, which needs less where that is not in parts)
+        split = false;
+        p = wgrad_plan(k, m, n, va, vb, false);
+    }
     if (d_ws == nullptr || ws_bytes < p.ws_bytes) {
         set_error("weight_grad: workspace too small (%zu < %zu)", ws_bytes, p.ws_bytes);
         return FGL_ERR_WORKSPACE;

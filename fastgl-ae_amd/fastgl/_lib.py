@@ -69,6 +69,7 @@ SIGNATURES = {
     "fgl_edge_softmax": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i32, C.c_float, _vp, _vp]),
     "fgl_head_scores": (_i32, [_vp, _i64, _i64, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),
     "fgl_weight_grad_workspace_bytes": (_sz, [_i64, _i32, _i32]),
+    "fgl_weight_grad_workspace_bytes_for": (_sz, [_i64, _i32, _i32, _i32]),
     "fgl_weight_grad": (_i32, [_vp, _i64, _vp, _i64, _i64, _i32, _i32, _i32, _vp, _i64, _vp, _vp, _sz, _vp]),
     "fgl_product_last_kernel": (C.c_char_p, []),
     "fgl_row_product_sum": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _i64, _vp, _i64, _i32, _i32, _i64, _i32, _i32, _vp, _vp, _i64, _vp]),

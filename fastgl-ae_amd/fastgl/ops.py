@@ -504,11 +504,12 @@ def weight_grad(a, b, column_sums=False):
         return (d_w, a.sum(0)) if column_sums else d_w
     lib = L.lib()
     dev = a.device
+    dtype = L.F32 if a.dtype == torch.float32 else L.BF16
     with _on_device(dev):
         d_w = torch.empty((m, n), dtype=a.dtype, device=dev)
         sums = torch.empty(m, dtype=a.dtype, device=dev) if column_sums else None
-        ws = L.workspace(lib.fgl_weight_grad_workspace_bytes(k, m, n), dev)
-        L.check(lib.fgl_weight_grad(at[0], lda, at[1], ldb, k, m, n, L.F32 if a.dtype == torch.float32 else L.BF16, d_w.data_ptr(), n, L.ptr(sums),
+        ws = L.workspace(lib.fgl_weight_grad_workspace_bytes_for(k, m, n, dtype), dev)
+        L.check(lib.fgl_weight_grad(at[0], lda, at[1], ldb, k, m, n, dtype, d_w.data_ptr(), n, L.ptr(sums),
                                     ws.data_ptr(), ws.numel(), L.stream_handle()))
     return (d_w, sums) if column_sums else d_w
 

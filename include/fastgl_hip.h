@@ -435,8 +435,11 @@ int fgl_row_product_add(const void* d_a, int64_t lda, const void* d_b, int64_t l
  * d_sum_a (may be NULL): m elements of `dtype`, the column sums of A (with A = the gradient of the layer's output: its
  * bias gradient), from the same pass.
  * Meant for k far above m and n; the k splits are added in a fixed order (the same bits on every run).
+ * Workspace: what fgl_weight_grad_workspace_bytes_for says for the type, or without it for either.  Less than that is an error, unless the
+ * fp32 form that needs less takes it.
  * ------------------------------------------------------------------------------- */
 size_t fgl_weight_grad_workspace_bytes(int64_t k, int m, int n);
+size_t fgl_weight_grad_workspace_bytes_for(int64_t k, int m, int n, int dtype);
 int fgl_weight_grad(const void* d_a, int64_t lda, const void* d_b, int64_t ldb, int64_t k, int m, int n, int dtype,
                     void* d_c, int64_t ldc, void* d_sum_a, void* d_ws, size_t ws_bytes, void* stream);
 

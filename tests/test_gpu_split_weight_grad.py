@@ -84,3 +84,18 @@ def test_line_between_the_forms(cuda, k, m, n, kernel):
     assert rc == 0 and L.lib().fgl_product_last_kernel() == kernel
     want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
     assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
+
+
+def test_workspace_of_the_fp32_form(cuda):
+    """A caller whose workspace was sized for another k, of which the parts are not asked: the fp32 form, an error only below what that needs."""
+    lib, k, m, n = L.lib(), 3000, 602, 1000
+    gen = torch.Generator(device=cuda).manual_seed(9)
+    a, b = torch.randn((k, m), generator=gen, device=cuda), torch.randn((k, n), generator=gen, device=cuda)
+    whole, less = lib.fgl_weight_grad_workspace_bytes_for(k, m, n, L.F32), lib.fgl_weight_grad_workspace_bytes_for(k, m, n, L.BF16)
+    assert less < whole
+    want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+    for ws_bytes, kernel in ((whole, b"wgrad_kernel in parts"), (less, b"wgrad_kernel")):
+        rc, got = _through_c(a, b, ws_bytes)
+        assert rc == 0 and lib.fgl_product_last_kernel() == kernel
+        assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
+    assert _through_c(a, b, 1024)[0] != 0
