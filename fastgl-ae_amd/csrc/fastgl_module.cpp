@@ -170,7 +170,7 @@ torch::Tensor aggregate(const torch::Tensor& indptr, const torch::Tensor& indice
     auto out = torch::empty({n_rows, D}, feat.options());
     if (n_rows == 0) return out;
     const void* idx = indices.numel() ? indices.data_ptr() : indptr.data_ptr();  // a block without entries: never read
-    const size_t ws_bytes = fgl_aggregate_workspace_bytes(indices.numel(), (int)D, mode, longest_row);
+    const size_t ws_bytes = fgl_aggregate_workspace_bytes_for(indices.numel(), n_rows, feat.size(0), (int)D, dtype_of(feat), mode, longest_row);
     torch::Tensor ws;
     if (ws_bytes > 0) ws = torch::empty({(int64_t)ws_bytes}, feat.options().dtype(torch::kUInt8));
     ok(fgl_aggregate_ws(indptr.data_ptr<int32_t>(), static_cast<const int32_t*>(idx), n_rows, nullptr, feat.data_ptr(), feat.stride(0),

@@ -147,6 +147,7 @@ struct AggArgs {
     int col_norm_is_ptr;        // col_norm is an offsets array, the counts are its differences
     void* ws;                   // scratch of aggregate_workspace_bytes(n_entries_max, D) bytes: long rows go in segments (NULL: row by row)
     int64_t n_entries_max;      // (with ws) no fewer entries than the rows hold
+    bool classes;               // ws holds what segments in classes take
     const int32_t* order;       // aggregate_kernel<.., ORDERED>: lane group i takes row order[i] ...
     const int32_t* in_order;    // ... in the tiles of 2^tile_log rows that are marked here
     int tile_log;
@@ -1205,20 +1206,16 @@ static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, bool classes, 
     return l;
 }
 
-// Scratch for classes, where there may be any: the caller's sizes decide, and the launch among those by what it also knows.
-static size_t class_bytes(int64_t n_entries_max, int D)
+// What classes take, 0 where they do not pay.  (The rows that are gathered are the source's; as few rows of results are blocks, of which nothing was measured.)
+static size_t class_bytes(int64_t n_entries_max, int64_t n_rows_max, int64_t n_source_rows, int D, int dtype, int64_t longest_row_max)
 {
-    if (n_entries_max < kClassMinEntries || D * (int64_t)sizeof(float) < kClassMinRow) return 0;
+    const int64_t row = D * (int64_t)(dtype == FGL_F32 ? sizeof(float) : sizeof(uint16_t)), rows = n_rows_max < n_source_rows ? n_rows_max : n_source_rows;
+    if (n_entries_max < kClassMinEntries || row < kClassMinRow || rows * row < kClassMinBytes || (longest_row_max >= 0 && longest_row_max <= kClassEntries)) return 0;
     size_t bytes = 0;
     (void)seg_lists(nullptr, n_entries_max, D, true, &bytes);
     return bytes <= kClassMaxBytes ? bytes : 0;
 }
-static SegLists seg_lists_of(const AggArgs& g, size_t element)
-{
-    const int64_t row = g.D * (int64_t)element;
-    const bool classes = class_bytes(g.n_entries_max, g.D) > 0 && row >= kClassMinRow && g.n_rows_max * row >= kClassMinBytes;
-    return seg_lists(g.ws, g.n_entries_max, g.D, classes, nullptr);
-}
+static SegLists seg_lists_of(const AggArgs& g) { return seg_lists(g.ws, g.n_entries_max, g.D, g.classes, nullptr); }
 
 __global__ void seg_init_kernel(int32_t* __restrict__ counts)
 {
@@ -1728,11 +1725,11 @@ size_t transpose_workspace_bytes(int64_t n_cols_max, int64_t n_edges_max, int so
 // ---- dispatch ----------------------------------------------------------------------
 // Which lane mapping the calling thread's last fgl_aggregate call chose (for benchmarks and bug reports).
 static thread_local char g_mapping[96] = "";
-static void note_mapping(const char* kernel, int lpr, int extra, bool second_pass, bool segments = false)
+static void note_mapping(const char* kernel, int lpr, int extra, bool second_pass, bool segments = false, bool classes = false)
 {
     snprintf(g_mapping, sizeof(g_mapping), "%s lanes/row=%d%s%s", kernel, lpr,
              extra > 1 ? (extra >= 100 ? " (rows bundled by 4)" : " (groups/row>1)") : "",
-             !second_pass ? "" : segments ? " + segments" : " + long_rows");
+             !second_pass ? "" : classes ? " + classes + segments" : segments ? " + segments" : " + long_rows");
 }
 
 // From this many rows on, the tiles of a large block with long rows among them are looked at for an order by length (rows of up to 32 lanes: a
@@ -1759,17 +1756,18 @@ static void launch_seg_lists(const SegLists& l, hipStream_t stream, const AggArg
         hipLaunchKernelGGL((seg_lists_kernel<PER_WAVE, kSegFewRows>), grid, dim3(kSegBlock), 0, stream, g, l, order, in_order);
 }
 
-// The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
-// for large inputs), else a workgroup per row.
-// Workgroups for what the device counts: as many as there may be, up to so many, which then take turns (empty launches of 32 K and twice 8 K workgroups took 20 us, of 8 K and twice 4 K within the runs' differences)
+// Workgroups for what the device counts: as many as there may be, up to so many, which then take turns (empty launches of 32 K and twice
+// 8 K workgroups took 20 us, of 8 K and twice 4 K within the runs' differences)
 static unsigned at_most(int64_t blocks, int64_t most) { return (unsigned)(blocks < most ? blocks : most); }
 
+// The launches for the rows that the first one has left out: in segments where there is scratch for them (the caller provides it
+// for large inputs), else a workgroup per row.
 template <typename T, int VEC, int LPR, int MODE>
 static void launch_long_rows(unsigned gy, hipStream_t stream, const AggArgs& g)
 {
     if constexpr (MODE != FGL_AGG_EDGE) {
         if (g.ws != nullptr) {
-            const SegLists l = seg_lists_of(g, sizeof(T));
+            const SegLists l = seg_lists_of(g);
             if (g.order == nullptr) launch_seg_lists<0>(l, stream, g, nullptr, nullptr);  // (else listed with the rows' order)
             // (a unit has more than kLongRowEntries entries, or is one of at most two per kSegEntries > 2 * kLongRowEntries of them)
             static_assert(kSegEntries > 2 * kLongRowEntries, "the bound on the number of units");
@@ -1810,13 +1808,13 @@ static int launch_agg_mode(int mode, bool long_rows_possible, dim3 grid, hipStre
         return FGL_OK;
       }
     }
-    note_mapping("aggregate_kernel", LPR, 1, second_pass, g.ws != nullptr);
+    note_mapping("aggregate_kernel", LPR, 1, second_pass, g.ws != nullptr, g.classes);
     g.turn = second_pass;
     bool ordered = false;
     if constexpr (LPR <= 32) {
         if (second_pass && g.ws != nullptr && mode != FGL_AGG_EDGE && g.n_rows_max >= kOrderMinRows) {
             // (in the place of the partial sums, which the launches behind the gather fill; the launch that lists the long rows finds the order)
-            const SegLists l = seg_lists_of(g, sizeof(T));
+            const SegLists l = seg_lists_of(g);
             const int tile = seg_tile(g.n_rows_max);
             if ((int64_t)l.cap_seg * l.ldp * l.classes >= g.n_rows_max + ceil_div(g.n_rows_max, tile)) {
                 int32_t* order = reinterpret_cast<int32_t*>(l.partial);
@@ -1859,7 +1857,7 @@ static int launch_agg_flat(int mode, int64_t longest_row_max, int lanes, bool bu
     const int known = bundle && limit < kBundleKnownEntries ? kBundleKnownEntries : limit;
     const bool long_rows_possible = longest_row_max < 0 || longest_row_max > known;
     g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;
-    note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible, g.ws != nullptr);
+    note_mapping(bundle ? "aggregate_flat_bundle_kernel" : "aggregate_flat_kernel", lanes, bundle ? 100 : 1, long_rows_possible, g.ws != nullptr, g.classes);
     const int64_t blocks = ceil_div((bundle ? ceil_div(g.n_rows_max, kBundleRows) : g.n_rows_max) * lanes, kBlock);
     if (blocks > 0x7FFFFFFF) {
         set_error("aggregate: grid too large (%lld workgroups)", (long long)blocks);
@@ -1925,7 +1923,7 @@ static int launch_agg_bundle(int mode, int64_t longest_row_max, unsigned gy, hip
     const bool long_rows_possible = longest_row_max < 0 || longest_row_max > kLongRowEntries;
     const int limit = long_row_limit(true, g);
     g.skip_rows_longer_than = long_rows_possible ? limit : 0x7FFFFFFF;
-    note_mapping("aggregate_bundle_kernel", LPR, 100, long_rows_possible, g.ws != nullptr);
+    note_mapping("aggregate_bundle_kernel", LPR, 100, long_rows_possible, g.ws != nullptr, g.classes);
     const int64_t gx = ceil_div(ceil_div(g.n_rows_max, kBundleRows), kBlock / LPR);
 #define FGL_LAUNCH_BUNDLE(M)                                                                                          \
     do {                                                                                                              \
@@ -2074,7 +2072,14 @@ FGL_EXPORT size_t fgl_aggregate_workspace_bytes(int64_t n_entries_max, int D, in
     if (longest_row_max >= 0 && longest_row_max <= kLongRowEntries) return 0;
     size_t bytes = 0;
     (void)seg_lists(nullptr, n_entries_max, D, false, &bytes);
-    const size_t in_classes = class_bytes(n_entries_max, D);
+    return bytes;
+}
+
+FGL_EXPORT size_t fgl_aggregate_workspace_bytes_for(int64_t n_entries_max, int64_t n_rows_max, int64_t n_source_rows, int D, int dtype, int mode,
+                                                    int64_t longest_row_max)
+{
+    const size_t bytes = fgl_aggregate_workspace_bytes(n_entries_max, D, mode, longest_row_max);
+    const size_t in_classes = bytes > 0 ? class_bytes(n_entries_max, n_rows_max, n_source_rows, D, dtype, longest_row_max) : 0;
     return bytes > in_classes ? bytes : in_classes;
 }
 
@@ -2112,6 +2117,9 @@ FGL_EXPORT int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indice
     g.n_heads = n_heads > 0 ? n_heads : 1; g.unit_dim = D / g.n_heads; g.col_norm_is_ptr = col_norm_is_ptr;
     const size_t ws_needed = n_rows_max <= 0x7FFFFFFF ? fgl_aggregate_workspace_bytes(n_entries_max, D, mode, longest_row_max) : 0;
     g.ws = ws_needed > 0 && d_ws != nullptr && ws_bytes >= ws_needed ? d_ws : nullptr;
+    // (how many rows x has the caller knows: who asks with that number gets scratch for classes only where they pay)
+    const size_t in_classes = g.ws != nullptr ? class_bytes(n_entries_max, n_rows_max, n_rows_max, D, dtype, longest_row_max) : 0;
+    g.classes = in_classes > 0 && ws_bytes >= in_classes;
     g.n_entries_max = n_entries_max;
     g.order = nullptr;
     g.in_order = nullptr;

@@ -62,6 +62,7 @@ SIGNATURES = {
     "fgl_aggregate": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _i64,
                              _vp, _i64, _vp]),
     "fgl_aggregate_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64]),
+    "fgl_aggregate_workspace_bytes_for": (_sz, [_i64, _i64, _i64, _i32, _i32, _i32, _i64]),
     "fgl_aggregate_ws": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _vp, _i64,
                                 _vp, _i64, _vp, _sz, _vp]),
     "fgl_zero_empty_rows": (_i32, [_vp, _i64, _vp, _vp, _i64, _i32, _i32, _vp]),

@@ -594,12 +594,13 @@ def aggregate(indptr, indices, feat, mode="sum", zero_policy="self", row_norm=No
             idx_ptr = L.ptr(indices) if indices.numel() else L.ptr(indptr)
             n_entries = int(indices.numel()) if mapping == "auto" else -1
             longest_known = longest_host if mapping == "auto" else -1
+            dtype = L.F32 if feat.dtype == torch.float32 else L.BF16
             ws, ws_bytes = None, 0
             if n_entries >= L.AGG_SEG_MIN_ENTRIES:
-                ws_bytes = L.lib().fgl_aggregate_workspace_bytes(n_entries, D, m, longest_known)
+                ws_bytes = L.lib().fgl_aggregate_workspace_bytes_for(n_entries, n, int(feat.size(0)), D, dtype, m, longest_known)
                 ws = L.workspace(ws_bytes, dev) if ws_bytes else None
             L.check(L.lib().fgl_aggregate_ws(L.ptr(indptr), idx_ptr, n, L.ptr(n_rows_dev), L.ptr(feat), int(feat.stride(0)), D,
-                                             L.F32 if feat.dtype == torch.float32 else L.BF16, m, z, L.ptr(row_norm),
+                                             dtype, m, z, L.ptr(row_norm),
                                              L.ptr(col_norm), L.ptr(edge_weight), int(n_heads), L.ptr(edge_index),
                                              longest_known, L.ptr(longest_dev), n_entries, L.ptr(out),
                                              int(out.stride(0)), L.ptr(ws), ws_bytes, L.stream_handle()))

@@ -371,8 +371,13 @@ int fgl_aggregate(const int32_t* d_indptr, const int32_t* d_indices,
                   void* d_out, int64_t ldo, void* stream);
 /* fgl_aggregate with scratch for the hub rows of large inputs: given fgl_aggregate_workspace_bytes bytes (0: none is used, and
  * less than that is not used either), rows of hundreds of entries are summed in segments that are spread over the
- * chip.  n_entries_max must then be no smaller than the number of entries the rows hold. */
+ * chip.  n_entries_max must then be no smaller than the number of entries the rows hold.
+ * fgl_aggregate_workspace_bytes_for, which also knows the rows of the result, the rows of X and the type, asks for more where the segments of a
+ * large graph gain by being gathered class by class of their neighbours (the ids once more and eight sums a segment, at most 4 GiB); they are
+ * where the workspace holds that. */
 size_t fgl_aggregate_workspace_bytes(int64_t n_entries_max, int D, int mode, int64_t longest_row_max);
+size_t fgl_aggregate_workspace_bytes_for(int64_t n_entries_max, int64_t n_rows_max, int64_t n_source_rows, int D, int dtype, int mode,
+                                         int64_t longest_row_max);
 int fgl_aggregate_ws(const int32_t* d_indptr, const int32_t* d_indices,
                      int64_t n_rows_max, const int32_t* d_n_rows,
                      const void* d_x, int64_t ldx, int D, int dtype, int mode, int zero_policy,

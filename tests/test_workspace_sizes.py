@@ -10,3 +10,18 @@ def test_weight_grad():
         fp32, bf16 = (lib.fgl_weight_grad_workspace_bytes_for(k, m, n, d) for d in (L.F32, L.BF16))
         assert bf16 <= fp32 == lib.fgl_weight_grad_workspace_bytes(k, m, n)
     assert 4 * lib.fgl_weight_grad_workspace_bytes_for(3000, 602, 4000, L.BF16) < lib.fgl_weight_grad_workspace_bytes_for(3000, 602, 4000, L.F32)
+
+
+def test_aggregate():
+    lib, n, nodes = L.lib(), 54_000_000, 2_400_000
+
+    def size(D, dtype, rows=nodes, sources=nodes, longest=-1, entries=n):
+        return lib.fgl_aggregate_workspace_bytes_for(entries, rows, sources, D, dtype, L.AGG_GCN, longest)
+
+    plain = lib.fgl_aggregate_workspace_bytes(n, 64, L.AGG_GCN, -1)
+    assert plain < 64 << 20 < size(64, L.F32)  # (a sum a segment; eight, and the ids)
+    # rows of 128 bytes, few rows on either side, no row long enough: what is never gathered by classes asks for no more than the segments take
+    assert plain == size(64, L.BF16) == size(64, L.F32, rows=8192) == size(64, L.F32, sources=8192) == size(64, L.F32, longest=256)
+    assert size(64, L.F32, longest=257) > plain
+    assert size(64, L.F32, longest=128) == 0 and size(64, L.F32, entries=1000) == 0
+    assert size(3000, L.F32, entries=2_000_000_000) == lib.fgl_aggregate_workspace_bytes(2_000_000_000, 3000, L.AGG_GCN, -1)  # (classes would take more than 4 GiB)
