@@ -22,7 +22,7 @@
 //     Within a bucket a column is 16 bits.  Traffic: 2 reads of the ids, 2 writes and reads of the rows, 1 write and 2 reads of
 //     half the columns.
 //     (54 M entries of a 2.4 M-node graph, hubs of 85 K, us: counts, with an atomic per entry 5900 / 13200 -- unordered / sorted
-//     ids --, with 4-byte stores all over the buckets 499 / 674, now 276 / 177; transpose 24700, 1550, now 700.)
+//     ids --, with 4-byte stores all over the buckets 499 / 674, now 276 / 187; transpose 24700, 1550, now 700.)
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_tile_rows.hpp"
@@ -160,13 +160,20 @@ __device__ __forceinline__ void load_columns(const BucketArgs& g, int64_t first,
         if (c[j] >= g.n_cols) c[j] = -1;
 }
 
-// A tile's entries by bucket.  (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's rows -- would otherwise be 64
-// updates of one counter at a time, one after the other.)
-// DIRECT (counting only): a tile that is runs of equal ids -- at most four begin inside the sixteen entries of seven lanes in eight of its first wave: the destinations of an edge list in order -- is
-// counted here,
-// one atomic a run in device memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.  (Whole counts, us, before / with it: 54 M ids
-// over 2.4 M counters, sorted 276 / 177, in no order 275 / 276; 20 M over 100 K, sorted 82 / 42; 5 M over 600 K, sorted 42 / 37, in no order 38.3 / 38.8; 8 M over 2.4 M, sorted,
-// three and a third a run and so not direct, 67.7 / 68.7.)
+// A tile's entries by bucket.  (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's
+// rows -- would otherwise be 64 updates of one counter at a time, one after the other.)
+// DIRECT (counting only): a tile of runs of equal ids in ascending order -- kDirectRun entries a run on average, and its first id
+// none below the last of the tile before: the destinations of an edge list in order -- is counted here, one atomic a run in device
+// memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.  Runs in no order may be of the
+// same few ids over and over, whose updates LDS takes and device memory does not, and ascending ones too, in every few tiles, which
+// is why they have to be long.  (Whole counts, us, by buckets alone / with it: 54 M destinations of an R-MAT graph of 2.4 M nodes
+// 274 / 187, sorted uniform ids 268 / 182, in no order 282 / 284; 20 M over 100 K, sorted 82 / 50; 5 M over 600 K, sorted, eight a
+// run and so not direct, 40.7 / 42.0, in no order 37.5 / 38.2.  In ascending stretches of 1 M ids over 100 K, ten a run, 179 / 181,
+// of 2 M, twenty, 179 / 141.  kDirectRun of 8: the graph 176, the stretches 210 and 141, of 20 K ids over 2 K 255 / 669.  When the
+// tile's first wave alone was looked at, for runs of four, fives of two ids in turn took 122477, tiles in order up to their eighth
+// 1857.)
+constexpr int kDirectRun = 14;
+
 template <bool DIRECT>
 __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
 {
@@ -177,29 +184,50 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketA
     const int tid = (int)threadIdx.x;
     for (int b = tid; b < g.buckets; b += kBucketBlock) s_cnt[b] = 0;
     int32_t c[kBucketItems];
+    int32_t before = -1;  // the last entry of the tile before
+    if (DIRECT && tid == 0 && tile > 0 && tile * kBucketTile <= n) before = g.ids[tile * kBucketTile - 1];
     load_columns(g, tile * kBucketTile + (int64_t)tid * kBucketItems, n, c);
     bool direct = false;
     if constexpr (DIRECT) {
+        constexpr int kWaves = kBucketBlock / kWave;
+        __shared__ int s_direct, s_runs, s_last[kBucketBlock], s_first[kWaves];
+        const int lane = lane_id(), wave = tid / kWave;
         // one wave looks at its 1024 entries, for all: what the others would see costs an input in no order 2 % of the whole count
-        __shared__ int s_direct;
-        if (tid < kWave) {
-            int begin = 0;
+        // (the runs that begin in the wave, and whether the lane's ids ascend)
+        auto look = [&](int last, bool& ascends) {
+            int begin = c[0] != last;
+            ascends = c[0] >= last;
 #pragma unroll
-            for (int j = 1; j < kBucketItems; ++j) begin += c[j] != c[j - 1];
-            const int few = __popcll(__ballot(begin <= kBucketItems / 4));
+            for (int j = 1; j < kBucketItems; ++j) {
+                begin += c[j] != c[j - 1];
+                ascends &= c[j] >= c[j - 1];
+            }
+            int runs = 0;
+#pragma unroll
+            for (int b = 0; b < 5; ++b) runs += __popcll(__ballot(begin >> b & 1)) << b;
+            return runs;
+        };
+        bool ascends;
+        if (tid < kWave) {
+            const int last = __shfl_up(c[kBucketItems - 1], 1, kWave);
+            const int runs = look(tid > 0 ? last : before < g.n_cols ? before : -1, ascends);
+            const bool may_be = __all(ascends) && runs <= kWave * kBucketItems / kDirectRun;
             if (tid == 0) {
-                s_direct = few >= kWave / 8 * 7;
-                g.direct[tile] = few >= kWave / 8 * 7;
+                s_direct = may_be;
+                s_runs = 0;
             }
         }
         __syncthreads();
         direct = s_direct != 0;
-        if (direct) {  // (the whole workgroup)
-            constexpr int kWaves = kBucketBlock / kWave;
-            __shared__ int s_last[kBucketBlock], s_first[kWaves];
-            const int lane = lane_id(), wave = tid / kWave;
+        if (direct) {  // (the whole workgroup): now all of it
             s_last[tid] = c[kBucketItems - 1];
             __syncthreads();
+            const int runs = look(tid > 0 ? s_last[tid - 1] : -1, ascends);
+            if (lane == 0) atomicAdd(&s_runs, runs);
+            direct = __syncthreads_and(ascends) != 0 && s_runs <= kBucketTile / kDirectRun;
+        }
+        if (tid == 0) g.direct[tile] = direct;
+        if (direct) {
             uint32_t heads = 0;  // where runs begin: bit j for the lane's entry j
 #pragma unroll
             for (int j = 1; j < kBucketItems; ++j) heads |= c[j] != c[j - 1] ? 1u << j : 0u;
