@@ -8,8 +8,11 @@
 // grew with k.  Against 64-bit sums, 2-norm, normal / non-negative operands (the fp32 instructions in brackets): k = 100 5.8e-8 / 4.7e-8 (1.8e-7 / 1.4e-7),
 // k = 256 7.0e-8 / 5.1e-8 (2.9e-7 / 2.5e-7), k = 800 1.1e-7 / 7.1e-8 (5.1e-7 / 3.8e-7).  Added to the accumulators directly the errors of k = 602 were
 // those of the fp32 instructions and larger, because the cut then is at the accumulator's 26 bits.
-// Values without such parts: infinite, not a number or rounded to infinity ones make results that are no finite numbers, and bits below 2^-133, bf16's last, matter
-// only to a row of A or a column of B whose largest value is below 2^-85.  A tile with such a result, row or column is formed again in fp32 matrix instructions.
+// Values without such parts: infinite, not a number or rounded to infinity ones make results that are no finite numbers.  Values below 2^-110 may have bits below
+// 2^-133, bf16's last, which are lost; they matter to a result that is not large beside them (sp_least), and subnormal results have no room for the small products.
+// 32 columns of a tile with a result of these kinds are formed again in fp32 matrix instructions.  (us, 107 K x 256 x 256, B transposed / not: 90 / 90; one column
+// of B at 1e-36 191 / 232, where the fp32 kernel alone takes 161 / 144; a hundredth of A's rows at 1e-37 158 / 181; a hundredth of A's values, or one row of B, at
+// 1e-37, which change no result, 97 / 95.)
 //
 // What bounds it: for short k and few columns the pass over A and C, beyond that the matrix cores and the vector unit beside them.
 //
@@ -78,7 +81,7 @@ __device__ __forceinline__ int sp_column(int t, int i)
 // The steps of B's columns from col0 on -> img[step * NT + tile][part][lane], and the largest magnitude of each (magnitudes are in order as whole numbers too).  Four eights of k of one column a thread at a time, so that
 // their loads are in flight together.
 template <int NT, bool BT, int THREADS>
-__device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, SpU4* img, float* most)
+__device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, SpU4* img, float* most, uint32_t* rest)
 {
     constexpr int kVec = NT < 4 ? NT : 4, kCols = 32 * NT, kBatch = 4;
     const float* b = static_cast<const float*>(x.b);
@@ -115,7 +118,9 @@ __device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int
             sp_most(v[i], m);
             atomicMax(reinterpret_cast<int*>(most + col), __float_as_int(m));
             SpU4 p[3];
-            sp_split(v[i], p);
+            uint32_t r = 0;
+            sp_split(v[i], p, r);
+            if (sp_loses(r)) rest[col] = 1;
             SpU4* to = img + ((oct / 2) * NT + t) * 3 * kWave + oct % 2 * 32 + in_group / kVec;
 #pragma unroll
             for (int q = 0; q < 3; ++q) to[q * kWave] = p[q];
@@ -133,12 +138,15 @@ struct SpWave {
     SpU4 b[2][kTiles][3];     // B's values of this round and the next
     SpU4 a[2][3];             // A's of this step and the next
     float x[8], y[2][8];      // A's as loaded: the chunk's second step, the next chunk
-    float most, next_most;    // the largest magnitude of the row as far as it is split, and of the next chunk's first step
+    // of the row as far as it is split, and of the next chunk's first step: what tells whether bits are lost (sp_split), the largest magnitude
+    uint32_t rest, next_rest;
+    float most, next_most;
 
     __device__ __forceinline__ void clear()
     {
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = SpF32x16{};
+        rest = 0;
         most = 0.0f;
     }
     template <int BUF>
@@ -174,7 +182,7 @@ struct SpWave {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[before + t][i] += sum[buf ^ 1][t][i];
             if (j == kRounds - 1) {
-                sp_split(r, a[(U + 1) & 1]);
+                sp_split(r, a[(U + 1) & 1], U == 0 ? rest : next_rest);
                 sp_most(r, U == 0 ? most : next_most);
             }
 #pragma unroll
@@ -200,33 +208,43 @@ struct SpWave {
     }
 };
 
-// One pair of operands in fp32 matrix instructions
-template <int NT, bool BT>
-__device__ __forceinline__ void sp_plain(const RowProductSide& x, const float* a, int col0, int n, SpF32x16 (&acc)[NT])
+// acc += one pair of operands, 32 columns, in fp32 matrix instructions.  a: the lane's row of A, col: its column of B.  Lanes of the lower
+// half have the first four k of every eight, those of the upper half the others.
+template <bool BT>
+__device__ __forceinline__ void sp_plain(const float* a, const RowProductSide& x, int col, SpF32x16& acc)
 {
-    const int lane = lane_id(), half = lane / 32;
+    constexpr int U = 4;
+    const int k = x.k, ldb = (int)x.ldb, half = lane_id() / 32;
     const float* b = static_cast<const float*>(x.b);
-    for (int k0 = 0; k0 < x.k; k0 += 2) {
-        const int k = k0 + half;
-        const bool in = k < x.k;
-        const float va = in ? a[k] : 0.0f;
+    const uint32_t off = BT ? 0 : (uint32_t)(U * half * ldb + col);  // (split_product_pays keeps ldb below 2^27)
+    const float* bt = b + (int64_t)col * ldb;
+    for (int k0 = 0; k0 < k; k0 += 2 * U) {
+        const int kl = k0 + U * half;
+        SpF4 va = {}, vb = {};
+        if (kl + U <= k) {
+            va = *reinterpret_cast<const SpF4*>(a + kl);
+            if constexpr (BT) vb = *reinterpret_cast<const SpF4*>(bt + kl);
+        } else {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int col = col0 + sp_column<NT>(t, lane % 32);
-            float vb = 0.0f;
-            if (in && col < n) vb = BT ? b[(int64_t)col * x.ldb + k] : b[(int64_t)k * x.ldb + col];
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, vb, acc[t], 0, 0, 0);
+            for (int j = 0; j < U; ++j) {
+                if (kl + j < k) va[j] = a[kl + j];
+                if (BT && kl + j < k) vb[j] = bt[kl + j];
+            }
         }
+        if constexpr (!BT) {
+#pragma unroll
+            for (int j = 0; j < U; ++j)
+                if (kl + j < k) vb[j] = (b + (int64_t)(k0 + j) * ldb)[off];
+        }
+#pragma unroll
+        for (int j = 0; j < U; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[j], vb[j], acc, 0, 0, 0);
     }
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(0.0f, 0.0f, acc, 0, 0, 0);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(0.0f, 0.0f, acc[t], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            float s = acc[t][i] + 0.0f;
-            asm volatile("" : "+v"(s));
-            acc[t][i] = s;
-        }
+    for (int i = 0; i < 16; ++i) {
+        float s = acc[i] + 0.0f;
+        asm volatile("" : "+v"(s));
+        acc[i] = s;
     }
 }
 
@@ -235,7 +253,8 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
 {
     constexpr int kVec = NT < 4 ? NT : 4, kThreads = W * kWave;
     extern __shared__ SpU4 s_img[];
-    __shared__ float s_most[2][32 * NT];
+    __shared__ float s_most[2][32 * NT];     // of each column: its largest magnitude, and whether its values lose bits
+    __shared__ uint32_t s_rest[2][32 * NT];
     const int lane = lane_id(), half = lane / 32;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const unsigned per_group = 8u * (unsigned)g.tiles_n;
@@ -277,19 +296,23 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
     };
     SpWave<NT> w;
     load(w.y);
-    if (threadIdx.x < 64 * NT) (&s_most[0][0])[threadIdx.x] = 0.0f;  // (64 NT <= kThreads)
+    if (threadIdx.x < 64 * NT) {  // (64 NT <= kThreads)
+        (&s_most[0][0])[threadIdx.x] = 0.0f;
+        (&s_rest[0][0])[threadIdx.x] = 0;
+    }
     __syncthreads();
-    sp_stage<NT, BT, kThreads>(g.side[0], 2 * chunks0, col0, g.n, s_img, s_most[0]);
-    if constexpr (FORM == kRpSum) sp_stage<NT, BT, kThreads>(g.side[1], 2 * (chunks - chunks0), col0, g.n, s_img + chunks0 * 2 * NT * 3 * kWave, s_most[1]);
+    sp_stage<NT, BT, kThreads>(g.side[0], 2 * chunks0, col0, g.n, s_img, s_most[0], s_rest[0]);
+    if constexpr (FORM == kRpSum) sp_stage<NT, BT, kThreads>(g.side[1], 2 * (chunks - chunks0), col0, g.n, s_img + chunks0 * 2 * NT * 3 * kWave, s_most[1], s_rest[1]);
     __syncthreads();
     if (tile >= row_tiles) return;  // (uniform over the wave; no barrier follows)
-    bool small_column = false;
-    for (int i = lane; i < 64 * NT; i += kWave) small_column |= sp_small((&s_most[0][0])[i]);
-    small_column = __any(small_column);
+    bool columns_lose = false;
+    for (int i = lane; i < 64 * NT; i += kWave) columns_lose |= (&s_rest[0][0])[i] != 0;
+    columns_lose = __any(columns_lose);
     w.clear();
 #pragma unroll
     for (int t = 0; t < SpWave<NT>::kTiles; ++t) w.sum[1][t] = SpF32x16{};
-    sp_split(w.y[0], w.a[0]);
+    w.next_rest = 0;
+    sp_split(w.y[0], w.a[0], w.next_rest);
     w.next_most = 0.0f;
     sp_most(w.y[0], w.next_most);
 #pragma unroll
@@ -299,6 +322,8 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
     for (;;) {
         for (int c = 0; c < chunks; ++c) {
             load(w.y);
+            w.rest |= w.next_rest;
+            w.next_rest = 0;
             w.most = w.most < w.next_most ? w.next_most : w.most;
             w.next_most = 0.0f;
             const SpU4* after = c + 1 == chunks ? s_img + lane : img + 2 * NT * 3 * kWave;
@@ -312,15 +337,39 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
         w.template flush<1>();
         SpF32x16 (&acc)[NT] = w.acc;
         const int64_t row0 = tile * 32;
-        bool odd = small_column || sp_small(fmaxf(w.most, __shfl_xor(w.most, 32, kWave)));
+        uint32_t odd = 0;  // bit t: tile t has a sum that is not to be had in parts
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) odd |= __builtin_amdgcn_classf(acc[t][i], 0x207);  // (infinite or not a number)
-        if (__any(odd)) {
-            w.clear();
-            sp_plain<NT, BT>(g.side[0], row_of(g.side[0], tile) - half * 8, col0, g.n, acc);
-            if constexpr (FORM == kRpSum) sp_plain<NT, BT>(g.side[1], row_of(g.side[1], tile) - half * 8, col0, g.n, acc);
+            for (int i = 0; i < 16; ++i) odd |= sp_odd(acc[t][i]) ? 1u << t : 0u;
+        const bool row_loses = sp_loses(w.rest | __shfl_xor(w.rest, 32, kWave));
+        if (columns_lose || __any(row_loses || odd != 0)) {  // (uniform)
+            int own = lane % 32;
+            asm volatile("" : "+v"(own));  // (else the compiler keeps what follows from it in registers all the while)
+            auto row_again = [&](const RowProductSide& x) {
+                const int64_t row = tile * 32 + own < g.m ? tile * 32 + own : g.m - 1;
+                return static_cast<const float*>(x.a) + row * x.lda;
+            };
+            // (sums of fewer than 1024 terms, which is more than B's room allows; the larger of two pairs' values for either)
+            float row_most[16];  // of the rows of the lane's sums: negative where the row loses bits
+            const float mine = fmaxf(w.most, __shfl_xor(w.most, 32, kWave));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) row_most[i] = __shfl(row_loses ? -mine : mine, 8 * (i / 4) + 4 * half + i % 4, kWave);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int c = sp_column<NT>(t, own), col = col0 + c < g.n ? col0 + c : g.n - 1;
+                const bool column_loses = (s_rest[0][c] | s_rest[1][c]) != 0;
+                const float column_most = fmaxf(s_most[0][c], s_most[1][c]);
+                bool small = (odd >> t & 1) != 0;
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    small |= !(fabsf(acc[t][i]) >= sp_least(1024.0f, row_most[i] < 0.0f, fabsf(row_most[i]), column_loses, column_most));
+                if (!__any(small)) continue;
+                acc[t] = SpF32x16{};
+                sp_plain<BT>(row_again(g.side[0]), g.side[0], col, acc[t]);
+                if constexpr (FORM == kRpSum) sp_plain<BT>(row_again(g.side[1]), g.side[1], col, acc[t]);
+            }
+            w.template read_b<0>(s_img + lane);  // (what was read ahead: its registers are free above)
         }
         float* out = static_cast<float*>(g.c) + (row0 + 4 * half) * g.ldc + col0;
         const bool rows = row0 + 32 <= g.m;  // (uniform)
@@ -399,7 +448,7 @@ static int sp_tiles(const RowProductArgs& g)
 bool split_product_pays(const RowProductArgs& g)
 {
     const int k = g.side[0].k + g.side[1].k;
-    if (sp_lds(g, 1) > (size_t)kSpLds || k <= 32 || g.m < 2000) return false;
+    if (sp_lds(g, 1) > (size_t)kSpLds || k <= 32 || g.m < 2000 || (g.side[0].ldb | g.side[1].ldb) >> 27 != 0) return false;
     const double outputs = (double)g.m * g.n;
     if (outputs < (g.m < 5000 ? 2.1e6 : 1.6e6)) return false;
     const int nt = sp_tiles(g);

@@ -30,8 +30,9 @@
 // tiles of 64 x 64, two waves a SIMD: one splits (88 instructions for a step's 64 columns) while the other multiplies.  Every step's products are added up from
 // zero before they are added to the accumulators; and since what a matrix instruction cuts off is cut downwards, which over 10^4 .. 10^6 rows adds up (7e-7 of the
 // result's 2-norm for k = 107 K where the fp32 form has 2.8e-7), every other step is formed of A's negative and subtracted: 1.4e-7.
-// us, fp32 / split: 100 x 256 k = 107 K 75 / 68, k = 16 K 33 / 21, k = 2000 26 / 12; 256 x 256 k = 17 K 36 / 29, k = 5000 31 / 16; 128 x 128 k = 60 K 37 / 28;
-// 602 x 256 k = 8192 41 / 38; 256 x 47 k = 20 K 20 / 16.  What it waits for now is the rows: one step ahead is half a microsecond at these rates.
+// us, fp32 / split: 100 x 256 k = 107 K 68 / 65, k = 16 K 33 / 21, k = 2000 26 / 12; 256 x 256 k = 17 K 36 / 29, k = 5000 31 / 16; 128 x 128 k = 60 K 37 / 28;
+// 602 x 256 k = 8192 41 / 38; 256 x 47 k = 20 K 19 / 16.  Waves that meet values of which bits are lost to a result, or results that are no numbers, form their rows again
+// (one column of the first of these at 1e-36: 121).  What it waits for now is the rows: one step ahead is half a microsecond at these rates.
 // Tried: blocks of 128 x 128 through LDS, in which every value is split once (65 us for the first of these, but 34 and 41 for 256 x 256 and 602 x 256), and two steps ahead, for
 // which the registers do not suffice (89).
 //
@@ -174,12 +175,12 @@ struct WgradEights {
         }
     }
     // sign times column c in three parts, and the largest magnitude of it so far
-    __device__ __forceinline__ void split(int c, float sign, SpU4 (&p)[3], float& most) const
+    __device__ __forceinline__ void split(int c, float sign, SpU4 (&p)[3], uint32_t& rest, float& most) const
     {
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = r[i][c] * sign;
-        sp_split(v, p);
+        sp_split<true>(v, p, rest);
         sp_most(v, most);
     }
     __device__ __forceinline__ void add_columns(float (&sum)[V]) const
@@ -283,11 +284,18 @@ __device__ __forceinline__ bool wgrad_split_rows(const WgradArgs& g, int64_t k0,
     const int n = k1 - last < kRows ? (k1 > last ? (int)(k1 - last) : 0) : kRows;
     WgradEights<VA> a;
     WgradEights<VB> b;
+    uint32_t rest_a[VA], rest_b[VB];
     float most_a[VA], most_b[VB];
 #pragma unroll
-    for (int i = 0; i < VA; ++i) most_a[i] = 0.0f;
+    for (int i = 0; i < VA; ++i) {
+        rest_a[i] = 0;
+        most_a[i] = 0.0f;
+    }
 #pragma unroll
-    for (int j = 0; j < VB; ++j) most_b[j] = 0.0f;
+    for (int j = 0; j < VB; ++j) {
+        rest_b[j] = 0;
+        most_b[j] = 0.0f;
+    }
     auto load = [&](int i) {
         if (i < whole) {
             a.load(ra, g.lda, off_a);
@@ -305,9 +313,9 @@ __device__ __forceinline__ bool wgrad_split_rows(const WgradArgs& g, int64_t k0,
         if (sums) a.add_columns(sum);
         SpU4 pa[VA][3], pb[VB][3];
 #pragma unroll
-        for (int i = 0; i < VA; ++i) a.split(i, sign, pa[i], most_a[i]);
+        for (int i = 0; i < VA; ++i) a.split(i, sign, pa[i], rest_a[i], most_a[i]);
 #pragma unroll
-        for (int j = 0; j < VB; ++j) b.split(j, 1.0f, pb[j], most_b[j]);
+        for (int j = 0; j < VB; ++j) b.split(j, 1.0f, pb[j], rest_b[j], most_b[j]);
         if (s < whole) load(s + 1);  // (on the way while these are multiplied)
         __builtin_amdgcn_sched_barrier(0);
         F32x16 part[VA * VB];
@@ -327,13 +335,38 @@ __device__ __forceinline__ bool wgrad_split_rows(const WgradArgs& g, int64_t k0,
     }
     bool odd = false;
 #pragma unroll
-    for (int i = 0; i < VA; ++i) odd |= sp_small(fmaxf(most_a[i], __shfl_xor(most_a[i], 32, kWave)));
-#pragma unroll
-    for (int j = 0; j < VB; ++j) odd |= sp_small(fmaxf(most_b[j], __shfl_xor(most_b[j], 32, kWave)));
-#pragma unroll
     for (int t = 0; t < VA * VB; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) odd |= __builtin_amdgcn_classf(acc[t][i], 0x207);  // (infinite or not a number)
+        for (int i = 0; i < 16; ++i) odd |= sp_odd(acc[t][i]);
+    bool loses = false;
+#pragma unroll
+    for (int i = 0; i < VA; ++i) {
+        rest_a[i] = (rest_a[i] | __shfl_xor(rest_a[i], 32, kWave)) & 0xFFFFu;
+        loses |= rest_a[i] != 0;
+    }
+#pragma unroll
+    for (int j = 0; j < VB; ++j) {
+        rest_b[j] = (rest_b[j] | __shfl_xor(rest_b[j], 32, kWave)) & 0xFFFFu;
+        loses |= rest_b[j] != 0;
+    }
+    if (__any(loses)) {
+#pragma unroll
+        for (int i = 0; i < VA; ++i) most_a[i] = fmaxf(most_a[i], __shfl_xor(most_a[i], 32, kWave));
+#pragma unroll
+        for (int j = 0; j < VB; ++j) most_b[j] = fmaxf(most_b[j], __shfl_xor(most_b[j], 32, kWave));
+        const float terms = (float)(whole + 1) * kRows;
+#pragma unroll
+        for (int i = 0; i < VA; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = 8 * (r / 4) + 4 * half + r % 4;  // of the tile: the lane with that column of A
+                const bool row_loses = __shfl((int)rest_a[i], row, kWave) != 0;
+                const float row_most = __shfl(most_a[i], row, kWave);
+#pragma unroll
+                for (int j = 0; j < VB; ++j)
+                    odd |= !(fabsf(acc[i * VB + j][r]) >= sp_least(terms, row_loses, row_most, rest_b[j] != 0, most_b[j]));
+            }
+    }
     return odd;
 }
 
@@ -518,7 +551,7 @@ static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, boo
 
 // Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
 // faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
-// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 75 / 68, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237;
+// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 68 / 65, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237;
 // with 65 to 128 columns on one side, two tiles, 100 x 4000 k = 20 K 174 / 203, 100 x 602 k = 110 K 159 / 166, 100 x 1000 k = 60 K 142 / 136).  A split's workgroups are one XCD's,
 // so that fewer than eight splits leave XCDs idle; four times the tiles leave room for fewer of them where k allows few: k = 1000, 1000 x 1000 61 / 83 (four splits / two),
 // 2000 x 602 104 / 162, 256 x 4000 61 / 82; k = 3000 119 / 79, 214 / 97, 120 / 77.

@@ -94,6 +94,37 @@ def test_values_without_three_parts(cuda, transposed):
     _check(got[neighbours], clean[neighbours].double() * 0.01, (k + 4) * 2.0 ** -23 * (a[neighbours].double().abs() @ w.abs()))
 
 
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,k,n", [(90_000, 100, 64), (100_001, 64, 129), (6_500, 416, 250), (6_500, 417, 250)])
+def test_values_whose_last_bits_bf16_has_not(cuda, m, k, n, transposed):
+    """Tiny values beside large ones in one row or column: they are lost in three parts (below 2^-133) and count where the others meet zeros."""
+    gen = torch.Generator(device=cuda).manual_seed(6)
+    a, b = torch.randn((m, k), generator=gen, device=cuda), torch.randn((k, n), generator=gen, device=cuda)
+    tiny = torch.rand((m, k), generator=gen, device=cuda) < 0.01
+    a[tiny] *= 1e-37                      # (which do not count)
+    few = 2.0 ** -120 * (1 + 2.0 ** -20)  # 21 bits, of which bf16 holds 14
+    rows = [5, 1000, m - 1]
+    a[rows] = 0
+    a[rows, 0], a[rows, 1] = 1, few
+    b[0, 7], b[1, 7] = 0, 2.0 ** 110
+    b[:, n - 1] = 0                       # the same in a column
+    b[2, n - 1], b[k - 1, n - 1] = 1, few
+    a[77], a[77, k - 1] = 0, 2.0 ** 110
+    w = b.t().contiguous() if transposed else b
+    got = ops.row_product(a, w, transposed)
+    assert _kernel() == b"split_product_kernel"
+    want = a.double() @ b.double()
+    one = torch.cat((got[rows, 7], got[77, n - 1:]))
+    assert bool((one == few * 2.0 ** 110).all())
+    rest = torch.ones((m, n), dtype=torch.bool, device=cuda)
+    rest[77], rest[:, 7] = False, False
+    assert bool(((got.double() - want).abs() <= (k + 2) * 2.0 ** -24 * (a.double().abs() @ b.double().abs()))[rest].all())
+    # results that are subnormal: each term and each sum is rounded to a multiple of 2^-149 once
+    a, b = torch.randn((m, k), generator=gen, device=cuda) * 1e-28, torch.randn((k, n), generator=gen, device=cuda) * 1e-12
+    got = ops.row_product(a, b.t().contiguous() if transposed else b, transposed)
+    assert bool(((got.double() - a.double() @ b.double()).abs() <= (k + 2) * 2.0 ** -149).all())
+
+
 @pytest.mark.parametrize("m,k,n,split", [(1_300_001, 100, 64, True), (1_300_001, 100, 66, False), (8192, 256, 602, True), (3000, 256, 602, False), (8192, 602, 256, False),
                                          (2048, 256, 2000, True), (1999, 256, 2000, False), (3000, 256, 1000, False), (3000, 100, 2000, True), (200, 256, 20000, False),
                                          (300_001, 200, 160, False), (600_001, 384, 40, False)])

@@ -99,3 +99,26 @@ def test_workspace_of_the_fp32_form(cuda):
         assert rc == 0 and lib.fgl_product_last_kernel() == kernel
         assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size).all())
     assert _through_c(a, b, 1024)[0] != 0
+
+
+@pytest.mark.parametrize("k", [64, 5000, 30011])
+def test_values_whose_last_bits_bf16_has_not(cuda, k):
+    """Tiny values beside large ones in one column: they are lost in three parts (below 2^-133) and count where the others meet zeros."""
+    m, n = 100, 256
+    gen = torch.Generator(device=cuda).manual_seed(k)
+    a, b = torch.randn((k, m), generator=gen, device=cuda), torch.randn((k, n), generator=gen, device=cuda)
+    b[torch.rand((k, n), generator=gen, device=cuda) < 0.001] *= 1e-37  # (which do not count)
+    few = 2.0 ** -120 * (1 + 2.0 ** -20)
+    a[:, 20] = 0
+    a[0, 20], a[k - 1, 20] = 1, few
+    b[0, 7], b[k - 1, 7] = 0, 2.0 ** 110
+    b[:, 200] = 0
+    b[3, 200], b[k // 2, 200] = 1, few
+    a[3, 50], a[k // 2, 50] = 0, 2.0 ** 110
+    got = ops.weight_grad(a, b)
+    assert L.lib().fgl_product_last_kernel() == b"wgrad_kernel in parts"
+    assert float(got[20, 7]) == float(got[50, 200]) == few * 2.0 ** 110
+    want, size = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+    keep = torch.ones((m, n), dtype=torch.bool, device=cuda)
+    keep[50], keep[:, 7] = False, False
+    assert bool(((got.double() - want).abs() <= (k / 16 + 16) * 2.0 ** -24 * size)[keep].all())
