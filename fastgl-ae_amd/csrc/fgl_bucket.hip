@@ -162,17 +162,21 @@ __device__ __forceinline__ void load_columns(const BucketArgs& g, int64_t first,
 
 // A tile's entries by bucket.  (A lane's entries are neighbours, and equal ones are counted together: sorted ids -- a CSR's
 // rows -- would otherwise be 64 updates of one counter at a time, one after the other.)
-// DIRECT (counting only): a tile of runs of equal ids in ascending order -- kDirectRun entries a run on average, and its first id
-// none below the last of the tile before: the destinations of an edge list in order -- is counted here, one atomic a run in device
-// memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.  Runs in no order may be of the
-// same few ids over and over, whose updates LDS takes and device memory does not, and ascending ones too, in every few tiles, which
-// is why they have to be long.  (Whole counts, us, by buckets alone / with it: 54 M destinations of an R-MAT graph of 2.4 M nodes
-// 274 / 187, sorted uniform ids 268 / 182, in no order 282 / 284; 20 M over 100 K, sorted 82 / 50; 5 M over 600 K, sorted, eight a
-// run and so not direct, 40.7 / 42.0, in no order 37.5 / 38.2.  In ascending stretches of 1 M ids over 100 K, ten a run, 179 / 181,
-// of 2 M, twenty, 179 / 141.  kDirectRun of 8: the graph 176, the stretches 210 and 141, of 20 K ids over 2 K 255 / 669.  When the
-// tile's first wave alone was looked at, for runs of four, fives of two ids in turn took 122477, tiles in order up to their eighth
-// 1857.)
-constexpr int kDirectRun = 14;
+// DIRECT (counting only): a tile of an input in order, in runs of equal ids -- the destinations of an edge list -- is counted
+// here, one atomic a run in device memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.
+// In order is more than the tile's own ids: device memory does not take updates of the same few counters from all over the chip.
+// So the first ids of the input's 64 parts of neighbouring tiles have to ascend, and the tile's ids, from the tile before on, to
+// lie between those of its part and the next one: a counter is touched by tiles of one part, most of them one XCD's, or of parts
+// that hold one id.  Within a part ids may still recur, which costs least where runs are long.
+// Whole counts, us, by buckets alone / with it: 54 M destinations of an R-MAT graph of 2.4 M nodes 274 / 183, sorted uniform ids,
+// 22 a run, 270 / 187, 11 a run 277 / 252, in no order 280 / 284; 20 M over 100 K, sorted 82 / 53; 5 M over 400 K, sorted, 43 /
+// 39, over 600 K, eight a run and so not direct, 41 / 42, in no order 37.4 / 38.5.  Sorted stretches, which only cost the look:
+// 54 M in stretches of two tiles over 500 ids 254 / 262, of 2 M ids over 130 K 180 / 187.
+// kDirectRun of 8: 11 a run 251, but stretches of two tiles whose ids begin anew for each 64th part, eight a run, 180 / 204; of 4
+// 180 / 510 for such of five a run; of 14 the graph 192.  Without the parts, stretches of two tiles over 500 ids took 879; when
+// the tile's first wave alone was looked at, for runs of four, fives of two ids in turn 122477, tiles in order up to their eighth
+// 1857.
+constexpr int kDirectRun = 10;
 
 template <bool DIRECT>
 __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
@@ -190,10 +194,10 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketA
     bool direct = false;
     if constexpr (DIRECT) {
         constexpr int kWaves = kBucketBlock / kWave;
-        __shared__ int s_direct, s_runs, s_last[kBucketBlock], s_first[kWaves];
+        __shared__ int s_direct, s_most, s_runs, s_last[kBucketBlock], s_first[kWaves];
         const int lane = lane_id(), wave = tid / kWave;
-        // one wave looks at its 1024 entries, for all: what the others would see costs an input in no order 2 % of the whole count
-        // (the runs that begin in the wave, and whether the lane's ids ascend)
+        // one wave looks at its 1024 entries, for all: what the others would see costs an input in no order 2 % of the whole
+        // count (the runs that begin in the wave, and whether the lane's ids ascend)
         auto look = [&](int last, bool& ascends) {
             int begin = c[0] != last;
             ascends = c[0] >= last;
@@ -211,9 +215,24 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketA
         if (tid < kWave) {
             const int last = __shfl_up(c[kBucketItems - 1], 1, kWave);
             const int runs = look(tid > 0 ? last : before < g.n_cols ? before : -1, ascends);
-            const bool may_be = __all(ascends) && runs <= kWave * kBucketItems / kDirectRun;
+            bool may_be = __all(ascends) && runs <= kWave * kBucketItems / kDirectRun;
+            int most = INT32_MAX;
+            if (may_be) {  // (uniform) the first ids of the input's parts, a lane each
+                const int per = (int)((g.tiles + kWave - 1) / kWave), part = (int)tile / per;
+                const int64_t at = (int64_t)lane * per * kBucketTile;
+                int begin = INT32_MAX;
+                if (at < n) {
+                    begin = g.ids[at];
+                    if (begin >= g.n_cols) begin = -1;
+                }
+                int next = __shfl_down(begin, 1, kWave);
+                if (lane == kWave - 1) next = INT32_MAX;
+                most = __shfl(next, part, kWave);
+                may_be = __all(begin <= next) && __all(c[0] >= __shfl(begin, part, kWave));
+            }
             if (tid == 0) {
                 s_direct = may_be;
+                s_most = most;
                 s_runs = 0;
             }
         }
@@ -224,7 +243,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketA
             __syncthreads();
             const int runs = look(tid > 0 ? s_last[tid - 1] : -1, ascends);
             if (lane == 0) atomicAdd(&s_runs, runs);
-            direct = __syncthreads_and(ascends) != 0 && s_runs <= kBucketTile / kDirectRun;
+            direct = __syncthreads_and(ascends && c[kBucketItems - 1] <= s_most) != 0 && s_runs <= kBucketTile / kDirectRun;
         }
         if (tid == 0) g.direct[tile] = direct;
         if (direct) {

@@ -1,6 +1,7 @@
-"""Counts of large inputs that lie in runs of equal ids (csrc/fgl_bucket.hip): sorted ids, hubs over several tiles of 8192, runs on
-either side of the limit of fourteen entries, in order and in none, tiles of either kind in turn, tiles in order only at their beginning or
-up to their last entries, ids that no counter has -- against torch.bincount; and that ids which recur in runs take no longer."""
+"""Counts of large inputs that lie in runs of equal ids (csrc/fgl_bucket.hip): sorted ids, hubs over several tiles of 8192, runs
+on either side of the limit of ten entries, in order and in none, tiles of either kind in turn, tiles in order only at their
+beginning or up to their last entries, sorted stretches one after another, also as long as the 64th parts of the input or with ids
+beyond those, ids that no counter has -- against torch.bincount; and that ids which recur in runs take no longer."""
 import pytest
 import torch
 
@@ -8,7 +9,7 @@ from fastgl import ops
 
 pytestmark = pytest.mark.gpu
 N, BINS, TILE = 3_000_017, 700_000, 8192
-UP = {"fives up": 5, "thirteens up": 13, "fourteens up": 14, "fifteens up": 15, "hundreds up": 100, "hundreds down": 100}
+UP = {"fives up": 5, "nines up": 9, "tens up": 10, "elevens up": 11, "hundreds up": 100, "hundreds down": 100}
 
 
 def _ids(kind, gen, dev):
@@ -32,6 +33,11 @@ def _ids(kind, gen, dev):
         x = torch.randint(0, BINS, (N,), generator=gen, device=dev)
         in_runs = (torch.arange(N, device=dev) // TILE) % 2 == 0
         return torch.where(in_runs, torch.arange(N, device=dev) // 23 % BINS, x)
+    if kind.startswith("stretches"):  # sorted ones, of two tiles, of a part of six tiles, of five tiles with a few high ids at their ends
+        i = torch.arange(N, device=dev)
+        long = {"stretches": 2, "stretches of a part": 6, "stretches beyond": 5}[kind] * TILE
+        base = i // long * (long // 16) if kind == "stretches of a part" else 0
+        return torch.where((i % long > long - 20) & (kind == "stretches beyond"), BINS - 1, base + i % long // 16)
     x = torch.randint(0, BINS // (8 if kind.startswith("long") else 1), (N,), generator=gen, device=dev).sort()[0]
     if kind == "long sorted":  # (34 a run: counted where their histogram is taken)
         return x
@@ -42,7 +48,7 @@ def _ids(kind, gen, dev):
     return x
 
 
-@pytest.mark.parametrize("kind", ["sorted", "long sorted", "hub", "threes", "fours", "fives", *UP, "beginnings", "mixed", "gaps", "long gaps"])
+@pytest.mark.parametrize("kind", ["sorted", "long sorted", "hub", "threes", "fours", "fives", *UP, "stretches", "stretches of a part", "stretches beyond", "beginnings", "mixed", "gaps", "long gaps"])
 def test_counts(cuda, kind):
     print("runs", kind, flush=True)
     x = _ids(kind, torch.Generator(device=cuda).manual_seed(7), cuda)
@@ -52,12 +58,12 @@ def test_counts(cuda, kind):
         assert torch.equal(ops.cal_deg(part, BINS), want)
 
 
-@pytest.mark.parametrize("bins", [2, 1000, 2048])
-def test_ids_that_recur_in_runs(cuda, bins):
-    """An atomic a run in device memory would take hundreds of times as long here (54 M ids, fives of two ids in turn: 122 ms against 0.26)."""
-    n = 5_000_000
+@pytest.mark.parametrize("n,bins,times", [(5_000_000, 2, 10), (5_000_000, 1000, 10), (5_000_000, 2048, 10), (54_000_000, 497, 2)])
+def test_ids_that_recur_in_runs(cuda, n, bins, times):
+    """An atomic a run in device memory would take hundreds of times as long for the first of these (54 M ids, fives of two ids in
+    turn: 122 ms against 0.26), and more than three times as long for the last, sorted stretches of two tiles (880 us against 260)."""
     i = torch.arange(n, device=cuda)
-    runs = (i % TILE // 4 if bins == 2048 else i // 5 % bins).int()
+    runs = (i % (2 * TILE) // 33 if bins == 497 else i % TILE // 4 if bins == 2048 else i // 5 % bins).int()
     no_order = torch.randint(0, bins, (n,), device=cuda, dtype=torch.int32)
 
     def time(x):
@@ -72,4 +78,4 @@ def test_ids_that_recur_in_runs(cuda, bins):
             best = min(best, begin.elapsed_time(end))
         return best
 
-    assert time(runs) < 10 * time(no_order)
+    assert time(runs) < times * time(no_order)
