@@ -19,6 +19,7 @@ struct RowProductArgs {
     int n;
     int tiles_n;          // tiles of C along n
     int64_t row_blocks;   // workgroups along m
+    int vec_log;          // (split products) log2 of the neighbouring columns a lane stores
 };
 
 __device__ __forceinline__ uint32_t rp_bf16_bits(float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)v); }

@@ -70,20 +70,16 @@ __device__ __forceinline__ int sp_first(int s, int k)
 // The k of one product in steps of 16, two steps to a chunk.  (Where the steps are odd in number the last is one of zeros.)
 __device__ __host__ __forceinline__ int sp_chunks(int k) { return (k + 31) / 32; }
 
-// Column of tile t, lane i (of 32), from the workgroup's first one: a lane's columns are neighbours by fours
-template <int NT>
-__device__ __forceinline__ int sp_column(int t, int i)
-{
-    constexpr int kVec = NT < 4 ? NT : 4;
-    return t / kVec * 32 * kVec + i * kVec + t % kVec;
-}
+// Column of tile t, lane i (of 32), from the workgroup's first one: a lane's columns are neighbours by ones, twos or fours (1 << vl), as wide as its
+// stores may be and no wider than they are aligned (n = 126 in misaligned vectors of four: 600 K x 64 x 126 164 us where 124 columns take 99).
+__device__ __forceinline__ int sp_column(int vl, int t, int i) { return ((t >> vl) << (5 + vl)) + (i << vl) + (t & ((1 << vl) - 1)); }
 
 // The steps of B's columns from col0 on -> img[step * NT + tile][part][lane], and the largest magnitude of each (magnitudes are in order as whole numbers too).  Four eights of k of one column a thread at a time, so that
 // their loads are in flight together.
 template <int NT, bool BT, int THREADS>
-__device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, SpU4* img, float* most, uint32_t* rest)
+__device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, int vl, SpU4* img, float* most, uint32_t* rest)
 {
-    constexpr int kVec = NT < 4 ? NT : 4, kCols = 32 * NT, kBatch = 4;
+    constexpr int kCols = 32 * NT, kBatch = 4;
     const float* b = static_cast<const float*>(x.b);
     const int items = steps * 2 * kCols;
     for (int first = (int)threadIdx.x; first < items; first += THREADS * kBatch) {
@@ -113,7 +109,7 @@ __device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int
         for (int i = 0; i < kBatch; ++i) {
             const int at = first + i * THREADS, oct = at / kCols, col = at % kCols;
             if (at >= items) break;
-            const int in_group = col % (32 * kVec), t = col / (32 * kVec) * kVec + in_group % kVec;
+            const int t = (col >> (5 + vl) << vl) + (col & ((1 << vl) - 1)), i_of = (col >> vl) & 31;
             float m = 0.0f;
             sp_most(v[i], m);
             atomicMax(reinterpret_cast<int*>(most + col), __float_as_int(m));
@@ -121,7 +117,7 @@ __device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int
             uint32_t r = 0;
             sp_split(v[i], p, r);
             if (sp_loses(r)) rest[col] = 1;
-            SpU4* to = img + ((oct / 2) * NT + t) * 3 * kWave + oct % 2 * 32 + in_group / kVec;
+            SpU4* to = img + ((oct / 2) * NT + t) * 3 * kWave + oct % 2 * 32 + i_of;
 #pragma unroll
             for (int q = 0; q < 3; ++q) to[q * kWave] = p[q];
         }
@@ -248,10 +244,52 @@ __device__ __forceinline__ void sp_plain(const float* a, const RowProductSide& x
     }
 }
 
+// A tile of 32 rows to C, V neighbouring columns a lane.
+template <int NT, int V, int FORM>
+__device__ __forceinline__ void sp_store_tile(const RowProductArgs& g, int64_t row0, int col0, const SpF32x16 (&acc)[NT])
+{
+    int64_t ldc = g.ldc;
+    int lane = lane_id();
+    asm volatile("" : "+s"(ldc), "+v"(lane));  // (else what all widths make of them is kept in registers, and others spilled, all the while)
+    const int half = lane / 32;
+    float* out = static_cast<float*>(g.c) + (row0 + 4 * half) * ldc + col0;
+    const bool rows = row0 + 32 <= g.m;  // (uniform)
+#pragma unroll
+    for (int q = 0; q < NT / V; ++q) {
+        const int at = 32 * V * q + lane % 32 * V, left = g.n - col0 - at;
+        float add[V];
+#pragma unroll
+        for (int t = 0; t < V; ++t) {
+            add[t] = 0.0f;
+            if (g.bias != nullptr && t < left) add[t] = static_cast<const float*>(g.bias)[col0 + at + t];
+        }
+        if (rows && left >= V) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float* p = out + at + (8 * (r / 4) + r % 4) * ldc;
+                float v[V];
+#pragma unroll
+                for (int t = 0; t < V; ++t) v[t] = acc[q * V + t][r] + add[t];
+                if constexpr (FORM == kRpAdd) rp_add<float, V>(p, v);
+                rp_store<float, V>(p, v);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float* p = out + at + (8 * (r / 4) + r % 4) * ldc;
+                const bool in = row0 + 8 * (r / 4) + 4 * half + r % 4 < g.m;
+#pragma unroll
+                for (int t = 0; t < V; ++t)
+                    if (in && t < left) p[t] = (acc[q * V + t][r] + add[t]) + (FORM == kRpAdd ? p[t] : 0.0f);
+            }
+        }
+    }
+}
+
 template <int NT, int W, bool BT, int FORM>
 __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowProductArgs g)
 {
-    constexpr int kVec = NT < 4 ? NT : 4, kThreads = W * kWave;
+    constexpr int kThreads = W * kWave;
     extern __shared__ SpU4 s_img[];
     __shared__ float s_most[2][32 * NT];     // of each column: its largest magnitude, and whether its values lose bits
     __shared__ uint32_t s_rest[2][32 * NT];
@@ -301,8 +339,8 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
         (&s_rest[0][0])[threadIdx.x] = 0;
     }
     __syncthreads();
-    sp_stage<NT, BT, kThreads>(g.side[0], 2 * chunks0, col0, g.n, s_img, s_most[0], s_rest[0]);
-    if constexpr (FORM == kRpSum) sp_stage<NT, BT, kThreads>(g.side[1], 2 * (chunks - chunks0), col0, g.n, s_img + chunks0 * 2 * NT * 3 * kWave, s_most[1], s_rest[1]);
+    sp_stage<NT, BT, kThreads>(g.side[0], 2 * chunks0, col0, g.n, g.vec_log, s_img, s_most[0], s_rest[0]);
+    if constexpr (FORM == kRpSum) sp_stage<NT, BT, kThreads>(g.side[1], 2 * (chunks - chunks0), col0, g.n, g.vec_log, s_img + chunks0 * 2 * NT * 3 * kWave, s_most[1], s_rest[1]);
     __syncthreads();
     if (tile >= row_tiles) return;  // (uniform over the wave; no barrier follows)
     bool columns_lose = false;
@@ -357,7 +395,7 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
             for (int i = 0; i < 16; ++i) row_most[i] = __shfl(row_loses ? -mine : mine, 8 * (i / 4) + 4 * half + i % 4, kWave);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int c = sp_column<NT>(t, own), col = col0 + c < g.n ? col0 + c : g.n - 1;
+                const int c = sp_column(g.vec_log, t, own), col = col0 + c < g.n ? col0 + c : g.n - 1;
                 const bool column_loses = (s_rest[0][c] | s_rest[1][c]) != 0;
                 const float column_most = fmaxf(s_most[0][c], s_most[1][c]);
                 bool small = (odd >> t & 1) != 0;
@@ -371,38 +409,9 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
             }
             w.template read_b<0>(s_img + lane);  // (what was read ahead: its registers are free above)
         }
-        float* out = static_cast<float*>(g.c) + (row0 + 4 * half) * g.ldc + col0;
-        const bool rows = row0 + 32 <= g.m;  // (uniform)
-#pragma unroll
-        for (int q = 0; q < NT / kVec; ++q) {
-            const int at = sp_column<NT>(q * kVec, lane % 32), left = g.n - col0 - at;
-            float add[kVec];
-#pragma unroll
-            for (int t = 0; t < kVec; ++t) {
-                add[t] = 0.0f;
-                if (g.bias != nullptr && t < left) add[t] = static_cast<const float*>(g.bias)[col0 + at + t];
-            }
-            if (rows && left >= kVec) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    float* p = out + at + (8 * (r / 4) + r % 4) * g.ldc;
-                    float v[kVec];
-#pragma unroll
-                    for (int t = 0; t < kVec; ++t) v[t] = acc[q * kVec + t][r] + add[t];
-                    if constexpr (FORM == kRpAdd) rp_add<float, kVec>(p, v);
-                    rp_store<float, kVec>(p, v);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    float* p = out + at + (8 * (r / 4) + r % 4) * g.ldc;
-                    const bool in = row0 + 8 * (r / 4) + 4 * half + r % 4 < g.m;
-#pragma unroll
-                    for (int t = 0; t < kVec; ++t)
-                        if (in && t < left) p[t] = (acc[q * kVec + t][r] + add[t]) + (FORM == kRpAdd ? p[t] : 0.0f);
-                }
-            }
-        }
+        if (NT >= 4 && g.vec_log == 2) sp_store_tile<NT, NT < 4 ? 1 : 4, FORM>(g, row0, col0, acc);
+        else if (NT >= 2 && g.vec_log == 1) sp_store_tile<NT, NT < 2 ? 1 : 2, FORM>(g, row0, col0, acc);
+        else sp_store_tile<NT, 1, FORM>(g, row0, col0, acc);
         tile += stride;
         if (tile >= row_tiles) return;
         w.clear();
@@ -441,6 +450,9 @@ static int launch_split_product(RowProductArgs g, hipStream_t stream)
     // eight waves a CU (two a SIMD, as the registers allow), in as many workgroups as their LDS allows
     int64_t per_cu = kSpLds / (int64_t)lds;
     if (per_cu > 8 / W) per_cu = 8 / W;
+    // as many neighbouring columns a lane as every row's start allows
+    const uint64_t starts = (uintptr_t)g.c | (uint64_t)g.ldc * sizeof(float);
+    g.vec_log = NT >= 4 && starts % 16 == 0 ? 2 : NT >= 2 && starts % 8 == 0 ? 1 : 0;
     g.row_blocks = sp_row_blocks(ceil_div(g.m, 32), W, 32 * per_cu, g.tiles_n);
     const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
     FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");

@@ -190,3 +190,41 @@ def test_fewer_columns_take_no_longer(cuda, m, k, fewer, more):
         x = a[rows].double()
         _check(got[rows], x @ w.double().t(), (k + 2) * 2.0 ** -24 * (x.abs() @ w.double().abs().t()))
     assert _time(lambda: ops.row_product(a, w, True)) < 1.05 * _time(lambda: ops.row_product(a, b, True))
+
+
+@pytest.mark.parametrize("first,ldc", [(0, 132), (1, 132), (2, 132), (0, 130), (3, 131), (0, 127)])
+@pytest.mark.parametrize("m,k,n", [(180_001, 48, 127), (100_001, 100, 126), (50_001, 832, 33)])
+def test_rows_of_every_alignment(cuda, m, k, n, first, ldc):
+    """Results of which every row starts on a vector of four, of two or of one value: all of them, and nothing beside them."""
+    gen = torch.Generator(device=cuda).manual_seed(ldc)
+    a, b, bias = (torch.randn(s, generator=gen, device=cuda) for s in ((m, k), (k, n), (n,)))
+    base = torch.randn(m * ldc + 8, generator=gen, device=cuda)
+    want = base.clone().as_strided((m, n), (ldc, 1), first)
+    w, lib = b.double(), L.lib()
+    for transposed in (False, True):
+        x = b.t().contiguous() if transposed else b
+        for add in (False, True):
+            buf = base.clone()
+            out = buf.as_strided((m, n), (ldc, 1), first)
+            if add:
+                L.check(lib.fgl_row_product_add(a.data_ptr(), k, x.data_ptr(), x.size(1), int(transposed), m, k, n, L.F32, out.data_ptr(), ldc, L.stream_handle()))
+            else:
+                L.check(lib.fgl_row_product(a.data_ptr(), k, x.data_ptr(), x.size(1), int(transposed), m, k, n, L.F32, bias.data_ptr(), out.data_ptr(), ldc,
+                                            L.stream_handle()))
+            assert _kernel() == b"split_product_kernel"
+            for rows in (slice(0, 3000), slice(m - 3000, m)):
+                more = want[rows].double() if add else bias.double()
+                r = a[rows].double()
+                _check(out[rows], r @ w + more, (k + 2) * 2.0 ** -24 * (r.abs() @ w.abs() + more.abs()))
+            out.copy_(base.as_strided((m, n), (ldc, 1), first))
+            assert torch.equal(buf, base)
+
+
+@pytest.mark.parametrize("n", [125, 126])
+def test_columns_that_fill_no_vectors(cuda, n):
+    """Misaligned stores of four values a lane took 1.7 times as long as aligned ones."""
+    gen = torch.Generator(device=cuda).manual_seed(n)
+    a, b = torch.randn((600_000, 64), generator=gen, device=cuda), torch.randn((128, 64), generator=gen, device=cuda)
+    w = b[:n].contiguous()
+    assert n == 125 or _time(lambda: ops.row_product(a, w, True)) < 1.45 * _time(lambda: ops.row_product(a, b, True))
+    assert _time(lambda: ops.row_product(a, w, True)) < 1.6 * _time(lambda: ops.row_product(a, b, True))
