@@ -263,24 +263,45 @@ __device__ __forceinline__ void sp_store_tile(const RowProductArgs& g, int64_t r
             add[t] = 0.0f;
             if (g.bias != nullptr && t < left) add[t] = static_cast<const float*>(g.bias)[col0 + at + t];
         }
-        if (rows && left >= V) {
+        // What C holds is read for several rows at a time: the compiler keeps each row's loads behind the stores before them, and a row a round trip made
+        // 895 K x 64 x 47 added to C 266 us, this 126 (600 K x 64 x 128, in vectors, 177 and 158).
+        constexpr int kBatch = FORM == kRpAdd ? 16 / V : 16;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float* p = out + at + (8 * (r / 4) + r % 4) * ldc;
+        for (int r0 = 0; r0 < 16; r0 += kBatch) {
+            typedef float Vec __attribute__((ext_vector_type(V), aligned(4)));
+            float* p[kBatch];
+            Vec held[kBatch];
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const int r = r0 + i, row = 8 * (r / 4) + r % 4;
+                p[i] = out + at + row * ldc;
+                held[i] = Vec{};
+                if constexpr (FORM == kRpAdd) {
+                    if (rows && left >= V) {
+                        held[i] = *reinterpret_cast<const Vec*>(p[i]);
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < V; ++t)
+                            if (row0 + 4 * half + row < g.m && t < left) held[i][t] = p[i][t];
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const int r = r0 + i, row = 8 * (r / 4) + r % 4;
                 float v[V];
 #pragma unroll
-                for (int t = 0; t < V; ++t) v[t] = acc[q * V + t][r] + add[t];
-                if constexpr (FORM == kRpAdd) rp_add<float, V>(p, v);
-                rp_store<float, V>(p, v);
-            }
-        } else {
+                for (int t = 0; t < V; ++t) {
+                    v[t] = acc[q * V + t][r] + add[t];
+                    if constexpr (FORM == kRpAdd) v[t] += held[i][t];
+                }
+                if (rows && left >= V) {
+                    rp_store<float, V>(p[i], v);
+                } else {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float* p = out + at + (8 * (r / 4) + r % 4) * ldc;
-                const bool in = row0 + 8 * (r / 4) + 4 * half + r % 4 < g.m;
-#pragma unroll
-                for (int t = 0; t < V; ++t)
-                    if (in && t < left) p[t] = (acc[q * V + t][r] + add[t]) + (FORM == kRpAdd ? p[t] : 0.0f);
+                    for (int t = 0; t < V; ++t)
+                        if (row0 + 4 * half + row < g.m && t < left) p[i][t] = v[t];
+                }
             }
         }
     }
