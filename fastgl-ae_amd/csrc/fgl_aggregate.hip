@@ -2016,27 +2016,43 @@ static int launch_agg_vec(int mode, int64_t longest_row_max, int64_t n_entries_m
     }
 }
 
-// Rows of x without entries in the CSR become zeros.  A wave looks at kZeroRows rows, a lane each, and clears those found one after another,
-// T bytes a lane.  What bounds it is one wave's chain of stores, not their bytes, where a third of the rows are
-// empty: 64 rows a wave and two bytes a lane 10.4 us a launch, 16 rows and 16 bytes 4.2 (the layers of a step over 107 K rows of 100 and 17 K of
-// 256 fp32 columns, about what a launch alone takes).
-constexpr int kZeroRows = 16;
+// Rows of x without entries in the CSR become zeros.  A wave looks at ROWS rows, a lane each, and clears those found one after another,
+// T bytes a lane.  What bounds it is one wave's chain of stores, not their bytes, where a third of the rows are empty and the chip is not
+// full of waves: 64 rows a wave and two bytes a lane 10.4 us a launch, 16 rows and 16 bytes 4.2 (the layers of a step over 107 K rows of 100
+// and 17 K of 256 fp32 columns, about what a launch alone takes).  From a million rows on the waves' number counts instead: us, 64 / 16 rows,
+// of 64 fp32 columns, one row in a hundred / three in ten / all empty: 700 K 4.7 / 4.9, 11.2 / 11.4, 26 / 24; 1 M 4.8 / 5.2, 14.0 / 14.6, 40 / 43;
+// 2.7 M 4.9 / 11.1, 40 / 45, 131 / 120.
+constexpr int64_t kZeroManyRows = 1000000;
 
-template <typename T>
+template <typename T, int ROWS>
 __global__ __launch_bounds__(kBlock) void zero_empty_rows_kernel(const int32_t* __restrict__ indptr, int64_t n_rows_max,
                                                                  const int32_t* __restrict__ d_n_rows, char* __restrict__ x,
                                                                  int64_t row_stride, int row_values)
 {
     const int64_t n_rows = actual_count(n_rows_max, d_n_rows);
-    const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * kZeroRows;
+    const int64_t first = ((int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * ROWS;
     const int64_t row = first + lane_id();
-    unsigned long long todo = __ballot(lane_id() < kZeroRows && row < n_rows && indptr[row] == indptr[row + 1]);
+    unsigned long long todo = __ballot(lane_id() < ROWS && row < n_rows && indptr[row] == indptr[row + 1]);
     while (todo != 0) {
         const int64_t r = first + __ffsll((long long)todo) - 1;
         todo &= todo - 1;
         T* p = reinterpret_cast<T*>(x + r * row_stride);
         for (int i = lane_id(); i < row_values; i += kWave) p[i] = T{};
     }
+}
+
+template <typename T>
+static int launch_zero_empty_rows(const int32_t* d_indptr, int64_t n_rows_max, const int32_t* d_n_rows, void* d_x, int64_t stride, int bytes, hipStream_t s)
+{
+    const int rows = n_rows_max >= kZeroManyRows ? 64 : 16, values = bytes / (int)sizeof(T);
+    const int64_t blocks = ceil_div(n_rows_max, rows * (kBlock / kWave));
+    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "zero_empty_rows: too many rows");
+    const dim3 grid((unsigned)blocks);
+    char* x = static_cast<char*>(d_x);
+    if (rows == 64) hipLaunchKernelGGL((zero_empty_rows_kernel<T, 64>), grid, dim3(kBlock), 0, s, d_indptr, n_rows_max, d_n_rows, x, stride, values);
+    else hipLaunchKernelGGL((zero_empty_rows_kernel<T, 16>), grid, dim3(kBlock), 0, s, d_indptr, n_rows_max, d_n_rows, x, stride, values);
+    FGL_CHECK_LAUNCH("zero_empty_rows_kernel");
+    return FGL_OK;
 }
 
 // bf16 rows can be moved eight elements at a time when every row starts on a 4-byte boundary
@@ -2138,20 +2154,14 @@ FGL_EXPORT int fgl_zero_empty_rows(const int32_t* d_indptr, int64_t n_rows_max, 
     FGL_REQUIRE(dtype == FGL_F32 || dtype == FGL_BF16, "zero_empty_rows: unknown dtype %d", dtype);
     if (n_rows_max == 0) return FGL_OK;
     FGL_REQUIRE(d_indptr && d_x, "zero_empty_rows: null pointer");
-    const int64_t blocks = ceil_div(n_rows_max, kZeroRows * (kBlock / kWave));
-    FGL_REQUIRE(blocks <= 0x7FFFFFFF, "zero_empty_rows: too many rows");
     const int size = dtype == FGL_F32 ? 4 : 2;
     const int64_t stride = ldx * size;
     const int bytes = D * size;
     const uint64_t starts = (uintptr_t)d_x | (uint64_t)stride | (uint64_t)bytes;  // the widest store that fits every row's start and length
-    const dim3 grid((unsigned)blocks);
     hipStream_t s = as_stream(stream);
-    char* x = static_cast<char*>(d_x);
-    if (starts % 16 == 0) hipLaunchKernelGGL(zero_empty_rows_kernel<uint4>, grid, dim3(kBlock), 0, s, d_indptr, n_rows_max, d_n_rows, x, stride, bytes / 16);
-    else if (starts % 4 == 0) hipLaunchKernelGGL(zero_empty_rows_kernel<uint32_t>, grid, dim3(kBlock), 0, s, d_indptr, n_rows_max, d_n_rows, x, stride, bytes / 4);
-    else hipLaunchKernelGGL(zero_empty_rows_kernel<uint16_t>, grid, dim3(kBlock), 0, s, d_indptr, n_rows_max, d_n_rows, x, stride, bytes / 2);
-    FGL_CHECK_LAUNCH("zero_empty_rows_kernel");
-    return FGL_OK;
+    if (starts % 16 == 0) return launch_zero_empty_rows<uint4>(d_indptr, n_rows_max, d_n_rows, d_x, stride, bytes, s);
+    if (starts % 4 == 0) return launch_zero_empty_rows<uint32_t>(d_indptr, n_rows_max, d_n_rows, d_x, stride, bytes, s);
+    return launch_zero_empty_rows<uint16_t>(d_indptr, n_rows_max, d_n_rows, d_x, stride, bytes, s);
 }
 
 FGL_EXPORT const char* fgl_aggregate_last_mapping(void) { return g_mapping; }
