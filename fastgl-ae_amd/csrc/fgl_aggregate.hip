@@ -1038,9 +1038,10 @@ __global__ __launch_bounds__(kLongBlock) void aggregate_long_rows_kernel(const A
             float acc[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) acc[k] = 0.0f;
-            // chunks of at most LPR entries, of one length so that the groups share the list evenly: 140 entries for eight groups of 64 lanes are five
-            // chunks of 32, two loads of sixteen rows after each other instead of the four of three chunks of 64
-            // (the hubs of a sampled block's transpose: 256 fp32 columns 17.1 -> 11.7 us, with weights 17.8 -> 14.0, bf16 13.7 -> 11.1)
+            // chunks of at most LPR entries, of one length so that the groups share the list evenly: 140 entries for eight groups
+            // of 64 lanes are five chunks of 32, two loads of sixteen rows after each other instead of the four of three chunks
+            // of 64 (the hubs of a sampled block's transpose: 256 fp32 columns 17.1 -> 11.7 us, with weights 17.8 -> 14.0, bf16
+            // 13.7 -> 11.1)
             const int rounds = (b - a - 1) / kLongBlock + 1;
             const int chunk = LPR <= kInFlight ? LPR : ((b - a - 1) / (kGroups * rounds) + kInFlight) / kInFlight * kInFlight;
             for (int64_t base = (int64_t)a + (int64_t)grp * chunk; base < b; base += (int64_t)kGroups * chunk) {
@@ -1160,18 +1161,21 @@ struct SegLists {
 };
 
 // ---- segments in classes ---------------------------------------------------------------
-// Each XCD has its own L2 of 4 MB, 16 K rows of 256 bytes, and a gather that runs on all of them has the same 16 K most mentioned rows in every one.  Here the
-// neighbours are in eight classes by a hash of their ids, an XCD gathers one class of every segment, and its L2 has to hold an eighth of
-// the rows: 128 K different ones on the chip.  On an R-MAT graph of 2.4 M nodes and 54 M entries the 16 K most mentioned rows are 44 % of all mentions and the 128 K
-// most mentioned 78 %; a third of the accesses hit the L2 before, and what missed came through the fabric at 6.2 TB/s, which is what it gives.
-// A launch puts every segment's ids in order of class (a wave a segment, by ballots: the sums' order does not depend on scheduling), the next takes (segment, class)
-// by lane group, workgroup w the class w mod 8 -- workgroups go to the XCDs in turn -- and a row's sums are added up in their order.  32 neighbouring ids are of one class,
-// so that a line of their entry counts is read by one XCD as well.  Right on any mapping of workgroups; only the speed depends on it.
-// MI355X, gcn weights, us, segments as they come / in classes: that graph, 64 fp32 columns 2455 / 1935 -- of it the rows of more than 256 entries 1300 / 800: 655 gathering (11 TB/s of
-// rows), 86 the ids' order, 54 the sums -- 100 columns 3730 / 3120, 128 4800 / 4000, 128 bf16 columns 2560 / 2065; 1.2 M nodes, 27 M entries, 100 fp32 columns 1700 / 1420;
-// 600 K, 13 M, 64 columns 525 / 470, in another place of memory 413 / 413.  The lines: 600 K, 9 M 335 / 330, 1.2 M, 9 M 423 / 434, 300 K, 6.5 M 199 / 218; rows of 128 bytes, of which an L2 holds twice as
-// many, 1165 / 1250.  Graphs without long rows pay two launches more that end at once (600 K rows of 40 entries 1106 / 1106).  Marking the loads of little-mentioned rows
-// as non-temporal instead changed nothing.
+// Each XCD has its own L2 of 4 MB, 16 K rows of 256 bytes, and a gather that runs on all of them has the same 16 K most mentioned
+// rows in every one.  Here the neighbours are in eight classes by a hash of their ids, an XCD gathers one class of every segment,
+// and its L2 has to hold an eighth of the rows: 128 K different ones on the chip.  On an R-MAT graph of 2.4 M nodes and 54 M
+// entries the 16 K most mentioned rows are 44 % of all mentions and the 128 K most mentioned 78 %; a third of the accesses hit
+// the L2 before, and what missed came through the fabric at 6.2 TB/s, which is what it gives. A launch puts every segment's ids
+// in order of class (a wave a segment, by ballots: the sums' order does not depend on scheduling), the next takes (segment,
+// class) by lane group, workgroup w the class w mod 8 -- workgroups go to the XCDs in turn -- and a row's sums are added up in
+// their order.  32 neighbouring ids are of one class, so that a line of their entry counts is read by one XCD as well.  Right on
+// any mapping of workgroups; only the speed depends on it. MI355X, gcn weights, us, segments as they come / in classes: that
+// graph, 64 fp32 columns 2455 / 1935 -- of it the rows of more than 256 entries 1300 / 800: 655 gathering (11 TB/s of rows), 86
+// the ids' order, 54 the sums -- 100 columns 3730 / 3120, 128 4800 / 4000, 128 bf16 columns 2560 / 2065; 1.2 M nodes, 27 M
+// entries, 100 fp32 columns 1700 / 1420; 600 K, 13 M, 64 columns 525 / 470, in another place of memory 413 / 413.  The lines: 600
+// K, 9 M 335 / 330, 1.2 M, 9 M 423 / 434, 300 K, 6.5 M 199 / 218; rows of 128 bytes, of which an L2 holds twice as many, 1165 /
+// 1250.  Graphs without long rows pay two launches more that end at once (600 K rows of 40 entries 1106 / 1106).  Marking the
+// loads of little-mentioned rows as non-temporal instead changed nothing.
 constexpr int kClasses = 8;
 constexpr int kClassEntries = 256;                       // rows of fewer entries have too few a class to be worth eight sums
 constexpr int64_t kClassMinEntries = (int64_t)3 << 22;
@@ -1206,7 +1210,8 @@ static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, bool classes, 
     return l;
 }
 
-// What classes take, 0 where they do not pay.  (The rows that are gathered are the source's; as few rows of results are blocks, of which nothing was measured.)
+// What classes take, 0 where they do not pay.  (The rows that are gathered are the source's; as few rows of results are blocks,
+// of which nothing was measured.)
 static size_t class_bytes(int64_t n_entries_max, int64_t n_rows_max, int64_t n_source_rows, int D, int dtype, int64_t longest_row_max)
 {
     const int64_t row = D * (int64_t)(dtype == FGL_F32 ? sizeof(float) : sizeof(uint16_t)), rows = n_rows_max < n_source_rows ? n_rows_max : n_source_rows;
@@ -1548,8 +1553,9 @@ __global__ __launch_bounds__(kBlock) void aggregate_classes_kernel(const AggArgs
     }
 }
 
-// The rows of several segments: a wave adds a row's partial sums, its lane groups every second, fourth or eighth run of eight of them, and then their sums by a
-// __shfl_xor tree -- an order that depends on the row's length alone.  (A lane group a row, one run after the other, waited 110 us for the 1328 sums in classes of an 85 K-entry row.)
+// The rows of several segments: a wave adds a row's partial sums, its lane groups every second, fourth or eighth run of eight of
+// them, and then their sums by a __shfl_xor tree -- an order that depends on the row's length alone.  (A lane group a row, one
+// run after the other, waited 110 us for the 1328 sums in classes of an 85 K-entry row.)
 template <typename T, int VEC, int LPR>
 __global__ __launch_bounds__(kBlock) void seg_reduce_kernel(const AggArgs g, const SegLists l)
 {
@@ -2016,12 +2022,12 @@ static int launch_agg_vec(int mode, int64_t longest_row_max, int64_t n_entries_m
     }
 }
 
-// Rows of x without entries in the CSR become zeros.  A wave looks at ROWS rows, a lane each, and clears those found one after another,
-// T bytes a lane.  What bounds it is one wave's chain of stores, not their bytes, where a third of the rows are empty and the chip is not
-// full of waves: 64 rows a wave and two bytes a lane 10.4 us a launch, 16 rows and 16 bytes 4.2 (the layers of a step over 107 K rows of 100
-// and 17 K of 256 fp32 columns, about what a launch alone takes).  From a million rows on the waves' number counts instead: us, 64 / 16 rows,
-// of 64 fp32 columns, one row in a hundred / three in ten / all empty: 700 K 4.7 / 4.9, 11.2 / 11.4, 26 / 24; 1 M 4.8 / 5.2, 14.0 / 14.6, 40 / 43;
-// 2.7 M 4.9 / 11.1, 40 / 45, 131 / 120.
+// Rows of x without entries in the CSR become zeros.  A wave looks at ROWS rows, a lane each, and clears those found one after
+// another, T bytes a lane.  What bounds it is one wave's chain of stores, not their bytes, where a third of the rows are empty
+// and the chip is not full of waves: 64 rows a wave and two bytes a lane 10.4 us a launch, 16 rows and 16 bytes 4.2 (the layers
+// of a step over 107 K rows of 100 and 17 K of 256 fp32 columns, about what a launch alone takes).  From a million rows on the
+// waves' number counts instead: us, 64 / 16 rows, of 64 fp32 columns, one row in a hundred / three in ten / all empty: 700 K 4.7
+// / 4.9, 11.2 / 11.4, 26 / 24; 1 M 4.8 / 5.2, 14.0 / 14.6, 40 / 43; 2.7 M 4.9 / 11.1, 40 / 45, 131 / 120.
 constexpr int64_t kZeroManyRows = 1000000;
 
 template <typename T, int ROWS>

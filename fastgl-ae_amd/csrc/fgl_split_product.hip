@@ -1,34 +1,41 @@
-// Products over the rows of a block in fp32 (what fgl_row_product.hip forms, which see), on the bf16 matrix cores: C[m, n] = A[m, k] B[k, n].
+// Products over the rows of a block in fp32 (what fgl_row_product.hip forms, which see), on the bf16 matrix cores: C[m, n] = A[m,
+// k] B[k, n].
 //
-// Why: the fp32 matrix instructions reach 157 TFLOP/s, the bf16 ones 2500.  An fp32 value is the sum of three bf16 values, exactly, so a product is six
-// bf16 products and loses only terms below 2^-26 of it: a2 b0, a0 b2, a1 b1, a1 b0, a0 b1, a0 b0 of a = a0 + a1 + a2, b = b0 + b1 + b2, 2.6 times the rate.
+// Why: the fp32 matrix instructions reach 157 TFLOP/s, the bf16 ones 2500.  An fp32 value is the sum of three bf16 values,
+// exactly, so a product is six bf16 products and loses only terms below 2^-26 of it: a2 b0, a0 b2, a1 b1, a1 b0, a0 b1, a0 b0 of
+// a = a0 + a1 + a2, b = b0 + b1 + b2, 2.6 times the rate.
 //
-// How exact.  Every product of two parts is exact, and what a matrix instruction adds up is cut to 26 bits of its largest term.  So the 32 k of a chunk are
-// added up from zero, the small products first, and only their sum is added to the accumulators, in fp32: errors of a sum of k terms grow with k / 32 where they
-// grew with k.  Against 64-bit sums, 2-norm, normal / non-negative operands (the fp32 instructions in brackets): k = 100 5.8e-8 / 4.7e-8 (1.8e-7 / 1.4e-7),
-// k = 256 7.0e-8 / 5.1e-8 (2.9e-7 / 2.5e-7), k = 800 1.1e-7 / 7.1e-8 (5.1e-7 / 3.8e-7).  Added to the accumulators directly the errors of k = 602 were
-// those of the fp32 instructions and larger, because the cut then is at the accumulator's 26 bits.
-// Values without such parts: infinite, not a number or rounded to infinity ones make results that are no finite numbers.  Values below 2^-110 may have bits below
-// 2^-133, bf16's last, which are lost; they matter to a result that is not large beside them (sp_least), and subnormal results have no room for the small products.
-// 32 columns of a tile with a result of these kinds are formed again in fp32 matrix instructions.  (us, 107 K x 256 x 256, B transposed / not: 90 / 90; one column
-// of B at 1e-36 191 / 232, where the fp32 kernel alone takes 161 / 144; a hundredth of A's rows at 1e-37 158 / 181; a hundredth of A's values, or one row of B, at
-// 1e-37, which change no result, 97 / 95.)
+// How exact.  Every product of two parts is exact, and what a matrix instruction adds up is cut to 26 bits of its largest term.
+// So the 32 k of a chunk are added up from zero, the small products first, and only their sum is added to the accumulators, in
+// fp32: errors of a sum of k terms grow with k / 32 where they grew with k.  Against 64-bit sums, 2-norm, normal / non-negative
+// operands (the fp32 instructions in brackets): k = 100 5.8e-8 / 4.7e-8 (1.8e-7 / 1.4e-7), k = 256 7.0e-8 / 5.1e-8 (2.9e-7 /
+// 2.5e-7), k = 800 1.1e-7 / 7.1e-8 (5.1e-7 / 3.8e-7).  Added to the accumulators directly the errors of k = 602 were those of the
+// fp32 instructions and larger, because the cut then is at the accumulator's 26 bits.
+// Values without such parts: infinite, not a
+// number or rounded to infinity ones make results that are no finite numbers.  Values below 2^-110 may have bits below 2^-133,
+// bf16's last, which are lost; they matter to a result that is not large beside them (sp_least), and subnormal results have no
+// room for the small products. 32 columns of a tile with a result of these kinds are formed again in fp32 matrix instructions.
+// (us, 107 K x 256 x 256, B transposed / not: 90 / 90; one column of B at 1e-36 191 / 232, where the fp32 kernel alone takes 161
+// / 144; a hundredth of A's rows at 1e-37 158 / 181; a hundredth of A's values, or one row of B, at 1e-37, which change no
+// result, 97 / 95.)
 //
 // What bounds it: for short k and few columns the pass over A and C, beyond that the matrix cores and the vector unit beside them.
 //
-// Split: a workgroup keeps its 32 NT columns of B in LDS, already in parts and in the order in which the lanes take them, and its waves go over the rows of
-// A in tiles of 32, each by itself: no barrier after the first.  A lane reads its row of A straight to registers, a chunk ahead, and splits it; so the
-// splitting costs each wave once for NT tiles, and no row is staged.  B is staged once for as many rows as there are, which is what a row tile a workgroup cannot do (both
-// operands through LDS by tiles of 128 x 128: 107 K x 100 x 256 60 us where this takes 49).
-// Beside each matrix instruction (32 cycles) the vector unit has room for about six others: the splitting of the next step (44 a step) and the addition of the last
-// round's sums (16 a tile) are dealt out between them, which the compiler does not do by itself.  Left to its order, with the same instructions, 107 K x 256 x 256 takes 96 us.
+// Split: a workgroup keeps its 32 NT columns of B in LDS, already in parts and in the order in which the lanes take them, and its
+// waves go over the rows of A in tiles of 32, each by itself: no barrier after the first.  A lane reads its row of A straight to
+// registers, a chunk ahead, and splits it; so the splitting costs each wave once for NT tiles, and no row is staged.  B is staged
+// once for as many rows as there are, which is what a row tile a workgroup cannot do (both operands through LDS by tiles of 128 x
+// 128: 107 K x 100 x 256 60 us where this takes 49). Beside each matrix instruction (32 cycles) the vector unit has room for
+// about six others: the splitting of the next step (44 a step) and the addition of the last round's sums (16 a tile) are dealt
+// out between them, which the compiler does not do by itself.  Left to its order, with the same instructions, 107 K x 256 x 256
+// takes 96 us.
 //
-// Measured (MI355X, us: the fp32 instructions / the library / this; a transposed B costs no more here): 2.4 M x 100 x 64 550 / 512 / 338 (4.7 TB/s),
-// 2.4 M x 64 x 100 450 / 627 / 325 (4.8 TB/s), 107 K x 100 x 256 77 / 80 / 49, 107 K x 256 x 256 142 / 137 / 85, 17 K x 256 x 256 42 / 24 / 18,
-// 200 K x 128 x 128 85 / 80 / 47, 8192 x 602 x 256 29 / 28 / 25, 8192 x 256 x 602 43 / 36 / 29.
+// Measured (MI355X, us: the fp32 instructions / the library / this; a transposed B costs no more here): 2.4 M x 100 x 64 550 / 511 /
+// 345 (4.6 TB/s), 2.4 M x 64 x 100 449 / 625 / 332 (4.7 TB/s), 107 K x 100 x 256 78 / 81 / 51, 107 K x 256 x 256 149 / 138 / 90,
+// 17 K x 256 x 256 42 / 25 / 27, 200 K x 128 x 128 85 / 81 / 50, 8192 x 602 x 256 27 / 27 / 26, 8192 x 256 x 602 42 / 36 / 28.
 //
-// Rows past the end repeat the last one and are not stored, nor are columns past the end, which repeat the last one too; the last step of k ends with k, and what the step before has
-// of it is zero in LDS.  No access leaves the operands.
+// Rows past the end repeat the last one and are not stored, nor are columns past the end, which repeat the last one too; the last
+// step of k ends with k, and what the step before has of it is zero in LDS.  No access leaves the operands.
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_row_product.hpp"
@@ -70,12 +77,13 @@ __device__ __forceinline__ int sp_first(int s, int k)
 // The k of one product in steps of 16, two steps to a chunk.  (Where the steps are odd in number the last is one of zeros.)
 __device__ __host__ __forceinline__ int sp_chunks(int k) { return (k + 31) / 32; }
 
-// Column of tile t, lane i (of 32), from the workgroup's first one: a lane's columns are neighbours by ones, twos or fours (1 << vl), as wide as its
-// stores may be and no wider than they are aligned (n = 126 in misaligned vectors of four: 600 K x 64 x 126 164 us where 124 columns take 99).
+// Column of tile t, lane i (of 32), from the workgroup's first one: a lane's columns are neighbours by ones, twos or fours (1 <<
+// vl), as wide as its stores may be and no wider than they are aligned (n = 126 in misaligned vectors of four: 600 K x 64 x 126
+// 164 us where 124 columns take 99).
 __device__ __forceinline__ int sp_column(int vl, int t, int i) { return ((t >> vl) << (5 + vl)) + (i << vl) + (t & ((1 << vl) - 1)); }
 
-// The steps of B's columns from col0 on -> img[step * NT + tile][part][lane], and the largest magnitude of each (magnitudes are in order as whole numbers too).  Four eights of k of one column a thread at a time, so that
-// their loads are in flight together.
+// The steps of B's columns from col0 on -> img[step * NT + tile][part][lane], and the largest magnitude of each (magnitudes are
+// in order as whole numbers too).  Four eights of k of one column a thread at a time, so that their loads are in flight together.
 template <int NT, bool BT, int THREADS>
 __device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int col0, int n, int vl, SpU4* img, float* most, uint32_t* rest)
 {
@@ -124,8 +132,9 @@ __device__ __forceinline__ void sp_stage(const RowProductSide& x, int steps, int
     }
 }
 
-// What a wave multiplies and what it has on the way.  A step of 16 k takes P = NT / 2 rounds of two tiles (one, where NT is 1); a round is six matrix
-// instructions a tile, and the vector unit meanwhile adds the round before's sums to the accumulators and splits the step after's values of A.
+// What a wave multiplies and what it has on the way.  A step of 16 k takes P = NT / 2 rounds of two tiles (one, where NT is 1); a
+// round is six matrix instructions a tile, and the vector unit meanwhile adds the round before's sums to the accumulators and
+// splits the step after's values of A.
 template <int NT>
 struct SpWave {
     static constexpr int kTiles = NT < 2 ? 1 : 2, kRounds = NT / kTiles;
@@ -134,7 +143,8 @@ struct SpWave {
     SpU4 b[2][kTiles][3];     // B's values of this round and the next
     SpU4 a[2][3];             // A's of this step and the next
     float x[8], y[2][8];      // A's as loaded: the chunk's second step, the next chunk
-    // of the row as far as it is split, and of the next chunk's first step: what tells whether bits are lost (sp_split), the largest magnitude
+    // of the row as far as it is split, and of the next chunk's first step: what tells whether bits are lost (sp_split), the
+    // largest magnitude
     uint32_t rest, next_rest;
     float most, next_most;
 
@@ -263,8 +273,8 @@ __device__ __forceinline__ void sp_store_tile(const RowProductArgs& g, int64_t r
             add[t] = 0.0f;
             if (g.bias != nullptr && t < left) add[t] = static_cast<const float*>(g.bias)[col0 + at + t];
         }
-        // What C holds is read for several rows at a time: the compiler keeps each row's loads behind the stores before them, and a row a round trip made
-        // 895 K x 64 x 47 added to C 266 us, this 126 (600 K x 64 x 128, in vectors, 177 and 158).
+        // What C holds is read for several rows at a time: the compiler keeps each row's loads behind the stores before them, and
+        // a row a round trip made 895 K x 64 x 47 added to C 266 us, this 126 (600 K x 64 x 128, in vectors, 177 and 158).
         constexpr int kBatch = FORM == kRpAdd ? 16 / V : 16;
 #pragma unroll
         for (int r0 = 0; r0 < 16; r0 += kBatch) {
@@ -441,11 +451,11 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
 
 static size_t sp_lds(const RowProductArgs& g, int nt) { return (size_t)(sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)) * 2 * nt * 3 * kWave * sizeof(SpU4); }
 
-// Row blocks, 8 at a time, one to an XCD with all of its tiles along n.  An XCD has `places` for workgroups at once, and one more than that
-// takes as long as as many again: 7 tiles of 128 columns in 64 places are 9 row blocks (63), not 10.  Where much would be left empty (13 tiles: 4
-// row blocks, 52) more of them in two to four rounds may end sooner: a workgroup takes as long as its waves have row tiles, and two tiles' time to stage B.
-// (us, with one block more than fits / with this: 209 K x 64 x 896 248 / 209, 100 K x 128 x 376 95 / 77, added to C 168 / 112, 119 K x (256 + 256) x 165
-// 302 / 210, 80 K x 256 x 1064 424 / 302.)
+// Row blocks, 8 at a time, one to an XCD with all of its tiles along n.  An XCD has `places` for workgroups at once, and one more
+// than that takes as long as as many again: 7 tiles of 128 columns in 64 places are 9 row blocks (63), not 10.  Where much would
+// be left empty (13 tiles: 4 row blocks, 52) more of them in two to four rounds may end sooner: a workgroup takes as long as its
+// waves have row tiles, and two tiles' time to stage B. (us, with one block more than fits / with this: 209 K x 64 x 896 248 /
+// 209, 100 K x 128 x 376 95 / 77, added to C 168 / 112, 119 K x (256 + 256) x 165 302 / 210, 80 K x 256 x 1064 424 / 302.)
 static int64_t sp_row_blocks(int64_t row_tiles, int waves, int64_t places, int64_t tiles_n)
 {
     const int64_t want = ceil_div(ceil_div(row_tiles, waves), 8);  // (of an XCD: a tile a wave)
@@ -482,8 +492,9 @@ static int launch_split_product(RowProductArgs g, hipStream_t stream)
     return FGL_OK;
 }
 
-// Columns of a workgroup: 64, so that a split value of A serves two tiles and B fits up to k = 416; 32 for fewer columns or a longer k; 128 where k is short
-// and the pass over A is what counts (2.4 M x 64 x 100: 325 us against 404; 200 K x 128 x 128, with one workgroup of four waves left a CU, 50 against 46).
+// Columns of a workgroup: 64, so that a split value of A serves two tiles and B fits up to k = 416; 32 for fewer columns or a
+// longer k; 128 where k is short and the pass over A is what counts (2.4 M x 64 x 100: 325 us against 404; 200 K x 128 x 128,
+// with one workgroup of four waves left a CU, 50 against 46).
 static int sp_tiles(const RowProductArgs& g)
 {
     const int steps = 2 * (sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k));
@@ -491,12 +502,15 @@ static int sp_tiles(const RowProductArgs& g)
     return g.n > 32 && sp_lds(g, 2) <= (size_t)kSpLds ? 2 : 1;
 }
 
-// Whether the split pays, against the fp32 instructions' kernel, which has nothing to stage first and pads less.  A step here is 32 k and 32 to 128 columns: what they
-// pad makes the line higher (us, that kernel / this: 909 K x 8 x 33 42 / 70, 454 K x 8 x 66 31 / 60, 234 K x 16 x 128 27 / 29, 106 K x 33 x 66 18 / 28, but 140 K x 33 x 100
-// 30 / 24), and up to two steps it is higher by another quarter (54 K x 64 x 128 17 / 21, 109 K x 64 x 128 30 / 27).  Otherwise it lies at 4.3e8 multiplications: 100 x 64:
-// 39 K rows 13 / 14, 62 K 15 / 13; 100 x 256: 9800 13 / 12, 27 K 22 / 20; 200 x 128: 13 K 12 / 14, 20 K 21 / 15; 256 x 66: 25 K 21 / 18; 602 x 256: 6400 30 / 24.
-// Workgroups of one row block go to one XCD, eight blocks at a time, so that fewer than 2000 rows leave XCDs idle: 1000 x 256 x 4000 22 / 36, 500 x 602 x 16000 192 / 356,
-// 250 x 832 x 30000 521 / 909, 2000 x 256 x 4000 44 / 40.  Results as few as 1.6e6 take that many rows' worth twice: 3000 x 602 x 602 31 / 44, 4000 x 400 x 400 19 / 21.
+// Whether the split pays, against the fp32 instructions' kernel, which has nothing to stage first and pads less.  A step here is
+// 32 k and 32 to 128 columns: what they pad makes the line higher (us, that kernel / this: 909 K x 8 x 33 42 / 70, 454 K x 8 x 66
+// 31 / 60, 234 K x 16 x 128 27 / 29, 106 K x 33 x 66 19 / 22, but 140 K x 33 x 100 28 / 24).  Otherwise it lies at 4.3e8
+// multiplications: 100 x 64: 39 K rows 13 / 12, 62 K 15 / 13; 100 x 256: 9800 13 / 12, 27 K 22 / 20; 200 x 128: 13 K 12 / 15, 20 K
+// 21 / 15; 256 x 66: 25 K 21 / 17; 602 x 256: 6400 30 / 24; up to two steps at 5e8, where it is ahead by more (64 x 128: 54 K 17 /
+// 16, 109 K 31 / 24).
+// Workgroups of one row block go to one XCD, eight blocks at a time, so that fewer than 2000 rows leave XCDs idle: 1000 x 256 x
+// 4000 22 / 36, 500 x 602 x 16000 192 / 356, 250 x 832 x 30000 521 / 909, 2000 x 256 x 4000 44 / 39.  Results as few as 1.6e6 take
+// that many rows' worth twice: 3000 x 602 x 602 30 / 38, 4000 x 400 x 400 21 / 22.
 bool split_product_pays(const RowProductArgs& g)
 {
     const int k = g.side[0].k + g.side[1].k;

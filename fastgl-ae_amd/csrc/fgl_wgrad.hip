@@ -25,16 +25,18 @@
 // 602 x 256, k = 8192: 57 -> 42 us; bf16 100 x 256, k = 105 K: 245 -> 25 us, 100 x 64, k = 2.4 M: 2745 -> 148 us (5.3 TB/s).
 // Eight rows a step and one step ahead: 16 and 24 rows measured the same within 3 %.
 //
-// The split form of fp32: the fp32 matrix instructions' rate is what the wide tiles wait for, and their 256 accumulators a lane leave one wave a SIMD, which nothing
-// covers while it waits for rows.  Each value is three bf16 parts instead, a product six bf16 products (fgl_split_product.hip says which and how exact that is), in
-// tiles of 64 x 64, two waves a SIMD: one splits (88 instructions for a step's 64 columns) while the other multiplies.  Every step's products are added up from
-// zero before they are added to the accumulators; and since what a matrix instruction cuts off is cut downwards, which over 10^4 .. 10^6 rows adds up (7e-7 of the
-// result's 2-norm for k = 107 K where the fp32 form has 2.8e-7), every other step is formed of A's negative and subtracted: 1.4e-7.
-// us, fp32 / split: 100 x 256 k = 107 K 68 / 65, k = 16 K 33 / 21, k = 2000 26 / 12; 256 x 256 k = 17 K 36 / 29, k = 5000 31 / 16; 128 x 128 k = 60 K 37 / 28;
-// 602 x 256 k = 8192 41 / 38; 256 x 47 k = 20 K 19 / 16.  Waves that meet values of which bits are lost to a result, or results that are no numbers, form their rows again
-// (one column of the first of these at 1e-36: 121).  What it waits for now is the rows: one step ahead is half a microsecond at these rates.
-// Tried: blocks of 128 x 128 through LDS, in which every value is split once (65 us for the first of these, but 34 and 41 for 256 x 256 and 602 x 256), and two steps ahead, for
-// which the registers do not suffice (89).
+// The split form of fp32: the fp32 matrix instructions' rate is what the wide tiles wait for, and their 256 accumulators a lane
+// leave one wave a SIMD, which nothing covers while it waits for rows.  Each value is three bf16 parts instead, a product six
+// bf16 products (fgl_split_product.hip says which and how exact that is), in tiles of 64 x 64, two waves a SIMD: one splits (88
+// instructions for a step's 64 columns) while the other multiplies.  Every step's products are added up from zero before they are
+// added to the accumulators; and since what a matrix instruction cuts off is cut downwards, which over 10^4 .. 10^6 rows adds up
+// (7e-7 of the result's 2-norm for k = 107 K where the fp32 form has 2.8e-7), every other step is formed of A's negative and
+// subtracted: 1.4e-7. us, fp32 / split: 100 x 256 k = 107 K 68 / 65, k = 16 K 33 / 21, k = 2000 26 / 12; 256 x 256 k = 17 K 36 /
+// 29, k = 5000 31 / 16; 128 x 128 k = 60 K 37 / 28; 602 x 256 k = 8192 41 / 38; 256 x 47 k = 20 K 19 / 16.  Waves that meet
+// values of which bits are lost to a result, or results that are no numbers, form their rows again (one column of the first of
+// these at 1e-36: 121).  What it waits for now is the rows: one step ahead is half a microsecond at these rates. Tried: blocks of
+// 128 x 128 through LDS, in which every value is split once (65 us for the first of these, but 34 and 41 for 256 x 256 and 602 x
+// 256), and two steps ahead, for which the registers do not suffice (89).
 //
 // A lane whose columns would leave the row takes the row's last VA columns instead (its sums are then bit-equal copies of
 // its neighbour's); rows past the end are replaced by zeros.  No access leaves the operands.
@@ -214,7 +216,8 @@ __device__ __forceinline__ int wgrad_column(int tile, int i, int n)
     return c + V <= n ? c : n - V;
 }
 
-// acc += the products of the wave's rows between k0 and k1, and sum += the column sums of A's.  col_a, col_b: the lane's first column of either.
+// acc += the products of the wave's rows between k0 and k1, and sum += the column sums of A's.  col_a, col_b: the lane's first
+// column of either.
 template <typename T, int VA, int VB>
 __device__ __forceinline__ void wgrad_rows(const WgradArgs& g, int64_t k0, int64_t k1, int wave, int col_a, int col_b, bool sums, F32x16 (&acc)[VA * VB], float (&sum)[VA])
 {
@@ -265,7 +268,8 @@ __device__ __forceinline__ void wgrad_rows(const WgradArgs& g, int64_t k0, int64
     wgrad_multiply<VA, VB>(a1, b1, acc);
 }
 
-// The same in three bf16 parts a value, the wave's rows being others; true where the lane met values that have none (then acc is not the sum)
+// The same in three bf16 parts a value, the wave's rows being others; true where the lane met values that have none (then acc is
+// not the sum)
 template <int VA, int VB>
 __device__ __forceinline__ bool wgrad_split_rows(const WgradArgs& g, int64_t k0, int64_t k1, int wave, int col_a, int col_b, bool sums, F32x16 (&acc)[VA * VB],
                                                  float (&sum)[VA])
@@ -532,8 +536,8 @@ static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, boo
     const int64_t most = ceil_div(k, 256);  // 256 rows and more per split: the sum over the splits costs as much as they do otherwise
     if (splits > most) splits = most;
     if (splits > 8) splits = splits / 8 * 8;
-    // With many tiles eights of splits fill the chip badly (602 x 256 in 40 tiles: 320 workgroups of 512 places): the first number of them that leaves less than an
-    // eighth of the places empty, also if it takes two rounds
+    // With many tiles eights of splits fill the chip badly (602 x 256 in 40 tiles: 320 workgroups of 512 places): the first
+    // number of them that leaves less than an eighth of the places empty, also if it takes two rounds
     for (int64_t s = 8; split && splits < 32 && s <= 32 && s <= most; s += 8) {
         const int64_t rounds = ceil_div(s * p.tiles, 512) * 512;
         splits = s;
@@ -549,14 +553,16 @@ static WgradPlan wgrad_plan(int64_t k, int m, int n, bool va_ok, bool vb_ok, boo
     return p;
 }
 
-// Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane (with narrow ones it is as fast or
-// faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11; 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that
-// reading the operands once for each tile of 64 is what counts (100 x 256 k = 107 K 68 / 65, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237;
-// with 65 to 128 columns on one side, two tiles, 100 x 4000 k = 20 K 174 / 203, 100 x 602 k = 110 K 159 / 166, 100 x 1000 k = 60 K 142 / 136).  A split's workgroups are one XCD's,
-// so that fewer than eight splits leave XCDs idle; four times the tiles leave room for fewer of them where k allows few: k = 1000, 1000 x 1000 61 / 83 (four splits / two),
-// 2000 x 602 104 / 162, 256 x 4000 61 / 82; k = 3000 119 / 79, 214 / 97, 120 / 77.
-// Fewer rows than a step has are the fp32 form's, whose sums of one and two products are the more exact ones: rms errors against 64 bits, fp32 / split, k = 1
-// 2.5e-8 / 3.5e-8, k = 2 3.1e-8 / 3.4e-8, k = 16 6.1e-8 / 3.4e-8, k = 17 6.5e-8 / 4.3e-8, k = 64 8.6e-8 / 5.5e-8.
+// Whether three parts a value pay: where the fp32 form has wide tiles, of which few waves hold 128 or 256 accumulators a lane
+// (with narrow ones it is as fast or faster: us, fp32 / split, 64 x 64 k = 8000 11 / 12, 64 K 16 / 18; 96 x 40 k = 3000 9 / 11;
+// 172 x 2 k = 20 K 11 / 12), and not where there is so much to multiply that reading the operands once for each tile of 64 is
+// what counts (100 x 256 k = 107 K 68 / 65, 400 K 232 / 247; 256 x 256 k = 130 K 155 / 152, 200 K 227 / 237; with 65 to 128
+// columns on one side, two tiles, 100 x 4000 k = 20 K 174 / 203, 100 x 602 k = 110 K 159 / 166, 100 x 1000 k = 60 K 142 / 136).
+// A split's workgroups are one XCD's, so that fewer than eight splits leave XCDs idle; four times the tiles leave room for fewer
+// of them where k allows few: k = 1000, 1000 x 1000 61 / 83 (four splits / two), 2000 x 602 104 / 162, 256 x 4000 61 / 82; k =
+// 3000 119 / 79, 214 / 97, 120 / 77. Fewer rows than a step has are the fp32 form's, whose sums of one and two products are the
+// more exact ones: rms errors against 64 bits, fp32 / split, k = 1 2.5e-8 / 3.5e-8, k = 2 3.1e-8 / 3.4e-8, k = 16 6.1e-8 /
+// 3.4e-8, k = 17 6.5e-8 / 4.3e-8, k = 64 8.6e-8 / 5.5e-8.
 static bool wgrad_split_pays(int64_t k, int m, int n)
 {
     const int least = m < n ? m : n;

@@ -420,14 +420,17 @@ def _product_operands(a, b, transposed, m, k, n):
 
 
 def _forms_split_product(a, b, transposed, m, k, n):
-    """What ``_forms_row_product`` leaves, and the fp32 kernel on the bf16 matrix cores (csrc/fgl_split_product.hip) forms ahead of the library: more than 8e9
-    multiplications, or weights of more than 100000 values.  GPU time over the library's (N: plain, T: transposed weight), 9e9 multiplications: k = 64 .. 256
-    and n = 64, 100, 128, 256, 300 0.5 .. 0.95 in both layouts (2.4 M x 100 x 64 338 / 512 us, x 64 x 100 325 / 627); but n = 66, which takes two workgroups' columns, 1.03 .. 1.09, n = 160,
-    which takes three and is whole vectors to the library, 1.06 .. 1.18 from k = 200 on, and n = 33 and 47 1.02 .. 1.11 from k = 384 on.  Wide weights: 256 x 602
-    N 0.84 / 0.76 / 0.58, T 0.98 / 0.71 / 0.71 (8192 / 20 K / 60 K rows), 400 x 300 0.61 / 0.49 / 0.77, 300 x 400 0.85 / 0.88 / 0.80; but 4000 rows of these two, fewer
-    than 2.1e6 results, 1.01 .. 1.16, and a k beyond 400, of which only 32 columns at a time fit, 0.9 .. 1.2 (602 x 256: 0.96 .. 1.10).  From 4000 rows on, up to 30000 columns,
-    0.5 .. 0.83; fewer where they fill the XCDs' turns, 2048 rows each, 1024 up to k = 192 (2000 rows: k = 33 .. 400 0.6 .. 0.95; 3000 rows: k = 33 .. 100 0.56 .. 0.9, but
-    200 and 256 up to 1.1; 1500 rows up to 1.3, 1000 rows up to 1.5, 250 rows 3 .. 6)."""
+    """What ``_forms_row_product`` leaves, and the fp32 kernel on the bf16 matrix cores (csrc/fgl_split_product.hip) forms ahead of the
+    library: more than 8e9 multiplications, or weights of more than 100000 values.  us, the library / that kernel, plain weight (T: transposed):
+    2.4 M x 100 x 64 511 / 345, 2.4 M x 64 x 100 626 / 332, 1.2 M x 100 x 128 415 / 322; wide weights 8192 x 256 x 602 36 / 28 (T 33 / 28), 20 K
+    rows 70 / 51 (69 / 52), 60 K 270 / 124 (218 / 126), 400 x 300: 8192 38 / 23, 60 K 179 / 99, 300 x 400: 8192 26 / 23; but 4000 rows of
+    these two, fewer than 2.1e6 results, 18 / 22, and a k beyond 400, of which only 32 columns at a time fit, gains little or nothing: 602 x 256
+    8192 rows 26.9 / 26.4, 20 K 53 / 60, 60 K 151 / 152, 107 K 320 / 300.  n = 66 to 71 in two workgroups' columns, n = 129 to 160 from
+    k = 129 on and n of 33 to 48 from k = 257 on stay the library's too; that was ahead there by up to a fifth of misaligned stores and a last round
+    with few workgroups, without which the kernel is (2.4 M x 100 x 66 655 / 556, 400 K x 200 x 160 330 / 240, 400 K x 400 x 47 204 / 178).
+    From 4000 rows on, up to 30000 columns, 0.5 .. 0.83 of the library's time; fewer where they fill the XCDs' turns, 2048 rows each, 1024 up to
+    k = 192 (2000 rows: k = 33 .. 400 0.6 .. 0.95; 3000 rows: k = 33 .. 100 0.56 .. 0.9, but 200 and 256 up to 1.1; 1500 rows up to 1.3, 1000 rows
+    up to 1.5, 250 rows 3 .. 6)."""
     if not (a.dtype == torch.float32 and 32 < k <= 400 and m * n >= 2.1e6 and not 64 < n < 72 and not (k > 128 and 128 < n <= 160) and
             not (k > 256 and n <= 48)):
         return None
