@@ -236,3 +236,21 @@ def test_an_addition_costs_what_it_reads(cuda):
     a, b, out = (torch.randn(s, generator=gen, device=cuda) for s in ((895_000, 64), (64, 47), (895_000, 47)))
     assert _time(lambda: ops.row_product_add_(out, a, b)) < 2.0 * _time(lambda: ops.row_product(a, b))
     assert _kernel() == b"split_product_kernel"
+
+
+@pytest.mark.parametrize("e", [12, 13, 14, 20])
+def test_parts_below_the_smallest_normal_number(cuda, e):
+    """A value whose second part is subnormal in bf16 (up to e = 13 none of its bits are lost there) and the only one that counts: its product is exact."""
+    m, k, n = 100_001, 100, 64
+    few = 2.0 ** -120 * (1 + 2.0 ** -e)
+    a, b = torch.zeros((m, k), device=cuda), torch.zeros((k, n), device=cuda)
+    a[:, 7], b[7] = few, 2.0 ** 110
+    got = ops.row_product(a, b)
+    assert _kernel() == b"split_product_kernel" and bool((got == few * 2.0 ** 110).all())
+    a[:, 7], b[7] = 2.0 ** 110, few
+    assert bool((ops.row_product(a, b) == few * 2.0 ** 110).all())
+    x, y = torch.zeros((5000, 100), device=cuda), torch.zeros((5000, 256), device=cuda)
+    for row in (0, 4999):
+        x.zero_(), y.zero_()
+        x[row], y[row] = few, 2.0 ** 110
+        assert bool((ops.weight_grad(x, y) == few * 2.0 ** 110).all()) and _kernel() == b"wgrad_kernel in parts"
