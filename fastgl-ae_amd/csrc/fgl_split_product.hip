@@ -1,6 +1,9 @@
 // Products over the rows of a block in fp32 (what fgl_row_product.hip forms, which see), on the bf16 matrix cores: C[m, n] = A[m,
 // k] B[k, n].
 //
+// (The parts: G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019; how they are summed and when they are not taken is this file's.)
+//
 // Why: the fp32 matrix instructions reach 157 TFLOP/s, the bf16 ones 2500.  An fp32 value is the sum of three bf16 values,
 // exactly, so a product is six bf16 products and loses only terms below 2^-26 of it: a2 b0, a0 b2, a1 b1, a1 b0, a0 b1, a0 b0 of
 // a = a0 + a1 + a2, b = b0 + b1 + b2, 2.6 times the rate.
@@ -329,7 +332,7 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
     const unsigned per_group = 8u * (unsigned)g.tiles_n;
     const int64_t rb = (int64_t)(blockIdx.x / per_group) * 8 + blockIdx.x % per_group % 8;
     const int col0 = (int)(blockIdx.x % per_group / 8) * 32 * NT;
-    if (rb >= g.row_blocks) return;  // (uniform over the workgroup)
+    if (rb * W * 32 >= g.m) return;  // (uniform over the workgroup: no row tile for it)
     const int chunks0 = sp_chunks(g.side[0].k), chunks = chunks0 + (FORM == kRpSum ? sp_chunks(g.side[1].k) : 0);
     const int64_t row_tiles = (g.m + 31) / 32, stride = g.row_blocks * W;
     int64_t tile = rb * W + wave;
@@ -503,23 +506,39 @@ static int sp_tiles(const RowProductArgs& g)
 }
 
 // Whether the split pays, against the fp32 instructions' kernel, which has nothing to stage first and pads less.  A step here is
-// 32 k and 32 to 128 columns: what they pad makes the line higher (us, that kernel / this: 909 K x 8 x 33 42 / 70, 454 K x 8 x 66
-// 31 / 60, 234 K x 16 x 128 27 / 29, 106 K x 33 x 66 19 / 22, but 140 K x 33 x 100 28 / 24).  Otherwise it lies at 4.3e8
-// multiplications: 100 x 64: 39 K rows 13 / 12, 62 K 15 / 13; 100 x 256: 9800 13 / 12, 27 K 22 / 20; 200 x 128: 13 K 12 / 15, 20 K
-// 21 / 15; 256 x 66: 25 K 21 / 17; 602 x 256: 6400 30 / 24; up to two steps at 5e8, where it is ahead by more (64 x 128: 54 K 17 /
-// 16, 109 K 31 / 24).
+// 32 k and 32 to 128 columns: the line lies at 1.6e8 multiplications, higher by what k and the columns are padded (us, that kernel /
+// this: 909 K x 8 x 33 42 / 70, 106 K x 33 x 66 19 / 22, but 140 K x 33 x 100 28 / 24), by the staging of a longer k (200 x 128: 13 K
+// rows 12 / 15, 20 K 21 / 15; 602 x 64: 7800 13 / 22, 13 K 26 / 23), and where fewer than 1100 tiles of 32 rows leave more than half of
+// the chip's 2048 places for waves empty (100 + 100 x 64: 29 K 13 / 17).  Of 900 products of 17 to 832 k, 2 to
+// 3000 columns and 8e7 to 1.2e9 multiplications it took 0.8 % longer than the faster one, and 10 more than a tenth longer than that
+// kernel (22 x 85 added to C, 265 K rows, 41 / 58; the others up to 1.18).
+// Up to 32 k, of which half a chunk or more may be zeros, the line lies twice as far out and the pass over C is what counts: this is
+// ahead where that kernel goes over A three times (130 M results: 18 x 92 222 / 138, 12 x 92 209 / 149; 30 M: 18 x 91 33 / 40), in
+// narrow tiles (25 M and 130 M: 18 x 33 48 / 45, 256 / 249, 18 x 64 32 / 24, 158 / 126; but 16 x 33 36 / 45, 202 / 253, 18 x 16 46 / 57)
+// and, of 17 k and more, where a row is one workgroup's or whole lines of 128 bytes are (18 x 100 145 / 135, 18 x 128 128 / 119, 18 x
+// 256 123 / 108, 27 x 256, 38 M, 48 / 30; but 16 x 128, 240 M, 200 / 212, 24 x 127 137 / 245, 24 x 254 147 / 192, 24 x 380 141 / 166).
+// One to three terms are that kernel's, which rounds their sum more exactly.  Odd rows in tiles of 128 columns, stored value by value,
+// need a k that hides that (130 M: 40 x 127 194 / 260, 40 x 126 195 / 213, 40 x 380 202 / 176; 64 x 125, 75 M, 150 / 142).
 // Workgroups of one row block go to one XCD, eight blocks at a time, so that fewer than 2000 rows leave XCDs idle: 1000 x 256 x
 // 4000 22 / 36, 500 x 602 x 16000 192 / 356, 250 x 832 x 30000 521 / 909, 2000 x 256 x 4000 44 / 39.  Results as few as 1.6e6 take
 // that many rows' worth twice: 3000 x 602 x 602 30 / 38, 4000 x 400 x 400 21 / 22.
 bool split_product_pays(const RowProductArgs& g)
 {
     const int k = g.side[0].k + g.side[1].k;
-    if (sp_lds(g, 1) > (size_t)kSpLds || k <= 32 || g.m < 2000 || (g.side[0].ldb | g.side[1].ldb) >> 27 != 0) return false;
+    if (sp_lds(g, 1) > (size_t)kSpLds || g.m < 2000 || (g.side[0].ldb | g.side[1].ldb) >> 27 != 0) return false;
     const double outputs = (double)g.m * g.n;
     if (outputs < (g.m < 5000 ? 2.1e6 : 1.6e6)) return false;
-    const int nt = sp_tiles(g);
-    const double padded_k = 32.0 * (sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)), wide = (double)(ceil_div(g.n, 32 * nt) * 32 * nt), narrow = (double)(ceil_div(g.n, 32) * 32);
-    return outputs * k >= (k <= 64 ? 5e8 : 4.3e8) * (padded_k / k) * (wide / narrow);
+    const int tiles = sp_tiles(g);
+    const int64_t padded_k = 32 * (sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)), column_tiles = ceil_div(g.n, 32 * tiles);
+    const uint64_t starts = (uintptr_t)g.c | (uint64_t)g.ldc * sizeof(float);
+    if (k < 4 || (k <= 16 && (g.n <= 64 || g.n > 96))) return false;
+    if (k <= 32 && (g.n <= 32 || (g.n > 96 && starts % (column_tiles == 1 ? 16 : 128) != 0))) return false;
+    if (k < 56 && g.n > 96 && tiles == 4 && starts % 8 != 0) return false;
+    double line = 1.6e8 + 1e6 * (double)(padded_k > 128 ? padded_k - 128 : 0);
+    line *= (double)padded_k / k * (double)(column_tiles * tiles) / (double)ceil_div(g.n, 32);
+    if (ceil_div(g.m, 32) * column_tiles < 1100) line *= 1.3;
+    if (k <= 32) line *= 2.0;
+    return outputs * k >= line;
 }
 
 template <bool BT, int FORM>

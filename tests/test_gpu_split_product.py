@@ -9,10 +9,12 @@ from fastgl import ops
 pytestmark = pytest.mark.gpu
 
 # (rows, k, columns) on both sides of the line between the kernels: those that are in parts, and those that the fp32 instructions form
-IN_PARTS = [(480_001, 33, 63), (180_001, 48, 129), (440_001, 49, 31), (100_001, 64, 129), (26_001, 100, 256), (95_003, 96, 66), (6_417, 256, 300), (6_500, 416, 250),
-            (6_500, 417, 250), (50_001, 832, 33), (2000, 256, 1100)]
+IN_PARTS = [(480_001, 33, 63), (180_001, 48, 130), (440_001, 49, 31), (100_001, 64, 129), (26_001, 100, 256), (95_003, 96, 66), (6_417, 256, 300), (6_500, 416, 250),
+            (6_500, 417, 250), (50_001, 832, 33), (2000, 256, 1100), (33_269, 100, 128), (1_000_001, 17, 65), (400_003, 32, 40), (5_000_001, 12, 90),
+            (476_628, 100, 6), (24_000, 256, 72), (200_001, 56, 127), (147_000, 27, 256), (700_001, 18, 100)]
 PLAIN = [(1_600_001, 1, 128), (450_017, 7, 65), (210_031, 15, 64), (210_001, 16, 64), (400_033, 17, 31), (97_001, 33, 63), (909_001, 8, 33), (50_001, 833, 33),
-         (1990, 256, 1200), (4000, 400, 400), (32_003, 96, 66)]
+         (1990, 256, 1200), (4000, 400, 400), (32_003, 96, 66), (5_000_001, 3, 90), (1_000_001, 16, 97), (1_000_001, 24, 32), (5_500, 256, 256), (1_000_001, 32, 102),
+         (200_001, 55, 127), (180_001, 48, 129), (300_001, 32, 380)]
 
 
 def _kernel():
@@ -193,7 +195,7 @@ def test_fewer_columns_take_no_longer(cuda, m, k, fewer, more):
 
 
 @pytest.mark.parametrize("first,ldc", [(0, 132), (1, 132), (2, 132), (0, 130), (3, 131), (0, 127)])
-@pytest.mark.parametrize("m,k,n", [(180_001, 48, 127), (100_001, 100, 126), (50_001, 832, 33)])
+@pytest.mark.parametrize("m,k,n", [(180_001, 60, 127), (100_001, 100, 126), (50_001, 832, 33)])
 def test_rows_of_every_alignment(cuda, m, k, n, first, ldc):
     """Results of which every row starts on a vector of four, of two or of one value: all of them, and nothing beside them."""
     gen = torch.Generator(device=cuda).manual_seed(ldc)
