@@ -454,20 +454,22 @@ __global__ __launch_bounds__(W * kWave, 2) void split_product_kernel(const RowPr
 
 static size_t sp_lds(const RowProductArgs& g, int nt) { return (size_t)(sp_chunks(g.side[0].k) + sp_chunks(g.side[1].k)) * 2 * nt * 3 * kWave * sizeof(SpU4); }
 
-// Row blocks, 8 at a time, one to an XCD with all of its tiles along n.  An XCD has `places` for workgroups at once, and one more
-// than that takes as long as as many again: 7 tiles of 128 columns in 64 places are 9 row blocks (63), not 10.  Where much would
-// be left empty (13 tiles: 4 row blocks, 52) more of them in two to four rounds may end sooner: a workgroup takes as long as its
-// waves have row tiles, and two tiles' time to stage B. (us, with one block more than fits / with this: 209 K x 64 x 896 248 /
-// 209, 100 K x 128 x 376 95 / 77, added to C 168 / 112, 119 K x (256 + 256) x 165 302 / 210, 80 K x 256 x 1064 424 / 302.)
-static int64_t sp_row_blocks(int64_t row_tiles, int waves, int64_t places, int64_t tiles_n)
+// Row blocks, 8 at a time, one to an XCD with all of its tiles along n.  An XCD has `places` for workgroups at once, one or two a CU,
+// and one more than that begins when the others end: 7 tiles of 128 columns in 64 places are 9 row blocks (63), not 10.  Where much would
+// be left empty (13 tiles: 4 row blocks, 52) more of them in up to four rounds may end sooner: a workgroup takes as long as its waves have
+// row tiles, and two tiles' time to stage B; six tenths of that in a last round that has the CUs to itself, so that half rounds count too.
+// (us, with one block more than fits / with this: 209 K x 64 x 896 248 / 209, 100 K x 128 x 376 95 / 77, added to C 168 / 112, 119 K x (256 +
+// 256) x 165 302 / 210, 80 K x 256 x 1064 424 / 302; whole rounds only / with this: 19 K x 128 x 2970 126 / 113.)
+static int64_t sp_row_blocks(int64_t row_tiles, int waves, int per_cu, int64_t tiles_n)
 {
-    const int64_t want = ceil_div(ceil_div(row_tiles, waves), 8);  // (of an XCD: a tile a wave)
+    const int64_t places = 32 * per_cu, want = ceil_div(ceil_div(row_tiles, waves), 8);  // (of an XCD: a tile a wave)
     int64_t best = 1, least = INT64_MAX;
-    for (int64_t rounds = 1; rounds <= 4; ++rounds) {
-        int64_t n = places * rounds / tiles_n;
+    for (int64_t halves = 2; halves <= 8; ++halves) {
+        int64_t n = places * halves / (2 * tiles_n);
         if (n < 1) n = 1;
         if (n > want) n = want;
-        const int64_t time = ceil_div(n * tiles_n, places) * (2 + ceil_div(row_tiles, 8 * n * waves));
+        const int64_t rest = n * tiles_n % places, last = rest == 0 ? 0 : per_cu == 2 && rest <= 32 && n * tiles_n > places ? 6 : 10;
+        const int64_t time = (n * tiles_n / places * 10 + last) * (2 + ceil_div(row_tiles, 8 * n * waves));
         if (time < least) {
             least = time;
             best = n;
@@ -487,7 +489,7 @@ static int launch_split_product(RowProductArgs g, hipStream_t stream)
     // as many neighbouring columns a lane as every row's start allows
     const uint64_t starts = (uintptr_t)g.c | (uint64_t)g.ldc * sizeof(float);
     g.vec_log = NT >= 4 && starts % 16 == 0 ? 2 : NT >= 2 && starts % 8 == 0 ? 1 : 0;
-    g.row_blocks = sp_row_blocks(ceil_div(g.m, 32), W, 32 * per_cu, g.tiles_n);
+    g.row_blocks = sp_row_blocks(ceil_div(g.m, 32), W, (int)per_cu, g.tiles_n);
     const int64_t blocks = ceil_div(g.row_blocks, 8) * 8 * g.tiles_n;
     FGL_REQUIRE(blocks <= 0x7FFFFFFF, "row_product: grid too large");
     hipLaunchKernelGGL((split_product_kernel<NT, W, BT, FORM>), dim3((unsigned)blocks), dim3(W * kWave), lds, stream, g);
