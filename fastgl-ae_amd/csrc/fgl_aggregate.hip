@@ -1180,7 +1180,8 @@ constexpr int kClasses = 8;
 constexpr int kClassEntries = 256;                       // rows of fewer entries have too few a class to be worth eight sums
 constexpr int64_t kClassMinEntries = (int64_t)3 << 22;
 constexpr int kClassMinRow = 256;                        // bytes of a gathered row: of shorter ones an L2 holds enough as it is
-constexpr int64_t kClassMinBytes = (int64_t)64 << 20;    // of the gathered rows: twice what the L2s hold together
+constexpr int64_t kClassMinBytes = (int64_t)64 << 20;    // of the rows of results
+constexpr int64_t kClassMinSource = (int64_t)12 << 20;   // of the gathered rows: what three L2s hold (see class_bytes)
 constexpr size_t kClassMaxBytes = (size_t)4 << 30;       // of scratch
 __device__ __forceinline__ int neighbour_class(int id) { return (int)(((uint32_t)id >> 5) * 0x9E3779B1u >> 29); }
 
@@ -1210,12 +1211,15 @@ static SegLists seg_lists(void* ws, int64_t n_entries_max, int D, bool classes, 
     return l;
 }
 
-// What classes take, 0 where they do not pay.  (The rows that are gathered are the source's; as few rows of results are blocks,
-// of which nothing was measured.)
+// What classes take, 0 where they do not pay.  Sources of a few L2s stay in each of them as they are (us, segments as they come / in
+// classes, 1.2 M rows of 20 entries and hubs: 256-byte fp32 rows, 16 K of them 1600 / 2190, 32 K 1980 / 2300, 64 K 2870 / 2530, 128 K
+// 3390 / 2690, 256 K 3760 / 3040; 400 bytes, 16 K 3170 / 3650, 32 K 4660 / 4120, 64 K 5960 / 4500; 128 bf16 columns, 32 K 2190 / 2650,
+// 64 K 2860 / 2780, 128 K 3440 / 3000).  Few rows of results are blocks, of which nothing was measured.
 static size_t class_bytes(int64_t n_entries_max, int64_t n_rows_max, int64_t n_source_rows, int D, int dtype, int64_t longest_row_max)
 {
-    const int64_t row = D * (int64_t)(dtype == FGL_F32 ? sizeof(float) : sizeof(uint16_t)), rows = n_rows_max < n_source_rows ? n_rows_max : n_source_rows;
-    if (n_entries_max < kClassMinEntries || row < kClassMinRow || rows * row < kClassMinBytes || (longest_row_max >= 0 && longest_row_max <= kClassEntries)) return 0;
+    const int64_t row = D * (int64_t)(dtype == FGL_F32 ? sizeof(float) : sizeof(uint16_t));
+    if (n_entries_max < kClassMinEntries || row < kClassMinRow || n_rows_max * row < kClassMinBytes || n_source_rows * row < kClassMinSource) return 0;
+    if (longest_row_max >= 0 && longest_row_max <= kClassEntries) return 0;
     size_t bytes = 0;
     (void)seg_lists(nullptr, n_entries_max, D, true, &bytes);
     return bytes <= kClassMaxBytes ? bytes : 0;

@@ -23,5 +23,6 @@ def test_aggregate():
     # rows of 128 bytes, few rows on either side, no row long enough: what is never gathered by classes asks for no more than the segments take
     assert plain == size(64, L.BF16) == size(64, L.F32, rows=8192) == size(64, L.F32, sources=8192) == size(64, L.F32, longest=256)
     assert size(64, L.F32, longest=257) > plain
+    assert size(64, L.F32, sources=49_152) > plain == size(64, L.F32, sources=49_151)  # (12 MB of gathered rows)
     assert size(64, L.F32, longest=128) == 0 and size(64, L.F32, entries=1000) == 0
     assert size(3000, L.F32, entries=2_000_000_000) == lib.fgl_aggregate_workspace_bytes(2_000_000_000, 3000, L.AGG_GCN, -1)  # (classes would take more than 4 GiB)
