@@ -79,3 +79,25 @@ def test_ids_that_recur_in_runs(cuda, n, bins, times):
         return best
 
     assert time(runs) < times * time(no_order)
+
+
+@pytest.mark.parametrize("n", [8_886_435, 8_886_272])
+def test_sorted_ids_of_few_counters(cuda, n):
+    """A last tile that is not full counts as in order too: alone in buckets it kept the launches behind waiting, half as long again."""
+    x = torch.randint(0, 176, (n,), device=cuda, dtype=torch.int32).sort()[0]
+    for part in (x, x[:-1], x[:-8000], x[5:]):
+        part = part.contiguous()
+        assert torch.equal(ops.cal_deg(part, 176), torch.bincount(part.long(), minlength=176).int())
+    best = []
+    for ids in (x, x[:8192 * 1084].contiguous()):
+        times = []
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(20):
+                ops.cal_deg(ids, 176)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        best.append(min(times))
+    assert best[0] < 1.25 * best[1]
