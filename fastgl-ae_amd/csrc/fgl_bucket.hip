@@ -22,7 +22,7 @@
 //     Within a bucket a column is 16 bits.  Traffic: 2 reads of the ids, 2 writes and reads of the rows, 1 write and 2 reads of
 //     half the columns.
 //     (54 M entries of a 2.4 M-node graph, hubs of 85 K, us: counts, with an atomic per entry 5900 / 13200 -- unordered / sorted
-//     ids --, with 4-byte stores all over the buckets 499 / 674, now 276 / 187; transpose 24700, 1550, now 700.)
+//     ids --, with 4-byte stores all over the buckets 499 / 674, now 276 / 180; transpose 24700, 1550, now 700.)
 #include "fgl_common.hpp"
 #include "fgl_kernels.hpp"
 #include "fgl_tile_rows.hpp"
@@ -165,18 +165,18 @@ __device__ __forceinline__ void load_columns(const BucketArgs& g, int64_t first,
 // DIRECT (counting only): a tile of an input in order, in runs of equal ids -- the destinations of an edge list -- is counted
 // here, one atomic a run in device memory, and the launches behind pass it by; what two tiles share of a hub is one atomic each.
 // In order is more than the tile's own ids: device memory does not take updates of the same few counters from all over the chip.
-// So the first ids of the input's 64 parts of neighbouring tiles have to ascend, and the tile's ids, from the tile before on, to
-// lie between those of its part and the next one: a counter is touched by tiles of one part, most of them one XCD's, or of parts
-// that hold one id.  Within a part ids may still recur, which costs least where runs are long.
-// Whole counts, us, by buckets alone / with it: 54 M destinations of an R-MAT graph of 2.4 M nodes 274 / 183, sorted uniform ids,
-// 22 a run, 270 / 187, 11 a run 277 / 252, in no order 280 / 284; 20 M over 100 K, sorted 82 / 53; 5 M over 400 K, sorted, 43 /
-// 39, over 600 K, eight a run and so not direct, 41 / 42, in no order 37.4 / 38.5.  Sorted stretches, which only cost the look:
-// 54 M in stretches of two tiles over 500 ids 254 / 262, of 2 M ids over 130 K 180 / 187.
-// kDirectRun of 8: 11 a run 251, but stretches of two tiles whose ids begin anew for each 64th part, eight a run, 180 / 204; of 4
-// 180 / 510 for such of five a run; of 14 the graph 192.  Without the parts, stretches of two tiles over 500 ids took 879; when
-// the tile's first wave alone was looked at, for runs of four, fives of two ids in turn 122477, tiles in order up to their eighth
-// 1857.
-constexpr int kDirectRun = 10;
+// So the first ids of the input's 64 parts of neighbouring tiles have to ascend, and those of 64 tiles of the tile's own part (all of
+// them up to 33 M ids), and the tile's ids, from the tile before on, to lie between those of its part and the next one: a counter is
+// touched by neighbouring tiles, most of them one XCD's, or by parts that hold one id.
+// Whole counts, us, by buckets alone / with it: 54 M destinations of an R-MAT graph of 2.4 M nodes 272 / 179, sorted uniform ids,
+// 22 a run, 270 / 180, 11 a run 277 / 251, in no order 280 / 280; 20 M over 900 K, sorted 82 / 70; 5 M over 500 K, sorted, 46 / 35,
+// over 600 K, eight a run, 42 / 39, in no order 37.4 / 38.3.  Sorted stretches, which only cost the look: 54 M in stretches of two tiles
+// over 500 ids 254 / 264, of such that begin anew for each 64th part 201 / 210.
+// kDirectRun of 5: sorted uniform ids of five a run 348, six 341 where 6 takes 310 and 292; of 8: 310 and 280, but skewed sorted ids (u^4
+// of 2.5 M, 22 a run) 256 where 6 takes 213 (buckets 274).  Without the parts, stretches of two tiles over 500 ids took 879; without the
+// tiles of a part, such that begin anew for each part, five a run, 510; when the tile's first wave alone was looked at, for runs of four,
+// fives of two ids in turn 122477, tiles in order up to their eighth 1857.
+constexpr int kDirectRun = 6;
 
 template <bool DIRECT>
 __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketArgs g)
@@ -233,6 +233,17 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_hist_kernel(const BucketA
                 if (lane == kWave - 1) next = INT32_MAX;
                 most = __shfl(next, part, kWave);
                 may_be = __all(begin <= next) && __all(c[0] >= __shfl(begin, part, kWave) || left == 0);
+                if (may_be) {  // and the first ids of 64 tiles of its part
+                    const int64_t from = ((int64_t)part * per + (int64_t)lane * per / kWave) * kBucketTile;
+                    int id = INT32_MAX;
+                    if (from < n) {
+                        id = g.ids[from];
+                        if (id >= g.n_cols) id = -1;
+                    }
+                    int after = __shfl_down(id, 1, kWave);
+                    if (lane == kWave - 1) after = most;
+                    may_be = __all(id <= after);
+                }
             }
             if (tid == 0) {
                 s_direct = may_be;

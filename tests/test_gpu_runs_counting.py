@@ -1,5 +1,5 @@
 """Counts of large inputs that lie in runs of equal ids (csrc/fgl_bucket.hip): sorted ids, hubs over several tiles of 8192, runs
-on either side of the limit of ten entries, in order and in none, tiles of either kind in turn, tiles in order only at their
+on either side of the limit of six entries, in order and in none, tiles of either kind in turn, tiles in order only at their
 beginning or up to their last entries, sorted stretches one after another, also as long as the 64th parts of the input or with ids
 beyond those, ids that no counter has -- against torch.bincount; and that ids which recur in runs take no longer."""
 import pytest
@@ -9,7 +9,7 @@ from fastgl import ops
 
 pytestmark = pytest.mark.gpu
 N, BINS, TILE = 3_000_017, 700_000, 8192
-UP = {"fives up": 5, "nines up": 9, "tens up": 10, "elevens up": 11, "hundreds up": 100, "hundreds down": 100}
+UP = {"fives up": 5, "sixes up": 6, "sevens up": 7, "tens up": 10, "hundreds up": 100, "hundreds down": 100}
 
 
 def _ids(kind, gen, dev):
@@ -58,12 +58,14 @@ def test_counts(cuda, kind):
         assert torch.equal(ops.cal_deg(part, BINS), want)
 
 
-@pytest.mark.parametrize("n,bins,times", [(5_000_000, 2, 10), (5_000_000, 1000, 10), (5_000_000, 2048, 10), (54_000_000, 497, 2)])
+@pytest.mark.parametrize("n,bins,times", [(5_000_000, 2, 10), (5_000_000, 1000, 10), (5_000_000, 2048, 10), (54_000_000, 497, 2), (54_000_000, 600_000, 2)])
 def test_ids_that_recur_in_runs(cuda, n, bins, times):
     """An atomic a run in device memory would take hundreds of times as long for the first of these (54 M ids, fives of two ids in
-    turn: 122 ms against 0.26), and more than three times as long for the last, sorted stretches of two tiles (880 us against 260)."""
+    turn: 122 ms against 0.26), and more than three times as long for the
+    last but one, sorted stretches of two tiles (880 us against 260); such that begin anew for each 64th part of the input, the last, pass a look at the parts alone."""
     i = torch.arange(n, device=cuda)
-    runs = (i % (2 * TILE) // 33 if bins == 497 else i % TILE // 4 if bins == 2048 else i // 5 % bins).int()
+    part = (n // TILE + 64) // 64 * TILE
+    runs = (i // part * 8000 + i % (2 * TILE) // 8 if bins == 600_000 else i % (2 * TILE) // 33 if bins == 497 else i % TILE // 4 if bins == 2048 else i // 5 % bins).int()
     no_order = torch.randint(0, bins, (n,), device=cuda, dtype=torch.int32)
 
     def time(x):
